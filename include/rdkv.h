@@ -126,6 +126,28 @@ int rdkv_dequant_f16(const uint8_t *packed, int64_t rows, int n_cols_unpacked, i
                      const void *scale_f16, const void *zp_f16, int per_row,
                      void *out_f16, int64_t out_row_stride, void *stream);
 
+/* A packed layer back to dense fp16 (unpack_k_mixed packing.py:581-709; _unpack_v_perhead and the
+ * zone B rows, trizone_decompress.py:91-182), one launch per side, every byte of the output written.
+ * rdkv_unpack_layer_k: out [H_kv, T, D]; K2/K4/K8 [H_kv, T, n2p/4 | n4p/2 | n8w] bytes (NULL where the
+ * width is 0), scale / zp [H_kv, n2p + n4p + n8w], sort_idx int64 [H_kv or 1 (stride 0), sort_n]: the
+ * channel of every kept slot in order; kept channels per class from counts (device int32 [H_kv, 3]) or,
+ * when counts is NULL, n2, n4, n8 for all heads.  Channels that are not kept are +0.
+ * rdkv_unpack_layer_v: out [H_kv, max_tv + n16, D]: a head's counts[h] = (n2, n4, n8) tokens (at most
+ * m2, m4, m8: the rows of V2 / V4 / V8, stored back to back), zero rows up to max_tv, then the n16 rows
+ * of V16 [H_kv, n16, D] fp16.  Counts beyond the rows that exist are clamped. */
+int rdkv_unpack_layer_k(const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t,
+                        const uint8_t *K4, int64_t k4_stride_h, int64_t k4_stride_t,
+                        const uint8_t *K8, int64_t k8_stride_h, int64_t k8_stride_t,
+                        const void *scale_f16, const void *zp_f16, int64_t ks_stride_h,
+                        const int64_t *sort_idx, int64_t sort_stride_h, int sort_n, const int32_t *counts,
+                        int n2, int n4, int n8, int n2p, int n4p, int n8w, int H_kv, int64_t T, int D,
+                        void *out_f16, void *stream);
+int rdkv_unpack_layer_v(const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h,
+                        const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
+                        int64_t s_stride_h, const int32_t *counts, int m2, int m4, int m8, int64_t max_tv,
+                        const void *V16_f16, int64_t v16_stride_h, int n16, int H_kv, int D,
+                        void *out_f16, void *stream);
+
 /* ---- triton_k_kernel.py : k_mixed_qk_dot_into (:1211-1411) ---------------- */
 /* out[hq, t] = (sum_c code[hkv,t,c] * q[hq, perm[c]] * s[hkv,c] - sum_c z*q*s) / sqrt(128),
  * t < T_eff, reading the reference's padded layout.  q: [H_q,128] of q_dtype.

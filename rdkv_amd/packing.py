@@ -342,40 +342,65 @@ def _dequant(packed: Tensor, ncols: int, n_bits: int, scale: Tensor, zp: Tensor,
     return out.reshape(*packed.shape[:-1], ncols)
 
 
-def unpack_k_mixed(packed: "PackedKVLayer", D: int) -> Tensor:
-    """Dequantize packed K to fp16 [1,H_kv,T,D]; pruned channels are 0 (packing.py:581-709)."""
+def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional[Tensor]]:
+    """``unpack_k_mixed`` as one launch: the dense rows, and the per-head class counts that were read on
+    the device and are yet to be checked against the segments (``_check_k_counts``)."""
     if packed.K_ch_scale is None:
         raise ValueError("unpack_k_mixed: K_ch_scale missing")
     dev = _lib.require_device(packed.K_ch_scale)
     H = packed.K_ch_scale.shape[1]
     T = packed.T_eff_k if packed.T_eff_k > 0 else packed.T_eff
     m2, m4, m8 = packed.K_ch_seg_bounds
-    m2p, m4p = _seg_padded_len(m2, 4), _seg_padded_len(m4, 2)
-    K_hat = torch.zeros(1, H, T, D, dtype=torch.float16, device=dev)
-    segs = ((packed.K_2bit, m2p, 2, 0), (packed.K_4bit, m4p, 4, m2p), (packed.K_8bit, m8, 8, m2p + m4p))
-    if not any(t is not None and w > 0 for t, w, _, _ in segs):
-        return K_hat
-    per_head = packed.K_ch_seg_bounds_per_head is not None
-    if per_head:
-        assert packed.K_ch_sort_idx_per_head is not None, "per-head layout requires K_ch_sort_idx_per_head"
-        counts = packed.K_ch_seg_bounds_per_head.detach().cpu().tolist()
-        sort_rows = packed.K_ch_sort_idx_per_head
-    for h in range(H):
-        sc = packed.K_ch_scale[0, h, 0]
-        zz = packed.K_ch_zp[0, h, 0]
-        n2, n4, n8 = counts[h] if per_head else (m2, m4, m8)
-        if n2 + n4 + n8 == 0:
+    widths = (_seg_padded_len(m2, 4), _seg_padded_len(m4, 2), m8)
+    segs = []
+    for t, w, bits in zip((packed.K_2bit, packed.K_4bit, packed.K_8bit), widths, (2, 4, 8)):
+        if t is None or w == 0:
+            segs.append((None, 0, 0, 0))
             continue
-        pieces = []
-        for (t, width, bits, off), n in zip(segs, (n2, n4, n8)):
-            if t is None or width == 0 or n == 0:
-                assert n == 0 or t is not None
-                continue
-            deq = _dequant(t[0, h], width, bits, sc[off:off + width], zz[off:off + width], per_row=False)
-            pieces.append(deq[:, :n])
-        idx = (sort_rows[h, :n2 + n4 + n8] if per_head else packed.K_ch_sort_idx[:n2 + n4 + n8])
-        K_hat[0, h].index_copy_(1, idx, torch.cat(pieces, dim=1))
-    return K_hat
+        t = t if t.stride(3) == 1 else t.contiguous()
+        assert t.shape[1:] == (H, T, w * bits // 8), f"K segment {tuple(t.shape)} for {H} heads, {T} tokens, {w} channels"
+        segs.append((t, t.stride(1), t.stride(2), w))
+    if not any(s[3] for s in segs):
+        return torch.zeros(1, H, T, D, dtype=torch.float16, device=dev), None
+    sc, zz = packed.K_ch_scale, packed.K_ch_zp
+    if sc.stride(3) != 1 or zz.stride() != sc.stride():
+        sc, zz = sc.contiguous(), zz.contiguous()
+    counts, limits = None, tuple(n if s[3] else 0 for n, s in zip((m2, m4, m8), segs))
+    if packed.K_ch_seg_bounds_per_head is not None:
+        assert packed.K_ch_sort_idx_per_head is not None, "per-head layout requires K_ch_sort_idx_per_head"
+        counts = packed.K_ch_seg_bounds_per_head.to(device=dev, dtype=torch.int32).contiguous()
+        sort = packed.K_ch_sort_idx_per_head
+    else:
+        assert limits == (m2, m4, m8), "a K segment is missing"
+        sort = packed.K_ch_sort_idx
+    sort = sort.to(torch.long)
+    sort = sort if sort.stride(-1) == 1 else sort.contiguous()
+    out = torch.empty(1, H, T, D, dtype=torch.float16, device=dev)
+    (K2, k2h, k2t, w2), (K4, k4h, k4t, w4), (K8, k8h, k8t, w8) = segs
+    if [w for w in (w2, w4, w8)] != list(widths):
+        # slots of a missing segment do not exist: scales and zero points without their columns
+        keep = torch.cat([torch.arange(o, o + w, device=dev) for o, w in
+                          zip((0, widths[0], widths[0] + widths[1]), (w2, w4, w8))])
+        sc, zz = sc.index_select(3, keep), zz.index_select(3, keep)
+    _lib.check(_lib.load().rdkv_unpack_layer_k(
+        _lib.ptr(K2), k2h, k2t, _lib.ptr(K4), k4h, k4t, _lib.ptr(K8), k8h, k8t, _lib.ptr(sc), _lib.ptr(zz), sc.stride(1),
+        _lib.ptr(sort), sort.stride(0) if sort.dim() == 2 else 0, int(sort.shape[-1]), _lib.ptr(counts), *limits,
+        w2, w4, w8, H, T, D, _lib.ptr(out), _lib.stream_of(dev)))
+    return out, counts
+
+
+def _check_k_counts(packed: "PackedKVLayer", counts: Sequence[Sequence[int]]) -> None:
+    for row in counts:
+        for n, t in zip(row, (packed.K_2bit, packed.K_4bit, packed.K_8bit)):
+            assert n == 0 or t is not None, f"a head keeps {n} channels of a K segment that is missing"
+
+
+def unpack_k_mixed(packed: "PackedKVLayer", D: int) -> Tensor:
+    """Dequantize packed K to fp16 [1,H_kv,T,D]; pruned channels are 0 (packing.py:581-709)."""
+    out, counts = _unpack_k_enqueue(packed, D)
+    if counts is not None:
+        _check_k_counts(packed, counts.tolist())
+    return out
 
 
 # ---------------------------------------------------------------------------

@@ -11,7 +11,8 @@ from typing import List, Optional, Tuple
 import torch
 from torch import Tensor
 
-from .packing import PackedKVLayer, TriZoneCache, unpack_k_mixed, unpack_v_segment
+from . import _lib
+from .packing import PackedKVLayer, TriZoneCache, _check_k_counts, _unpack_k_enqueue, unpack_v_segment
 
 
 def _unpack_v_zone_a(pl: PackedKVLayer) -> Tensor:
@@ -35,25 +36,50 @@ def _is_perhead_layout(pl: PackedKVLayer) -> bool:
     return pl.seg_bounds_per_head is not None
 
 
+def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int) -> Tuple[Tensor, Tensor]:
+    """The stripe's dense V, ``zone_b`` rows behind it, in one launch; and the device's per-head counts
+    (2-, 4-, 8-bit, all), yet to be checked (``_check_v_counts``)."""
+    max_T_v = int(pl.T_eff)
+    H_kv = pl.V_scale.shape[1]
+    dev = _lib.require_device(pl.V_scale)
+    counts = pl.seg_bounds_per_head.to(device=dev, dtype=torch.int32).contiguous()
+    check = torch.cat([counts, pl.T_eff_per_head.to(device=dev, dtype=torch.int32).reshape(H_kv, 1)], dim=1)
+    n16 = 0 if zone_b is None else int(zone_b.shape[2])
+    out = torch.empty(1, H_kv, max_T_v + n16, head_dim, dtype=torch.float16, device=dev)
+    segs = []
+    for seg, bits in zip((pl.V_2bit, pl.V_4bit, pl.V_8bit), (2, 4, 8)):
+        if seg is None or seg.numel() == 0:
+            segs.append((None, 0, 0))
+            continue
+        width = head_dim * bits // 8
+        assert seg.shape[3] == width, f"V rows of {seg.shape[3]} bytes, expected {width}"
+        seg = seg if seg.stride(3) == 1 and seg.stride(2) == width else seg.contiguous()
+        segs.append((seg, seg.stride(1), int(seg.shape[2])))
+    sc, zp = pl.V_scale, pl.V_zp
+    if sc.numel() and not (sc.stride(2) == 1 and zp.stride() == sc.stride()):
+        sc, zp = sc.contiguous(), zp.contiguous()
+    if zone_b is not None and not (zone_b.stride(3) == 1 and zone_b.stride(2) == head_dim):
+        zone_b = zone_b.contiguous()
+    (V2, v2h, m2), (V4, v4h, m4), (V8, v8h, m8) = segs
+    _lib.check(_lib.load().rdkv_unpack_layer_v(
+        _lib.ptr(V2), v2h, _lib.ptr(V4), v4h, _lib.ptr(V8), v8h, _lib.ptr(sc), _lib.ptr(zp), sc.stride(1),
+        counts.data_ptr(), m2, m4, m8, max_T_v, _lib.ptr(zone_b), zone_b.stride(1) if n16 else 0, n16, H_kv, head_dim,
+        _lib.ptr(out), _lib.stream_of(dev)))
+    return out, check
+
+
+def _check_v_counts(counts) -> None:
+    for h, row in enumerate(counts):
+        assert sum(row[:3]) == row[3], f"head {h}: seg_bounds_per_head {row[:3]} != T_eff_per_head {row[3]}"
+
+
 def _unpack_v_perhead(pl: PackedKVLayer, *, head_dim: int) -> Tensor:
     """Stripe layout: [1,H_kv,max_T_v,D] fp16, head h filled on [0,T_v_h), zeros after
     (trizone_decompress.py:91-144)."""
-    max_T_v = int(pl.T_eff)
-    H_kv = pl.V_scale.shape[1]
-    out = torch.zeros(1, H_kv, max_T_v, head_dim, dtype=torch.float16, device=pl.V_scale.device)
-    if max_T_v == 0:
-        return out
-    counts = pl.seg_bounds_per_head.cpu().tolist()
-    tv = pl.T_eff_per_head.cpu().tolist()
-    for h in range(H_kv):
-        assert sum(counts[h]) == tv[h], f"head {h}: seg_bounds_per_head {counts[h]} != T_eff_per_head {tv[h]}"
-        off = 0
-        for n, seg, bits in zip(counts[h], (pl.V_2bit, pl.V_4bit, pl.V_8bit), (2, 4, 8)):
-            if n > 0 and seg is not None:
-                out[:, h:h + 1, off:off + n] = unpack_v_segment(
-                    seg[:, h:h + 1, :n], pl.V_scale[:, h:h + 1, off:off + n],
-                    pl.V_zp[:, h:h + 1, off:off + n], bits)
-                off += n
+    if int(pl.T_eff) == 0:
+        return torch.zeros(1, pl.V_scale.shape[1], 0, head_dim, dtype=torch.float16, device=pl.V_scale.device)
+    out, check = _unpack_v_enqueue(pl, None, head_dim)
+    _check_v_counts(check.tolist())
     return out
 
 
@@ -66,16 +92,26 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
     shared-layout layers) (trizone_decompress.py:185-333)."""
     past_kv: List[Tuple[Tensor, Tensor]] = []
     masks: List[Optional[Tensor]] = []
+    unchecked: List[Tuple[Optional[PackedKVLayer], Tensor]] = []     # per-head counts the launches below read
     for i, pl in enumerate(dual_cache.packed):
-        K_full = unpack_k_mixed(pl, D=head_dim)
+        K_full, k_counts = _unpack_k_enqueue(pl, head_dim)
+        if k_counts is not None:
+            unchecked.append((pl, k_counts))
         zone_b = dual_cache.new_v_only[i] if i < len(dual_cache.new_v_only) else None
         if _is_perhead_layout(pl):
-            zone_a = _unpack_v_perhead(pl, head_dim=head_dim)
+            rows_b = None
             if int(pl.n_v16) > 0:
                 assert zone_b is not None, f"layer {i}: max_n_v16={pl.n_v16} > 0 but new_v_only is None"
-                V_full = torch.cat([zone_a, zone_b], dim=2) if int(pl.T_eff) > 0 else zone_b
+                rows_b = zone_b
+            if int(pl.T_eff) == 0:
+                V_full = rows_b if rows_b is not None else _unpack_v_perhead(pl, head_dim=head_dim)
             else:
-                V_full = zone_a
+                joined = rows_b is not None and rows_b.dtype == torch.float16 and rows_b.shape[:2] == pl.V_scale.shape[:2] \
+                    and rows_b.shape[3] == head_dim and rows_b.device == pl.V_scale.device
+                V_full, v_counts = _unpack_v_enqueue(pl, rows_b if joined else None, head_dim)
+                unchecked.append((None, v_counts))
+                if rows_b is not None and not joined:
+                    V_full = torch.cat([V_full, rows_b], dim=2)
         else:
             zone_a = _unpack_v_zone_a(pl)
             if zone_b is not None and zone_b.shape[2] > 0:
@@ -103,4 +139,13 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
                 masks.append(m4.contiguous())
             else:
                 masks.append(None)
+    # the counts of every layer in one read, behind the launches (which clamp what they follow)
+    if unchecked:
+        rows = iter(_lib.download(torch.cat([c.reshape(-1) for _, c in unchecked])).tolist())
+        for pl, c in unchecked:
+            table = [[next(rows) for _ in range(c.shape[1])] for _ in range(c.shape[0])]
+            if pl is None:
+                _check_v_counts(table)
+            else:
+                _check_k_counts(pl, table)
     return (tuple(past_kv), masks) if return_masks else tuple(past_kv)

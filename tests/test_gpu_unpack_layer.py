@@ -1,0 +1,86 @@
+"""The whole-layer dequantizers (``rdkv_unpack_layer_k`` / ``rdkv_unpack_layer_v``) at the edges of
+their tiles and of their fast paths, bit for bit against the oracle's unpackers: token counts around
+the 64-row tile, head dimensions that are no multiple of the 8-channel and 32-channel forms or need
+several channel chunks, segments that are views of wider tensors, a head without tokens or channels."""
+import dataclasses
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import rdkv_oracle as O
+from rdkv_amd import packing, trizone_decompress as tz
+from tests.gpu_util import DEV, assert_bits_equal, layer_to_device, require_gpu, t2n, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _widened(t, dim):
+    """The same values as a view into a larger tensor (row stride no longer the row length)."""
+    if t is None:
+        return None
+    shape = list(t.shape)
+    shape[dim] += 3
+    wide = torch.full(shape, 0xAB, dtype=t.dtype, device=t.device)
+    view = wide.narrow(dim, 0, t.shape[dim])
+    view.copy_(t)
+    return view
+
+
+@pytest.mark.parametrize("D,T,H", [(128, 1, 1), (128, 63, 2), (128, 64, 3), (128, 65, 2), (128, 1500, 8),
+                                   (8, 70, 2), (36, 130, 2), (64, 129, 3), (256, 200, 2), (264, 67, 2)])
+def test_whole_layer_dequantizers_against_the_oracle(D, T, H):
+    require_gpu()
+    rng = np.random.default_rng(1000 * D + T)
+    K = rng.standard_normal((1, H, T, D)).astype(np.float16)
+    V = rng.standard_normal((1, H, T, D)).astype(np.float16)
+    vb = rng.choice(np.array([0, 2, 4, 8, 16]), size=(H, T))
+    vb[0, 0] = 4
+    kb = rng.choice(np.array([0, 2, 4, 8]), size=(H, D))
+    kb[0, :4] = (2, 4, 8, 8)
+    if H > 1:
+        vb[-1] = 0                       # a head that keeps nothing, with channels all the same
+    ora, ora_nvo = O.pack_layer_per_head(K, V, vb, kb, 2)
+    pl = layer_to_device(ora)
+    exp_k, exp_v = O.unpack_k_mixed(ora, D), O._unpack_v_perhead(ora, head_dim=D)
+    strided = dataclasses.replace(pl, **{n: _widened(getattr(pl, n), 3) for n in ("K_2bit", "K_4bit", "K_8bit")},
+                                  **{n: _widened(getattr(pl, n), 2) for n in ("V_2bit", "V_4bit", "V_8bit")})
+    for layer in (pl, strided):
+        assert_bits_equal(t2n(packing.unpack_k_mixed(layer, D=D)), exp_k)
+        assert_bits_equal(t2n(tz._unpack_v_perhead(layer, head_dim=D)), exp_v)
+        nvo = to_dev(ora_nvo) if ora_nvo is not None else None
+        cache = packing.TriZoneCache((layer,), [nvo], [None], [None], T)
+        (k, v), = tz.unpack_trizone_to_past_kv(cache, head_dim=D)
+        assert_bits_equal(t2n(k), exp_k)
+        assert_bits_equal(t2n(v), exp_v if ora_nvo is None else np.concatenate([exp_v, ora_nvo], axis=2))
+
+
+def test_zero_points_that_are_not_whole_numbers():
+    """Layers of other origin may carry such zero points; they take the fp32 form."""
+    require_gpu()
+    rng = np.random.default_rng(9)
+    K, V = (rng.standard_normal((1, 2, 90, 128)).astype(np.float16) for _ in range(2))
+    vb, kb = rng.choice(np.array([2, 4, 8]), size=(2, 90)), rng.choice(np.array([2, 4, 8]), size=(2, 128))
+    ora, _ = O.pack_layer_per_head(K, V, vb, kb, 2)
+    ora.K_ch_zp[:, 1, :, 5] += np.float16(0.3)
+    ora.V_zp[:, 0, 3] += np.float16(0.7)
+    ora.V_zp[:, 1, 60:] = np.float16(3000.5)
+    pl = layer_to_device(ora)
+    assert_bits_equal(t2n(packing.unpack_k_mixed(pl, D=128)), O.unpack_k_mixed(ora, 128))
+    assert_bits_equal(t2n(tz._unpack_v_perhead(pl, head_dim=128)), O._unpack_v_perhead(ora, head_dim=128))
+
+
+def test_counts_that_do_not_fit_the_layer_are_reported():
+    require_gpu()
+    rng = np.random.default_rng(3)
+    K, V = (torch.from_numpy(rng.standard_normal((1, 2, 100, 128)).astype(np.float16)).to(DEV) for _ in range(2))
+    vb = torch.from_numpy(rng.choice(np.array([2, 4, 8]), size=(2, 100)))
+    kb = torch.from_numpy(rng.choice(np.array([2, 4]), size=(2, 128)))
+    pl, nvo = packing.pack_layer_per_head(K, V, vb, kb, 2)
+    pl.seg_bounds_per_head = pl.seg_bounds_per_head + 1          # within the rows the kernel clamps to
+    cache = packing.TriZoneCache((pl,), [nvo], [None], [None], 100)
+    with pytest.raises(AssertionError, match="T_eff_per_head"):
+        tz.unpack_trizone_to_past_kv(cache, head_dim=128)
+    pl.K_ch_seg_bounds_per_head = pl.K_ch_seg_bounds_per_head + 1          # 8-bit channels, no 8-bit segment
+    with pytest.raises(AssertionError, match="segment that is missing"):
+        packing.unpack_k_mixed(pl, D=128)
