@@ -1027,20 +1027,26 @@ merge_kernel(const RdkvUnit *__restrict__ units, const float *__restrict__ parti
 //    everything else at once - the token count, the step's write row, the query rows and rotation
 //    table, the step's own key / value row, the partials' max / sum columns and accumulator
 //    columns, and the first 64 zone C tokens' K and V rows (requested before the count is known:
-//    rows up to the buffer's end exist, a row past the count is discarded);
-//  * one workgroup of eight wavefronts per unit; wavefront w owns tokens 8w .. 8w + 7 of every
-//    chunk of 64 and keeps its own online-softmax state, so the token loop has no barrier and no
-//    LDS traffic beyond the query: a token's K row is split over eight lanes (16-byte loads, 128
-//    contiguous bytes per token and instruction), the partial dot products are folded inside the
-//    eight lanes and the maximum / sum across the wavefront's eight tokens by data-parallel moves
-//    and lane-permute swaps, the weights are read lane to lane for weight x V (lane = channel
-//    pair, one whole 512-byte row per load instruction), the next chunk's rows in flight meanwhile;
-//  * the eight wavefront states and the zones A+B state are combined once, in a fixed order.
+//    rows up to the buffer's end exist, a row past the count is discarded).  The parts of the preparation are dealt to different wavefronts;
+//  * a workgroup of eight wavefronts takes HW of a unit's G heads (grid: units x G / HW); wavefront w
+//    owns tokens 8w .. 8w + 7 of every chunk of 64.  Both rows of a token are split over the same
+//    eight lanes (16-byte loads, 128 contiguous bytes per token and instruction), and every group of
+//    eight lanes keeps an online-softmax state of its own for each head, so the token loop exchanges
+//    nothing between tokens (a sum inside the eight lanes is all) and has no barrier; the next chunk is
+//    requested as soon as the registers are free, the other wavefronts work meanwhile (a second
+//    register set changed nothing at 700 tokens and took a resident workgroup);
+//  * the 64 lane-group states and the zones A+B state are combined once, in a fixed order.
 // The step's own token never comes back through memory: its rotated key and its value are kept
 // in LDS and stand in for whatever the row's loads returned.
+//
+// The token loop is bound by its vector instructions on one compute unit, which is why a step of few
+// units is spread over its heads (HW = 1): nothing ties the heads together unless the block scores
+// of blockwise decode are summed over them.  The workgroups of a unit are n_units apart in launch
+// order, which for the usual multiples of eight puts them on one die, whose L2 serves the repeats.
 constexpr int kZcChunk = 64;
 constexpr int kZcWaves = 8;
 constexpr int kZcInlineUnits = 16;
+constexpr int kZcWorkgroups = 256;
 // The new token's un-rotated key and value rows (k == nullptr: nothing to append).
 struct ZcAppend {
   const void *k, *v;
@@ -1071,15 +1077,6 @@ __device__ __forceinline__ float zc_tokens_reduce(float v) {
   auto t = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   return op(__builtin_bit_cast(float, (unsigned)t[0]), __builtin_bit_cast(float, (unsigned)t[1]));
 }
-// Maximum / sum over all 64 lanes, the same bits in every lane.
-template <bool MAX>
-__device__ __forceinline__ float zc_wave_reduce(float v) {
-  auto op = [](float a, float b) { return MAX ? fmaxf(a, b) : a + b; };
-  v = op(v, rdkv_dpp_mov<0xB1>(v));    // quad_perm [1,0,3,2]
-  v = op(v, rdkv_dpp_mov<0x4E>(v));    // quad_perm [2,3,0,1]
-  v = op(v, rdkv_dpp_mov<0x141>(v));   // row_half_mirror
-  return zc_tokens_reduce<MAX>(v);
-}
 // Sum over the eight lanes that share (lane >> 3), the same bits in each of them (exchanges at
 // distance 1 and 2 inside a quad, then a mirror inside the eight lanes).
 __device__ __forceinline__ float zc_oct_sum(float v) {
@@ -1088,12 +1085,36 @@ __device__ __forceinline__ float zc_oct_sum(float v) {
   return v + rdkv_dpp_mov<0x141>(v);   // row_half_mirror
 }
 
-// G is a template parameter: the per-head loops unroll into straight-line code (with a run-time
-// G every head of every token is a scalar branch).
+// The sum over the eight lane groups of a lane's sixteen channels v[j] (the channels 32 j + 4 kc ..),
+// four of which a lane keeps: the two rows of a half exchange half of their values each and add what
+// they hold twice, then the two halves, then the two groups of a row.  Lanes of row r = lane >> 4
+// return the four channels of j = 2 (r & 1) + (r >> 1).  (Every lane summing all sixteen took three
+// times the instructions: 1.7 us of the launch at four heads.)
+__device__ __forceinline__ floatx4 zc_groups_sum(const floatx4 (&v)[4]) {
+  float a[8], b[4];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, (float)v[i >> 2][i & 3]),
+                                              __builtin_bit_cast(unsigned, (float)v[2 + (i >> 2)][i & 3]), false, false);
+    a[i] = __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a[i]), __builtin_bit_cast(unsigned, a[4 + i]),
+                                              false, false);
+    b[i] = __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+    b[i] += rdkv_dpp_mov<0x128>(b[i]);   // row_ror:8 - the other group of a row of 16 lanes
+  }
+  return floatx4{b[0], b[1], b[2], b[3]};
+}
+
+// HW, the heads of a workgroup, is a template parameter: the per-head loops unroll into
+// straight-line code (with a run-time count every head of every token is a scalar branch).  Every
+// head's arithmetic is written out in the same operations and order whatever HW is: the same bits.
 // INLINE: the units' merge fields come with the kernel arguments (iu), not from the table.
-template <int G, bool INLINE>
-__global__ void __launch_bounds__(64 * kZcWaves)
-merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float *__restrict__ partials,
+template <int HW, bool INLINE>
+__global__ void __launch_bounds__(64 * kZcWaves) __attribute__((amdgpu_waves_per_eu(HW <= 2 ? 4 : 2)))
+merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float *__restrict__ partials, int G,
                     const void *__restrict__ q, int q_dtype, int64_t q_stride,
                     const void *__restrict__ rope_cos, const void *__restrict__ rope_sin, int rope_dtype,
                     float *k_new, float *v_new, int64_t new_stride_unit,   // written when a row is appended
@@ -1102,16 +1123,18 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
                     float *zc_w, int64_t zc_w_stride, ZcAppend ap, void *__restrict__ q_rot_out,
                     int64_t q_rot_stride, RdkvTailScores ts) {
   constexpr int kThreads = 64 * kZcWaves;
-  constexpr int kCols = (G * kD + kThreads - 1) / kThreads;   // output columns per thread
+  constexpr int kCols = (HW * kD + kThreads - 1) / kThreads;  // output columns per thread
   constexpr int kAhead = kMergeAhead;                         // partials whose accumulators are requested at once
+  constexpr int kOwnWave = kZcWaves - 1;                      // takes the step's own token
   __shared__ __align__(16) float scratch[kMergeScratchFloats]; // the merge of zones A+B (see merge_unit)
-  __shared__ __align__(16) float qz[8][kD];                   // q * log2(e) / sqrt(D)
+  __shared__ __align__(16) float qz[HW][kD];                  // q * log2(e) / sqrt(D)
   __shared__ __align__(16) float k_self[kD], v_self[kD];      // the step's own token (rotated key, value)
-  __shared__ float w_m[kZcWaves][8], w_l[kZcWaves][8];        // every wavefront's zone C softmax state ...
-  __shared__ __align__(8) float w_acc[kZcWaves][8][kD];       // ... and its share of sum weight x V
-  __shared__ float fin_m[8], fin_l[8];                        // softmax maximum and sum over the union, per head
+  __shared__ float w_m[kZcWaves][HW], w_l[kZcWaves][HW];      // every wavefront's zone C softmax state ...
+  __shared__ __align__(16) float w_acc[kZcWaves][HW][kD];     // ... and its share of sum weight x V
+  __shared__ float fin_m[HW], fin_l[HW];                      // softmax maximum and sum over the union, per head
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int head0 = blockIdx.y * HW;
 
   // ---- the unit: from the kernel arguments, or the first round trip ------------------------------
   int work_count, q_row, work_begin;
@@ -1127,6 +1150,7 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
   }
   if (work_count == 0) return;  // a further source of an output row: merged by the row's first unit
   const int kv_row = q_row / G;    // zone-C tensors are indexed by output (group, KV head)
+  q_row += head0;
 
   // ---- one round trip: everything else, requested before anything is used ------------------------
   // The zone-C row of this step (device-held, so that a replayed graph needs nothing from the host)
@@ -1138,11 +1162,11 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
   const int32_t *cnt_ptr = (n_new_per_unit ? n_new_per_unit + kv_row : reinterpret_cast<const int32_t *>(units)) + lane_zero;
   const int64_t step_row_v = *row_ptr;
   const int32_t n_new_v = *cnt_ptr;
-  // (a) the step's own key / value row and its rotation angles (first wavefront): lane l takes
+  // (a) the step's own key / value row and its rotation angles (one wavefront): lane l takes
   // channels l and l + 64
   uint32_t a_raw[6] = {0u, 0u, 0u, 0u, 0u, 0u};
   const int64_t a_ko = (int64_t)kv_row * ap.k_stride_h, a_vo = (int64_t)kv_row * ap.v_stride_h;
-  if (ap.k && wave == 0) {
+  if (ap.k && wave == kOwnWave) {
     a_raw[0] = rdkv_load_dword_of(ap.k, ap.dtype, a_ko + lane);
     a_raw[1] = rdkv_load_dword_of(ap.k, ap.dtype, a_ko + lane + 64);
     a_raw[2] = rdkv_load_dword_of(ap.v, ap.dtype, a_vo + lane);
@@ -1157,80 +1181,75 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
 #pragma unroll
   for (int j = 0; j < kCols; ++j) {
     const int i = tid + j * kThreads;
-    const int ic = i < G * kD ? i : 0;
-    const int c = ic & 127;
-    const int64_t row = (int64_t)(q_row + (ic >> 7)) * q_stride;
-    q_raw[j][0] = rdkv_load_dword_of(q, q_dtype, row + c);
-    q_raw[j][1] = q_raw[j][2] = q_raw[j][3] = 0u;
-    if (rope_cos) {
-      q_raw[j][1] = rdkv_load_dword_of(q, q_dtype, row + (c ^ 64));
-      q_raw[j][2] = rdkv_load_dword_of(rope_cos, rope_dtype, c & 63);
-      q_raw[j][3] = rdkv_load_dword_of(rope_sin, rope_dtype, c & 63);
+    q_raw[j][0] = q_raw[j][1] = q_raw[j][2] = q_raw[j][3] = 0u;
+    if (i < HW * kD) {                   // uniform
+      const int c = i & 127;
+      const int64_t row = (int64_t)(q_row + (i >> 7)) * q_stride;
+      q_raw[j][0] = rdkv_load_dword_of(q, q_dtype, row + c);
+      if (rope_cos) {
+        q_raw[j][1] = rdkv_load_dword_of(q, q_dtype, row + (c ^ 64));
+        q_raw[j][2] = rdkv_load_dword_of(rope_cos, rope_dtype, c & 63);
+        q_raw[j][3] = rdkv_load_dword_of(rope_sin, rope_dtype, c & 63);
+      }
     }
   }
-  // (c) the partials: max / sum columns (thread i takes partial i / G, head i % G), then the first
+  // (c) the partials: max / sum columns (a wavefront per head, lane = partial), then the first
   // kAhead accumulator values of each of the thread's output columns, eight partials at a time
   const int n_part = work_count;
   const int64_t pstride = (int64_t)G * kPartialStride;
-  const float *base0 = partials + (int64_t)work_begin * pstride;
+  const float *base0 = partials + (int64_t)work_begin * pstride + (int64_t)head0 * kPartialStride;
   const bool staged = n_part <= kMergeMaxK;        // the max / sum columns fit in LDS (else: plain loops)
-  constexpr int kMl = (kMergeMaxK * G + kThreads - 1) / kThreads;
+  const int f_head = (wave - 2 * HW) & (kZcWaves - 1);     // (of few heads: not the wavefronts of (b))
+  constexpr int kMl = kMergeMaxK / 64;
   float pm[kMl], pl[kMl];
 #pragma unroll
   for (int j = 0; j < kMl; ++j) {
+    const int k = lane + 64 * j;
     pm[j] = pl[j] = 0.0f;
-    if (j * kThreads < n_part * G) {      // uniform: later batches only for units with many partials
-      const int i = tid + j * kThreads;
-      const int ic = (staged && i < n_part * G) ? i : 0;
-      const int k = ic / G, h = ic - k * G;
-      pm[j] = base0[k * pstride + h * kPartialStride + 128];
-      pl[j] = base0[k * pstride + h * kPartialStride + 129];
+    if (staged && f_head < HW && k < n_part) {
+      pm[j] = base0[k * pstride + f_head * kPartialStride + 128];
+      pl[j] = base0[k * pstride + f_head * kPartialStride + 129];
     }
   }
   float ahead[kCols][kAhead];
 #pragma unroll
   for (int j = 0; j < kCols; ++j) {
     const int i = tid + j * kThreads;
-    const int ic = i < G * kD ? i : 0;
-    const float *b0 = base0 + (ic >> 7) * kPartialStride + (ic & 127);
+    const float *b0 = base0 + (i >> 7) * kPartialStride + (i & 127);
 #pragma unroll
     for (int e0 = 0; e0 < kAhead; e0 += 8) {
 #pragma unroll
       for (int e = e0; e < e0 + 8; ++e) ahead[j][e] = 0.0f;
-      if (e0 < n_part) {                  // uniform
+      if (e0 < n_part && i < HW * kD) {   // uniform
 #pragma unroll
         for (int e = e0; e < e0 + 8; ++e) ahead[j][e] = b0[(e < n_part ? e : 0) * pstride];
       }
     }
   }
-  // (d) the first chunk of zone C.  K: token 8 * wave + lane / 8, sixteen of its channels (four
-  // 16-byte pieces, piece j of lane group member c being floats 32j + 4c ..); V: tokens 8 * wave + i,
-  // channels 2 * lane and 2 * lane + 1.  Rows are requested up to the buffer's last row.
+  // (d) the first chunk of zone C: lane group tg holds a token, its lane kc the channels 32 j + 4 kc
+  // .. + 3 of both rows.  Rows are requested up to the buffer's last row.
   const int tg = lane >> 3, kc = lane & 7;
   const float *kn = k_new + (int64_t)kv_row * new_stride_unit;
   const float *vn = v_new + (int64_t)kv_row * new_stride_unit;
   const int last_row = n_new_all > 0 ? n_new_all - 1 : 0;
   const bool have_rows = n_new_all > 0 && k_new != nullptr;
-  float4 kreg[4];
-  float2 vreg[8];
-  auto request_chunk = [&](int t0) __attribute__((always_inline)) {
-    const int tw = t0 + 8 * wave;
-    if (!have_rows || tw > last_row) return;     // uniform
-    const int tr = tw + tg < last_row ? tw + tg : last_row;
-    const float4 *kr = reinterpret_cast<const float4 *>(kn + (int64_t)tr * new_stride_tok);
+  typedef floatx4 __attribute__((aligned(4))) floatx4_a4;   // only the key rows' alignment is required of a caller
+  struct Rows { floatx4 k[4], v[4]; };
+  auto request = [&](Rows &r, int base) __attribute__((always_inline)) {
+    const int tr = base + tg < last_row ? base + tg : last_row;
+    const floatx4 *kr = reinterpret_cast<const floatx4 *>(kn + (int64_t)tr * new_stride_tok);
+    const floatx4_a4 *vr = reinterpret_cast<const floatx4_a4 *>(vn + (int64_t)tr * new_stride_tok);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) kreg[j] = kr[8 * j + kc];
+    for (int j = 0; j < 4; ++j) r.k[j] = kr[8 * j + kc];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int tvr = tw + i < last_row ? tw + i : last_row;
-      vreg[i] = reinterpret_cast<const float2 *>(vn + (int64_t)tvr * new_stride_tok)[lane];
-    }
+    for (int j = 0; j < 4; ++j) r.v[j] = vr[8 * j + kc];
   };
+  const floatx4 zero4 = {0.f, 0.f, 0.f, 0.f};
+  const int first = 8 * wave;                      // this wavefront's tokens: first + tg, + kZcChunk, ...
+  Rows rows;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) kreg[j] = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) vreg[i] = make_float2(0.f, 0.f);
-  request_chunk(0);
+  for (int j = 0; j < 4; ++j) rows.k[j] = rows.v[j] = zero4;
+  if (have_rows && first <= last_row) request(rows, first);
   const int64_t step_row = ap.k ? (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(step_row_v >> 32)) << 32) |
                                             (uint32_t)__builtin_amdgcn_readfirstlane((int)step_row_v))
                                 : -1;
@@ -1239,10 +1258,11 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
   n_new = n_new > 0 ? n_new : 0;
   const bool appending = ap.k != nullptr && step_row >= 0 && step_row < ap.capacity;
 
-  // ---- the step's own token joins zone C (first wavefront) --------------------------------------
+  // ---- the step's own token joins zone C (one wavefront) ------------------------------------------
   // k rotated and rounded to its storage type as the in-place rotation stores it, k and v widened
-  // to fp32; the row goes to memory for the steps to come and to LDS for this one.
-  if (ap.k && wave == 0) {
+  // to fp32; the row goes to LDS for this step and to memory for the steps to come (by the workgroup
+  // of the first head; what the others' loads of that row return is discarded).
+  if (ap.k && wave == kOwnWave) {
     const float k_lo = rdkv_decode_dword(a_raw[0], ap.k, ap.dtype, a_ko + lane);
     const float k_hi = rdkv_decode_dword(a_raw[1], ap.k, ap.dtype, a_ko + lane + 64);
     const float v_lo = rdkv_decode_dword(a_raw[2], ap.v, ap.dtype, a_vo + lane);
@@ -1259,7 +1279,7 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
     k_self[lane + 64] = out_hi;
     v_self[lane] = v_lo;
     v_self[lane + 64] = v_hi;
-    if (appending) {
+    if (appending && head0 == 0) {
       const int64_t off = (int64_t)kv_row * new_stride_unit + step_row * new_stride_tok;
       float *kd = k_new + off, *vd = v_new + off;
       kd[lane] = out_lo;
@@ -1274,7 +1294,7 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
 #pragma unroll
   for (int j = 0; j < kCols; ++j) {
     const int i = tid + j * kThreads;
-    if (i < G * kD) {
+    if (i < HW * kD) {
       const int c = i & 127;
       const int64_t row = (int64_t)(q_row + (i >> 7)) * q_stride;
       float v = rdkv_decode_dword(q_raw[j][0], q, q_dtype, row + c);
@@ -1297,123 +1317,131 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
                                   (ts.q_rotated_stride_tok ? step_row * ts.q_rotated_stride_tok : 0) + c, v);
     }
   }
-  // ---- the partials' max / sum columns ----------------------------------------------------------
-  if (staged) {
+  // ---- zones A+B: the softmax factors of the unit's partials, once per (partial, head) (stages 1 and
+  // 2 of the merge; a lane reads back the columns it wrote itself)
+  if (staged && f_head < HW) {
 #pragma unroll
     for (int j = 0; j < kMl; ++j) {
-      const int i = tid + j * kThreads;
-      if (i < n_part * G) {
-        const int k = i / G, h = i - k * G;
-        scratch[kMergeM + k * 8 + h] = pm[j];
-        scratch[kMergeL + k * 8 + h] = pl[j];
+      const int k = lane + 64 * j;
+      if (k < n_part) {
+        scratch[kMergeM + k * 8 + f_head] = pm[j];
+        scratch[kMergeL + k * 8 + f_head] = pl[j];
+      }
+    }
+    merge_factors(n_part, HW, f_head, lane, kZcWaves, scratch);
+  }
+  __syncthreads();   // qz, k_self / v_self, the factors
+
+  // ---- zones A+B: this thread's columns of the partials under their factors, normalized (stage 3 of
+  // the merge; ahead of the token loop, whose registers the requested values would otherwise add to)
+  float o_ab[kCols], mab[kCols];
+#pragma unroll
+  for (int j = 0; j < kCols; ++j) {
+    const int i = tid + j * kThreads, h = i >> 7;
+    o_ab[j] = 0.0f;
+    mab[j] = -INFINITY;
+    if (i < HW * kD) {
+      const float *base = base0 + h * kPartialStride;
+      if (staged) {
+        o_ab[j] = merge_column<false>(n_part, h, ahead[j], base + (i & 127), pstride, scratch);
+        mab[j] = scratch[kMergeL2 + h];
+      } else {
+        o_ab[j] = merge_column_long<false>(n_part, base, i & 127, pstride, mab[j]);
       }
     }
   }
-  __syncthreads();   // qz, k_self / v_self, s_m / s_l
 
-  // ---- zones A+B: the softmax factors of the unit's partials, once per (partial, head) ------------
-  // (stage 2 of the merge; the accumulator columns are weighted with these factors after the token
-  // loop, behind the barrier that ends it)
-  if (staged) merge_factors(n_part, G, wave, lane, kZcWaves, scratch);
-
-  // ---- zone C, 64 tokens at a time, eight per wavefront ------------------------------------------
-  float m_run[G], l_run[G], acc[G][2];
+  // ---- zone C, 64 tokens at a time, eight per wavefront, one per lane group ------------------------
+  float m_run[HW], l_run[HW];
+  floatx4 acc[HW][4], q_own[4];
 #pragma unroll
-  for (int h = 0; h < G; ++h) {
+  for (int h = 0; h < HW; ++h) {
     m_run[h] = -INFINITY;
     l_run[h] = 0.0f;
-    acc[h][0] = acc[h][1] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[h][j] = zero4;
   }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) q_own[j] = reinterpret_cast<const floatx4 *>(qz[0])[8 * j + kc];
   const int self_tok = appending ? (int)step_row : -1;
-  const float2 v_own = reinterpret_cast<const float2 *>(v_self)[lane];
-  for (int t0 = 0; t0 + 8 * wave < n_new; t0 += kZcChunk) {
-    const int tw = t0 + 8 * wave;                 // this wavefront's first token of the chunk: exists
-    // this chunk's rows, the step's own token from LDS; then the next chunk's rows are requested
-    float4 kcur[4];
-    float2 vcur[8];
-    const bool k_is_self = tw + tg == self_tok;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float4 ks = reinterpret_cast<const float4 *>(k_self)[8 * j + kc];
-      kcur[j] = k_is_self ? ks : kreg[j];
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      vcur[i] = tw + i == self_tok ? v_own : vreg[i];
-      if (tw + i >= n_new) vcur[i] = make_float2(0.f, 0.f);     // a row past the count may hold anything
-    }
-    if (tw + kZcChunk < n_new) request_chunk(t0 + kZcChunk);
-    // scores of this lane group's token against the G query heads: sixteen channels per lane
-    const bool tok_valid = tw + tg < n_new;
-    float wt[G];
-#pragma unroll
-    for (int h = 0; h < G; ++h) {
-      float a = 0.0f;
+  auto consume = [&](Rows &r, int base) __attribute__((always_inline)) {
+    const int t = base + tg;
+    if (self_tok >= base && self_tok < base + 8) {      // uniform: the tokens with the step's own
+      const bool is_self = t == self_tok;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float4 qq = reinterpret_cast<const float4 *>(qz[h])[8 * j + kc];
-        a += kcur[j].x * qq.x + kcur[j].y * qq.y + kcur[j].z * qq.z + kcur[j].w * qq.w;
+        const floatx4 ks = reinterpret_cast<const floatx4 *>(k_self)[8 * j + kc];
+        const floatx4 vs = reinterpret_cast<const floatx4 *>(v_self)[8 * j + kc];
+        r.k[j] = is_self ? ks : r.k[j];
+        r.v[j] = is_self ? vs : r.v[j];
       }
-      const float sh = tok_valid ? zc_oct_sum(a) : -INFINITY;
+    }
+    if (t >= n_new) return;                             // a row past the count may hold anything
+#pragma unroll
+    for (int h = 0; h < HW; ++h) {
+      float a[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const floatx4 qq = h == 0 ? q_own[j] : reinterpret_cast<const floatx4 *>(qz[h])[8 * j + kc];
+        a[j] = fmaf(r.k[j].w, qq.w, fmaf(r.k[j].z, qq.z, fmaf(r.k[j].y, qq.y, r.k[j].x * qq.x)));
+      }
+      const float s = zc_oct_sum((a[0] + a[1]) + (a[2] + a[3]));
       // raw scores now, turned into weights once the union's maximum and sum are known
-      if (zc_w && kc == 0 && tok_valid) zc_w[(int64_t)(q_row + h) * zc_w_stride + tw + tg] = sh;
-      const float m_new = fmaxf(m_run[h], zc_tokens_reduce<true>(sh));    // finite: token tw exists
-      const float f = fast_exp2(m_run[h] - m_new);                         // 0 on the first chunk
-      wt[h] = fast_exp2(sh - m_new);                                       // 0 for a token past the count
-      l_run[h] = l_run[h] * f + zc_tokens_reduce<false>(wt[h]);
-      acc[h][0] *= f;
-      acc[h][1] *= f;
+      if (zc_w && kc == 0) zc_w[(int64_t)(q_row + h) * zc_w_stride + t] = s;
+      const float m_new = fmaxf(m_run[h], s);
+      const float ref = m_new == -INFINITY ? 0.0f : m_new;        // scores of -inf so far: weights of zero
+      const float f = fast_exp2(m_run[h] - ref), w = fast_exp2(s - ref);
+      l_run[h] = fmaf(l_run[h], f, w);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        acc[h][j].x = fmaf(w, r.v[j].x, acc[h][j].x * f);
+        acc[h][j].y = fmaf(w, r.v[j].y, acc[h][j].y * f);
+        acc[h][j].z = fmaf(w, r.v[j].z, acc[h][j].z * f);
+        acc[h][j].w = fmaf(w, r.v[j].w, acc[h][j].w * f);
+      }
       m_run[h] = m_new;
     }
-    // values: token tw + i, its weight read from the first lane of its group
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-#pragma unroll
-      for (int h = 0; h < G; ++h) {
-        const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wt[h]), 8 * i));
-        acc[h][0] += w * vcur[i].x;
-        acc[h][1] += w * vcur[i].y;
-      }
-    }
+  };
+  for (int base = first; base < n_new; base += kZcChunk) {
+    consume(rows, base);
+    if (base + kZcChunk < n_new) request(rows, base + kZcChunk);
   }
+  // the eight states of the wavefront (one without tokens says so by its maximum)
 #pragma unroll
-  for (int h = 0; h < G; ++h) {
-    if (lane == 0) {
-      w_m[wave][h] = m_run[h];
-      w_l[wave][h] = l_run[h];
+  for (int h = 0; h < HW; ++h) {
+    float M = -INFINITY, l = 0.0f;
+    if (first < n_new) {       // uniform
+      M = zc_tokens_reduce<true>(m_run[h]);
+      const float f = m_run[h] == -INFINITY ? 0.0f : fast_exp2(m_run[h] - M);
+      l = zc_tokens_reduce<false>(l_run[h] * f);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[h][j] *= f;
+      const floatx4 sum = zc_groups_sum(acc[h]);
+      if ((lane & 8) == 0) reinterpret_cast<floatx4 *>(w_acc[wave][h])[8 * (2 * (tg >> 1 & 1) + (tg >> 2)) + kc] = sum;
     }
-    reinterpret_cast<float2 *>(w_acc[wave][h])[lane] = make_float2(acc[h][0], acc[h][1]);
+    if (lane == 0) {
+      w_m[wave][h] = M;
+      w_l[wave][h] = l;
+    }
   }
   __syncthreads();
   // ---- the union: zones A+B as one pseudo-token, the eight wavefront states of zone C ------------
 #pragma unroll
   for (int j = 0; j < kCols; ++j) {
     const int i = tid + j * kThreads;
-    if (i < G * kD) {
+    if (i < HW * kD) {
       const int h = i >> 7, d = i & 127;
-      // zones A+B: this column of the partials under their factors, normalized (stage 3 of the merge)
-      float o_ab, mab;
-      if (staged) {
-        o_ab = merge_column<false>(n_part, h, ahead[j], base0 + h * kPartialStride + d, pstride, scratch);
-        mab = scratch[kMergeL2 + h];
-      } else {
-        o_ab = merge_column_long<false>(n_part, base0 + h * kPartialStride, d, pstride, mab);
-      }
-      float M = mab;
+      float M = mab[j];
 #pragma unroll
       for (int w = 0; w < kZcWaves; ++w) M = fmaxf(M, w_m[w][h]);
-      float o = 0.0f, l = 0.0f;
-      {
-        const float f = mab == -INFINITY ? 0.0f : fast_exp2(mab - M);
-        o = f * o_ab;
-        l = f;
-      }
+      const float fab = mab[j] == -INFINITY ? 0.0f : fast_exp2(mab[j] - M);
+      float o = fab * o_ab[j], l = fab;
 #pragma unroll
       for (int w = 0; w < kZcWaves; ++w) {
-        const float mw = w_m[w][h];
+        const float mw = w_m[w][h], aw = w_acc[w][h][d];
         const float f = mw == -INFINITY ? 0.0f : fast_exp2(mw - M);
-        o += f * w_acc[w][h][d];
-        l += f * w_l[w][h];
+        o = fmaf(f, mw == -INFINITY ? 0.0f : aw, o);      // (nothing was written for it)
+        l = fmaf(f, w_l[w][h], l);
       }
       out[(int64_t)(q_row + h) * out_stride + d] = l > 0.0f ? o / l : 0.0f;
       if (lse && d == 0) lse[q_row + h] = l > 0.0f ? (M + log2f(l)) * kLn2 : -INFINITY;
@@ -1426,12 +1454,12 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
   if (zc_w) {   // softmax weights of the zone C tokens over the union (fast_decode.py:1753-1755 w_new)
     __syncthreads();
     for (int t = tid; t < n_new; t += kThreads) {
-      // everything this token needs is requested first (the raw scores of the G heads, the two block
+      // everything this token needs is requested first (the raw scores of the heads, the two block
       // scores it adds to): stores to one row may not be moved past loads of another by the compiler,
       // which made this a chain of G + 2 round trips
-      float raw[G];
+      float raw[HW];
 #pragma unroll
-      for (int h = 0; h < G; ++h) raw[h] = zc_w[(int64_t)(q_row + h) * zc_w_stride + t];
+      for (int h = 0; h < HW; ++h) raw[h] = zc_w[(int64_t)(q_row + h) * zc_w_stride + t];
       // online block scores of blockwise decode (blockwise_decode.py:2085-2109): the query's weights
       // on its own block, and on the first block when the query belongs to the second
       const bool to_self = ts.self_scores && t >= q_block_start;
@@ -1442,7 +1470,7 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
       const float next_old = to_next ? *next_at : 0.0f;
       float s = 0.0f;     // over the group's heads in head order, as rdkv_tail_scores sums them
 #pragma unroll
-      for (int h = 0; h < G; ++h) {
+      for (int h = 0; h < HW; ++h) {
 #pragma clang fp contract(off)   // the stored weight is what is summed: no fusing with the product
         const float inv = fin_l[h] > 0.0f ? 1.0f / fin_l[h] : 0.0f;
         const float w = fast_exp2(raw[h] - fin_m[h]) * inv;
@@ -1454,7 +1482,6 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
     }
   }
 }
-
 }  // namespace
 
 RDKV_API int64_t rdkv_decode_fused_workspace_bytes(int n_work, int G) {
@@ -1636,18 +1663,28 @@ static int launch_merge_zone_c(const char *fn, const RdkvUnit *units, const Rdkv
       iu.work_count[i] = units_host[i].work_count;
     }
   }
-#define RDKV_LAUNCH_ZC_I(GT, INL)                                                                             \
-  hipLaunchKernelGGL((merge_zone_c_kernel<GT, INL>), dim3(n_units), dim3(64 * kZcWaves), 0, (hipStream_t)stream, \
-                     units, iu, (const float *)workspace, q, q_dtype, q_stride_row, rope_cos, rope_sin,         \
-                     rope_dtype, const_cast<float *>(k_new), const_cast<float *>(v_new), new_stride_unit,       \
-                     new_stride_tok, n_new, n_new_per_unit, out, out_stride_row, lse, zone_c_weights,           \
-                     zone_c_weights_stride_row, append, q_rot_out, q_rot_stride, tail)
-#define RDKV_LAUNCH_ZC(GT)                  \
+  // Heads per workgroup (any choice gives the same bits).  All of them where the block scores are
+  // summed over the heads.  One while that leaves a compute unit per workgroup (a device has 256);
+  // beyond, where workgroups share a compute unit and their preparation counts, two.  Measured, one
+  // / two / four heads, G = 4: 8 units with 17 and 700 tokens 22.7 / 23.5 / 25.1 and 26.9 / 29.1 /
+  // 36.6 us per step (32k prompt), 128 units with 300 tokens 31.0 / 29.0 / 31.0, 384 units 73 / 58 / 60.
+  int hw = G;
+  if (!tail.self_scores) {
+    if ((int64_t)n_units * G <= kZcWorkgroups) hw = 1;
+    else if (G % 2 == 0) hw = 2;
+  }
+#define RDKV_LAUNCH_ZC_I(HW, INL)                                                                             \
+  hipLaunchKernelGGL((merge_zone_c_kernel<HW, INL>), dim3(n_units, G / HW), dim3(64 * kZcWaves), 0,             \
+                     (hipStream_t)stream, units, iu, (const float *)workspace, G, q, q_dtype, q_stride_row,     \
+                     rope_cos, rope_sin, rope_dtype, const_cast<float *>(k_new), const_cast<float *>(v_new),    \
+                     new_stride_unit, new_stride_tok, n_new, n_new_per_unit, out, out_stride_row, lse,          \
+                     zone_c_weights, zone_c_weights_stride_row, append, q_rot_out, q_rot_stride, tail)
+#define RDKV_LAUNCH_ZC(HW)                  \
   do {                                      \
-    if (iu.n > 0) RDKV_LAUNCH_ZC_I(GT, true); \
-    else RDKV_LAUNCH_ZC_I(GT, false);       \
+    if (iu.n > 0) RDKV_LAUNCH_ZC_I(HW, true); \
+    else RDKV_LAUNCH_ZC_I(HW, false);       \
   } while (0)
-  switch (G) {
+  switch (hw) {
     case 1: RDKV_LAUNCH_ZC(1); break;
     case 2: RDKV_LAUNCH_ZC(2); break;
     case 3: RDKV_LAUNCH_ZC(3); break;
