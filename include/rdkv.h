@@ -183,6 +183,16 @@ int rdkv_softmax_rows_ws(const float *scores_old, int64_t so_stride_h, const flo
                          float *w_new, int64_t wn_stride_h, int H_q, void *workspace,
                          int64_t workspace_bytes, void *stream);
 
+/* The same with the scores of the new zone formed by the launch itself (fast_decode.py:1730-1733):
+ * scores_new[hq, t] = sum_d (q[hq, d] / sqrt(128)) * k_new[hkv, t, d] in fp32, written to w_new and
+ * turned into weights there.  k_new fp32, unit last stride, rows 16-byte aligned (else RDKV_EINVAL). */
+int rdkv_softmax_rows_new_keys(const float *scores_old, int64_t so_stride_h, const float *mask,
+                               int64_t mask_stride_h, int64_t T_old, const void *q, int q_dtype,
+                               int64_t q_stride_h, const float *k_new, int64_t kn_stride_h,
+                               int64_t kn_stride_t, int64_t n_new, float *w_old, int64_t wo_stride_h,
+                               float *w_new, int64_t wn_stride_h, int H_q, int H_kv, void *workspace,
+                               int64_t workspace_bytes, void *stream);
+
 /* ---- triton_v_kernel.py : v_dequant_weighted_sum_dispatch_into (:1729-1760) */
 /* out[hq,d] = sum over 2/4/8-bit segments of w*(code-zp)*scale + fp16 zone B
  * (kernel math triton_v_kernel.py:638-750).  seg_bounds_dev: int32 [H_kv,3] per-head
@@ -202,6 +212,18 @@ int rdkv_v_weighted_sum(const float *w, int64_t w_stride_h, int H_q, int H_kv,
                         int64_t max_T_v,
                         float *out, int64_t out_stride_h,
                         void *workspace, int64_t workspace_bytes, void *stream);
+
+/* The same plus the new zone (fast_decode.py:1780-1784): out[hq] += sum over t < n_new of
+ * w_new[hq, t] * v_new[hkv, t, :].  v_new fp32, unit last stride, rows 16-byte aligned (else RDKV_EINVAL). */
+int rdkv_v_weighted_sum_new_values(const float *w, int64_t w_stride_h, int H_q, int H_kv, const uint8_t *V2,
+                                   int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h,
+                                   const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16,
+                                   const void *zp_f16, int64_t vs_stride_h, const int32_t *seg_bounds_dev,
+                                   int N2, int N4, int N8, const void *V16_f16, int64_t v16_stride_h,
+                                   const int32_t *n_v16_dev, int64_t max_T_v, const float *w_new,
+                                   int64_t wn_stride_h, const float *v_new, int64_t vn_stride_h,
+                                   int64_t vn_stride_t, int64_t n_new, float *out, int64_t out_stride_h,
+                                   void *workspace, int64_t workspace_bytes, void *stream);
 
 /* ---- fast_decode.py : the per-token operations around the attention ------- */
 /* fast_decode.py:628-633 (_rms_norm) with the residual add in front of it (:1786, :1808):

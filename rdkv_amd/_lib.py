@@ -60,8 +60,11 @@ SIGNATURES = {
     "rdkv_softmax_rows": (I, [P, L, P, L, L, P, L, L, P, L, P, L, I, P]),
     "rdkv_softmax_rows_workspace_bytes": (L, [I]),
     "rdkv_softmax_rows_ws": (I, [P, L, P, L, L, P, L, L, P, L, P, L, I, P, L, P]),
+    "rdkv_softmax_rows_new_keys": (I, [P, L, P, L, L, P, I, L, P, L, L, L, P, L, P, L, I, I, P, L, P]),
     "rdkv_v_weighted_sum_workspace_bytes": (L, [I]),
     "rdkv_v_weighted_sum": (I, [P, L, I, I, P, L, P, L, P, L, P, P, L, P, I, I, I, P, L, P, L, P, L, P, L, P]),
+    "rdkv_v_weighted_sum_new_values": (I, [P, L, I, I, P, L, P, L, P, L, P, P, L, P, I, I, I, P, L, P, L, P, L, P, L, L, L,
+                                           P, L, P, L, P]),
     "rdkv_stream_plan_layer": (I, [P, L, P, L, I, I, I, I, I, P, P, I, P]),
     "rdkv_stream_partition": (I, [P, I, I, P, ctypes.c_double, ctypes.c_double, P, I, I, P, I, P, P]),
     "rdkv_stream_work_scales": (I, [P, I, P, I]),

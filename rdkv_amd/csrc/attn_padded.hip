@@ -106,6 +106,7 @@ k_qk_dot_strided_kernel(const void *__restrict__ q, int q_dtype, int64_t q_strid
 
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef floatx4 __attribute__((aligned(4))) floatx4_a4;   // a 16-byte load from any float
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ half4_t mk_op(uint32_t a, uint32_t b) {
@@ -547,6 +548,59 @@ __global__ void zero_rows_kernel(float *out, int64_t out_sh, int64_t T) {
 // ---------------------------------------------------------------------------
 // softmax over [scores_old + mask | scores_new], one block per query head.
 // ---------------------------------------------------------------------------
+// Keys of the new zone, for a launch that forms their scores itself (k == nullptr: the scores are
+// given): k fp32 [H_kv, n_new, 128], rows 16-byte aligned; q as rdkv_k_qk_dot takes it.
+struct NewKeys {
+  const void *q;
+  int64_t q_sh;
+  int q_dtype, G;
+  const float *k;
+  int64_t k_sh, k_st;
+};
+
+// scores[t] = sum_d (q[d] / sqrt(128)) k[t][d] for the keys a .. b of query head h, by the whole workgroup:
+// eight lanes per key (sixteen channels each, 16-byte loads), two keys per lane group in flight.
+// The caller's barrier makes them visible.  (As launches of their own - the scaled query, a library
+// product, the copy into the score rows - these few hundred dot products and the weighted values took
+// 24 us of a 76 us layer and four of its ten launches; 32k layer 102 -> 51 us, 128k 115.5 -> 97.)
+__device__ __forceinline__ void new_zone_scores(const NewKeys &nk, int h, int64_t a, int64_t b, float *scores) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int tg = lane >> 3, kc = lane & 7;
+  const float *kh = nk.k + (int64_t)(h / nk.G) * nk.k_sh;
+  if (a + wave * 8 >= b) return;
+  float qv[16];
+  auto q_loads = [&](auto elem) __attribute__((always_inline)) {   // one straight run of loads per query type
+#pragma unroll
+    for (int i = 0; i < 16; ++i) qv[i] = elem(h * nk.q_sh + 32 * (i >> 2) + 4 * kc + (i & 3)) * kInvSqrtD;
+  };
+  if (nk.q_dtype == RDKV_DTYPE_F32)
+    q_loads([&](int64_t i) { return reinterpret_cast<const float *>(nk.q)[i]; });
+  else if (nk.q_dtype == RDKV_DTYPE_F16)
+    q_loads([&](int64_t i) { return __half2float(reinterpret_cast<const __half *>(nk.q)[i]); });
+  else
+    q_loads([&](int64_t i) { return __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(nk.q)[i] << 16); });
+  for (int64_t t0 = a + wave * 8 + tg; t0 < b; t0 += 16 * nw) {
+    floatx4 kr[2][4];
+    const int64_t t1 = t0 + 8 * nw < b ? t0 + 8 * nw : t0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) kr[0][j] = reinterpret_cast<const floatx4 *>(kh + t0 * nk.k_st)[8 * j + kc];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) kr[1][j] = reinterpret_cast<const floatx4 *>(kh + t1 * nk.k_st)[8 * j + kc];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      float p[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        p[j] = fmaf(kr[u][j].w, qv[4 * j + 3], fmaf(kr[u][j].z, qv[4 * j + 2], fmaf(kr[u][j].y, qv[4 * j + 1], kr[u][j].x * qv[4 * j])));
+      float v = (p[0] + p[1]) + (p[2] + p[3]);
+      v += rdkv_dpp_mov<0xB1>(v);          // quad_perm [1,0,3,2]
+      v += rdkv_dpp_mov<0x4E>(v);          // quad_perm [2,3,0,1]
+      v += rdkv_dpp_mov<0x141>(v);         // row_half_mirror: the other quad of the eight lanes
+      if (kc == 0) scores[u ? t1 : t0] = v;   // (t1 == t0 writes its score again)
+    }
+  }
+}
+
 __device__ float block_reduce(float v, bool is_max, float *scratch) {
   v = is_max ? rdkv_wave_max(v) : rdkv_wave_sum(v);
   const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -560,14 +614,18 @@ __device__ float block_reduce(float v, bool is_max, float *scratch) {
 
 __global__ void __launch_bounds__(1024)
 softmax_rows_kernel(const float *__restrict__ so, int64_t so_sh, const float *__restrict__ mask,
-                    int64_t mask_sh, int64_t T_old, const float *__restrict__ sn, int64_t sn_sh,
-                    int64_t n_new, float *__restrict__ wo, int64_t wo_sh, float *__restrict__ wn,
-                    int64_t wn_sh) {
+                    int64_t mask_sh, int64_t T_old, const float *sn, int64_t sn_sh,
+                    int64_t n_new, float *__restrict__ wo, int64_t wo_sh, float *wn,
+                    int64_t wn_sh, NewKeys nk) {
   __shared__ float scratch[16];
   const int h = blockIdx.x;
   const float *a = so ? so + h * so_sh : nullptr;
   const float *m = mask ? mask + h * mask_sh : nullptr;
   const float *b = sn ? sn + h * sn_sh : nullptr;
+  if (nk.k) {
+    new_zone_scores(nk, h, 0, n_new, wn + h * wn_sh);
+    __syncthreads();
+  }
   float mx = -INFINITY;
   for (int64_t t = threadIdx.x; t < T_old; t += blockDim.x) mx = fmaxf(mx, a[t] + (m ? m[t] : 0.0f));
   for (int64_t t = threadIdx.x; t < n_new; t += blockDim.x) mx = fmaxf(mx, b[t]);
@@ -586,38 +644,35 @@ softmax_rows_kernel(const float *__restrict__ so, int64_t so_sh, const float *__
 // and row strides 16-byte aligned): a thread keeps its share of the row in registers (NV float4:
 // rows of up to 4096 * NV scores are read once and written once; mask added on the way in), or
 // (NV = 0, longer rows) streams the row three times with 16-byte accesses.  In place is fine: a
-// thread only ever rewrites elements it has read itself.  MASK_VEC: the mask rows are 16-byte
-// aligned too; otherwise (the packer's mask rows are as long as the layer has keys, any number) the
-// four mask values of a float4 of scores are loaded one by one.
-template <int NV, bool MASK_VEC>
+// thread only ever rewrites elements it has read itself.  The mask rows are as long as the layer has
+// keys, any number, so they start at any float; they too are read 16 bytes at a time (the load only
+// needs dword alignment; a variant per alignment took the same time).
+template <int NV>
 __global__ void __launch_bounds__(1024)
 softmax_rows_vec_kernel(const float *__restrict__ so, int64_t so_sh, const float *__restrict__ mask,
-                        int64_t mask_sh, int64_t T_old, const float *__restrict__ sn, int64_t sn_sh,
-                        int64_t n_new, float *wo, int64_t wo_sh, float *wn, int64_t wn_sh) {
+                        int64_t mask_sh, int64_t T_old, const float *sn, int64_t sn_sh,
+                        int64_t n_new, float *wo, int64_t wo_sh, float *wn, int64_t wn_sh, NewKeys nk) {
   __shared__ float scratch[16];
   const int h = blockIdx.x, tid = threadIdx.x;
   const float *a = so + h * so_sh;
   const float *m = mask ? mask + h * mask_sh : nullptr;
   const float *b = sn ? sn + h * sn_sh : nullptr;
   const float4 *a4 = reinterpret_cast<const float4 *>(a);
-  const float4 *m4 = reinterpret_cast<const float4 *>(m);
+  const floatx4_a4 *m4 = reinterpret_cast<const floatx4_a4 *>(m);
   float4 *w4 = reinterpret_cast<float4 *>(wo + h * wo_sh);
   const int64_t n4 = T_old >> 2;
   constexpr int kKeep = NV > 0 ? NV : 1;
   float4 x[kKeep];
-  auto mask4 = [&](int64_t i) {
-    if (MASK_VEC) return m4[i];
-    return make_float4(m[4 * i], m[4 * i + 1], m[4 * i + 2], m[4 * i + 3]);
-  };
   auto load4 = [&](int64_t i) {
     float4 v = a4[i];
     if (m) {
-      const float4 k = mask4(i);
+      const floatx4 k = m4[i];
       v.x += k.x; v.y += k.y; v.z += k.z; v.w += k.w;
     }
     return v;
   };
   float mx = -INFINITY;
+  if (NV > 8 && nk.k) new_zone_scores(nk, h, 0, n_new, wn + h * wn_sh);   // (no registers for both)
   if (NV > 0) {
 #pragma unroll
     for (int k = 0; k < kKeep; ++k) {
@@ -625,6 +680,7 @@ softmax_rows_vec_kernel(const float *__restrict__ so, int64_t so_sh, const float
       x[k] = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
       if (i < n4) x[k] = a4[i];
     }
+    if (NV <= 8 && nk.k) new_zone_scores(nk, h, 0, n_new, wn + h * wn_sh);   // (behind the row's requests)
     if (m && n4 > 0) {
       // The mask values of eight float4s are requested together and none of the loads is conditional
       // (a slot past the row reads the row's first float4 and drops it): with the load inside the
@@ -633,11 +689,11 @@ softmax_rows_vec_kernel(const float *__restrict__ so, int64_t so_sh, const float
       constexpr int kB = kKeep < 8 ? kKeep : 8;
 #pragma unroll
       for (int k0 = 0; k0 < kKeep; k0 += kB) {
-        float4 mk[kB];
+        floatx4 mk[kB];
 #pragma unroll
         for (int j = 0; j < kB; ++j) {
           const int64_t i = tid + (int64_t)(k0 + j) * 1024;
-          mk[j] = mask4(i < n4 ? i : 0);
+          mk[j] = m4[i < n4 ? i : 0];
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -652,11 +708,13 @@ softmax_rows_vec_kernel(const float *__restrict__ so, int64_t so_sh, const float
 #pragma unroll
     for (int k = 0; k < kKeep; ++k) mx = fmaxf(fmaxf(mx, fmaxf(x[k].x, x[k].y)), fmaxf(x[k].z, x[k].w));
   } else {
+    if (nk.k) new_zone_scores(nk, h, 0, n_new, wn + h * wn_sh);
     for (int64_t i = tid; i < n4; i += 1024) {
       const float4 v = load4(i);
       mx = fmaxf(fmaxf(mx, fmaxf(v.x, v.y)), fmaxf(v.z, v.w));
     }
   }
+  if (nk.k) __syncthreads();
   // the last T_old % 4 scores and the new zone, element by element
   for (int64_t t = 4 * n4 + tid; t < T_old; t += 1024) mx = fmaxf(mx, a[t] + (m ? m[t] : 0.0f));
   for (int64_t t = tid; t < n_new; t += 1024) mx = fmaxf(mx, b[t]);
@@ -703,28 +761,30 @@ softmax_rows_vec_kernel(const float *__restrict__ so, int64_t so_sh, const float
 // of few heads (one workgroup per head leaves most compute units idle): the first launch leaves
 // every piece's maximum and its sum of exp(x - maximum) in the workspace, the second combines
 // the S pairs of its row in index order (every workgroup the same arithmetic) and writes the
-// weights of its piece.  A piece is at most 4096 float4s, held in registers within a launch; the
-// last piece also takes the last T_old % 4 scores and the new zone.  Same alignment conditions as
+// weights of its piece.  A piece is at most 4096 float4s, held in registers within a launch, and its
+// share of the new zone; the last piece also takes the last T_old % 4 scores.  Same alignment conditions as
 // softmax_rows_vec_kernel; in place is fine for the same reason.
 constexpr int kSoftmaxMaxSplit = 32;
 constexpr int kSoftmaxPieceVec = 4;      // float4s per thread and piece
 constexpr int64_t kSoftmaxSplitMinRow = 65537;   // up to 64k scores a row is read once by one workgroup: 12.4 us at 38k against 14.7 split
 
-template <bool MASK_VEC, bool WRITE>
+template <bool WRITE>
 __global__ void __launch_bounds__(1024)
 softmax_rows_split_kernel(const float *__restrict__ so, int64_t so_sh, const float *__restrict__ mask,
-                          int64_t mask_sh, int64_t T_old, const float *__restrict__ sn, int64_t sn_sh,
-                          int64_t n_new, float *wo, int64_t wo_sh, float *wn, int64_t wn_sh, float *ws) {
+                          int64_t mask_sh, int64_t T_old, const float *sn, int64_t sn_sh,
+                          int64_t n_new, float *wo, int64_t wo_sh, float *wn, int64_t wn_sh, float *ws, NewKeys nk) {
   __shared__ float scratch[16];
   const int h = blockIdx.y, c = blockIdx.x, S = gridDim.x, tid = threadIdx.x;
   const float *a = so + h * so_sh;
   const float *m = mask ? mask + h * mask_sh : nullptr;
   const float *b = sn ? sn + h * sn_sh : nullptr;
   const float4 *a4 = reinterpret_cast<const float4 *>(a);
-  const float4 *m4 = reinterpret_cast<const float4 *>(m);
+  const floatx4_a4 *m4 = reinterpret_cast<const floatx4_a4 *>(m);
   const int64_t n4 = T_old >> 2, per = (n4 + S - 1) / S;
   const int64_t lo = c * per, hi = lo + per < n4 ? lo + per : n4;
   const bool last = c == S - 1;
+  const int64_t n_per = (n_new + S - 1) / S, n_lo = c * n_per < n_new ? c * n_per : n_new,
+                n_hi = n_lo + n_per < n_new ? n_lo + n_per : n_new;
   float4 x[kSoftmaxPieceVec];
 #pragma unroll
   for (int k = 0; k < kSoftmaxPieceVec; ++k) {
@@ -732,14 +792,18 @@ softmax_rows_split_kernel(const float *__restrict__ so, int64_t so_sh, const flo
     x[k] = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
     if (i < hi) x[k] = a4[i];
   }
+  if (!WRITE && nk.k) {
+    new_zone_scores(nk, h, n_lo, n_hi, wn + h * wn_sh);
+    __syncthreads();
+  }
   if (m && lo < hi) {
     // (all mask loads of the piece requested together, none conditional: see softmax_rows_vec_kernel)
-    float4 mk[kSoftmaxPieceVec];
+    floatx4 mk[kSoftmaxPieceVec];
 #pragma unroll
     for (int k = 0; k < kSoftmaxPieceVec; ++k) {
       const int64_t i = lo + tid + (int64_t)k * 1024;
       const int64_t ic = i < hi ? i : lo;
-      mk[k] = MASK_VEC ? m4[ic] : make_float4(m[4 * ic], m[4 * ic + 1], m[4 * ic + 2], m[4 * ic + 3]);
+      mk[k] = m4[ic];
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -755,20 +819,18 @@ softmax_rows_split_kernel(const float *__restrict__ so, int64_t so_sh, const flo
     float mx = -INFINITY;
 #pragma unroll
     for (int k = 0; k < kSoftmaxPieceVec; ++k) mx = fmaxf(fmaxf(mx, fmaxf(x[k].x, x[k].y)), fmaxf(x[k].z, x[k].w));
-    if (last) {
+    if (last)
       for (int64_t t = 4 * n4 + tid; t < T_old; t += 1024) mx = fmaxf(mx, a[t] + (m ? m[t] : 0.0f));
-      for (int64_t t = tid; t < n_new; t += 1024) mx = fmaxf(mx, b[t]);
-    }
+    for (int64_t t = n_lo + tid; t < n_hi; t += 1024) mx = fmaxf(mx, b[t]);
     mx = block_reduce(mx, true, scratch);
     float sum = 0.0f;
     if (mx > -INFINITY) {        // (a piece that is masked out entirely adds nothing)
 #pragma unroll
       for (int k = 0; k < kSoftmaxPieceVec; ++k)
         sum += (__expf(x[k].x - mx) + __expf(x[k].y - mx)) + (__expf(x[k].z - mx) + __expf(x[k].w - mx));
-      if (last) {
+      if (last)
         for (int64_t t = 4 * n4 + tid; t < T_old; t += 1024) sum += __expf(a[t] + (m ? m[t] : 0.0f) - mx);
-        for (int64_t t = tid; t < n_new; t += 1024) sum += __expf(b[t] - mx);
-      }
+      for (int64_t t = n_lo + tid; t < n_hi; t += 1024) sum += __expf(b[t] - mx);
     }
     sum = block_reduce(sum, false, scratch);
     if (tid == 0) {
@@ -796,8 +858,7 @@ softmax_rows_split_kernel(const float *__restrict__ so, int64_t so_sh, const flo
         w4[i] = make_float4(__expf(x[k].x - mx) * inv, __expf(x[k].y - mx) * inv, __expf(x[k].z - mx) * inv,
                             __expf(x[k].w - mx) * inv);
     }
-    if (last)
-      for (int64_t t = tid; t < n_new; t += 1024) wn[h * wn_sh + t] = __expf(b[t] - mx) * inv;
+    for (int64_t t = n_lo + tid; t < n_hi; t += 1024) wn[h * wn_sh + t] = __expf(b[t] - mx) * inv;
   }
 }
 
@@ -1004,6 +1065,31 @@ __device__ __forceinline__ void v_class_sum(const uint8_t *__restrict__ codes, i
   }
 }
 
+// The fp32 value rows of the new zone (v == nullptr: none) and their weights.
+struct NewValues {
+  const float *v, *w;
+  int64_t v_sh, v_st, w_sh;
+  int64_t n;
+};
+
+// Tokens [a, b) of the new zone of one KV head, added like a class of the packed ones (lane li of a
+// token owns channels 16 li .. + 15).
+template <int GB>
+__device__ __forceinline__ void v_new_zone_sum(const NewValues &nv, int hkv, int hq0, int64_t a, int64_t b, int ng,
+                                               float (&acc)[GB][16], int lane, int wave) {
+  const int sub = lane >> 3, li = lane & 7;
+  for (int64_t t = a + wave * 8 + sub; t < b; t += kVWaves * 8) {
+    const floatx4 *p = reinterpret_cast<const floatx4 *>(nv.v + hkv * nv.v_sh + t * nv.v_st + 16 * li);
+    const floatx4 r[4] = {p[0], p[1], p[2], p[3]};
+#pragma unroll
+    for (int g = 0; g < GB; ++g) {
+      const float w = g < ng ? nv.w[(int64_t)(hq0 + g) * nv.w_sh + t] : 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[g][i] += w * r[i >> 2][i & 3];
+    }
+  }
+}
+
 // v + the values of the lanes that differ from this one in bits 3, 4 and 5 of the lane index (the
 // eight token lanes that own the same channels): a rotation by 8 inside each row of 16 lanes, then
 // an exchange of neighbouring rows and of the two halves of the wavefront, all in the vector ALU
@@ -1026,7 +1112,7 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
                       const __half *__restrict__ scale, const __half *__restrict__ zp, int64_t vs_sh,
                       const int32_t *__restrict__ seg_bounds, int N2h, int N4h, int N8h,
                       const __half *__restrict__ V16, int64_t v16_sh, const int32_t *__restrict__ n_v16,
-                      int64_t max_T_v, float *__restrict__ partial, int H_q) {
+                      int64_t max_T_v, NewValues nv, float *__restrict__ partial, int H_q) {
   static_assert(GB <= 2 * kGB, "accumulator slots");
   const int hkv = blockIdx.y, chunk = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1066,6 +1152,7 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
     if (N16 > 0)
       v_class_sum<3, GB, GROUPED>(reinterpret_cast<const uint8_t *>(V16 + hkv * v16_sh), lo(N16), hi(N16), sc, zz, 0, wr,
                          max_T_v, ng, acc, zacc, lane, wave, w16);
+    if (nv.v) v_new_zone_sum<GB>(nv, hkv, hkv * G + g0, lo(nv.n), hi(nv.n), ng, acc, lane, wave);
     // fold the eight token lanes of the wavefront (same li), then the wavefronts, in a fixed order
     // (a head's sixteen folds first, then one guarded run of 16-byte stores: with the store inside
     // the loop every fold was a chain of dependent cross-lane moves behind its own exec-mask
@@ -1191,11 +1278,10 @@ RDKV_API int64_t rdkv_softmax_rows_workspace_bytes(int H_q) {
   return (int64_t)(H_q > 0 ? H_q : 0) * kSoftmaxMaxSplit * 2 * (int64_t)sizeof(float);
 }
 
-RDKV_API int rdkv_softmax_rows_ws(const float *scores_old, int64_t so_stride_h, const float *mask,
-                                  int64_t mask_stride_h, int64_t T_old, const float *scores_new,
-                                  int64_t sn_stride_h, int64_t n_new, float *w_old, int64_t wo_stride_h,
-                                  float *w_new, int64_t wn_stride_h, int H_q, void *workspace,
-                                  int64_t workspace_bytes, void *stream) {
+static int softmax_rows(const float *scores_old, int64_t so_stride_h, const float *mask, int64_t mask_stride_h,
+                        int64_t T_old, const float *scores_new, int64_t sn_stride_h, int64_t n_new, float *w_old,
+                        int64_t wo_stride_h, float *w_new, int64_t wn_stride_h, const NewKeys &nk, int H_q,
+                        void *workspace, int64_t workspace_bytes, void *stream) {
   RDKV_REQUIRE(H_q > 0 && H_q <= 65535 && T_old >= 0 && n_new >= 0, "rdkv_softmax_rows: bad sizes");
   RDKV_REQUIRE(T_old + n_new > 0, "rdkv_softmax_rows: empty rows");
   RDKV_REQUIRE(T_old == 0 || (scores_old && w_old), "rdkv_softmax_rows: null old-zone pointer");
@@ -1203,7 +1289,6 @@ RDKV_API int rdkv_softmax_rows_ws(const float *scores_old, int64_t so_stride_h, 
   // 16-byte accesses need aligned rows; views that are not go element by element
   const bool vec = T_old >= 4 && ((uintptr_t)scores_old % 16) == 0 && so_stride_h % 4 == 0 &&
                    ((uintptr_t)w_old % 16) == 0 && wo_stride_h % 4 == 0;
-  const bool mask_vec = !mask || (((uintptr_t)mask % 16) == 0 && mask_stride_h % 4 == 0);
   // Pieces per row: enough workgroups for two per compute unit, pieces of at most 4096 float4s;
   // rows that one workgroup holds in registers (64k scores), or heads enough to fill the device, stay with one.
   if (vec && workspace && T_old >= kSoftmaxSplitMinRow) {
@@ -1211,12 +1296,12 @@ RDKV_API int rdkv_softmax_rows_ws(const float *scores_old, int64_t so_stride_h, 
     int64_t S = std::min<int64_t>(kSoftmaxMaxSplit, (2 * (int64_t)compute_units()) / H_q);
     S = std::max(S, rdkv_cdiv(n4, 1024 * kSoftmaxPieceVec));
     if (S >= 2 && S <= kSoftmaxMaxSplit && workspace_bytes >= rdkv_softmax_rows_workspace_bytes(H_q)) {
-#define RDKV_LAUNCH_SPLIT(MV, WR)                                                                                 \
-  hipLaunchKernelGGL((softmax_rows_split_kernel<MV, WR>), dim3((unsigned)S, H_q), dim3(1024), 0,                  \
+#define RDKV_LAUNCH_SPLIT(WR)                                                                                     \
+  hipLaunchKernelGGL((softmax_rows_split_kernel<WR>), dim3((unsigned)S, H_q), dim3(1024), 0,                  \
                      (hipStream_t)stream, scores_old, so_stride_h, mask, mask_stride_h, T_old, scores_new,        \
-                     sn_stride_h, n_new, w_old, wo_stride_h, w_new, wn_stride_h, (float *)workspace)
-      if (mask_vec) { RDKV_LAUNCH_SPLIT(true, false); RDKV_LAUNCH_SPLIT(true, true); }
-      else { RDKV_LAUNCH_SPLIT(false, false); RDKV_LAUNCH_SPLIT(false, true); }
+                     sn_stride_h, n_new, w_old, wo_stride_h, w_new, wn_stride_h, (float *)workspace, nk)
+      RDKV_LAUNCH_SPLIT(false);
+      RDKV_LAUNCH_SPLIT(true);
 #undef RDKV_LAUNCH_SPLIT
       RDKV_CHECK_LAUNCH("rdkv_softmax_rows");
       return RDKV_OK;
@@ -1224,12 +1309,8 @@ RDKV_API int rdkv_softmax_rows_ws(const float *scores_old, int64_t so_stride_h, 
   }
 #define RDKV_LAUNCH_SOFTMAX(KERNEL)                                                                             \
   hipLaunchKernelGGL(KERNEL, dim3(H_q), dim3(1024), 0, (hipStream_t)stream, scores_old, so_stride_h, mask,      \
-                     mask_stride_h, T_old, scores_new, sn_stride_h, n_new, w_old, wo_stride_h, w_new, wn_stride_h)
-#define RDKV_LAUNCH_SOFTMAX_NV(NV)                                             \
-  do {                                                                         \
-    if (mask_vec) RDKV_LAUNCH_SOFTMAX((softmax_rows_vec_kernel<NV, true>));    \
-    else RDKV_LAUNCH_SOFTMAX((softmax_rows_vec_kernel<NV, false>));            \
-  } while (0)
+                     mask_stride_h, T_old, scores_new, sn_stride_h, n_new, w_old, wo_stride_h, w_new, wn_stride_h, nk)
+#define RDKV_LAUNCH_SOFTMAX_NV(NV) RDKV_LAUNCH_SOFTMAX((softmax_rows_vec_kernel<NV>))
   if (!vec) RDKV_LAUNCH_SOFTMAX(softmax_rows_kernel);
   else if (T_old <= 4096 * 2) RDKV_LAUNCH_SOFTMAX_NV(2);
   else if (T_old <= 4096 * 8) RDKV_LAUNCH_SOFTMAX_NV(8);
@@ -1239,6 +1320,35 @@ RDKV_API int rdkv_softmax_rows_ws(const float *scores_old, int64_t so_stride_h, 
 #undef RDKV_LAUNCH_SOFTMAX
   RDKV_CHECK_LAUNCH("rdkv_softmax_rows");
   return RDKV_OK;
+}
+
+RDKV_API int rdkv_softmax_rows_ws(const float *scores_old, int64_t so_stride_h, const float *mask,
+                                  int64_t mask_stride_h, int64_t T_old, const float *scores_new,
+                                  int64_t sn_stride_h, int64_t n_new, float *w_old, int64_t wo_stride_h,
+                                  float *w_new, int64_t wn_stride_h, int H_q, void *workspace,
+                                  int64_t workspace_bytes, void *stream) {
+  return softmax_rows(scores_old, so_stride_h, mask, mask_stride_h, T_old, scores_new, sn_stride_h, n_new, w_old,
+                      wo_stride_h, w_new, wn_stride_h, NewKeys{nullptr, 0, 0, 1, nullptr, 0, 0}, H_q, workspace,
+                      workspace_bytes, stream);
+}
+
+RDKV_API int rdkv_softmax_rows_new_keys(const float *scores_old, int64_t so_stride_h, const float *mask,
+                                        int64_t mask_stride_h, int64_t T_old, const void *q, int q_dtype,
+                                        int64_t q_stride_h, const float *k_new, int64_t kn_stride_h,
+                                        int64_t kn_stride_t, int64_t n_new, float *w_old, int64_t wo_stride_h,
+                                        float *w_new, int64_t wn_stride_h, int H_q, int H_kv, void *workspace,
+                                        int64_t workspace_bytes, void *stream) {
+  const char *fn = "rdkv_softmax_rows_new_keys";
+  RDKV_REQUIRE(H_q > 0 && H_kv > 0 && H_q % H_kv == 0, "%s: H_q=%d not a multiple of H_kv=%d", fn, H_q, H_kv);
+  RDKV_REQUIRE(q_dtype >= 0 && q_dtype <= 2, "%s: unknown q dtype %d", fn, q_dtype);
+  RDKV_REQUIRE(n_new == 0 || (q && k_new), "%s: null pointer", fn);
+  RDKV_REQUIRE(n_new <= 1 || kn_stride_t >= kD, "%s: key rows overlap", fn);
+  RDKV_REQUIRE(((uintptr_t)k_new % 16) == 0 && kn_stride_h % 4 == 0 && kn_stride_t % 4 == 0,
+               "%s: key rows must be 16-byte aligned", fn);
+  return softmax_rows(scores_old, so_stride_h, mask, mask_stride_h, T_old, w_new, wn_stride_h, n_new, w_old,
+                      wo_stride_h, w_new, wn_stride_h,
+                      NewKeys{q, q_stride_h, q_dtype, H_q / H_kv, n_new > 0 ? k_new : nullptr, kn_stride_h, kn_stride_t},
+                      H_q, workspace, workspace_bytes, stream);
 }
 
 RDKV_API int rdkv_softmax_rows(const float *scores_old, int64_t so_stride_h, const float *mask,
@@ -1253,13 +1363,12 @@ RDKV_API int64_t rdkv_v_weighted_sum_workspace_bytes(int H_q) {
   return (int64_t)kVChunks * (H_q > 0 ? H_q : 0) * kD * (int64_t)sizeof(float);
 }
 
-RDKV_API int rdkv_v_weighted_sum(const float *w, int64_t w_stride_h, int H_q, int H_kv, const uint8_t *V2,
-                                 int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h, const uint8_t *V8,
-                                 int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
-                                 int64_t vs_stride_h, const int32_t *seg_bounds_dev, int N2, int N4, int N8,
-                                 const void *V16_f16, int64_t v16_stride_h, const int32_t *n_v16_dev,
-                                 int64_t max_T_v, float *out, int64_t out_stride_h, void *workspace,
-                                 int64_t workspace_bytes, void *stream) {
+static int v_weighted_sum(const float *w, int64_t w_stride_h, int H_q, int H_kv, const uint8_t *V2, int64_t v2_stride_h,
+                          const uint8_t *V4, int64_t v4_stride_h, const uint8_t *V8, int64_t v8_stride_h,
+                          const void *scale_f16, const void *zp_f16, int64_t vs_stride_h,
+                          const int32_t *seg_bounds_dev, int N2, int N4, int N8, const void *V16_f16,
+                          int64_t v16_stride_h, const int32_t *n_v16_dev, int64_t max_T_v, const NewValues &nv, float *out,
+                          int64_t out_stride_h, void *workspace, int64_t workspace_bytes, void *stream) {
   RDKV_REQUIRE(H_q > 0 && H_kv > 0 && H_q % H_kv == 0, "rdkv_v_weighted_sum: H_q=%d not a multiple of H_kv=%d",
                H_q, H_kv);
   RDKV_REQUIRE(w && out, "rdkv_v_weighted_sum: null pointer");
@@ -1285,7 +1394,7 @@ RDKV_API int rdkv_v_weighted_sum(const float *w, int64_t w_stride_h, int H_q, in
   hipLaunchKernelGGL((v_weighted_sum_kernel<GB, GROUPED>), dim3(kVChunks, H_kv), dim3(64 * kVWaves), 0, s, w, w_stride_h, G, \
                      V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, (const __half *)scale_f16,             \
                      (const __half *)zp_f16, vs_stride_h, seg_bounds_dev, N2, N4, N8, (const __half *)V16_f16, \
-                     v16_stride_h, n_v16_dev, max_T_v, (float *)workspace, H_q)
+                     v16_stride_h, n_v16_dev, max_T_v, nv, (float *)workspace, H_q)
   const bool long_rows = (int64_t)N2 + N4 + N8 >= 65536;   // four consecutive tokens per lane group pay from here on
   if (G <= 2) { if (long_rows) RDKV_LAUNCH_V(2, true); else RDKV_LAUNCH_V(2, false); }
   else if (G <= 4 || G > 8) { if (long_rows) RDKV_LAUNCH_V(4, true); else RDKV_LAUNCH_V(4, false); }
@@ -1294,4 +1403,33 @@ RDKV_API int rdkv_v_weighted_sum(const float *w, int64_t w_stride_h, int H_q, in
   hipLaunchKernelGGL(v_reduce_kernel, dim3(H_q), dim3(8 * kD), 0, s, (const float *)workspace, H_q, out, out_stride_h);
   RDKV_CHECK_LAUNCH("rdkv_v_weighted_sum");
   return RDKV_OK;
+}
+
+RDKV_API int rdkv_v_weighted_sum(const float *w, int64_t w_stride_h, int H_q, int H_kv, const uint8_t *V2,
+                                 int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h, const uint8_t *V8,
+                                 int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
+                                 int64_t vs_stride_h, const int32_t *seg_bounds_dev, int N2, int N4, int N8,
+                                 const void *V16_f16, int64_t v16_stride_h, const int32_t *n_v16_dev,
+                                 int64_t max_T_v, float *out, int64_t out_stride_h, void *workspace,
+                                 int64_t workspace_bytes, void *stream) {
+  return v_weighted_sum(w, w_stride_h, H_q, H_kv, V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, scale_f16, zp_f16,
+                        vs_stride_h, seg_bounds_dev, N2, N4, N8, V16_f16, v16_stride_h, n_v16_dev, max_T_v, NewValues{}, out,
+                        out_stride_h, workspace, workspace_bytes, stream);
+}
+
+RDKV_API int rdkv_v_weighted_sum_new_values(
+    const float *w, int64_t w_stride_h, int H_q, int H_kv, const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4,
+    int64_t v4_stride_h, const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
+    int64_t vs_stride_h, const int32_t *seg_bounds_dev, int N2, int N4, int N8, const void *V16_f16,
+    int64_t v16_stride_h, const int32_t *n_v16_dev, int64_t max_T_v, const float *w_new, int64_t wn_stride_h,
+    const float *v_new, int64_t vn_stride_h, int64_t vn_stride_t, int64_t n_new, float *out, int64_t out_stride_h,
+    void *workspace, int64_t workspace_bytes, void *stream) {
+  const char *fn = "rdkv_v_weighted_sum_new_values";
+  RDKV_REQUIRE(n_new >= 0 && (n_new == 0 || (w_new && v_new)), "%s: bad new zone", fn);
+  RDKV_REQUIRE(((uintptr_t)v_new % 16) == 0 && vn_stride_h % 4 == 0 && vn_stride_t % 4 == 0,
+               "%s: value rows must be 16-byte aligned", fn);
+  return v_weighted_sum(w, w_stride_h, H_q, H_kv, V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, scale_f16, zp_f16,
+                        vs_stride_h, seg_bounds_dev, N2, N4, N8, V16_f16, v16_stride_h, n_v16_dev, max_T_v, 
+                        NewValues{n_new > 0 ? v_new : nullptr, w_new, vn_stride_h, vn_stride_t, wn_stride_h, n_new}, out,
+                        out_stride_h, workspace, workspace_bytes, stream);
 }

@@ -24,7 +24,7 @@ from . import _lib
 from .k_kernel import INV_SQRT_D, k_mixed_qk_dot_into
 from .packing import PackedKVLayer
 from .stream_cache import StreamCache, build_stream_cache, decode_attn_fused
-from .v_kernel import v_dequant_weighted_sum_dispatch_into
+from .v_kernel import _weighted_sum_with_new_zone, v_dequant_weighted_sum_dispatch_into  # noqa: F401
 
 
 def _rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, *, delta: Optional[torch.Tensor] = None,
@@ -221,30 +221,38 @@ def trizone_attention(q_2d: torch.Tensor, sp: PackedKVLayer, V16: Optional[torch
         scores_buf = torch.empty(H_q, T_old + n_new, dtype=torch.float32, device=dev)
     if out is None:
         out = torch.empty(H_q, D, dtype=torch.float32, device=dev)
-    q32 = q_2d.float()
+    if scores_buf.dim() != 2 or scores_buf.shape[0] < H_q or scores_buf.shape[1] < T_old + n_new:
+        raise RuntimeError(f"scores_buf must hold [{H_q}, {T_old + n_new}] scores, got {tuple(scores_buf.shape)}")
+    if q_2d.dtype not in _lib.DTYPE_CODE or q_2d.stride(1) != 1:
+        q_2d = q_2d.float().contiguous()
+    K_new, V_new = (_new_zone_rows(t, H_kv, n_new) for t in (K_new, V_new))
     s_old = scores_buf[:, :T_old]
     s_new = scores_buf[:, T_old:T_old + n_new]
     if T_old > 0:
-        k_mixed_qk_dot_into(q32, sp, T_old, s_old)
-    # zone C scores: fp32 bmm of the scaled query group with the appended keys (:1730-1733)
-    q_gqa = q32.view(H_kv, num_kv_groups, D) * INV_SQRT_D
-    s_new.copy_(torch.bmm(q_gqa, K_new.transpose(-1, -2)).reshape(H_q, n_new))
-    # mask + global softmax over [A | B | C], written back in place as weights (:1743-1755)
+        k_mixed_qk_dot_into(q_2d, sp, T_old, s_old)
+    # zone C scores (:1730-1733), then mask + global softmax over [A | B | C], written back in place as
+    # weights (:1743-1755)
     mask = sp.softmax_mask if (T_old > 0 and sp.softmax_mask is not None) else None
     ws = _lib.workspace(dev, lib.rdkv_softmax_rows_workspace_bytes(H_q))
-    _lib.check(lib.rdkv_softmax_rows_ws(
-        _lib.ptr(s_old), scores_buf.stride(0), _lib.ptr(mask), mask.stride(0) if mask is not None else 0,
-        T_old, s_new.data_ptr(), scores_buf.stride(0), n_new,
-        _lib.ptr(s_old), scores_buf.stride(0), s_new.data_ptr(), scores_buf.stride(0), H_q,
+    row = scores_buf.stride(0)
+    _lib.check(lib.rdkv_softmax_rows_new_keys(
+        _lib.ptr(s_old), row, _lib.ptr(mask), mask.stride(0) if mask is not None else 0,
+        T_old, q_2d.data_ptr(), _lib.DTYPE_CODE[q_2d.dtype], q_2d.stride(0), K_new.data_ptr(), K_new.stride(0),
+        K_new.stride(1), n_new, _lib.ptr(s_old), row, s_new.data_ptr(), row, H_q, H_kv,
         ws.data_ptr(), ws.numel(), _lib.stream_of(dev)))
-    if T_old > 0:
-        v_dequant_weighted_sum_dispatch_into(s_old, sp, out, V16=V16, n_v16_per_head=n_v16_per_head,
-                                             max_T_v=T_v)
-    else:
-        out.zero_()
-    # zone C values (:1780-1784)
-    out.add_(torch.bmm(s_new.reshape(H_kv, num_kv_groups, n_new), V_new).reshape(H_q, D))
+    # values of all three zones (:1777-1784)
+    _weighted_sum_with_new_zone(s_old if T_old > 0 else s_new, sp if T_old > 0 else None, out, V16, n_v16_per_head,
+                                T_v, s_new, V_new)
     return out
+
+
+def _new_zone_rows(t: torch.Tensor, H_kv: int, n_new: int) -> torch.Tensor:
+    """Appended keys / values as the kernels read them: fp32 [H_kv, n_new, 128], rows 16-byte aligned."""
+    if t.dtype != torch.float32 or t.shape != (H_kv, n_new, 128):
+        raise RuntimeError(f"appended keys / values must be fp32 [{H_kv}, {n_new}, 128], got {tuple(t.shape)} {t.dtype}")
+    if t.stride(2) != 1 or t.stride(0) % 4 or t.stride(1) % 4 or t.data_ptr() % 16 or (n_new > 1 and t.stride(1) < 128):
+        t = t.clone(memory_format=torch.contiguous_format)
+    return t
 
 
 def merge_zone_c(out_ab: torch.Tensor, lse_ab: torch.Tensor, q_2d: torch.Tensor, K_new: torch.Tensor,

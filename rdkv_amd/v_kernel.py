@@ -70,7 +70,9 @@ def _seg(t, width):
 
 
 def _launch(attn_weights, V_2bit, V_4bit, V_8bit, V_scale, V_zp, seg_bounds_per_head, seg_bounds,
-            out, V16, n_v16_per_head, max_T_v):
+            out, V16, n_v16_per_head, max_T_v, new=None):
+    """``new`` = (weights [H_q, n], values fp32 [H_kv, n, 128] with 16-byte aligned rows): a further zone,
+    added by the same launch; V_scale may then be None (nothing packed)."""
     # (this runs once per layer and decode step: views and helper calls are kept to what the launch needs)
     lib = _lib.load()
     w = attn_weights
@@ -79,7 +81,7 @@ def _launch(attn_weights, V_2bit, V_4bit, V_8bit, V_scale, V_zp, seg_bounds_per_
     dev = w.device
     H_q = w.shape[0]
     sc, zp = _sq(V_scale), _sq(V_zp)
-    H_kv = sc.shape[0]
+    H_kv = sc.shape[0] if sc is not None else new[1].shape[0]
     if w.dtype != torch.float32:
         w = w.float()
     if w.stride(1) != 1:
@@ -89,7 +91,7 @@ def _launch(attn_weights, V_2bit, V_4bit, V_8bit, V_scale, V_zp, seg_bounds_per_
     keep4, V4, v4h = _seg(V_4bit, D // 2)
     keep8, V8, v8h = _seg(V_8bit, D)
     # scale / zero point rows: [H_kv, T] or [H_kv, T, 1] with unit token stride
-    n_meta = sc.numel()
+    n_meta = sc.numel() if sc is not None else 0
     if n_meta and not (sc.stride(1) == 1 and zp.stride(1) == 1 and zp.stride(0) == sc.stride(0)):
         sc, zp = sc.reshape(H_kv, -1).contiguous(), zp.reshape(H_kv, -1).contiguous()
     N2, N4, N8 = seg_bounds
@@ -105,12 +107,18 @@ def _launch(attn_weights, V_2bit, V_4bit, V_8bit, V_scale, V_zp, seg_bounds_per_
         v16 = keep16.data_ptr() if keep16.numel() else None
     stream = _lib.stream_of(dev)
     ws = _lib.workspace(dev, lib.rdkv_v_weighted_sum_workspace_bytes(H_q))
-    _lib.check(lib.rdkv_v_weighted_sum(
+    packed = (
         w.data_ptr(), w.stride(0), H_q, H_kv, V2, v2h, V4, v4h, V8, v8h,
         sc.data_ptr() if n_meta else None, zp.data_ptr() if n_meta else None, sc.stride(0) if n_meta else 0,
         None if seg_bounds_per_head is None else seg_bounds_per_head.data_ptr(), int(N2), int(N4), int(N8),
-        v16, v16h or 0, n16 if v16 is not None else None, int(max_T_v),
-        out.data_ptr(), out.stride(0), ws.data_ptr(), ws.numel(), stream))
+        v16, v16h or 0, n16 if v16 is not None else None, int(max_T_v))
+    result = (out.data_ptr(), out.stride(0), ws.data_ptr(), ws.numel(), stream)
+    if new is None:
+        _lib.check(lib.rdkv_v_weighted_sum(*packed, *result))
+    else:
+        wn, vn = new
+        _lib.check(lib.rdkv_v_weighted_sum_new_values(*packed, wn.data_ptr(), wn.stride(0), vn.data_ptr(), vn.stride(0),
+                                                      vn.stride(1), vn.shape[1], *result))
     del keep2, keep4, keep8, keep16     # dense copies live until the launch above is enqueued
 
 
@@ -203,6 +211,23 @@ def v_dequant_weighted_sum_dispatch_into(attn_weights_old, packed_layer, out, V1
         return
     v_dequant_weighted_sum_unified_into(attn_weights_old, pl.V_2bit, pl.V_4bit, pl.V_8bit,
                                         pl.V_scale, pl.V_zp, pl.seg_bounds, out)
+
+
+def _weighted_sum_with_new_zone(attn_weights_old, packed_layer, out, V16, n_v16_per_head, max_T_v, w_new, V_new):
+    """``v_dequant_weighted_sum_dispatch_into`` plus ``w_new`` . ``V_new``, in the same launches;
+    ``packed_layer`` None: the new zone alone."""
+    pl, new = packed_layer, (w_new, V_new)
+    per_head = getattr(pl, "seg_bounds_per_head", None)
+    if per_head is None:
+        V16 = None
+    if pl is None or (sum(int(v) for v in pl.seg_bounds) == 0 and V16 is None):
+        res = out if out.dtype == torch.float32 and out.stride(1) == 1 else torch.empty(out.shape, device=out.device)
+        _launch(attn_weights_old, None, None, None, None, None, None, (0, 0, 0), res, None, None, 0, new)
+        if res is not out:
+            out.copy_(res)
+    else:
+        _launch(attn_weights_old, pl.V_2bit, pl.V_4bit, pl.V_8bit, pl.V_scale, pl.V_zp, per_head, pl.seg_bounds, out, V16,
+                n_v16_per_head, max_T_v if per_head is not None else 0, new)
 
 
 def v_dequant_weighted_sum_dispatch(attn_weights_old, packed_layer, V16=None, n_v16_per_head=None,

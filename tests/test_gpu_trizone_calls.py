@@ -1,0 +1,74 @@
+"""``trizone_attention``: the appended tokens' scores formed inside the softmax launch and their values
+added inside the V launch, against float64 over the packed zones' own K scores and V sums: token
+counts around the eight keys of a wavefront and the 128 of a workgroup's pass, rows of every softmax
+form, appended rows that are views or start at an odd float, no packed tokens at all."""
+import numpy as np
+import pytest
+import torch
+
+from rdkv_amd import fast_decode, packing, triton_k_kernel as kk, triton_v_kernel as vk
+from tests.gpu_util import DEV, require_gpu, t2n
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(H, T, G, seed):
+    g = torch.Generator().manual_seed(seed)
+    K, V = (torch.randn(1, H, T, 128, generator=g).half().to(DEV) for _ in range(2))
+    v_bits = torch.tensor([2, 4, 8, 16])[torch.randint(0, 4, (H, T), generator=g)]
+    k_bits = torch.tensor([0, 2, 4, 8])[torch.randint(0, 4, (H, 128), generator=g)]
+    k_bits[:, :3] = torch.tensor([2, 4, 8])
+    layer, v16 = packing.pack_layer_per_head(K, V, v_bits, k_bits, G)
+    return fast_decode._pre_squeeze_packed((layer,))[0], v16[0].contiguous()
+
+
+@pytest.mark.parametrize("H,T,G,n_new,dtype,form", [
+    (2, 3, 4, 1, torch.float16, "dense"), (2, 300, 4, 7, torch.bfloat16, "dense"), (3, 1200, 1, 8, torch.float32, "dense"),
+    (2, 1200, 2, 9, torch.float16, "kv"), (2, 9000, 5, 127, torch.float16, "odd"), (1, 9000, 8, 128, torch.bfloat16, "dense"),
+    (2, 34000, 4, 129, torch.float16, "kv"), (2, 34001, 9, 257, torch.float16, "dense"), (1, 66001, 4, 1, torch.float16, "dense"),
+    (1, 66001, 4, 1030, torch.float16, "odd"), (2, 0, 4, 33, torch.float16, "dense")])
+def test_trizone_attention_new_zone(H, T, G, n_new, dtype, form):
+    require_gpu()
+    g = torch.Generator().manual_seed(T + n_new)
+    wide = torch.randn(H, n_new, 260, generator=g).to(DEV)
+    k_new, v_new = {"dense": (wide[:, :, :128].contiguous(), wide[:, :, 128:256].contiguous()),
+                    "kv": (wide[:, :, :128], wide[:, :, 128:256]), "odd": (wide[:, :, 1:129], wide[:, :, 130:258])}[form]
+    q = torch.randn(H * G, 128, generator=g).to(dtype).to(DEV)
+    layer, v16 = _layer(H, max(T, 5), G, 7)
+    if T == 0:
+        layer.T_eff = layer.T_eff_k = 0
+    t_v = int(layer.T_eff)
+    t_old = int(layer.T_eff_k) if layer.T_eff_k > 0 else t_v
+    buf = torch.empty(H * G, -(-(t_old + n_new) // 4) * 4, device=DEV)
+    out = fast_decode.trizone_attention(q, layer, v16, layer.n_v16_per_head, k_new, v_new, G, scores_buf=buf)
+    q64 = t2n(q.float()).astype(np.float64).reshape(H, G, 128)
+    k64, v64 = (t2n(t).astype(np.float64) for t in (k_new, v_new))
+    s = (q64 @ k64.transpose(0, 2, 1) / np.sqrt(128.0)).reshape(H * G, n_new)
+    if t_old:
+        a = t2n(kk.k_mixed_qk_dot(q, layer, t_old)).astype(np.float64)
+        if layer.softmax_mask is not None:
+            a = a + t2n(layer.softmax_mask)
+        s = np.concatenate([a, s], axis=1)
+    w = np.exp(s - s.max(1, keepdims=True))
+    w /= w.sum(1, keepdims=True)
+    exp = (w[:, t_old:].reshape(H, G, n_new) @ v64).reshape(H * G, 128)
+    if t_old:
+        w_old = torch.from_numpy(w[:, :t_old].astype(np.float32)).to(DEV)
+        exp = exp + t2n(vk.v_dequant_weighted_sum_dispatch(w_old, layer, V16=v16, n_v16_per_head=layer.n_v16_per_head,
+                                                           max_T_v=t_v))
+    # fp32 scores, weights and sums: a few 2^-24 of values of order one
+    np.testing.assert_allclose(t2n(out), exp, rtol=0, atol=1e-5)
+    np.testing.assert_allclose(t2n(buf)[:, :t_old + n_new], w, rtol=1e-4, atol=1e-7)   # the buffer holds the weights
+
+
+def test_buffers_and_rows_that_do_not_fit_are_refused():
+    require_gpu()
+    layer, v16 = _layer(2, 40, 4, 1)
+    q, kv = torch.randn(8, 128, device=DEV), torch.randn(2, 6, 128, device=DEV)
+    args = (q, layer, v16, layer.n_v16_per_head)
+    with pytest.raises(RuntimeError):
+        fast_decode.trizone_attention(*args, kv, kv, 4, scores_buf=torch.empty(8, 45, device=DEV))
+    with pytest.raises(RuntimeError):
+        fast_decode.trizone_attention(*args, kv.half(), kv, 4)
+    with pytest.raises(RuntimeError):
+        fast_decode.trizone_attention(*args, kv, kv[:, :5], 4)
