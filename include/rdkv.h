@@ -630,9 +630,10 @@ int rdkv_pool_scores(const float *scores, int64_t stride_b, int B, int64_t T, in
  * or device [B, n_options] int32, tokens per option.  T <= 2^20 (the width sums stay exact).
  * group_rows: the doubling rounds end together for every group_rows consecutive rows (what
  * was one call of the reference; 0 = the whole batch), so many calls can share one launch.
- * workspace: rdkv_knapsack_workspace_bytes(B) bytes.  Two launches, no host synchronization.
- * Batches of few long rows (T >= 8192, max_iters <= 64, so few rows that each can have 16 or
- * more resident workgroups) run with every row shared by 16, 32 or 64 workgroups that exchange
+ * workspace: rdkv_knapsack_workspace_bytes(B) bytes.  Two launches (one for rows of at most
+ * 256 scores in groups of at most 16), no host synchronization.
+ * Batches of few long rows (max_iters <= 64; T >= 8192 and so few rows that each can have 16 or
+ * more resident workgroups, or 4096 <= T < 8192 and at most 64 rows) run with every row shared by 8, 16, 32 or 64 workgroups that exchange
  * integer width sums once per pass of 15 doublings or four bisection levels (the first pass takes
  * the starting multiplier and the first four levels together); the same bits.  The
  * workgroups wait for each other with a bound: should a wait not end (it cannot while the launch

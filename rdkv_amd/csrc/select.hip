@@ -628,6 +628,155 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same solver for short rows (a head's channels): a wavefront per row with the row in registers
+// and a workgroup per group of rows, so that a pass has no barrier, the rows' doublings meet in LDS,
+// and one launch replaces two.  Bound by its chain of dependent passes (a wavefront sum each).
+// A call of 8 rows of 128 / 256 scores 18.3 / 19.7 -> 11.3 / 11.6 us (the host side of the call), 256
+// rows of 128 19.9 -> 11.2.
+// ---------------------------------------------------------------------------------------------
+constexpr int kGroupMaxRows = kMaxThreads / 64;
+constexpr int kGroupMaxHeld = 4;
+
+// Sum over the wavefront, in every lane.
+__device__ __forceinline__ int wave_sum_uniform(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);     // lane ^ 1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);     // lane ^ 2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xF, 0xF, false);    // mirror within eight
+  v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xF, 0xF, false);    // mirror within sixteen
+  return __builtin_amdgcn_readlane(v, 0) + __builtin_amdgcn_readlane(v, 16) + __builtin_amdgcn_readlane(v, 32) +
+         __builtin_amdgcn_readlane(v, 48);
+}
+
+template <int HELD, int NOPT>
+__global__ void __launch_bounds__(kMaxThreads)
+knapsack_group_kernel(const float* __restrict__ scores, int64_t stride_b, int group_rows, int T,
+                      const float* __restrict__ budget, Options o, int max_iters, float tol, void* __restrict__ out,
+                      int out_elem_size, int64_t out_stride_b, int* __restrict__ counts) {
+  __shared__ float s_lam0[kGroupMaxRows];
+  __shared__ int s_d[kGroupMaxRows];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.x * group_rows + wave;
+  const float* row = scores + (int64_t)b * stride_b;
+  const float bud = budget[b];
+  float se[HELD][NOPT];       // score times eps (+inf for the options past the last: never the smallest)
+  float m = -__builtin_inff();
+#pragma unroll
+  for (int j = 0; j < HELD; ++j) {
+    const int t = lane + 64 * j;
+    const float v = t < T ? row[t] : 0.f;
+    if (t < T) m = fmaxf(m, v);
+#pragma unroll
+    for (int k = 0; k < NOPT; ++k) se[j][k] = k < o.n ? __fmul_rn(v, o.eps[k]) : __builtin_inff();
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+  // the option of held score j at the lambda whose products are in lb: index and width
+  auto pick = [&](int j, const float (&lb)[NOPT], int& width) __attribute__((always_inline)) {
+    float best = __fadd_rn(se[j][0], lb[0]);
+    int idx = 0;
+    width = o.ibits[0];
+#pragma unroll
+    for (int k = 1; k < NOPT; ++k) {
+      const float cst = __fadd_rn(se[j][k], lb[k]);
+      const bool lt = cst < best;                                  // strict: the first minimum wins
+      best = lt ? cst : best;
+      idx = lt ? k : idx;
+      width = lt ? o.ibits[k] : width;
+    }
+    return idx;
+  };
+  auto solve = [&](float lam) __attribute__((always_inline)) {
+    float lb[NOPT];
+#pragma unroll
+    for (int k = 0; k < NOPT; ++k) lb[k] = __fmul_rn(lam, o.bits[k]);
+    int acc = 0;
+#pragma unroll
+    for (int j = 0; j < HELD; ++j) {
+      int width;
+      pick(j, lb, width);
+      acc += lane + 64 * j < T ? width : 0;
+    }
+    return __fdiv_rn((float)wave_sum_uniform(acc), (float)T);
+  };
+
+  // the doublings the row asks for on its own
+  const float lam0 = fmaxf(__fmul_rn(m, 0.375f), 1e-8f);
+  int d = 0;
+  {
+    float lam = lam0;
+    for (; d < kMaxDoublings; ++d) {
+      if (!(solve(lam) > bud)) break;
+      lam = __fmul_rn(lam, 2.0f);
+    }
+  }
+  if (lane == 0) {
+    s_lam0[wave] = lam0;
+    s_d[wave] = d;
+  }
+  __syncthreads();
+  // the rounds its group executes (as in knapsack_bisect_kernel): lane r replays row r
+  int dmax = 0, gmax = 0;
+  if (lane < group_rows) {
+    float lam = s_lam0[lane];
+    dmax = s_d[lane];
+    gmax = kMaxDoublings + 1;                      // never reaches 1e12
+    for (int it = 0; it < kMaxDoublings; ++it) {
+      if (it < dmax) lam = __fmul_rn(lam, 2.0f);
+      if (lam >= 1e12f) { gmax = it; break; }
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    dmax = max(dmax, __shfl_xor(dmax, off, 64));
+    gmax = max(gmax, __shfl_xor(gmax, off, 64));
+  }
+  const int mine = min(d, min(min(dmax, gmax + 1), kMaxDoublings));
+  float lam_hi = lam0;
+  for (int i = 0; i < mine; ++i) lam_hi = __fmul_rn(lam_hi, 2.0f);
+
+  float lam_lo = 0.f, lam_final = 0.f;
+  if (!(solve(0.f) <= bud)) {
+    const float denom = fmaxf(bud, 1e-8f);
+    for (int it = 0; it < max_iters; ++it) {
+      const float mid = __fdiv_rn(__fadd_rn(lam_lo, lam_hi), 2.0f);
+      const float avg = solve(mid);
+      lam_final = mid;
+      const float rel = __fdiv_rn(fabsf(__fsub_rn(avg, bud)), denom);
+      if (rel < tol) break;
+      if (avg > bud) lam_lo = mid; else lam_hi = mid;
+    }
+  }
+  float lb[NOPT];
+#pragma unroll
+  for (int k = 0; k < NOPT; ++k) lb[k] = __fmul_rn(lam_final, o.bits[k]);
+  uint8_t* out_row = reinterpret_cast<uint8_t*>(out) + (int64_t)b * out_stride_b * out_elem_size;
+  int cnt[NOPT];
+#pragma unroll
+  for (int k = 0; k < NOPT; ++k) cnt[k] = 0;
+#pragma unroll
+  for (int j = 0; j < HELD; ++j) {
+    const int t = lane + 64 * j;
+    int w;
+    const int idx = pick(j, lb, w);
+    if (t < T) {
+#pragma unroll
+      for (int k = 0; k < NOPT; ++k) cnt[k] += k == idx ? 1 : 0;
+      if (out_elem_size == 1) out_row[t] = (uint8_t)w;
+      else reinterpret_cast<int64_t*>(out_row)[t] = (int64_t)w;
+    }
+  }
+  if (counts != nullptr) {
+#pragma unroll
+    for (int k = 0; k < NOPT; ++k) {
+      if (k < o.n) {
+        const int total = wave_sum_uniform(cnt[k]);
+        if (lane == 0) counts[(int64_t)b * o.n + k] = total;
+      }
+    }
+  }
+}
+
 // Independent rows with lambda kept in double (the single-row solver applied to each row).
 __global__ void __launch_bounds__(kMaxThreads)
 knapsack_rows_kernel(const float* __restrict__ scores, int64_t stride_b, int T,
@@ -739,7 +888,10 @@ static int coop_held_index(int64_t chunk) { return chunk <= 2 * kCoopThreads ? 0
 // form): a power of two, chunks of at least 512 scores, at most 64 per row, the whole launch on at
 // most half of the workgroup slots the device has for the kernel variant the chunk length selects,
 // and only when that gives a row at least sixteen (with fewer, one workgroup per row was as fast or
-// faster on 64 rows of 32k scores).
+// faster on 64 rows of 32k scores) - or its full eight for a row of 4096 .. 8191 in a launch of at most
+// kCoopShortGrid workgroups: 8 rows of 4096 / 6000 scores 41.1 / 54.0 -> 33.5 / 40.8 us a call, 64 rows
+// 46.8 / 56.6 -> 36.4 / 44.6, 256 rows (four or fewer each) 47.3 against 60.2.
+constexpr int64_t kCoopShortGrid = 512;
 static int coop_split(int B, int64_t T, int max_iters) {
   if (B <= 0 || T < 4096 || max_iters > kCoopMaxIters) return 0;
   // workgroup slots of the device for the kernel that holds 2 / 4 / 8 scores per thread
@@ -772,7 +924,7 @@ static int coop_split(int B, int64_t T, int max_iters) {
     if (S <= cap) break;
     S = pow2_floor(cap);
   }
-  if (S < 16) return 0;
+  if (S < 16 && !(T < 8192 && S == 8 && (int64_t)B * S <= kCoopShortGrid)) return 0;
   const int64_t chunk = (T + S - 1) / S;
   if ((int64_t)B * S > slots_of_device[dev][coop_held_index(chunk)] / 2) return 0;
   // (a chunk's width sum must fit the 24 value bits of an exchange word)
@@ -815,6 +967,19 @@ RDKV_API int rdkv_knapsack_batched(const float* scores, int64_t stride_b, int B,
     auto kernel = held == 0 ? knapsack_coop_kernel<2> : (held == 1 ? knapsack_coop_kernel<4> : knapsack_coop_kernel<8>);
     hipLaunchKernelGGL(kernel, dim3((unsigned)(B * S)), dim3(kCoopThreads), 0, s, scores, stride_b, group_rows, (int)T, S,
                        budget, o, max_iters, tol, state, out, out_elem_size, out_stride_b, counts);
+    RDKV_CHECK_LAUNCH("rdkv_knapsack_batched");
+    return RDKV_OK;
+  }
+  if (T <= 64 * kGroupMaxHeld && group_rows <= kGroupMaxRows) {
+    // short rows: a wavefront per row, a workgroup per group (the rows of a group meet in LDS: at most sixteen, the
+    // wavefronts of a workgroup; longer rows have no registers left per lane and are the other form's)
+#define RDKV_LAUNCH_GROUP(HELD, NOPT)                                                                              \
+  hipLaunchKernelGGL((knapsack_group_kernel<HELD, NOPT>), dim3(B / group_rows), dim3(64 * group_rows), 0, s, scores, \
+                     stride_b, group_rows, (int)T, budget, o, max_iters, tol, out, out_elem_size, out_stride_b, counts)
+    if (T <= 128 && o.n <= 5) RDKV_LAUNCH_GROUP(2, 5);
+    else if (o.n <= 5) RDKV_LAUNCH_GROUP(4, 5);
+    else RDKV_LAUNCH_GROUP(4, kMaxOptions);
+#undef RDKV_LAUNCH_GROUP
     RDKV_CHECK_LAUNCH("rdkv_knapsack_batched");
     return RDKV_OK;
   }
