@@ -221,8 +221,12 @@ def trizone_attention(q_2d: torch.Tensor, sp: PackedKVLayer, V16: Optional[torch
         scores_buf = torch.empty(H_q, T_old + n_new, dtype=torch.float32, device=dev)
     if out is None:
         out = torch.empty(H_q, D, dtype=torch.float32, device=dev)
-    if scores_buf.dim() != 2 or scores_buf.shape[0] < H_q or scores_buf.shape[1] < T_old + n_new:
-        raise RuntimeError(f"scores_buf must hold [{H_q}, {T_old + n_new}] scores, got {tuple(scores_buf.shape)}")
+    if H_q % num_kv_groups:
+        raise RuntimeError(f"{H_q} query heads in groups of {num_kv_groups}")
+    if scores_buf.dim() != 2 or scores_buf.shape[0] != H_q or scores_buf.shape[1] < T_old + n_new \
+            or scores_buf.dtype != torch.float32 or scores_buf.stride(1) != 1:
+        raise RuntimeError(f"scores_buf must be fp32 [{H_q}, >= {T_old + n_new}] with unit column stride, "
+                           f"got {tuple(scores_buf.shape)} {scores_buf.dtype}")
     if q_2d.dtype not in _lib.DTYPE_CODE or q_2d.stride(1) != 1:
         q_2d = q_2d.float().contiguous()
     K_new, V_new = (_new_zone_rows(t, H_kv, n_new) for t in (K_new, V_new))

@@ -68,9 +68,13 @@ def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int
     return out, check
 
 
-def _check_v_counts(counts) -> None:
+def _check_v_counts(pl: PackedKVLayer, counts) -> None:
+    segs = (pl.V_2bit, pl.V_4bit, pl.V_8bit)
     for h, row in enumerate(counts):
         assert sum(row[:3]) == row[3], f"head {h}: seg_bounds_per_head {row[:3]} != T_eff_per_head {row[3]}"
+        for n, seg in zip(row, segs):
+            assert seg is None or n <= seg.shape[2], f"head {h}: {n} tokens in a V segment of {seg.shape[2]}"
+        assert row[3] <= int(pl.T_eff), f"head {h}: {row[3]} tokens in a stripe of {pl.T_eff}"
 
 
 def _unpack_v_perhead(pl: PackedKVLayer, *, head_dim: int) -> Tensor:
@@ -79,7 +83,7 @@ def _unpack_v_perhead(pl: PackedKVLayer, *, head_dim: int) -> Tensor:
     if int(pl.T_eff) == 0:
         return torch.zeros(1, pl.V_scale.shape[1], 0, head_dim, dtype=torch.float16, device=pl.V_scale.device)
     out, check = _unpack_v_enqueue(pl, None, head_dim)
-    _check_v_counts(check.tolist())
+    _check_v_counts(pl, check.tolist())
     return out
 
 
@@ -92,11 +96,11 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
     shared-layout layers) (trizone_decompress.py:185-333)."""
     past_kv: List[Tuple[Tensor, Tensor]] = []
     masks: List[Optional[Tensor]] = []
-    unchecked: List[Tuple[Optional[PackedKVLayer], Tensor]] = []     # per-head counts the launches below read
+    unchecked = []        # (check, layer, per-head counts that the launches below read)
     for i, pl in enumerate(dual_cache.packed):
         K_full, k_counts = _unpack_k_enqueue(pl, head_dim)
         if k_counts is not None:
-            unchecked.append((pl, k_counts))
+            unchecked.append((_check_k_counts, pl, k_counts))
         zone_b = dual_cache.new_v_only[i] if i < len(dual_cache.new_v_only) else None
         if _is_perhead_layout(pl):
             rows_b = None
@@ -109,7 +113,7 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
                 joined = rows_b is not None and rows_b.dtype == torch.float16 and rows_b.shape[:2] == pl.V_scale.shape[:2] \
                     and rows_b.shape[3] == head_dim and rows_b.device == pl.V_scale.device
                 V_full, v_counts = _unpack_v_enqueue(pl, rows_b if joined else None, head_dim)
-                unchecked.append((None, v_counts))
+                unchecked.append((_check_v_counts, pl, v_counts))
                 if rows_b is not None and not joined:
                     V_full = torch.cat([V_full, rows_b], dim=2)
         else:
@@ -141,11 +145,7 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
                 masks.append(None)
     # the counts of every layer in one read, behind the launches (which clamp what they follow)
     if unchecked:
-        rows = iter(_lib.download(torch.cat([c.reshape(-1) for _, c in unchecked])).tolist())
-        for pl, c in unchecked:
-            table = [[next(rows) for _ in range(c.shape[1])] for _ in range(c.shape[0])]
-            if pl is None:
-                _check_v_counts(table)
-            else:
-                _check_k_counts(pl, table)
+        rows = iter(_lib.download(torch.cat([c.reshape(-1) for _, _, c in unchecked])).tolist())
+        for check, pl, c in unchecked:
+            check(pl, [[next(rows) for _ in range(c.shape[1])] for _ in range(c.shape[0])])
     return (tuple(past_kv), masks) if return_masks else tuple(past_kv)

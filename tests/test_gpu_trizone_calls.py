@@ -72,3 +72,9 @@ def test_buffers_and_rows_that_do_not_fit_are_refused():
         fast_decode.trizone_attention(*args, kv.half(), kv, 4)
     with pytest.raises(RuntimeError):
         fast_decode.trizone_attention(*args, kv, kv[:, :5], 4)
+    with pytest.raises(RuntimeError):
+        fast_decode.trizone_attention(*args, kv, kv, 4, scores_buf=torch.empty(9, 48, device=DEV))
+    with pytest.raises(RuntimeError):
+        fast_decode.trizone_attention(*args, kv, kv, 4, scores_buf=torch.empty(8, 48, device=DEV, dtype=torch.float16))
+    with pytest.raises(RuntimeError):
+        fast_decode.trizone_attention(torch.randn(10, 128, device=DEV), *args[1:], kv, kv, 4)

@@ -84,3 +84,14 @@ def test_counts_that_do_not_fit_the_layer_are_reported():
     pl.K_ch_seg_bounds_per_head = pl.K_ch_seg_bounds_per_head + 1          # 8-bit channels, no 8-bit segment
     with pytest.raises(AssertionError, match="segment that is missing"):
         packing.unpack_k_mixed(pl, D=128)
+    pl, nvo = packing.pack_layer_per_head(K, V, vb, kb, 2)
+    counts = pl.seg_bounds_per_head.clone()
+    counts[:, 0] += 100                                          # more 2-bit tokens than the segment has, sums alike
+    pl.seg_bounds_per_head, pl.T_eff_per_head = counts, pl.T_eff_per_head + 100
+    with pytest.raises(AssertionError, match="V segment"):
+        tz._unpack_v_perhead(pl, head_dim=128)
+    counts = pl.K_ch_seg_bounds_per_head.clone()
+    counts[:, 0] += 200                                          # more 2-bit channels than the segment has
+    pl.K_ch_seg_bounds_per_head = counts
+    with pytest.raises(AssertionError, match="K segments of"):
+        packing.unpack_k_mixed(pl, D=128)
