@@ -1,11 +1,21 @@
 // y[n] = sum_k W[n, k] * x[k] (+ bias[n]) for one activation row: the matrix-vector products of a
 // decode step (q/k/v, output, gate/up, down projections and the LM head; reference:
 // obkv_accel/fast_decode.py:1650-1656, 1786, 1797-1804, 1826 as F.linear calls).  The work is a
-// single pass over W, so the kernel is an HBM stream: a wavefront owns a run of rows and takes
-// R of them at a time, every lane reading 16 bytes (eight weights) per row and step with
-// 4 * R loads in flight; x sits in LDS and is read once per step for all R rows; products are
-// accumulated in fp32 (two-element dot instructions for fp16) and the 64 lanes are summed with
-// shuffles in a fixed order, so results are reproducible run to run.
+// single pass over W, so the kernel is an HBM stream: a wavefront takes one row at a time, every
+// lane reading 16 bytes (eight weights) per load with four to eight loads in flight; x sits in LDS;
+// products are accumulated in fp32 (two-element dot instructions for fp16) and the 64 lanes are
+// summed with shuffles in a fixed order, so results are reproducible run to run and do not depend
+// on how the rows are dealt.
+//
+// Rows are dealt round-robin over all wavefronts of the launch, so the device reads one contiguous
+// front and every compute unit holds the same number of wavefronts to within one row.  (Runs of
+// rows per wavefront, four or two rows at a time, rounded the runs up: 28672 rows left a quarter of
+// the compute units with half the wavefronts, and 6144 half of them.)  Matrices of fp16, cold, us
+// before -> now: 28672 x 4096 42.4 -> 37.6 (6.25 TB/s, near the 6.3 .. 7 of a large read),
+// 4096 x 14336 with SiLU 24.0 -> 21.8, 6144 x 4096 12.3 -> 11.3, 4096 x 4096 8.5 -> 7.9,
+// 128256 x 4096 157.7 -> 148.5 (7.1 TB/s); the short ones are bound by launch, staging and the
+// first round trip.  Tiles of two loads were slower (12.4 / 152.9 at 6144 / 128256 rows), tiles of
+// eight equal on short matrices and slower on long ones (11.5 / 155.9).
 #include "rdkv_common.h"
 #include "rope_device.h"
 
@@ -81,44 +91,38 @@ struct RowSource {
 };
 
 // K % 512 == 0 (every lane takes whole 16-byte pieces: K / 512 per row), rows 16-byte aligned.
-template <int dtype, int R, int MODE>
-__global__ void __launch_bounds__(256)
+template <int dtype, int MODE, int BT>
+__global__ void __launch_bounds__(BT)
 gemv_kernel(const uint16_t *__restrict__ W, int64_t w_stride_row, RowSource src,
-            const uint16_t *__restrict__ bias, int N, int K, int rows_per_wave, uint16_t *__restrict__ y) {
+            const uint16_t *__restrict__ bias, int N, int K, uint16_t *__restrict__ y) {
   extern __shared__ uint4 xs[];      // K / 8 pieces of x (kNorm: then K / 8 pieces of the norm weight + 4 floats)
   const int k8 = K >> 3;
-  // A wavefront walks its rows R at a time and each group of rows in pieces of 256 x 16 bytes
-  // ("tiles": 4 loads per row and lane).  The loads of the next tile are issued before the
-  // current one is consumed, and those of the first tile before the row is staged, so the
-  // staging and every reduction overlap a weight fetch that is already in flight.
+  // A wavefront walks each of its rows in pieces of 256 x 16 bytes ("tiles": 4 loads per lane).  The
+  // loads of the next tile are issued before the current one is consumed, and those of the first
+  // tile before the row is staged, so the staging and every reduction overlap a weight fetch that
+  // is already in flight.
+  static_assert(MODE != kNorm || BT == 256, "the sum of squares adds four wavefronts' parts in a fixed order");
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-  const int row_begin = wave * rows_per_wave;
-  const int row_end = min(N, row_begin + rows_per_wave);
+  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * (BT / 64) + (threadIdx.x >> 6));
+  const int n_waves = gridDim.x * (BT / 64);
   const int n_j = (k8 + 255) >> 8;
-  struct Cur { int r0, jj; };
+  struct Cur { int row, jj; };
   auto next = [&](Cur c) __attribute__((always_inline)) -> Cur {
-    if (c.jj + 1 < n_j) return Cur{c.r0, c.jj + 1};
-    return Cur{c.r0 + R, 0};
+    if (c.jj + 1 < n_j) return Cur{c.row, c.jj + 1};
+    return Cur{c.row + n_waves, 0};
   };
-  auto load_tile = [&](Cur c, uint4 (&wv)[R][4]) __attribute__((always_inline)) {
+  auto load_tile = [&](Cur c, uint4 (&wv)[4]) __attribute__((always_inline)) {
+    const uint4 *p = reinterpret_cast<const uint4 *>(W + (int64_t)c.row * w_stride_row);
     const int j0 = lane + 256 * c.jj;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int j = j0 + 64 * u < k8 ? j0 + 64 * u : j0;
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int row = c.r0 + r < row_end ? c.r0 + r : c.r0;
-        wv[r][u] = load_stream(reinterpret_cast<const uint4 *>(W + (int64_t)row * w_stride_row) + j);
-      }
-    }
+    for (int u = 0; u < 4; ++u) wv[u] = load_stream(p + (j0 + 64 * u < k8 ? j0 + 64 * u : j0));
   };
-  uint4 wa[R][4], wb[R][4];
-  Cur ca{row_begin, 0};
-  if (ca.r0 < row_end) load_tile(ca, wa);
+  uint4 wa[4], wb[4];
+  Cur ca{wave, 0};
+  if (ca.row < N) load_tile(ca, wa);
   if (MODE == kFromF32) {
     const float4 *xf = reinterpret_cast<const float4 *>(src.a);
-    for (int i = threadIdx.x; i < k8; i += 256) {
+    for (int i = threadIdx.x; i < k8; i += BT) {
       const float4 a = xf[2 * i], b = xf[2 * i + 1];
       const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
       xs[i] = pack8<dtype>(v);
@@ -130,7 +134,7 @@ gemv_kernel(const uint16_t *__restrict__ W, int64_t w_stride_row, RowSource src,
     const uint4 *pb = reinterpret_cast<const uint4 *>(src.b ? src.b : src.a);   // loads stay unconditional
     const uint4 *pc = reinterpret_cast<const uint4 *>(src.c);
     float ss = 0.0f;
-    for (int i = threadIdx.x; i < k8; i += 256) {
+    for (int i = threadIdx.x; i < k8; i += BT) {
       const uint4 va = pa[i], vb = pb[i];
       ws[i] = pc[i];
       float fa[8], fb[8];
@@ -152,7 +156,7 @@ gemv_kernel(const uint16_t *__restrict__ W, int64_t w_stride_row, RowSource src,
     if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = ss;
     __syncthreads();
     const float rs = rsqrtf((s_part[0] + s_part[1] + s_part[2] + s_part[3]) / (float)K + src.eps);
-    for (int i = threadIdx.x; i < k8; i += 256) {   // the pieces this thread wrote itself
+    for (int i = threadIdx.x; i < k8; i += BT) {   // the pieces this thread wrote itself
       float fr[8], fw[8];
       unpack8<dtype>(xs[i], fr);
       unpack8<dtype>(ws[i], fw);
@@ -162,7 +166,7 @@ gemv_kernel(const uint16_t *__restrict__ W, int64_t w_stride_row, RowSource src,
     }
   } else if (MODE == kSilu) {
     const uint4 *pa = reinterpret_cast<const uint4 *>(src.a), *pb = reinterpret_cast<const uint4 *>(src.b);
-    for (int i = threadIdx.x; i < k8; i += 256) {
+    for (int i = threadIdx.x; i < k8; i += BT) {
       float g[8], u[8];
       unpack8<dtype>(pa[i], g);
       unpack8<dtype>(pb[i], u);
@@ -175,41 +179,31 @@ gemv_kernel(const uint16_t *__restrict__ W, int64_t w_stride_row, RowSource src,
       xs[i] = pack8<dtype>(g);
     }
   } else {
-    for (int i = threadIdx.x; i < k8; i += 256) xs[i] = reinterpret_cast<const uint4 *>(src.a)[i];
+    for (int i = threadIdx.x; i < k8; i += BT) xs[i] = reinterpret_cast<const uint4 *>(src.a)[i];
   }
   __syncthreads();
-  float acc[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) acc[r] = 0.0f;
-  auto compute_tile = [&](Cur c, const uint4 (&wv)[R][4]) __attribute__((always_inline)) {
+  float acc = 0.0f;
+  auto compute_tile = [&](Cur c, const uint4 (&wv)[4]) __attribute__((always_inline)) {
     const int j0 = lane + 256 * c.jj;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      if (j0 + 64 * u < k8) {
-        const uint4 xv = xs[j0 + 64 * u];
-#pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] = dot8<dtype>(wv[r][u], xv, acc[r]);
-      }
-    }
+    for (int u = 0; u < 4; ++u)
+      if (j0 + 64 * u < k8) acc = dot8<dtype>(wv[u], xs[j0 + 64 * u], acc);
     if (c.jj + 1 == n_j) {
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float s = rdkv_wave_sum(acc[r]);
-        if (lane == 0 && c.r0 + r < row_end) {
-          const float b = bias ? rdkv_load_as_float(bias, dtype, c.r0 + r) : 0.0f;
-          rdkv_store_from_float(y, dtype, c.r0 + r, s + b);
-        }
-        acc[r] = 0.0f;
+      const float s = rdkv_wave_sum(acc);
+      if (lane == 0) {
+        const float b = bias ? rdkv_load_as_float(bias, dtype, c.row) : 0.0f;
+        rdkv_store_from_float(y, dtype, c.row, s + b);
       }
+      acc = 0.0f;
     }
   };
-  while (ca.r0 < row_end) {
+  while (ca.row < N) {
     const Cur cb = next(ca);
-    if (cb.r0 < row_end) load_tile(cb, wb);
+    if (cb.row < N) load_tile(cb, wb);
     compute_tile(ca, wa);
-    if (cb.r0 >= row_end) break;
+    if (cb.row >= N) break;
     ca = next(cb);
-    if (ca.r0 < row_end) load_tile(ca, wa);
+    if (ca.row < N) load_tile(ca, wa);
     compute_tile(cb, wb);
   }
 }
@@ -217,21 +211,22 @@ gemv_kernel(const uint16_t *__restrict__ W, int64_t w_stride_row, RowSource src,
 template <int dtype, int MODE>
 void launch_gemv(const void *W, int64_t w_stride_row, const RowSource &src, const void *bias, int N, int K, void *y,
                  int n_cu, hipStream_t s) {
-  // eight wavefronts per compute unit when there are rows enough; a wavefront takes at least R rows
-  const int max_waves = n_cu * 8;
-  const int R = N >= 4 * max_waves ? 4 : 2;
-  int waves = (int)rdkv_cdiv(N, R);
-  if (waves > max_waves) waves = max_waves;
-  int rows_per_wave = (int)rdkv_cdiv(N, waves);
-  rows_per_wave = (int)rdkv_cdiv(rows_per_wave, R) * R;
-  const int blocks = (int)rdkv_cdiv(rdkv_cdiv(N, rows_per_wave), 4);
+  // Sixteen wavefronts per compute unit while it has at most 32 rows (4096 x 4096: 7.9 us against 8.4
+  // with eight, 6144 x 4096 11.3 against 11.7), eight beyond, where fewer streams read faster (28672 x 4096
+  // 37.6 against 38.2, 128256 x 4096 148.5 against 156.5).
+  const int max_waves = n_cu * (N <= 32 * n_cu ? 16 : 8);
+  const int waves = N < max_waves ? N : max_waves;
   const size_t lds = MODE == kNorm ? (size_t)K * 4 + 16 : (size_t)K * 2;
-  if (R == 4)
-    hipLaunchKernelGGL((gemv_kernel<dtype, 4, MODE>), dim3(blocks), dim3(256), lds, s, (const uint16_t *)W,
-                       w_stride_row, src, (const uint16_t *)bias, N, K, rows_per_wave, (uint16_t *)y);
+  // Workgroups of eight wavefronts when the row is long: it is staged half as often (4096 x 14336 with
+  // SiLU 21.8 us against 25.2 with four).  A row with its norm keeps four: at most 8192 long, and the order
+  // in which its squares are summed.
+  constexpr int kLong = MODE == kNorm ? 256 : 512;
+  if (K > 8192)
+    hipLaunchKernelGGL((gemv_kernel<dtype, MODE, kLong>), dim3((unsigned)rdkv_cdiv(waves, kLong / 64)), dim3(kLong), lds, s,
+                       (const uint16_t *)W, w_stride_row, src, (const uint16_t *)bias, N, K, (uint16_t *)y);
   else
-    hipLaunchKernelGGL((gemv_kernel<dtype, 2, MODE>), dim3(blocks), dim3(256), lds, s, (const uint16_t *)W,
-                       w_stride_row, src, (const uint16_t *)bias, N, K, rows_per_wave, (uint16_t *)y);
+    hipLaunchKernelGGL((gemv_kernel<dtype, MODE, 256>), dim3((unsigned)rdkv_cdiv(waves, 4)), dim3(256), lds, s,
+                       (const uint16_t *)W, w_stride_row, src, (const uint16_t *)bias, N, K, (uint16_t *)y);
 }
 
 int compute_units() {
