@@ -392,12 +392,12 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
 def _check_k_counts(packed: "PackedKVLayer", counts: Sequence[Sequence[int]]) -> None:
     m2, m4, m8 = packed.K_ch_seg_bounds
     widths = (_seg_padded_len(m2, 4), _seg_padded_len(m4, 2), m8)
-    listed = packed.K_ch_sort_idx_per_head.shape[-1]
-    for row in counts:
-        for n, t in zip(row, (packed.K_2bit, packed.K_4bit, packed.K_8bit)):
-            assert n == 0 or t is not None, f"a head keeps {n} channels of a K segment that is missing"
-        assert all(n <= w for n, w in zip(row, widths)), f"a head keeps {row} channels of K segments of {widths}"
-        assert sum(row) <= listed, f"a head keeps {sum(row)} channels, {listed} are listed"
+    most = [max(column) for column in zip(*counts)]
+    for n, t in zip(most, (packed.K_2bit, packed.K_4bit, packed.K_8bit)):
+        assert n == 0 or t is not None, f"a head keeps {n} channels of a K segment that is missing"
+    assert all(n <= w for n, w in zip(most, widths)), f"heads keep {most} channels of K segments of {widths}"
+    kept, listed = max(map(sum, counts)), packed.K_ch_sort_idx_per_head.shape[-1]
+    assert kept <= listed, f"a head keeps {kept} channels, {listed} are listed"
 
 
 def unpack_k_mixed(packed: "PackedKVLayer", D: int) -> Tensor:

@@ -69,12 +69,12 @@ def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int
 
 
 def _check_v_counts(pl: PackedKVLayer, counts) -> None:
-    segs = (pl.V_2bit, pl.V_4bit, pl.V_8bit)
-    for h, row in enumerate(counts):
-        assert sum(row[:3]) == row[3], f"head {h}: seg_bounds_per_head {row[:3]} != T_eff_per_head {row[3]}"
-        for n, seg in zip(row, segs):
-            assert seg is None or n <= seg.shape[2], f"head {h}: {n} tokens in a V segment of {seg.shape[2]}"
-        assert row[3] <= int(pl.T_eff), f"head {h}: {row[3]} tokens in a stripe of {pl.T_eff}"
+    rows = [seg.shape[2] if seg is not None else n for n, seg in zip(map(max, zip(*counts)), (pl.V_2bit, pl.V_4bit, pl.V_8bit))]
+    r2, r4, r8 = rows
+    for h, (n2, n4, n8, n) in enumerate(counts):
+        assert n2 + n4 + n8 == n, f"head {h}: seg_bounds_per_head {[n2, n4, n8]} != T_eff_per_head {n}"
+        assert n2 <= r2 and n4 <= r4 and n8 <= r8, f"head {h}: {[n2, n4, n8]} tokens in V segments of {rows}"
+        assert n <= pl.T_eff, f"head {h}: {n} tokens in a stripe of {pl.T_eff}"
 
 
 def _unpack_v_perhead(pl: PackedKVLayer, *, head_dim: int) -> Tensor:
@@ -145,7 +145,9 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
                 masks.append(None)
     # the counts of every layer in one read, behind the launches (which clamp what they follow)
     if unchecked:
-        rows = iter(_lib.download(torch.cat([c.reshape(-1) for _, _, c in unchecked])).tolist())
+        flat, at = _lib.download(torch.cat([c.reshape(-1) for _, _, c in unchecked])).tolist(), 0
         for check, pl, c in unchecked:
-            check(pl, [[next(rows) for _ in range(c.shape[1])] for _ in range(c.shape[0])])
+            end, width = at + c.numel(), c.shape[1]
+            check(pl, [flat[i:i + width] for i in range(at, end, width)])
+            at = end
     return (tuple(past_kv), masks) if return_masks else tuple(past_kv)

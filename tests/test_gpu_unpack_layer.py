@@ -88,7 +88,7 @@ def test_counts_that_do_not_fit_the_layer_are_reported():
     counts = pl.seg_bounds_per_head.clone()
     counts[:, 0] += 100                                          # more 2-bit tokens than the segment has, sums alike
     pl.seg_bounds_per_head, pl.T_eff_per_head = counts, pl.T_eff_per_head + 100
-    with pytest.raises(AssertionError, match="V segment"):
+    with pytest.raises(AssertionError, match="V segments"):
         tz._unpack_v_perhead(pl, head_dim=128)
     counts = pl.K_ch_seg_bounds_per_head.clone()
     counts[:, 0] += 200                                          # more 2-bit channels than the segment has
