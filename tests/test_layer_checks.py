@@ -1,0 +1,85 @@
+"""What the attention and dequantize entry points refuse before they launch anything, without a device:
+the library is a recorder, host tensors play the device's and ``meta`` tensors those of another one.
+The kernels take addresses, so a shape or device that slips through is a read or write out of range."""
+import dataclasses
+
+import pytest
+import torch
+
+from rdkv_amd import _lib, fast_decode, packing, trizone_decompress as tz
+
+
+class _Recorder:
+    """Stands for the library: every entry point succeeds and is noted down."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        def call(*args):
+            self.calls.append(name)
+            return 0
+        return call
+
+
+def _one_device(*tensors):
+    devices = {t.device.type for t in tensors if t is not None}
+    if devices != {"cpu"}:
+        raise RuntimeError(f"tensors on different devices: {devices}")
+    return torch.device("cpu")
+
+
+@pytest.fixture
+def lib(monkeypatch):
+    recorder = _Recorder()
+    monkeypatch.setattr(_lib, "load", lambda: recorder)
+    monkeypatch.setattr(_lib, "available", lambda: True)
+    monkeypatch.setattr(_lib, "require_device", _one_device)
+    monkeypatch.setattr(_lib, "stream_of", lambda dev: 0)
+    monkeypatch.setattr(_lib, "workspace", lambda dev, n: torch.empty(64, dtype=torch.uint8))
+    monkeypatch.setattr(_lib, "download", lambda t: t.numpy())
+    return recorder
+
+
+def _layer(H=2, T=6, D=128, G=4, n16=3, n_k=(4, 6, 5), per_head=True):
+    """A layer of T packed and n16 fp16 tokens per head, n_k channels per class, as the packers lay it out."""
+    def codes(rows, width):
+        return torch.zeros(1, H, rows, width, dtype=torch.uint8)
+
+    def full(n):
+        return torch.full((H,), n, dtype=torch.int32)
+
+    v = (T - 2 * (T // 3), T // 3, T // 3)
+    widths = (packing._seg_padded_len(n_k[0], 4), packing._seg_padded_len(n_k[1], 2), n_k[2])
+    rows, kept = T + n16, sum(n_k)
+    sort = torch.arange(kept).expand(H, kept).contiguous()
+    layer = packing.PackedKVLayer(
+        K_2bit=codes(rows, widths[0] // 4), K_4bit=codes(rows, widths[1] // 2), K_8bit=codes(rows, widths[2]),
+        K_ch_scale=torch.ones(1, H, 1, sum(widths)).half(), K_ch_zp=torch.zeros(1, H, 1, sum(widths)).half(),
+        K_ch_sort_idx=sort[0], K_ch_seg_bounds=n_k, K_ch_perm_padded_idx=torch.zeros(sum(widths), dtype=torch.long),
+        V_2bit=codes(v[0], D // 4), V_4bit=codes(v[1], D // 2), V_8bit=codes(v[2], D),
+        V_scale=torch.ones(1, H, T, 1).half(), V_zp=torch.zeros(1, H, T, 1).half(),
+        sort_idx=torch.zeros(T, dtype=torch.long), seg_bounds=v, T_eff=T, T_eff_k=rows, n_v16=n16)
+    if per_head:
+        layer = dataclasses.replace(
+            layer, seg_bounds_per_head=torch.tensor([v] * H, dtype=torch.int32), T_eff_per_head=full(T),
+            K_ch_sort_idx_per_head=sort, K_ch_seg_bounds_per_head=torch.tensor([n_k] * H, dtype=torch.int32),
+            T_eff_k_per_head=full(rows), n_v16_per_head=full(n16))
+    return layer
+
+
+def _attend(layer, lib, H_q=8, H_kv=2, n=5, G=4, width=128, **kw):
+    kv = torch.zeros(H_kv, n, 128)
+    v16 = torch.zeros(layer.K_ch_scale.shape[1], int(layer.n_v16), 128).half()
+    return fast_decode.trizone_attention(torch.zeros(H_q, width), layer, v16, layer.n_v16_per_head, kv, kv, G, **kw)
+
+
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("rows", [4, 7, 16])
+def test_attention_refuses_an_output_of_other_height(lib, packed, rows):
+    layer = _layer() if packed else dataclasses.replace(_layer(), T_eff=0, T_eff_k=0)
+    with pytest.raises(RuntimeError):
+        _attend(layer, lib, out=torch.empty(rows, 128))
+    assert not packed or lib.calls == []
+    _attend(layer, lib, out=torch.empty(8, 128))
+    assert any(name.startswith("rdkv_v_weighted_sum") for name in lib.calls)
