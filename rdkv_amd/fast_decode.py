@@ -229,6 +229,10 @@ def trizone_attention(q_2d: torch.Tensor, sp: PackedKVLayer, V16: Optional[torch
                            f"got {tuple(scores_buf.shape)} {scores_buf.dtype}")
     if out.shape != (H_q, D):
         raise RuntimeError(f"out must be [{H_q}, {D}], got {tuple(out.shape)}")
+    if T_old > 0:
+        layer_heads = sp.V_scale.shape[1] if sp.V_scale.dim() == 4 else sp.V_scale.shape[0]
+        if layer_heads != H_kv:
+            raise RuntimeError(f"{H_q} query heads in groups of {num_kv_groups} over a layer of {layer_heads} KV heads")
     if q_2d.dtype not in _lib.DTYPE_CODE or q_2d.stride(1) != 1:
         q_2d = q_2d.float().contiguous()
     K_new, V_new = (_new_zone_rows(t, H_kv, n_new) for t in (K_new, V_new))

@@ -83,3 +83,20 @@ def test_attention_refuses_an_output_of_other_height(lib, packed, rows):
     assert not packed or lib.calls == []
     _attend(layer, lib, out=torch.empty(8, 128))
     assert any(name.startswith("rdkv_v_weighted_sum") for name in lib.calls)
+
+
+@pytest.mark.parametrize("H_q,G,H_kv", [(8, 4, 2), (8, 2, 4), (16, 8, 2), (4, 4, 1)])
+def test_attention_refuses_groups_that_do_not_fit_the_layer(lib, H_q, G, H_kv):
+    """The V launch walks the layer's KV heads through the appended values: both must have as many."""
+    fits = _layer(H=H_kv)
+    for layer in (fits, fast_decode._pre_squeeze_packed((fits,))[0]):
+        _attend(layer, lib, H_q=H_q, H_kv=H_kv, G=G)
+    lib.calls.clear()
+    for H in (1, 2, 4, 8):
+        if H == H_kv or H_q % H:
+            continue
+        other = _layer(H=H)
+        for layer in (other, fast_decode._pre_squeeze_packed((other,))[0]):
+            with pytest.raises(RuntimeError):
+                _attend(layer, lib, H_q=H_q, H_kv=H_kv, G=G)
+    assert lib.calls == []
