@@ -70,7 +70,7 @@ def _layer(H=2, T=6, D=128, G=4, n16=3, n_k=(4, 6, 5), per_head=True):
 
 def _attend(layer, lib, H_q=8, H_kv=2, n=5, G=4, width=128, **kw):
     kv = torch.zeros(H_kv, n, 128)
-    v16 = torch.zeros(layer.K_ch_scale.shape[1], int(layer.n_v16), 128).half()
+    v16 = torch.zeros(layer.n_v16_per_head.numel(), int(layer.n_v16), 128).half()
     return fast_decode.trizone_attention(torch.zeros(H_q, width), layer, v16, layer.n_v16_per_head, kv, kv, G, **kw)
 
 
