@@ -227,6 +227,8 @@ def trizone_attention(q_2d: torch.Tensor, sp: PackedKVLayer, V16: Optional[torch
             or scores_buf.dtype != torch.float32 or scores_buf.stride(1) != 1:
         raise RuntimeError(f"scores_buf must be fp32 [{H_q}, >= {T_old + n_new}] with unit column stride, "
                            f"got {tuple(scores_buf.shape)} {scores_buf.dtype}")
+    if D != 128:
+        raise RuntimeError(f"query rows of 128 channels expected, got {D}")
     if out.shape != (H_q, D):
         raise RuntimeError(f"out must be [{H_q}, {D}], got {tuple(out.shape)}")
     if T_old > 0:

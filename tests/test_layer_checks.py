@@ -100,3 +100,15 @@ def test_attention_refuses_groups_that_do_not_fit_the_layer(lib, H_q, G, H_kv):
             with pytest.raises(RuntimeError):
                 _attend(layer, lib, H_q=H_q, H_kv=H_kv, G=G)
     assert lib.calls == []
+
+
+@pytest.mark.parametrize("width", [64, 127, 129, 256])
+@pytest.mark.parametrize("packed", [True, False])
+def test_attention_refuses_queries_of_other_width(lib, packed, width):
+    """The scores of the appended tokens read 128 channels of every query row."""
+    layer = _layer() if packed else dataclasses.replace(_layer(), T_eff=0, T_eff_k=0)
+    with pytest.raises((RuntimeError, AssertionError)):
+        _attend(layer, lib, width=width)
+    with pytest.raises((RuntimeError, AssertionError)):
+        _attend(layer, lib, width=width, out=torch.empty(8, 128))
+    assert lib.calls == []
