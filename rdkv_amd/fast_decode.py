@@ -210,7 +210,7 @@ def trizone_attention(q_2d: torch.Tensor, sp: PackedKVLayer, V16: Optional[torch
     fp16 or None; K_new / V_new [H_kv, n_new, 128] fp32 including the current token (n_new >= 1).
     Returns fp32 [H_q,128].  ``scores_buf`` [H_q, >= T_old + n_new] fp32 and ``out`` may be
     passed to avoid allocations (e.g. under graph capture)."""
-    dev = _lib.require_device(q_2d, K_new, V_new)
+    dev = _lib.require_device(q_2d, K_new, V_new, scores_buf, out)
     lib = _lib.load()
     H_q, D = q_2d.shape
     H_kv = H_q // num_kv_groups

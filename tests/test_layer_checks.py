@@ -112,3 +112,11 @@ def test_attention_refuses_queries_of_other_width(lib, packed, width):
     with pytest.raises((RuntimeError, AssertionError)):
         _attend(layer, lib, width=width, out=torch.empty(8, 128))
     assert lib.calls == []
+
+
+@pytest.mark.parametrize("name,shape", [("out", (8, 128)), ("scores_buf", (8, 16))])
+def test_attention_refuses_buffers_of_another_device(lib, name, shape):
+    layer = dataclasses.replace(_layer(), T_eff=0, T_eff_k=0)
+    with pytest.raises(RuntimeError):
+        _attend(layer, lib, **{name: torch.empty(shape, device="meta")})
+    assert lib.calls == []
