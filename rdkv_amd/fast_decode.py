@@ -229,9 +229,9 @@ def trizone_attention(q_2d: torch.Tensor, sp: PackedKVLayer, V16: Optional[torch
                            f"got {tuple(scores_buf.shape)} {scores_buf.dtype}")
     if D != 128:
         raise RuntimeError(f"query rows of 128 channels expected, got {D}")
-    if out.shape != (H_q, D):
-        raise RuntimeError(f"out must be [{H_q}, {D}], got {tuple(out.shape)}")
     if T_old > 0:
+        if out.shape != (H_q, D):
+            raise RuntimeError(f"out must be [{H_q}, {D}], got {tuple(out.shape)}")
         layer_heads = sp.V_scale.shape[1] if sp.V_scale.dim() == 4 else sp.V_scale.shape[0]
         if layer_heads != H_kv:
             raise RuntimeError(f"{H_q} query heads in groups of {num_kv_groups} over a layer of {layer_heads} KV heads")

@@ -221,10 +221,12 @@ def _weighted_sum_with_new_zone(attn_weights_old, packed_layer, out, V16, n_v16_
     if per_head is None:
         V16 = None
     if pl is None or (sum(int(v) for v in pl.seg_bounds) == 0 and V16 is None):
-        res = out if out.dtype == torch.float32 and out.stride(1) == 1 else torch.empty(out.shape, device=out.device)
+        rows = attn_weights_old.shape[0]
+        fits = out.shape == (rows, D) and out.dtype == torch.float32 and out.stride(1) == 1
+        res = out if fits else torch.empty(rows, D, dtype=torch.float32, device=out.device)
         _launch(attn_weights_old, None, None, None, None, None, None, (0, 0, 0), res, None, None, 0, new)
-        if res is not out:
-            out.copy_(res)
+        if not fits:
+            out.zero_().add_(res)
     else:
         _launch(attn_weights_old, pl.V_2bit, pl.V_4bit, pl.V_8bit, pl.V_scale, pl.V_zp, per_head, pl.seg_bounds, out, V16,
                 n_v16_per_head, max_T_v if per_head is not None else 0, new)

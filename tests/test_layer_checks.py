@@ -69,7 +69,7 @@ def _layer(H=2, T=6, D=128, G=4, n16=3, n_k=(4, 6, 5), per_head=True):
 
 
 def _attend(layer, lib, H_q=8, H_kv=2, n=5, G=4, width=128, **kw):
-    kv = torch.zeros(H_kv, n, 128)
+    kv = torch.zeros(H_kv, n, 128, dtype=torch.float32)
     v16 = torch.zeros(layer.n_v16_per_head.numel(), int(layer.n_v16), 128).half()
     return fast_decode.trizone_attention(torch.zeros(H_q, width), layer, v16, layer.n_v16_per_head, kv, kv, G, **kw)
 
@@ -120,3 +120,19 @@ def test_attention_refuses_buffers_of_another_device(lib, name, shape):
     with pytest.raises(RuntimeError):
         _attend(layer, lib, **{name: torch.empty(shape, device="meta")})
     assert lib.calls == []
+
+
+@pytest.mark.parametrize("make", [lambda: torch.empty(8, 128, dtype=torch.float16), lambda: torch.empty(1, 8, 128),
+                                  lambda: torch.empty(3, 8, 128, dtype=torch.float64), lambda: torch.empty(128, 8).t()])
+@pytest.mark.parametrize("default", [torch.float32, torch.float64, torch.bfloat16])
+def test_attention_without_packed_tokens_fills_outputs_of_any_kind(lib, make, default):
+    """The sum goes to a tensor of the kernel's form and from there to what the caller gave."""
+    layer, out = dataclasses.replace(_layer(), T_eff=0, T_eff_k=0), make()
+    torch.set_default_dtype(default)
+    try:
+        assert _attend(layer, lib, out=out) is out
+    finally:
+        torch.set_default_dtype(torch.float32)
+    assert "rdkv_v_weighted_sum_new_values" in lib.calls
+    with pytest.raises(RuntimeError):
+        _attend(layer, lib, out=torch.empty(8, 128, dtype=torch.int64))
