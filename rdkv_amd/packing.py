@@ -347,6 +347,8 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
     the device and are yet to be checked against the segments (``_check_k_counts``)."""
     if packed.K_ch_scale is None:
         raise ValueError("unpack_k_mixed: K_ch_scale missing")
+    per_head = packed.K_ch_seg_bounds_per_head is not None
+    sort = packed.K_ch_sort_idx_per_head if per_head else packed.K_ch_sort_idx
     dev = _lib.require_device(packed.K_ch_scale)
     H = packed.K_ch_scale.shape[1]
     T = packed.T_eff_k if packed.T_eff_k > 0 else packed.T_eff
@@ -357,27 +359,36 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
         if t is None or w == 0:
             segs.append((None, 0, 0, 0))
             continue
+        if t.dim() != 4 or t.shape[1] < H or t.shape[2:] != (T, w * bits // 8):
+            raise RuntimeError(f"K segment {tuple(t.shape)} for {H} heads, {T} tokens, {w} channels")
         t = t if t.stride(3) == 1 else t.contiguous()
-        assert t.shape[1:] == (H, T, w * bits // 8), f"K segment {tuple(t.shape)} for {H} heads, {T} tokens, {w} channels"
         segs.append((t, t.stride(1), t.stride(2), w))
     if not any(s[3] for s in segs):
         return torch.zeros(1, H, T, D, dtype=torch.float16, device=dev), None
+    (K2, k2h, k2t, w2), (K4, k4h, k4t, w4), (K8, k8h, k8t, w8) = segs
+    # everything the kernel indexes by head, slot and token, before it gets the addresses
     sc, zz = packed.K_ch_scale, packed.K_ch_zp
-    if sc.stride(3) != 1 or zz.stride() != sc.stride():
-        sc, zz = sc.contiguous(), zz.contiguous()
+    assert sort is not None, "per-head layout requires K_ch_sort_idx_per_head"
+    _lib.require_device(sc, zz, sort, K2, K4, K8)
+    Dp = sum(widths)
+    for t in (sc, zz):
+        if t.dim() != 4 or t.shape[1] < H or t.shape[3] < Dp:
+            raise RuntimeError(f"K scales / zero points {tuple(t.shape)} for {H} heads of {Dp} channels")
+    if sort.dtype != torch.long or sort.dim() != (2 if per_head else 1) or (per_head and sort.shape[0] < H):
+        raise RuntimeError(f"channel index {tuple(sort.shape)} {sort.dtype} for {H} heads")
+    if sc.shape != zz.shape or sc.stride(3) != 1 or zz.stride() != sc.stride():
+        sc, zz = (t[:1, :H, :1, :Dp].contiguous() for t in (sc, zz))
     counts, limits = None, tuple(n if s[3] else 0 for n, s in zip((m2, m4, m8), segs))
-    if packed.K_ch_seg_bounds_per_head is not None:
-        assert packed.K_ch_sort_idx_per_head is not None, "per-head layout requires K_ch_sort_idx_per_head"
-        counts = packed.K_ch_seg_bounds_per_head.to(device=dev, dtype=torch.int32).contiguous()
-        sort = packed.K_ch_sort_idx_per_head
+    if per_head:
+        counts = packed.K_ch_seg_bounds_per_head
+        if counts.dim() != 2 or counts.shape[0] < H or counts.shape[1] != 3:
+            raise RuntimeError(f"channel counts {tuple(counts.shape)} for {H} heads")
+        counts = counts[:H].to(device=dev, dtype=torch.int32).contiguous()
     else:
         assert limits == (m2, m4, m8), "a K segment is missing"
-        sort = packed.K_ch_sort_idx
-    sort = sort.to(torch.long)
     sort = sort if sort.stride(-1) == 1 else sort.contiguous()
     out = torch.empty(1, H, T, D, dtype=torch.float16, device=dev)
-    (K2, k2h, k2t, w2), (K4, k4h, k4t, w4), (K8, k8h, k8t, w8) = segs
-    if [w for w in (w2, w4, w8)] != list(widths):
+    if (w2, w4, w8) != widths:
         # slots of a missing segment do not exist: scales and zero points without their columns
         keep = torch.cat([torch.arange(o, o + w, device=dev) for o, w in
                           zip((0, widths[0], widths[0] + widths[1]), (w2, w4, w8))])

@@ -136,3 +136,54 @@ def test_attention_without_packed_tokens_fills_outputs_of_any_kind(lib, make, de
     assert "rdkv_v_weighted_sum_new_values" in lib.calls
     with pytest.raises(RuntimeError):
         _attend(layer, lib, out=torch.empty(8, 128, dtype=torch.int64))
+
+
+def _cut(t, dim, n=1):
+    return t.narrow(dim, 0, t.shape[dim] - n)
+
+
+def _refused(lib, call, layer, **changes):
+    with pytest.raises((RuntimeError, IndexError)):
+        call(dataclasses.replace(layer, **changes))
+    assert not any(name.startswith("rdkv_unpack") for name in lib.calls), "refused behind the launch"
+
+
+K_TENSORS = ("K_2bit", "K_4bit", "K_8bit", "K_ch_scale", "K_ch_zp")
+
+
+@pytest.mark.parametrize("per_head", [True, False])
+def test_dense_keys_refuse_tensors_that_do_not_fit(lib, per_head):
+    layer = _layer(per_head=per_head)
+    index = "K_ch_sort_idx_per_head" if per_head else "K_ch_sort_idx"
+
+    def call(pl):
+        return packing._unpack_k_enqueue(pl, 128)
+
+    call(layer)
+    assert lib.calls == ["rdkv_unpack_layer_k"]
+    lib.calls.clear()
+    for name in K_TENSORS + (index,):
+        t = getattr(layer, name)
+        _refused(lib, call, layer, **{name: t.to("meta")})                      # of another device
+        if name != index:
+            _refused(lib, call, layer, **{name: _cut(t, 3)})                    # too few channels
+    for name in ("K_2bit", "K_4bit", "K_8bit"):
+        _refused(lib, call, layer, **{name: _cut(getattr(layer, name), 1)})     # too few heads
+        _refused(lib, call, layer, **{name: _cut(getattr(layer, name), 2)})     # too few tokens
+    _refused(lib, call, layer, K_ch_zp=_cut(layer.K_ch_zp, 1))
+    _refused(lib, call, layer, **{index: getattr(layer, index).int()})
+    if per_head:
+        _refused(lib, call, layer, K_ch_sort_idx_per_head=_cut(layer.K_ch_sort_idx_per_head, 0))
+        _refused(lib, call, layer, K_ch_seg_bounds_per_head=_cut(layer.K_ch_seg_bounds_per_head, 0))
+        _refused(lib, call, layer, K_ch_seg_bounds_per_head=_cut(layer.K_ch_seg_bounds_per_head, 1))
+
+
+def test_dense_keys_take_scales_and_counts_wider_than_needed(lib):
+    """As the layer's fields allow: only the padded channels and the heads that exist are read."""
+    layer = _layer()
+    wide = torch.nn.functional.pad
+    packing._unpack_k_enqueue(dataclasses.replace(
+        layer, K_ch_zp=wide(layer.K_ch_zp, (0, 7)), K_8bit=torch.cat([layer.K_8bit] * 2, dim=1),
+        K_ch_sort_idx_per_head=torch.cat([layer.K_ch_sort_idx_per_head] * 2),
+        K_ch_seg_bounds_per_head=wide(layer.K_ch_seg_bounds_per_head, (0, 0, 0, 1), value=99)), 128)
+    assert lib.calls == ["rdkv_unpack_layer_k"]
