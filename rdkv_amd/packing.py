@@ -386,6 +386,8 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
         counts = counts[:H].to(device=dev, dtype=torch.int32).contiguous()
     else:
         assert limits == (m2, m4, m8), "a K segment is missing"
+        if sort.shape[0] < sum(limits):
+            raise RuntimeError(f"{sum(limits)} channels kept, {sort.shape[0]} listed")
     sort = sort if sort.stride(-1) == 1 else sort.contiguous()
     out = torch.empty(1, H, T, D, dtype=torch.float16, device=dev)
     if (w2, w4, w8) != widths:

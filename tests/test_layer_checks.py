@@ -187,3 +187,11 @@ def test_dense_keys_take_scales_and_counts_wider_than_needed(lib):
         K_ch_sort_idx_per_head=torch.cat([layer.K_ch_sort_idx_per_head] * 2),
         K_ch_seg_bounds_per_head=wide(layer.K_ch_seg_bounds_per_head, (0, 0, 0, 1), value=99)), 128)
     assert lib.calls == ["rdkv_unpack_layer_k"]
+
+
+@pytest.mark.parametrize("listed", [0, 1, 14])
+def test_dense_keys_refuse_a_shared_index_that_lists_too_few_channels(lib, listed):
+    layer = _layer(per_head=False)                      # keeps 15 channels
+    _refused(lib, lambda pl: packing.unpack_k_mixed(pl, 128), layer, K_ch_sort_idx=layer.K_ch_sort_idx[:listed])
+    packing.unpack_k_mixed(dataclasses.replace(layer, K_ch_sort_idx=torch.arange(20)), 128)
+    assert lib.calls == ["rdkv_unpack_layer_k"]
