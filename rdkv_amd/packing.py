@@ -406,6 +406,7 @@ def _check_k_counts(packed: "PackedKVLayer", counts: Sequence[Sequence[int]]) ->
     m2, m4, m8 = packed.K_ch_seg_bounds
     widths = (_seg_padded_len(m2, 4), _seg_padded_len(m4, 2), m8)
     most = [max(column) for column in zip(*counts)]
+    assert min(map(min, counts)) >= 0, f"heads keep a negative number of channels: {counts}"
     for n, t in zip(most, (packed.K_2bit, packed.K_4bit, packed.K_8bit)):
         assert n == 0 or t is not None, f"a head keeps {n} channels of a K segment that is missing"
     assert all(n <= w for n, w in zip(most, widths)), f"heads keep {most} channels of K segments of {widths}"

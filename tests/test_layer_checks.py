@@ -195,3 +195,12 @@ def test_dense_keys_refuse_a_shared_index_that_lists_too_few_channels(lib, liste
     _refused(lib, lambda pl: packing.unpack_k_mixed(pl, 128), layer, K_ch_sort_idx=layer.K_ch_sort_idx[:listed])
     packing.unpack_k_mixed(dataclasses.replace(layer, K_ch_sort_idx=torch.arange(20)), 128)
     assert lib.calls == ["rdkv_unpack_layer_k"]
+
+
+@pytest.mark.parametrize("counts", [(-2, 6, 5), (4, -1, 5), (4, 6, -3), (-4, 6, 9)])
+def test_dense_keys_report_negative_counts(lib, counts):
+    layer = _layer()
+    bad = layer.K_ch_seg_bounds_per_head.clone()
+    bad[1] = torch.tensor(counts)
+    with pytest.raises(AssertionError, match="negative"):
+        packing.unpack_k_mixed(dataclasses.replace(layer, K_ch_seg_bounds_per_head=bad), 128)
