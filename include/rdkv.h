@@ -142,6 +142,15 @@ int rdkv_unpack_layer_k(const uint8_t *K2, int64_t k2_stride_h, int64_t k2_strid
                         const int64_t *sort_idx, int64_t sort_stride_h, int sort_n, const int32_t *counts,
                         int n2, int n4, int n8, int n2p, int n4p, int n8w, int H_kv, int64_t T, int D,
                         void *out_f16, void *stream);
+/* The same; check, device int32 [H_kv, 4], gets per head the three counts as the launch read them and
+ * whether one of the kept channels is outside 0 .. D - 1 (such a channel is dropped).  T > 0. */
+int rdkv_unpack_layer_k_checked(const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t,
+                                const uint8_t *K4, int64_t k4_stride_h, int64_t k4_stride_t,
+                                const uint8_t *K8, int64_t k8_stride_h, int64_t k8_stride_t,
+                                const void *scale_f16, const void *zp_f16, int64_t ks_stride_h,
+                                const int64_t *sort_idx, int64_t sort_stride_h, int sort_n,
+                                const int32_t *counts, int n2, int n4, int n8, int n2p, int n4p, int n8w, int H_kv,
+                                int64_t T, int D, void *out_f16, int32_t *check, void *stream);
 int rdkv_unpack_layer_v(const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h,
                         const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
                         int64_t s_stride_h, const int32_t *counts, int m2, int m4, int m8, int64_t max_tv,

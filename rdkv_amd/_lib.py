@@ -55,6 +55,7 @@ SIGNATURES = {
     "rdkv_pack_layer_k_rows": (I, [P, L, L, I, I, P, L, P, L, I, P, I, I, I, P, P, P, P, P, P, I, P]),
     "rdkv_dequant_f16": (I, [P, L, I, I, P, P, I, P, L, P]),
     "rdkv_unpack_layer_k": (I, [P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, P, I, I, I, I, I, I, I, L, I, P, P]),
+    "rdkv_unpack_layer_k_checked": (I, [P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, P, I, I, I, I, I, I, I, L, I, P, P, P]),
     "rdkv_unpack_layer_v": (I, [P, L, P, L, P, L, P, P, L, P, I, I, I, L, P, L, I, I, I, P, P]),
     "rdkv_k_qk_dot": (I, [P, I, L, I, I, P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, I, I, L, P, L, P]),
     "rdkv_softmax_rows": (I, [P, L, P, L, L, P, L, L, P, L, P, L, I, P]),

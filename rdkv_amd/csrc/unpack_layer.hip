@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(256)
 unpack_k_kernel(KSeg s2, KSeg s4, KSeg s8, const __half *__restrict__ scale, const __half *__restrict__ zp,
                 int64_t ks_sh, const int64_t *__restrict__ sort_idx, int64_t sort_sh, int sort_n,
                 const int32_t *__restrict__ counts, int c2, int c4, int c8, int64_t T, int D, int rows,
-                uint16_t *__restrict__ out) {
+                uint16_t *__restrict__ out, int32_t *__restrict__ check) {
   extern __shared__ __attribute__((aligned(16))) uint8_t s_rows[];
   // per channel: where its code lies in a row (LDS offset | segment << 16 | shift << 18) and
   // its scale | zero point
@@ -81,14 +81,20 @@ unpack_k_kernel(KSeg s2, KSeg s4, KSeg s8, const __half *__restrict__ scale, con
     n8 = counts[3 * h + 2];
   }
   // (counts of a tensor that was overwritten must not lead outside the rows; the host reports them)
+  if (check && blockIdx.x == 0 && blockIdx.z == 0 && tid == 0) {
+    check[4 * h] = n2;
+    check[4 * h + 1] = n4;
+    check[4 * h + 2] = n8;
+  }
   n2 = min(max(n2, 0), n2p);
   n4 = min(max(n4, 0), n4p);
   n8 = min(max(n8, 0), s8.sub);
   const int kept = min(n2 + n4 + n8, sort_n);
   __syncthreads();
-  bool whole = true;
+  bool whole = true, outside = false;
   for (int i = tid; i < kept; i += 256) {
     const int64_t ch = sort_idx[h * sort_sh + i] - ch0;
+    outside = outside || ch + ch0 < 0 || ch + ch0 >= D;
     const int slot = i < n2 ? i : i < n2 + n4 ? n2p + (i - n2) : n2p + n4p + (i - n2 - n4);
     const __half sc = scale[h * ks_sh + slot], zz = zp[h * ks_sh + slot];
     uint32_t at;
@@ -104,6 +110,10 @@ unpack_k_kernel(KSeg s2, KSeg s4, KSeg s8, const __half *__restrict__ scale, con
     whole = whole && whole_zp(__half2float(zz));
   }
   whole = __syncthreads_and(whole);
+  if (check && blockIdx.x == 0 && blockIdx.z == 0) {
+    outside = __syncthreads_or(outside);
+    if (tid == 0) check[4 * h + 3] = outside ? 1 : 0;
+  }
   const int oct = tid & 15, c0 = 8 * oct;
   int at[8], step[8], seg[8], shift[8], width[8];
   uint32_t sz[8];
@@ -278,12 +288,12 @@ unpack_v_kernel(const uint8_t *__restrict__ V2, int64_t v2_sh, const uint8_t *__
 
 }  // namespace
 
-RDKV_API int rdkv_unpack_layer_k(const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t, const uint8_t *K4,
-                                 int64_t k4_stride_h, int64_t k4_stride_t, const uint8_t *K8, int64_t k8_stride_h,
-                                 int64_t k8_stride_t, const void *scale_f16, const void *zp_f16, int64_t ks_stride_h,
-                                 const int64_t *sort_idx, int64_t sort_stride_h, int sort_n, const int32_t *counts,
-                                 int n2, int n4, int n8, int n2p, int n4p, int n8w, int H_kv, int64_t T, int D,
-                                 void *out_f16, void *stream) {
+static int unpack_layer_k(const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t, const uint8_t *K4,
+                          int64_t k4_stride_h, int64_t k4_stride_t, const uint8_t *K8, int64_t k8_stride_h,
+                          int64_t k8_stride_t, const void *scale_f16, const void *zp_f16, int64_t ks_stride_h,
+                          const int64_t *sort_idx, int64_t sort_stride_h, int sort_n, const int32_t *counts, int n2,
+                          int n4, int n8, int n2p, int n4p, int n8w, int H_kv, int64_t T, int D, void *out_f16,
+                          int32_t *check, void *stream) {
   RDKV_REQUIRE(H_kv >= 1 && H_kv <= 65535 && T >= 0 && D >= 1 && D <= 65535 * kChan, "rdkv_unpack_layer_k: bad shape");
   RDKV_REQUIRE(n2p >= 0 && n2p % 4 == 0 && n4p >= 0 && n4p % 2 == 0 && n8w >= 0 && sort_n >= 0,
                "rdkv_unpack_layer_k: bad segment widths %d/%d/%d", n2p, n4p, n8w);
@@ -307,9 +317,32 @@ RDKV_API int rdkv_unpack_layer_k(const uint8_t *K2, int64_t k2_stride_h, int64_t
   dim3 g((unsigned)per_head, H_kv, chunks);
   hipLaunchKernelGGL(dense ? unpack_k_kernel<true> : unpack_k_kernel<false>, g, dim3(256), lds, (hipStream_t)stream, s2, s4,
                      s8, (const __half *)scale_f16, (const __half *)zp_f16, ks_stride_h, sort_idx, sort_stride_h, sort_n,
-                     counts, n2, n4, n8, T, D, rows, (uint16_t *)out_f16);
+                     counts, n2, n4, n8, T, D, rows, (uint16_t *)out_f16, check);
   RDKV_CHECK_LAUNCH("rdkv_unpack_layer_k");
   return RDKV_OK;
+}
+
+RDKV_API int rdkv_unpack_layer_k(const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t, const uint8_t *K4,
+                                 int64_t k4_stride_h, int64_t k4_stride_t, const uint8_t *K8, int64_t k8_stride_h,
+                                 int64_t k8_stride_t, const void *scale_f16, const void *zp_f16, int64_t ks_stride_h,
+                                 const int64_t *sort_idx, int64_t sort_stride_h, int sort_n, const int32_t *counts,
+                                 int n2, int n4, int n8, int n2p, int n4p, int n8w, int H_kv, int64_t T, int D,
+                                 void *out_f16, void *stream) {
+  return unpack_layer_k(K2, k2_stride_h, k2_stride_t, K4, k4_stride_h, k4_stride_t, K8, k8_stride_h, k8_stride_t, scale_f16,
+                        zp_f16, ks_stride_h, sort_idx, sort_stride_h, sort_n, counts, n2, n4, n8, n2p, n4p, n8w, H_kv, T, D,
+                        out_f16, nullptr, stream);
+}
+
+RDKV_API int rdkv_unpack_layer_k_checked(
+    const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t, const uint8_t *K4, int64_t k4_stride_h,
+    int64_t k4_stride_t, const uint8_t *K8, int64_t k8_stride_h, int64_t k8_stride_t, const void *scale_f16,
+    const void *zp_f16, int64_t ks_stride_h, const int64_t *sort_idx, int64_t sort_stride_h, int sort_n,
+    const int32_t *counts, int n2, int n4, int n8, int n2p, int n4p, int n8w, int H_kv, int64_t T, int D, void *out_f16,
+    int32_t *check, void *stream) {
+  RDKV_REQUIRE(check && T > 0, "rdkv_unpack_layer_k_checked: nothing to check into or no rows");
+  return unpack_layer_k(K2, k2_stride_h, k2_stride_t, K4, k4_stride_h, k4_stride_t, K8, k8_stride_h, k8_stride_t, scale_f16,
+                        zp_f16, ks_stride_h, sort_idx, sort_stride_h, sort_n, counts, n2, n4, n8, n2p, n4p, n8w, H_kv, T, D,
+                        out_f16, check, stream);
 }
 
 RDKV_API int rdkv_unpack_layer_v(const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h,

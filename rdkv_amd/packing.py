@@ -343,8 +343,10 @@ def _dequant(packed: Tensor, ncols: int, n_bits: int, scale: Tensor, zp: Tensor,
 
 
 def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional[Tensor]]:
-    """``unpack_k_mixed`` as one launch: the dense rows, and the per-head class counts that were read on
-    the device and are yet to be checked against the segments (``_check_k_counts``)."""
+    """``unpack_k_mixed`` as one launch: the dense rows and, of a per-head layer, what the launch found of every
+    head: the class counts and whether a kept channel is outside the head dimension, yet to be checked
+    (``_check_k_counts``).  A shared layer's call reads nothing back: its counts are the host's, and kept
+    channels outside the head dimension are left out."""
     if packed.K_ch_scale is None:
         raise ValueError("unpack_k_mixed: K_ch_scale missing")
     per_head = packed.K_ch_seg_bounds_per_head is not None
@@ -395,14 +397,21 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
         keep = torch.cat([torch.arange(o, o + w, device=dev) for o, w in
                           zip((0, widths[0], widths[0] + widths[1]), (w2, w4, w8))])
         sc, zz = sc.index_select(3, keep), zz.index_select(3, keep)
-    _lib.check(_lib.load().rdkv_unpack_layer_k(
-        _lib.ptr(K2), k2h, k2t, _lib.ptr(K4), k4h, k4t, _lib.ptr(K8), k8h, k8t, _lib.ptr(sc), _lib.ptr(zz), sc.stride(1),
-        _lib.ptr(sort), sort.stride(0) if sort.dim() == 2 else 0, int(sort.shape[-1]), _lib.ptr(counts), *limits,
-        w2, w4, w8, H, T, D, _lib.ptr(out), _lib.stream_of(dev)))
-    return out, counts
+    args = (_lib.ptr(K2), k2h, k2t, _lib.ptr(K4), k4h, k4t, _lib.ptr(K8), k8h, k8t, _lib.ptr(sc), _lib.ptr(zz), sc.stride(1),
+            _lib.ptr(sort), sort.stride(0) if per_head else 0, int(sort.shape[-1]), _lib.ptr(counts), *limits,
+            w2, w4, w8, H, T, D, _lib.ptr(out))
+    if not per_head:
+        _lib.check(_lib.load().rdkv_unpack_layer_k(*args, _lib.stream_of(dev)))
+        return out, None
+    if T == 0:
+        return out, torch.nn.functional.pad(counts, (0, 1))
+    check = torch.empty(H, 4, dtype=torch.int32, device=dev)
+    _lib.check(_lib.load().rdkv_unpack_layer_k_checked(*args, check.data_ptr(), _lib.stream_of(dev)))
+    return out, check
 
 
-def _check_k_counts(packed: "PackedKVLayer", counts: Sequence[Sequence[int]]) -> None:
+def _check_k_counts(packed: "PackedKVLayer", found: Sequence[Sequence[int]]) -> None:
+    counts = [row[:3] for row in found]
     m2, m4, m8 = packed.K_ch_seg_bounds
     widths = (_seg_padded_len(m2, 4), _seg_padded_len(m4, 2), m8)
     most = [max(column) for column in zip(*counts)]
@@ -412,13 +421,15 @@ def _check_k_counts(packed: "PackedKVLayer", counts: Sequence[Sequence[int]]) ->
     assert all(n <= w for n, w in zip(most, widths)), f"heads keep {most} channels of K segments of {widths}"
     kept, listed = max(map(sum, counts)), packed.K_ch_sort_idx_per_head.shape[-1]
     assert kept <= listed, f"a head keeps {kept} channels, {listed} are listed"
+    if any(row[3] for row in found):
+        raise IndexError(f"heads {[h for h, row in enumerate(found) if row[3]]} keep channels outside the head dimension")
 
 
 def unpack_k_mixed(packed: "PackedKVLayer", D: int) -> Tensor:
     """Dequantize packed K to fp16 [1,H_kv,T,D]; pruned channels are 0 (packing.py:581-709)."""
-    out, counts = _unpack_k_enqueue(packed, D)
-    if counts is not None:
-        _check_k_counts(packed, counts.tolist())
+    out, check = _unpack_k_enqueue(packed, D)
+    if check is not None:
+        _check_k_counts(packed, check.tolist())
     return out
 
 

@@ -96,11 +96,11 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
     shared-layout layers) (trizone_decompress.py:185-333)."""
     past_kv: List[Tuple[Tensor, Tensor]] = []
     masks: List[Optional[Tensor]] = []
-    unchecked = []        # (check, layer, per-head counts that the launches below read)
+    unchecked = []        # (check, layer, per-head counts as the launches below read them)
     for i, pl in enumerate(dual_cache.packed):
-        K_full, k_counts = _unpack_k_enqueue(pl, head_dim)
-        if k_counts is not None:
-            unchecked.append((_check_k_counts, pl, k_counts))
+        K_full, k_check = _unpack_k_enqueue(pl, head_dim)
+        if k_check is not None:
+            unchecked.append((_check_k_counts, pl, k_check))
         zone_b = dual_cache.new_v_only[i] if i < len(dual_cache.new_v_only) else None
         if _is_perhead_layout(pl):
             rows_b = None

@@ -95,3 +95,22 @@ def test_counts_that_do_not_fit_the_layer_are_reported():
     pl.K_ch_seg_bounds_per_head = counts
     with pytest.raises(AssertionError, match="K segments of"):
         packing.unpack_k_mixed(pl, D=128)
+
+
+@pytest.mark.parametrize("D", [128, 200])
+@pytest.mark.parametrize("channel", [-1, None, 1 << 40])
+def test_channels_outside_the_head_are_reported(D, channel):
+    """The kernel leaves such a channel out and says so; padding behind the kept channels is not looked at."""
+    require_gpu()
+    rng = np.random.default_rng(D)
+    K, V = (torch.from_numpy(rng.standard_normal((1, 3, 40, D)).astype(np.float16)).to(DEV) for _ in range(2))
+    vb, kb = torch.from_numpy(rng.choice(np.array([2, 4, 8]), size=(3, 40))), torch.full((3, D), 4)
+    kb[1, :50] = 0
+    pl, _ = packing.pack_layer_per_head(K, V, vb, kb, 2)
+    exp, index = packing.unpack_k_mixed(pl, D=D), pl.K_ch_sort_idx_per_head
+    pl.K_ch_sort_idx_per_head = index.clone()
+    pl.K_ch_sort_idx_per_head[1, D - 50:] = D if channel is None else channel
+    assert torch.equal(packing.unpack_k_mixed(pl, D=D), exp)
+    pl.K_ch_sort_idx_per_head[1, D - 51] = D if channel is None else channel
+    with pytest.raises(IndexError, match="1"):
+        packing.unpack_k_mixed(pl, D=D)

@@ -1,6 +1,7 @@
 """What the attention and dequantize entry points refuse before they launch anything, without a device:
 the library is a recorder, host tensors play the device's and ``meta`` tensors those of another one.
 The kernels take addresses, so a shape or device that slips through is a read or write out of range."""
+import ctypes
 import dataclasses
 
 import pytest
@@ -11,6 +12,17 @@ from rdkv_amd import _lib, fast_decode, packing, trizone_decompress as tz
 
 class _Recorder:
     """Stands for the library: every entry point succeeds and is noted down."""
+
+    def rdkv_unpack_layer_k_checked(self, *args):
+        """Writes what the launch reports: the counts, and whether a kept channel is outside the head."""
+        self.calls.append("rdkv_unpack_layer_k_checked")
+        sort, stride, counts, H, D, check = (args[i] for i in (12, 13, 15, 22, 24, 26))
+        counts, check = (ctypes.c_int32 * (3 * H)).from_address(counts), (ctypes.c_int32 * (4 * H)).from_address(check)
+        for h in range(H):
+            n = counts[3 * h:3 * h + 3]
+            kept = (ctypes.c_int64 * max(sum(n), 0)).from_address(sort + 8 * stride * h)
+            check[4 * h:4 * h + 4] = n + [int(any(c < 0 or c >= D for c in kept))]
+        return 0
 
     def __init__(self):
         self.calls = []
@@ -160,7 +172,7 @@ def test_dense_keys_refuse_tensors_that_do_not_fit(lib, per_head):
         return packing._unpack_k_enqueue(pl, 128)
 
     call(layer)
-    assert lib.calls == ["rdkv_unpack_layer_k"]
+    assert lib.calls == ["rdkv_unpack_layer_k_checked" if per_head else "rdkv_unpack_layer_k"]
     lib.calls.clear()
     for name in K_TENSORS + (index,):
         t = getattr(layer, name)
@@ -186,7 +198,7 @@ def test_dense_keys_take_scales_and_counts_wider_than_needed(lib):
         layer, K_ch_zp=wide(layer.K_ch_zp, (0, 7)), K_8bit=torch.cat([layer.K_8bit] * 2, dim=1),
         K_ch_sort_idx_per_head=torch.cat([layer.K_ch_sort_idx_per_head] * 2),
         K_ch_seg_bounds_per_head=wide(layer.K_ch_seg_bounds_per_head, (0, 0, 0, 1), value=99)), 128)
-    assert lib.calls == ["rdkv_unpack_layer_k"]
+    assert lib.calls == ["rdkv_unpack_layer_k_checked"]
 
 
 @pytest.mark.parametrize("listed", [0, 1, 14])
@@ -204,3 +216,16 @@ def test_dense_keys_report_negative_counts(lib, counts):
     bad[1] = torch.tensor(counts)
     with pytest.raises(AssertionError, match="negative"):
         packing.unpack_k_mixed(dataclasses.replace(layer, K_ch_seg_bounds_per_head=bad), 128)
+
+
+@pytest.mark.parametrize("channel", [-1, 128, 1 << 40])
+def test_dense_keys_report_channels_outside_the_head(lib, channel):
+    layer = _layer()
+    index = layer.K_ch_sort_idx_per_head.clone()
+    index[1, 7] = channel
+    cache = packing.TriZoneCache((dataclasses.replace(layer, K_ch_sort_idx_per_head=index),),
+                                 [torch.zeros(1, 2, 3, 128).half()], [None], [None], 9)
+    with pytest.raises(IndexError):
+        packing.unpack_k_mixed(cache.packed[0], 128)
+    with pytest.raises(IndexError):
+        tz.unpack_trizone_to_past_kv(cache, head_dim=128)
