@@ -385,7 +385,7 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
         counts = packed.K_ch_seg_bounds_per_head
         if counts.dim() != 2 or counts.shape[0] < H or counts.shape[1] != 3:
             raise RuntimeError(f"channel counts {tuple(counts.shape)} for {H} heads")
-        counts = counts[:H].to(device=dev, dtype=torch.int32).contiguous()
+        counts = (counts[:H] if counts.shape[0] > H else counts).to(device=dev, dtype=torch.int32).contiguous()
     else:
         assert limits == (m2, m4, m8), "a K segment is missing"
         if sort.shape[0] < sum(limits):

@@ -41,23 +41,35 @@ def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int
     (2-, 4-, 8-bit, all), yet to be checked (``_check_v_counts``)."""
     max_T_v = int(pl.T_eff)
     H_kv = pl.V_scale.shape[1]
-    dev = _lib.require_device(pl.V_scale)
-    counts = pl.seg_bounds_per_head.to(device=dev, dtype=torch.int32).contiguous()
-    check = torch.cat([counts, pl.T_eff_per_head.to(device=dev, dtype=torch.int32).reshape(H_kv, 1)], dim=1)
-    n16 = 0 if zone_b is None else int(zone_b.shape[2])
-    out = torch.empty(1, H_kv, max_T_v + n16, head_dim, dtype=torch.float16, device=dev)
+    # everything the kernel indexes by head, class row and token, before it gets the addresses
+    dev = _lib.require_device(pl.V_scale, pl.V_zp, pl.V_2bit, pl.V_4bit, pl.V_8bit, zone_b)
     segs = []
     for seg, bits in zip((pl.V_2bit, pl.V_4bit, pl.V_8bit), (2, 4, 8)):
         if seg is None or seg.numel() == 0:
             segs.append((None, 0, 0))
             continue
         width = head_dim * bits // 8
-        assert seg.shape[3] == width, f"V rows of {seg.shape[3]} bytes, expected {width}"
+        if seg.dim() != 4 or seg.shape[1] < H_kv or seg.shape[3] != width:
+            raise RuntimeError(f"V segment {tuple(seg.shape)} for {H_kv} heads, rows of {width} bytes")
         seg = seg if seg.stride(3) == 1 and seg.stride(2) == width else seg.contiguous()
         segs.append((seg, seg.stride(1), int(seg.shape[2])))
     sc, zp = pl.V_scale, pl.V_zp
-    if sc.numel() and not (sc.stride(2) == 1 and zp.stride() == sc.stride()):
-        sc, zp = sc.contiguous(), zp.contiguous()
+    rows = min(max_T_v, sum(m for _, _, m in segs))      # of a head, at most: the kernel clamps its counts to these
+    for t in (sc, zp):
+        if t.dim() < 3 or t.shape[1] < H_kv or t.shape[2] < rows:
+            raise RuntimeError(f"V scales / zero points {tuple(t.shape)} for {H_kv} heads of {rows} tokens")
+    if sc.numel() and not (sc.shape == zp.shape and sc.stride(2) == 1 and zp.stride() == sc.stride()):
+        sc, zp = (t[:1, :H_kv, :rows].contiguous() for t in (sc, zp))
+    counts, totals = pl.seg_bounds_per_head, pl.T_eff_per_head
+    if counts.dim() != 2 or counts.shape[0] < H_kv or counts.shape[1] != 3 or totals.numel() < H_kv:
+        raise RuntimeError(f"V counts {tuple(counts.shape)}, {tuple(totals.shape)} for {H_kv} heads")
+    if counts.shape[0] > H_kv or totals.numel() > H_kv:
+        counts, totals = counts[:H_kv], totals.reshape(-1)[:H_kv]
+    counts = counts.to(device=dev, dtype=torch.int32).contiguous()
+    totals = totals.to(device=dev, dtype=torch.int32).reshape(H_kv, 1)
+    check = torch.cat([counts, totals], dim=1)
+    n16 = 0 if zone_b is None else int(zone_b.shape[2])
+    out = torch.empty(1, H_kv, max_T_v + n16, head_dim, dtype=torch.float16, device=dev)
     if zone_b is not None and not (zone_b.stride(3) == 1 and zone_b.stride(2) == head_dim):
         zone_b = zone_b.contiguous()
     (V2, v2h, m2), (V4, v4h, m4), (V8, v8h, m8) = segs

@@ -229,3 +229,42 @@ def test_dense_keys_report_channels_outside_the_head(lib, channel):
         packing.unpack_k_mixed(cache.packed[0], 128)
     with pytest.raises(IndexError):
         tz.unpack_trizone_to_past_kv(cache, head_dim=128)
+
+
+V_SEGMENTS = ("V_2bit", "V_4bit", "V_8bit")
+
+
+def test_dense_values_refuse_tensors_that_do_not_fit(lib):
+    layer = _layer()
+
+    def call(pl):
+        return tz._unpack_v_enqueue(pl, None, 128)
+
+    call(layer)
+    assert lib.calls == ["rdkv_unpack_layer_v"]
+    lib.calls.clear()
+    for name in V_SEGMENTS + ("V_scale", "V_zp"):
+        t = getattr(layer, name)
+        _refused(lib, call, layer, **{name: t.to("meta")})                      # of another device
+        if name != "V_scale":                                                   # (says how many heads there are)
+            _refused(lib, call, layer, **{name: _cut(t, 1)})                    # too few heads
+    for name in V_SEGMENTS:
+        _refused(lib, call, layer, **{name: getattr(layer, name)[0]})
+        _refused(lib, call, layer, **{name: torch.nn.functional.pad(getattr(layer, name), (0, 1))})
+    for name in ("V_scale", "V_zp"):
+        _refused(lib, call, layer, **{name: _cut(getattr(layer, name), 2)})     # fewer tokens than the stripe
+    for name in ("seg_bounds_per_head", "T_eff_per_head"):
+        _refused(lib, call, layer, **{name: _cut(getattr(layer, name), 0)})
+    _refused(lib, call, layer, seg_bounds_per_head=_cut(layer.seg_bounds_per_head, 1))
+    with pytest.raises(RuntimeError):
+        tz._unpack_v_enqueue(layer, torch.zeros(1, 2, 3, 128, device="meta").half(), 128)
+
+
+def test_dense_values_take_tensors_wider_than_needed(lib):
+    layer = _layer()
+    wide = torch.nn.functional.pad
+    _, check = tz._unpack_v_enqueue(dataclasses.replace(
+        layer, V_zp=wide(layer.V_zp, (0, 0, 0, 5)), V_4bit=torch.cat([layer.V_4bit] * 2, dim=1),
+        seg_bounds_per_head=wide(layer.seg_bounds_per_head, (0, 0, 0, 1), value=99),
+        T_eff_per_head=wide(layer.T_eff_per_head, (0, 1))), None, 128)
+    assert lib.calls == ["rdkv_unpack_layer_v"] and check.shape == (2, 4)
