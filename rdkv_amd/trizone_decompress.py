@@ -81,12 +81,14 @@ def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int
 
 
 def _check_v_counts(pl: PackedKVLayer, counts) -> None:
-    rows = [seg.shape[2] if seg is not None else n for n, seg in zip(map(max, zip(*counts)), (pl.V_2bit, pl.V_4bit, pl.V_8bit))]
-    r2, r4, r8 = rows
-    for h, (n2, n4, n8, n) in enumerate(counts):
-        assert n2 + n4 + n8 == n, f"head {h}: seg_bounds_per_head {[n2, n4, n8]} != T_eff_per_head {n}"
-        assert n2 <= r2 and n4 <= r4 and n8 <= r8, f"head {h}: {[n2, n4, n8]} tokens in V segments of {rows}"
-        assert n <= pl.T_eff, f"head {h}: {n} tokens in a stripe of {pl.T_eff}"
+    rows = [None if seg is None else int(seg.shape[2]) for seg in (pl.V_2bit, pl.V_4bit, pl.V_8bit)]
+    for h, (*classes, n) in enumerate(counts):
+        assert sum(classes) == n, f"head {h}: seg_bounds_per_head {classes} != T_eff_per_head {n}"
+        # rows that are there: tokens of a class without a tensor are left out, a negative count has none
+        there = [max(c, 0) for c, r in zip(classes, rows) if r is not None]
+        assert all(c <= r for c, r in zip(there, (r for r in rows if r is not None))), \
+            f"head {h}: {classes} tokens in V segments of {rows}"
+        assert sum(there) <= pl.T_eff, f"head {h}: {classes} tokens in a stripe of {pl.T_eff}"
 
 
 def _unpack_v_perhead(pl: PackedKVLayer, *, head_dim: int) -> Tensor:

@@ -268,3 +268,25 @@ def test_dense_values_take_tensors_wider_than_needed(lib):
         seg_bounds_per_head=wide(layer.seg_bounds_per_head, (0, 0, 0, 1), value=99),
         T_eff_per_head=wide(layer.T_eff_per_head, (0, 1))), None, 128)
     assert lib.calls == ["rdkv_unpack_layer_v"] and check.shape == (2, 4)
+
+
+@pytest.mark.parametrize("counts,total", [((-3, 4, 5), 6), ((4, -3, 5), 6), ((4, 5, -3), 6), ((-9, 4, 5), 0)])
+def test_dense_values_report_more_rows_than_the_stripe(lib, counts, total):
+    """A negative count adds no rows, so counts with the right sum may still have more rows than fit."""
+    layer = dataclasses.replace(_layer(T=6), **{n: torch.zeros(1, 2, 6, w, dtype=torch.uint8)
+                                                for n, w in zip(V_SEGMENTS, (32, 64, 128))})
+    bounds, totals = layer.seg_bounds_per_head.clone(), layer.T_eff_per_head.clone()
+    bounds[1], totals[1] = torch.tensor(counts), total
+    bad = dataclasses.replace(layer, seg_bounds_per_head=bounds, T_eff_per_head=totals)
+    with pytest.raises(AssertionError):
+        tz._unpack_v_perhead(bad, head_dim=128)
+
+
+def test_dense_values_of_a_layer_without_a_class_tensor(lib):
+    """Tokens counted for a class that has no rows are left out; the rows behind them decide what fits."""
+    layer = dataclasses.replace(_layer(T=6), V_2bit=None)                       # 2, 2 and 2 tokens
+    out = tz._unpack_v_perhead(layer, head_dim=128)
+    assert out.shape == (1, 2, 6, 128)
+    counts = torch.tensor([[7, 2, 2]] * 2, dtype=torch.int32)
+    tz._unpack_v_perhead(dataclasses.replace(layer, seg_bounds_per_head=counts,
+                                             T_eff_per_head=counts.sum(1, dtype=torch.int32)), head_dim=128)
