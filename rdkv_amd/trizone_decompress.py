@@ -101,6 +101,19 @@ def _unpack_v_perhead(pl: PackedKVLayer, *, head_dim: int) -> Tensor:
     return out
 
 
+def _read_checks(unchecked) -> None:
+    """Calls every (check, layer, [H, n] device tensor) with the tensor's rows: one read per device."""
+    by_device: dict = {}
+    for entry in unchecked:
+        by_device.setdefault(entry[2].device, []).append(entry)
+    for entries in by_device.values():
+        flat, at = _lib.download(torch.cat([c.reshape(-1) for _, _, c in entries])).tolist(), 0
+        for check, pl, c in entries:
+            end, width = at + c.numel(), c.shape[1]
+            check(pl, [flat[i:i + width] for i in range(at, end, width)])
+            at = end
+
+
 def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
                               device: Optional[torch.device] = None, dtype: torch.dtype = torch.float16,
                               return_masks: bool = False, H_q: Optional[int] = None,
@@ -157,11 +170,5 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
                 masks.append(m4.contiguous())
             else:
                 masks.append(None)
-    # the counts of every layer in one read, behind the launches (which clamp what they follow)
-    if unchecked:
-        flat, at = _lib.download(torch.cat([c.reshape(-1) for _, _, c in unchecked])).tolist(), 0
-        for check, pl, c in unchecked:
-            end, width = at + c.numel(), c.shape[1]
-            check(pl, [flat[i:i + width] for i in range(at, end, width)])
-            at = end
+    _read_checks(unchecked)        # (behind the launches, which clamp what they follow)
     return (tuple(past_kv), masks) if return_masks else tuple(past_kv)

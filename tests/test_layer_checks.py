@@ -290,3 +290,15 @@ def test_dense_values_of_a_layer_without_a_class_tensor(lib):
     counts = torch.tensor([[7, 2, 2]] * 2, dtype=torch.int32)
     tz._unpack_v_perhead(dataclasses.replace(layer, seg_bounds_per_head=counts,
                                              T_eff_per_head=counts.sum(1, dtype=torch.int32)), head_dim=128)
+
+
+def test_counts_of_layers_on_several_devices_are_read_device_by_device(lib, monkeypatch):
+    reads = []
+    monkeypatch.setattr(_lib, "download", lambda t: (reads.append((t.device.type, t.numel())),
+                                                     torch.arange(t.numel()).numpy())[1])
+    seen = []
+    note = lambda layer, rows: seen.append((layer, rows))
+    tensors = [torch.zeros(2, 4, dtype=torch.int32, device=d) for d in ("cpu", "meta", "cpu", "meta")]
+    tz._read_checks([(note, i, t) for i, t in enumerate(tensors)])
+    assert sorted(reads) == [("cpu", 16), ("meta", 16)]
+    assert sorted(seen) == [(i, [[8 * (i // 2) + 4 * h + c for c in range(4)] for h in range(2)]) for i in range(4)]
