@@ -217,7 +217,7 @@ unpack_v_kernel(const uint8_t *__restrict__ V2, int64_t v2_sh, const uint8_t *__
   const int64_t e4 = min(e2 + min(max(counts[3 * h + 1], 0), m4), max_tv);
   const int64_t e8 = min(e4 + min(max(counts[3 * h + 2], 0), m8), max_tv);
   if (c0 >= D) return;
-  const int q2 = D / 4, q4 = D / 2;
+  const int q2 = max(D / 4, 1), q4 = max(D / 2, 1);    // (not used by rows of a width that D cannot have)
   const int off2 = c0 % q2, off4 = c0 % q4, sh2 = 2 * (c0 / q2), sh4 = 4 * (c0 / q4);
   u32x2 codes[kTok];
   __half sc[kTok], zz[kTok];
@@ -350,8 +350,10 @@ RDKV_API int rdkv_unpack_layer_v(const uint8_t *V2, int64_t v2_stride_h, const u
                                  int64_t s_stride_h, const int32_t *counts, int m2, int m4, int m8, int64_t max_tv,
                                  const void *V16_f16, int64_t v16_stride_h, int n16, int H_kv, int D, void *out_f16,
                                  void *stream) {
-  RDKV_REQUIRE(H_kv >= 1 && H_kv <= 65535 && max_tv >= 0 && n16 >= 0 && D >= 4 && D % 4 == 0 && D <= 65535 * kChan,
+  RDKV_REQUIRE(H_kv >= 1 && H_kv <= 65535 && max_tv >= 0 && n16 >= 0 && D >= 1 && D <= 65535 * kChan,
                "rdkv_unpack_layer_v: bad shape");
+  RDKV_REQUIRE((!V2 || m2 <= 0 || D % 4 == 0) && (!V4 || m4 <= 0 || D % 2 == 0),
+               "rdkv_unpack_layer_v: rows of %d codes that are no whole bytes", D);
   const int64_t T = max_tv + n16;
   if (T == 0) return RDKV_OK;
   if (!V2) m2 = 0;

@@ -55,6 +55,29 @@ def test_whole_layer_dequantizers_against_the_oracle(D, T, H):
         assert_bits_equal(t2n(v), exp_v if ora_nvo is None else np.concatenate([exp_v, ora_nvo], axis=2))
 
 
+@pytest.mark.parametrize("D,widths", [(1, (8,)), (3, (8,)), (6, (4, 8)), (6, (8,)), (130, (4, 8)), (131, (8,))])
+def test_head_dimensions_that_only_some_widths_pack(D, widths):
+    """A class needs whole bytes per row, a class that is not there needs nothing."""
+    require_gpu()
+    rng = np.random.default_rng(D)
+    H, n = 2, 37
+    code = {b: rng.integers(0, 1 << b, (1, H, n, D)) for b in widths}
+    seg = {8: lambda c: c, 4: lambda c: c[..., :D // 2] | c[..., D // 2:] << 4}
+    T = n * len(widths)
+    scale = rng.uniform(0.1, 2.0, (1, H, T, 1)).astype(np.float16)
+    zp = rng.integers(0, 8, (1, H, T, 1)).astype(np.float16)
+    v16 = rng.standard_normal((1, H, 5, D)).astype(np.float16)
+    counts = np.array([[0, n if 4 in widths else 0, n]] * H, np.int32)
+    none = dict.fromkeys(f.name for f in dataclasses.fields(packing.PackedKVLayer))
+    pl = packing.PackedKVLayer(**{**none, **{f"V_{b}bit": to_dev(seg[b](code[b]).astype(np.uint8)) for b in widths},
+                                  "V_scale": to_dev(scale), "V_zp": to_dev(zp), "T_eff": T,
+                                  "seg_bounds_per_head": to_dev(counts), "T_eff_per_head": to_dev(counts.sum(1).astype(np.int32))})
+    codes = np.concatenate([code[b] for b in widths], axis=2).astype(np.float32)
+    exp = ((codes - zp.astype(np.float32)) * scale.astype(np.float32)).astype(np.float16)
+    assert_bits_equal(t2n(tz._unpack_v_perhead(pl, head_dim=D)), exp)
+    assert_bits_equal(t2n(tz._unpack_v_enqueue(pl, to_dev(v16), D)[0]), np.concatenate([exp, v16], axis=2))
+
+
 def test_zero_points_that_are_not_whole_numbers():
     """Layers of other origin may carry such zero points; they take the fp32 form."""
     require_gpu()
