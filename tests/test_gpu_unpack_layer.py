@@ -137,3 +137,52 @@ def test_channels_outside_the_head_are_reported(D, channel):
     pl.K_ch_sort_idx_per_head[1, D - 51] = D if channel is None else channel
     with pytest.raises(IndexError, match="1"):
         packing.unpack_k_mixed(pl, D=D)
+
+
+def _random_k_layer(H, T, D, n_k, counts, seed, strided):
+    """A per-head K layer of random codes (no packer: the large sizes are about the launch), head h keeping
+    counts[h] channels of the classes, laid out for n_k."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    widths = (-(-n_k[0] // 4) * 4, -(-n_k[1] // 2) * 2, n_k[2])
+    segs = [torch.randint(0, 256, (1, H, T, w * b // 8), generator=g, device=DEV).to(torch.uint8) if w else None
+            for w, b in zip(widths, (2, 4, 8))]
+    Dp, kept = sum(widths), max(map(sum, counts))
+    index = torch.stack([torch.randperm(D, generator=g, device=DEV)[:kept] for _ in range(H)])
+    scale = torch.rand(1, H, 1, Dp, generator=g, device=DEV).half()
+    zp = torch.randint(0, 256, (1, H, 1, Dp), generator=g, device=DEV).half()
+    none = dict.fromkeys(f.name for f in dataclasses.fields(packing.PackedKVLayer))
+    K = [_widened(s, 3) if strided else s for s in segs]
+    layer = packing.PackedKVLayer(**{**none, "K_2bit": K[0], "K_4bit": K[1], "K_8bit": K[2], "K_ch_scale": scale, "K_ch_zp": zp,
+                                     "K_ch_seg_bounds": n_k, "K_ch_sort_idx_per_head": index, "T_eff": T, "T_eff_k": T,
+                                     "K_ch_seg_bounds_per_head": torch.tensor(counts, dtype=torch.int32, device=DEV)})
+    exp = torch.zeros(1, H, T, D, dtype=torch.float16, device=DEV)
+    for h in range(H):
+        at = slot = 0
+        for s, w, b, n in zip(segs, widths, (2, 4, 8), counts[h]):
+            if n:
+                rows = packing._dequant(s[0, h], w, b, scale[0, h, 0, slot:slot + w], zp[0, h, 0, slot:slot + w], per_row=False)
+                exp[0, h].index_copy_(1, index[h, at:at + n], rows[:, :n])
+            at, slot = at + n, slot + w
+    return layer, exp
+
+
+@pytest.mark.parametrize("strided", [False, True])
+@pytest.mark.parametrize("H,T,D", [(8, 17001, 128), (1, 131137, 128), (3, 43713, 128), (4, 17000, 200)])
+def test_workgroups_that_walk_several_tiles(H, T, D, strided):
+    """More rows than one tile per workgroup of the launch (64 x 2048 over all heads and channel chunks):
+    LDS filled again behind a barrier, another misalignment per tile, a short last tile."""
+    require_gpu()
+    counts = [[(5 * h) % 14, (7 * h + 3) % 23, (11 * h + 2) % 20] for h in range(H)]
+    counts[-1] = [13, 22, 19]
+    layer, exp = _random_k_layer(H, T, D, (13, 22, 19), counts, T, strided)
+    assert torch.equal(packing.unpack_k_mixed(layer, D=D).view(torch.int16), exp.view(torch.int16))
+
+
+@pytest.mark.parametrize("missing", [(0,), (1,), (2,), (0, 1), (0, 2), (1, 2)])
+def test_a_class_without_a_tensor_has_no_slots(missing):
+    """Its columns of the scales are skipped as long as no head keeps channels of it."""
+    require_gpu()
+    counts = [[0 if c in missing else n for c, n in enumerate(row)] for row in ((13, 22, 19), (3, 5, 7))]
+    layer, exp = _random_k_layer(2, 70, 128, (13, 22, 19), counts, 4, False)
+    layer = dataclasses.replace(layer, **{("K_2bit", "K_4bit", "K_8bit")[c]: None for c in missing})
+    assert torch.equal(packing.unpack_k_mixed(layer, D=128).view(torch.int16), exp.view(torch.int16))
