@@ -1028,7 +1028,7 @@ merge_kernel(const RdkvUnit *__restrict__ units, const float *__restrict__ parti
 //    table, the step's own key / value row, the partials' max / sum columns and accumulator
 //    columns, and the first 64 zone C tokens' K and V rows (requested before the count is known:
 //    rows up to the buffer's end exist, a row past the count is discarded).  The parts of the preparation are dealt to different wavefronts;
-//  * a workgroup of eight wavefronts takes HW of a unit's G heads (grid: units x G / HW); wavefront w
+//  * a workgroup of eight wavefronts takes HW of a unit's G heads; wavefront w
 //    owns tokens 8w .. 8w + 7 of every chunk of 64.  Both rows of a token are split over the same
 //    eight lanes (16-byte loads, 128 contiguous bytes per token and instruction), and every group of
 //    eight lanes keeps an online-softmax state of its own for each head, so the token loop exchanges
@@ -1041,8 +1041,11 @@ merge_kernel(const RdkvUnit *__restrict__ units, const float *__restrict__ parti
 //
 // The token loop is bound by its vector instructions on one compute unit, which is why a step of few
 // units is spread over its heads (HW = 1): nothing ties the heads together unless the block scores
-// of blockwise decode are summed over them.  The workgroups of a unit are n_units apart in launch
-// order, which for the usual multiples of eight puts them on one die, whose L2 serves the repeats.
+// of blockwise decode are summed over them.  The workgroups of a unit all read its rows: they are eight
+// apart in launch order, which puts them on one die at about the same time, so that its L2 serves the
+// repeats.  (All first workgroups ahead of all second ones, n_units apart, read the rows from memory every
+// time once the units' rows outgrew the caches: 384 units with 1000 tokens each, G = 4 / 8: 155 / 283 us a
+// step, now 118 / 166; with 300 tokens 73 / 119, now 64 / 85.)
 constexpr int kZcChunk = 64;
 constexpr int kZcWaves = 8;
 constexpr int kZcInlineUnits = 16;
@@ -1115,7 +1118,7 @@ __device__ __forceinline__ floatx4 zc_groups_sum(const floatx4 (&v)[4]) {
 template <int HW, bool INLINE>
 __global__ void __launch_bounds__(64 * kZcWaves) __attribute__((amdgpu_waves_per_eu(HW <= 2 ? 4 : 2)))
 merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float *__restrict__ partials, int G,
-                    const void *__restrict__ q, int q_dtype, int64_t q_stride,
+                    int n_units, const void *__restrict__ q, int q_dtype, int64_t q_stride,
                     const void *__restrict__ rope_cos, const void *__restrict__ rope_sin, int rope_dtype,
                     float *k_new, float *v_new, int64_t new_stride_unit,   // written when a row is appended
                     int64_t new_stride_tok, int n_new_all, const int32_t *__restrict__ n_new_per_unit,
@@ -1134,16 +1137,18 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
   __shared__ float fin_m[HW], fin_l[HW];                      // softmax maximum and sum over the union, per head
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int unit = blockIdx.z * 8 + blockIdx.x;      // grid: (8, G / HW, units / 8), or (units) if HW is G
   const int head0 = blockIdx.y * HW;
+  if (unit >= n_units) return;
 
   // ---- the unit: from the kernel arguments, or the first round trip ------------------------------
   int work_count, q_row, work_begin;
   if (INLINE) {
-    q_row = iu.q_row[blockIdx.x];
-    work_begin = iu.work_begin[blockIdx.x];
-    work_count = iu.work_count[blockIdx.x];
+    q_row = iu.q_row[unit];
+    work_begin = iu.work_begin[unit];
+    work_count = iu.work_count[unit];
   } else {
-    const RdkvUnit *u = units + blockIdx.x;
+    const RdkvUnit *u = units + unit;
     q_row = u->q_row;
     work_begin = u->work_begin;
     work_count = u->work_count;
@@ -1666,16 +1671,18 @@ static int launch_merge_zone_c(const char *fn, const RdkvUnit *units, const Rdkv
   // Heads per workgroup (any choice gives the same bits).  All of them where the block scores are
   // summed over the heads.  One while that leaves a compute unit per workgroup (a device has 256);
   // beyond, where workgroups share a compute unit and their preparation counts, two.  Measured, one
-  // / two / four heads, G = 4: 8 units with 17 and 700 tokens 22.7 / 23.5 / 25.1 and 26.9 / 29.1 /
-  // 36.6 us per step (32k prompt), 128 units with 300 tokens 31.0 / 29.0 / 31.0, 384 units 73 / 58 / 60.
+  // / two / all heads, us per step: 8 units, G = 4, 17 and 700 tokens 22.7 / 23.5 / 25.1 and 26.9 / 29.1 /
+  // 36.6 (32k prompt); 384 units (1k prompt), G = 4, 17 / 300 / 1000 tokens 52 / 50 / 53, 74 / 64 / 71 and
+  // 152 / 118 / 127; G = 8 79 / 71 / 75, 101 / 85 / 96 and 220 / 166 / 162.
   int hw = G;
-  if (!tail.self_scores) {
+  if (!tail.self_scores && n_units <= 8 * 65535) {   // (the last dimension of a grid of heads)
     if ((int64_t)n_units * G <= kZcWorkgroups) hw = 1;
     else if (G % 2 == 0) hw = 2;
   }
+  const dim3 grid = hw == G ? dim3(n_units) : dim3(8, G / hw, (unsigned)rdkv_cdiv(n_units, 8));
 #define RDKV_LAUNCH_ZC_I(HW, INL)                                                                             \
-  hipLaunchKernelGGL((merge_zone_c_kernel<HW, INL>), dim3(n_units, G / HW), dim3(64 * kZcWaves), 0,             \
-                     (hipStream_t)stream, units, iu, (const float *)workspace, G, q, q_dtype, q_stride_row,     \
+  hipLaunchKernelGGL((merge_zone_c_kernel<HW, INL>), grid, dim3(64 * kZcWaves), 0, (hipStream_t)stream, units,  \
+                     iu, (const float *)workspace, G, n_units, q, q_dtype, q_stride_row,                        \
                      rope_cos, rope_sin, rope_dtype, const_cast<float *>(k_new), const_cast<float *>(v_new),    \
                      new_stride_unit, new_stride_tok, n_new, n_new_per_unit, out, out_stride_row, lse,          \
                      zone_c_weights, zone_c_weights_stride_row, append, q_rot_out, q_rot_stride, tail)

@@ -109,3 +109,37 @@ def test_scores_of_minus_infinity_have_no_weight():
     exp, exp_lse = stream_cache.decode_attn_fused(cache, q, zone_c=(k[:, keep].contiguous(), v[:, keep].contiguous()))
     torch.testing.assert_close(out, exp, rtol=0, atol=1e-6)
     torch.testing.assert_close(lse, exp_lse, rtol=0, atol=1e-6)
+
+
+@pytest.mark.parametrize("G", [1, 2, 3, 4, 5, 6, 7, 8])
+@pytest.mark.parametrize("layers,heads", [(1, 1), (1, 7), (1, 9), (3, 5), (7, 11), (13, 11), (67, 5)])
+def test_same_bits_with_the_heads_apart_and_together(G, layers, heads):
+    """The same cache with block scores (all heads of a unit in one workgroup) and without (one, two or
+    all of them, by the number of units, here at numbers that are no multiple of eight): every unit is
+    merged, with the same bits, and the weights are those of the softmax over the union."""
+    require_gpu()
+    cache = _cache(G, layers, heads, G + layers)
+    n, cap, row = layers * heads, 140, 131
+    g = torch.Generator().manual_seed(layers + G)
+    counts = torch.tensor([COUNTS[i % 10] if i else row + 1 for i in range(n)], dtype=torch.int32).to(DEV)
+    fill = torch.randn(n, cap, 256, generator=g).to(DEV)
+    k, v = (torch.randn(n, 128, generator=g).half().to(DEV) for _ in range(2))
+    q = torch.randn(cache.rows, 128, generator=g).half().to(DEV)
+    row_t = torch.full((1,), row, dtype=torch.int64, device=DEV)
+    got = []
+    for scored in (True, False):
+        buf, w = fill.clone(), torch.full((cache.rows, cap), float("nan"), device=DEV)
+        out, lse = torch.full((cache.rows, 128), float("nan"), device=DEV), torch.full((cache.rows,), float("nan"), device=DEV)
+        tail = (torch.zeros(n, cap, device=DEV), torch.zeros(n, 256, device=DEV), None, 256) if scored else None
+        stream_cache.decode_attn_fused(cache, q, out, lse, zone_c=(buf[:, :, :128], buf[:, :, 128:], counts),
+                                       append=(k, v, row_t), zone_c_weights=w, tail_scores=tail)
+        got.append((out, lse, w.nan_to_num(nan=-1.0), buf))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    out, lse, w, buf = got[0]
+    assert bool(torch.isfinite(out).all()) and bool(torch.isfinite(lse).all())
+    s = torch.einsum("ugd,utd->ugt", q.double().view(n, G, 128), buf[:, :, :128].double()).view(cache.rows, cap) / 128 ** 0.5
+    there = (torch.arange(cap, device=DEV)[None] < counts[:, None]).repeat_interleave(G, 0)
+    exp = torch.where(there, torch.exp(s - lse.double()[:, None]), -1.0)
+    # scores of a few units in 32 bits: a few 2^-24 of them, times weights of at most one
+    torch.testing.assert_close(w.double(), exp, rtol=1e-5, atol=1e-7)
