@@ -1673,11 +1673,15 @@ static int launch_merge_zone_c(const char *fn, const RdkvUnit *units, const Rdkv
   // beyond, where workgroups share a compute unit and their preparation counts, two.  Measured, one
   // / two / all heads, us per step: 8 units, G = 4, 17 and 700 tokens 22.7 / 23.5 / 25.1 and 26.9 / 29.1 /
   // 36.6 (32k prompt); 384 units (1k prompt), G = 4, 17 / 300 / 1000 tokens 52 / 50 / 53, 74 / 64 / 71 and
-  // 152 / 118 / 127; G = 8 79 / 71 / 75, 101 / 85 / 96 and 220 / 166 / 162.
+  // 152 / 118 / 127; G = 8 79 / 71 / 75, 101 / 85 / 96 and 220 / 166 / 162.  Groups of 3, 5 and 7 cannot
+  // be paired: one head up to two workgroups per compute unit, all beyond.  One / all heads with 17 / 300 /
+  // 1000 tokens: 64 units, G = 5 29.8 / 32.2, 33.9 / 39.6, 48.5 / 57.6, G = 7 30.6 / 34.8, 35.3 / 45.3, 50.4 /
+  // 68.7; 128 units, G = 3 33.4 / 34.9, 40.6 / 42.4, 56.3 / 53.6; 384 units, G = 7 76 / 72, 96 / 91, 201 / 155.
   int hw = G;
   if (!tail.self_scores && n_units <= 8 * 65535) {   // (the last dimension of a grid of heads)
     if ((int64_t)n_units * G <= kZcWorkgroups) hw = 1;
     else if (G % 2 == 0) hw = 2;
+    else if ((int64_t)n_units * G <= 2 * kZcWorkgroups) hw = 1;
   }
   const dim3 grid = hw == G ? dim3(n_units) : dim3(8, G / hw, (unsigned)rdkv_cdiv(n_units, 8));
 #define RDKV_LAUNCH_ZC_I(HW, INL)                                                                             \
