@@ -642,7 +642,8 @@ int rdkv_pool_scores(const float *scores, int64_t stride_b, int B, int64_t T, in
  * workspace: rdkv_knapsack_workspace_bytes(B) bytes.  Two launches (one for rows of at most
  * 256 scores in groups of at most 16), no host synchronization.
  * Batches of few long rows (max_iters <= 64; T >= 8192 and so few rows that each can have 16 or
- * more resident workgroups, or 4096 <= T < 8192 and at most 64 rows) run with every row shared by 8, 16, 32 or 64 workgroups that exchange
+ * more resident workgroups, or 4096 <= T < 8192 and at most 64 rows) run with every row shared by
+ * 8, 16, 32 or 64 workgroups that exchange
  * integer width sums once per pass of 15 doublings or four bisection levels (the first pass takes
  * the starting multiplier and the first four levels together); the same bits.  The
  * workgroups wait for each other with a bound: should a wait not end (it cannot while the launch

@@ -1429,7 +1429,7 @@ RDKV_API int rdkv_v_weighted_sum_new_values(
   RDKV_REQUIRE(((uintptr_t)v_new % 16) == 0 && vn_stride_h % 4 == 0 && vn_stride_t % 4 == 0,
                "%s: value rows must be 16-byte aligned", fn);
   return v_weighted_sum(w, w_stride_h, H_q, H_kv, V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, scale_f16, zp_f16,
-                        vs_stride_h, seg_bounds_dev, N2, N4, N8, V16_f16, v16_stride_h, n_v16_dev, max_T_v, 
+                        vs_stride_h, seg_bounds_dev, N2, N4, N8, V16_f16, v16_stride_h, n_v16_dev, max_T_v,
                         NewValues{n_new > 0 ? v_new : nullptr, w_new, vn_stride_h, vn_stride_t, wn_stride_h, n_new}, out,
                         out_stride_h, workspace, workspace_bytes, stream);
 }

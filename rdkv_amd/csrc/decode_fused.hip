@@ -1027,10 +1027,10 @@ merge_kernel(const RdkvUnit *__restrict__ units, const float *__restrict__ parti
 //    everything else at once - the token count, the step's write row, the query rows and rotation
 //    table, the step's own key / value row, the partials' max / sum columns and accumulator
 //    columns, and the first 64 zone C tokens' K and V rows (requested before the count is known:
-//    rows up to the buffer's end exist, a row past the count is discarded).  The parts of the preparation are dealt to different wavefronts;
-//  * a workgroup of eight wavefronts takes HW of a unit's G heads; wavefront w
-//    owns tokens 8w .. 8w + 7 of every chunk of 64.  Both rows of a token are split over the same
-//    eight lanes (16-byte loads, 128 contiguous bytes per token and instruction), and every group of
+//    rows up to the buffer's end exist, a row past the count is discarded).  The parts of the
+//    preparation are dealt to different wavefronts;
+//  * a workgroup of eight wavefronts takes HW of a unit's G heads; wavefront w owns tokens
+//    8w .. 8w + 7 of every chunk of 64.  Both rows of a token are split over the same eight lanes (16-byte loads, 128 contiguous bytes per token and instruction), and every group of
 //    eight lanes keeps an online-softmax state of its own for each head, so the token loop exchanges
 //    nothing between tokens (a sum inside the eight lanes is all) and has no barrier; the next chunk is
 //    requested as soon as the registers are free, the other wavefronts work meanwhile (a second
@@ -1371,7 +1371,8 @@ merge_zone_c_kernel(const RdkvUnit *__restrict__ units, ZcInline iu, const float
   const int self_tok = appending ? (int)step_row : -1;
   // A lane group's first token has nothing to rescale: the same bits, a third of the loop's vector
   // instructions less, which counts where several heads share a workgroup and the tail is short (eight heads,
-  // 8 units, 1 / 17 / 100 tokens 33.2 / 32.9 / 37.0 -> 32.4 / 32.3 / 35.9 us a step).  One or two heads gain nothing and keep the shorter code.
+  // 8 units, 1 / 17 / 100 tokens 33.2 / 32.9 / 37.0 -> 32.4 / 32.3 / 35.9 us a step).  One or two heads gain
+  // nothing and keep the shorter code.
   auto consume = [&](Rows &r, int base, auto first_token) __attribute__((always_inline)) {
     constexpr bool kFirst = decltype(first_token)::value;
     const int t = base + tg;
@@ -1683,15 +1684,16 @@ static int launch_merge_zone_c(const char *fn, const RdkvUnit *units, const Rdkv
   // beyond, where workgroups share a compute unit and their preparation counts, two.  Measured, one
   // / two / all heads, us per step: 8 units, G = 4, 17 and 700 tokens 22.7 / 23.5 / 25.1 and 26.9 / 29.1 /
   // 36.6 (32k prompt); 384 units (1k prompt), G = 4, 17 / 300 / 1000 tokens 52 / 50 / 53, 74 / 64 / 71 and
-  // 152 / 118 / 127; G = 8 79 / 71 / 75, 101 / 85 / 96 and 220 / 166 / 162.  Groups of 3, 5 and 7 cannot
-  // be paired: one head up to two workgroups per compute unit, all beyond.  One / all heads with 17 / 300 /
+  // 152 / 118 / 127; G = 8 79 / 71 / 75, 101 / 85 / 96 and 220 / 166 / 162.  Groups of 5 and 7 cannot be
+  // paired: one head up to two workgroups per compute unit, all beyond.  One / all heads with 17 / 300 /
   // 1000 tokens: 64 units, G = 5 29.8 / 32.2, 33.9 / 39.6, 48.5 / 57.6, G = 7 30.6 / 34.8, 35.3 / 45.3, 50.4 /
-  // 68.7; 128 units, G = 3 33.4 / 34.9, 40.6 / 42.4, 56.3 / 53.6; 384 units, G = 7 76 / 72, 96 / 91, 201 / 155.
+  // 68.7; 384 units, G = 7 76 / 72, 96 / 91, 201 / 155.  Three heads are few enough to stay together:
+  // 128 units 33.3 / 34.4, 40.0 / 41.8, 55.9 / 53.5.
   int hw = G;
   if (!tail.self_scores && n_units <= 8 * 65535) {   // (the last dimension of a grid of heads)
     if ((int64_t)n_units * G <= kZcWorkgroups) hw = 1;
     else if (G % 2 == 0) hw = 2;
-    else if ((int64_t)n_units * G <= 2 * kZcWorkgroups) hw = 1;
+    else if (G > 3 && (int64_t)n_units * G <= 2 * kZcWorkgroups) hw = 1;
   }
   const dim3 grid = hw == G ? dim3(n_units) : dim3(8, G / hw, (unsigned)rdkv_cdiv(n_units, 8));
 #define RDKV_LAUNCH_ZC_I(HW, INL)                                                                             \
