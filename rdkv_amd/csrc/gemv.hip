@@ -213,8 +213,10 @@ void launch_gemv(const void *W, int64_t w_stride_row, const RowSource &src, cons
                  int n_cu, hipStream_t s) {
   // Sixteen wavefronts per compute unit while it has at most 32 rows (4096 x 4096: 7.9 us against 8.4
   // with eight, 6144 x 4096 11.3 against 11.7), eight beyond, where fewer streams read faster (28672 x 4096
-  // 37.6 against 38.2, 128256 x 4096 148.5 against 156.5).
-  const int max_waves = n_cu * (N <= 32 * n_cu ? 16 : 8);
+  // 37.6 against 38.2, 128256 x 4096 148.5 against 156.5) - but for rows below 4096 elements, which leave eight
+  // wavefronts with too few bytes in flight (a tile of 512 elements is a quarter full): 64000 x 512 34.0 -> 23.6,
+  // 128256 x 1024 77.0 -> 54.9, 28672 x 2048 23.5 -> 20.4, 64000 x 3584 72.9 -> 71.2.
+  const int max_waves = n_cu * (N <= 32 * n_cu || K < 4096 ? 16 : 8);
   const int waves = N < max_waves ? N : max_waves;
   const size_t lds = MODE == kNorm ? (size_t)K * 4 + 16 : (size_t)K * 2;
   // Workgroups of eight wavefronts when the row is long: it is staged half as often (4096 x 14336 with
