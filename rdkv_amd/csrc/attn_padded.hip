@@ -601,6 +601,15 @@ __device__ __forceinline__ void new_zone_scores(const NewKeys &nk, int h, int64_
   }
 }
 
+// The same as a launch of its own, kNewPerBlock keys of a head per workgroup (a pass of its wavefronts).
+constexpr int kNewPerBlock = 256;
+constexpr int64_t kNewOwnLaunch = 1024;
+__global__ void __launch_bounds__(1024)
+new_zone_scores_kernel(NewKeys nk, int64_t n_new, float *__restrict__ scores, int64_t stride_h) {
+  const int64_t a = (int64_t)blockIdx.x * kNewPerBlock, b = a + kNewPerBlock < n_new ? a + kNewPerBlock : n_new;
+  new_zone_scores(nk, blockIdx.y, a, b, scores + blockIdx.y * stride_h);
+}
+
 __device__ float block_reduce(float v, bool is_max, float *scratch) {
   v = is_max ? rdkv_wave_max(v) : rdkv_wave_sum(v);
   const int w = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -1280,7 +1289,7 @@ RDKV_API int64_t rdkv_softmax_rows_workspace_bytes(int H_q) {
 
 static int softmax_rows(const float *scores_old, int64_t so_stride_h, const float *mask, int64_t mask_stride_h,
                         int64_t T_old, const float *scores_new, int64_t sn_stride_h, int64_t n_new, float *w_old,
-                        int64_t wo_stride_h, float *w_new, int64_t wn_stride_h, const NewKeys &nk, int H_q,
+                        int64_t wo_stride_h, float *w_new, int64_t wn_stride_h, NewKeys nk, int H_q,
                         void *workspace, int64_t workspace_bytes, void *stream) {
   RDKV_REQUIRE(H_q > 0 && H_q <= 65535 && T_old >= 0 && n_new >= 0, "rdkv_softmax_rows: bad sizes");
   RDKV_REQUIRE(T_old + n_new > 0, "rdkv_softmax_rows: empty rows");
@@ -1306,6 +1315,16 @@ static int softmax_rows(const float *scores_old, int64_t so_stride_h, const floa
       RDKV_CHECK_LAUNCH("rdkv_softmax_rows");
       return RDKV_OK;
     }
+  }
+  // One workgroup per head reads that head's keys on its own: from 1024 appended tokens on their scores are a
+  // launch of their own, over the whole device.  8 KV heads, G = 4, 40k-token layer, us a call with / without
+  // it: 512 tokens 49.2 / 49.4, 1024 49.8 / 52.6, 4096 54 / 72, 16384 78 / 151; without packed tokens 512
+  // 16.9 / 17.0, 1024 17.7 / 18.8, 4096 23.5 / 41.8, 16384 49 / 122.  (The split form above deals the keys to
+  // its pieces: 131k layer, 4096 tokens 103.5 / 101.9, 16384 138.4 / 138.1.)
+  if (nk.k && n_new >= kNewOwnLaunch) {
+    hipLaunchKernelGGL(new_zone_scores_kernel, dim3((unsigned)rdkv_cdiv(n_new, kNewPerBlock), H_q), dim3(1024), 0,
+                       (hipStream_t)stream, nk, n_new, w_new, wn_stride_h);
+    nk.k = nullptr;
   }
 #define RDKV_LAUNCH_SOFTMAX(KERNEL)                                                                             \
   hipLaunchKernelGGL(KERNEL, dim3(H_q), dim3(1024), 0, (hipStream_t)stream, scores_old, so_stride_h, mask,      \

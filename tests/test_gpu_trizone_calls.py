@@ -26,7 +26,10 @@ def _layer(H, T, G, seed):
     (2, 3, 4, 1, torch.float16, "dense"), (2, 300, 4, 7, torch.bfloat16, "dense"), (3, 1200, 1, 8, torch.float32, "dense"),
     (2, 1200, 2, 9, torch.float16, "kv"), (2, 9000, 5, 127, torch.float16, "odd"), (1, 9000, 8, 128, torch.bfloat16, "dense"),
     (2, 34000, 4, 129, torch.float16, "kv"), (2, 34001, 9, 257, torch.float16, "dense"), (1, 66001, 4, 1, torch.float16, "dense"),
-    (1, 66001, 4, 1030, torch.float16, "odd"), (2, 0, 4, 33, torch.float16, "dense")])
+    (1, 66001, 4, 1030, torch.float16, "odd"), (2, 0, 4, 33, torch.float16, "dense"),
+    # around the length from which the scores are a launch of their own, and its 256 keys per workgroup
+    (2, 300, 4, 1023, torch.float16, "dense"), (2, 300, 4, 1024, torch.float16, "odd"), (3, 9000, 5, 1025, torch.bfloat16, "kv"),
+    (1, 34000, 8, 1281, torch.float32, "dense"), (2, 0, 1, 1279, torch.float16, "dense"), (2, 1200, 9, 5000, torch.float16, "kv")])
 def test_trizone_attention_new_zone(H, T, G, n_new, dtype, form):
     require_gpu()
     g = torch.Generator().manual_seed(T + n_new)
@@ -78,3 +81,24 @@ def test_buffers_and_rows_that_do_not_fit_are_refused():
         fast_decode.trizone_attention(*args, kv, kv, 4, scores_buf=torch.empty(8, 48, device=DEV, dtype=torch.float16))
     with pytest.raises(RuntimeError):
         fast_decode.trizone_attention(torch.randn(10, 128, device=DEV), *args[1:], kv, kv, 4)
+
+
+@pytest.mark.parametrize("T,n_new", [(0, 9), (0, 1500), (50, 9), (50, 1500), (9000, 300), (9000, 1500)])
+def test_score_buffers_of_any_alignment(T, n_new):
+    """Rows at odd floats take the element-wise softmax: the same weights and output to rounding."""
+    require_gpu()
+    g = torch.Generator().manual_seed(T + n_new)
+    layer, v16 = _layer(2, max(T, 5), 4, 3)
+    if T == 0:
+        layer.T_eff = layer.T_eff_k = 0
+    t_old = int(layer.T_eff_k) if layer.T_eff_k > 0 else int(layer.T_eff)
+    q, kn, vn = (torch.randn(*s, generator=g).to(DEV) for s in ((8, 128), (2, n_new, 128), (2, n_new, 128)))
+    got = []
+    for shift in (0, 1, 3):
+        row = -(-(t_old + n_new) // 4) * 4 + shift
+        buf = torch.empty(8, row + shift, device=DEV)[:, shift:]
+        out = fast_decode.trizone_attention(q, layer, v16, layer.n_v16_per_head, kn, vn, 4, scores_buf=buf)
+        got.append((out, buf[:, :t_old + n_new]))
+    for out, w in got[1:]:
+        torch.testing.assert_close(out, got[0][0], rtol=0, atol=1e-5)
+        torch.testing.assert_close(w, got[0][1], rtol=1e-4, atol=1e-7)
