@@ -602,12 +602,16 @@ __device__ __forceinline__ void new_zone_scores(const NewKeys &nk, int h, int64_
 }
 
 // The same as a launch of its own, kNewPerBlock keys of a head per workgroup (a pass of its wavefronts).
+// grid = (8, G, H_kv * eighths of the pieces): the G heads that read a piece are eight apart in launch order,
+// on one die, whose L2 serves the repeats.
 constexpr int kNewPerBlock = 256;
 constexpr int64_t kNewOwnLaunch = 1024;
 __global__ void __launch_bounds__(1024)
-new_zone_scores_kernel(NewKeys nk, int64_t n_new, float *__restrict__ scores, int64_t stride_h) {
-  const int64_t a = (int64_t)blockIdx.x * kNewPerBlock, b = a + kNewPerBlock < n_new ? a + kNewPerBlock : n_new;
-  new_zone_scores(nk, blockIdx.y, a, b, scores + blockIdx.y * stride_h);
+new_zone_scores_kernel(NewKeys nk, int64_t n_new, int eighths, float *__restrict__ scores, int64_t stride_h) {
+  const int kv = blockIdx.z / eighths, h = kv * nk.G + blockIdx.y;
+  const int64_t a = ((int64_t)(blockIdx.z - kv * eighths) * 8 + blockIdx.x) * kNewPerBlock;
+  const int64_t b = a + kNewPerBlock < n_new ? a + kNewPerBlock : n_new;
+  new_zone_scores(nk, h, a, b, scores + h * stride_h);
 }
 
 __device__ float block_reduce(float v, bool is_max, float *scratch) {
@@ -1321,9 +1325,10 @@ static int softmax_rows(const float *scores_old, int64_t so_stride_h, const floa
   // it: 512 tokens 49.2 / 49.4, 1024 49.8 / 52.6, 4096 54 / 72, 16384 78 / 151; without packed tokens 512
   // 16.9 / 17.0, 1024 17.7 / 18.8, 4096 23.5 / 41.8, 16384 49 / 122.  (The split form above deals the keys to
   // its pieces: 131k layer, 4096 tokens 103.5 / 101.9, 16384 138.4 / 138.1.)
-  if (nk.k && n_new >= kNewOwnLaunch) {
-    hipLaunchKernelGGL(new_zone_scores_kernel, dim3((unsigned)rdkv_cdiv(n_new, kNewPerBlock), H_q), dim3(1024), 0,
-                       (hipStream_t)stream, nk, n_new, w_new, wn_stride_h);
+  const int64_t eighths = rdkv_cdiv(n_new, 8 * kNewPerBlock);
+  if (nk.k && n_new >= kNewOwnLaunch && nk.G <= 65535 && eighths * (H_q / nk.G) <= 65535) {
+    hipLaunchKernelGGL(new_zone_scores_kernel, dim3(8, nk.G, (unsigned)(eighths * (H_q / nk.G))), dim3(1024), 0,
+                       (hipStream_t)stream, nk, n_new, (int)eighths, w_new, wn_stride_h);
     nk.k = nullptr;
   }
 #define RDKV_LAUNCH_SOFTMAX(KERNEL)                                                                             \
