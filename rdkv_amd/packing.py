@@ -361,7 +361,7 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
         if t is None or w == 0:
             segs.append((None, 0, 0, 0))
             continue
-        if t.dim() != 4 or t.shape[1] < H or t.shape[2:] != (T, w * bits // 8):
+        if t.shape != (1, H, T, w * bits // 8) and (t.dim() != 4 or t.shape[1] < H or t.shape[2:] != (T, w * bits // 8)):
             raise RuntimeError(f"K segment {tuple(t.shape)} for {H} heads, {T} tokens, {w} channels")
         t = t if t.stride(3) == 1 else t.contiguous()
         segs.append((t, t.stride(1), t.stride(2), w))
@@ -373,19 +373,21 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
     assert sort is not None, "per-head layout requires K_ch_sort_idx_per_head"
     _lib.require_device(sc, zz, sort, K2, K4, K8)
     Dp = sum(widths)
-    for t in (sc, zz):
-        if t.dim() != 4 or t.shape[1] < H or t.shape[3] < Dp:
-            raise RuntimeError(f"K scales / zero points {tuple(t.shape)} for {H} heads of {Dp} channels")
-    if sort.dtype != torch.long or sort.dim() != (2 if per_head else 1) or (per_head and sort.shape[0] < H):
+    exact = sc.shape == zz.shape == (1, H, 1, Dp)
+    if not exact and any(t.dim() != 4 or t.shape[1] < H or t.shape[3] < Dp for t in (sc, zz)):
+        raise RuntimeError(f"K scales / zero points {tuple(sc.shape)}, {tuple(zz.shape)} for {H} heads of {Dp} channels")
+    if sort.dtype != torch.long or sort.dim() != (2 if per_head else 1) or (per_head and len(sort) < H):
         raise RuntimeError(f"channel index {tuple(sort.shape)} {sort.dtype} for {H} heads")
-    if sc.shape != zz.shape or sc.stride(3) != 1 or zz.stride() != sc.stride():
+    if not exact or sc.stride(3) != 1 or zz.stride() != sc.stride():
         sc, zz = (t[:1, :H, :1, :Dp].contiguous() for t in (sc, zz))
     counts, limits = None, tuple(n if s[3] else 0 for n, s in zip((m2, m4, m8), segs))
     if per_head:
         counts = packed.K_ch_seg_bounds_per_head
-        if counts.dim() != 2 or counts.shape[0] < H or counts.shape[1] != 3:
-            raise RuntimeError(f"channel counts {tuple(counts.shape)} for {H} heads")
-        counts = (counts[:H] if counts.shape[0] > H else counts).to(device=dev, dtype=torch.int32).contiguous()
+        if counts.shape != (H, 3):
+            if counts.dim() != 2 or len(counts) < H or counts.shape[1] != 3:
+                raise RuntimeError(f"channel counts {tuple(counts.shape)} for {H} heads")
+            counts = counts[:H]
+        counts = counts.to(device=dev, dtype=torch.int32).contiguous()
     else:
         assert limits == (m2, m4, m8), "a K segment is missing"
         if sort.shape[0] < sum(limits):
@@ -411,18 +413,18 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
 
 
 def _check_k_counts(packed: "PackedKVLayer", found: Sequence[Sequence[int]]) -> None:
-    counts = [row[:3] for row in found]
+    *classes, outside = zip(*found)          # by column: this runs for every head of every layer
     m2, m4, m8 = packed.K_ch_seg_bounds
     widths = (_seg_padded_len(m2, 4), _seg_padded_len(m4, 2), m8)
-    most = [max(column) for column in zip(*counts)]
-    assert min(map(min, counts)) >= 0, f"heads keep a negative number of channels: {counts}"
+    most, least = [max(c) for c in classes], min(map(min, classes))
+    assert least >= 0, f"a head keeps a negative number of channels ({least})"
     for n, t in zip(most, (packed.K_2bit, packed.K_4bit, packed.K_8bit)):
         assert n == 0 or t is not None, f"a head keeps {n} channels of a K segment that is missing"
     assert all(n <= w for n, w in zip(most, widths)), f"heads keep {most} channels of K segments of {widths}"
-    kept, listed = max(map(sum, counts)), packed.K_ch_sort_idx_per_head.shape[-1]
+    kept, listed = max(map(sum, zip(*classes))), packed.K_ch_sort_idx_per_head.shape[-1]
     assert kept <= listed, f"a head keeps {kept} channels, {listed} are listed"
-    if any(row[3] for row in found):
-        raise IndexError(f"heads {[h for h, row in enumerate(found) if row[3]]} keep channels outside the head dimension")
+    if any(outside):
+        raise IndexError(f"heads {[h for h, bad in enumerate(outside) if bad]} keep channels outside the head dimension")
 
 
 def unpack_k_mixed(packed: "PackedKVLayer", D: int) -> Tensor:

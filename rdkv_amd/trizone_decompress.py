@@ -55,15 +55,15 @@ def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int
         segs.append((seg, seg.stride(1), int(seg.shape[2])))
     sc, zp = pl.V_scale, pl.V_zp
     rows = min(max_T_v, sum(m for _, _, m in segs))      # of a head, at most: the kernel clamps its counts to these
-    for t in (sc, zp):
-        if t.dim() < 3 or t.shape[1] < H_kv or t.shape[2] < rows:
-            raise RuntimeError(f"V scales / zero points {tuple(t.shape)} for {H_kv} heads of {rows} tokens")
-    if sc.numel() and not (sc.shape == zp.shape and sc.stride(2) == 1 and zp.stride() == sc.stride()):
+    exact = sc.shape == zp.shape == (1, H_kv, max_T_v, 1)
+    if not exact and any(t.dim() < 3 or t.shape[1] < H_kv or t.shape[2] < rows for t in (sc, zp)):
+        raise RuntimeError(f"V scales / zero points {tuple(sc.shape)}, {tuple(zp.shape)} for {H_kv} heads of {rows} tokens")
+    if rows and not (exact and sc.stride(2) == 1 and zp.stride() == sc.stride()):
         sc, zp = (t[:1, :H_kv, :rows].contiguous() for t in (sc, zp))
     counts, totals = pl.seg_bounds_per_head, pl.T_eff_per_head
-    if counts.dim() != 2 or counts.shape[0] < H_kv or counts.shape[1] != 3 or totals.numel() < H_kv:
-        raise RuntimeError(f"V counts {tuple(counts.shape)}, {tuple(totals.shape)} for {H_kv} heads")
-    if counts.shape[0] > H_kv or totals.numel() > H_kv:
+    if counts.shape != (H_kv, 3) or totals.shape != (H_kv,):
+        if counts.dim() != 2 or len(counts) < H_kv or counts.shape[1] != 3 or totals.numel() < H_kv:
+            raise RuntimeError(f"V counts {tuple(counts.shape)}, {tuple(totals.shape)} for {H_kv} heads")
         counts, totals = counts[:H_kv], totals.reshape(-1)[:H_kv]
     counts = counts.to(device=dev, dtype=torch.int32).contiguous()
     totals = totals.to(device=dev, dtype=torch.int32).reshape(H_kv, 1)
@@ -81,14 +81,19 @@ def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int
 
 
 def _check_v_counts(pl: PackedKVLayer, counts) -> None:
-    rows = [None if seg is None else int(seg.shape[2]) for seg in (pl.V_2bit, pl.V_4bit, pl.V_8bit)]
-    for h, (*classes, n) in enumerate(counts):
-        assert sum(classes) == n, f"head {h}: seg_bounds_per_head {classes} != T_eff_per_head {n}"
+    segs = (pl.V_2bit, pl.V_4bit, pl.V_8bit)
+    rows = [0 if seg is None else int(seg.shape[2]) for seg in segs]
+    *classes, totals = zip(*counts)
+    sums = tuple(map(sum, zip(*classes)))
+    if sums == totals and max(totals) <= pl.T_eff and min(map(min, classes)) >= 0 \
+            and all(max(c) <= r for c, r in zip(classes, rows)):
+        return
+    for h, (*row, n) in enumerate(counts):
+        assert sum(row) == n, f"head {h}: seg_bounds_per_head {row} != T_eff_per_head {n}"
         # rows that are there: tokens of a class without a tensor are left out, a negative count has none
-        there = [max(c, 0) for c, r in zip(classes, rows) if r is not None]
-        assert all(c <= r for c, r in zip(there, (r for r in rows if r is not None))), \
-            f"head {h}: {classes} tokens in V segments of {rows}"
-        assert sum(there) <= pl.T_eff, f"head {h}: {classes} tokens in a stripe of {pl.T_eff}"
+        there = [max(c, 0) if seg is not None else 0 for c, seg in zip(row, segs)]
+        assert all(c <= r for c, r in zip(there, rows)), f"head {h}: {row} tokens in V segments of {rows}"
+        assert sum(there) <= pl.T_eff, f"head {h}: {row} tokens in a stripe of {pl.T_eff}"
 
 
 def _unpack_v_perhead(pl: PackedKVLayer, *, head_dim: int) -> Tensor:
