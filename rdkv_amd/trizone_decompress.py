@@ -36,9 +36,9 @@ def _is_perhead_layout(pl: PackedKVLayer) -> bool:
     return pl.seg_bounds_per_head is not None
 
 
-def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int) -> Tuple[Tensor, Tensor]:
-    """The stripe's dense V, ``zone_b`` rows behind it, in one launch; and the device's per-head counts
-    (2-, 4-, 8-bit, all), yet to be checked (``_check_v_counts``)."""
+def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int) -> Tuple[Tensor, Tensor, Tensor]:
+    """The stripe's dense V, ``zone_b`` rows behind it, in one launch; and the per-head counts on the device,
+    [H, 3] by class and [H] in all, yet to be checked (``_check_v_counts``)."""
     max_T_v = int(pl.T_eff)
     H_kv = pl.V_scale.shape[1]
     # everything the kernel indexes by head, class row and token, before it gets the addresses
@@ -66,8 +66,7 @@ def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int
             raise RuntimeError(f"V counts {tuple(counts.shape)}, {tuple(totals.shape)} for {H_kv} heads")
         counts, totals = counts[:H_kv], totals.reshape(-1)[:H_kv]
     counts = counts.to(device=dev, dtype=torch.int32).contiguous()
-    totals = totals.to(device=dev, dtype=torch.int32).reshape(H_kv, 1)
-    check = torch.cat([counts, totals], dim=1)
+    totals = totals.to(device=dev, dtype=torch.int32)
     n16 = 0 if zone_b is None else int(zone_b.shape[2])
     out = torch.empty(1, H_kv, max_T_v + n16, head_dim, dtype=torch.float16, device=dev)
     if zone_b is not None and not (zone_b.stride(3) == 1 and zone_b.stride(2) == head_dim):
@@ -77,18 +76,17 @@ def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int
         _lib.ptr(V2), v2h, _lib.ptr(V4), v4h, _lib.ptr(V8), v8h, _lib.ptr(sc), _lib.ptr(zp), sc.stride(1),
         counts.data_ptr(), m2, m4, m8, max_T_v, _lib.ptr(zone_b), zone_b.stride(1) if n16 else 0, n16, H_kv, head_dim,
         _lib.ptr(out), _lib.stream_of(dev)))
-    return out, check
+    return out, counts, totals
 
 
-def _check_v_counts(pl: PackedKVLayer, counts) -> None:
+def _check_v_counts(pl: PackedKVLayer, counts, totals) -> None:
     segs = (pl.V_2bit, pl.V_4bit, pl.V_8bit)
     rows = [0 if seg is None else int(seg.shape[2]) for seg in segs]
-    *classes, totals = zip(*counts)
-    sums = tuple(map(sum, zip(*classes)))
-    if sums == totals and max(totals) <= pl.T_eff and min(map(min, classes)) >= 0 \
+    classes = list(zip(*counts))
+    if list(map(sum, counts)) == totals and max(totals) <= pl.T_eff and min(map(min, classes)) >= 0 \
             and all(max(c) <= r for c, r in zip(classes, rows)):
         return
-    for h, (*row, n) in enumerate(counts):
+    for h, (row, n) in enumerate(zip(counts, totals)):
         assert sum(row) == n, f"head {h}: seg_bounds_per_head {row} != T_eff_per_head {n}"
         # rows that are there: tokens of a class without a tensor are left out, a negative count has none
         there = [max(c, 0) if seg is not None else 0 for c, seg in zip(row, segs)]
@@ -101,22 +99,25 @@ def _unpack_v_perhead(pl: PackedKVLayer, *, head_dim: int) -> Tensor:
     (trizone_decompress.py:91-144)."""
     if int(pl.T_eff) == 0:
         return torch.zeros(1, pl.V_scale.shape[1], 0, head_dim, dtype=torch.float16, device=pl.V_scale.device)
-    out, check = _unpack_v_enqueue(pl, None, head_dim)
-    _check_v_counts(pl, check.tolist())
+    out, *found = _unpack_v_enqueue(pl, None, head_dim)
+    _read_checks([(_check_v_counts, pl, found)])
     return out
 
 
 def _read_checks(unchecked) -> None:
-    """Calls every (check, layer, [H, n] device tensor) with the tensor's rows: one read per device."""
+    """Calls every (check, layer, device tensors) with the tensors' values as lists: one read per device."""
     by_device: dict = {}
     for entry in unchecked:
-        by_device.setdefault(entry[2].device, []).append(entry)
+        by_device.setdefault(entry[2][0].device, []).append(entry)
     for entries in by_device.values():
-        flat, at = _lib.download(torch.cat([c.reshape(-1) for _, _, c in entries])).tolist(), 0
-        for check, pl, c in entries:
-            end, width = at + c.numel(), c.shape[1]
-            check(pl, [flat[i:i + width] for i in range(at, end, width)])
-            at = end
+        flat, at = _lib.download(torch.cat([t.reshape(-1) for _, _, ts in entries for t in ts])).tolist(), 0
+        for check, pl, ts in entries:
+            values = []
+            for t in ts:
+                end, width = at + t.numel(), t.shape[-1]
+                values.append([flat[i:i + width] for i in range(at, end, width)] if t.dim() == 2 else flat[at:end])
+                at = end
+            check(pl, *values)
 
 
 def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
@@ -128,11 +129,11 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
     shared-layout layers) (trizone_decompress.py:185-333)."""
     past_kv: List[Tuple[Tensor, Tensor]] = []
     masks: List[Optional[Tensor]] = []
-    unchecked = []        # (check, layer, per-head counts as the launches below read them)
+    unchecked = []        # (check, layer, per-head counts the launches below read)
     for i, pl in enumerate(dual_cache.packed):
         K_full, k_check = _unpack_k_enqueue(pl, head_dim)
         if k_check is not None:
-            unchecked.append((_check_k_counts, pl, k_check))
+            unchecked.append((_check_k_counts, pl, (k_check,)))
         zone_b = dual_cache.new_v_only[i] if i < len(dual_cache.new_v_only) else None
         if _is_perhead_layout(pl):
             rows_b = None
@@ -144,7 +145,7 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
             else:
                 joined = rows_b is not None and rows_b.dtype == torch.float16 and rows_b.shape[:2] == pl.V_scale.shape[:2] \
                     and rows_b.shape[3] == head_dim and rows_b.device == pl.V_scale.device
-                V_full, v_counts = _unpack_v_enqueue(pl, rows_b if joined else None, head_dim)
+                V_full, *v_counts = _unpack_v_enqueue(pl, rows_b if joined else None, head_dim)
                 unchecked.append((_check_v_counts, pl, v_counts))
                 if rows_b is not None and not joined:
                     V_full = torch.cat([V_full, rows_b], dim=2)

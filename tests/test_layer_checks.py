@@ -263,11 +263,11 @@ def test_dense_values_refuse_tensors_that_do_not_fit(lib):
 def test_dense_values_take_tensors_wider_than_needed(lib):
     layer = _layer()
     wide = torch.nn.functional.pad
-    _, check = tz._unpack_v_enqueue(dataclasses.replace(
+    _, counts, totals = tz._unpack_v_enqueue(dataclasses.replace(
         layer, V_zp=wide(layer.V_zp, (0, 0, 0, 5)), V_4bit=torch.cat([layer.V_4bit] * 2, dim=1),
         seg_bounds_per_head=wide(layer.seg_bounds_per_head, (0, 0, 0, 1), value=99),
         T_eff_per_head=wide(layer.T_eff_per_head, (0, 1))), None, 128)
-    assert lib.calls == ["rdkv_unpack_layer_v"] and check.shape == (2, 4)
+    assert lib.calls == ["rdkv_unpack_layer_v"] and counts.shape == (2, 3) and totals.shape == (2,)
 
 
 @pytest.mark.parametrize("counts,total", [((-3, 4, 5), 6), ((4, -3, 5), 6), ((4, 5, -3), 6), ((-9, 4, 5), 0)])
@@ -299,6 +299,6 @@ def test_counts_of_layers_on_several_devices_are_read_device_by_device(lib, monk
     seen = []
     note = lambda layer, rows: seen.append((layer, rows))
     tensors = [torch.zeros(2, 4, dtype=torch.int32, device=d) for d in ("cpu", "meta", "cpu", "meta")]
-    tz._read_checks([(note, i, t) for i, t in enumerate(tensors)])
+    tz._read_checks([(note, i, (t,)) for i, t in enumerate(tensors)])
     assert sorted(reads) == [("cpu", 16), ("meta", 16)]
     assert sorted(seen) == [(i, [[8 * (i // 2) + 4 * h + c for c in range(4)] for h in range(2)]) for i in range(4)]
