@@ -342,6 +342,13 @@ def _dequant(packed: Tensor, ncols: int, n_bits: int, scale: Tensor, zp: Tensor,
     return out.reshape(*packed.shape[:-1], ncols)
 
 
+def _int32_on(dev: torch.device, t: Tensor) -> Tensor:
+    """``t`` as dense int32 on ``dev`` (which counts mostly are: asking is cheaper than converting to the same)."""
+    if t.dtype is torch.int32 and t.device == dev and t.is_contiguous():
+        return t
+    return t.to(device=dev, dtype=torch.int32).contiguous()
+
+
 def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional[Tensor]]:
     """``unpack_k_mixed`` as one launch: the dense rows and, of a per-head layer, what the launch found of every
     head: the class counts and whether a kept channel is outside the head dimension, yet to be checked
@@ -376,7 +383,7 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
     exact = sc.shape == zz.shape == (1, H, 1, Dp)
     if not exact and any(t.dim() != 4 or t.shape[1] < H or t.shape[3] < Dp for t in (sc, zz)):
         raise RuntimeError(f"K scales / zero points {tuple(sc.shape)}, {tuple(zz.shape)} for {H} heads of {Dp} channels")
-    if sort.dtype != torch.long or sort.dim() != (2 if per_head else 1) or (per_head and len(sort) < H):
+    if sort.dtype != torch.long or sort.dim() != (2 if per_head else 1) or (per_head and sort.shape[0] < H):
         raise RuntimeError(f"channel index {tuple(sort.shape)} {sort.dtype} for {H} heads")
     if not exact or sc.stride(3) != 1 or zz.stride() != sc.stride():
         sc, zz = (t[:1, :H, :1, :Dp].contiguous() for t in (sc, zz))
@@ -384,10 +391,10 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
     if per_head:
         counts = packed.K_ch_seg_bounds_per_head
         if counts.shape != (H, 3):
-            if counts.dim() != 2 or len(counts) < H or counts.shape[1] != 3:
+            if counts.dim() != 2 or counts.shape[0] < H or counts.shape[1] != 3:
                 raise RuntimeError(f"channel counts {tuple(counts.shape)} for {H} heads")
             counts = counts[:H]
-        counts = counts.to(device=dev, dtype=torch.int32).contiguous()
+        counts = _int32_on(dev, counts)
     else:
         assert limits == (m2, m4, m8), "a K segment is missing"
         if sort.shape[0] < sum(limits):

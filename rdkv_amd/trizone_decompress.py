@@ -12,7 +12,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from .packing import PackedKVLayer, TriZoneCache, _check_k_counts, _unpack_k_enqueue, unpack_v_segment
+from .packing import PackedKVLayer, TriZoneCache, _check_k_counts, _int32_on, _unpack_k_enqueue, unpack_v_segment
 
 
 def _unpack_v_zone_a(pl: PackedKVLayer) -> Tensor:
@@ -62,11 +62,10 @@ def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int
         sc, zp = (t[:1, :H_kv, :rows].contiguous() for t in (sc, zp))
     counts, totals = pl.seg_bounds_per_head, pl.T_eff_per_head
     if counts.shape != (H_kv, 3) or totals.shape != (H_kv,):
-        if counts.dim() != 2 or len(counts) < H_kv or counts.shape[1] != 3 or totals.numel() < H_kv:
+        if counts.dim() != 2 or counts.shape[0] < H_kv or counts.shape[1] != 3 or totals.numel() < H_kv:
             raise RuntimeError(f"V counts {tuple(counts.shape)}, {tuple(totals.shape)} for {H_kv} heads")
         counts, totals = counts[:H_kv], totals.reshape(-1)[:H_kv]
-    counts = counts.to(device=dev, dtype=torch.int32).contiguous()
-    totals = totals.to(device=dev, dtype=torch.int32)
+    counts, totals = _int32_on(dev, counts), _int32_on(dev, totals)
     n16 = 0 if zone_b is None else int(zone_b.shape[2])
     out = torch.empty(1, H_kv, max_T_v + n16, head_dim, dtype=torch.float16, device=dev)
     if zone_b is not None and not (zone_b.stride(3) == 1 and zone_b.stride(2) == head_dim):
