@@ -358,8 +358,8 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
         raise ValueError("unpack_k_mixed: K_ch_scale missing")
     per_head = packed.K_ch_seg_bounds_per_head is not None
     sort = packed.K_ch_sort_idx_per_head if per_head else packed.K_ch_sort_idx
-    dev = _lib.require_device(packed.K_ch_scale)
-    H = packed.K_ch_scale.shape[1]
+    sc, zz = packed.K_ch_scale, packed.K_ch_zp
+    H = sc.shape[1]
     T = packed.T_eff_k if packed.T_eff_k > 0 else packed.T_eff
     m2, m4, m8 = packed.K_ch_seg_bounds
     widths = (_seg_padded_len(m2, 4), _seg_padded_len(m4, 2), m8)
@@ -372,13 +372,12 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
             raise RuntimeError(f"K segment {tuple(t.shape)} for {H} heads, {T} tokens, {w} channels")
         t = t if t.stride(3) == 1 else t.contiguous()
         segs.append((t, t.stride(1), t.stride(2), w))
-    if not any(s[3] for s in segs):
-        return torch.zeros(1, H, T, D, dtype=torch.float16, device=dev), None
     (K2, k2h, k2t, w2), (K4, k4h, k4t, w4), (K8, k8h, k8t, w8) = segs
+    if not (w2 or w4 or w8):
+        return torch.zeros(1, H, T, D, dtype=torch.float16, device=_lib.require_device(sc)), None
     # everything the kernel indexes by head, slot and token, before it gets the addresses
-    sc, zz = packed.K_ch_scale, packed.K_ch_zp
     assert sort is not None, "per-head layout requires K_ch_sort_idx_per_head"
-    _lib.require_device(sc, zz, sort, K2, K4, K8)
+    dev = _lib.require_device(sc, zz, sort, K2, K4, K8)
     Dp = sum(widths)
     exact = sc.shape == zz.shape == (1, H, 1, Dp)
     if not exact and any(t.dim() != 4 or t.shape[1] < H or t.shape[3] < Dp for t in (sc, zz)):
@@ -387,7 +386,7 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
         raise RuntimeError(f"channel index {tuple(sort.shape)} {sort.dtype} for {H} heads")
     if not exact or sc.stride(3) != 1 or zz.stride() != sc.stride():
         sc, zz = (t[:1, :H, :1, :Dp].contiguous() for t in (sc, zz))
-    counts, limits = None, tuple(n if s[3] else 0 for n, s in zip((m2, m4, m8), segs))
+    counts, limits = None, (m2 if w2 else 0, m4 if w4 else 0, m8 if w8 else 0)
     if per_head:
         counts = packed.K_ch_seg_bounds_per_head
         if counts.shape != (H, 3):
