@@ -2,11 +2,11 @@
 // Lagrangian knapsack that assigns every token (or channel) a bit width.
 //
 // The knapsack is a bisection on lambda; one evaluation ("solve") picks, per token, the option
-// minimising  score*eps[n] + lambda*bits[n]  and averages the chosen widths over the row.  One
-// workgroup owns one row and runs the whole bisection in a single launch: per solve every
-// thread walks its share of the row (coalesced, L2-resident after the first pass), the widths
-// are summed as integers (exact, order-free) and the next lambda is derived redundantly by all
-// threads from the reduced sum, so there is no host round trip and no inter-workgroup wait.
+// minimising  score*eps[n] + lambda*bits[n]  and averages the chosen widths over the row.  Widths are
+// summed as integers (exact, order-free) and the next lambda is derived redundantly by every thread that
+// needs it, so there is no host round trip.  Three forms, the same bits: a workgroup per row (the usual
+// one: coalesced, L2-resident after the first pass, no wait between workgroups), few long rows shared by
+// several workgroups each, and short rows as a wavefront each with the row in registers.
 // All lambda arithmetic is single IEEE operations in the order the reference's tensor
 // expressions imply; this file is compiled without floating-point contraction.
 #include "rdkv_common.h"
