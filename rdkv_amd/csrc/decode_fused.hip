@@ -1029,12 +1029,13 @@ merge_kernel(const RdkvUnit *__restrict__ units, const float *__restrict__ parti
 //    columns, and the first 64 zone C tokens' K and V rows (requested before the count is known:
 //    rows up to the buffer's end exist, a row past the count is discarded).  The parts of the
 //    preparation are dealt to different wavefronts;
-//  * a workgroup of eight wavefronts takes HW of a unit's G heads; wavefront w owns tokens
-//    8w .. 8w + 7 of every chunk of 64.  Both rows of a token are split over the same eight lanes (16-byte loads, 128 contiguous bytes per token and instruction), and every group of
-//    eight lanes keeps an online-softmax state of its own for each head, so the token loop exchanges
-//    nothing between tokens (a sum inside the eight lanes is all) and has no barrier; the next chunk is
-//    requested as soon as the registers are free, the other wavefronts work meanwhile (a second
-//    register set changed nothing at 700 tokens and took a resident workgroup);
+//  * a workgroup of eight wavefronts takes HW of a unit's G heads; wavefront w owns tokens 8w .. 8w + 7
+//    of every chunk of 64.  Both rows of a token are split over the same eight lanes (16-byte loads, 128
+//    contiguous bytes per token and instruction), and every group of eight lanes keeps an online-softmax
+//    state of its own for each head, so the token loop exchanges nothing between tokens (a sum inside the
+//    eight lanes is all) and has no barrier; the next chunk is requested as soon as the registers are free,
+//    the other wavefronts work meanwhile (a second register set changed nothing at 700 tokens and took a
+//    resident workgroup);
 //  * the 64 lane-group states and the zones A+B state are combined once, in a fixed order.
 // The step's own token never comes back through memory: its rotated key and its value are kept
 // in LDS and stand in for whatever the row's loads returned.

@@ -87,6 +87,7 @@ def _launch(attn_weights, V_2bit, V_4bit, V_8bit, V_scale, V_zp, seg_bounds_per_
     if w.stride(1) != 1:
         w = w.contiguous()
     assert out.dtype == torch.float32 and out.stride(1) == 1 and out.shape[1] == D
+    assert new is None or (new[1].shape[0] == H_kv and out.shape[0] == H_q), "new zone or output of another height"
     keep2, V2, v2h = _seg(V_2bit, D // 4)
     keep4, V4, v4h = _seg(V_4bit, D // 2)
     keep8, V8, v8h = _seg(V_8bit, D)

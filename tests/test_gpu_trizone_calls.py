@@ -81,6 +81,15 @@ def test_buffers_and_rows_that_do_not_fit_are_refused():
         fast_decode.trizone_attention(*args, kv, kv, 4, scores_buf=torch.empty(8, 48, device=DEV, dtype=torch.float16))
     with pytest.raises(RuntimeError):
         fast_decode.trizone_attention(torch.randn(10, 128, device=DEV), *args[1:], kv, kv, 4)
+    for rows in (4, 16):
+        with pytest.raises(RuntimeError):
+            fast_decode.trizone_attention(*args, kv, kv, 4, out=torch.empty(rows, 128, device=DEV))
+    with pytest.raises(RuntimeError):                                    # the layer has two KV heads, not four or one
+        fast_decode.trizone_attention(*args, kv.repeat(2, 1, 1), kv.repeat(2, 1, 1), 2)
+    with pytest.raises(RuntimeError):
+        fast_decode.trizone_attention(*args, kv[:1], kv[:1], 8)
+    with pytest.raises(RuntimeError):
+        fast_decode.trizone_attention(*args, kv, kv, 4, scores_buf=torch.empty(8, 48))
 
 
 @pytest.mark.parametrize("T,n_new", [(0, 9), (0, 1500), (50, 9), (50, 1500), (9000, 300), (9000, 1500)])
