@@ -385,6 +385,15 @@ int rdkv_stream_partition(RdkvUnit *units, int n_units, int n_groups, const doub
                           double cost_k_dword, double cost_item, const double *speed, int n_speed,
                           int multi_source, RdkvWork *work, int work_capacity, int32_t *groups, int *n_work);
 
+/* The decomposition for few units: every unit is cut on its own into runs of equal cost (costs as above,
+ * without an item cost), one work item and one workgroup each (the streaming launch then takes no group
+ * table).  The units share n_items runs so that the longest is as short as can be; every unit gets at
+ * least one, none more than its tiles or 96.  Written as by rdkv_stream_partition, without groups;
+ * work_capacity >= max(n_items, n_units).  costs[2]: of the longest run, of all tiles. */
+int rdkv_stream_partition_units(RdkvUnit *units, int n_units, int n_items, const double *cost_tile,
+                                double cost_k_dword, int multi_source, RdkvWork *work, int work_capacity,
+                                int *n_work, double *costs);
+
 /* k_scale_max and v_shift of every work item from its unit's largest scales (host memory):
  * scale_max[2 * unit] = largest K channel scale, [2 * unit + 1] = largest V token scale, as
  * rdkv_pack_layer_stream reports them.  v_shift: the smallest e >= 0 with scale * 2^(6 - e) < 2^15,

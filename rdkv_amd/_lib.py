@@ -68,6 +68,7 @@ SIGNATURES = {
                                            P, L, P, L, P]),
     "rdkv_stream_plan_layer": (I, [P, L, P, L, I, I, I, I, I, P, P, I, P]),
     "rdkv_stream_partition": (I, [P, I, I, P, ctypes.c_double, ctypes.c_double, P, I, I, P, I, P, P]),
+    "rdkv_stream_partition_units": (I, [P, I, I, P, ctypes.c_double, I, P, I, P, P]),
     "rdkv_stream_work_scales": (I, [P, I, P, I]),
     "rdkv_pack_layer_stream_ws_init": (I, [P, I, P]),
     "rdkv_pack_layer_stream": (I, [P, P, L, L, I, P, L, P, P, I, L, I, I, I, L, I, P, P, I, I, P, L, P, I, P, P]),

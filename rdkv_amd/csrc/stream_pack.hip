@@ -668,6 +668,119 @@ RDKV_API int rdkv_stream_plan_layer(const int32_t *tok_counts, int64_t tok_strid
   return RDKV_OK;
 }
 
+// The unit that merges an output row - the unit itself, or the first source of its row (which then carries
+// the row's item count, the others 0) - and its item range and the unit's descriptor in every work item.
+static void finish_work(RdkvUnit *units, int U, int multi_source, RdkvWork *work, int nw) {
+  std::vector<int32_t> merger((size_t)U);
+  if (multi_source) {
+    int first = 0;
+    for (int u = 0; u < U; ++u) {
+      if (u == 0 || units[u].q_row != units[u - 1].q_row) first = u;
+      else {
+        units[first].work_count += units[u].work_count;
+        units[u].work_count = 0;
+      }
+      merger[u] = first;
+    }
+  } else {
+    for (int u = 0; u < U; ++u) merger[u] = u;
+  }
+  for (int i = 0; i < nw; ++i) {
+    RdkvWork &w = work[i];
+    const int m = merger[(size_t)w.unit];
+    w.u = units[w.unit];
+    w.merge_unit = m;
+    w.merge_begin = units[m].work_begin;
+    w.merge_count = units[m].work_count;
+  }
+}
+
+// The other decomposition, for caches of few units: every unit is cut on its own, into runs of equal cost
+// (costs as in rdkv_stream_partition, without an item cost), and every run is a work item and a workgroup
+// of its own (no group table).  A unit gets as many of the n_items runs as its share of the cost asks for, at
+// least one, none more than its tiles or kMaxRuns: the longest run is as short as n_items of them can make it.
+// A workgroup that holds the end of one unit and the start of the next works through two items one after the
+// other, 4 us more than one of the same number of tiles, and every workgroup waits for the slowest: 8 units of
+// 4k / 16k / 32k tokens, a decode step 19.4 / 19.5 / 22.5 us with a boundary inside some workgroups, 15.1 / 16.6 /
+// 19.4 without; 256 units of 2k tokens 37.1 / 26.8.
+constexpr int kMaxRuns = 96;      // (the merge takes up to 128 partials of a row in one pass)
+RDKV_API int rdkv_stream_partition_units(RdkvUnit *units, int n_units, int n_items, const double *cost_tile,
+                                         double cost_k_dword, int multi_source, RdkvWork *work, int work_capacity,
+                                         int *n_work, double *costs) {
+  const char *fn = "rdkv_stream_partition_units";
+  RDKV_REQUIRE(units && cost_tile && work && n_work && costs && n_units >= 0 && n_items >= 1, "%s: bad arguments", fn);
+  RDKV_REQUIRE(work_capacity >= std::max(n_items, n_units), "%s: work table too small", fn);
+  const int U = n_units;
+  std::vector<double> tile_cost((size_t)U * 4), unit_cost((size_t)U, 0.0);
+  std::vector<int64_t> tiles((size_t)U * 4), unit_tiles((size_t)U, 0);
+  double all = 0.0;
+  for (int u = 0; u < U; ++u) {
+    const double k_row = cost_k_dword * (double)((int64_t)units[u].d8 + units[u].d4 + units[u].d2);
+    for (int c = 0; c < 4; ++c) {
+      RDKV_REQUIRE(units[u].n_tok[c] >= 0, "%s: negative token count", fn);
+      tile_cost[4 * u + c] = k_row + cost_tile[c];
+      tiles[4 * u + c] = ((int64_t)units[u].n_tok[c] + RDKV_TILE - 1) / RDKV_TILE;
+      unit_tiles[u] += tiles[4 * u + c];
+      unit_cost[u] += tile_cost[4 * u + c] * (double)tiles[4 * u + c];
+    }
+    RDKV_REQUIRE(unit_tiles[u] <= 0x7fffffffLL, "%s: too many tiles", fn);
+    all += unit_cost[u];
+  }
+  // the shortest run length that n_items runs can keep to, by bisection above the mean
+  auto runs_of = [&](int u, double length) -> int64_t {
+    if (unit_tiles[u] == 0 || !(length > 0.0)) return 1;
+    const double k = ceil(unit_cost[u] / length), most = (double)std::min<int64_t>(kMaxRuns, unit_tiles[u]);
+    return std::max<int64_t>(1, (int64_t)std::min(k, most));
+  };
+  auto fit = [&](double length) {
+    int64_t n = 0;
+    for (int u = 0; u < U; ++u) n += runs_of(u, length);
+    return n <= n_items;
+  };
+  double length = all, low = all / n_items;      // (`all` leaves every unit one run)
+  if (fit(low)) length = low;
+  else
+    for (int it = 0; it < 50; ++it) {
+      const double mid = 0.5 * (length + low);
+      (fit(mid) ? length : low) = mid;
+    }
+  int nw = 0;
+  double longest = 0.0;
+  for (int u = 0; u < U; ++u) {
+    const int64_t k = runs_of(u, length);
+    units[u].work_begin = nw;
+    units[u].work_count = (int32_t)k;
+    int64_t t = 0, left = tiles[4 * u];      // tiles given out; tiles left of class c
+    double acc = 0.0;
+    int c = 0;
+    for (int64_t i = 0; i < k; ++i) {
+      RdkvWork &w = work[nw++];
+      memset(&w, 0, sizeof(w));
+      w.unit = u;
+      w.tile_begin = (int32_t)t;
+      // run i goes to the tile boundary nearest (i + 1) / k of the unit's cost, takes one tile at least and
+      // leaves one to every later run
+      const double from = acc, want = unit_cost[u] * (double)(i + 1) / (double)k;
+      const int64_t last = unit_tiles[u] - (k - 1 - i);
+      for (bool first = true; t < last; first = false) {
+        while (left == 0) left = tiles[4 * u + ++c];
+        const double cost = tile_cost[4 * u + c];
+        if (!first && i + 1 < k && acc + 0.5 * cost > want) break;
+        acc += cost;
+        --left;
+        ++t;
+      }
+      w.tile_end = (int32_t)t;
+      longest = std::max(longest, acc - from);
+    }
+  }
+  finish_work(units, U, multi_source, work, nw);
+  *n_work = nw;
+  costs[0] = longest;
+  costs[1] = all;
+  return RDKV_OK;
+}
+
 // Host side of the fused kernel's work decomposition (no GPU work): cut the unit-major, class-minor
 // sequence of 64-token tiles into n_groups contiguous runs of equal modelled cost (shares
 // proportional to speed[g % n_speed]), one run per workgroup; a run that crosses a unit boundary
@@ -776,29 +889,7 @@ RDKV_API int rdkv_stream_partition(RdkvUnit *units, int n_units, int n_groups, c
       groups[gg] = i;
     }
   }
-  // the unit that merges an output row: the unit itself, or the first source of its row
-  std::vector<int32_t> merger((size_t)U);
-  if (multi_source) {
-    int first = 0;
-    for (int u = 0; u < U; ++u) {
-      if (u == 0 || units[u].q_row != units[u - 1].q_row) first = u;
-      else {
-        units[first].work_count += units[u].work_count;
-        units[u].work_count = 0;
-      }
-      merger[u] = first;
-    }
-  } else {
-    for (int u = 0; u < U; ++u) merger[u] = u;
-  }
-  for (int i = 0; i < nw; ++i) {
-    RdkvWork &w = work[i];
-    const int m = merger[(size_t)w.unit];
-    w.u = units[w.unit];
-    w.merge_unit = m;
-    w.merge_begin = units[m].work_begin;
-    w.merge_count = units[m].work_count;
-  }
+  finish_work(units, U, multi_source, work, nw);
   *n_work = nw;
   return RDKV_OK;
 }

@@ -118,6 +118,12 @@ class StreamCache:
         return self.units.device
 
     @property
+    def groups_arg(self) -> tuple:
+        """The group table and group count of the fused entry points.  A group per work item needs no
+        table: the workgroup's index is the item's, one dependent load less before anything else."""
+        return (None, 0) if self.n_groups == self.n_work else (_lib.ptr(self.groups), self.n_groups)
+
+    @property
     def row_dwords_arg(self) -> int:
         """The ``max_row_dwords`` argument of the fused entry points: the longest K row, and in
         bits 8 and up the one row shape of all units (the library has kernels for some shapes)."""
@@ -588,6 +594,21 @@ def _partition_units(units_np: np.ndarray, n_groups: int, cost: dict, multi_sour
     return units_np, work_np[:int(n_work[0])], groups_np
 
 
+def _partition_whole_units(units_np: np.ndarray, n_items: int, cost: dict, multi_source: bool):
+    """As ``_partition_units``, every unit cut on its own: at most ``n_items`` runs in all (one per unit at
+    least), a workgroup each (``rdkv_stream_partition_units``); and the modelled cost of the longest run and
+    of all tiles."""
+    units_np = np.ascontiguousarray(units_np).copy()
+    n_items = max(n_items, len(units_np), 1)
+    work_np = np.empty(n_items, dtype=WORK_DTYPE)
+    tile, n_work, costs = np.asarray(cost["tile"], dtype=np.float64), np.zeros(1, dtype=np.int32), np.zeros(2)
+    _lib.check(_lib.load().rdkv_stream_partition_units(
+        units_np.ctypes.data, len(units_np), n_items, tile.ctypes.data, float(cost["k_dword"]),
+        int(bool(multi_source)), work_np.ctypes.data, len(work_np), n_work.ctypes.data, costs.ctypes.data))
+    n = int(n_work[0])
+    return (units_np, work_np[:n], np.arange(n + 1, dtype=np.int32)), float(costs[0]), float(costs[1])
+
+
 def _finish_cache(units_np: np.ndarray, blobs, G: int, H_q: int, stream_bytes: int, kv_algo_bytes: int,
                   scale_max: np.ndarray, *, multi_source: bool, work_bytes, n_groups, groups_per_cu: int,
                   cost) -> StreamCache:
@@ -620,6 +641,8 @@ def _finish_caches(specs) -> List[StreamCache]:
             units_np = units_np[order]
         tiles_np = -(-units_np["n_tok"].astype(np.int64) // TILE)
         R_np = (units_np["d8"] + units_np["d4"] + units_np["d2"]).astype(np.int64)
+        model = cost or (DEFAULT_COST if G <= 4 else DEFAULT_COST_TWO_HEAD_GROUPS)
+        whole = None
         if work_bytes is None and n_groups is None:
             # Every group costs a fixed amount (set-up, its partials, their merge), every tile a fixed
             # amount per group that shares the stream: the step time a*tiles/n + b*n is least at
@@ -627,8 +650,22 @@ def _finish_caches(specs) -> List[StreamCache]:
             # caches get one group per compute unit, tiny ones at least 4 tiles per group.
             total_tiles = int(tiles_np.sum())
             n_groups = max(1, min(opt["groups_per_cu"] * cus, int(round((6.0 * total_tiles) ** 0.5)), total_tiles // 4))
-        model = cost or (DEFAULT_COST if G <= 4 else DEFAULT_COST_TWO_HEAD_GROUPS)
-        if work_bytes is None:
+            # No more units than compute units: runs that keep to one unit, unless they come out more uneven
+            # than the second item of a workgroup costs.  A step costs a * tiles / runs + b * runs / rows (the
+            # partials a row's merge reads), least at runs ~ sqrt(tiles * rows); measured with 32 / 64 / 96 / 128 /
+            # 192 / 256 runs: 8 units of 4k tokens 17.4 / 15.9 / 15.1 / 15.1 / 15.5 / 15.9 us, of 16k 27.4 / 21.0 / 18.4 /
+            # 17.5 / 16.8 / 16.9; 2 of 4k 14.9 / 15.6 / 16.1 / 16.8, 4 of 32k 26.7 / 21.3 / 19.0 / 18.4 / 18.2 / 18.6 (in
+            # runs across units 19.4, 19.5, 19.1, 19.8).  More than one per compute unit: 23.7 against 14.9.
+            # 64 units of 32k tokens, four runs each, are uneven: 58.2 us against 56.6.
+            n_rows = len(np.unique(units_np["q_row"])) if multi_source else len(units_np)
+            if 0 < len(units_np) <= cus and opt["groups_per_cu"] == 1:
+                whole, longest, total = _partition_whole_units(
+                    units_np, min(cus, int(round((5.3 * total_tiles * n_rows) ** 0.5))), model, multi_source)
+                if longest > 0.97 * (total + model["item"] * len(units_np)) / n_groups:
+                    whole = None
+        if whole is not None:
+            units_np, work_np, groups_np = whole
+        elif work_bytes is None:
             units_np, work_np, groups_np = _partition_units(units_np, int(n_groups), model, multi_source)
         else:
             work_np, groups_np, wb, wc = partition_work(tiles_np, R_np, n_groups=n_groups, work_bytes=work_bytes,
@@ -832,7 +869,7 @@ def decode_attn_fused(cache: StreamCache, q: torch.Tensor, out: Optional[torch.T
     if one_launch:
         _lib.check(lib.rdkv_decode_fused_one_launch(
             None, cache.units.data_ptr(), cache.n_units, cache.work.data_ptr(), cache.n_work,
-            _lib.ptr(cache.groups), cache.n_groups, cache.row_dwords_arg,
+            *cache.groups_arg, cache.row_dwords_arg,
             q.data_ptr(), _lib.DTYPE_CODE[q.dtype], q.stride(0), cache.G, _lib.ptr(rc), _lib.ptr(rs), rope_dt,
             out.data_ptr(), out.stride(0), lse.data_ptr(), ws.data_ptr(), ws.numel(), cache.tickets.data_ptr(),
             stream))
@@ -840,7 +877,7 @@ def decode_attn_fused(cache: StreamCache, q: torch.Tensor, out: Optional[torch.T
     if zone_c is None:
         _lib.check(lib.rdkv_decode_fused(
             None, cache.units.data_ptr(), cache.n_units, cache.work.data_ptr(), cache.n_work,
-            _lib.ptr(cache.groups), cache.n_groups, cache.row_dwords_arg,
+            *cache.groups_arg, cache.row_dwords_arg,
             q.data_ptr(), _lib.DTYPE_CODE[q.dtype], q.stride(0), cache.G, _lib.ptr(rc), _lib.ptr(rs), rope_dt,
             out.data_ptr(), out.stride(0), lse.data_ptr(), ws.data_ptr(), ws.numel(), stream))
         return out, lse
@@ -856,7 +893,7 @@ def decode_attn_fused(cache: StreamCache, q: torch.Tensor, out: Optional[torch.T
         assert counts.dtype == torch.int32 and counts.numel() == n_kv_rows and counts.is_contiguous()
     _lib.check(lib.rdkv_decode_fused_partials(
         None, cache.units.data_ptr(), cache.n_units, cache.work.data_ptr(), cache.n_work,
-        _lib.ptr(cache.groups), cache.n_groups, cache.row_dwords_arg,
+        *cache.groups_arg, cache.row_dwords_arg,
         q.data_ptr(), _lib.DTYPE_CODE[q.dtype], q.stride(0), cache.G, _lib.ptr(rc), _lib.ptr(rs), rope_dt,
         ws.data_ptr(), ws.numel(), stream))
     n_new = int(K_new.shape[1])

@@ -261,6 +261,54 @@ def test_stream_plan_layer_matches_the_slot_plan_and_lays_sections_out_in_order(
         sc._plan_entry_units([(1, 0, 0, 0)], [(100, 100, 0)], 100, 100, 0, 1)
 
 
+@pytest.mark.parametrize("multi", [False, True])
+def test_partition_by_whole_units(multi):
+    """Runs that keep to one unit: every tile once and in order, a workgroup per item, no more items than
+    asked for (one per unit at least, none without tiles except an empty unit's), runs no longer than the
+    best even cut allows, the row's first source carrying the count; the costs reported."""
+    from rdkv_amd import stream_cache as sc
+    rng = np.random.default_rng(11)
+    for case in range(60):
+        U = int(rng.integers(1, 30))
+        units = np.zeros(U, dtype=sc.UNIT_DTYPE)
+        units["n_tok"] = rng.choice([0, 0, 1, 64, 65, 300, 5000, 40000], size=(U, 4))
+        if case == 3:
+            units["n_tok"] = 0
+        units["d8"], units["d4"], units["d2"] = rng.integers(0, 12, U), rng.integers(0, 10, U), rng.integers(0, 8, U)
+        units["q_row"] = np.sort(rng.integers(0, max(1, U // 3), U)) * 8 if multi else np.arange(U) * 8
+        n_items = int(rng.choice([1, U, 2 * U, 64, 256]))
+        cost = sc.DEFAULT_COST if case % 2 else sc.DEFAULT_COST_TWO_HEAD_GROUPS
+        (got, work, groups), longest, total = sc._partition_whole_units(units, n_items, cost, multi)
+        tiles = -(-units["n_tok"].astype(np.int64) // 64)
+        R = (units["d8"] + units["d4"] + units["d2"]).astype(np.int64)
+        begin = np.searchsorted(work["unit"], np.arange(U), side="left")
+        count = np.searchsorted(work["unit"], np.arange(U), side="right") - begin
+        _check_partition(tiles, R, work, None, begin, count)
+        assert np.array_equal(groups, np.arange(len(work) + 1)) and len(work) <= max(n_items, U) and count.max() <= 96
+        costs = sc._tile_costs(tiles, R, {**cost, "item": 0.0})
+        cum = np.concatenate([[0.0], np.cumsum(costs)])
+        start = np.concatenate([[0], np.cumsum(tiles.sum(axis=1))])
+        runs = cum[start[work["unit"]] + work["tile_end"]] - cum[start[work["unit"]] + work["tile_begin"]]
+        assert np.isclose(runs.max(), longest) and np.isclose(cum[-1], total)
+        # a unit's runs are even up to a tile; another split of the items over the units is no shorter
+        unit_cost = np.bincount(work["unit"], weights=runs, minlength=U)
+        biggest = (np.asarray(cost["tile"]).max() + cost["k_dword"] * R)
+        assert (runs <= unit_cost[work["unit"]] / count[work["unit"]] + 2 * biggest[work["unit"]] + 1e-6).all()
+        even, most = unit_cost / count, np.minimum(tiles.sum(axis=1), 96)
+        slowest = int(even.argmax())
+        if count[slowest] < most[slowest]:      # one run more for the slowest unit does not fit at this length
+            needed = np.maximum(1, np.minimum(most, np.ceil(unit_cost / max(even.max(), 1e-9) * (1 + 1e-6)))).sum()
+            assert needed + 1 > n_items or needed >= len(work)
+        first = np.concatenate([[True], np.diff(units["q_row"]) != 0]) if multi else np.ones(U, dtype=bool)
+        merger = np.maximum.accumulate(np.where(first, np.arange(U), 0))
+        sums = np.bincount(merger, weights=count, minlength=U).astype(np.int64)
+        assert np.array_equal(got["work_begin"], begin) and np.array_equal(got["work_count"], sums)
+        assert np.array_equal(work["merge_unit"], merger[work["unit"]])
+        assert np.array_equal(work["merge_count"], sums[merger[work["unit"]]])
+        assert np.array_equal(work["merge_begin"], begin[merger[work["unit"]]])
+        assert work["u"].tobytes() == got[work["unit"]].tobytes()
+
+
 def test_library_partition_matches_partition_work():
     """The library's host-side work partition against ``partition_work`` and the merge bookkeeping
     restated here, on random unit tables: empty units (leading, trailing, in runs), single-tile
