@@ -279,23 +279,31 @@ __device__ __forceinline__ void merge_unit(const float *partials, int work_begin
   }
 }
 
-constexpr int kBatch = 2;  // work items a workgroup handles between two barriers
+__device__ __forceinline__ float row16_sum(float v) {      // over the 16 lanes of a row, in every lane
+  v += rdkv_dpp_mov<0x128>(v);
+  v += rdkv_dpp_mov<0x124>(v);
+  v += rdkv_dpp_mov<0x122>(v);
+  return v + rdkv_dpp_mov<0x121>(v);
+}
 
-template <int NH, int NW>
+constexpr int kSlotParts = (4 * RDKV_MAX_STEPS + 63) / 64;   // wavefronts that cover the slots of a head
+
+// KB: work items a workgroup handles between two barriers.
+template <int NH, int NW, int KB>
 struct Smem {
-  alignas(16) _Float16 qs[kBatch][RDKV_MAX_STEPS][NH][2][4][4];  // [item][step][head group][hi|lo][head][k]
+  alignas(16) _Float16 qs[KB][RDKV_MAX_STEPS][NH][2][4][4];  // [item][step][head group][hi|lo][head][k]
   alignas(16) _Float16 p[NW][16][NH][4][4];                      // [wave][quad][head group][head][k]
-  float bias[kBatch][NH * 4];
-  float qmaxw[kBatch][NH * 4 * 2];                               // max |q| per 64 query elements (half a head)
-  float kup[kBatch];                                             // 2^e: the item's q*scale operands carry 2^-e
-  float qraw[kBatch][NH * 4][kD];                                // the unit's query rows as loaded
-  float slot_scale[kBatch][4 * RDKV_MAX_STEPS], slot_zp[kBatch][4 * RDKV_MAX_STEPS];
-  uint16_t slot_channel[kBatch][4 * RDKV_MAX_STEPS];
+  float bias[KB][NH * 4][kSlotParts];                            // sum of zp * qs over 64 slots each
+  float qmaxw[KB][NH * 4 * 2];                               // max |q| per 64 query elements (half a head)
+  float kup[KB];                                             // 2^e: the item's q*scale operands carry 2^-e
+  float qraw[KB][NH * 4][kD];                                // the unit's query rows as loaded
+  float slot_scale[KB][4 * RDKV_MAX_STEPS], slot_zp[KB][4 * RDKV_MAX_STEPS];
+  uint16_t slot_channel[KB][4 * RDKV_MAX_STEPS];
   int progress[16];                                              // tiles done per wavefront
-  int ticket[kBatch];                                            // arrival order of the batch's partials at their units
-  float wm[kBatch][NW][NH * 4];                                  // per-wavefront results of an item
-  float wl[kBatch][NW][NH * 4];
-  alignas(16) float wo[kBatch][NW][NH * 4][kD];                  // (also the scratch of a merge inside the launch)
+  int ticket[KB];                                            // arrival order of the batch's partials at their units
+  float wm[KB][NW][NH * 4];                                  // per-wavefront results of an item
+  float wl[KB][NW][NH * 4];
+  alignas(16) float wo[KB][NW][NH * 4][kD];                  // (also the scratch of a merge inside the launch)
 };
 
 // Register images of the loads in flight.  The K row of the lane's token and the {scale,zp}
@@ -332,7 +340,7 @@ __device__ __forceinline__ T sel4(int c, T a0, T a1, T a2, T a3) {
 
 // A workgroup fills a whole compute unit: 4 * WPE wavefronts (WPE per SIMD), all of the same
 // age, so the hardware's oldest-first issue order cannot favour one part of the work.
-// It walks the work items of its group kBatch at a time: the query operands of the batch are
+// It walks the work items of its group KB at a time: the query operands of the batch are
 // staged first, then every wavefront runs through its tiles of all items of the batch without
 // waiting for the others (wavefronts drift apart by several tiles over an item; a barrier per
 // item cost 12-15 us of idle time each), parks its result per item in LDS, and one barrier
@@ -342,7 +350,9 @@ __device__ __forceinline__ T sel4(int c, T a0, T a1, T a2, T a3) {
 // with fixed numbers, its LDS operands requested two steps ahead, and RMAX is the row rounded up
 // to whole 16-byte chunks.  A unit of another shape is skipped (none of its tiles is read) and
 // its partials are written as NaN (merged output rows: NaN, lse -inf).
-template <int NH, int RMAX, int WPE, bool MERGE, int SHAPE = 0>
+// KB = 1 is the kernel of launches without a group table, a workgroup per item: half of the staging and of
+// the result buffers.  Its set-up is what a call of one layer waits for.
+template <int NH, int RMAX, int WPE, bool MERGE, int SHAPE, int KB>
 __global__ void __launch_bounds__(256 * WPE) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
 decode_fused_kernel(const uint8_t *__restrict__ blob,
                     const RdkvWork *__restrict__ work, const int32_t *__restrict__ groups,
@@ -351,13 +361,13 @@ decode_fused_kernel(const uint8_t *__restrict__ blob,
                     float *partials, int32_t *tickets, float *__restrict__ out, int64_t out_stride,
                     float *__restrict__ lse) {
   constexpr int kWaves = 4 * WPE, kThreads = 64 * kWaves;
-  __shared__ Smem<NH, kWaves> sm;
+  __shared__ Smem<NH, kWaves, KB> sm;
   const int tid = threadIdx.x, lane = tid & 63;
   // the wavefront index is uniform; say so, or every tile-level decision becomes per-lane
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 3, lb = lane >> 2;
-  const int item_begin = groups ? groups[blockIdx.x] : (int)blockIdx.x;
-  const int item_end = groups ? groups[blockIdx.x + 1] : (int)blockIdx.x + 1;
+  const int item_begin = KB > 1 && groups ? groups[blockIdx.x] : (int)blockIdx.x;
+  const int item_end = KB > 1 && groups ? groups[blockIdx.x + 1] : (int)blockIdx.x + 1;
   constexpr int kD8 = (SHAPE >> 16) & 255, kD4 = (SHAPE >> 8) & 255, kD2 = SHAPE & 255, kR = kD8 + kD4 + kD2;
   static_assert(SHAPE == 0 || (kR >= 1 && RMAX == (kR + 3) / 4 * 4), "RMAX of a fixed shape is its row in whole chunks");
 
@@ -467,8 +477,8 @@ decode_fused_kernel(const uint8_t *__restrict__ blob,
     }
   };
 
-  for (int batch = item_begin; batch < item_end; batch += kBatch) {
-  const int nb = item_end - batch < kBatch ? item_end - batch : kBatch;
+  for (int batch = item_begin; batch < item_end; batch += KB) {
+  const int nb = item_end - batch < KB ? item_end - batch : KB;
   // Index values used only before and after the tile loops are re-derived per batch from a
   // fresh read of the lane id: hoisted out of the loop (or derived from the thread id the
   // kernel was entered with) they would stay live across the tile loops and push the kernel
@@ -487,10 +497,10 @@ decode_fused_kernel(const uint8_t *__restrict__ blob,
   it = load_item(batch);
   set_tile(c0, it.tile_begin + wave);
   constexpr int kQPer = (NH * 4 * kD + kThreads - 1) / kThreads;   // query elements per thread
-  uint2 st_slot[kBatch];
-  uint32_t st_q[kBatch][kQPer], st_qo[kBatch][kQPer], st_cs[kBatch][kQPer], st_sn[kBatch][kQPer];
+  uint2 st_slot[KB];
+  uint32_t st_q[KB][kQPer], st_qo[KB][kQPer], st_cs[KB][kQPer], st_sn[KB][kQPer];
 #pragma unroll
-  for (int b = 0; b < kBatch; ++b) {
+  for (int b = 0; b < KB; ++b) {
     const Item sb = load_item(batch + (b < nb ? b : 0));
     const uint2 *tab = reinterpret_cast<const uint2 *>(sb.qtab_base);
     st_slot[b] = tab[tid_o < 4 * sb.NS ? tid_o : 0];
@@ -512,7 +522,7 @@ decode_fused_kernel(const uint8_t *__restrict__ blob,
   issue_k(c0.ti, c0.valid);
   issue_v(c0, va, c0.valid);
 #pragma unroll
-  for (int b = 0; b < kBatch; ++b) {
+  for (int b = 0; b < KB; ++b) {
     if (tid_o < 4 * RDKV_MAX_STEPS) {
       sm.slot_channel[b][tid_o] = (uint16_t)(st_slot[b].x & 0xffffu);
       sm.slot_scale[b][tid_o] = (float)__builtin_bit_cast(_Float16, (uint16_t)(st_slot[b].x >> 16));
@@ -538,25 +548,31 @@ decode_fused_kernel(const uint8_t *__restrict__ blob,
         }
         sm.qraw[b][i >> 7][c] = v;
         // (a wavefront holds 64 consecutive elements of one head: uniform branch, whole-wave maximum)
-        const float am = rdkv_wave_max(fabsf(v));
+        const float am = wave_reduce<true>(fabsf(v));
         if (lane_o == 0) sm.qmaxw[b][i >> 6] = am;
       }
     }
   }
   __syncthreads();
-  for (int b = 0; b < nb; ++b) {
+  // A wavefront per (item, head, 64 slots): the operands and what they add to the bias
+  // bias[h] = sum_slot qs[h][slot] * zp[slot] / 2^8, whose parts are added, in order, where it is used.
+  // (Together with the combination below and one item's staging instead of two, against operands dealt to
+  // the threads one by one, the bias behind a barrier of its own and sums through the LDS crossbar: 3 us of
+  // every workgroup; one layer of 8 x 4k / 32k tokens, the launch 11.2 / 15.6 -> 8.4 / 12.4 us, a 128k step
+  // of eight heads per group 36.8 -> 33.2.)
+  for (int task = wave; task < nb * NH * 4 * kSlotParts; task += kWaves) {
+    const int part = task % kSlotParts, head = task / kSlotParts % (NH * 4), b = task / (kSlotParts * NH * 4);
     const Item ib = load_item(batch + b);
-    const int nslot = 4 * ib.NS;
     // the item's power of two: 2^-e brings the largest possible |q * scale * 2^8| below 2^15
-    float qm = 0.0f;
-    for (int w2 = 0; w2 < 2 * G; ++w2) qm = fmaxf(qm, sm.qmaxw[b][w2]);
+    const float qm = wave_reduce<true>(lane_o < 2 * G ? sm.qmaxw[b][lane_o < 2 * G ? lane_o : 0] : 0.0f);
     const float bound = qm * ib.k_scale_max * (kLog2eOverSqrtD * kQScale);
     int e = (int)((__float_as_uint(bound) >> 23) & 0xffu) - 127 - 14;
     e = bound < kOperandLimit ? 0 : (e > 100 ? 100 : e);
-    const float down = __uint_as_float((uint32_t)(127 - e) << 23);
-    if (tid_o == 0) sm.kup[b] = __uint_as_float((uint32_t)(127 + e) << 23);
-    for (int i = tid_o; i < nslot * NH * 4; i += kThreads) {
-      const int slot = i % nslot, head = i / nslot;
+    const float down = __uint_as_float((uint32_t)(127 - e) << 23), up = __uint_as_float((uint32_t)(127 + e) << 23);
+    if (part == 0 && lane_o == 0) sm.kup[b] = up;
+    const int slot = part * 64 + lane_o;
+    float bsum = 0.0f;
+    if (slot < 4 * ib.NS) {
       _Float16 hi = (_Float16)0.0f, lo = (_Float16)0.0f;
       if (head < G) {
         // two fp16 terms carry ~22 bits of q*scale: one fp16 alone loses the outlier channels'
@@ -565,22 +581,13 @@ decode_fused_kernel(const uint8_t *__restrict__ blob,
                         (kLog2eOverSqrtD * kQScale) * down;
         hi = (_Float16)x;
         lo = (_Float16)(x - (float)hi);
+        bsum = ((float)hi + (float)lo) * sm.slot_zp[b][slot];
       }
       sm.qs[b][slot >> 2][head >> 2][0][head & 3][slot & 3] = hi;
       sm.qs[b][slot >> 2][head >> 2][1][head & 3][slot & 3] = lo;
     }
-  }
-  __syncthreads();
-  // bias[h] = sum_slot qs[h][slot] * zp[slot] / 2^8, one wavefront per (item, head), fixed tree
-  for (int bh = wave; bh < nb * NH * 4; bh += kWaves) {
-    const int b = bh / (NH * 4), head = bh - b * (NH * 4);
-    const int nslot = 4 * load_item(batch + b).NS;
-    float bsum = 0.0f;
-    for (int slot = lane_o; slot < nslot; slot += 64)
-      bsum += ((float)sm.qs[b][slot >> 2][head >> 2][0][head & 3][slot & 3] +
-               (float)sm.qs[b][slot >> 2][head >> 2][1][head & 3][slot & 3]) * sm.slot_zp[b][slot];
-    bsum = rdkv_wave_sum(bsum);
-    if (lane_o == 0) sm.bias[b][head] = bsum * (1.0f / kQScale) * sm.kup[b];
+    bsum = wave_reduce<false>(bsum);
+    if (lane_o == 0) sm.bias[b][head][part] = bsum * (1.0f / kQScale) * up;
   }
   __syncthreads();
 
@@ -602,7 +609,9 @@ decode_fused_kernel(const uint8_t *__restrict__ blob,
     m_run[hg] = -INFINITY;
     l_run[hg] = 0.0f;
     zb_run[hg] = 0.0f;
-    bias_own[hg] = sm.bias[b][hg * 4 + ln];
+    bias_own[hg] = 0.0f;
+#pragma unroll
+    for (int part = 0; part < kSlotParts; ++part) bias_own[hg] += sm.bias[b][hg * 4 + ln][part];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       accq[hg][j] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -937,18 +946,18 @@ decode_fused_kernel(const uint8_t *__restrict__ blob,
   for (int b = 0; b < nb; ++b) {
     float *part = partials + (int64_t)(batch + b) * G * kPartialStride;
     for (int i = tid_o; i < G * kD; i += kThreads) {
-      const int h = i >> 7, d = i & 127;
-      float M = sm.wm[b][0][h];
+      const int h = __builtin_amdgcn_readfirstlane(i >> 7), d = i & 127;
+      // lane w of every row of sixteen takes wavefront w's maximum and sum; its factor reaches the
+      // columns by lane reads (instead of sixteen exponentials and 32 dependent LDS reads per thread)
+      const int lw = lane_o & 15;
+      const float mw = lw < kWaves ? sm.wm[b][lw < kWaves ? lw : 0][h] : -INFINITY;
+      float M = rdkv_row16_max(mw);
+      const float f = mw == -INFINITY ? 0.0f : fast_exp2(mw - M);  // idle wavefront contributes nothing
+      const float l = row16_sum(f * (lw < kWaves ? sm.wl[b][lw < kWaves ? lw : 0][h] : 0.0f));
+      float o = 0.0f;
 #pragma unroll
-      for (int w = 1; w < kWaves; ++w) M = fmaxf(M, sm.wm[b][w][h]);
-      float o = 0.0f, l = 0.0f;
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const float mw = sm.wm[b][w][h];
-        const float f = mw == -INFINITY ? 0.0f : exp2f(mw - M);  // idle wavefront contributes nothing
-        o += f * sm.wo[b][w][h][d];
-        l += f * sm.wl[b][w][h];
-      }
+      for (int w = 0; w < kWaves; ++w)
+        o = fmaf(__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), w)), sm.wo[b][w][h][d], o);
       if (SHAPE != 0 && !load_item(batch + b).shape_ok) o = M = __builtin_nanf("");
       pstore(part + h * kPartialStride + d, o);
       if (d == 0) {
@@ -1553,14 +1562,15 @@ static int launch_fused(const char *fn, const uint8_t *blob, const RdkvUnit *uni
   // keeps everything in registers; spilling costs far more than the lost occupancy.
   // (the variant that merges in the launch is a kernel of its own: the merge's registers would
   // otherwise push the two-launch form into scratch memory)
-#define RDKV_LAUNCH_FUSED_M(NH, RMAX, WPE, MERGE, SHAPE)                                                      \
-  hipLaunchKernelGGL((decode_fused_kernel<NH, RMAX, WPE, MERGE, SHAPE>), dim3(n_wg), dim3(256 * WPE), 0, s,   \
+#define RDKV_LAUNCH_FUSED_M(NH, RMAX, WPE, MERGE, SHAPE, KB)                                                  \
+  hipLaunchKernelGGL((decode_fused_kernel<NH, RMAX, WPE, MERGE, SHAPE, KB>), dim3(n_wg), dim3(256 * WPE), 0, s,   \
                      blob, work, groups, q, q_dtype, q_stride_row, G, rope_cos, rope_sin, rope_dtype,         \
                      partials, tickets, out, out_stride_row, lse)
 #define RDKV_LAUNCH_FUSED_SHAPE(NH, RMAX, WPE, SHAPE)                                                      \
   do {                                                                                                     \
-    if (tickets) RDKV_LAUNCH_FUSED_M(NH, RMAX, WPE, true, SHAPE);                                          \
-    else RDKV_LAUNCH_FUSED_M(NH, RMAX, WPE, false, SHAPE);                                                 \
+    if (tickets) RDKV_LAUNCH_FUSED_M(NH, RMAX, WPE, true, SHAPE, 2);                                       \
+    else if (groups) RDKV_LAUNCH_FUSED_M(NH, RMAX, WPE, false, SHAPE, 2);                                  \
+    else RDKV_LAUNCH_FUSED_M(NH, RMAX, WPE, false, SHAPE, 1);                                              \
   } while (0)
 #define RDKV_LAUNCH_FUSED_WPE(NH, RMAX, WPE) RDKV_LAUNCH_FUSED_SHAPE(NH, RMAX, WPE, 0)
   // Row shapes with a kernel of their own: every channel at 8, at 4 or at 2 bits, and the 4- / 2-bit
