@@ -876,206 +876,229 @@ softmax_rows_split_kernel(const float *__restrict__ so, int64_t so_sh, const flo
 }
 
 // ---------------------------------------------------------------------------
-// V weighted sum.  grid = (kVChunks, H_kv), block = 4 wavefronts.
-// Each class of the head's tokens (2-bit | 4-bit | 8-bit | fp16 zone B) is cut into kVChunks equal
-// pieces and a workgroup sums one piece of every class; partial sums go to the workspace and are
-// added in chunk order by v_reduce_kernel.  Every class is read with wide loads: eight lanes share a
-// quantized token (4 / 8 / 16 bytes per lane for 2 / 4 / 8 bit, sixteen channels each), sixteen
-// lanes an fp16 token (16 bytes, eight channels each), so one load instruction of a wavefront
-// covers eight (four) tokens.  A lane accumulates its channels for GB query heads; the token
-// lanes are folded with shuffles, the wavefronts through LDS, always in the same order.
+// V weighted sum.  grid = (kVChunks, H_kv, quads of query heads), block = 4 wavefronts.
+// A step is 64 consecutive tokens of a quantized class of the head (2 | 4 | 8 bit) or 32 of the fp16 zone B;
+// the wavefronts of a head take its steps in turn, the next step's loads in flight under a step's arithmetic.
+// Eight lanes share four tokens: lane li owns channels 16 li .. + 15 in every class (in a 2- or 4-bit row
+// these are one field of sixteen bytes), 16 bytes of each token per load (fp16: two).
+// The sums run on v_mfma_f32_4x4x4_16b_f16 (16 blocks of 4 heads x 4 tokens x 4 channels):
+// * values: the codes of two tokens, one byte permute and one multiply-add per pair.  An integer below 256
+//   in an fp16 register is that integer times 2^-24; times 2^15 it is a normal number.  (The matrix cores
+//   take subnormals, but drop bits of their products that normal numbers keep: 3e-6 of the result.)  Half of
+//   the largest code is taken off it and off the zero point: smaller sums that cancel;
+// * weights (times the token's scale): an fp16 pair, value and remainder, after a power of two per head
+//   that puts the largest weight so far at 2^11 .. 2^15: 22 bits of a weight and at least 2^-36 of the largest,
+//   which is what fp32 sums keep of it.  A larger weight rescales the sums (a few times per wavefront).
+// Error against 64 bits over random layers of 1.5k .. 128k tokens: 1.1e-7 .. 2.9e-7 of the result in the 2-norm,
+// with fp32 products and sums of uncentred codes 1.4e-7 .. 5.7e-7.
+// What bounds it: set-up and the latency of a few steps per wavefront at 32k, loads at 128k.  On the vector
+// ALU (a conversion and a multiply-add per head and code, 5.5 instructions against 1.5 and half a matrix
+// instruction) the sum of 8 KV heads x 1.5k / 32k / 128k (low-bit) took 10.4 / 19.3 / 36.0 us with its
+// reduction, now 9.5 / 13.6 / 23.0; eight query heads per KV head, 32k: 24.7, now 20.3 (two workgroups of
+// four heads, eight apart in the launch, so that a die's L2 serves the second; one workgroup for all eight
+// had no registers for a step in flight: 24.9).
+// Weights or values that are not finite take the wavefront's sums again in plain fp32 arithmetic
+// (v_plain_class), for the same infinities and NaNs.
 // ---------------------------------------------------------------------------
 constexpr int kVChunks = 64;
 constexpr int kVWaves = 4;
+constexpr int kVParts = kVChunks * kVWaves;   // wavefronts that share a head's steps
+constexpr int kVNew = 8;                      // appended tokens a wavefront takes at a time
+constexpr int kVCodeUnit = 9;                 // codes enter as code * 2^-9
+constexpr int v_step_tokens(int cls) { return cls == 3 ? 32 : 64; }   // tokens of a step: 128 bytes of codes a lane
 
-// Adds tokens [a, b) (class-local) of class CLS, weighted for query heads g0 .. g0+GB-1, to
-// acc[g][i]: lane li (0..7) of a token always owns channels 16*li .. 16*li+15, whatever the class,
-// so one set of accumulators serves all four classes.  In a 4-bit row (byte j = channels j and
-// j+64) those channels are one nibble of bytes 16*(li&3)..; in a 2-bit row (byte j = channels j,
-// j+32, j+64, j+96) one field of bytes 16*(li&1)..; an fp16 token is two 16-byte loads per lane.
-// wbase: column of class-local token 0 in the weight rows.
-// One quantized token of a lane (its 16 bytes of codes) for GB query heads.
-// sum_t w s (code - z) = sum_t (w s) code - sum_t (w s) z: the token's factor is folded into its
-// weights once, a code costs its conversion (one byte of a dword whose field has been shifted
-// down and masked for all four bytes at once) and one multiply-add per query head; the second
-// sum is the same for all channels of a head and is carried in zacc.
-template <int CLS, int GB>
-__device__ __forceinline__ void v_token_quant(const uint4 r, float s, float z, const float (&wv)[GB], int shift,
-                                              float (&acc)[GB][16], float (&zacc)[GB]) {
-  float ws[GB];
+typedef floatx4 __attribute__((aligned(4))) floatx4_w;
+typedef unsigned long long __attribute__((aligned(2))) u64_a2;   // four fp16 values from any element
+
+// What a lane holds of a step: quantized rows raw[4 a + k] of tokens t0 + 32 a + 4 sub + k, fp16 rows
+// raw[2 k], raw[2 k + 1] of tokens t0 + 4 sub + k; weights of head lane % 4, scales, zero points.
+// Where the four tokens of an a pass the end of the class, w, s and z start up to three columns early (v_tail).
+struct VTile {
+  uint4 raw[8];
+  floatx4 w[2];
+  unsigned long long s[2], z[2];
+};
+
+// A class of the head's tokens: its rows, how many, the column of the first in the weight (and scale) rows.
+struct VClass {
+  const uint8_t *codes;
+  int n;
+  int64_t col;
+};
+
+__device__ __forceinline__ int v_lane_offset(int cls, int li) { return cls == 3 ? 32 * li : 16 * (li & ((2 << cls) - 1)); }
+
+// The loads of a step of any class, without a branch on the class or on the end of its tokens (a load in
+// a branch of its own is waited for there): rows past the end are the last row again, columns are held
+// back to the last four (the first four of the row, if these are not there; the caller sees to it that they are).
+__device__ __forceinline__ void v_load(int cls, const VClass c, const uint16_t *sc, const uint16_t *zz, int t0,
+                                       const float *wrow, int sub, int li, VTile &L) {
+  const int row_log = 5 + cls;
+  const bool wide = cls == 3;
+  const uint8_t *base = c.codes + v_lane_offset(cls, li);
+  const int t = t0 + 4 * sub;
 #pragma unroll
-  for (int g = 0; g < GB; ++g) {
-    ws[g] = wv[g] * s;
-    zacc[g] += ws[g] * z;
+  for (int j = 0; j < 8; ++j) {
+    const int tj = t + (wide ? j >> 1 : 32 * (j >> 2) + (j & 3));
+    const uint64_t at = (uint64_t)(uint32_t)min(tj, c.n - 1) << row_log;
+    L.raw[j] = *reinterpret_cast<const uint4 *>(base + at + (wide ? 16 * (j & 1) : 0));
   }
-  const uint32_t dw[4] = {r.x, r.y, r.z, r.w};
+  const int64_t end = c.col + c.n - 4;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const uint32_t f = CLS == 0 ? ((dw[q] >> shift) & 0x03030303u)
-                                : (CLS == 1 ? ((dw[q] >> shift) & 0x0F0F0F0Fu) : dw[q]);
-    const float c0 = (float)(f & 255u), c1 = (float)((f >> 8) & 255u), c2 = (float)((f >> 16) & 255u),
-                c3 = (float)(f >> 24);
+  for (int a = 0; a < 2; ++a) {
+    int64_t col = c.col + t + 32 * a;
+    col = col < end ? col : end;
+    col = col > 0 ? col : 0;
+    L.w[a] = *reinterpret_cast<const floatx4_w *>(wrow + col);
+    // (fp16 rows have no scales: eight bytes of the rows themselves, not looked at)
+    L.s[a] = *reinterpret_cast<const u64_a2 *>(wide ? reinterpret_cast<const uint16_t *>(c.codes) : sc + col);
+    L.z[a] = *reinterpret_cast<const u64_a2 *>(wide ? reinterpret_cast<const uint16_t *>(c.codes) : zz + col);
+  }
+}
+
+// The last step of a class: what was read early moves to its place, weights past the end become 0.
+template <bool WIDE>
+__device__ __forceinline__ void v_tail(const VClass c, int t0, int sub, VTile &L) {
 #pragma unroll
-    for (int g = 0; g < GB; ++g) {
-      acc[g][4 * q + 0] += ws[g] * c0;
-      acc[g][4 * q + 1] += ws[g] * c1;
-      acc[g][4 * q + 2] += ws[g] * c2;
-      acc[g][4 * q + 3] += ws[g] * c3;
+  for (int a = 0; a < (WIDE ? 1 : 2); ++a) {
+    const int t = t0 + 4 * sub + 32 * a;
+    int64_t col = c.col + (t < c.n - 4 ? t : c.n - 4);
+    col = col > 0 ? col : 0;
+    const int64_t early = c.col + t - col;
+    const int d = early < 4 ? (int)early : 4;
+    if (!WIDE) {
+      L.s[a] = d < 4 ? L.s[a] >> (16 * d) : 0;
+      L.z[a] = d < 4 ? L.z[a] >> (16 * d) : 0;
+    }
+    floatx4 w = L.w[a];
+#pragma unroll
+    for (int r = 1; r <= 3; ++r)
+      if (d >= r) w = floatx4{w[1], w[2], w[3], w[3]};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) L.w[a][k] = t + k < c.n ? w[k] : 0.0f;
+  }
+}
+
+// Sums of a wavefront: acc[c][i] is channel 16 li + c of head i over the lane's tokens, in units
+// of 2^unit of that head (every lane keeps the state of head lane % 4).
+struct VSums {
+  floatx4 acc[16];
+  float zacc;      // sum of weight * scale * zero point of the lane's own head
+  float up, lim;   // the power of two on the weights; the largest weight it is good for
+  int unit;
+};
+
+template <int I>
+__device__ __forceinline__ float v_quad_lane(float v) { return rdkv_dpp_mov<0x55 * I>(v); }
+__device__ __forceinline__ float v_quad_value(float v, int i) {   // (i is a constant after unrolling)
+  return i == 0 ? v_quad_lane<0>(v) : i == 1 ? v_quad_lane<1>(v) : i == 2 ? v_quad_lane<2>(v) : v_quad_lane<3>(v);
+}
+
+// New scaling for the heads whose weights have outgrown theirs; base: the unit of the values (a power of
+// two).  Never so fine that a sum in hand would leave its range (40 bits below its unit is nothing to it); at
+// 2^126 an fp16 remainder still reaches below the smallest fp32 number.
+__device__ __forceinline__ void v_rescale(VSums &S, float mx, int base) {
+  mx = fmaxf(mx, rdkv_dpp_mov<0x124>(mx));
+  mx = fmaxf(mx, rdkv_dpp_mov<0x128>(mx));
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));          // the head's largest
+  float f = 1.0f;
+  if (mx > S.lim) {
+    const int x = (int)(__float_as_uint(mx) >> 23) - 126;            // mx = m * 2^x, 0.5 <= m < 1
+    const int e = min(min(max(12 - x, -100), 126), base - S.unit + 40);
+    f = ldexpf(1.0f, S.unit - (base - e));
+    S.unit = base - e;
+    S.up = __uint_as_float((uint32_t)(127 + e) << 23);
+    S.lim = ldexpf(1.0f, 15 - e);
+  }
+  float fi[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) fi[i] = v_quad_value(f, i);
+#pragma unroll
+  for (int c = 0; c < 16; ++c)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) S.acc[c][i] *= fi[i];
+}
+
+// The widths share one body (shift and mask at run time): a body each made a small call wait for their
+// instructions (1.5k tokens: 11.9 us of V, not 9.5).
+template <bool WIDE>
+__device__ __forceinline__ void v_step(const VTile &L, int cls, int li, VSums &S) {
+  constexpr int kDwords = WIDE ? 8 : 4, kValues = 16 / kDwords;
+  const float mid = cls == 0 ? 1.5f : cls == 1 ? 7.5f : 127.5f;       // half of the largest code
+  const _Float16 mid16 = (_Float16)(mid * (1.0f / 512.0f));
+  const int shift = cls == 0 ? 2 * (li >> 1) : cls == 1 ? 4 * (li >> 2) : 0;    // field inside each byte
+  const uint32_t mask = cls == 0 ? 0x03030303u : cls == 1 ? 0x0F0F0F0Fu : 0xFFFFFFFFu;
+  float mx = 0.0f;
+#pragma unroll
+  for (int a = 0; a < (WIDE ? 1 : 2); ++a)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      mx = fmaxf(mx, fabsf(L.w[a][k] * (WIDE ? 1.0f : rdkv_h2f((uint16_t)(L.s[a] >> (16 * k))))));
+  if (__builtin_amdgcn_ballot_w64(mx > S.lim) != 0) v_rescale(S, mx, WIDE ? 0 : kVCodeUnit);
+#pragma unroll
+  for (int a = 0; a < (WIDE ? 1 : 2); ++a) {
+    half4_t hi, lo;
+    floatx4 ws = L.w[a];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (!WIDE) {
+        ws[k] *= rdkv_h2f((uint16_t)(L.s[a] >> (16 * k)));
+        S.zacc += ws[k] * (rdkv_h2f((uint16_t)(L.z[a] >> (16 * k))) - mid);
+      }
+      const float x = ws[k] * S.up;
+      hi[k] = (_Float16)x;
+      lo[k] = (_Float16)(x - (float)hi[k]);
+    }
+#pragma unroll
+    for (int q = 0; q < kDwords; ++q) {
+      uint32_t f[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint4 r = WIDE ? L.raw[2 * k + (q >> 2)] : L.raw[4 * a + k];
+        const uint32_t d = (q & 3) == 0 ? r.x : (q & 3) == 1 ? r.y : (q & 3) == 2 ? r.z : r.w;
+        f[k] = WIDE ? d : (d >> shift) & mask;
+      }
+      half4_t b[kValues];
+#pragma unroll
+      for (int j = 0; j < kValues; ++j) {
+        // value j of tokens 0 | 1 and of tokens 2 | 3
+        const uint32_t sel = WIDE ? (j ? 0x07060302u : 0x05040100u) : 0x0c040c00u + 0x00010001u * (uint32_t)j;
+        b[j] = mk_op(__builtin_amdgcn_perm(f[1], f[0], sel), __builtin_amdgcn_perm(f[3], f[2], sel));
+        if (!WIDE) b[j] = b[j] * (_Float16)32768.0f - mid16;
+      }
+#pragma unroll
+      for (int j = 0; j < kValues; ++j)
+        S.acc[kValues * q + j] = __builtin_amdgcn_mfma_f32_4x4x4f16(hi, b[j], S.acc[kValues * q + j], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < kValues; ++j)
+        S.acc[kValues * q + j] = __builtin_amdgcn_mfma_f32_4x4x4f16(lo, b[j], S.acc[kValues * q + j], 0, 0, 0);
     }
   }
 }
 
-// Tokens [a, b) one at a time per lane group (any alignment of the weight and scale rows): the
-// eight lane groups of the block's wavefronts take tokens 32 apart, four of them in flight.
-template <int CLS, int GB>
-__device__ __forceinline__ void v_class_range(const uint8_t *__restrict__ codes, int64_t a, int64_t b,
-                                              const __half *__restrict__ sc, const __half *__restrict__ zz,
-                                              int64_t meta0, const float *const *wr, int64_t wbase, int ng,
-                                              float (&acc)[GB][16], float (&zacc)[GB], int lane, int wave) {
-  if (a >= b) return;
-  constexpr int ROW = CLS == 0 ? 32 : (CLS == 1 ? 64 : (CLS == 2 ? 128 : 256));   // bytes per token
-  constexpr int NL = CLS == 3 ? 2 : 1;                                            // 16-byte loads per lane
-  const int sub = lane >> 3, li = lane & 7;
-  const int off = CLS == 0 ? 16 * (li & 1) : (CLS == 1 ? 16 * (li & 3) : (CLS == 2 ? 16 * li : 32 * li));
-  const int shift = CLS == 0 ? 2 * (li >> 1) : (CLS == 1 ? 4 * (li >> 2) : 0);    // field inside each byte
-  constexpr int kUnroll = (CLS == 3 || GB > 4) ? 2 : 4;   // tokens in flight per lane group
-  constexpr int kStep = kVWaves * 8;               // tokens per block step
-  for (int64_t t0 = a + wave * 8 + sub; t0 < b; t0 += (int64_t)kUnroll * kStep) {
-    uint4 raw[kUnroll][NL];
-    float s[kUnroll], z[kUnroll], wv[kUnroll][GB];
-    bool in[kUnroll];
+// The steps part, part + kVParts, ... of a class and one query head (its weight row w) in plain fp32
+// arithmetic: a token a lane group.
+__device__ __forceinline__ void v_plain_class(int cls, const VClass c, const uint16_t *sc, const uint16_t *zz, const float *w,
+                                              int before, int part, int sub, int li, float (&acc)[16], float &zacc) {
+  const int shift = cls == 0 ? 2 * (li >> 1) : cls == 1 ? 4 * (li >> 2) : 0, ntok = v_step_tokens(cls);
+  const uint32_t mask = cls == 0 ? 3u : cls == 1 ? 15u : 255u;
+#pragma unroll 1
+  for (int s = (part - before % kVParts + kVParts) % kVParts; (int64_t)s * ntok < c.n; s += kVParts)
+#pragma unroll 1
+    for (int t = s * ntok + sub; t < min(s * ntok + ntok, c.n); t += 8) {
+      const uint8_t *p = c.codes + v_lane_offset(cls, li) + ((int64_t)t << (5 + cls));
+      float ws = w[c.col + t];
+      if (cls != 3) {
+        ws *= rdkv_h2f(sc[c.col + t]);
+        zacc += ws * rdkv_h2f(zz[c.col + t]);
+      }
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      const int64_t t = t0 + (int64_t)u * kStep;
-      in[u] = t < b;
-      s[u] = z[u] = 0.0f;
-#pragma unroll
-      for (int g = 0; g < GB; ++g) wv[u][g] = 0.0f;
-      if (in[u]) {
-        const uint4 *p = reinterpret_cast<const uint4 *>(codes + t * ROW + off);
-#pragma unroll
-        for (int k = 0; k < NL; ++k) raw[u][k] = p[k];
-        if (CLS != 3) {
-          s[u] = __half2float(sc[meta0 + t]);
-          z[u] = __half2float(zz[meta0 + t]);
-        }
-#pragma unroll
-        for (int g = 0; g < GB; ++g)
-          if (g < ng) wv[u][g] = wr[g][wbase + t];
+      for (int i = 0; i < 16; ++i) {
+        const float v = cls == 3 ? rdkv_h2f(reinterpret_cast<const uint16_t *>(p)[i]) : (float)((p[i] >> shift) & mask);
+        acc[i] += ws * v;
       }
     }
-#pragma unroll
-    for (int u = 0; u < kUnroll; ++u) {
-      if (!in[u]) continue;
-      if (CLS == 3) {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const uint4 r = raw[u][i >> 3];
-          const uint32_t wd = ((i >> 1) & 3) == 0 ? r.x : (((i >> 1) & 3) == 1 ? r.y : (((i >> 1) & 3) == 2 ? r.z : r.w));
-          const float v = __half2float(__ushort_as_half((uint16_t)(wd >> (16 * (i & 1)))));
-#pragma unroll
-          for (int g = 0; g < GB; ++g) acc[g][i] += wv[u][g] * v;
-        }
-      } else {
-        v_token_quant<CLS, GB>(raw[u][0], s[u], z[u], wv[u], shift, acc, zacc);
-      }
-    }
-  }
-}
-
-// Adds tokens [a, b) (class-local) of class CLS, weighted for query heads g0 .. g0+GB-1, to
-// acc[g][i]: lane li (0..7) of a token always owns channels 16*li .. 16*li+15, whatever the class,
-// so one set of accumulators serves all four classes.  In a 4-bit row (byte j = channels j and
-// j+64) those channels are one nibble of bytes 16*(li&3)..; in a 2-bit row (byte j = channels j,
-// j+32, j+64, j+96) one field of bytes 16*(li&1)..; an fp16 token is two 16-byte loads per lane.
-// wbase: column of class-local token 0 in the weight rows.
-// A quantized class whose weight rows allow 16-byte loads (w16: row bases and strides 16-byte
-// aligned) is walked four consecutive tokens per lane group from the first token whose weight
-// column is a multiple of four: one 16-byte load per query head brings the four weights, one
-// 8-byte load the four scales and one the zero points (when those addresses are 8-byte aligned),
-// instead of 4 (GB + 2) scalar loads - the per-token scalars were most of the kernel's load
-// instructions.  What precedes and follows the aligned run goes token by token.  (GROUPED is the
-// launch's choice: it pays on long rows, 55 -> 43 us on a 128k layer with four query heads per KV
-// head, costs a microsecond at 32k, and with eight query heads the registers of the wider loads halve
-// the resident wavefronts.)
-template <int CLS, int GB, bool GROUPED>
-__device__ __forceinline__ void v_class_sum(const uint8_t *__restrict__ codes, int64_t a, int64_t b,
-                                            const __half *__restrict__ sc, const __half *__restrict__ zz,
-                                            int64_t meta0, const float *const *wr, int64_t wbase, int ng,
-                                            float (&acc)[GB][16], float (&zacc)[GB], int lane, int wave, bool w16) {
-  if (a >= b) return;
-  if (CLS == 3 || !GROUPED) {
-    v_class_range<CLS, GB>(codes, a, b, sc, zz, meta0, wr, wbase, ng, acc, zacc, lane, wave);
-    return;
-  }
-  constexpr int ROW = CLS == 0 ? 32 : (CLS == 1 ? 64 : 128);
-  const int sub = lane >> 3, li = lane & 7;
-  const int off = CLS == 0 ? 16 * (li & 1) : (CLS == 1 ? 16 * (li & 3) : 16 * li);
-  const int shift = CLS == 0 ? 2 * (li >> 1) : (CLS == 1 ? 4 * (li >> 2) : 0);
-  // groups of TOK tokens whose weight column is a multiple of TOK (four, or two with eight query
-  // heads: the wider loads must not cost a resident wavefront); the first and the last group may
-  // stick out of [a, b): their tokens outside get weight 0 and are loaded one by one
-  constexpr int TOK = GB > 4 ? 2 : 4;
-  const int64_t t_first = a - ((wbase + a) & (TOK - 1));
-  const int64_t groups = (b - t_first + TOK - 1) / TOK;
-  const bool meta_vec = (((uintptr_t)(sc + meta0 + t_first)) & (2 * TOK - 1)) == 0 &&
-                        (((uintptr_t)(zz + meta0 + t_first)) & (2 * TOK - 1)) == 0;
-  for (int64_t gi = wave * 8 + sub; gi < groups; gi += kVWaves * 8) {
-    const int64_t t = t_first + TOK * gi;
-    const bool full = w16 && t >= a && t + TOK - 1 < b;   // (rows that do not allow vector loads: every group one by one)
-    uint4 raw[TOK];
-    float s4[TOK], z4[TOK], wv[TOK][GB];
-    if (full) {
-#pragma unroll
-      for (int u = 0; u < TOK; ++u) raw[u] = *reinterpret_cast<const uint4 *>(codes + (t + u) * ROW + off);
-#pragma unroll
-      for (int g = 0; g < GB; ++g) {
-        if (TOK == 4) {
-          const float4 w4 = g < ng ? *reinterpret_cast<const float4 *>(wr[g] + wbase + t) : make_float4(0.f, 0.f, 0.f, 0.f);
-          wv[0][g] = w4.x; wv[1][g] = w4.y; wv[TOK - 2][g] = w4.z; wv[TOK - 1][g] = w4.w;
-        } else {
-          const float2 w2 = g < ng ? *reinterpret_cast<const float2 *>(wr[g] + wbase + t) : make_float2(0.f, 0.f);
-          wv[0][g] = w2.x; wv[1][g] = w2.y;
-        }
-      }
-      if (meta_vec) {
-        uint32_t sr[2], zr[2];
-        if (TOK == 4) {
-          const uint2 a2 = *reinterpret_cast<const uint2 *>(sc + meta0 + t), b2 = *reinterpret_cast<const uint2 *>(zz + meta0 + t);
-          sr[0] = a2.x; sr[1] = a2.y; zr[0] = b2.x; zr[1] = b2.y;
-        } else {
-          sr[0] = *reinterpret_cast<const uint32_t *>(sc + meta0 + t);
-          zr[0] = *reinterpret_cast<const uint32_t *>(zz + meta0 + t);
-          sr[1] = zr[1] = 0;
-        }
-#pragma unroll
-        for (int u = 0; u < TOK; ++u) {
-          s4[u] = rdkv_h2f((uint16_t)(sr[u >> 1] >> (16 * (u & 1))));
-          z4[u] = rdkv_h2f((uint16_t)(zr[u >> 1] >> (16 * (u & 1))));
-        }
-      } else {
-#pragma unroll
-        for (int u = 0; u < TOK; ++u) {
-          s4[u] = __half2float(sc[meta0 + t + u]);
-          z4[u] = __half2float(zz[meta0 + t + u]);
-        }
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < TOK; ++u) {
-        const int64_t tu = t + u;
-        const bool in = tu >= a && tu < b;
-        const int64_t tc = in ? tu : a;                  // a token that exists, weighted 0
-        raw[u] = *reinterpret_cast<const uint4 *>(codes + tc * ROW + off);
-        s4[u] = __half2float(sc[meta0 + tc]);
-        z4[u] = __half2float(zz[meta0 + tc]);
-#pragma unroll
-        for (int g = 0; g < GB; ++g) wv[u][g] = (in && g < ng) ? wr[g][wbase + tc] : 0.0f;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < TOK; ++u) v_token_quant<CLS, GB>(raw[u], s4[u], z4[u], wv[u], shift, acc, zacc);
-  }
 }
 
 // The fp32 value rows of the new zone (v == nullptr: none) and their weights.
@@ -1085,50 +1108,28 @@ struct NewValues {
   int64_t n;
 };
 
-// Tokens [a, b) of the new zone of one KV head, added like a class of the packed ones (lane li of a
-// token owns channels 16 li .. + 15).
-template <int GB>
-__device__ __forceinline__ void v_new_zone_sum(const NewValues &nv, int hkv, int hq0, int64_t a, int64_t b, int ng,
-                                               float (&acc)[GB][16], int lane, int wave) {
-  const int sub = lane >> 3, li = lane & 7;
-  for (int64_t t = a + wave * 8 + sub; t < b; t += kVWaves * 8) {
-    const floatx4 *p = reinterpret_cast<const floatx4 *>(nv.v + hkv * nv.v_sh + t * nv.v_st + 16 * li);
-    const floatx4 r[4] = {p[0], p[1], p[2], p[3]};
-#pragma unroll
-    for (int g = 0; g < GB; ++g) {
-      const float w = g < ng ? nv.w[(int64_t)(hq0 + g) * nv.w_sh + t] : 0.0f;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[g][i] += w * r[i >> 2][i & 3];
-    }
-  }
+// The two values a lane keeps of two sums over lanes l and l ^ 32 (l ^ 16): lanes of the lower half (of even
+// rows) the first, the others the second, in the vector ALU.
+__device__ __forceinline__ float fold32(float a, float b) {
+  auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+}
+__device__ __forceinline__ float fold16(float a, float b) {
+  auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b), false, false);
+  return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
 }
 
-// v + the values of the lanes that differ from this one in bits 3, 4 and 5 of the lane index (the
-// eight token lanes that own the same channels): a rotation by 8 inside each row of 16 lanes, then
-// an exchange of neighbouring rows and of the two halves of the wavefront, all in the vector ALU
-// (three shuffles through the LDS crossbar, for each of 64 accumulators, were a third of the kernel).
-__device__ __forceinline__ float fold_token_lanes(float v) {
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, true));
-  unsigned u = __builtin_bit_cast(unsigned, v);
-  auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-  v = __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
-  u = __builtin_bit_cast(unsigned, v);
-  auto t = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  return __builtin_bit_cast(float, (unsigned)t[0]) + __builtin_bit_cast(float, (unsigned)t[1]);
-}
-
-template <int GB, bool GROUPED>
-__global__ void __launch_bounds__(64 * kVWaves)
+__global__ void __launch_bounds__(64 * kVWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
                       const uint8_t *__restrict__ V2, int64_t v2_sh, const uint8_t *__restrict__ V4,
                       int64_t v4_sh, const uint8_t *__restrict__ V8, int64_t v8_sh,
-                      const __half *__restrict__ scale, const __half *__restrict__ zp, int64_t vs_sh,
+                      const uint16_t *__restrict__ scale, const uint16_t *__restrict__ zp, int64_t vs_sh,
                       const int32_t *__restrict__ seg_bounds, int N2h, int N4h, int N8h,
-                      const __half *__restrict__ V16, int64_t v16_sh, const int32_t *__restrict__ n_v16,
+                      const uint8_t *__restrict__ V16, int64_t v16_sh, const int32_t *__restrict__ n_v16,
                       int64_t max_T_v, NewValues nv, float *__restrict__ partial, int H_q) {
-  static_assert(GB <= 2 * kGB, "accumulator slots");
   const int hkv = blockIdx.y, chunk = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sub = lane >> 3, li = lane & 7;
   int N2 = N2h, N4 = N4h, N8 = N8h;
   if (seg_bounds) {
     N2 = seg_bounds[hkv * 3 + 0];
@@ -1136,60 +1137,136 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
     N8 = seg_bounds[hkv * 3 + 2];
   }
   const int N16 = (V16 && n_v16) ? n_v16[hkv] : 0;
-  const __half *sc = scale + hkv * vs_sh;
-  const __half *zz = zp + hkv * vs_sh;
-  __shared__ float s_acc[kVWaves][kGB * 2][kD];
-  // every class is cut into kVChunks equal pieces and a workgroup takes one piece of each, so all
-  // workgroups of a head read the same number of bytes and dequantize the same number of tokens
-  const int64_t c1 = N2, c2 = c1 + N4;
-  auto lo = [&](int64_t n) { const int64_t per = (n + kVChunks - 1) / kVChunks, a = chunk * per; return a < n ? a : n; };
-  auto hi = [&](int64_t n) { const int64_t per = (n + kVChunks - 1) / kVChunks, b = (chunk + 1) * per; return b < n ? b : n; };
-
-  const int sub = lane >> 3, li = lane & 7;
-  const bool w16 = (((uintptr_t)w) & 15) == 0 && (w_sh & 3) == 0;   // weight rows allow 16-byte loads
-  for (int g0 = 0; g0 < G; g0 += GB) {
-    const int ng = G - g0 < GB ? G - g0 : GB;
-    const float *wr[GB];
+  const uint16_t *sc = scale + hkv * vs_sh, *zz = zp + hkv * vs_sh;
+  const VClass c0{V2 + hkv * v2_sh, V2 ? max(N2, 0) : 0, 0}, c1{V4 + hkv * v4_sh, V4 ? max(N4, 0) : 0, N2},
+      c2{V8 + hkv * v8_sh, V8 ? max(N8, 0) : 0, (int64_t)N2 + N4}, c3{V16 + 2 * hkv * v16_sh, max(N16, 0), max_T_v};
+  // steps of a class and those before it
+  const int e0 = (c0.n + 63) / 64, e1 = e0 + (c1.n + 63) / 64, e2 = e1 + (c2.n + 63) / 64, e3 = e2 + (c3.n + 31) / 32;
+  const int part = chunk * kVWaves + wave, g0 = 4 * blockIdx.z, ng = min(G - g0, 4);
+  const bool live = (lane & 3) < ng;
+  const float *w0 = w + (int64_t)(hkv * G + g0) * w_sh, *wrow = w0 + (live ? lane & 3 : 0) * w_sh;
+  __shared__ float s_acc[kVWaves][4][kD];
+  VSums S;
+  S.zacc = S.lim = 0.0f;
+  S.up = 1.0f;
+  S.unit = -1000;      // (nothing summed: any unit will do)
 #pragma unroll
-    for (int g = 0; g < GB; ++g) wr[g] = w + (int64_t)(hkv * G + (g < ng ? g0 + g : g0)) * w_sh;
-    float acc[GB][16], zacc[GB];   // zacc: this lane's sum of weight * scale * zero point per head
-#pragma unroll
-    for (int g = 0; g < GB; ++g) {
-      zacc[g] = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[g][i] = 0.0f;
+  for (int c = 0; c < 16; ++c) S.acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+  // (weight or scale rows of fewer than four columns: the plain sums below)
+  const bool narrow = (e2 > 0 && (int64_t)N2 + N4 + N8 < 4) || (N16 > 0 && max_T_v + N16 < 4);
+  const int todo = narrow ? 0 : e3;
+  // (assignments: a conditional of two variables is an address the compiler keeps in scratch memory)
+  auto class_of = [&](int s, VClass &c, int &before) __attribute__((always_inline)) {
+    int cls = 3;
+    c = c3;
+    before = e2;
+    if (s < e2) { c = c2; cls = 2; before = e1; }
+    if (s < e1) { c = c1; cls = 1; before = e0; }
+    if (s < e0) { c = c0; cls = 0; before = 0; }
+    return cls;
+  };
+  auto load = [&](int s, VTile &L) __attribute__((always_inline)) {
+    VClass c;
+    int before;
+    const int cls = class_of(s, c, before);
+    v_load(cls, c, sc, zz, v_step_tokens(cls) * (s - before), wrow, sub, li, L);
+  };
+  VTile cur, nxt;
+  int s = part;
+  if (s < todo) load(s, cur);
+  auto run = [&](auto wide_c, int end) __attribute__((always_inline)) {
+    constexpr bool WIDE = decltype(wide_c)::value;
+    while (s < min(todo, end)) {
+      load(s + kVParts < todo ? s + kVParts : s, nxt);      // (nothing left: the same step again, from the cache)
+      int before;
+      VClass c;
+      const int cls = class_of(s, c, before), t0 = v_step_tokens(cls) * (s - before);
+      if (t0 + v_step_tokens(cls) > c.n) v_tail<WIDE>(c, t0, sub, cur);
+      if (!live) cur.w[0] = cur.w[1] = floatx4{0.f, 0.f, 0.f, 0.f};
+      v_step<WIDE>(cur, cls, li, S);
+      cur = nxt;
+      s += kVParts;
     }
-    if (V2) v_class_sum<0, GB, GROUPED>(V2 + hkv * v2_sh, lo(N2), hi(N2), sc, zz, 0, wr, 0, ng, acc, zacc, lane, wave, w16);
-    if (V4) v_class_sum<1, GB, GROUPED>(V4 + hkv * v4_sh, lo(N4), hi(N4), sc, zz, c1, wr, c1, ng, acc, zacc, lane, wave, w16);
-    if (V8) v_class_sum<2, GB, GROUPED>(V8 + hkv * v8_sh, lo(N8), hi(N8), sc, zz, c2, wr, c2, ng, acc, zacc, lane, wave, w16);
-    if (N16 > 0)
-      v_class_sum<3, GB, GROUPED>(reinterpret_cast<const uint8_t *>(V16 + hkv * v16_sh), lo(N16), hi(N16), sc, zz, 0, wr,
-                         max_T_v, ng, acc, zacc, lane, wave, w16);
-    if (nv.v) v_new_zone_sum<GB>(nv, hkv, hkv * G + g0, lo(nv.n), hi(nv.n), ng, acc, lane, wave);
-    // fold the eight token lanes of the wavefront (same li), then the wavefronts, in a fixed order
-    // (a head's sixteen folds first, then one guarded run of 16-byte stores: with the store inside
-    // the loop every fold was a chain of dependent cross-lane moves behind its own exec-mask
-    // change, 2.5 us of a 13 us workgroup)
+  };
+  run(std::false_type{}, e2);
+  S.lim = 0.0f;      // (other values, other unit: the sums are rescaled when the first weights come in)
+  run(std::true_type{}, e3);
+  float odd = narrow ? __builtin_nanf("") : 0.0f;
 #pragma unroll
-    for (int g = 0; g < GB; ++g) {
-      float v[16];
+  for (int c = 0; c < 16; ++c)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = fold_token_lanes(acc[g][i] - zacc[g]);
-      if (sub == 0) {
-        float4 *dst = reinterpret_cast<float4 *>(&s_acc[wave][g][16 * li]);
+    for (int i = 0; i < 4; ++i) odd = fmaf(S.acc[c][i], 0.0f, odd);
+  const bool plain = __builtin_amdgcn_ballot_w64(!(odd == 0.0f)) != 0;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) dst[k] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+  for (int i = 0; i < 4; ++i) {
+    const float zi = v_quad_value(S.zacc, i), unit = v_quad_value(ldexpf(1.0f, S.unit), i);      // (2^-1000: 0 of 0)
+#pragma unroll
+    for (int c = 0; c < 16; ++c) S.acc[c][i] = plain ? 0.0f : fmaf(S.acc[c][i], unit, -zi);
+  }
+  // the new zone, fp32: eight tokens at a time, the last wavefronts first (they have the fewest steps)
+  if (nv.v) {
+    const float *vh = nv.v + hkv * nv.v_sh + 16 * li, *wh = nv.w + (int64_t)(hkv * G + g0 + (live ? lane & 3 : 0)) * nv.w_sh;
+    for (int64_t t0 = (int64_t)kVNew * (kVParts - 1 - part); t0 < nv.n; t0 += (int64_t)kVNew * kVParts) {
+      const bool in = t0 + sub < nv.n;
+      const int64_t t = in ? t0 + sub : t0;
+      floatx4 r[4];
+      float wn = wh[t];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r[j] = reinterpret_cast<const floatx4 *>(vh + t * nv.v_st)[j];
+      if (!in) {
+        wn = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r[j] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
+#pragma unroll
+      for (int c = 0; c < 16; ++c) S.acc[c] = __builtin_amdgcn_mfma_f32_4x4x1f32(wn, r[c >> 2][c & 3], S.acc[c], 0, 0, 0);
+    }
+  }
+  // Fold the eight token lanes of the wavefront, halving the channels a lane keeps with every exchange:
+  // in the end lane (b5, b4, b3, li) has channels 16 li + 8 b5 + 4 b4 + 2 b3 and the next.  (Folding all
+  // sixteen on every lane takes 320 instructions instead of 112.)  Then the wavefronts, in a fixed order.
+  const bool b3 = lane & 8;
+  const int ch = 16 * li + 8 * (lane >> 5) + 4 * ((lane >> 4) & 1) + 2 * ((lane >> 3) & 1);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float a[8], b[4], r[2];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) a[c] = fold32(S.acc[c][i], S.acc[c + 8][i]);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) b[c] = fold16(a[c], a[c + 4]);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) r[c] = (b3 ? b[c + 2] : b[c]) + rdkv_dpp_mov<0x128>(b3 ? b[c] : b[c + 2]);
+    *reinterpret_cast<float2 *>(&s_acc[wave][i][ch]) = make_float2(r[0], r[1]);
+  }
+  if (plain) {
+#pragma unroll 1
+    for (int g = 0; g < ng; ++g) {
+      float acc[16], zacc = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+#pragma unroll 1
+      for (int cls = 0; cls < 4; ++cls) {
+        const int first = cls == 0 ? 0 : cls == 1 ? e0 : cls == 2 ? e1 : e2, last = cls == 0 ? e0 : cls == 1 ? e1 : cls == 2 ? e2 : e3;
+        int before;
+        VClass c;
+        class_of(first, c, before);
+        if (first < last) v_plain_class(cls, c, sc, zz, w0 + g * w_sh, first, part, sub, li, acc, zacc);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        float v = acc[i] - zacc;
+        for (int o = 8; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
+        if (sub == 0) s_acc[wave][g][16 * li + i] += v;      // (behind the new zone's sums, same wavefront)
       }
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < ng * kD; i += blockDim.x) {
-      const int g = i / kD, d = i % kD;
-      float v = s_acc[0][g][d];
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < ng * kD; i += blockDim.x) {
+    const int g = i / kD, d = i % kD;
+    float v = s_acc[0][g][d];
 #pragma unroll
-      for (int wv = 1; wv < kVWaves; ++wv) v += s_acc[wv][g][d];
-      partial[((int64_t)chunk * H_q + hkv * G + g0 + g) * kD + d] = v;
-    }
-    __syncthreads();
+    for (int wv = 1; wv < kVWaves; ++wv) v += s_acc[wv][g][d];
+    partial[((int64_t)chunk * H_q + hkv * G + g0 + g) * kD + d] = v;
   }
 }
 
@@ -1414,16 +1491,12 @@ static int v_weighted_sum(const float *w, int64_t w_stride_h, int H_q, int H_kv,
                    v8_stride_h % 16 == 0 && v16_stride_h % 8 == 0,
                "rdkv_v_weighted_sum: V segments must be 16-byte aligned");
   const int G = H_q / H_kv;
-#define RDKV_LAUNCH_V(GB, GROUPED)                                                                             \
-  hipLaunchKernelGGL((v_weighted_sum_kernel<GB, GROUPED>), dim3(kVChunks, H_kv), dim3(64 * kVWaves), 0, s, w, w_stride_h, G, \
-                     V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, (const __half *)scale_f16,             \
-                     (const __half *)zp_f16, vs_stride_h, seg_bounds_dev, N2, N4, N8, (const __half *)V16_f16, \
-                     v16_stride_h, n_v16_dev, max_T_v, nv, (float *)workspace, H_q)
-  const bool long_rows = (int64_t)N2 + N4 + N8 >= 65536;   // four consecutive tokens per lane group pay from here on
-  if (G <= 2) { if (long_rows) RDKV_LAUNCH_V(2, true); else RDKV_LAUNCH_V(2, false); }
-  else if (G <= 4 || G > 8) { if (long_rows) RDKV_LAUNCH_V(4, true); else RDKV_LAUNCH_V(4, false); }
-  else RDKV_LAUNCH_V(8, false);   // (two-token groups with eight heads: 68 against 62 us on a 128k layer)
-#undef RDKV_LAUNCH_V
+  const int64_t quads = rdkv_cdiv(G, 4);
+  RDKV_REQUIRE(H_kv <= 65535 && quads <= 65535, "rdkv_v_weighted_sum: too many heads");
+  hipLaunchKernelGGL(v_weighted_sum_kernel, dim3(kVChunks, H_kv, (unsigned)quads), dim3(64 * kVWaves), 0, s, w, w_stride_h, G,
+                     V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, (const uint16_t *)scale_f16,
+                     (const uint16_t *)zp_f16, vs_stride_h, seg_bounds_dev, N2, N4, N8, (const uint8_t *)V16_f16,
+                     v16_stride_h, n_v16_dev, max_T_v, nv, (float *)workspace, H_q);
   hipLaunchKernelGGL(v_reduce_kernel, dim3(H_q), dim3(8 * kD), 0, s, (const float *)workspace, H_q, out, out_stride_h);
   RDKV_CHECK_LAUNCH("rdkv_v_weighted_sum");
   return RDKV_OK;
