@@ -202,6 +202,22 @@ int rdkv_softmax_rows_new_keys(const float *scores_old, int64_t so_stride_h, con
                                float *w_new, int64_t wn_stride_h, int H_q, int H_kv, void *workspace,
                                int64_t workspace_bytes, void *stream);
 
+/* The scores of rows [packed | appended keys] in one call, T_old > 0: scores[hq, t] = rdkv_k_qk_dot + mask for
+ * t < T_old, then the appended keys' as rdkv_softmax_rows_new_keys forms them.  *n_pairs > 0: the rows hold
+ * scores, and `workspace` (rdkv_attn_scores_workspace_bytes(H_q) bytes) their softmax as that many partial
+ * {maximum, sum of exp} pairs a row, for rdkv_v_weighted_sum_scores.  *n_pairs == 0 (K rows not stored back to
+ * back, no kept channels): the rows hold the weights. */
+int64_t rdkv_attn_scores_workspace_bytes(int H_q);
+int rdkv_attn_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int H_kv,
+                     const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t,
+                     const uint8_t *K4, int64_t k4_stride_h, int64_t k4_stride_t,
+                     const uint8_t *K8, int64_t k8_stride_h, int64_t k8_stride_t,
+                     const void *scale_f16, const void *zp_f16, int64_t ks_stride_h,
+                     const int64_t *perm, int64_t perm_stride_h, int n2p, int n4p, int n8, int64_t T_old,
+                     const float *mask, int64_t mask_stride_h, const float *k_new, int64_t kn_stride_h,
+                     int64_t kn_stride_t, int64_t n_new, float *scores, int64_t stride_h, void *workspace,
+                     int64_t workspace_bytes, int *n_pairs, void *stream);
+
 /* ---- triton_v_kernel.py : v_dequant_weighted_sum_dispatch_into (:1729-1760) */
 /* out[hq,d] = sum over 2/4/8-bit segments of w*(code-zp)*scale + fp16 zone B
  * (kernel math triton_v_kernel.py:638-750).  seg_bounds_dev: int32 [H_kv,3] per-head
@@ -233,6 +249,17 @@ int rdkv_v_weighted_sum_new_values(const float *w, int64_t w_stride_h, int H_q, 
                                    int64_t wn_stride_h, const float *v_new, int64_t vn_stride_h,
                                    int64_t vn_stride_t, int64_t n_new, float *out, int64_t out_stride_h,
                                    void *workspace, int64_t workspace_bytes, void *stream);
+
+/* The same over rows that rdkv_attn_scores wrote (softmax_ws, n_pairs: its workspace and pairs, not
+ * overlapping `workspace`); keep_weights: the rows hold the weights afterwards. */
+int rdkv_v_weighted_sum_scores(float *scores, int64_t stride_h, int H_q, int H_kv, const uint8_t *V2,
+                               int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h, const uint8_t *V8,
+                               int64_t v8_stride_h, const void *scale_f16, const void *zp_f16, int64_t vs_stride_h,
+                               const int32_t *seg_bounds_dev, int N2, int N4, int N8, const void *V16_f16,
+                               int64_t v16_stride_h, const int32_t *n_v16_dev, int64_t max_T_v, int64_t T_old,
+                               const float *v_new, int64_t vn_stride_h, int64_t vn_stride_t, int64_t n_new,
+                               void *softmax_ws, int n_pairs, int keep_weights, float *out, int64_t out_stride_h,
+                               void *workspace, int64_t workspace_bytes, void *stream);
 
 /* ---- fast_decode.py : the per-token operations around the attention ------- */
 /* fast_decode.py:628-633 (_rms_norm) with the residual add in front of it (:1786, :1808):

@@ -66,6 +66,11 @@ SIGNATURES = {
     "rdkv_v_weighted_sum": (I, [P, L, I, I, P, L, P, L, P, L, P, P, L, P, I, I, I, P, L, P, L, P, L, P, L, P]),
     "rdkv_v_weighted_sum_new_values": (I, [P, L, I, I, P, L, P, L, P, L, P, P, L, P, I, I, I, P, L, P, L, P, L, P, L, L, L,
                                            P, L, P, L, P]),
+    "rdkv_attn_scores_workspace_bytes": (L, [I]),
+    "rdkv_attn_scores": (I, [P, I, L, I, I, P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, I, I, L, P, L, P, L, L, L, P, L,
+                             P, L, P, P]),
+    "rdkv_v_weighted_sum_scores": (I, [P, L, I, I, P, L, P, L, P, L, P, P, L, P, I, I, I, P, L, P, L, L, P, L, L, L,
+                                       P, I, I, P, L, P, L, P]),
     "rdkv_stream_plan_layer": (I, [P, L, P, L, I, I, I, I, I, P, P, I, P]),
     "rdkv_stream_partition": (I, [P, I, I, P, ctypes.c_double, ctypes.c_double, P, I, I, P, I, P, P]),
     "rdkv_stream_partition_units": (I, [P, I, I, P, ctypes.c_double, I, P, I, P, P]),

@@ -137,6 +137,19 @@ __device__ __forceinline__ float wave_max_alu(float v) {
   return fmaxf(__builtin_bit_cast(float, (unsigned)t[0]), __builtin_bit_cast(float, (unsigned)t[1]));
 }
 
+// Sum over the 16 lanes of a row, in every lane.
+__device__ __forceinline__ float row16_sum(float v) {
+  v += rdkv_dpp_mov<0x128>(v);
+  v += rdkv_dpp_mov<0x124>(v);
+  v += rdkv_dpp_mov<0x122>(v);
+  return v + rdkv_dpp_mov<0x121>(v);
+}
+
+// Softmax of a row in pieces: a piece's maximum m and its sum l of exp(x - m).  Where all of a piece is -inf,
+// exp(x - 0) keeps the sum at 0 (NaN: NaN); the weights themselves are exp(x - m) / l with the row's own m.
+__device__ __forceinline__ float softmax_at(float m) { return m == -INFINITY ? 0.0f : m; }
+__device__ __forceinline__ void softmax_rebase(float m, float &l, float to) { l *= __expf(m - softmax_at(to)); }
+
 // A barrier for what went through LDS, without waiting for loads in flight.
 __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
@@ -178,6 +191,14 @@ __device__ __forceinline__ int k_slot(int width, int p, int j) {
 // The reference layout pads every head's segments to the widest head's: channels whose stored scale is zero
 // contribute exactly nothing, blocks past a head's last such channel are skipped.
 // CPT = channels per thread (Dp <= 256 CPT).
+// STATS: the launch also forms the scores of the appended keys (its first st.new_groups workgroups of a KV head),
+// adds the mask, and every workgroup leaves its part of a row's softmax, maximum and sum, as a pair, so no
+// launch reads the rows again for them (13.3 us at 32k, 13.4 + 10.1 in two launches at 128k).  With it this
+// launch takes 13.8 us where the scores alone take 13.4, 19.1 for 18.2 at 128k, with eight query heads per KV
+// head 19.8 for 16.9 at 32k and 39 for 30 at 100k; the sum takes 1.2 .. 4 us more.  Error of the weights against 64
+// bits 5.1e-8 .. 6.4e-8 in the 2-norm (a launch of their own: 6.4e-8 .. 1.2e-7).  A layer's call, us: 8 KV heads x
+// 32k 40.0 -> 35.9 (issued one by one; the launches 44 -> 34), 128k low-bit 61.2 -> 47.3, eight heads 32k
+// 50.7 -> 47.2, 100k 96 -> 86.
 // Dynamic LDS: KSetup, then one or two tiles of 16-byte pieces, each with 128 bytes that reads past the
 // last row may touch.
 template <int NG>
@@ -189,21 +210,122 @@ struct KSetup {
   float last[4][4];                                 // by wavefront: last channel of a width that counts
 };
 
+// What a STATS launch takes besides: the additive mask (or null), the appended keys, fp32 rows of 16-byte
+// alignment, `per_group` of them a workgroup, and where the pairs go, [H_q][gridDim.x].
+struct KStats {
+  const float *mask;
+  int64_t mask_sh;
+  const float *k_new;
+  int64_t kn_sh, kn_st, n_new;
+  int new_groups, per_group;
+  float2 *pairs;
+};
+
+constexpr int kKNewKeys = 64;      // appended keys of a pass of a workgroup: two for each eight lanes
+constexpr int kKNewGroups = 128;   // workgroups of a KV head that take appended keys, at most
+constexpr int kKMaxPairs = 1024 + kKNewGroups;
+
 constexpr int kKResident = 4;      // workgroups per compute unit (wavefronts per SIMD) the kernel is compiled for
 
 // 16-byte pieces of a tile of 256 rows of `sub` bytes that may start and end anywhere in a piece.
 constexpr int k_tile_pieces(int sub) { return sub ? (256 * sub + 30) / 16 : 0; }
 
-template <int NG, int CPT>
+// One pair per query head of a workgroup from its wavefronts' (su.big: maxima, su.rest: sums).
+template <int NG>
+__device__ __forceinline__ void k_write_pairs(const KSetup<NG> &su, int tl, int heads, int64_t first, const KStats &st) {
+  lds_barrier();
+  if (tl < heads) {
+    const float m = fmaxf(fmaxf(su.big[0][tl], su.big[1][tl]), fmaxf(su.big[2][tl], su.big[3][tl]));
+    float l = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      float lw = su.rest[w][tl];
+      softmax_rebase(su.big[w][tl], lw, m);
+      l += lw;
+    }
+    st.pairs[(first + tl) * gridDim.x + blockIdx.x] = make_float2(m, l);
+  }
+}
+
+// scores[t] = sum_d (q[d] / sqrt(128)) k[t][d] for the workgroup's appended keys and NHD query heads: eight
+// lanes per key (sixteen channels each, 16-byte loads), two keys per lane group in flight; lane kc of the
+// eight keeps head kc.  The same products and sums as new_zone_scores below.
+template <int NG>
+__device__ __forceinline__ void k_new_keys(KSetup<NG> &su, const float (&qrow)[2 * NG], int G, int g0, int64_t T,
+                                           float *__restrict__ out, int64_t out_sh, const KStats &st) {
+  constexpr int NHD = 4 * NG;
+  const int tl = threadIdx.x, lane = tl & 63, wave = tl >> 6, tg = lane >> 3, kc = lane & 7, hkv = blockIdx.y;
+#pragma unroll
+  for (int u = 0; u < 2 * NG; ++u) (&su.q[0][0])[tl + 256 * u] = qrow[u] * kInvSqrtD;
+  lds_barrier();
+  const float *kh = st.k_new + hkv * st.kn_sh;
+  const int64_t a = (int64_t)blockIdx.x * st.per_group, b = min(a + st.per_group, st.n_new);
+  const bool mine = kc < NHD && g0 + kc < G;
+  float *dst = out + (int64_t)(hkv * G + g0 + kc) * out_sh + T;
+  float m = -INFINITY, l = 0.0f;
+  for (int64_t t0 = a + wave * 8 + tg; t0 < b; t0 += kKNewKeys) {
+    floatx4 kr[2][4];
+    const bool two = t0 + 32 < b;
+    const int64_t t1 = two ? t0 + 32 : t0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) kr[0][j] = reinterpret_cast<const floatx4 *>(kh + t0 * st.kn_st)[8 * j + kc];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) kr[1][j] = reinterpret_cast<const floatx4 *>(kh + t1 * st.kn_st)[8 * j + kc];
+    float own[2] = {0.0f, 0.0f};
+#pragma unroll 1
+    for (int g = 0; g < NHD; ++g) {
+      floatx4 qv[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) qv[j] = *reinterpret_cast<const floatx4 *>(&su.q[g][32 * j + 4 * kc]);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        float p[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          p[j] = fmaf(kr[u][j].w, qv[j].w, fmaf(kr[u][j].z, qv[j].z, fmaf(kr[u][j].y, qv[j].y, kr[u][j].x * qv[j].x)));
+        float v = (p[0] + p[1]) + (p[2] + p[3]);
+        v += rdkv_dpp_mov<0xB1>(v);          // quad_perm [1,0,3,2]
+        v += rdkv_dpp_mov<0x4E>(v);          // quad_perm [2,3,0,1]
+        v += rdkv_dpp_mov<0x141>(v);         // row_half_mirror: the other quad of the eight lanes
+        own[u] = kc == g ? v : own[u];
+      }
+    }
+    if (!two) own[1] = -INFINITY;
+    const float to = fmaxf(m, fmaxf(own[0], own[1]));
+    softmax_rebase(m, l, to);
+    m = to;
+    l += __expf(own[0] - softmax_at(m)) + (two ? __expf(own[1] - softmax_at(m)) : 0.0f);
+    if (mine) {
+      dst[t0] = own[0];
+      if (two) dst[t1] = own[1];
+    }
+  }
+  // the lanes of a head: kc + 8 k
+  float M = fmaxf(m, rdkv_dpp_mov<0x128>(m));
+  M = fmaxf(M, __shfl_xor(M, 16, 64));
+  M = fmaxf(M, __shfl_xor(M, 32, 64));
+  softmax_rebase(m, l, M);
+  l += rdkv_dpp_mov<0x128>(l);
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (lane < NHD) {
+    su.big[wave][lane] = M;
+    su.rest[wave][lane] = l;
+  }
+  k_write_pairs<NG>(su, tl, min(NHD, G - g0), (int64_t)hkv * G + g0, st);
+}
+
+template <int NG, int CPT, bool STATS>
 __global__ void __launch_bounds__(256, kKResident)
 k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h, int G, int g0,
                      const uint8_t *__restrict__ K2, int64_t k2_sh, const uint8_t *__restrict__ K4,
                      int64_t k4_sh, const uint8_t *__restrict__ K8, int64_t k8_sh,
                      const __half *__restrict__ scale, const __half *__restrict__ zp, int64_t ks_sh,
                      const int64_t *__restrict__ perm, int64_t perm_sh, int n2p, int n4p, int n8,
-                     int64_t T, float *__restrict__ out, int64_t out_sh, int tile_lds) {
+                     int64_t T, float *__restrict__ out, int64_t out_sh, int tile_lds, KStats st) {
   extern __shared__ __align__(16) float smem[];
   constexpr int NHD = 4 * NG;
+  constexpr bool kMaskAhead = NG == 1;
   const int Dp = n2p + n4p + n8;
   const int hkv = blockIdx.y;
   const int sub2 = n2p >> 2, sub4 = n4p >> 1;
@@ -245,9 +367,11 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
   };
 
   // ---- set-up: channel tables and query rows (no load waits for another), then the first tile's rows ---------
-  int tile = blockIdx.x;
+  const int walkers = STATS ? gridDim.x - st.new_groups : gridDim.x;    // workgroups that walk the tiles
+  int tile = STATS ? (int)blockIdx.x - st.new_groups : blockIdx.x;
   int ch[CPT][NHD];
   float scv[CPT], zpv[CPT], qrow[2 * NG];
+  floatx4 mask_next[NG];
 #pragma unroll
   for (int u = 0; u < CPT; ++u) {
     const int c = min(tl + 256 * u, Dp - 1);
@@ -272,11 +396,40 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     q_loads([&](int64_t i) { return __half2float(reinterpret_cast<const __half *>(q)[i]); });
   else
     q_loads([&](int64_t i) { return __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(q)[i] << 16); });
+  if (STATS && (int)blockIdx.x < st.new_groups) {
+    k_new_keys<NG>(su, qrow, G, g0, T, out, out_sh, st);
+    return;
+  }
+  const int r = lane & 15, grp = lane >> 4;
+  // the mask values of a lane's four tokens and NG heads
+  auto load_mask = [&](int tile) __attribute__((always_inline)) {
+    const int64_t t = (int64_t)tile * 256 + wave * 64 + 4 * r;
+#pragma unroll
+    for (int hg = 0; hg < NG; ++hg) mask_next[hg] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if (!st.mask) return;
+#pragma unroll
+    for (int hg = 0; hg < NG; ++hg) {
+      const float *row = st.mask + (int64_t)(hkv * G + min(g0 + 4 * hg + grp, G - 1)) * st.mask_sh;
+      if ((int64_t)tile * 256 + 256 <= T) {
+        mask_next[hg] = *reinterpret_cast<const floatx4_a4 *>(row + t);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mask_next[hg][i] = row[min(t + i, T - 1)];
+      }
+    }
+  };
+  float m_run[NG], l_run[NG];
+#pragma unroll
+  for (int hg = 0; hg < NG; ++hg) {
+    m_run[hg] = -INFINITY;
+    l_run[hg] = 0.0f;
+  }
   for (int i = tl; i < (int)(sizeof(su.digit) + sizeof(su.zero)) / 16; i += 256)
     reinterpret_cast<u32x4 *>(smem)[i] = u32x4{0, 0, 0, 0};
 #pragma unroll
   for (int u = 0; u < 2 * NG; ++u) (&su.q[0][0])[tl + 256 * u] = qrow[u];
   // (behind the wait for the small loads: loads return in order, and theirs would wait for the rows)
+  if (STATS && kMaskAhead) load_mask(tile);
   issue_rows(tile, 0);
   lds_barrier();
   float qv[CPT][NHD];
@@ -359,7 +512,6 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
             e8 = __builtin_amdgcn_readfirstlane((int)ext[2]);
   const int blocks[3] = {(min(e2, sub2) + 15) >> 4, (min(e4, sub4) + 31) >> 5, (e8 + 63) >> 6};
   lds_barrier();
-  const int r = lane & 15, grp = lane >> 4;
   intx4 dig[kKBlocks][NG], start[NG];
 #pragma unroll
   for (int hg = 0; hg < NG; ++hg) start[hg] = intx4{0, 0, 0, 0};
@@ -376,6 +528,8 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     }
   }
   float half_up[NG], factor[NG], offset[NG];    // of this lane's head, lane / 16 of the group: 2^-e in two parts
+  constexpr bool kParked = STATS && NG > 1;     // (eight heads and their softmax: no registers for these)
+  floatx4 *parked = reinterpret_cast<floatx4 *>(su.q);   // (the query is done with) by head: the sums' start, then these
 #pragma unroll
   for (int hg = 0; hg < NG; ++hg) {
 #pragma unroll
@@ -387,14 +541,25 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     half_up[hg] = ldexpf(1.0f, -(e >> 1));
     factor[hg] = big <= 3.0e38f ? ldexpf(kInvSqrtD, (e >> 1) - e) : __builtin_nanf("");
     offset[hg] = -((su.rest[0][g] + su.rest[1][g]) + (su.rest[2][g] + su.rest[3][g])) * kInvSqrtD;
+    if (kParked && wave == 0 && r == 0) {
+      reinterpret_cast<intx4 *>(parked)[8 * hg + grp] = start[hg];
+      parked[8 * hg + 4 + grp] = floatx4{half_up[hg], factor[hg], offset[hg], 0.f};
+    }
   }
 
   // ---- tiles: a wavefront's 64 tokens are four products of sixteen, lane r of product j token 4 r + j ------
   for (int buffer = 0;; buffer ^= 1) {
     __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): this wavefront's pieces are in LDS
     __syncthreads();                         // all are; and every wavefront has done with the other buffer
-    const int next = tile + gridDim.x;
+    const int next = tile + walkers;
     const bool more = next < ntiles;
+    floatx4 mask[NG];
+    if (STATS) {      // (ahead of the next rows: loads return in order; a tile ahead where there are registers)
+      if (!kMaskAhead) load_mask(tile);
+#pragma unroll
+      for (int hg = 0; hg < NG; ++hg) mask[hg] = mask_next[hg];
+      if (kMaskAhead && more) load_mask(next);
+    }
     if (more) issue_rows(next, buffer ^ 1);
     const int64_t t0 = (int64_t)tile * 256;
     const int ntok = T - t0 < 256 ? (int)(T - t0) : 256;
@@ -403,7 +568,7 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int hg = 0; hg < NG; ++hg) acc[j][hg] = start[hg];
+      for (int hg = 0; hg < NG; ++hg) acc[j][hg] = kParked ? reinterpret_cast<const intx4 *>(parked)[8 * hg + grp] : start[hg];
     {
       const Run r0 = run_of(tile, 0), r1 = run_of(tile, 1), r2 = run_of(tile, 2);
       const int begin = rows_off + buffer * tile_lds;
@@ -444,7 +609,8 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     for (int hg = 0; hg < NG; ++hg) {
       const int g = g0 + 4 * hg + grp;
       if (g < G && tok < ntok) {
-        floatx4 v;
+        floatx4 v, join{half_up[hg], factor[hg], offset[hg], 0.f};
+        if (kParked) join = parked[8 * hg + 4 + grp];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const intx4 x = acc[j][hg];
@@ -452,7 +618,17 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
           const int top = x[3] * 256 + x[2];
           const float head = (float)top, left = (float)(top - (int)head);
           const float sum = fmaf(head, 65536.0f, fmaf(left, 65536.0f, fmaf((float)x[1], 256.0f, (float)x[0])));
-          v[j] = fmaf(sum * half_up[hg], factor[hg], offset[hg]);
+          v[j] = fmaf(sum * join[0], join[1], join[2]);
+          if (STATS) v[j] += mask[hg][j];
+        }
+        if (STATS) {
+          float to = m_run[hg];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) to = tok + j < ntok ? fmaxf(to, v[j]) : to;
+          softmax_rebase(m_run[hg], l_run[hg], to);
+          m_run[hg] = to;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) l_run[hg] += tok + j < ntok ? __expf(v[j] - softmax_at(to)) : 0.0f;
         }
         float *dst = out + (int64_t)(hkv * G + g) * out_sh + t0 + tok;
         if (tok + 3 < ntok) {
@@ -466,6 +642,19 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     }
     if (!more) break;
     tile = next;
+  }
+  if (STATS) {
+#pragma unroll
+    for (int hg = 0; hg < NG; ++hg) {
+      const float m = rdkv_row16_max(m_run[hg]);
+      softmax_rebase(m_run[hg], l_run[hg], m);
+      const float l = row16_sum(l_run[hg]);
+      if (r == 0) {
+        su.big[wave][4 * hg + grp] = m;
+        su.rest[wave][4 * hg + grp] = l;
+      }
+    }
+    k_write_pairs<NG>(su, tl, min(NHD, G - g0), (int64_t)hkv * G + g0, st);
   }
 }
 
@@ -1022,10 +1211,72 @@ __device__ __forceinline__ void v_step(const VTile &L, int cls, int li, VSums &S
   }
 }
 
+// The weight of a score; weights that are given are {0, 1, false}.
+struct VWeights {
+  float m, inv;
+  bool scores;
+  __device__ __forceinline__ float operator()(float s) const { return scores ? __expf(s - m) * inv : s; }
+};
+
+// What a launch over scores takes: their softmax in pairs, [H_q][n_pairs] (k_qk_dot_mfma_kernel), and where
+// a head's {maximum, 1 / sum} goes for the launch that turns the scores themselves into weights.
+struct VScores {
+  const float2 *pairs;
+  int n_pairs;
+  float2 *rows;
+};
+
+// {maximum, 1 / sum} of query head lane % 4 of the workgroup's four, by the whole workgroup: a head's pairs on
+// 64 lanes, up to four of them requested at once.
+__device__ __forceinline__ VWeights v_row_softmax(const VScores vs, int first, int ng, float2 (&scratch)[kVWaves][4]) {
+  const int tl = threadIdx.x, h = tl & 3, lane = tl & 63;
+  const float2 *p = vs.pairs + (int64_t)(first + min(h, ng - 1)) * vs.n_pairs;
+  float m = -INFINITY, l = 0.0f;
+  for (int i0 = tl >> 2; i0 < vs.n_pairs; i0 += 256) {
+    float2 x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = p[min(i0 + 64 * u, vs.n_pairs - 1)];
+#pragma unroll
+    for (int u = 1; u < 4; ++u)
+      if (i0 + 64 * u >= vs.n_pairs) x[u] = make_float2(-INFINITY, 0.0f);
+    const float to = fmaxf(fmaxf(fmaxf(x[0].x, x[1].x), fmaxf(x[2].x, x[3].x)), m);
+    softmax_rebase(m, l, to);
+    m = to;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      softmax_rebase(x[u].x, x[u].y, to);
+      l += x[u].y;
+    }
+  }
+  float M = fmaxf(m, rdkv_dpp_mov<0x124>(m));      // the lanes of a head: h + 4 k
+  M = fmaxf(M, rdkv_dpp_mov<0x128>(M));
+  M = fmaxf(M, __shfl_xor(M, 16, 64));
+  M = fmaxf(M, __shfl_xor(M, 32, 64));
+  softmax_rebase(m, l, M);
+  l += rdkv_dpp_mov<0x124>(l);
+  l += rdkv_dpp_mov<0x128>(l);
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (lane < 4) scratch[tl >> 6][lane] = make_float2(M, l);
+  lds_barrier();
+  float2 y[kVWaves];
+#pragma unroll
+  for (int w = 0; w < kVWaves; ++w) y[w] = scratch[w][h];
+  m = fmaxf(fmaxf(y[0].x, y[1].x), fmaxf(y[2].x, y[3].x));
+  l = 0.0f;
+#pragma unroll
+  for (int w = 0; w < kVWaves; ++w) {
+    softmax_rebase(y[w].x, y[w].y, m);
+    l += y[w].y;
+  }
+  return VWeights{m, 1.0f / l, true};
+}
+
 // The steps part, part + kVParts, ... of a class and one query head (its weight row w) in plain fp32
 // arithmetic: a token a lane group.
 __device__ __forceinline__ void v_plain_class(int cls, const VClass c, const uint16_t *sc, const uint16_t *zz, const float *w,
-                                              int before, int part, int sub, int li, float (&acc)[16], float &zacc) {
+                                              int before, int part, int sub, int li, float (&acc)[16], float &zacc,
+                                              const VWeights of) {
   const int shift = cls == 0 ? 2 * (li >> 1) : cls == 1 ? 4 * (li >> 2) : 0, ntok = v_step_tokens(cls);
   const uint32_t mask = cls == 0 ? 3u : cls == 1 ? 15u : 255u;
 #pragma unroll 1
@@ -1033,7 +1284,7 @@ __device__ __forceinline__ void v_plain_class(int cls, const VClass c, const uin
 #pragma unroll 1
     for (int t = s * ntok + sub; t < min(s * ntok + ntok, c.n); t += 8) {
       const uint8_t *p = c.codes + v_lane_offset(cls, li) + ((int64_t)t << (5 + cls));
-      float ws = w[c.col + t];
+      float ws = of(w[c.col + t]);
       if (cls != 3) {
         ws *= rdkv_h2f(sc[c.col + t]);
         zacc += ws * rdkv_h2f(zz[c.col + t]);
@@ -1064,6 +1315,7 @@ __device__ __forceinline__ float fold16(float a, float b) {
   return __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
 }
 
+template <bool SCORES>
 __global__ void __launch_bounds__(64 * kVWaves) __attribute__((amdgpu_waves_per_eu(2, 2)))
 v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
                       const uint8_t *__restrict__ V2, int64_t v2_sh, const uint8_t *__restrict__ V4,
@@ -1071,7 +1323,7 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
                       const uint16_t *__restrict__ scale, const uint16_t *__restrict__ zp, int64_t vs_sh,
                       const int32_t *__restrict__ seg_bounds, int N2h, int N4h, int N8h,
                       const uint8_t *__restrict__ V16, int64_t v16_sh, const int32_t *__restrict__ n_v16,
-                      int64_t max_T_v, NewValues nv, float *__restrict__ partial, int H_q) {
+                      int64_t max_T_v, NewValues nv, float *__restrict__ partial, int H_q, VScores vs) {
   const int hkv = blockIdx.y, chunk = blockIdx.x;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = lane >> 3, li = lane & 7;
@@ -1119,6 +1371,12 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
   VTile cur, nxt;
   int s = part;
   if (s < todo) load(s, cur);
+  VWeights weight{0.0f, 1.0f, false};       // of the lane's own head
+  if (SCORES) {
+    __shared__ float2 s_row[kVWaves][4];
+    weight = v_row_softmax(vs, hkv * G + g0, ng, s_row);
+    if (chunk == 0 && (int)threadIdx.x < ng) vs.rows[hkv * G + g0 + threadIdx.x] = make_float2(weight.m, weight.inv);
+  }
   auto run = [&](auto wide_c, int end) __attribute__((always_inline)) {
     constexpr bool WIDE = decltype(wide_c)::value;
     while (s < min(todo, end)) {
@@ -1126,6 +1384,12 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
       int before;
       VClass c;
       const int cls = class_of(s, c, before), t0 = v_step_tokens(cls) * (s - before);
+      if (SCORES) {
+#pragma unroll
+        for (int a = 0; a < (WIDE ? 1 : 2); ++a)
+#pragma unroll
+          for (int k = 0; k < 4; ++k) cur.w[a][k] = weight(cur.w[a][k]);
+      }
       if (t0 + v_step_tokens(cls) > c.n) v_tail<WIDE>(c, t0, sub, cur);
       if (!live) cur.w[0] = cur.w[1] = floatx4{0.f, 0.f, 0.f, 0.f};
       v_step<WIDE>(cur, cls, li, S);
@@ -1155,7 +1419,7 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
       const bool in = t0 + sub < nv.n;
       const int64_t t = in ? t0 + sub : t0;
       floatx4 r[4];
-      float wn = wh[t];
+      float wn = weight(wh[t]);
 #pragma unroll
       for (int j = 0; j < 4; ++j) r[j] = reinterpret_cast<const floatx4 *>(vh + t * nv.v_st)[j];
       if (!in) {
@@ -1195,7 +1459,8 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
         int before;
         VClass c;
         class_of(first, c, before);
-        if (first < last) v_plain_class(cls, c, sc, zz, w0 + g * w_sh, first, part, sub, li, acc, zacc);
+        const VWeights of{__shfl(weight.m, g, 64), __shfl(weight.inv, g, 64), SCORES};
+        if (first < last) v_plain_class(cls, c, sc, zz, w0 + g * w_sh, first, part, sub, li, acc, zacc, of);
       }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
@@ -1215,10 +1480,39 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
   }
 }
 
-// out[hq, d] = sum over chunks in chunk order: eight groups of chunks in parallel, then the groups
+// Rows of scores that become weights in place, n of them each (s == nullptr: none).
+struct ScoreRows {
+  float *s;
+  int64_t sh, n;
+  const float2 *rows;      // {maximum, 1 / sum} by head
+};
+constexpr int kRowPiece = 8192;      // scores a workgroup turns
+
+// out[hq, d] = sum over chunks in chunk order: eight groups of chunks in parallel, then the groups.  The
+// workgroups behind the first H_q turn a piece of a score row each, beside the sums (32 rows of 24k scores: 4.8 us, the sums alone 3.9).
 __global__ void __launch_bounds__(1024)
-v_reduce_kernel(const float *__restrict__ partial, int H_q, float *__restrict__ out, int64_t out_sh) {
+v_reduce_kernel(const float *__restrict__ partial, int H_q, float *__restrict__ out, int64_t out_sh, ScoreRows sr) {
   __shared__ float s_part[8][kD];
+  if ((int)blockIdx.x >= H_q) {
+    const int h = (blockIdx.x - H_q) % H_q;
+    const int64_t a = (int64_t)((blockIdx.x - H_q) / H_q) * kRowPiece, left = sr.n - a;
+    float *x = sr.s + h * sr.sh + a;
+    const float2 row = sr.rows[h];
+    const VWeights weight{row.x, row.y, true};
+    if (left >= kRowPiece) {
+      floatx4_a4 *x4 = reinterpret_cast<floatx4_a4 *>(x) + threadIdx.x;
+      floatx4 v[2] = {x4[0], x4[1024]};
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[i][k] = weight(v[i][k]);
+      x4[0] = v[0];
+      x4[1024] = v[1];
+    } else {
+      for (int t = threadIdx.x; t < (int)left; t += 1024) x[t] = weight(x[t]);
+    }
+    return;
+  }
   const int hq = blockIdx.x, d = threadIdx.x & 127, grp = threadIdx.x >> 7;
   constexpr int per = kVChunks / 8;
   float s = 0.0f;
@@ -1236,12 +1530,14 @@ v_reduce_kernel(const float *__restrict__ partial, int H_q, float *__restrict__ 
 
 }  // namespace
 
-RDKV_API int rdkv_k_qk_dot(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int H_kv,
-                           const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t, const uint8_t *K4,
-                           int64_t k4_stride_h, int64_t k4_stride_t, const uint8_t *K8, int64_t k8_stride_h,
-                           int64_t k8_stride_t, const void *scale_f16, const void *zp_f16,
-                           int64_t ks_stride_h, const int64_t *perm, int64_t perm_stride_h, int n2p, int n4p,
-                           int n8, int64_t T_eff, float *out, int64_t out_stride_h, void *stream) {
+// stats (or null): mask and appended keys of a launch that leaves the rows' softmax in pairs; *n_pairs of them a
+// row, 0 where the scores of the packed keys are all that was formed.
+static int k_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int H_kv, const uint8_t *K2,
+                    int64_t k2_stride_h, int64_t k2_stride_t, const uint8_t *K4, int64_t k4_stride_h, int64_t k4_stride_t,
+                    const uint8_t *K8, int64_t k8_stride_h, int64_t k8_stride_t, const void *scale_f16, const void *zp_f16,
+                    int64_t ks_stride_h, const int64_t *perm, int64_t perm_stride_h, int n2p, int n4p, int n8,
+                    int64_t T_eff, float *out, int64_t out_stride_h, KStats *stats, int *n_pairs, void *stream) {
+  *n_pairs = 0;
   RDKV_REQUIRE(H_q > 0 && H_kv > 0 && H_q % H_kv == 0, "rdkv_k_qk_dot: H_q=%d not a multiple of H_kv=%d", H_q,
                H_kv);
   RDKV_REQUIRE(H_kv <= 65535, "rdkv_k_qk_dot: H_kv=%d exceeds the launch grid", H_kv);
@@ -1275,23 +1571,44 @@ RDKV_API int rdkv_k_qk_dot(const void *q, int q_dtype, int64_t q_stride_h, int H
     // Workgroups per KV head: a tile each where all are resident at once (or LDS has no room for two tiles), else
     // an even share of the tiles, the next one's rows loaded under the current one.
     const int64_t cus = compute_units();
-    auto resident = [&](size_t lds) { return std::max<int64_t>(1, std::min<int64_t>(kKResident, (160 * 1024) / (int64_t)(lds + 512)) * cus / H_kv); };
+    if (stats && stats->n_new > 0) {
+      const int64_t passes = rdkv_cdiv(stats->n_new, kKNewKeys), per = rdkv_cdiv(passes, kKNewGroups);
+      stats->per_group = (int)std::min<int64_t>(per * kKNewKeys, 0x7fffffc0);
+      stats->new_groups = (int)rdkv_cdiv(passes, per);
+    }
+    // (the workgroups of the appended keys come first; what walks the tiles fills the rest of the device)
+    const int64_t beside = stats ? stats->new_groups : 0;
+    auto resident = [&](size_t lds) {
+      const int64_t all = std::max<int64_t>(1, std::min<int64_t>(kKResident, (160 * 1024) / (int64_t)(lds + 512)) * cus / H_kv);
+      return std::max(all - beside, (all + 1) / 2);
+    };
     size_t staged = setup + tile_lds;
     int64_t wph = tblocks;
     if (tblocks > resident(staged) && staged + tile_lds <= 64 * 1024) {
       staged += tile_lds;
       wph = rdkv_cdiv(tblocks, rdkv_cdiv(tblocks, resident(staged)));
     }
-#define RDKV_LAUNCH_K_MFMA(NG_, CPT_)                                                                              \
+    if (wph + beside > kKMaxPairs) stats = nullptr;    // (single tiles of very wide rows: the softmax is a launch of its own)
+    if (stats) {
+      *n_pairs = (int)(wph + beside);
+      wph += beside;
+    }
+#define RDKV_LAUNCH_K_MFMA(NG_, CPT_, STATS_)                                                                      \
   for (int g0 = 0; g0 < G; g0 += 4 * NG_)                                                                          \
-  hipLaunchKernelGGL((k_qk_dot_mfma_kernel<NG_, CPT_>), dim3((unsigned)wph, H_kv), dim3(256), staged, s, q,     \
-                     q_dtype, q_stride_h, G, g0, K2, k2_stride_h, K4, k4_stride_h, K8, k8_stride_h,                \
+  hipLaunchKernelGGL((k_qk_dot_mfma_kernel<NG_, CPT_, STATS_>), dim3((unsigned)wph, H_kv), dim3(256), staged, s,   \
+                     q, q_dtype, q_stride_h, G, g0, K2, k2_stride_h, K4, k4_stride_h, K8, k8_stride_h,             \
                      (const __half *)scale_f16, (const __half *)zp_f16, ks_stride_h, perm, perm_stride_h, n2p,     \
-                     n4p, n8, T_eff, out, out_stride_h, tile_lds)
-    if (ng == 1 && Dp <= 256) RDKV_LAUNCH_K_MFMA(1, 1);
-    else if (ng == 1) RDKV_LAUNCH_K_MFMA(1, 2);
-    else if (Dp <= 256) RDKV_LAUNCH_K_MFMA(2, 1);
-    else RDKV_LAUNCH_K_MFMA(2, 2);
+                     n4p, n8, T_eff, out, out_stride_h, tile_lds, stats ? *stats : KStats{})
+#define RDKV_LAUNCH_K_MFMA_S(NG_, CPT_)                                                                            \
+  do {                                                                                                             \
+    if (stats) RDKV_LAUNCH_K_MFMA(NG_, CPT_, true);                                                                \
+    else RDKV_LAUNCH_K_MFMA(NG_, CPT_, false);                                                                     \
+  } while (0)
+    if (ng == 1 && Dp <= 256) RDKV_LAUNCH_K_MFMA_S(1, 1);
+    else if (ng == 1) RDKV_LAUNCH_K_MFMA_S(1, 2);
+    else if (Dp <= 256) RDKV_LAUNCH_K_MFMA_S(2, 1);
+    else RDKV_LAUNCH_K_MFMA_S(2, 2);
+#undef RDKV_LAUNCH_K_MFMA_S
 #undef RDKV_LAUNCH_K_MFMA
   } else {
     hipLaunchKernelGGL(k_qk_dot_strided_kernel, dim3((unsigned)tblocks, H_kv), dim3(256), shmem, s, q, q_dtype,
@@ -1301,6 +1618,18 @@ RDKV_API int rdkv_k_qk_dot(const void *q, int q_dtype, int64_t q_stride_h, int H
   }
   RDKV_CHECK_LAUNCH("rdkv_k_qk_dot");
   return RDKV_OK;
+}
+
+RDKV_API int rdkv_k_qk_dot(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int H_kv,
+                           const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t, const uint8_t *K4,
+                           int64_t k4_stride_h, int64_t k4_stride_t, const uint8_t *K8, int64_t k8_stride_h,
+                           int64_t k8_stride_t, const void *scale_f16, const void *zp_f16,
+                           int64_t ks_stride_h, const int64_t *perm, int64_t perm_stride_h, int n2p, int n4p,
+                           int n8, int64_t T_eff, float *out, int64_t out_stride_h, void *stream) {
+  int n_pairs;
+  return k_scores(q, q_dtype, q_stride_h, H_q, H_kv, K2, k2_stride_h, k2_stride_t, K4, k4_stride_h, k4_stride_t, K8,
+                  k8_stride_h, k8_stride_t, scale_f16, zp_f16, ks_stride_h, perm, perm_stride_h, n2p, n4p, n8, T_eff, out,
+                  out_stride_h, nullptr, &n_pairs, stream);
 }
 
 RDKV_API int64_t rdkv_softmax_rows_workspace_bytes(int H_q) {
@@ -1391,6 +1720,39 @@ RDKV_API int rdkv_softmax_rows_new_keys(const float *scores_old, int64_t so_stri
                       H_q, workspace, workspace_bytes, stream);
 }
 
+RDKV_API int64_t rdkv_attn_scores_workspace_bytes(int H_q) {
+  return (int64_t)(H_q > 0 ? H_q : 0) * (1 + kKMaxPairs) * (int64_t)sizeof(float2);
+}
+
+RDKV_API int rdkv_attn_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int H_kv, const uint8_t *K2,
+                              int64_t k2_stride_h, int64_t k2_stride_t, const uint8_t *K4, int64_t k4_stride_h,
+                              int64_t k4_stride_t, const uint8_t *K8, int64_t k8_stride_h, int64_t k8_stride_t,
+                              const void *scale_f16, const void *zp_f16, int64_t ks_stride_h, const int64_t *perm,
+                              int64_t perm_stride_h, int n2p, int n4p, int n8, int64_t T_old, const float *mask,
+                              int64_t mask_stride_h, const float *k_new, int64_t kn_stride_h, int64_t kn_stride_t,
+                              int64_t n_new, float *scores, int64_t stride_h, void *workspace, int64_t workspace_bytes,
+                              int *n_pairs, void *stream) {
+  const char *fn = "rdkv_attn_scores";
+  RDKV_REQUIRE(n_pairs && scores && T_old > 0 && n_new >= 0, "%s: bad arguments", fn);
+  RDKV_REQUIRE(n_new == 0 || (q && k_new), "%s: null pointer", fn);
+  RDKV_REQUIRE(n_new <= 1 || kn_stride_t >= kD, "%s: key rows overlap", fn);
+  RDKV_REQUIRE(((uintptr_t)k_new % 16) == 0 && kn_stride_h % 4 == 0 && kn_stride_t % 4 == 0,
+               "%s: key rows must be 16-byte aligned", fn);
+  RDKV_REQUIRE(H_q > 0 && H_q <= 65535, "%s: H_q=%d", fn, H_q);
+  if (!workspace || workspace_bytes < rdkv_attn_scores_workspace_bytes(H_q)) {
+    rdkv_set_error("rdkv_attn_scores: workspace of %lld bytes required", (long long)rdkv_attn_scores_workspace_bytes(H_q));
+    return RDKV_EWORKSPACE;
+  }
+  KStats stats{mask, mask_stride_h, k_new, kn_stride_h, kn_stride_t, n_new, 0, 0, (float2 *)workspace + H_q};
+  const int rc = k_scores(q, q_dtype, q_stride_h, H_q, H_kv, K2, k2_stride_h, k2_stride_t, K4, k4_stride_h, k4_stride_t, K8,
+                          k8_stride_h, k8_stride_t, scale_f16, zp_f16, ks_stride_h, perm, perm_stride_h, n2p, n4p, n8, T_old,
+                          scores, stride_h, &stats, n_pairs, stream);
+  if (rc != RDKV_OK || *n_pairs > 0) return rc;
+  return rdkv_softmax_rows_new_keys(scores, stride_h, mask, mask_stride_h, T_old, q, q_dtype, q_stride_h, k_new, kn_stride_h,
+                                    kn_stride_t, n_new, scores, stride_h, scores + T_old, stride_h, H_q, H_kv, workspace,
+                                    workspace_bytes, stream);
+}
+
 RDKV_API int rdkv_softmax_rows(const float *scores_old, int64_t so_stride_h, const float *mask,
                                int64_t mask_stride_h, int64_t T_old, const float *scores_new,
                                int64_t sn_stride_h, int64_t n_new, float *w_old, int64_t wo_stride_h,
@@ -1407,8 +1769,9 @@ static int v_weighted_sum(const float *w, int64_t w_stride_h, int H_q, int H_kv,
                           const uint8_t *V4, int64_t v4_stride_h, const uint8_t *V8, int64_t v8_stride_h,
                           const void *scale_f16, const void *zp_f16, int64_t vs_stride_h,
                           const int32_t *seg_bounds_dev, int N2, int N4, int N8, const void *V16_f16,
-                          int64_t v16_stride_h, const int32_t *n_v16_dev, int64_t max_T_v, const NewValues &nv, float *out,
-                          int64_t out_stride_h, void *workspace, int64_t workspace_bytes, void *stream) {
+                          int64_t v16_stride_h, const int32_t *n_v16_dev, int64_t max_T_v, const NewValues &nv,
+                          const VScores &vs, const ScoreRows &sr, float *out, int64_t out_stride_h, void *workspace,
+                          int64_t workspace_bytes, void *stream) {
   RDKV_REQUIRE(H_q > 0 && H_kv > 0 && H_q % H_kv == 0, "rdkv_v_weighted_sum: H_q=%d not a multiple of H_kv=%d",
                H_q, H_kv);
   RDKV_REQUIRE(w && out, "rdkv_v_weighted_sum: null pointer");
@@ -1432,11 +1795,18 @@ static int v_weighted_sum(const float *w, int64_t w_stride_h, int H_q, int H_kv,
   const int G = H_q / H_kv;
   const int64_t quads = rdkv_cdiv(G, 4);
   RDKV_REQUIRE(H_kv <= 65535 && quads <= 65535, "rdkv_v_weighted_sum: too many heads");
-  hipLaunchKernelGGL(v_weighted_sum_kernel, dim3(kVChunks, H_kv, (unsigned)quads), dim3(64 * kVWaves), 0, s, w, w_stride_h, G,
-                     V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, (const uint16_t *)scale_f16,
-                     (const uint16_t *)zp_f16, vs_stride_h, seg_bounds_dev, N2, N4, N8, (const uint8_t *)V16_f16,
-                     v16_stride_h, n_v16_dev, max_T_v, nv, (float *)workspace, H_q);
-  hipLaunchKernelGGL(v_reduce_kernel, dim3(H_q), dim3(8 * kD), 0, s, (const float *)workspace, H_q, out, out_stride_h);
+  const int64_t pieces = sr.s ? rdkv_cdiv(sr.n, kRowPiece) : 0;
+  RDKV_REQUIRE((1 + pieces) * H_q <= 0x7fffffffLL, "rdkv_v_weighted_sum: rows too long");
+#define RDKV_LAUNCH_V(SCORES_)                                                                                        \
+  hipLaunchKernelGGL(v_weighted_sum_kernel<SCORES_>, dim3(kVChunks, H_kv, (unsigned)quads), dim3(64 * kVWaves), 0, s, \
+                     w, w_stride_h, G, V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, (const uint16_t *)scale_f16, \
+                     (const uint16_t *)zp_f16, vs_stride_h, seg_bounds_dev, N2, N4, N8, (const uint8_t *)V16_f16,     \
+                     v16_stride_h, n_v16_dev, max_T_v, nv, (float *)workspace, H_q, vs)
+  if (vs.pairs) RDKV_LAUNCH_V(true);
+  else RDKV_LAUNCH_V(false);
+#undef RDKV_LAUNCH_V
+  hipLaunchKernelGGL(v_reduce_kernel, dim3((unsigned)((1 + pieces) * H_q)), dim3(8 * kD), 0, s, (const float *)workspace, H_q,
+                     out, out_stride_h, sr);
   RDKV_CHECK_LAUNCH("rdkv_v_weighted_sum");
   return RDKV_OK;
 }
@@ -1449,8 +1819,8 @@ RDKV_API int rdkv_v_weighted_sum(const float *w, int64_t w_stride_h, int H_q, in
                                  int64_t max_T_v, float *out, int64_t out_stride_h, void *workspace,
                                  int64_t workspace_bytes, void *stream) {
   return v_weighted_sum(w, w_stride_h, H_q, H_kv, V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, scale_f16, zp_f16,
-                        vs_stride_h, seg_bounds_dev, N2, N4, N8, V16_f16, v16_stride_h, n_v16_dev, max_T_v, NewValues{}, out,
-                        out_stride_h, workspace, workspace_bytes, stream);
+                        vs_stride_h, seg_bounds_dev, N2, N4, N8, V16_f16, v16_stride_h, n_v16_dev, max_T_v, NewValues{}, VScores{},
+                        ScoreRows{}, out, out_stride_h, workspace, workspace_bytes, stream);
 }
 
 RDKV_API int rdkv_v_weighted_sum_new_values(
@@ -1466,6 +1836,27 @@ RDKV_API int rdkv_v_weighted_sum_new_values(
                "%s: value rows must be 16-byte aligned", fn);
   return v_weighted_sum(w, w_stride_h, H_q, H_kv, V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, scale_f16, zp_f16,
                         vs_stride_h, seg_bounds_dev, N2, N4, N8, V16_f16, v16_stride_h, n_v16_dev, max_T_v,
-                        NewValues{n_new > 0 ? v_new : nullptr, w_new, vn_stride_h, vn_stride_t, wn_stride_h, n_new}, out,
-                        out_stride_h, workspace, workspace_bytes, stream);
+                        NewValues{n_new > 0 ? v_new : nullptr, w_new, vn_stride_h, vn_stride_t, wn_stride_h, n_new},
+                        VScores{}, ScoreRows{}, out, out_stride_h, workspace, workspace_bytes, stream);
+}
+
+RDKV_API int rdkv_v_weighted_sum_scores(
+    float *scores, int64_t stride_h, int H_q, int H_kv, const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4,
+    int64_t v4_stride_h, const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
+    int64_t vs_stride_h, const int32_t *seg_bounds_dev, int N2, int N4, int N8, const void *V16_f16,
+    int64_t v16_stride_h, const int32_t *n_v16_dev, int64_t max_T_v, int64_t T_old, const float *v_new,
+    int64_t vn_stride_h, int64_t vn_stride_t, int64_t n_new, void *softmax_ws, int n_pairs, int keep_weights, float *out,
+    int64_t out_stride_h, void *workspace, int64_t workspace_bytes, void *stream) {
+  const char *fn = "rdkv_v_weighted_sum_scores";
+  RDKV_REQUIRE(scores && softmax_ws && T_old >= 0 && n_new >= 0 && (n_new == 0 || v_new), "%s: bad arguments", fn);
+  RDKV_REQUIRE(n_pairs >= 0 && n_pairs <= kKMaxPairs, "%s: %d pairs", fn, n_pairs);
+  RDKV_REQUIRE(((uintptr_t)v_new % 16) == 0 && vn_stride_h % 4 == 0 && vn_stride_t % 4 == 0,
+               "%s: value rows must be 16-byte aligned", fn);
+  float2 *rows = (float2 *)softmax_ws;
+  const VScores vs = n_pairs > 0 ? VScores{rows + H_q, n_pairs, rows} : VScores{};
+  const ScoreRows sr = n_pairs > 0 && keep_weights ? ScoreRows{scores, stride_h, T_old + n_new, rows} : ScoreRows{};
+  return v_weighted_sum(scores, stride_h, H_q, H_kv, V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, scale_f16, zp_f16,
+                        vs_stride_h, seg_bounds_dev, N2, N4, N8, V16_f16, v16_stride_h, n_v16_dev, max_T_v,
+                        NewValues{n_new > 0 ? v_new : nullptr, scores + T_old, vn_stride_h, vn_stride_t, stride_h, n_new}, vs,
+                        sr, out, out_stride_h, workspace, workspace_bytes, stream);
 }

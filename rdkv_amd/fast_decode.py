@@ -13,6 +13,7 @@ fused streaming kernel, and with ``use_cuda_graph`` the whole step is one HIP gr
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from dataclasses import dataclass, field
 from typing import List, Optional, Tuple
@@ -20,7 +21,7 @@ from typing import List, Optional, Tuple
 import torch
 import torch.nn.functional as F
 
-from . import _lib
+from . import _lib, k_kernel
 from .k_kernel import INV_SQRT_D, k_mixed_qk_dot_into
 from .packing import PackedKVLayer
 from .stream_cache import StreamCache, build_stream_cache, decode_attn_fused
@@ -217,6 +218,7 @@ def trizone_attention(q_2d: torch.Tensor, sp: PackedKVLayer, V16: Optional[torch
     n_new = K_new.shape[1]
     T_v = int(sp.T_eff)
     T_old = int(sp.T_eff_k) if sp.T_eff_k > 0 else T_v
+    caller_buf = scores_buf is not None
     if scores_buf is None:
         scores_buf = torch.empty(H_q, T_old + n_new, dtype=torch.float32, device=dev)
     if out is None:
@@ -240,21 +242,34 @@ def trizone_attention(q_2d: torch.Tensor, sp: PackedKVLayer, V16: Optional[torch
     K_new, V_new = (_new_zone_rows(t, H_kv, n_new) for t in (K_new, V_new))
     s_old = scores_buf[:, :T_old]
     s_new = scores_buf[:, T_old:T_old + n_new]
-    if T_old > 0:
-        k_mixed_qk_dot_into(q_2d, sp, T_old, s_old)
-    # zone C scores (:1730-1733), then mask + global softmax over [A | B | C], written back in place as
-    # weights (:1743-1755)
+    # zone C scores (:1730-1733), then mask + global softmax over [A | B | C] (:1743-1755), whose weights the
+    # caller's buffer holds afterwards
     mask = sp.softmax_mask if (T_old > 0 and sp.softmax_mask is not None) else None
-    ws = _lib.workspace(dev, lib.rdkv_softmax_rows_workspace_bytes(H_q))
-    row = scores_buf.stride(0)
-    _lib.check(lib.rdkv_softmax_rows_new_keys(
-        _lib.ptr(s_old), row, _lib.ptr(mask), mask.stride(0) if mask is not None else 0,
-        T_old, q_2d.data_ptr(), _lib.DTYPE_CODE[q_2d.dtype], q_2d.stride(0), K_new.data_ptr(), K_new.stride(0),
-        K_new.stride(1), n_new, _lib.ptr(s_old), row, s_new.data_ptr(), row, H_q, H_kv,
-        ws.data_ptr(), ws.numel(), _lib.stream_of(dev)))
+    row, mask_row = scores_buf.stride(0), mask.stride(0) if mask is not None else 0
+    scores = None
+    if T_old > 0 and not k_kernel._DIAG_ENABLED:
+        args, _, keep = k_kernel._scores_args(q_2d, sp, T_old, s_old)
+        taken = -(-lib.rdkv_attn_scores_workspace_bytes(H_q) // 256) * 256
+        ws = _lib.workspace(dev, taken + lib.rdkv_v_weighted_sum_workspace_bytes(H_q))
+        pairs = ctypes.c_int(0)
+        _lib.check(lib.rdkv_attn_scores(
+            *args, _lib.ptr(mask), mask_row, K_new.data_ptr(), K_new.stride(0), K_new.stride(1), n_new,
+            s_old.data_ptr(), row, ws.data_ptr(), taken, ctypes.addressof(pairs), _lib.stream_of(dev)))
+        del keep
+        if pairs.value > 0:
+            scores = (ws, taken, pairs.value, int(caller_buf))
+    else:
+        if T_old > 0:
+            k_mixed_qk_dot_into(q_2d, sp, T_old, s_old)
+        ws = _lib.workspace(dev, lib.rdkv_softmax_rows_workspace_bytes(H_q))
+        _lib.check(lib.rdkv_softmax_rows_new_keys(
+            _lib.ptr(s_old), row, _lib.ptr(mask), mask_row,
+            T_old, q_2d.data_ptr(), _lib.DTYPE_CODE[q_2d.dtype], q_2d.stride(0), K_new.data_ptr(), K_new.stride(0),
+            K_new.stride(1), n_new, _lib.ptr(s_old), row, s_new.data_ptr(), row, H_q, H_kv,
+            ws.data_ptr(), ws.numel(), _lib.stream_of(dev)))
     # values of all three zones (:1777-1784)
     _weighted_sum_with_new_zone(s_old if T_old > 0 else s_new, sp if T_old > 0 else None, out, V16, n_v16_per_head,
-                                T_v, s_new, V_new)
+                                T_v, s_new, V_new, scores)
     return out
 
 

@@ -80,6 +80,21 @@ def k_mixed_qk_dot_into(Q: torch.Tensor, packed_layer, T_eff: int, out: torch.Te
     per-head Q permutation is applied inside the kernel instead of a separate gather."""
     if not _lib.available():
         raise RuntimeError("rdkv HIP backend is not available.")
+    args, dev, keep = _scores_args(Q, packed_layer, T_eff, out)
+    t0 = 0.0
+    if _DIAG_ENABLED:
+        torch.cuda.synchronize()
+        t0 = time.perf_counter()
+    _lib.check(_lib.load().rdkv_k_qk_dot(*args, out.data_ptr(), out.stride(0), _lib.stream_of(dev)))
+    del keep     # what the launch above reads lives until it is enqueued
+    if _DIAG_ENABLED:
+        torch.cuda.synchronize()
+        _DIAG["kernel_ms"] += (time.perf_counter() - t0) * 1000.0
+        _DIAG["n_calls"] += 1
+
+
+def _scores_args(Q: torch.Tensor, packed_layer, T_eff: int, out: torch.Tensor):
+    """What the K launches take of a query and a layer, checked -> (arguments, device, tensors they point into)."""
     H_q = Q.shape[0]
     assert Q.shape[1] == D, f"Q head_dim {Q.shape[1]} != {D}"
     dev = _lib.require_device(Q, out)
@@ -101,20 +116,10 @@ def k_mixed_qk_dot_into(Q: torch.Tensor, packed_layer, T_eff: int, out: torch.Te
     K2, k2h, k2t = _seg3(packed_layer.K_2bit)
     K4, k4h, k4t = _seg3(packed_layer.K_4bit)
     K8, k8h, k8t = _seg3(packed_layer.K_8bit)
-    t0 = 0.0
-    if _DIAG_ENABLED:
-        torch.cuda.synchronize()
-        t0 = time.perf_counter()
-    _lib.check(_lib.load().rdkv_k_qk_dot(
-        Q.data_ptr(), _lib.DTYPE_CODE[Q.dtype], Q.stride(0), H_q, H_kv,
-        _lib.ptr(K2), k2h, k2t, _lib.ptr(K4), k4h, k4t, _lib.ptr(K8), k8h, k8t,
-        _lib.ptr(sc), _lib.ptr(zp), sc.stride(0) if sc.numel() else 0,
-        _lib.ptr(perm), perm_sh, n2p, n4p, n8, int(T_eff),
-        out.data_ptr(), out.stride(0), _lib.stream_of(dev)))
-    if _DIAG_ENABLED:
-        torch.cuda.synchronize()
-        _DIAG["kernel_ms"] += (time.perf_counter() - t0) * 1000.0
-        _DIAG["n_calls"] += 1
+    return (Q.data_ptr(), _lib.DTYPE_CODE[Q.dtype], Q.stride(0), H_q, H_kv,
+            _lib.ptr(K2), k2h, k2t, _lib.ptr(K4), k4h, k4t, _lib.ptr(K8), k8h, k8t,
+            _lib.ptr(sc), _lib.ptr(zp), sc.stride(0) if sc.numel() else 0,
+            _lib.ptr(perm), perm_sh, n2p, n4p, n8, int(T_eff)), dev, (Q, K2, K4, K8)
 
 
 def k_mixed_qk_dot(Q: torch.Tensor, packed_layer, T_eff: int) -> torch.Tensor:

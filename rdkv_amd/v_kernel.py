@@ -72,7 +72,8 @@ def _seg(t, width):
 def _launch(attn_weights, V_2bit, V_4bit, V_8bit, V_scale, V_zp, seg_bounds_per_head, seg_bounds,
             out, V16, n_v16_per_head, max_T_v, new=None):
     """``new`` = (weights [H_q, n], values fp32 [H_kv, n, 128] with 16-byte aligned rows): a further zone,
-    added by the same launch; V_scale may then be None (nothing packed)."""
+    added by the same launch; V_scale may then be None (nothing packed).  A third entry (workspace, how much of
+    it ``rdkv_attn_scores`` took, its pairs, keep the weights): the rows ``attn_weights`` | weights hold scores."""
     # (this runs once per layer and decode step: views and helper calls are kept to what the launch needs)
     lib = _lib.load()
     w = attn_weights
@@ -107,15 +108,21 @@ def _launch(attn_weights, V_2bit, V_4bit, V_8bit, V_scale, V_zp, seg_bounds_per_
         n16 = n_v16_per_head.data_ptr()
         v16 = keep16.data_ptr() if keep16.numel() else None
     stream = _lib.stream_of(dev)
-    ws = _lib.workspace(dev, lib.rdkv_v_weighted_sum_workspace_bytes(H_q))
+    scores = new[2] if new is not None and len(new) > 2 else None
+    ws_bytes = lib.rdkv_v_weighted_sum_workspace_bytes(H_q)
+    ws, taken = (_lib.workspace(dev, ws_bytes), 0) if scores is None else scores[:2]
     packed = (
         w.data_ptr(), w.stride(0), H_q, H_kv, V2, v2h, V4, v4h, V8, v8h,
         sc.data_ptr() if n_meta else None, zp.data_ptr() if n_meta else None, sc.stride(0) if n_meta else 0,
         None if seg_bounds_per_head is None else seg_bounds_per_head.data_ptr(), int(N2), int(N4), int(N8),
         v16, v16h or 0, n16 if v16 is not None else None, int(max_T_v))
-    result = (out.data_ptr(), out.stride(0), ws.data_ptr(), ws.numel(), stream)
+    result = (out.data_ptr(), out.stride(0), ws.data_ptr() + taken, ws.numel() - taken, stream)
     if new is None:
         _lib.check(lib.rdkv_v_weighted_sum(*packed, *result))
+    elif scores is not None:
+        vn, (_, _, pairs, keep) = new[1], scores
+        _lib.check(lib.rdkv_v_weighted_sum_scores(*packed, w.shape[1], vn.data_ptr(), vn.stride(0), vn.stride(1),
+                                                  vn.shape[1], ws.data_ptr(), pairs, keep, *result))
     else:
         wn, vn = new
         _lib.check(lib.rdkv_v_weighted_sum_new_values(*packed, wn.data_ptr(), wn.stride(0), vn.data_ptr(), vn.stride(0),
@@ -214,10 +221,10 @@ def v_dequant_weighted_sum_dispatch_into(attn_weights_old, packed_layer, out, V1
                                         pl.V_scale, pl.V_zp, pl.seg_bounds, out)
 
 
-def _weighted_sum_with_new_zone(attn_weights_old, packed_layer, out, V16, n_v16_per_head, max_T_v, w_new, V_new):
+def _weighted_sum_with_new_zone(attn_weights_old, packed_layer, out, V16, n_v16_per_head, max_T_v, w_new, V_new, scores=None):
     """``v_dequant_weighted_sum_dispatch_into`` plus ``w_new`` . ``V_new``, in the same launches;
-    ``packed_layer`` None: the new zone alone."""
-    pl, new = packed_layer, (w_new, V_new)
+    ``packed_layer`` None: the new zone alone; ``scores``: see ``_launch``."""
+    pl, new = packed_layer, (w_new, V_new) if scores is None else (w_new, V_new, scores)
     per_head = getattr(pl, "seg_bounds_per_head", None)
     if per_head is None:
         V16 = None
