@@ -28,6 +28,7 @@ extern "C" {
 #define RDKV_EUNSUPPORTED -2   /* valid request this build does not implement */
 #define RDKV_ELAUNCH      -3   /* HIP reported a launch/runtime error         */
 #define RDKV_EWORKSPACE   -4   /* workspace missing or too small              */
+#define RDKV_EWAIT        -5   /* numbers of a launch not there in the time given */
 
 #define RDKV_DTYPE_F32  0
 #define RDKV_DTYPE_F16  1
@@ -106,7 +107,8 @@ int rdkv_pack_layer_per_head(const void *K_f16, const void *V_f16, int64_t strid
  * (V rows: pack_v_segments, packing.py:885; K rows: the deferred pack_k_mixed_per_head of the
  * stacking step, packing.py:1185-1213).  minmax_start: NULL, or the K half's
  * minmax_ws, whose start values this launch then writes; pass minmax_started != 0 to the K
- * half in that case (both calls on one stream, V half first). */
+ * half in that case (both calls on one stream, V half first); minmax_started == 2: minmax_ws holds the
+ * min / max themselves (rdkv_pack_layers_k_minmax). */
 int rdkv_pack_layer_v_rows(const void *V_f16, int64_t stride_h, int64_t stride_t, int H_kv, int D,
                            const int32_t *order, int64_t order_stride_h, const int32_t *counts,
                            int mN2, int mN4, int mN8, int64_t max_tv, int max_n16,
@@ -468,7 +470,8 @@ int rdkv_stream_relayout_layer(const uint8_t *K2, int64_t k2_stride_h, int64_t k
  * the quantizer of every channel).  minmax_ws_ready = 0: the call starts the accumulators itself (one
  * more small launch); != 0: they already hold their start values - after
  * rdkv_pack_layer_stream_ws_init, and after every earlier call on the same stream, which leaves them
- * at their start values again - so a scratch that is kept needs preparing once.
+ * at their start values again - so a scratch that is kept needs preparing once; 2: they hold the min / max
+ * themselves (rdkv_pack_layers_k_minmax).
  * scale_max: float [2][H_kv]: receives per head the largest K channel scale and the largest V token
  * scale (as the fp16 values stored), which RdkvWork.k_scale_max / v_shift are made from.  K and V
  * rows must be 16-byte aligned (RDKV_EUNSUPPORTED otherwise). */
@@ -635,6 +638,27 @@ int rdkv_pack_layer_plan(const void *v_bits, int vb_elem_size, int64_t vb_stride
                          int kb_elem_size, int64_t kb_stride_h, int H_kv, int64_t T, int D,
                          int32_t *order, int64_t order_stride_h, int32_t *rank3, int64_t rank3_stride_h,
                          int32_t *plan, void *stream);
+
+/* The same, which also writes the start values of the K min / max accumulators: minmax_ws
+ * [H_kv][minmax_floats_per_head], D minima and D maxima in turn (NULL: none), and sends the H_kv * 12 values
+ * to the host by itself: host_words [H_kv][12] in pinned host memory (NULL: not), value | tag << 32, the tag other
+ * than what the words held before.  rdkv_pack_layer_plan_wait (host only) waits for them, at most
+ * wait_us microseconds (RDKV_EWAIT: not there yet), and writes them in plan's order. */
+int rdkv_pack_layer_plan_start(const void *v_bits, int vb_elem_size, int64_t vb_stride_h, const void *k_bits,
+                               int kb_elem_size, int64_t kb_stride_h, int H_kv, int64_t T, int D,
+                               int32_t *order, int64_t order_stride_h, int32_t *rank3, int64_t rank3_stride_h,
+                               int32_t *plan, float *minmax_ws, int minmax_floats_per_head, uint64_t *host_words,
+                               uint32_t tag, void *stream);
+int rdkv_pack_layer_plan_wait(const uint64_t *host_words, int n_heads, uint32_t tag, int32_t *plan, int64_t wait_us);
+
+/* K min / max of the kept rows of n_layers layers of one shape, from what the planning launches left on the
+ * device (order, counts: rows of layer l from l * H_kv on), before the host has read the class sizes: K_f16[l]
+ * with strides[2 l], strides[2 l + 1] (head, token), rows 4-byte aligned; layer l's accumulators, started, at
+ * minmax_ws + l * ws_stride.  rdkv_pack_layer_k_rows and rdkv_pack_layer_stream take them with
+ * minmax_started / minmax_ws_ready = 2. */
+int rdkv_pack_layers_k_minmax(const void *const *K_f16, const int64_t *strides, int n_layers, int H_kv, int64_t T, int D,
+                              const int32_t *order, int64_t order_stride_h, const int32_t *counts,
+                              float *minmax_ws, int64_t ws_stride, void *stream);
 
 /* Per-head tables and metadata of the stacked layer (packing.py:399-578 pack_k_mixed_per_head's
  * index tensors, :1245-1316 of _pad_and_stack_per_head_layers), from the layer's rows of the two

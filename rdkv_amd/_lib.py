@@ -100,6 +100,9 @@ SIGNATURES = {
     "rdkv_decode_fused_merge": (I, [P, I, I, I, P, L, P, P, L, P]),
     "rdkv_pack_layer_plan_ints": (L, [I, L]),
     "rdkv_pack_layer_plan": (I, [P, I, L, P, I, L, I, L, I, P, L, P, L, P, P]),
+    "rdkv_pack_layer_plan_start": (I, [P, I, L, P, I, L, I, L, I, P, L, P, L, P, P, I, P, ctypes.c_uint32, P]),
+    "rdkv_pack_layer_plan_wait": (I, [P, I, ctypes.c_uint32, P, L]),
+    "rdkv_pack_layers_k_minmax": (I, [P, P, I, I, L, I, P, L, P, P, L, P]),
     "rdkv_pack_layer_tables": (I, [P, I, L, I, I, I, P, P, I, I, I, I, L, I, P, L, P, L, I, L,
                                    P, P, P, P, P, P, P, P, P, P, P, P]),
     "rdkv_pool_scores": (I, [P, L, I, L, I, I, I, P, L, P]),

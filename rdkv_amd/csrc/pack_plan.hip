@@ -5,6 +5,8 @@
 // shapes of the packed tensors) and no per-head loop.
 #include "rdkv_common.h"
 
+#include <chrono>
+
 namespace {
 
 constexpr int kPlanThreads = 1024;
@@ -37,11 +39,12 @@ __device__ __forceinline__ int lanes_below(uint64_t mask) {
 
 // Token planning in two launches over a (chunk, head) grid, kPlanThreads tokens per chunk.
 // First launch: per-chunk class histogram hist[h][chunk][6]; the chunk-0 block of each head also
-// counts the head's channel classes.
+// counts the head's channel classes and writes the start values of its share of the K min / max scratch.
 __global__ void __launch_bounds__(kPlanThreads)
 plan_hist_kernel(const void *__restrict__ v_bits, int vb_es, int64_t vb_stride_h, int T,
                  const void *__restrict__ k_bits, int kb_es, int64_t kb_stride_h, int D,
-                 int32_t *__restrict__ hist, int32_t *__restrict__ info) {
+                 int32_t *__restrict__ hist, int32_t *__restrict__ info, uint32_t *__restrict__ minmax,
+                 int minmax_per_head) {
   __shared__ int cnt[kTokClasses];
   __shared__ int kcnt[4];
   const int h = blockIdx.y, chunk = blockIdx.x, nchunks = gridDim.x, tid = threadIdx.x, lane = tid & 63;
@@ -54,6 +57,10 @@ plan_hist_kernel(const void *__restrict__ v_bits, int vb_es, int64_t vb_stride_h
   for (int k = 0; k < kTokClasses; ++k) {
     const uint64_t m = __ballot(cls == k);
     if (lane == 0 && m) atomicAdd(&cnt[k], __popcll(m));
+  }
+  if (chunk == 0 && minmax) {
+    for (int i = tid; i < minmax_per_head; i += blockDim.x)
+      minmax[(int64_t)h * minmax_per_head + i] = rdkv_float_to_ordered(((i / D) & 1) ? -INFINITY : INFINITY);
   }
   if (chunk == 0) {
     int bad = 0;
@@ -81,7 +88,7 @@ __global__ void __launch_bounds__(kPlanThreads)
 plan_scatter_kernel(const void *__restrict__ v_bits, int vb_es, int64_t vb_stride_h, int T,
                     const int32_t *__restrict__ hist, int32_t *__restrict__ order, int64_t order_stride_h,
                     int32_t *__restrict__ rank3, int64_t rank3_stride_h, int32_t *__restrict__ counts4,
-                    int32_t *__restrict__ info) {
+                    int32_t *__restrict__ info, uint64_t *__restrict__ host_words, uint32_t tag) {
   __shared__ int wsum[kPlanThreads / 64][2 * kTokClasses];
   __shared__ int red[2 * kTokClasses];
   __shared__ int wcnt[kPlanThreads / 64][kTokClasses];
@@ -149,6 +156,12 @@ plan_scatter_kernel(const void *__restrict__ v_bits, int vb_es, int64_t vb_strid
     if (tid < 4) counts4[4 * h + tid] = red[tid];
     if (tid == 4) info[8 * h + 0] = red[4];
     if (tid == 5) info[8 * h + 1] = red[5];
+    // the head's twelve numbers to the host, each word with the call's tag: whole whenever its tag is there
+    if (host_words && tid < 12) {
+      const int v = tid < 6 ? red[tid] : info[8 * h + tid - 4];
+      __hip_atomic_store(host_words + 12 * (int64_t)h + tid, ((uint64_t)tag << 32) | (uint32_t)v, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
 }
 
@@ -276,10 +289,11 @@ RDKV_API int64_t rdkv_pack_layer_plan_ints(int H_kv, int64_t T) {
   return (int64_t)H_kv * (12 + kTokClasses * rdkv_cdiv(T, kPlanThreads));
 }
 
-RDKV_API int rdkv_pack_layer_plan(const void *v_bits, int vb_elem_size, int64_t vb_stride_h, const void *k_bits,
-                                  int kb_elem_size, int64_t kb_stride_h, int H_kv, int64_t T, int D,
-                                  int32_t *order, int64_t order_stride_h, int32_t *rank3,
-                                  int64_t rank3_stride_h, int32_t *plan, void *stream) {
+RDKV_API int rdkv_pack_layer_plan_start(const void *v_bits, int vb_elem_size, int64_t vb_stride_h, const void *k_bits,
+                                        int kb_elem_size, int64_t kb_stride_h, int H_kv, int64_t T, int D,
+                                        int32_t *order, int64_t order_stride_h, int32_t *rank3,
+                                        int64_t rank3_stride_h, int32_t *plan, float *minmax_ws,
+                                        int minmax_floats_per_head, uint64_t *host_words, uint32_t tag, void *stream) {
   const char *fn = "rdkv_pack_layer_plan";
   RDKV_REQUIRE(H_kv >= 1 && H_kv <= 65535 && D >= 1 && T >= 1 && T <= (1LL << 30), "%s: bad shape", fn);
   RDKV_REQUIRE(elem_size_ok(vb_elem_size) && elem_size_ok(kb_elem_size), "%s: element sizes must be 1, 2, 4 or 8", fn);
@@ -288,11 +302,43 @@ RDKV_API int rdkv_pack_layer_plan(const void *v_bits, int vb_elem_size, int64_t 
   int32_t *counts4 = plan, *info = plan + 4 * (int64_t)H_kv, *hist = plan + 12 * (int64_t)H_kv;
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(plan_hist_kernel, dim3((unsigned)nchunks, H_kv), dim3(kPlanThreads), 0, s, v_bits, vb_elem_size,
-                     vb_stride_h, (int)T, k_bits, kb_elem_size, kb_stride_h, D, hist, info);
+                     vb_stride_h, (int)T, k_bits, kb_elem_size, kb_stride_h, D, hist, info, (uint32_t *)minmax_ws,
+                     minmax_floats_per_head);
   hipLaunchKernelGGL(plan_scatter_kernel, dim3((unsigned)nchunks, H_kv), dim3(kPlanThreads), 0, s, v_bits,
                      vb_elem_size, vb_stride_h, (int)T, hist, order, order_stride_h, rank3, rank3_stride_h, counts4,
-                     info);
+                     info, host_words, tag);
   RDKV_CHECK_LAUNCH(fn);
+  return RDKV_OK;
+}
+
+RDKV_API int rdkv_pack_layer_plan(const void *v_bits, int vb_elem_size, int64_t vb_stride_h, const void *k_bits,
+                                  int kb_elem_size, int64_t kb_stride_h, int H_kv, int64_t T, int D,
+                                  int32_t *order, int64_t order_stride_h, int32_t *rank3,
+                                  int64_t rank3_stride_h, int32_t *plan, void *stream) {
+  return rdkv_pack_layer_plan_start(v_bits, vb_elem_size, vb_stride_h, k_bits, kb_elem_size, kb_stride_h, H_kv, T, D, order,
+                                    order_stride_h, rank3, rank3_stride_h, plan, nullptr, 0, nullptr, 0, stream);
+}
+
+RDKV_API int rdkv_pack_layer_plan_wait(const uint64_t *host_words, int n_heads, uint32_t tag, int32_t *plan, int64_t wait_us) {
+  RDKV_REQUIRE(host_words && plan && n_heads >= 0, "rdkv_pack_layer_plan_wait: bad arguments");
+  const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(wait_us);
+  for (int64_t i = 0; i < 12 * (int64_t)n_heads; ++i) {
+    const int64_t h = i / 12, k = i % 12;
+    for (int spins = 0;; ++spins) {
+      const uint64_t w = __atomic_load_n(host_words + i, __ATOMIC_ACQUIRE);
+      if ((uint32_t)(w >> 32) == tag) {
+        plan[k < 4 ? 4 * h + k : 4 * (int64_t)n_heads + 8 * h + (k - 4)] = (int32_t)(uint32_t)w;
+        break;
+      }
+      if ((spins & 255) == 255 && std::chrono::steady_clock::now() > until) {
+        rdkv_set_error("rdkv_pack_layer_plan_wait: not there after %lld us", (long long)wait_us);
+        return RDKV_EWAIT;
+      }
+#if defined(__x86_64__)
+      __builtin_ia32_pause();
+#endif
+    }
+  }
   return RDKV_OK;
 }
 

@@ -1304,13 +1304,13 @@ void rdkv_layer_k_minmax_init(float *minmax_ws, int H_kv, int D, hipStream_t s) 
 }
 
 // The K half: per-channel min/max over each head's kept rows, then scales, zero points and the
-// packed K segments.  `mm_ready` says the accumulators in `minmax_ws` already hold their start
-// values (the V half wrote them on the same stream).
+// packed K segments.  `mm_state`: 1 says the accumulators in `minmax_ws` already hold their start
+// values (the V half wrote them on the same stream), 2 the min / max themselves (rdkv_pack_layers_k_minmax).
 static int pack_layer_k_rows(const char *fn, const void *K_f16, int64_t stride_h, int64_t stride_t, int H_kv, int D,
                              const int32_t *order, int64_t order_stride_h, const int32_t *counts, int64_t max_tv,
                              int max_n16, const int32_t *slot_channel, int n2p, int n4p, int n8, uint8_t *K2,
                              uint8_t *K4, uint8_t *K8, void *K_scale_f16, void *K_zp_f16, float *minmax_ws,
-                             bool mm_ready, hipStream_t s) {
+                             int mm_state, hipStream_t s) {
   RDKV_REQUIRE(H_kv >= 1 && H_kv <= 65535 && D > 0 && D % 4 == 0, "%s: bad H_kv=%d / D=%d", fn, H_kv, D);
   RDKV_REQUIRE(max_n16 >= 0 && max_tv >= 0, "%s: negative counts", fn);
   RDKV_REQUIRE(n2p >= 0 && n4p >= 0 && n8 >= 0 && n2p % 4 == 0 && n4p % 2 == 0,
@@ -1328,9 +1328,9 @@ static int pack_layer_k_rows(const char *fn, const void *K_f16, int64_t stride_h
                "%s: null K output", fn);
   uint32_t *mm = reinterpret_cast<uint32_t *>(minmax_ws);
   const bool rows16 = D == 128 && stride_t % 8 == 0 && stride_h % 8 == 0 && ((uintptr_t)K_f16 % 16) == 0;
-  {
+  if (mm_state != 2) {
     const int rc = layer_k_minmax(fn, K_f16, stride_h, stride_t, H_kv, D, order, order_stride_h, counts, max_tk, mm,
-                                  !mm_ready, s);
+                                  mm_state == 0, s);
     if (rc != RDKV_OK) return rc;
   }
   const int rows_per_block = 64;
@@ -1373,7 +1373,7 @@ RDKV_API int rdkv_pack_layer_per_head(const void *K_f16, const void *V_f16, int6
                              k_half ? minmax_ws : nullptr, (hipStream_t)stream);
   if (rc != RDKV_OK) return rc;
   return pack_layer_k_rows(fn, K_f16, stride_h, stride_t, H_kv, D, order, order_stride_h, counts, max_tv, max_n16,
-                           slot_channel, n2p, n4p, n8, K2, K4, K8, K_scale_f16, K_zp_f16, minmax_ws, v_rows > 0,
+                           slot_channel, n2p, n4p, n8, K2, K4, K8, K_scale_f16, K_zp_f16, minmax_ws, v_rows > 0 ? 1 : 0,
                            (hipStream_t)stream);
 }
 
@@ -1394,5 +1394,26 @@ RDKV_API int rdkv_pack_layer_k_rows(const void *K_f16, int64_t stride_h, int64_t
                                     void *K_zp_f16, float *minmax_ws, int minmax_started, void *stream) {
   return pack_layer_k_rows("rdkv_pack_layer_k_rows", K_f16, stride_h, stride_t, H_kv, D, order, order_stride_h,
                            counts, max_tv, max_n16, slot_channel, n2p, n4p, n8, K2, K4, K8, K_scale_f16, K_zp_f16,
-                           minmax_ws, minmax_started != 0, (hipStream_t)stream);
+                           minmax_ws, minmax_started, (hipStream_t)stream);
+}
+
+RDKV_API int rdkv_pack_layers_k_minmax(const void *const *K_f16, const int64_t *strides, int n_layers, int H_kv, int64_t T, int D,
+                                       const int32_t *order, int64_t order_stride_h, const int32_t *counts,
+                                       float *minmax_ws, int64_t ws_stride, void *stream) {
+  const char *fn = "rdkv_pack_layers_k_minmax";
+  RDKV_REQUIRE(n_layers >= 0 && H_kv >= 1 && H_kv <= 65535 && D > 0 && D % 4 == 0 && T >= 1 && T <= (1LL << 30),
+               "%s: bad shape", fn);
+  RDKV_REQUIRE(n_layers == 0 || (K_f16 && strides && order && counts && minmax_ws && ws_stride >= (int64_t)H_kv * 2 * D),
+               "%s: bad arguments", fn);
+  for (int l = 0; l < n_layers; ++l) {
+    const int64_t sh = strides[2 * l], st = strides[2 * l + 1];
+    RDKV_REQUIRE(K_f16[l] && st % 2 == 0 && sh % 2 == 0 && ((uintptr_t)K_f16[l] % 4) == 0, "%s: rows must be 4-byte aligned",
+                 fn);
+    const int rc = layer_k_minmax(fn, K_f16[l], sh, st, H_kv, D, order + (int64_t)l * H_kv * order_stride_h, order_stride_h,
+                                  counts + 4 * (int64_t)l * H_kv, T, reinterpret_cast<uint32_t *>(minmax_ws + l * ws_stride),
+                                  false, (hipStream_t)stream);
+    if (rc != RDKV_OK) return rc;
+  }
+  RDKV_CHECK_LAUNCH(fn);
+  return RDKV_OK;
 }

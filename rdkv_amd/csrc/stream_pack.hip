@@ -520,9 +520,11 @@ RDKV_API int rdkv_pack_layer_stream(const void *K_f16, const void *V_f16, int64_
   hipStream_t s = (hipStream_t)stream;
   const int64_t max_tk = max_tv + max_n16;
   // per-channel min / max of every head's kept rows (the K canvas without its zero rows)
-  int rc = rdkv_layer_k_minmax(fn, K_f16, stride_h, stride_t, H_kv, kD, order, order_stride_h, counts, max_tk,
-                               minmax_ws, /*init=*/minmax_ws_ready == 0, s);
-  if (rc != RDKV_OK) return rc;
+  if (minmax_ws_ready != 2) {
+    const int rc = rdkv_layer_k_minmax(fn, K_f16, stride_h, stride_t, H_kv, kD, order, order_stride_h, counts, max_tk,
+                                       minmax_ws, /*init=*/minmax_ws_ready == 0, s);
+    if (rc != RDKV_OK) return rc;
+  }
   StreamPackArgs a;
   a.K = (const __half *)K_f16; a.V = (const __half *)V_f16;
   a.stride_h = stride_h; a.stride_t = stride_t;

@@ -18,7 +18,7 @@ from torch import Tensor
 from . import _lib
 from .knapsack_solver import (DEFAULT_EPSILON_K, DEFAULT_EPSILON_V, knapsack_allocate,   # noqa: F401 (re-exported
                               knapsack_bit_allocation_batched, load_epsilon_kv_from_calibration)  # as obkv_fast.py:38-46 does)
-from .packing import pack_layer_per_head, pack_layers_per_head
+from .packing import _pack_layer_per_head, pack_layer_per_head, pack_layers_per_head  # noqa: F401
 
 
 def apply_score_pooling(scores: Tensor, pool_type: str, kernel_size: int, padding_mode: str = "zero") -> Tensor:
@@ -167,10 +167,17 @@ def _perhead_select_and_pack_joint(
                                                epsilon=eps_K, bit_options=k_bit_options)
     t_k = stamp()
 
-    packed_layer, new_v_only = pack_layer_per_head(K, V, v_bits_all, k_bits_perhead, gqa_factor)
+    retained: list = []
+
+    def retain():      # (runs under the packer's host read)
+        retained.extend((v_bits_all.to(torch.int16), k_bits_perhead.to(torch.int16)))
+
+    packed_layer, new_v_only = _pack_layer_per_head(K, V, v_bits_all, k_bits_perhead, gqa_factor,
+                                                    retain if retain_allocation_metadata else None)
     if retain_allocation_metadata:
-        packed_layer.allocation_v_bits = v_bits_all.to(torch.int16)
-        packed_layer.allocation_k_bits = k_bits_perhead.to(torch.int16)
+        if not retained:
+            retain()
+        packed_layer.allocation_v_bits, packed_layer.allocation_k_bits = retained
     t_pack = stamp()
 
     if timing is not None:

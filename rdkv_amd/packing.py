@@ -13,6 +13,7 @@ from __future__ import annotations
 from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
 
+import ctypes
 import threading
 
 import torch
@@ -735,10 +736,54 @@ def _read_ints(t: Tensor, n: int) -> list:
     return buf[:n].tolist()
 
 
-def _plan_layers(v_bits: Tensor, k_bits: Tensor, dev):
+class _PlanWords:
+    """Pinned words that a planning launch fills for the host thread that waits for them, twelve a head, and
+    the tag of the last call.  Without a copy and a wait for the stream, what is launched behind the plan runs
+    while the host reads and sizes the outputs."""
+    WAIT_US = 100_000          # behind longer work than this the stream's own wait takes over
+
+    def __init__(self, heads: int):
+        with torch.inference_mode(False):      # (written outside the mode it may be made in)
+            self.words = torch.zeros(12 * heads, dtype=torch.int64, pin_memory=True)
+        self.heads, self.tag = heads, 0
+        self.ptr = self.words.data_ptr()
+
+
+_plan_words: dict = {}         # (device, host thread) -> its words
+_outgrown_words: list = []     # kept: a launch whose caller was interrupted may still write to them
+
+
+def _words_for(dev: torch.device, heads: int) -> _PlanWords:
+    key = (dev.index, threading.get_ident())
+    w = _plan_words.get(key)
+    if w is None or w.heads < heads:
+        if w is not None:
+            _outgrown_words.append(w)
+        w = _plan_words[key] = _PlanWords(max(256, 1 << (heads - 1).bit_length()))
+    w.tag = w.tag % 0xFFFFFFFF + 1             # (never 0, what fresh words hold)
+    return w
+
+
+# Tokens from which a layer's K min / max are launched ahead of the host's read of the plan.  Below, the host is
+# the longer side and their own call costs 3 .. 7 us of it.  Us a call ahead / behind, 8 KV heads: selection and packing
+# of 16k tokens 177 / 176, 31k 178 / 178, 64k 200 / 222, 100k 272 / 304; four layers to the streaming format 4k
+# 507 / 501, 16k 524 / 520, 24k 547 / 543, 32k 543 / 583.
+_EARLY_MINMAX_TOKENS = 28672
+
+
+def _early_minmax(Ks: Sequence[Tensor], dev) -> bool:
+    """Whether the K min / max of these layers can be taken as soon as the token order is planned."""
+    return all(K.dtype == torch.float16 and K.device == dev and K.dim() == 4 and K.shape[0] == 1 and K.stride(3) == 1
+               and K.shape[2] >= _EARLY_MINMAX_TOKENS and K.shape[3] % 4 == 0 and K.shape[3] <= 1024
+               and K.stride(1) % 2 == 0 and K.stride(2) % 2 == 0 and K.data_ptr() % 4 == 0 for K in Ks)
+
+
+def _plan_layers(v_bits: Tensor, k_bits: Tensor, dev, Ks: Sequence[Tensor] = (), minmax_per_head: int = 0, meanwhile=None):
     """Token order, quantized-token ranks and class sizes of ``[N, T]`` / ``[N, D]`` allocations
     (N = heads of one layer, or of several layers stacked) in one launch pair and one host read.
-    Returns (order, rank3, plan, counts rows [N][4], info rows [N][8], k_bits as passed on)."""
+    Returns (order, rank3, plan, counts rows [N][4], info rows [N][8], k_bits as passed on, K min / max).
+    ``Ks``: the layers' K (``_early_minmax``), whose min / max are launched right behind the plan and land in the
+    last entry, ``minmax_per_head`` floats a head, otherwise None; ``meanwhile``: further launches to enqueue there."""
     lib = _lib.load()
     vb = v_bits if v_bits.device == dev else v_bits.to(dev)
     kb = k_bits if k_bits.device == dev else k_bits.to(dev)
@@ -754,16 +799,34 @@ def _plan_layers(v_bits: Tensor, k_bits: Tensor, dev):
     order = torch.empty(N, T, dtype=torch.int32, device=dev)
     rank3 = torch.empty(N, T, dtype=torch.int32, device=dev)
     plan = torch.empty(lib.rdkv_pack_layer_plan_ints(N, T), dtype=torch.int32, device=dev)
-    _lib.check(lib.rdkv_pack_layer_plan(vb.data_ptr(), vb.element_size(), vb.stride(0), kb.data_ptr(),
-                                        kb.element_size(), kb.stride(0), N, T, int(kb.shape[1]), order.data_ptr(),
-                                        order.stride(0), rank3.data_ptr(), rank3.stride(0), plan.data_ptr(),
-                                        _lib.stream_of(dev)))
-    plan_h = _read_ints(plan, 12 * N)                           # the one synchronization
+    D = int(kb.shape[1])
+    mm = torch.empty(N * minmax_per_head, dtype=torch.float32, device=dev) if len(Ks) else None
+    # (a capture cannot wait for its launches: the stream's own wait says so)
+    words = None if torch.cuda.is_current_stream_capturing() else _words_for(plan.device, N)
+    _lib.check(lib.rdkv_pack_layer_plan_start(
+        vb.data_ptr(), vb.element_size(), vb.stride(0), kb.data_ptr(), kb.element_size(), kb.stride(0), N, T, D,
+        order.data_ptr(), order.stride(0), rank3.data_ptr(), rank3.stride(0), plan.data_ptr(),
+        mm.data_ptr() if mm is not None else None, minmax_per_head, words.ptr if words is not None else None,
+        words.tag if words is not None else 0, _lib.stream_of(dev)))
+    if mm is not None:
+        ptrs = (ctypes.c_void_p * len(Ks))(*[K.data_ptr() for K in Ks])
+        strides = (ctypes.c_int64 * (2 * len(Ks)))(*[s for K in Ks for s in (K.stride(1), K.stride(2))])
+        H = N // len(Ks)
+        _lib.check(lib.rdkv_pack_layers_k_minmax(ptrs, strides, len(Ks), H, T, D, order.data_ptr(), order.stride(0),
+                                                 plan.data_ptr(), mm.data_ptr(), H * minmax_per_head, _lib.stream_of(dev)))
+    if meanwhile is not None:
+        meanwhile()
+    # the one synchronization
+    numbers = (ctypes.c_int32 * (12 * N))()
+    if words is not None and lib.rdkv_pack_layer_plan_wait(words.ptr, N, words.tag, numbers, words.WAIT_US) == _lib.RDKV_OK:
+        plan_h = list(numbers)
+    else:
+        plan_h = _read_ints(plan, 12 * N)
     counts_h = [plan_h[4 * h:4 * h + 4] for h in range(N)]
     info_h = [plan_h[4 * N + 8 * h:4 * N + 8 * h + 8] for h in range(N)]
     assert all(row[1] == 0 for row in info_h), "v_bits must be in {0,2,4,8,16}"
     assert all(row[5] == 0 for row in info_h), "k_bits must be in {0,2,4,8,16}"
-    return order, rank3, plan, counts_h, info_h, kb
+    return order, rank3, plan, counts_h, info_h, kb, mm
 
 
 def _pack_planned_layer(K: Tensor, V: Tensor, gqa_factor: int, planned, first: int, n_total: int,
@@ -772,7 +835,7 @@ def _pack_planned_layer(K: Tensor, V: Tensor, gqa_factor: int, planned, first: i
     heads.  Returns None when the layer is degenerate (nothing kept / no channels kept / more
     than 1024 channels) and must take the composed path.  ``one_call`` packs V and K rows with
     the single ``rdkv_pack_layer_per_head`` call instead of its two halves (same result)."""
-    order, rank3, plan, counts_all, info_all, kb_all = planned
+    order, rank3, plan, counts_all, info_all, kb_all, mm_all = planned
     dev = K.device
     lib = _lib.load()
     stream = _lib.stream_of(dev)
@@ -815,13 +878,14 @@ def _pack_planned_layer(K: Tensor, V: Tensor, gqa_factor: int, planned, first: i
     V_scale = torch.empty(1, H_kv, max_tv, 1, dtype=torch.float16, device=dev)    # rows past a head's own
     V_zp = torch.empty_like(V_scale)                                               # tokens are zeroed by the call
     new_v_only = (torch.empty(1, H_kv, max_n16, D, dtype=torch.float16, device=dev) if max_n16 > 0 else None)
-    mm = torch.empty(H_kv * 2 * D, dtype=torch.float32, device=dev)
+    early = mm_all is not None and not one_call
+    mm = mm_all[first * 2 * D:] if early else torch.empty(H_kv * 2 * D, dtype=torch.float32, device=dev)
     v_rows = mN[0] + mN[1] + mN[2] + max_n16
     if not one_call:
         _lib.check(lib.rdkv_pack_layer_v_rows(
             Vf.data_ptr(), Kf.stride(0), Kf.stride(1), H_kv, D, order_l.data_ptr(), order_l.stride(0),
             counts4_ptr, mN[0], mN[1], mN[2], max_tv, max_n16, _lib.ptr(V2), _lib.ptr(V4), _lib.ptr(V8),
-            _lib.ptr(V_scale), _lib.ptr(V_zp), _lib.ptr(new_v_only), mm.data_ptr(), stream))
+            _lib.ptr(V_scale), _lib.ptr(V_zp), _lib.ptr(new_v_only), None if early else mm.data_ptr(), stream))
 
     i32 = dict(dtype=torch.int32, device=dev)
     i64 = dict(dtype=torch.int64, device=dev)
@@ -857,7 +921,7 @@ def _pack_planned_layer(K: Tensor, V: Tensor, gqa_factor: int, planned, first: i
         _lib.check(lib.rdkv_pack_layer_k_rows(
             Kf.data_ptr(), Kf.stride(0), Kf.stride(1), H_kv, D, order_l.data_ptr(), order_l.stride(0),
             counts4_ptr, max_tv, max_n16, slot_ch.data_ptr(), 4 * sub2, 2 * sub4, m8, _lib.ptr(K2), _lib.ptr(K4),
-            _lib.ptr(K8), ks.data_ptr(), kz.data_ptr(), mm.data_ptr(), 1 if v_rows > 0 else 0, stream))
+            _lib.ptr(K8), ks.data_ptr(), kz.data_ptr(), mm.data_ptr(), 2 if early else 1 if v_rows > 0 else 0, stream))
 
     # metadata exactly as _pad_and_stack_per_head_layers / pack_k_mixed_per_head produce it
     packed = PackedKVLayer(
@@ -890,6 +954,12 @@ def pack_layer_per_head(K: Tensor, V: Tensor, v_bits_per_head: Tensor, k_bits_pe
     what the reference's fp16 canvas does to it, packing.py:1186-1190; V of another type is quantized
     from its own values by the per-segment composition, and its fp16-kept rows are refused with
     TypeError); v_bits [H_kv,T] in {0,2,4,8,16}; k_bits [H_kv,D].  Returns (layer, new_v_only)."""
+    return _pack_layer_per_head(K, V, v_bits_per_head, k_bits_per_head, gqa_factor)
+
+
+def _pack_layer_per_head(K: Tensor, V: Tensor, v_bits_per_head: Tensor, k_bits_per_head: Tensor, gqa_factor: int,
+                         meanwhile=None) -> Tuple[PackedKVLayer, Optional[Tensor]]:
+    """``pack_layer_per_head``; ``meanwhile`` enqueues launches of the caller's that need not wait for the host."""
     dev = _lib.require_device(K, V)
     assert K.dim() == 4 and K.shape[0] == 1 and K.shape == V.shape, (
         f"Expected K, V [1,H_kv,T,D], got {tuple(K.shape)} / {tuple(V.shape)}")
@@ -897,7 +967,8 @@ def pack_layer_per_head(K: Tensor, V: Tensor, v_bits_per_head: Tensor, k_bits_pe
     assert tuple(v_bits_per_head.shape) == (H_kv, T) and tuple(k_bits_per_head.shape) == (H_kv, D)
     if T == 0:
         return _pack_layer_per_head_composed(K, V, v_bits_per_head, k_bits_per_head, gqa_factor)
-    planned = _plan_layers(v_bits_per_head, k_bits_per_head, dev)
+    planned = _plan_layers(v_bits_per_head, k_bits_per_head, dev,
+                           (K,) if V.dtype == torch.float16 and _early_minmax((K,), dev) else (), 2 * D, meanwhile)
     done = _pack_planned_layer(K, V, gqa_factor, planned, 0, H_kv)
     if done is None:
         return _pack_layer_per_head_composed(K, V, v_bits_per_head, k_bits_per_head, gqa_factor)
@@ -916,7 +987,9 @@ def pack_layers_per_head(Ks: Sequence[Tensor], Vs: Sequence[Tensor], v_bits: Ten
     assert tuple(v_bits.shape) == (L, H_kv, T) and tuple(k_bits.shape) == (L, H_kv, D)
     if T == 0:
         return [_pack_layer_per_head_composed(Ks[l], Vs[l], v_bits[l], k_bits[l], gqa_factor) for l in range(L)]
-    planned = _plan_layers(v_bits.reshape(L * H_kv, T), k_bits.reshape(L * H_kv, D), dev)
+    fp16 = all(V.dtype == torch.float16 for V in Vs) and all(K.shape == Ks[0].shape for K in Ks)
+    planned = _plan_layers(v_bits.reshape(L * H_kv, T), k_bits.reshape(L * H_kv, D), dev,
+                           Ks if fp16 and _early_minmax(Ks, dev) else (), 2 * D)
     out = []
     for l in range(L):
         assert Ks[l].shape == Ks[0].shape == Vs[l].shape

@@ -435,7 +435,9 @@ def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_
             return torch.cat(ts)
 
         vb_all, kb_all = joined(2, T), joined(3, 128)
-        order, _, plan, counts_h, info_h, kb_dev = packing._plan_layers(vb_all.reshape(-1, T), kb_all.reshape(-1, 128), dev)
+        Ks = [entries[i][0] for i in idx]
+        order, _, plan, counts_h, info_h, kb_dev, mm_all = packing._plan_layers(
+            vb_all.reshape(-1, T), kb_all.reshape(-1, 128), dev, Ks if packing._early_minmax(Ks, dev) else (), 768)
         plans = []
         counts_a = np.asarray(counts_h, dtype=np.int32).reshape(-1, 4)
         chan_a = np.ascontiguousarray(np.asarray(info_h, dtype=np.int32).reshape(-1, 8)[:, 2:5])
@@ -465,7 +467,7 @@ def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_
         live = [p for p in plans if p is not None]
         if live:
             units_dev, src_dev = _lib.upload(dev, units_grp[:n_live * H_kv], src_grp[:n_live * H_kv])
-            mm = _pack_scratch(dev, stream, H_kv)
+            mm = _pack_scratch(dev, stream, H_kv) if mm_all is None else None
             sm_all = torch.empty(len(live), 2, H_kv, dtype=torch.float32, device=dev)
         row = 0
         for j, (i, p) in enumerate(zip(idx, plans)):
@@ -491,12 +493,13 @@ def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_
                 kb_dev.element_size(), kb_dev.stride(0),
                 n2p, n4p, m8, max_tv, max_n16, units_dev.data_ptr() + row * UNIT_DTYPE.itemsize,
                 src_dev.data_ptr() + row * src_tab.shape[1] * 2, src_tab.shape[1], max_tiles, base, blob_bytes,
-                mm.data_ptr(), _SCRATCH_PREPARED, sm_all.data_ptr() + 4 * k * sm_all.stride(0), stream))
+                mm.data_ptr() if mm is not None else mm_all.data_ptr() + 4 * 768 * j * H_kv,
+                _SCRATCH_PREPARED if mm is not None else 2, sm_all.data_ptr() + 4 * k * sm_all.stride(0), stream))
             row += H_kv
             _add_base(units, base)
             pending.append((i, units, blob, sm_all[k], sb, ab, None))
         if live:
-            pending.append((None, None, None, None, 0, 0, (units_dev, src_dev, sm_all, kb_dev, order, plan)))
+            pending.append((None, None, None, None, 0, 0, (units_dev, src_dev, sm_all, kb_dev, order, plan, mm_all)))
     sm_dev = None
     if pending:
         sms = [pn[3] for pn in pending if pn[0] is not None]
