@@ -30,6 +30,11 @@ extern "C" {
 #define RDKV_EWORKSPACE   -4   /* workspace missing or too small              */
 #define RDKV_EWAIT        -5   /* numbers of a launch not there in the time given */
 
+/* Numbers that a launch sends to the host by itself: words in pinned host memory, value | tag << 32 (the tag other
+ * than what the words held before).  Host only: waits until all n are there, at most wait_us microseconds
+ * (RDKV_EWAIT), and writes their values. */
+int rdkv_host_words_wait(const uint64_t *words, int64_t n, uint32_t tag, int32_t *values, int64_t wait_us);
+
 #define RDKV_DTYPE_F32  0
 #define RDKV_DTYPE_F16  1
 #define RDKV_DTYPE_BF16 2
@@ -153,11 +158,25 @@ int rdkv_unpack_layer_k_checked(const uint8_t *K2, int64_t k2_stride_h, int64_t 
                                 const int64_t *sort_idx, int64_t sort_stride_h, int sort_n,
                                 const int32_t *counts, int n2, int n4, int n8, int n2p, int n4p, int n8w, int H_kv,
                                 int64_t T, int D, void *out_f16, int32_t *check, void *stream);
+/* The same four numbers a head to the host by itself (rdkv_host_words_wait): words [H_kv][4]. */
+int rdkv_unpack_layer_k_words(const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t,
+                              const uint8_t *K4, int64_t k4_stride_h, int64_t k4_stride_t,
+                              const uint8_t *K8, int64_t k8_stride_h, int64_t k8_stride_t,
+                              const void *scale_f16, const void *zp_f16, int64_t ks_stride_h,
+                              const int64_t *sort_idx, int64_t sort_stride_h, int sort_n,
+                              const int32_t *counts, int n2, int n4, int n8, int n2p, int n4p, int n8w, int H_kv,
+                              int64_t T, int D, void *out_f16, uint64_t *words, uint32_t tag, void *stream);
 int rdkv_unpack_layer_v(const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h,
                         const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
                         int64_t s_stride_h, const int32_t *counts, int m2, int m4, int m8, int64_t max_tv,
                         const void *V16_f16, int64_t v16_stride_h, int n16, int H_kv, int D,
                         void *out_f16, void *stream);
+/* The same; words [H_kv][4] gets per head its three counts and totals[h] (device int32). */
+int rdkv_unpack_layer_v_words(const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h,
+                        const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
+                        int64_t s_stride_h, const int32_t *counts, int m2, int m4, int m8, int64_t max_tv,
+                        const void *V16_f16, int64_t v16_stride_h, int n16, int H_kv, int D,
+                        void *out_f16, const int32_t *totals, uint64_t *words, uint32_t tag, void *stream);
 
 /* ---- triton_k_kernel.py : k_mixed_qk_dot_into (:1211-1411) ---------------- */
 /* out[hq, t] = (sum_c code[hkv,t,c] * q[hq, perm[c]] * s[hkv,c] - sum_c z*q*s) / sqrt(128),
@@ -641,15 +660,13 @@ int rdkv_pack_layer_plan(const void *v_bits, int vb_elem_size, int64_t vb_stride
 
 /* The same, which also writes the start values of the K min / max accumulators: minmax_ws
  * [H_kv][minmax_floats_per_head], D minima and D maxima in turn (NULL: none), and sends the H_kv * 12 values
- * to the host by itself: host_words [H_kv][12] in pinned host memory (NULL: not), value | tag << 32, the tag other
- * than what the words held before.  rdkv_pack_layer_plan_wait (host only) waits for them, at most
- * wait_us microseconds (RDKV_EWAIT: not there yet), and writes them in plan's order. */
+ * to the host by itself: host_words [H_kv][12] (NULL: not), a head's four counts, then its eight further
+ * numbers, for rdkv_host_words_wait. */
 int rdkv_pack_layer_plan_start(const void *v_bits, int vb_elem_size, int64_t vb_stride_h, const void *k_bits,
                                int kb_elem_size, int64_t kb_stride_h, int H_kv, int64_t T, int D,
                                int32_t *order, int64_t order_stride_h, int32_t *rank3, int64_t rank3_stride_h,
                                int32_t *plan, float *minmax_ws, int minmax_floats_per_head, uint64_t *host_words,
                                uint32_t tag, void *stream);
-int rdkv_pack_layer_plan_wait(const uint64_t *host_words, int n_heads, uint32_t tag, int32_t *plan, int64_t wait_us);
 
 /* K min / max of the kept rows of n_layers layers of one shape, from what the planning launches left on the
  * device (order, counts: rows of layer l from l * H_kv on), before the host has read the class sizes: K_f16[l]

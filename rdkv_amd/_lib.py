@@ -29,6 +29,7 @@ RDKV_EINVAL = -1
 RDKV_EUNSUPPORTED = -2
 RDKV_ELAUNCH = -3
 RDKV_EWORKSPACE = -4
+RDKV_EWAIT = -5
 
 DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 
@@ -56,7 +57,10 @@ SIGNATURES = {
     "rdkv_dequant_f16": (I, [P, L, I, I, P, P, I, P, L, P]),
     "rdkv_unpack_layer_k": (I, [P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, P, I, I, I, I, I, I, I, L, I, P, P]),
     "rdkv_unpack_layer_k_checked": (I, [P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, P, I, I, I, I, I, I, I, L, I, P, P, P]),
+    "rdkv_unpack_layer_k_words": (I, [P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, P, I, I, I, I, I, I, I, L, I, P, P,
+                                      ctypes.c_uint32, P]),
     "rdkv_unpack_layer_v": (I, [P, L, P, L, P, L, P, P, L, P, I, I, I, L, P, L, I, I, I, P, P]),
+    "rdkv_unpack_layer_v_words": (I, [P, L, P, L, P, L, P, P, L, P, I, I, I, L, P, L, I, I, I, P, P, P, ctypes.c_uint32, P]),
     "rdkv_k_qk_dot": (I, [P, I, L, I, I, P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, I, I, L, P, L, P]),
     "rdkv_softmax_rows": (I, [P, L, P, L, L, P, L, L, P, L, P, L, I, P]),
     "rdkv_softmax_rows_workspace_bytes": (L, [I]),
@@ -101,7 +105,7 @@ SIGNATURES = {
     "rdkv_pack_layer_plan_ints": (L, [I, L]),
     "rdkv_pack_layer_plan": (I, [P, I, L, P, I, L, I, L, I, P, L, P, L, P, P]),
     "rdkv_pack_layer_plan_start": (I, [P, I, L, P, I, L, I, L, I, P, L, P, L, P, P, I, P, ctypes.c_uint32, P]),
-    "rdkv_pack_layer_plan_wait": (I, [P, I, ctypes.c_uint32, P, L]),
+    "rdkv_host_words_wait": (I, [P, L, ctypes.c_uint32, P, L]),
     "rdkv_pack_layers_k_minmax": (I, [P, P, I, I, L, I, P, L, P, P, L, P]),
     "rdkv_pack_layer_tables": (I, [P, I, L, I, I, I, P, P, I, I, I, I, L, I, P, L, P, L, I, L,
                                    P, P, P, P, P, P, P, P, P, P, P, P]),
@@ -266,6 +270,54 @@ def upload(dev: torch.device, *arrays) -> list:
     ev.record(torch.cuda.current_stream(dev))
     slot[1] = ev
     return [d[o:o + max(int(a.nbytes), 0)] for a, o in zip(arrays, offs)]
+
+
+class HostWords:
+    """Pinned words that launches fill for the host thread that waits for them (``rdkv_host_words_wait``), and the tag
+    of the call.  Without a copy and a wait for the stream, what is launched behind them runs while the host goes
+    on.  A word holds what its launch knew when it wrote it, not that the launch has ended."""
+    WAIT_US = 100_000          # behind longer work than this the stream's own wait takes over
+
+    def __init__(self, size: int):
+        with torch.inference_mode(False):      # (written outside the mode it may be made in)
+            self.words = torch.zeros(size, dtype=torch.int64, pin_memory=True)
+        self.size, self.tag, self.used, self.pending = size, 0, 0, False
+        self.ptr = self.words.data_ptr()
+
+    def take(self, n: int) -> int:
+        """The address of the next ``n`` words."""
+        at = self.used
+        assert at + n <= self.size
+        self.used = at + n
+        return self.ptr + 8 * at
+
+    def read(self, dev: torch.device) -> list:
+        """The values of all words taken, in order."""
+        lib, values = load(), (ctypes.c_int32 * max(self.used, 1))()
+        rc = lib.rdkv_host_words_wait(self.ptr, self.used, self.tag, values, self.WAIT_US)
+        if rc == RDKV_EWAIT:
+            torch.cuda.current_stream(dev).synchronize()
+            rc = lib.rdkv_host_words_wait(self.ptr, self.used, self.tag, values, 0)
+        check(rc)
+        self.pending = False
+        return values[:self.used]
+
+
+_host_words: dict = {}         # (device, host thread) -> its words
+_retired_words: list = []      # kept: a launch whose call ended before it was read may still write to them
+
+
+def host_words(dev: torch.device, n: int) -> HostWords:
+    """Words for one call, ``n`` of them to take, until the next call by the same thread on the device."""
+    import threading
+    key = (dev.index, threading.get_ident())
+    w = _host_words.get(key)
+    if w is None or w.size < n or w.pending:
+        if w is not None:
+            _retired_words.append(w)
+        w = _host_words[key] = HostWords(max(4096, 1 << (max(n, 1) - 1).bit_length()))
+    w.tag, w.used, w.pending = w.tag % 0xFFFFFFFF + 1, 0, True            # (never 0, what fresh words hold)
+    return w
 
 
 _pinned_reads: dict = {}

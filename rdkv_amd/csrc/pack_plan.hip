@@ -5,8 +5,6 @@
 // shapes of the packed tensors) and no per-head loop.
 #include "rdkv_common.h"
 
-#include <chrono>
-
 namespace {
 
 constexpr int kPlanThreads = 1024;
@@ -159,8 +157,7 @@ plan_scatter_kernel(const void *__restrict__ v_bits, int vb_es, int64_t vb_strid
     // the head's twelve numbers to the host, each word with the call's tag: whole whenever its tag is there
     if (host_words && tid < 12) {
       const int v = tid < 6 ? red[tid] : info[8 * h + tid - 4];
-      __hip_atomic_store(host_words + 12 * (int64_t)h + tid, ((uint64_t)tag << 32) | (uint32_t)v, __ATOMIC_RELAXED,
-                         __HIP_MEMORY_SCOPE_SYSTEM);
+      rdkv_host_word(host_words, 12 * (int64_t)h + tid, tag, v);
     }
   }
 }
@@ -317,29 +314,6 @@ RDKV_API int rdkv_pack_layer_plan(const void *v_bits, int vb_elem_size, int64_t 
                                   int64_t rank3_stride_h, int32_t *plan, void *stream) {
   return rdkv_pack_layer_plan_start(v_bits, vb_elem_size, vb_stride_h, k_bits, kb_elem_size, kb_stride_h, H_kv, T, D, order,
                                     order_stride_h, rank3, rank3_stride_h, plan, nullptr, 0, nullptr, 0, stream);
-}
-
-RDKV_API int rdkv_pack_layer_plan_wait(const uint64_t *host_words, int n_heads, uint32_t tag, int32_t *plan, int64_t wait_us) {
-  RDKV_REQUIRE(host_words && plan && n_heads >= 0, "rdkv_pack_layer_plan_wait: bad arguments");
-  const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(wait_us);
-  for (int64_t i = 0; i < 12 * (int64_t)n_heads; ++i) {
-    const int64_t h = i / 12, k = i % 12;
-    for (int spins = 0;; ++spins) {
-      const uint64_t w = __atomic_load_n(host_words + i, __ATOMIC_ACQUIRE);
-      if ((uint32_t)(w >> 32) == tag) {
-        plan[k < 4 ? 4 * h + k : 4 * (int64_t)n_heads + 8 * h + (k - 4)] = (int32_t)(uint32_t)w;
-        break;
-      }
-      if ((spins & 255) == 255 && std::chrono::steady_clock::now() > until) {
-        rdkv_set_error("rdkv_pack_layer_plan_wait: not there after %lld us", (long long)wait_us);
-        return RDKV_EWAIT;
-      }
-#if defined(__x86_64__)
-      __builtin_ia32_pause();
-#endif
-    }
-  }
-  return RDKV_OK;
 }
 
 RDKV_API int rdkv_pack_layer_tables(const void *k_bits, int kb_elem_size, int64_t kb_stride_h, int H_kv, int D,

@@ -42,6 +42,12 @@ void rdkv_layer_k_minmax_init(float *minmax_ws, int H_kv, int D, hipStream_t s);
 
 #define RDKV_WAVE 64
 
+// A number to the host by the launch itself: word i of pinned host memory, with the call's tag in the upper half,
+// so that a word is whole whenever its tag is there and no order among the words matters (rdkv_host_words_wait).
+__device__ __forceinline__ void rdkv_host_word(uint64_t *words, int64_t i, uint32_t tag, int32_t v) {
+  __hip_atomic_store(words + i, ((uint64_t)tag << 32) | (uint32_t)v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __device__ __forceinline__ float rdkv_h2f(uint16_t bits) {
   return __half2float(__ushort_as_half(bits));
 }

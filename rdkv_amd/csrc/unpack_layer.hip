@@ -3,6 +3,9 @@
 // obkv_accel/packing.py:581-709, 1427-1444, trizone_decompress.py:91-182); here the channel scatter
 // of K, the class walk of V, the zero rows of the stripe and the fp16-kept rows are part of the
 // same pass, so nothing is dequantized into a temporary and copied again.
+// The per-head counts that the host checks leave the launches as words in host memory when their first workgroup
+// starts (rdkv_host_word): two layers of 16k / 31k / 64k tokens 107 / 121 / 261 us a call; with the
+// counts joined, copied and the stream waited for 174 / 174 / 313.
 #include "rdkv_common.h"
 
 namespace {
@@ -61,7 +64,7 @@ __global__ void __launch_bounds__(256)
 unpack_k_kernel(KSeg s2, KSeg s4, KSeg s8, const __half *__restrict__ scale, const __half *__restrict__ zp,
                 int64_t ks_sh, const int64_t *__restrict__ sort_idx, int64_t sort_sh, int sort_n,
                 const int32_t *__restrict__ counts, int c2, int c4, int c8, int64_t T, int D, int rows,
-                uint16_t *__restrict__ out, int32_t *__restrict__ check) {
+                uint16_t *__restrict__ out, int32_t *__restrict__ check, uint64_t *__restrict__ words, uint32_t tag) {
   extern __shared__ __attribute__((aligned(16))) uint8_t s_rows[];
   // per channel: where its code lies in a row (LDS offset | segment << 16 | shift << 18) and
   // its scale | zero point
@@ -81,10 +84,15 @@ unpack_k_kernel(KSeg s2, KSeg s4, KSeg s8, const __half *__restrict__ scale, con
     n8 = counts[3 * h + 2];
   }
   // (counts of a tensor that was overwritten must not lead outside the rows; the host reports them)
-  if (check && blockIdx.x == 0 && blockIdx.z == 0 && tid == 0) {
-    check[4 * h] = n2;
-    check[4 * h + 1] = n4;
-    check[4 * h + 2] = n8;
+  const bool reports = (check || words) && blockIdx.x == 0 && blockIdx.z == 0;
+  auto report = [&](int i, int v) {
+    if (check) check[4 * h + i] = v;
+    if (words) rdkv_host_word(words, 4 * (int64_t)h + i, tag, v);
+  };
+  if (reports && tid == 0) {
+    report(0, n2);
+    report(1, n4);
+    report(2, n8);
   }
   n2 = min(max(n2, 0), n2p);
   n4 = min(max(n4, 0), n4p);
@@ -110,9 +118,9 @@ unpack_k_kernel(KSeg s2, KSeg s4, KSeg s8, const __half *__restrict__ scale, con
     whole = whole && whole_zp(__half2float(zz));
   }
   whole = __syncthreads_and(whole);
-  if (check && blockIdx.x == 0 && blockIdx.z == 0) {
+  if (reports) {
     outside = __syncthreads_or(outside);
-    if (tid == 0) check[4 * h + 3] = outside ? 1 : 0;
+    if (tid == 0) report(3, outside ? 1 : 0);
   }
   const int oct = tid & 15, c0 = 8 * oct;
   int at[8], step[8], seg[8], shift[8], width[8];
@@ -208,10 +216,12 @@ unpack_v_kernel(const uint8_t *__restrict__ V2, int64_t v2_sh, const uint8_t *__
                 const uint8_t *__restrict__ V8, int64_t v8_sh, const __half *__restrict__ scale,
                 const __half *__restrict__ zp, int64_t s_sh, const int32_t *__restrict__ counts, int m2, int m4, int m8,
                 int64_t max_tv, const uint16_t *__restrict__ V16, int64_t v16_sh, int n16, int D,
-                uint16_t *__restrict__ out) {
+                uint16_t *__restrict__ out, const int32_t *__restrict__ totals, uint64_t *__restrict__ words, uint32_t tag) {
   constexpr int kTok = 4;
   const int h = blockIdx.y, c0 = blockIdx.z * kChan + 8 * (threadIdx.x & 15);
   const int64_t T = max_tv + n16;
+  if (words && blockIdx.x == 0 && blockIdx.z == 0 && threadIdx.x < 4)
+    rdkv_host_word(words, 4 * (int64_t)h + threadIdx.x, tag, threadIdx.x < 3 ? counts[3 * h + threadIdx.x] : totals[h]);
   // (clamped as above; a head never has more rows than the stripe)
   const int64_t e2 = min((int64_t)min(max(counts[3 * h], 0), m2), max_tv);
   const int64_t e4 = min(e2 + min(max(counts[3 * h + 1], 0), m4), max_tv);
@@ -293,7 +303,7 @@ static int unpack_layer_k(const uint8_t *K2, int64_t k2_stride_h, int64_t k2_str
                           int64_t k8_stride_t, const void *scale_f16, const void *zp_f16, int64_t ks_stride_h,
                           const int64_t *sort_idx, int64_t sort_stride_h, int sort_n, const int32_t *counts, int n2,
                           int n4, int n8, int n2p, int n4p, int n8w, int H_kv, int64_t T, int D, void *out_f16,
-                          int32_t *check, void *stream) {
+                          int32_t *check, uint64_t *words, uint32_t tag, void *stream) {
   RDKV_REQUIRE(H_kv >= 1 && H_kv <= 65535 && T >= 0 && D >= 1 && D <= 65535 * kChan, "rdkv_unpack_layer_k: bad shape");
   RDKV_REQUIRE(n2p >= 0 && n2p % 4 == 0 && n4p >= 0 && n4p % 2 == 0 && n8w >= 0 && sort_n >= 0,
                "rdkv_unpack_layer_k: bad segment widths %d/%d/%d", n2p, n4p, n8w);
@@ -317,7 +327,7 @@ static int unpack_layer_k(const uint8_t *K2, int64_t k2_stride_h, int64_t k2_str
   dim3 g((unsigned)per_head, H_kv, chunks);
   hipLaunchKernelGGL(dense ? unpack_k_kernel<true> : unpack_k_kernel<false>, g, dim3(256), lds, (hipStream_t)stream, s2, s4,
                      s8, (const __half *)scale_f16, (const __half *)zp_f16, ks_stride_h, sort_idx, sort_stride_h, sort_n,
-                     counts, n2, n4, n8, T, D, rows, (uint16_t *)out_f16, check);
+                     counts, n2, n4, n8, T, D, rows, (uint16_t *)out_f16, check, words, tag);
   RDKV_CHECK_LAUNCH("rdkv_unpack_layer_k");
   return RDKV_OK;
 }
@@ -330,7 +340,7 @@ RDKV_API int rdkv_unpack_layer_k(const uint8_t *K2, int64_t k2_stride_h, int64_t
                                  void *out_f16, void *stream) {
   return unpack_layer_k(K2, k2_stride_h, k2_stride_t, K4, k4_stride_h, k4_stride_t, K8, k8_stride_h, k8_stride_t, scale_f16,
                         zp_f16, ks_stride_h, sort_idx, sort_stride_h, sort_n, counts, n2, n4, n8, n2p, n4p, n8w, H_kv, T, D,
-                        out_f16, nullptr, stream);
+                        out_f16, nullptr, nullptr, 0, stream);
 }
 
 RDKV_API int rdkv_unpack_layer_k_checked(
@@ -342,14 +352,26 @@ RDKV_API int rdkv_unpack_layer_k_checked(
   RDKV_REQUIRE(check && T > 0, "rdkv_unpack_layer_k_checked: nothing to check into or no rows");
   return unpack_layer_k(K2, k2_stride_h, k2_stride_t, K4, k4_stride_h, k4_stride_t, K8, k8_stride_h, k8_stride_t, scale_f16,
                         zp_f16, ks_stride_h, sort_idx, sort_stride_h, sort_n, counts, n2, n4, n8, n2p, n4p, n8w, H_kv, T, D,
-                        out_f16, check, stream);
+                        out_f16, check, nullptr, 0, stream);
 }
 
-RDKV_API int rdkv_unpack_layer_v(const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h,
-                                 const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
-                                 int64_t s_stride_h, const int32_t *counts, int m2, int m4, int m8, int64_t max_tv,
-                                 const void *V16_f16, int64_t v16_stride_h, int n16, int H_kv, int D, void *out_f16,
-                                 void *stream) {
+RDKV_API int rdkv_unpack_layer_k_words(
+    const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t, const uint8_t *K4, int64_t k4_stride_h,
+    int64_t k4_stride_t, const uint8_t *K8, int64_t k8_stride_h, int64_t k8_stride_t, const void *scale_f16,
+    const void *zp_f16, int64_t ks_stride_h, const int64_t *sort_idx, int64_t sort_stride_h, int sort_n,
+    const int32_t *counts, int n2, int n4, int n8, int n2p, int n4p, int n8w, int H_kv, int64_t T, int D, void *out_f16,
+    uint64_t *words, uint32_t tag, void *stream) {
+  RDKV_REQUIRE(words && T > 0, "rdkv_unpack_layer_k_words: no words or no rows");
+  return unpack_layer_k(K2, k2_stride_h, k2_stride_t, K4, k4_stride_h, k4_stride_t, K8, k8_stride_h, k8_stride_t, scale_f16,
+                        zp_f16, ks_stride_h, sort_idx, sort_stride_h, sort_n, counts, n2, n4, n8, n2p, n4p, n8w, H_kv, T, D,
+                        out_f16, nullptr, words, tag, stream);
+}
+
+static int unpack_layer_v(const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h,
+                          const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
+                          int64_t s_stride_h, const int32_t *counts, int m2, int m4, int m8, int64_t max_tv,
+                          const void *V16_f16, int64_t v16_stride_h, int n16, int H_kv, int D, void *out_f16,
+                          const int32_t *totals, uint64_t *words, uint32_t tag, void *stream) {
   RDKV_REQUIRE(H_kv >= 1 && H_kv <= 65535 && max_tv >= 0 && n16 >= 0 && D >= 1 && D <= 65535 * kChan,
                "rdkv_unpack_layer_v: bad shape");
   RDKV_REQUIRE((!V2 || m2 <= 0 || D % 4 == 0) && (!V4 || m4 <= 0 || D % 2 == 0),
@@ -373,7 +395,26 @@ RDKV_API int rdkv_unpack_layer_v(const uint8_t *V2, int64_t v2_stride_h, const u
   hipLaunchKernelGGL(wide ? unpack_v_kernel<true> : unpack_v_kernel<false>, g, dim3(256), 0, (hipStream_t)stream, V2,
                      v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, (const __half *)scale_f16, (const __half *)zp_f16,
                      s_stride_h, counts, m2, m4, m8, max_tv, (const uint16_t *)V16_f16, v16_stride_h, n16, D,
-                     (uint16_t *)out_f16);
+                     (uint16_t *)out_f16, totals, words, tag);
   RDKV_CHECK_LAUNCH("rdkv_unpack_layer_v");
   return RDKV_OK;
+}
+
+RDKV_API int rdkv_unpack_layer_v(const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h,
+                                 const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
+                                 int64_t s_stride_h, const int32_t *counts, int m2, int m4, int m8, int64_t max_tv,
+                                 const void *V16_f16, int64_t v16_stride_h, int n16, int H_kv, int D, void *out_f16,
+                                 void *stream) {
+  return unpack_layer_v(V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, scale_f16, zp_f16, s_stride_h, counts, m2, m4, m8,
+                        max_tv, V16_f16, v16_stride_h, n16, H_kv, D, out_f16, nullptr, nullptr, 0, stream);
+}
+
+RDKV_API int rdkv_unpack_layer_v_words(const uint8_t *V2, int64_t v2_stride_h, const uint8_t *V4, int64_t v4_stride_h,
+                                       const uint8_t *V8, int64_t v8_stride_h, const void *scale_f16, const void *zp_f16,
+                                       int64_t s_stride_h, const int32_t *counts, int m2, int m4, int m8, int64_t max_tv,
+                                       const void *V16_f16, int64_t v16_stride_h, int n16, int H_kv, int D, void *out_f16,
+                                       const int32_t *totals, uint64_t *words, uint32_t tag, void *stream) {
+  RDKV_REQUIRE(words && totals && max_tv + n16 > 0, "rdkv_unpack_layer_v_words: no words, no totals or no rows");
+  return unpack_layer_v(V2, v2_stride_h, V4, v4_stride_h, V8, v8_stride_h, scale_f16, zp_f16, s_stride_h, counts, m2, m4, m8,
+                        max_tv, V16_f16, v16_stride_h, n16, H_kv, D, out_f16, totals, words, tag, stream);
 }

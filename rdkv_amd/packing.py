@@ -14,7 +14,6 @@ from dataclasses import dataclass
 from typing import List, Optional, Sequence, Tuple
 
 import ctypes
-import threading
 
 import torch
 from torch import Tensor
@@ -350,10 +349,10 @@ def _int32_on(dev: torch.device, t: Tensor) -> Tensor:
     return t.to(device=dev, dtype=torch.int32).contiguous()
 
 
-def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional[Tensor]]:
+def _unpack_k_enqueue(packed: "PackedKVLayer", D: int, words=None) -> Tuple[Tensor, Optional[Tensor]]:
     """``unpack_k_mixed`` as one launch: the dense rows and, of a per-head layer, what the launch found of every
     head: the class counts and whether a kept channel is outside the head dimension, yet to be checked
-    (``_check_k_counts``).  A shared layer's call reads nothing back: its counts are the host's, and kept
+    (``_check_k_counts``) - a device tensor, or, into the next 4 H of ``words``, H.  A shared layer's call reads nothing back: its counts are the host's, and kept
     channels outside the head dimension are left out."""
     if packed.K_ch_scale is None:
         raise ValueError("unpack_k_mixed: K_ch_scale missing")
@@ -414,6 +413,9 @@ def _unpack_k_enqueue(packed: "PackedKVLayer", D: int) -> Tuple[Tensor, Optional
         return out, None
     if T == 0:
         return out, torch.nn.functional.pad(counts, (0, 1))
+    if words is not None:
+        _lib.check(_lib.load().rdkv_unpack_layer_k_words(*args, words.take(4 * H), words.tag, _lib.stream_of(dev)))
+        return out, H
     check = torch.empty(H, 4, dtype=torch.int32, device=dev)
     _lib.check(_lib.load().rdkv_unpack_layer_k_checked(*args, check.data_ptr(), _lib.stream_of(dev)))
     return out, check
@@ -720,50 +722,6 @@ def _pad_and_stack_per_head_layers(
 
 _PLAN_INT_DTYPES = (torch.uint8, torch.int16, torch.int32, torch.int64)
 
-_pinned_ints: dict = {}
-
-
-def _read_ints(t: Tensor, n: int) -> list:
-    """The first ``n`` int32 of a device tensor as a Python list, through a pinned host buffer
-    that is kept (a pageable copy allocates and stages on every call)."""
-    key = (t.device.index, max(1024, 1 << (n - 1).bit_length()), threading.get_ident())   # one buffer per host thread
-    buf = _pinned_ints.get(key)
-    if buf is None:
-        with torch.inference_mode(False):      # a kept buffer must stay writable outside the mode it was made in
-            buf = _pinned_ints[key] = torch.empty(key[1], dtype=torch.int32, pin_memory=True)
-    buf[:n].copy_(t[:n], non_blocking=True)
-    torch.cuda.current_stream(t.device).synchronize()
-    return buf[:n].tolist()
-
-
-class _PlanWords:
-    """Pinned words that a planning launch fills for the host thread that waits for them, twelve a head, and
-    the tag of the last call.  Without a copy and a wait for the stream, what is launched behind the plan runs
-    while the host reads and sizes the outputs."""
-    WAIT_US = 100_000          # behind longer work than this the stream's own wait takes over
-
-    def __init__(self, heads: int):
-        with torch.inference_mode(False):      # (written outside the mode it may be made in)
-            self.words = torch.zeros(12 * heads, dtype=torch.int64, pin_memory=True)
-        self.heads, self.tag = heads, 0
-        self.ptr = self.words.data_ptr()
-
-
-_plan_words: dict = {}         # (device, host thread) -> its words
-_outgrown_words: list = []     # kept: a launch whose caller was interrupted may still write to them
-
-
-def _words_for(dev: torch.device, heads: int) -> _PlanWords:
-    key = (dev.index, threading.get_ident())
-    w = _plan_words.get(key)
-    if w is None or w.heads < heads:
-        if w is not None:
-            _outgrown_words.append(w)
-        w = _plan_words[key] = _PlanWords(max(256, 1 << (heads - 1).bit_length()))
-    w.tag = w.tag % 0xFFFFFFFF + 1             # (never 0, what fresh words hold)
-    return w
-
-
 # Tokens from which a layer's K min / max are launched ahead of the host's read of the plan.  Below, the host is
 # the longer side and their own call costs 3 .. 7 us of it.  Us a call ahead / behind, 8 KV heads: selection and packing
 # of 16k tokens 177 / 176, 31k 178 / 178, 64k 200 / 222, 100k 272 / 304; four layers to the streaming format 4k
@@ -801,13 +759,13 @@ def _plan_layers(v_bits: Tensor, k_bits: Tensor, dev, Ks: Sequence[Tensor] = (),
     plan = torch.empty(lib.rdkv_pack_layer_plan_ints(N, T), dtype=torch.int32, device=dev)
     D = int(kb.shape[1])
     mm = torch.empty(N * minmax_per_head, dtype=torch.float32, device=dev) if len(Ks) else None
-    # (a capture cannot wait for its launches: the stream's own wait says so)
-    words = None if torch.cuda.is_current_stream_capturing() else _words_for(plan.device, N)
+    if torch.cuda.is_current_stream_capturing():      # (a capture cannot wait for its launches)
+        torch.cuda.current_stream(dev).synchronize()
+    words = _lib.host_words(plan.device, 12 * N)
     _lib.check(lib.rdkv_pack_layer_plan_start(
         vb.data_ptr(), vb.element_size(), vb.stride(0), kb.data_ptr(), kb.element_size(), kb.stride(0), N, T, D,
         order.data_ptr(), order.stride(0), rank3.data_ptr(), rank3.stride(0), plan.data_ptr(),
-        mm.data_ptr() if mm is not None else None, minmax_per_head, words.ptr if words is not None else None,
-        words.tag if words is not None else 0, _lib.stream_of(dev)))
+        mm.data_ptr() if mm is not None else None, minmax_per_head, words.take(12 * N), words.tag, _lib.stream_of(dev)))
     if mm is not None:
         ptrs = (ctypes.c_void_p * len(Ks))(*[K.data_ptr() for K in Ks])
         strides = (ctypes.c_int64 * (2 * len(Ks)))(*[s for K in Ks for s in (K.stride(1), K.stride(2))])
@@ -816,14 +774,9 @@ def _plan_layers(v_bits: Tensor, k_bits: Tensor, dev, Ks: Sequence[Tensor] = (),
                                                  plan.data_ptr(), mm.data_ptr(), H * minmax_per_head, _lib.stream_of(dev)))
     if meanwhile is not None:
         meanwhile()
-    # the one synchronization
-    numbers = (ctypes.c_int32 * (12 * N))()
-    if words is not None and lib.rdkv_pack_layer_plan_wait(words.ptr, N, words.tag, numbers, words.WAIT_US) == _lib.RDKV_OK:
-        plan_h = list(numbers)
-    else:
-        plan_h = _read_ints(plan, 12 * N)
-    counts_h = [plan_h[4 * h:4 * h + 4] for h in range(N)]
-    info_h = [plan_h[4 * N + 8 * h:4 * N + 8 * h + 8] for h in range(N)]
+    numbers = words.read(plan.device)                           # the one synchronization
+    counts_h = [numbers[12 * h:12 * h + 4] for h in range(N)]
+    info_h = [numbers[12 * h + 4:12 * h + 12] for h in range(N)]
     assert all(row[1] == 0 for row in info_h), "v_bits must be in {0,2,4,8,16}"
     assert all(row[5] == 0 for row in info_h), "k_bits must be in {0,2,4,8,16}"
     return order, rank3, plan, counts_h, info_h, kb, mm

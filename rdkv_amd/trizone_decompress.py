@@ -36,9 +36,10 @@ def _is_perhead_layout(pl: PackedKVLayer) -> bool:
     return pl.seg_bounds_per_head is not None
 
 
-def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int) -> Tuple[Tensor, Tensor, Tensor]:
-    """The stripe's dense V, ``zone_b`` rows behind it, in one launch; and the per-head counts on the device,
-    [H, 3] by class and [H] in all, yet to be checked (``_check_v_counts``)."""
+def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int, words=None) -> tuple:
+    """The stripe's dense V, ``zone_b`` rows behind it, in one launch; and the per-head counts, yet to be checked
+    (``_check_v_counts``): on the device, [H, 3] by class and [H] in all, or, as the launch read them into the
+    next 4 H of ``words``, H."""
     max_T_v = int(pl.T_eff)
     H_kv = pl.V_scale.shape[1]
     # everything the kernel indexes by head, class row and token, before it gets the addresses
@@ -71,10 +72,14 @@ def _unpack_v_enqueue(pl: PackedKVLayer, zone_b: Optional[Tensor], head_dim: int
     if zone_b is not None and not (zone_b.stride(3) == 1 and zone_b.stride(2) == head_dim):
         zone_b = zone_b.contiguous()
     (V2, v2h, m2), (V4, v4h, m4), (V8, v8h, m8) = segs
-    _lib.check(_lib.load().rdkv_unpack_layer_v(
-        _lib.ptr(V2), v2h, _lib.ptr(V4), v4h, _lib.ptr(V8), v8h, _lib.ptr(sc), _lib.ptr(zp), sc.stride(1),
-        counts.data_ptr(), m2, m4, m8, max_T_v, _lib.ptr(zone_b), zone_b.stride(1) if n16 else 0, n16, H_kv, head_dim,
-        _lib.ptr(out), _lib.stream_of(dev)))
+    args = (_lib.ptr(V2), v2h, _lib.ptr(V4), v4h, _lib.ptr(V8), v8h, _lib.ptr(sc), _lib.ptr(zp), sc.stride(1),
+            counts.data_ptr(), m2, m4, m8, max_T_v, _lib.ptr(zone_b), zone_b.stride(1) if n16 else 0, n16, H_kv, head_dim,
+            _lib.ptr(out))
+    if words is not None and max_T_v + n16 > 0:
+        _lib.check(_lib.load().rdkv_unpack_layer_v_words(*args, totals.data_ptr(), words.take(4 * H_kv), words.tag,
+                                                         _lib.stream_of(dev)))
+        return out, H_kv
+    _lib.check(_lib.load().rdkv_unpack_layer_v(*args, _lib.stream_of(dev)))
     return out, counts, totals
 
 
@@ -103,8 +108,28 @@ def _unpack_v_perhead(pl: PackedKVLayer, *, head_dim: int) -> Tensor:
     return out
 
 
-def _read_checks(unchecked) -> None:
-    """Calls every (check, layer, device tensors) with the tensors' values as lists: one read per device."""
+def _words_of(dev: torch.device, words: dict, heads: int):
+    """The words of this call on ``dev``, for launches over ``heads`` heads in all (K and V); None where the
+    counts come back as tensors (no device, a capture)."""
+    if dev.type != "cuda" or torch.cuda.is_current_stream_capturing():
+        return None
+    if dev not in words:
+        words[dev] = _lib.host_words(dev, 4 * heads), []
+    return words[dev][0]
+
+
+def _read_checks(unchecked, words: Optional[dict] = None) -> None:
+    """Calls every (check, layer, device tensors) with the tensors' values as lists: one read per device.
+    ``words``: by device, what its launches filled and (check, layer, heads) in the order they took theirs."""
+    for dev, (filled, entries) in (words or {}).items():
+        flat, at = filled.read(dev), 0
+        for check, pl, heads in entries:
+            rows = [flat[i:i + 4] for i in range(at, at + 4 * heads, 4)]
+            at += 4 * heads
+            if check is _check_v_counts:
+                check(pl, [row[:3] for row in rows], [row[3] for row in rows])
+            else:
+                check(pl, rows)
     by_device: dict = {}
     for entry in unchecked:
         by_device.setdefault(entry[2][0].device, []).append(entry)
@@ -129,9 +154,14 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
     past_kv: List[Tuple[Tensor, Tensor]] = []
     masks: List[Optional[Tensor]] = []
     unchecked = []        # (check, layer, per-head counts the launches below read)
+    words: dict = {}      # the same from launches that send them to the host
+    heads = sum(int(t.shape[1]) for pl in dual_cache.packed for t in (pl.K_ch_scale, pl.V_scale) if t is not None)
     for i, pl in enumerate(dual_cache.packed):
-        K_full, k_check = _unpack_k_enqueue(pl, head_dim)
-        if k_check is not None:
+        to = _words_of(pl.K_ch_scale.device, words, heads) if pl.K_ch_scale is not None else None
+        K_full, k_check = _unpack_k_enqueue(pl, head_dim, to)
+        if isinstance(k_check, int):
+            words[pl.K_ch_scale.device][1].append((_check_k_counts, pl, k_check))
+        elif k_check is not None:
             unchecked.append((_check_k_counts, pl, (k_check,)))
         zone_b = dual_cache.new_v_only[i] if i < len(dual_cache.new_v_only) else None
         if _is_perhead_layout(pl):
@@ -144,8 +174,12 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
             else:
                 joined = rows_b is not None and rows_b.dtype == torch.float16 and rows_b.shape[:2] == pl.V_scale.shape[:2] \
                     and rows_b.shape[3] == head_dim and rows_b.device == pl.V_scale.device
-                V_full, *v_counts = _unpack_v_enqueue(pl, rows_b if joined else None, head_dim)
-                unchecked.append((_check_v_counts, pl, v_counts))
+                V_full, *v_counts = _unpack_v_enqueue(pl, rows_b if joined else None, head_dim,
+                                                      _words_of(pl.V_scale.device, words, heads))
+                if isinstance(v_counts[0], int):
+                    words[pl.V_scale.device][1].append((_check_v_counts, pl, v_counts[0]))
+                else:
+                    unchecked.append((_check_v_counts, pl, v_counts))
                 if rows_b is not None and not joined:
                     V_full = torch.cat([V_full, rows_b], dim=2)
         else:
@@ -175,5 +209,5 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
                 masks.append(m4.contiguous())
             else:
                 masks.append(None)
-    _read_checks(unchecked)        # (behind the launches, which clamp what they follow)
+    _read_checks(unchecked, words)        # (behind the launches, which clamp what they follow)
     return (tuple(past_kv), masks) if return_masks else tuple(past_kv)
