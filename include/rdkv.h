@@ -333,6 +333,11 @@ int rdkv_tail_scores(const float *w, int64_t w_stride_row, int H_kv, int G, int 
  * int64, each may be NULL) and counts[0..n_counts-1] += 1 (device int32, n_counts <= 1024). */
 int rdkv_argmax_advance(const void *logits, int n, int dtype, int64_t *token, int64_t *counter_a,
                         int64_t *counter_b, int32_t *counts, int n_counts, void *stream);
+/* The same; the token also goes to the host by itself (rdkv_host_words_wait): word[0] = token with the tag
+ * tag_base + counter_a's new value (mod 2^32). */
+int rdkv_argmax_advance_word(const void *logits, int n, int dtype, int64_t *token, int64_t *counter_a,
+                             int64_t *counter_b, int32_t *counts, int n_counts, uint64_t *word, uint32_t tag_base,
+                             void *stream);
 
 /* fast_decode.py:1650-1656, 1786, 1797-1804, 1826: the projections of a decode step, each
  * F.linear on one activation row there.  y[n] = sum_k W[n,k] * x[k] (+ bias[n]); W [N, K] with

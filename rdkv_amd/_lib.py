@@ -98,6 +98,7 @@ SIGNATURES = {
     "rdkv_silu_mul": (I, [P, P, L, I, P, P]),
     "rdkv_tail_scores": (I, [P, L, I, I, I, I, I, P, L, P, L, P]),
     "rdkv_argmax_advance": (I, [P, I, I, P, P, P, P, I, P]),
+    "rdkv_argmax_advance_word": (I, [P, I, I, P, P, P, P, I, P, ctypes.c_uint32, P]),
     "rdkv_gemv": (I, [P, L, P, I, P, I, I, I, P, P]),
     "rdkv_gemv_norm": (I, [P, L, P, P, P, F, P, P, I, I, I, P, P]),
     "rdkv_gemv_silu": (I, [P, L, P, P, P, I, I, I, P, P]),
@@ -318,6 +319,39 @@ def host_words(dev: torch.device, n: int) -> HostWords:
         w = _host_words[key] = HostWords(max(4096, 1 << (max(n, 1) - 1).bit_length()))
     w.tag, w.used, w.pending = w.tag % 0xFFFFFFFF + 1, 0, True            # (never 0, what fresh words hold)
     return w
+
+
+class StepWord:
+    """The pinned word that every step of a decode loop fills with the token it chose
+    (``rdkv_argmax_advance_word``), tagged with the position the step moved on to."""
+
+    def __init__(self, ptr: int, tag_base: int):
+        self.ptr, self.tag_base, self.value = ptr, tag_base & 0xFFFFFFFF, ctypes.c_int32(0)
+
+    def read(self, position: int) -> Optional[int]:
+        """The token of the step that moved on to ``position``; None: behind longer work than a wait is for."""
+        rc = load().rdkv_host_words_wait(self.ptr, 1, (self.tag_base + position) & 0xFFFFFFFF,
+                                         ctypes.addressof(self.value), HostWords.WAIT_US)
+        return self.value.value if rc == RDKV_OK else None
+
+
+_step_words: dict = {}         # (device, host thread) -> [words, next, last tag of each]
+
+
+def step_word(dev: torch.device, steps: int, position: int) -> StepWord:
+    """A word for a loop of up to ``steps`` steps from ``position`` on: each of the thread's last 64 loops
+    has its own (the last step of a loop may still be running when the next one starts), no tag comes twice."""
+    import threading
+    key = (dev.index, threading.get_ident())
+    ring = _step_words.get(key)
+    if ring is None:
+        with torch.inference_mode(False):
+            ring = _step_words[key] = [torch.zeros(64, dtype=torch.int64, pin_memory=True), 0, [0] * 64]
+    words, slot, tags = ring
+    ring[1] = (slot + 1) % 64
+    first = tags[slot] + 1
+    tags[slot] = (first + steps) & 0x7FFFFFFF
+    return StepWord(words.data_ptr() + 8 * slot, first - position)
 
 
 _pinned_reads: dict = {}

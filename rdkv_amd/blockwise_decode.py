@@ -772,16 +772,20 @@ def greedy_decode_blockwise(*, model, dual_cache: TriZoneCache, next_token_logit
             delta = _silu_linear_row(gate, up, lw.down_proj_weight)
         hidden = _rms_norm(h, W.final_norm_weight, W.final_norm_eps, delta=delta, residual_out=h)
         logits = _linear_row(hidden, W.lm_head_weight)
-        _argmax_advance(logits, next_token, position_ids, write_row, n_tail)
+        _argmax_advance(logits, next_token, position_ids, write_row, n_tail, word)
 
-    position_ids.fill_(int(decode_position_start))
+    position = int(decode_position_start)
+    word = _lib.step_word(next_token.device, max_new_tokens, position)
+    position_ids.fill_(position)
     write_row.zero_()
     n_tail.fill_(1)
     graph = None                  # the step recorded for the current set of unit tables
     eager_steps = 0               # steps run eagerly since the tables last changed
     with torch.inference_mode():
         for step in range(max_new_tokens):
-            token_id = int(next_token.item())
+            token_id = word.read(position + step) if step else None
+            if token_id is None:
+                token_id = int(next_token.item())
             if token_id in eos_set:
                 break
             generated.append(token_id)

@@ -137,7 +137,7 @@ template <int dtype>
 __global__ void __launch_bounds__(1024)
 argmax_advance_kernel(const void *__restrict__ logits, int n, int64_t *__restrict__ token,
                       int64_t *__restrict__ counter_a, int64_t *__restrict__ counter_b,
-                      int32_t *__restrict__ counts, int n_counts) {
+                      int32_t *__restrict__ counts, int n_counts, uint64_t *__restrict__ word, uint32_t tag_base) {
   constexpr int EPP = dtype == RDKV_DTYPE_F32 ? 4 : 8;     // elements per 16-byte piece
   __shared__ float s_v[16];
   __shared__ int s_i[16];
@@ -188,7 +188,12 @@ argmax_advance_kernel(const void *__restrict__ logits, int n, int64_t *__restric
     for (int w = 1; w < 16; ++w)
       if (best_before(s_v[w], s_i[w], bv, bi)) { bv = s_v[w]; bi = s_i[w]; }
     token[0] = bi;
-    if (counter_a) counter_a[0] += 1;
+    if (counter_a) {
+      const int64_t a = counter_a[0] + 1;
+      counter_a[0] = a;
+      // the token to the host, tagged with the counter: a launch that a graph replays needs nothing from the host
+      if (word) rdkv_host_word(word, 0, tag_base + (uint32_t)a, bi);
+    }
     if (counter_b) counter_b[0] += 1;
   }
   if (tid < n_counts) counts[tid] += 1;
@@ -293,23 +298,30 @@ RDKV_API int rdkv_silu_mul(const void *gate, const void *up, int64_t n, int dtyp
   return RDKV_OK;
 }
 
-RDKV_API int rdkv_argmax_advance(const void *logits, int n, int dtype, int64_t *token, int64_t *counter_a,
-                                 int64_t *counter_b, int32_t *counts, int n_counts, void *stream) {
+RDKV_API int rdkv_argmax_advance_word(const void *logits, int n, int dtype, int64_t *token, int64_t *counter_a,
+                                      int64_t *counter_b, int32_t *counts, int n_counts, uint64_t *word, uint32_t tag_base,
+                                      void *stream) {
   const char *fn = "rdkv_argmax_advance";
   RDKV_REQUIRE(logits && token && n >= 1, "%s: needs logits, a token slot and n >= 1", fn);
   RDKV_REQUIRE(dtype >= 0 && dtype <= 2, "%s: unknown dtype %d", fn, dtype);
   RDKV_REQUIRE(((uintptr_t)logits % 16) == 0, "%s: logits must be 16-byte aligned", fn);
   RDKV_REQUIRE(n_counts >= 0 && n_counts <= 1024 && (n_counts == 0 || counts), "%s: bad counts", fn);
+  RDKV_REQUIRE(!word || counter_a, "%s: a host word is tagged with the first counter", fn);
   hipStream_t s = (hipStream_t)stream;
   if (dtype == RDKV_DTYPE_F32)
     hipLaunchKernelGGL(argmax_advance_kernel<RDKV_DTYPE_F32>, dim3(1), dim3(1024), 0, s, logits, n, token,
-                       counter_a, counter_b, counts, n_counts);
+                       counter_a, counter_b, counts, n_counts, word, tag_base);
   else if (dtype == RDKV_DTYPE_F16)
     hipLaunchKernelGGL(argmax_advance_kernel<RDKV_DTYPE_F16>, dim3(1), dim3(1024), 0, s, logits, n, token,
-                       counter_a, counter_b, counts, n_counts);
+                       counter_a, counter_b, counts, n_counts, word, tag_base);
   else
     hipLaunchKernelGGL(argmax_advance_kernel<RDKV_DTYPE_BF16>, dim3(1), dim3(1024), 0, s, logits, n, token,
-                       counter_a, counter_b, counts, n_counts);
+                       counter_a, counter_b, counts, n_counts, word, tag_base);
   RDKV_CHECK_LAUNCH(fn);
   return RDKV_OK;
+}
+
+RDKV_API int rdkv_argmax_advance(const void *logits, int n, int dtype, int64_t *token, int64_t *counter_a,
+                                 int64_t *counter_b, int32_t *counts, int n_counts, void *stream) {
+  return rdkv_argmax_advance_word(logits, n, dtype, token, counter_a, counter_b, counts, n_counts, nullptr, 0, stream);
 }

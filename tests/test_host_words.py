@@ -7,7 +7,7 @@ import threading
 import pytest
 import torch
 
-from rdkv_amd import _lib, packing, stream_cache, trizone_decompress as tz
+from rdkv_amd import _lib, fast_decode, packing, stream_cache, trizone_decompress as tz
 from tests.gpu_util import DEV, require_gpu
 
 gpu = pytest.mark.gpu
@@ -132,6 +132,43 @@ def test_dense_counts_by_words(monkeypatch, late):
     with pytest.raises(IndexError):
         tz.unpack_trizone_to_past_kv(cache(K_ch_sort_idx_per_head=pl.K_ch_sort_idx_per_head + 100), head_dim=128)
     assert len(tz.unpack_trizone_to_past_kv(cache(), head_dim=128)) == n
+
+
+@gpu
+@pytest.mark.parametrize("position", [0, 41, (1 << 32) - 2])
+def test_token_words(position):
+    """Eager steps and a replayed graph leave each step's token under the position it moved on to."""
+    require_gpu()
+    logits = torch.randn(3, 1000, device=DEV).half()
+    row = logits[0].clone()
+    token = torch.zeros(1, 1, dtype=torch.long, device=DEV)
+    pos = torch.full((1, 1), position, dtype=torch.long, device=DEV)
+    for _ in range(2):
+        pos.fill_(position)
+        word = _lib.step_word(token.device, 5, position)
+        fast_decode._argmax_advance(row, token, pos, word=word)
+        assert word.read(position + 1) == int(logits[0].argmax()) == int(token)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            fast_decode._argmax_advance(row, token, pos, word=word)
+        for step in range(1, 4):
+            row.copy_(logits[step % 3])
+            graph.replay()
+            assert word.read(position + step + 1) == int(logits[step % 3].argmax()) == int(token)
+        row.copy_(logits[0])
+
+
+def test_words_of_loops_never_share_a_tag(monkeypatch):
+    """The ring's words come round with other tags; two loops in a row have words of their own."""
+    dev = torch.device("cuda", 63)
+    monkeypatch.setattr(_lib, "_step_words", {(63, threading.get_ident()): [torch.zeros(64, dtype=torch.int64), 0, [0] * 64]})
+    seen = set()
+    for loop in range(200):
+        steps, position = 1 + loop % 7, 1000 * loop
+        word = _lib.step_word(dev, steps, position)
+        tags = {(word.ptr, (word.tag_base + position + k) & 0xFFFFFFFF) for k in range(1, steps + 1)}
+        assert len(tags) == steps and not tags & seen and all(tag for _, tag in tags)
+        seen |= tags
 
 
 def _same(a, b):
