@@ -647,6 +647,19 @@ int rdkv_decode_fused_merge_zone_c_append(const RdkvUnit *units, const RdkvUnit 
                                           void *q_rotated_out, int64_t q_rotated_stride_row,
                                           const RdkvTailScores *tail_scores,
                                           void *workspace, int64_t workspace_bytes, void *stream);
+/* rdkv_decode_fused_partials, then rdkv_decode_fused_merge_zone_c_append (row_dev NULL: rdkv_decode_fused_merge_zone_c,
+ * capacity its n_new), in one call. */
+int rdkv_decode_fused_zone_c(const RdkvUnit *units, const RdkvUnit *units_host, int n_units, const RdkvWork *work,
+                             int n_work, const int32_t *groups, int n_groups, int max_row_dwords, int G,
+                             const void *q, int q_dtype, int64_t q_stride_row, const void *rope_cos,
+                             const void *rope_sin, int rope_dtype, float *k_new, float *v_new,
+                             int64_t new_stride_unit, int64_t new_stride_tok, int64_t capacity,
+                             const int32_t *n_new_per_unit, const void *k_step, int64_t k_stride_h,
+                             const void *v_step, int64_t v_stride_h, int kv_dtype, const int64_t *row_dev, float *out,
+                             int64_t out_stride_row, float *lse, float *zone_c_weights,
+                             int64_t zone_c_weights_stride_row, void *q_rotated_out, int64_t q_rotated_stride_row,
+                             const RdkvTailScores *tail_scores, void *workspace, int64_t workspace_bytes,
+                             void *stream);
 
 /* Planning for rdkv_pack_layer_per_head on the device (what the reference derives on the host:
  * packing.py:1417-1431 stable token sort by width, :241-294 channel classes).  v_bits [H_kv, T]

@@ -92,6 +92,8 @@ SIGNATURES = {
     "rdkv_decode_fused_merge_zone_c": (I, [P, P, I, I, I, P, I, L, P, P, I, P, P, L, L, I, P, P, L, P, P, L, P, L, P]),
     "rdkv_decode_fused_merge_zone_c_append": (I, [P, P, I, I, I, P, I, L, P, P, I, P, P, L, L, L, P, P, L, P, L, I, P,
                                                   P, L, P, P, L, P, L, P, P, L, P]),
+    "rdkv_decode_fused_zone_c": (I, [P, P, I, P, I, P, I, I, I, P, I, L, P, P, I, P, P, L, L, L, P, P, L, P, L, I, P, P, L, P,
+                                     P, L, P, L, P, P, L, P]),
     "rdkv_rope": (I, [P, L, I, P, L, I, I, I, P, P, I, P]),
     "rdkv_add_rms_norm": (I, [P, L, P, L, P, I, F, I, I, I, P, L, P, L, P]),
     "rdkv_rope_append_kv": (I, [P, L, P, L, I, I, I, P, P, I, P, L, L, P, L, P]),
@@ -231,6 +233,13 @@ def workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
         buf = torch.empty(max(int(nbytes), grown, 1 << 20), dtype=torch.uint8, device=dev)
         _workspaces[key] = buf
     return buf
+
+
+def stream_workspace(dev: torch.device):
+    """The current stream's handle and its scratch buffer as large as it is (``workspace`` grows it)."""
+    stream = stream_of(dev)
+    buf = _workspaces.get((dev.index, stream))
+    return stream, workspace(dev, 0) if buf is None else buf
 
 
 # ---- small host <-> device transfers that do not stall the host ---------------------------------

@@ -1785,6 +1785,37 @@ RDKV_API int rdkv_decode_fused_merge_zone_c_append(
                              workspace_bytes, ap, q_rotated_out, q_rotated_stride_row, tail, stream);
 }
 
+// The streaming launch and the merge launch in one call: what a layer of a decode loop pays on the host for two
+// (conversions of 55 arguments, one workspace lookup, one check of the result) it pays once.
+RDKV_API int rdkv_decode_fused_zone_c(
+    const RdkvUnit *units, const RdkvUnit *units_host, int n_units, const RdkvWork *work, int n_work, const int32_t *groups,
+    int n_groups, int max_row_dwords, int G, const void *q, int q_dtype, int64_t q_stride_row, const void *rope_cos,
+    const void *rope_sin, int rope_dtype, float *k_new, float *v_new, int64_t new_stride_unit, int64_t new_stride_tok,
+    int64_t capacity, const int32_t *n_new_per_unit, const void *k_step, int64_t k_stride_h, const void *v_step,
+    int64_t v_stride_h, int kv_dtype, const int64_t *row_dev, float *out, int64_t out_stride_row, float *lse,
+    float *zone_c_weights, int64_t zone_c_weights_stride_row, void *q_rotated_out, int64_t q_rotated_stride_row,
+    const RdkvTailScores *tail_scores, void *workspace, int64_t workspace_bytes, void *stream) {
+  if (workspace_bytes < rdkv_decode_fused_workspace_bytes(n_work, G)) {
+    rdkv_set_error("rdkv_decode_fused_zone_c: workspace of %lld bytes required",
+                   (long long)rdkv_decode_fused_workspace_bytes(n_work, G));
+    return RDKV_EWORKSPACE;
+  }
+  const int rc = rdkv_decode_fused_partials(nullptr, units, n_units, work, n_work, groups, n_groups, max_row_dwords, q, q_dtype,
+                                            q_stride_row, G, rope_cos, rope_sin, rope_dtype, workspace, workspace_bytes,
+                                            stream);
+  if (rc != RDKV_OK) return rc;
+  if (row_dev)
+    return rdkv_decode_fused_merge_zone_c_append(
+        units, units_host, n_units, n_work, G, q, q_dtype, q_stride_row, rope_cos, rope_sin, rope_dtype, k_new, v_new,
+        new_stride_unit, new_stride_tok, capacity, n_new_per_unit, k_step, k_stride_h, v_step, v_stride_h, kv_dtype, row_dev,
+        out, out_stride_row, lse, zone_c_weights, zone_c_weights_stride_row, q_rotated_out, q_rotated_stride_row, tail_scores,
+        workspace, workspace_bytes, stream);
+  return rdkv_decode_fused_merge_zone_c(units, units_host, n_units, n_work, G, q, q_dtype, q_stride_row, rope_cos, rope_sin,
+                                        rope_dtype, k_new, v_new, new_stride_unit, new_stride_tok, (int)capacity,
+                                        n_new_per_unit, out, out_stride_row, lse, zone_c_weights, zone_c_weights_stride_row,
+                                        workspace, workspace_bytes, stream);
+}
+
 // ---- rdkv_decode_fused for callers that cannot allocate ---------------------------------------
 // The partials of rdkv_decode_fused live in a fixed array in device memory instead of a workspace
 // the caller brings.  Each GPU the library runs on holds its own copy of the array (at its own

@@ -241,36 +241,36 @@ def trizone_attention(q_2d: torch.Tensor, sp: PackedKVLayer, V16: Optional[torch
     if q_2d.dtype not in _lib.DTYPE_CODE or q_2d.stride(1) != 1:
         q_2d = q_2d.float().contiguous()
     K_new, V_new = (_new_zone_rows(t, H_kv, n_new) for t in (K_new, V_new))
-    s_old = scores_buf[:, :T_old]
-    s_new = scores_buf[:, T_old:T_old + n_new]
     # zone C scores (:1730-1733), then mask + global softmax over [A | B | C] (:1743-1755), whose weights the
     # caller's buffer holds afterwards
-    mask = sp.softmax_mask if (T_old > 0 and sp.softmax_mask is not None) else None
+    mask = sp.softmax_mask if T_old > 0 else None
     row, mask_row = scores_buf.stride(0), mask.stride(0) if mask is not None else 0
-    scores = None
+    kn_sh, kn_st, _ = K_new.stride()
     if T_old > 0 and not k_kernel._DIAG_ENABLED:
-        args, _, keep = k_kernel._scores_args(q_2d, sp, T_old, s_old)
+        args, keep = k_kernel._scores_args(q_2d, sp, T_old)
         taken = -(-lib.rdkv_attn_scores_workspace_bytes(H_q) // 256) * 256
         ws = _lib.workspace(dev, taken + lib.rdkv_v_weighted_sum_workspace_bytes(H_q))
         pairs = ctypes.c_int(0)
         _lib.check(lib.rdkv_attn_scores(
-            *args, _lib.ptr(mask), mask_row, K_new.data_ptr(), K_new.stride(0), K_new.stride(1), n_new,
-            s_old.data_ptr(), row, ws.data_ptr(), taken, ctypes.addressof(pairs), _lib.stream_of(dev)))
+            *args, _lib.ptr(mask), mask_row, K_new.data_ptr(), kn_sh, kn_st, n_new, scores_buf.data_ptr(), row, ws.data_ptr(),
+            taken, ctypes.addressof(pairs), _lib.stream_of(dev)))
         del keep
         if pairs.value > 0:
-            scores = (ws, taken, pairs.value, int(caller_buf))
-    else:
+            _weighted_sum_with_new_zone(scores_buf, sp, out, V16, n_v16_per_head, T_v, None, V_new,
+                                        (ws, taken, pairs.value, int(caller_buf), T_old))
+            return out
+    s_old, s_new = scores_buf[:, :T_old], scores_buf[:, T_old:T_old + n_new]
+    if T_old == 0 or k_kernel._DIAG_ENABLED:
         if T_old > 0:
             k_mixed_qk_dot_into(q_2d, sp, T_old, s_old)
         ws = _lib.workspace(dev, lib.rdkv_softmax_rows_workspace_bytes(H_q))
         _lib.check(lib.rdkv_softmax_rows_new_keys(
-            _lib.ptr(s_old), row, _lib.ptr(mask), mask_row,
-            T_old, q_2d.data_ptr(), _lib.DTYPE_CODE[q_2d.dtype], q_2d.stride(0), K_new.data_ptr(), K_new.stride(0),
-            K_new.stride(1), n_new, _lib.ptr(s_old), row, s_new.data_ptr(), row, H_q, H_kv,
+            _lib.ptr(s_old), row, _lib.ptr(mask), mask_row, T_old, q_2d.data_ptr(), _lib.DTYPE_CODE[q_2d.dtype],
+            q_2d.stride(0), K_new.data_ptr(), kn_sh, kn_st, n_new, _lib.ptr(s_old), row, s_new.data_ptr(), row, H_q, H_kv,
             ws.data_ptr(), ws.numel(), _lib.stream_of(dev)))
     # values of all three zones (:1777-1784)
     _weighted_sum_with_new_zone(s_old if T_old > 0 else s_new, sp if T_old > 0 else None, out, V16, n_v16_per_head,
-                                T_v, s_new, V_new, scores)
+                                T_v, s_new, V_new)
     return out
 
 
@@ -278,7 +278,8 @@ def _new_zone_rows(t: torch.Tensor, H_kv: int, n_new: int) -> torch.Tensor:
     """Appended keys / values as the kernels read them: fp32 [H_kv, n_new, 128], rows 16-byte aligned."""
     if t.dtype != torch.float32 or t.shape != (H_kv, n_new, 128):
         raise RuntimeError(f"appended keys / values must be fp32 [{H_kv}, {n_new}, 128], got {tuple(t.shape)} {t.dtype}")
-    if t.stride(2) != 1 or t.stride(0) % 4 or t.stride(1) % 4 or t.data_ptr() % 16 or (n_new > 1 and t.stride(1) < 128):
+    sh, st, sc = t.stride()
+    if sc != 1 or sh % 4 or st % 4 or t.data_ptr() % 16 or (n_new > 1 and st < 128):
         t = t.clone(memory_format=torch.contiguous_format)
     return t
 

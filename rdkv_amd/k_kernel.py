@@ -68,9 +68,11 @@ def _seg3(t: Optional[torch.Tensor]):
     t = _as_3d(t)
     if t is None or t.numel() == 0:
         return None, 0, 0
-    if t.stride(2) != 1:
+    sh, st, sb = t.stride()
+    if sb != 1:
         t = t.contiguous()
-    return t, t.stride(0), t.stride(1)
+        sh, st, _ = t.stride()
+    return t, sh, st
 
 
 def k_mixed_qk_dot_into(Q: torch.Tensor, packed_layer, T_eff: int, out: torch.Tensor,
@@ -80,7 +82,10 @@ def k_mixed_qk_dot_into(Q: torch.Tensor, packed_layer, T_eff: int, out: torch.Te
     per-head Q permutation is applied inside the kernel instead of a separate gather."""
     if not _lib.available():
         raise RuntimeError("rdkv HIP backend is not available.")
-    args, dev, keep = _scores_args(Q, packed_layer, T_eff, out)
+    assert Q.shape[1] == D, f"Q head_dim {Q.shape[1]} != {D}"
+    dev = _lib.require_device(Q, out)
+    assert out.dtype == torch.float32 and out.stride(1) == 1, "out must be fp32 with unit column stride"
+    args, keep = _scores_args(Q, packed_layer, T_eff)
     t0 = 0.0
     if _DIAG_ENABLED:
         torch.cuda.synchronize()
@@ -93,17 +98,14 @@ def k_mixed_qk_dot_into(Q: torch.Tensor, packed_layer, T_eff: int, out: torch.Te
         _DIAG["n_calls"] += 1
 
 
-def _scores_args(Q: torch.Tensor, packed_layer, T_eff: int, out: torch.Tensor):
-    """What the K launches take of a query and a layer, checked -> (arguments, device, tensors they point into)."""
+def _scores_args(Q: torch.Tensor, packed_layer, T_eff: int):
+    """What the K launches take of a query and a layer -> (arguments, tensors they point into)."""
     H_q = Q.shape[0]
-    assert Q.shape[1] == D, f"Q head_dim {Q.shape[1]} != {D}"
-    dev = _lib.require_device(Q, out)
     n2, n4, n8 = (int(v) for v in packed_layer.K_ch_seg_bounds)
     n2p, n4p = _seg_padded_len(n2, 4), _seg_padded_len(n4, 2)
     sc = _as_3d(packed_layer.K_ch_scale)
     zp = _as_3d(packed_layer.K_ch_zp)
     H_kv = sc.shape[0]
-    assert out.dtype == torch.float32 and out.stride(1) == 1, "out must be fp32 with unit column stride"
     if Q.dtype not in _lib.DTYPE_CODE:
         Q = Q.float()
     if Q.stride(1) != 1:
@@ -117,9 +119,10 @@ def _scores_args(Q: torch.Tensor, packed_layer, T_eff: int, out: torch.Tensor):
     K4, k4h, k4t = _seg3(packed_layer.K_4bit)
     K8, k8h, k8t = _seg3(packed_layer.K_8bit)
     return (Q.data_ptr(), _lib.DTYPE_CODE[Q.dtype], Q.stride(0), H_q, H_kv,
-            _lib.ptr(K2), k2h, k2t, _lib.ptr(K4), k4h, k4t, _lib.ptr(K8), k8h, k8t,
-            _lib.ptr(sc), _lib.ptr(zp), sc.stride(0) if sc.numel() else 0,
-            _lib.ptr(perm), perm_sh, n2p, n4p, n8, int(T_eff)), dev, (Q, K2, K4, K8)
+            K2.data_ptr() if K2 is not None else None, k2h, k2t, K4.data_ptr() if K4 is not None else None, k4h, k4t,
+            K8.data_ptr() if K8 is not None else None, k8h, k8t,
+            sc.data_ptr() or None, zp.data_ptr() or None, sc.stride(0) if sc.numel() else 0,
+            perm.data_ptr() or None, perm_sh, n2p, n4p, n8, int(T_eff)), (Q, K2, K4, K8)
 
 
 def k_mixed_qk_dot(Q: torch.Tensor, packed_layer, T_eff: int) -> torch.Tensor:

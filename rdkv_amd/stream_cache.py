@@ -124,6 +124,16 @@ class StreamCache:
         return (None, 0) if self.n_groups == self.n_work else (_lib.ptr(self.groups), self.n_groups)
 
     @property
+    def units_host_arg(self) -> int:
+        """The address of ``units_host`` (a tensor over the same bytes gives it at a tenth of the array's time)."""
+        units, kept = self.units_host, self.__dict__.get("_units_bytes")
+        if kept is None or kept[0] is not units:
+            if not (units.flags.writeable and units.flags.c_contiguous):
+                return units.ctypes.data
+            kept = self.__dict__["_units_bytes"] = (units, torch.from_numpy(units.view(np.uint8)))
+        return kept[1].data_ptr()
+
+    @property
     def row_dwords_arg(self) -> int:
         """The ``max_row_dwords`` argument of the fused entry points: the longest K row, and in
         bits 8 and up the one row shape of all units (the library has kernels for some shapes)."""
@@ -846,73 +856,70 @@ def decode_attn_fused(cache: StreamCache, q: torch.Tensor, out: Optional[torch.T
     caches of at most ONE_LAUNCH_MAX_WORK work items (none, as shipped)."""
     lib = _lib.load()
     dev = _lib.require_device(q)
-    assert q.dim() == 2 and q.shape == (cache.rows, 128) and q.stride(1) == 1, f"q must be [{cache.rows},128]"
-    if q.dtype not in _lib.DTYPE_CODE:
-        q = q.float()
+    q_dt = _lib.DTYPE_CODE.get(q.dtype)
+    if q_dt is None:
+        q, q_dt = q.float(), 0
+    assert q.shape == (cache.rows, 128), f"q must be [{cache.rows},128]"
+    q_sh, q_st = q.stride()
+    assert q_st == 1, f"q must be [{cache.rows},128] with unit stride"
     if out is None:
         out = torch.empty(cache.rows, 128, dtype=torch.float32, device=dev)
     if lse is None:
         lse = torch.empty(cache.rows, dtype=torch.float32, device=dev)
-    assert out.dtype == torch.float32 and out.stride(1) == 1 and lse.dtype == torch.float32 and lse.is_contiguous()
-    rc = rs = None
+    out_sh, out_st = out.stride()
+    assert out.dtype == torch.float32 and out_st == 1 and lse.dtype == torch.float32 and lse.is_contiguous()
+    rc = rs = cos = sin = None
     rope_dt = 0
     if rope is not None:
         rc, rs = rope
-        _lib.require_device(rc, rs)
-        assert rc.numel() == 64 and rs.numel() == 64 and rc.dtype == rs.dtype and rc.dtype in _lib.DTYPE_CODE
+        _same_device(rc, rs)
+        rope_dt = _lib.DTYPE_CODE.get(rc.dtype)
+        assert rc.numel() == 64 and rs.numel() == 64 and rc.dtype == rs.dtype and rope_dt is not None
         rc, rs = rc.contiguous(), rs.contiguous()
-        rope_dt = _lib.DTYPE_CODE[rc.dtype]
-    need = lib.rdkv_decode_fused_workspace_bytes(cache.n_work, cache.G)
-    ws = _lib.workspace(dev, need)
-    stream = _lib.stream_of(dev)
+        cos, sin = rc.data_ptr(), rs.data_ptr()
     assert zone_c_weights is None or zone_c is not None, "zone_c_weights needs zone_c"
     if one_launch is None:
         one_launch = zone_c is None and cache.n_work <= ONE_LAUNCH_MAX_WORK
     assert not (one_launch and zone_c is not None), "one_launch does not take zone_c"
-    if one_launch:
-        _lib.check(lib.rdkv_decode_fused_one_launch(
-            None, cache.units.data_ptr(), cache.n_units, cache.work.data_ptr(), cache.n_work,
-            *cache.groups_arg, cache.row_dwords_arg,
-            q.data_ptr(), _lib.DTYPE_CODE[q.dtype], q.stride(0), cache.G, _lib.ptr(rc), _lib.ptr(rs), rope_dt,
-            out.data_ptr(), out.stride(0), lse.data_ptr(), ws.data_ptr(), ws.numel(), cache.tickets.data_ptr(),
-            stream))
-        return out, lse
     if zone_c is None:
-        _lib.check(lib.rdkv_decode_fused(
-            None, cache.units.data_ptr(), cache.n_units, cache.work.data_ptr(), cache.n_work,
-            *cache.groups_arg, cache.row_dwords_arg,
-            q.data_ptr(), _lib.DTYPE_CODE[q.dtype], q.stride(0), cache.G, _lib.ptr(rc), _lib.ptr(rs), rope_dt,
-            out.data_ptr(), out.stride(0), lse.data_ptr(), ws.data_ptr(), ws.numel(), stream))
+        ws = _lib.workspace(dev, lib.rdkv_decode_fused_workspace_bytes(cache.n_work, cache.G))
+        args = (None, cache.units.data_ptr(), cache.n_units, cache.work.data_ptr(), cache.n_work,
+                *cache.groups_arg, cache.row_dwords_arg, q.data_ptr(), q_dt, q_sh, cache.G, cos, sin, rope_dt,
+                out.data_ptr(), out_sh, lse.data_ptr(), ws.data_ptr(), ws.numel())
+        if one_launch:
+            _lib.check(lib.rdkv_decode_fused_one_launch(*args, cache.tickets.data_ptr(), _lib.stream_of(dev)))
+        else:
+            _lib.check(lib.rdkv_decode_fused(*args, _lib.stream_of(dev)))
         return out, lse
+    # (a layer of a decode loop comes through here once a step: its time is what these checks and the one call take)
     K_new, V_new = zone_c[0], zone_c[1]
     counts = zone_c[2] if len(zone_c) > 2 else None
-    _lib.require_device(K_new, V_new)
-    assert K_new.dtype == torch.float32 and V_new.dtype == torch.float32 and K_new.shape == V_new.shape
+    _same_device(K_new, V_new)
+    shape, stride = K_new.shape, K_new.stride()
+    assert K_new.dtype == torch.float32 and V_new.dtype == torch.float32 and shape == V_new.shape
     n_kv_rows = cache.rows // cache.G
-    assert K_new.dim() == 3 and K_new.shape[0] == n_kv_rows and K_new.shape[2] == 128, (
-        f"zone C tensors must be [rows / G = {n_kv_rows}, n_new, 128], got {tuple(K_new.shape)}")
-    assert K_new.stride() == V_new.stride() and K_new.stride(2) == 1
+    assert len(shape) == 3 and shape[0] == n_kv_rows and shape[2] == 128, (
+        f"zone C tensors must be [rows / G = {n_kv_rows}, n_new, 128], got {tuple(shape)}")
+    assert stride == V_new.stride() and stride[2] == 1
     if counts is not None:
         assert counts.dtype == torch.int32 and counts.numel() == n_kv_rows and counts.is_contiguous()
-    _lib.check(lib.rdkv_decode_fused_partials(
-        None, cache.units.data_ptr(), cache.n_units, cache.work.data_ptr(), cache.n_work,
-        *cache.groups_arg, cache.row_dwords_arg,
-        q.data_ptr(), _lib.DTYPE_CODE[q.dtype], q.stride(0), cache.G, _lib.ptr(rc), _lib.ptr(rs), rope_dt,
-        ws.data_ptr(), ws.numel(), stream))
-    n_new = int(K_new.shape[1])
+    n_new = shape[1]
+    k_step = v_step = row = tail = None
+    k_sh = v_sh = step_dt = q_rot_tok = 0
     if append is not None:
         k_step, v_step, row = append
-        _lib.require_device(k_step, v_step, row)
+        _same_device(k_step, v_step, row)
         assert counts is not None, "append needs the per-row token counts"
+        step_dt = _lib.DTYPE_CODE.get(k_step.dtype)
         assert k_step.shape == (n_kv_rows, 128) and v_step.shape == (n_kv_rows, 128)
-        assert k_step.dtype == v_step.dtype and k_step.dtype in _lib.DTYPE_CODE
-        assert k_step.stride(1) == 1 and v_step.stride(1) == 1 and row.dtype == torch.int64 and row.numel() == 1
+        assert k_step.dtype == v_step.dtype and step_dt is not None
+        (k_sh, k_st), (v_sh, v_st) = k_step.stride(), v_step.stride()
+        assert k_st == 1 and v_st == 1 and row.dtype == torch.int64 and row.numel() == 1
         if zone_c_weights is not None:
             _lib.require_device(zone_c_weights)
             assert zone_c_weights.dtype == torch.float32 and zone_c_weights.dim() == 2
             assert zone_c_weights.stride(1) == 1 and zone_c_weights.shape[0] == cache.rows
             assert zone_c_weights.shape[1] >= n_new, f"zone_c_weights rows must hold {n_new} tokens"
-        q_rot_tok = 0
         if q_rotated_out is not None:
             _lib.require_device(q_rotated_out)
             assert q_rotated_out.dtype == q.dtype and q_rotated_out.stride(-1) == 1
@@ -923,7 +930,6 @@ def decode_attn_fused(cache: StreamCache, q: torch.Tensor, out: Optional[torch.T
                 q_rot_tok = q_rotated_out.stride(1)
             else:
                 assert q_rotated_out.shape == q.shape
-        tail = None
         if tail_scores is not None:
             self_s, next_s, q_block_start, block = tail_scores
             assert zone_c_weights is not None, "tail_scores are summed from zone_c_weights"
@@ -936,30 +942,38 @@ def decode_attn_fused(cache: StreamCache, q: torch.Tensor, out: Optional[torch.T
             tail = _lib.RdkvTailScores(self_s.data_ptr(), self_s.stride(0), _lib.ptr(next_s),
                                        next_s.stride(0) if next_s is not None else 0,
                                        -1 if q_block_start is None else int(q_block_start), int(block), int(q_rot_tok))
-        _lib.check(lib.rdkv_decode_fused_merge_zone_c_append(
-            cache.units.data_ptr(), cache.units_host.ctypes.data, cache.n_units, cache.n_work, cache.G,
-            q.data_ptr(), _lib.DTYPE_CODE[q.dtype], q.stride(0), _lib.ptr(rc), _lib.ptr(rs), rope_dt,
-            _lib.ptr(K_new), _lib.ptr(V_new), K_new.stride(0), K_new.stride(1) if n_new else 128, n_new,
-            counts.data_ptr(), k_step.data_ptr(), k_step.stride(0), v_step.data_ptr(), v_step.stride(0),
-            _lib.DTYPE_CODE[k_step.dtype], row.data_ptr(), out.data_ptr(), out.stride(0), lse.data_ptr(),
-            _lib.ptr(zone_c_weights), zone_c_weights.stride(0) if zone_c_weights is not None else 0,
-            _lib.ptr(q_rotated_out), q_rotated_out.stride(0) if q_rotated_out is not None else 0,
-            ctypes.addressof(tail) if tail is not None else None,
-            ws.data_ptr(), ws.numel(), stream))
-        return out, lse
-    assert q_rotated_out is None and tail_scores is None, "q_rotated_out / tail_scores need append"
-    if zone_c_weights is not None:
-        _lib.require_device(zone_c_weights)
-        assert zone_c_weights.dtype == torch.float32 and zone_c_weights.dim() == 2 and zone_c_weights.stride(1) == 1
-        assert zone_c_weights.shape[0] == cache.rows and zone_c_weights.shape[1] >= n_new, (
-            f"zone_c_weights must be [rows = {cache.rows}, >= {n_new}], got {tuple(zone_c_weights.shape)}")
-    _lib.check(lib.rdkv_decode_fused_merge_zone_c(
-        cache.units.data_ptr(), cache.units_host.ctypes.data, cache.n_units, cache.n_work, cache.G,
-        q.data_ptr(), _lib.DTYPE_CODE[q.dtype], q.stride(0), _lib.ptr(rc), _lib.ptr(rs), rope_dt,
-        _lib.ptr(K_new), _lib.ptr(V_new), K_new.stride(0), K_new.stride(1) if n_new else 128, n_new,
-        _lib.ptr(counts), out.data_ptr(), out.stride(0), lse.data_ptr(), _lib.ptr(zone_c_weights),
-        zone_c_weights.stride(0) if zone_c_weights is not None else 0, ws.data_ptr(), ws.numel(), stream))
+    else:
+        assert q_rotated_out is None and tail_scores is None, "q_rotated_out / tail_scores need append"
+        if zone_c_weights is not None:
+            _lib.require_device(zone_c_weights)
+            assert zone_c_weights.dtype == torch.float32 and zone_c_weights.dim() == 2 and zone_c_weights.stride(1) == 1
+            assert zone_c_weights.shape[0] == cache.rows and zone_c_weights.shape[1] >= n_new, (
+                f"zone_c_weights must be [rows = {cache.rows}, >= {n_new}], got {tuple(zone_c_weights.shape)}")
+    groups, n_groups = cache.groups_arg
+    args = (cache.units.data_ptr(), cache.units_host_arg, cache.n_units, cache.work.data_ptr(),
+            cache.n_work, groups, n_groups, cache.row_dwords_arg, cache.G, q.data_ptr(), q_dt, q_sh, cos, sin, rope_dt,
+            K_new.data_ptr() or None, V_new.data_ptr() or None, stride[0], stride[1] if n_new else 128, n_new,
+            counts.data_ptr() if counts is not None else None,
+            k_step.data_ptr() if k_step is not None else None, k_sh, v_step.data_ptr() if v_step is not None else None, v_sh,
+            step_dt, row.data_ptr() if row is not None else None, out.data_ptr(), out_sh, lse.data_ptr(),
+            *((_lib.ptr(zone_c_weights), zone_c_weights.stride(0)) if zone_c_weights is not None else (None, 0)),
+            *((_lib.ptr(q_rotated_out), q_rotated_out.stride(0)) if q_rotated_out is not None else (None, 0)),
+            ctypes.addressof(tail) if tail is not None else None)
+    stream, ws = _lib.stream_workspace(dev)
+    rcode = lib.rdkv_decode_fused_zone_c(*args, ws.data_ptr(), ws.numel(), stream)
+    if rcode == _lib.RDKV_EWORKSPACE:
+        ws = _lib.workspace(dev, lib.rdkv_decode_fused_workspace_bytes(cache.n_work, cache.G))
+        rcode = lib.rdkv_decode_fused_zone_c(*args, ws.data_ptr(), ws.numel(), stream)
+    if rcode:
+        _lib.check(rcode)
     return out, lse
+
+
+def _same_device(a: torch.Tensor, b: torch.Tensor, c: Optional[torch.Tensor] = None) -> None:
+    """``_lib.require_device`` in a fraction of its time where all is well."""
+    d = a.get_device()
+    if d < 0 or b.get_device() != d or (c is not None and c.get_device() != d):
+        _lib.require_device(a, b, c)
 
 
 # ---------------------------------------------------------------------------

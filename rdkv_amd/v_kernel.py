@@ -73,7 +73,7 @@ def _launch(attn_weights, V_2bit, V_4bit, V_8bit, V_scale, V_zp, seg_bounds_per_
             out, V16, n_v16_per_head, max_T_v, new=None):
     """``new`` = (weights [H_q, n], values fp32 [H_kv, n, 128] with 16-byte aligned rows): a further zone,
     added by the same launch; V_scale may then be None (nothing packed).  A third entry (workspace, how much of
-    it ``rdkv_attn_scores`` took, its pairs, keep the weights): the rows ``attn_weights`` | weights hold scores."""
+    it ``rdkv_attn_scores`` took, its pairs, keep the weights, T_old): ``attn_weights`` is its whole rows of scores."""
     # (this runs once per layer and decode step: views and helper calls are kept to what the launch needs)
     lib = _lib.load()
     w = attn_weights
@@ -120,9 +120,10 @@ def _launch(attn_weights, V_2bit, V_4bit, V_8bit, V_scale, V_zp, seg_bounds_per_
     if new is None:
         _lib.check(lib.rdkv_v_weighted_sum(*packed, *result))
     elif scores is not None:
-        vn, (_, _, pairs, keep) = new[1], scores
-        _lib.check(lib.rdkv_v_weighted_sum_scores(*packed, w.shape[1], vn.data_ptr(), vn.stride(0), vn.stride(1),
-                                                  vn.shape[1], ws.data_ptr(), pairs, keep, *result))
+        vn, (_, _, pairs, keep, t_old) = new[1], scores
+        vn_sh, vn_st, _ = vn.stride()
+        _lib.check(lib.rdkv_v_weighted_sum_scores(*packed, t_old, vn.data_ptr(), vn_sh, vn_st, vn.shape[1], ws.data_ptr(),
+                                                  pairs, keep, *result))
     else:
         wn, vn = new
         _lib.check(lib.rdkv_v_weighted_sum_new_values(*packed, wn.data_ptr(), wn.stride(0), vn.data_ptr(), vn.stride(0),
