@@ -750,6 +750,15 @@ int rdkv_knapsack_batched(const float *scores, int64_t stride_b, int B, int64_t 
                           int out_elem_size, int64_t out_stride_b, int32_t *counts, void *workspace,
                           int64_t workspace_bytes, void *stream);
 
+/* The same with the budget formed in the launch: `value` for every row, or, with kept_counts (device int32
+ * [B, kept_options]), rdkv_k_budget_per_head's of these counts with k_budget_bits = value, T = tokens. */
+int rdkv_knapsack_batched_value(const float *scores, int64_t stride_b, int B, int64_t T, float value,
+                                const int32_t *kept_counts, int kept_options, int zero_option, int64_t tokens,
+                                int head_dim, const float *bits_host, const float *eps_host, int n_options,
+                                int max_iters, float tol, int group_rows, void *out, int out_elem_size,
+                                int64_t out_stride_b, int32_t *counts, void *workspace, int64_t workspace_bytes,
+                                void *stream);
+
 /* obkv_fast.py:1033-1035: the per-head K budget k_budget_bits / (head_dim * max(kept_h, 1)) as
  * the reference's fp32 tensor expression evaluates it (product, reciprocal, product), from the
  * per-option token counts of rdkv_knapsack_batched: kept_h = T - counts[h][zero_option]

@@ -125,17 +125,33 @@ __device__ float row_max(const float* __restrict__ row, int T, float* lds) {
   return block_reduce(m, MaxF(), lds);
 }
 
+// The budget of a row (average bits per element): from a tensor, one value for all, or the K budget that the V
+// allocation's counts leave a head (k_budget_kernel's expression).  Formed where it is used: the launches that
+// filled a tensor with it were 1.3 and 4 us and a gap each of a selected layer's serial chain, and 5 us of host.
+struct Budget {
+  const float* rows;
+  const int32_t* counts;
+  int n_options, zero_col, tokens;
+  float head_dim, value;
+  __device__ __forceinline__ float operator()(int b) const {
+    if (counts == nullptr) return rows ? rows[b] : value;
+    int kept = tokens - (zero_col >= 0 ? counts[(int64_t)b * n_options + zero_col] : 0);
+    if (kept < 1) kept = 1;
+    return __fmul_rn(__fdiv_rn(1.0f, __fmul_rn(head_dim, (float)kept)), value);
+  }
+};
+
 // Phase 1 of the batched form.  Per row: the starting upper bound and how many doublings the row
 // asks for on its own (kMaxDoublings if its average never drops to the budget).
 __global__ void __launch_bounds__(kMaxThreads)
 knapsack_expand_kernel(const float* __restrict__ scores, int64_t stride_b, int T,
-                       const float* __restrict__ budget, Options o, float* __restrict__ lam0_out,
+                       Budget budget, Options o, float* __restrict__ lam0_out,
                        int* __restrict__ doublings_out) {
   __shared__ int lds[32];
   const int b = blockIdx.x;
   const float* row = scores + (int64_t)b * stride_b;
   const float lam0 = fmaxf(__fmul_rn(row_max(row, T, reinterpret_cast<float*>(lds)), 0.375f), 1e-8f);
-  const float bud = budget[b];
+  const float bud = budget(b);
   float lam = lam0;
   int d = 0;
   for (; d < kMaxDoublings; ++d) {
@@ -149,7 +165,7 @@ knapsack_expand_kernel(const float* __restrict__ scores, int64_t stride_b, int T
 // row asks for more or when every bound has reached 1e12), then bisect this row.
 __global__ void __launch_bounds__(kMaxThreads)
 knapsack_bisect_kernel(const float* __restrict__ scores, int64_t stride_b, int group_rows, int T,
-                       const float* __restrict__ budget, Options o, int max_iters, float tol,
+                       Budget budget, Options o, int max_iters, float tol,
                        const float* __restrict__ lam0_all, const int* __restrict__ doublings_all,
                        void* __restrict__ out, int out_elem_size, int64_t out_stride_b,
                        int* __restrict__ counts) {
@@ -178,7 +194,7 @@ knapsack_bisect_kernel(const float* __restrict__ scores, int64_t stride_b, int g
   float lam_hi = lam0_all[b];
   for (int i = 0; i < mine; ++i) lam_hi = __fmul_rn(lam_hi, 2.0f);
 
-  const float bud = budget[b];
+  const float bud = budget(b);
   float lam_lo = 0.f, lam_final = 0.f;
   if (!(solve_avg(row, T, 0.f, o, lds) <= bud)) {
     const float denom = fmaxf(bud, 1e-8f);
@@ -366,7 +382,7 @@ __global__ void coop_init_kernel(uint32_t* state, int64_t n_words) {
 template <int HELD>
 __global__ void __launch_bounds__(kCoopThreads) __attribute__((amdgpu_waves_per_eu(4)))
 knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int group_rows, int T, int S,
-                     const float* __restrict__ budget, Options o, int max_iters, float tol,
+                     Budget budget, Options o, int max_iters, float tol,
                      uint32_t* __restrict__ state, void* __restrict__ out, int out_elem_size,
                      int64_t out_stride_b, int* __restrict__ counts) {
   __shared__ int lds[64];
@@ -387,7 +403,7 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
   if (threadIdx.x < kCoopWords) red[threadIdx.x] = 0;
   if (threadIdx.x == 0) failed = 0;
   const float* row = scores + (int64_t)b * stride_b;
-  const float bud = budget[b];
+  const float bud = budget(b);
   float se[HELD][kMaxOptions];
   bool valid[HELD];
   float m = -__builtin_inff();
@@ -651,14 +667,14 @@ __device__ __forceinline__ int wave_sum_uniform(int v) {
 template <int HELD, int NOPT>
 __global__ void __launch_bounds__(kMaxThreads)
 knapsack_group_kernel(const float* __restrict__ scores, int64_t stride_b, int group_rows, int T,
-                      const float* __restrict__ budget, Options o, int max_iters, float tol, void* __restrict__ out,
+                      Budget budget, Options o, int max_iters, float tol, void* __restrict__ out,
                       int out_elem_size, int64_t out_stride_b, int* __restrict__ counts) {
   __shared__ float s_lam0[kGroupMaxRows];
   __shared__ int s_d[kGroupMaxRows];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = blockIdx.x * group_rows + wave;
   const float* row = scores + (int64_t)b * stride_b;
-  const float bud = budget[b];
+  const float bud = budget(b);
   float se[HELD][NOPT];       // score times eps (+inf for the options past the last: never the smallest)
   float m = -__builtin_inff();
 #pragma unroll
@@ -838,16 +854,13 @@ int fail(const char* msg) {
   return RDKV_EINVAL;
 }
 
-// Per-head K budget of the joint selection: k_budget_bits / (head_dim * max(kept, 1)) evaluated
+// Per-head K budget of the joint selection as a launch of its own: k_budget_bits / (head_dim * max(kept, 1)) evaluated
 // the way the reference's tensor expression is: fp32 product, fp32 reciprocal, fp32 product.
 __global__ void k_budget_kernel(const int32_t* __restrict__ counts, int n_options, int zero_col, int rows,
                                 int tokens, float head_dim, float k_budget_bits, float* __restrict__ out) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= rows) return;
-  int kept = tokens - (zero_col >= 0 ? counts[(int64_t)r * n_options + zero_col] : 0);
-  if (kept < 1) kept = 1;
-  const float denom = __fmul_rn(head_dim, (float)kept);
-  out[r] = __fmul_rn(__fdiv_rn(1.0f, denom), k_budget_bits);
+  out[r] = Budget{nullptr, counts, n_options, zero_col, tokens, head_dim, k_budget_bits}(r);
 }
 
 int make_options(const float* bits_host, const float* eps_host, int n, Options* o) {
@@ -936,14 +949,13 @@ RDKV_API int64_t rdkv_knapsack_workspace_bytes(int B) {
   return b * 8 + 256 + b * (int64_t)kCoopRowWords * 4;
 }
 
-RDKV_API int rdkv_knapsack_batched(const float* scores, int64_t stride_b, int B, int64_t T,
-                                   const float* budget, const float* bits_host, const float* eps_host,
-                                   int n_options, int max_iters, float tol, int group_rows, void* out,
-                                   int out_elem_size, int64_t out_stride_b, int32_t* counts, void* workspace,
-                                   int64_t workspace_bytes, void* stream) {
+static int knapsack_batched(const float* scores, int64_t stride_b, int B, int64_t T, const Budget& budget,
+                            const void* given, const float* bits_host, const float* eps_host, int n_options, int max_iters, float tol,
+                            int group_rows, void* out, int out_elem_size, int64_t out_stride_b, int32_t* counts,
+                            void* workspace, int64_t workspace_bytes, void* stream) {
   Options o;
   if (int rc = make_options(bits_host, eps_host, n_options, &o)) return rc;
-  if (int rc = check_common(scores, B, T, budget, out, out_elem_size)) return rc;
+  if (int rc = check_common(scores, B, T, given, out, out_elem_size)) return rc;
   if (B == 0) return 0;
   if (workspace == nullptr || workspace_bytes < rdkv_knapsack_workspace_bytes(B))
   {
@@ -990,6 +1002,31 @@ RDKV_API int rdkv_knapsack_batched(const float* scores, int64_t stride_b, int B,
                      o, max_iters, tol, lam0, doublings, out, out_elem_size, out_stride_b, counts);
   RDKV_CHECK_LAUNCH("rdkv_knapsack_batched");
   return RDKV_OK;
+}
+
+RDKV_API int rdkv_knapsack_batched(const float* scores, int64_t stride_b, int B, int64_t T,
+                                   const float* budget, const float* bits_host, const float* eps_host,
+                                   int n_options, int max_iters, float tol, int group_rows, void* out,
+                                   int out_elem_size, int64_t out_stride_b, int32_t* counts, void* workspace,
+                                   int64_t workspace_bytes, void* stream) {
+  return knapsack_batched(scores, stride_b, B, T, Budget{budget, nullptr, 0, 0, 0, 0.f, 0.f}, budget, bits_host, eps_host,
+                          n_options, max_iters, tol, group_rows, out, out_elem_size, out_stride_b, counts, workspace,
+                          workspace_bytes, stream);
+}
+
+RDKV_API int rdkv_knapsack_batched_value(const float* scores, int64_t stride_b, int B, int64_t T, float value,
+                                         const int32_t* kept_counts, int kept_options, int zero_option, int64_t tokens,
+                                         int head_dim, const float* bits_host, const float* eps_host, int n_options,
+                                         int max_iters, float tol, int group_rows, void* out, int out_elem_size,
+                                         int64_t out_stride_b, int32_t* counts, void* workspace, int64_t workspace_bytes,
+                                         void* stream) {
+  if (kept_counts != nullptr && (kept_options < 1 || kept_options > kMaxOptions || zero_option >= kept_options || tokens < 0 ||
+                                 tokens > 0x7fffffffLL || head_dim < 1 || kept_counts == counts))
+    return fail("knapsack: bad counts for the budget");
+  return knapsack_batched(scores, stride_b, B, T,
+                          Budget{nullptr, kept_counts, kept_options, zero_option, (int)tokens, (float)head_dim, value}, scores,
+                          bits_host, eps_host, n_options, max_iters, tol, group_rows, out, out_elem_size, out_stride_b, counts,
+                          workspace, workspace_bytes, stream);
 }
 
 RDKV_API int rdkv_knapsack_rows(const float* scores, int64_t stride_b, int B, int64_t T, const double* budget,

@@ -10,7 +10,7 @@ from __future__ import annotations
 import ctypes
 import json
 import warnings
-from typing import Any, Dict, Optional, Tuple, Union
+from typing import Any, Dict, NamedTuple, Optional, Tuple, Union
 
 import torch
 from torch import Tensor
@@ -37,7 +37,18 @@ def _rows_f32(scores: Tensor) -> Tensor:
     return s if s.stride(-1) == 1 else s.contiguous()
 
 
-def knapsack_allocate(scores: Tensor, budget_per_token: Union[float, Tensor], epsilon=None, max_iters: int = 64,
+class KeptBudget(NamedTuple):
+    """The K budget that a V allocation leaves every head (obkv_fast.py:1033-1035): ``bits / (head_dim *
+    kept.clamp(min=1).float())`` in fp32 (which torch evaluates as reciprocal times number), kept = ``tokens``
+    less those that took the 0-bit option, column ``zero_col`` of ``counts`` [B, n_options] (-1: none)."""
+    counts: Tensor
+    zero_col: int
+    tokens: int
+    head_dim: int
+    bits: float
+
+
+def knapsack_allocate(scores: Tensor, budget_per_token: Union[float, Tensor, KeptBudget], epsilon=None, max_iters: int = 64,
                       tol: float = 0.01, bit_options: Optional[Tensor] = None, *, out_dtype=torch.uint8,
                       with_counts: bool = False, group_rows: int = 0):
     """``knapsack_bit_allocation_batched`` with the output type of the caller's choice (uint8 for
@@ -55,8 +66,14 @@ def knapsack_allocate(scores: Tensor, budget_per_token: Union[float, Tensor], ep
         assert budget_per_token.shape == (B,), (
             f"budget_per_token tensor must be [B={B}]; got {tuple(budget_per_token.shape)}")
         budget = budget_per_token.detach().float().to(dev).contiguous()
+        source = None
+    elif isinstance(budget_per_token, KeptBudget):
+        kept, zero_col, tokens, head_dim, kept_bits = budget_per_token
+        assert kept.shape[0] == B and kept.dtype == torch.int32 and kept.is_contiguous() and kept.device == dev, (
+            f"counts must be int32 [B={B}, options] on {dev}")
+        source = (kept_bits, kept.data_ptr(), int(kept.shape[1]), zero_col, tokens, head_dim)
     else:
-        budget = torch.full((B,), float(budget_per_token), dtype=torch.float32, device=dev)
+        source = (float(budget_per_token), None, 0, 0, 0, 0)
     bits_c, eps_c, n = _option_arrays(epsilon, bit_options)
     assert out_dtype in (torch.uint8, torch.int64)
     out = torch.empty(B, T, dtype=out_dtype, device=dev)
@@ -64,10 +81,12 @@ def knapsack_allocate(scores: Tensor, budget_per_token: Union[float, Tensor], ep
     lib = _lib.load()
     ws_bytes = lib.rdkv_knapsack_workspace_bytes(B)
     ws = _lib.workspace(dev, ws_bytes)
-    _lib.check(lib.rdkv_knapsack_batched(
-        _lib.ptr(s), s.stride(0), B, T, _lib.ptr(budget), bits_c, eps_c, n, int(max_iters), float(tol),
-        int(group_rows), _lib.ptr(out), out.element_size(), out.stride(0) if B else T, _lib.ptr(counts), ws.data_ptr(), ws_bytes,
-        _lib.stream_of(dev)))
+    rest = (bits_c, eps_c, n, int(max_iters), float(tol), int(group_rows), _lib.ptr(out), out.element_size(),
+            out.stride(0) if B else T, _lib.ptr(counts), ws.data_ptr(), ws_bytes, _lib.stream_of(dev))
+    if source is None:
+        _lib.check(lib.rdkv_knapsack_batched(_lib.ptr(s), s.stride(0), B, T, _lib.ptr(budget), *rest))
+    else:
+        _lib.check(lib.rdkv_knapsack_batched_value(_lib.ptr(s), s.stride(0), B, T, *source, *rest))
     return (out, counts) if with_counts else out
 
 

@@ -16,7 +16,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from .knapsack_solver import (DEFAULT_EPSILON_K, DEFAULT_EPSILON_V, knapsack_allocate,   # noqa: F401 (re-exported
+from .knapsack_solver import (DEFAULT_EPSILON_K, DEFAULT_EPSILON_V, KeptBudget, knapsack_allocate,   # noqa: F401 (re-exported
                               knapsack_bit_allocation_batched, load_epsilon_kv_from_calibration)  # as obkv_fast.py:38-46 does)
 from .packing import _pack_layer_per_head, pack_layer_per_head, pack_layers_per_head  # noqa: F401
 
@@ -99,18 +99,10 @@ def _allocate_k_bits_per_head(channel_scores: Tensor, k_avg: Union[float, Tensor
 
 
 def _k_budget_per_head(v_counts: Tensor, v_bit_options: Optional[Tensor], T: int, head_dim: int,
-                       k_budget_bits: float) -> Tensor:
-    """obkv_fast.py:1033-1035 from the per-option token counts of the V allocation: the tokens a
-    head keeps are those that did not take the 0-bit option, and its K budget is the reference's
-    fp32 expression ``k_budget_bits / (head_dim * kept.clamp(min=1).float())`` (which torch
-    evaluates as reciprocal times number), one value per row of ``v_counts``, on the device."""
+                       k_budget_bits: float) -> KeptBudget:
+    """obkv_fast.py:1033-1035: what the V allocation's per-option token counts leave the K allocation."""
     opts = [0.0, 2.0, 4.0, 8.0, 16.0] if v_bit_options is None else [float(b) for b in v_bit_options.tolist()]
-    zero_col = opts.index(0.0) if 0.0 in opts else -1
-    rows, n = int(v_counts.shape[0]), int(v_counts.shape[1])
-    out = torch.empty(rows, dtype=torch.float32, device=v_counts.device)
-    _lib.check(_lib.load().rdkv_k_budget_per_head(v_counts.data_ptr(), n, zero_col, rows, T, head_dim,
-                                                  float(k_budget_bits), _lib.ptr(out), _lib.stream_of(v_counts.device)))
-    return out
+    return KeptBudget(v_counts, opts.index(0.0) if 0.0 in opts else -1, T, head_dim, float(k_budget_bits))
 
 
 def _perhead_select_and_pack_joint(
@@ -163,8 +155,8 @@ def _perhead_select_and_pack_joint(
     t_v = stamp()
 
     k_avg_per_head = _k_budget_per_head(v_counts, v_bit_options, T, head_dim, k_budget_bits)
-    k_bits_perhead = _allocate_k_bits_per_head(channel_scores.float().to(dev), k_avg_per_head,
-                                               epsilon=eps_K, bit_options=k_bit_options)
+    k_bits_perhead = knapsack_allocate(channel_scores.float().to(dev), k_avg_per_head, epsilon=eps_K,
+                                       bit_options=k_bit_options)
     t_k = stamp()
 
     retained: list = []
