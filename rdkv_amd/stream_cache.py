@@ -127,11 +127,12 @@ class StreamCache:
     def units_host_arg(self) -> int:
         """The address of ``units_host`` (a tensor over the same bytes gives it at a tenth of the array's time)."""
         units, kept = self.units_host, self.__dict__.get("_units_bytes")
-        if kept is None or kept[0] is not units:
-            if not (units.flags.writeable and units.flags.c_contiguous):
-                return units.ctypes.data
-            kept = self.__dict__["_units_bytes"] = (units, torch.from_numpy(units.view(np.uint8)))
-        return kept[1].data_ptr()
+        if kept is not None and kept[0] is units and kept[1] is not None:
+            return kept[1].data_ptr()
+        # (made by the second call: it costs three lookups)
+        again = kept is not None and kept[0] is units and units.flags.writeable and units.flags.c_contiguous
+        self.__dict__["_units_bytes"] = (units, torch.from_numpy(units.view(np.uint8)) if again else None)
+        return units.ctypes.data
 
     @property
     def row_dwords_arg(self) -> int:
