@@ -315,7 +315,6 @@ class HostWords:
 
 
 _host_words: dict = {}         # (device, host thread) -> its words
-_retired_words: list = []      # kept: a launch whose call ended before it was read may still write to them
 
 
 def host_words(dev: torch.device, n: int) -> HostWords:
@@ -323,9 +322,9 @@ def host_words(dev: torch.device, n: int) -> HostWords:
     import threading
     key = (dev.index, threading.get_ident())
     w = _host_words.get(key)
-    if w is None or w.size < n or w.pending:
-        if w is not None:
-            _retired_words.append(w)
+    if w is not None and w.pending:     # a call that ended before it read them: its launches may still write
+        torch.cuda.synchronize(dev)
+    if w is None or w.size < n:
         w = _host_words[key] = HostWords(max(4096, 1 << (max(n, 1) - 1).bit_length()))
     w.tag, w.used, w.pending = w.tag % 0xFFFFFFFF + 1, 0, True            # (never 0, what fresh words hold)
     return w

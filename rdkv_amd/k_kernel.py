@@ -68,11 +68,11 @@ def _seg3(t: Optional[torch.Tensor]):
     t = _as_3d(t)
     if t is None or t.numel() == 0:
         return None, 0, 0
-    sh, st, sb = t.stride()
-    if sb != 1:
+    s = t.stride()
+    if s[2] != 1:
         t = t.contiguous()
-        sh, st, _ = t.stride()
-    return t, sh, st
+        s = t.stride()
+    return t, s[0], s[1]
 
 
 def k_mixed_qk_dot_into(Q: torch.Tensor, packed_layer, T_eff: int, out: torch.Tensor,

@@ -130,7 +130,7 @@ class StreamCache:
         if kept is not None and kept[0] is units and kept[1] is not None:
             return kept[1].data_ptr()
         # (made by the second call: it costs three lookups)
-        again = kept is not None and kept[0] is units and units.flags.writeable and units.flags.c_contiguous
+        again = kept is not None and kept[0] is units and units.size and units.flags.writeable and units.flags.c_contiguous
         self.__dict__["_units_bytes"] = (units, torch.from_numpy(units.view(np.uint8)) if again else None)
         return units.ctypes.data
 
@@ -867,8 +867,8 @@ def decode_attn_fused(cache: StreamCache, q: torch.Tensor, out: Optional[torch.T
         out = torch.empty(cache.rows, 128, dtype=torch.float32, device=dev)
     if lse is None:
         lse = torch.empty(cache.rows, dtype=torch.float32, device=dev)
-    out_sh, out_st = out.stride()
-    assert out.dtype == torch.float32 and out_st == 1 and lse.dtype == torch.float32 and lse.is_contiguous()
+    out_sh = out.stride(0)
+    assert out.dtype == torch.float32 and out.stride(1) == 1 and lse.dtype == torch.float32 and lse.is_contiguous()
     rc = rs = cos = sin = None
     rope_dt = 0
     if rope is not None:

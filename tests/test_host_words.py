@@ -87,17 +87,18 @@ def test_plan_and_its_numbers(monkeypatch, N, T):
 
 
 @gpu
-def test_words_of_a_call_that_was_not_read():
-    """The next call takes other words: a launch behind longer work may still write to the first."""
+def test_words_of_a_call_that_was_not_read(monkeypatch):
+    """The next call waits for the device first (a launch may still write to them), one that follows a read does not."""
     require_gpu()
     dev = torch.empty(1, device=DEV).device
-    first = _lib.host_words(dev, 24)
-    assert _lib.host_words(dev, 24) is not first
+    waits, sync = [], torch.cuda.synchronize
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: (waits.append(1), sync(*a))[1])
     vb, kb = (t.to(DEV) for t in _alloc(2, 30, 128, 1))
-    packing._plan_layers(vb, kb, dev)
-    kept = _lib._host_words[(dev.index, threading.get_ident())]
-    packing._plan_layers(vb, kb, dev)
-    assert _lib._host_words[(dev.index, threading.get_ident())] is kept
+    want = packing._plan_layers(vb, kb, dev)[3]
+    assert not waits
+    _lib.host_words(dev, 24)
+    assert packing._plan_layers(vb, kb, dev)[3] == want and waits == [1]
+    assert packing._plan_layers(vb, kb, dev)[3] == want and waits == [1]
 
 
 @gpu
