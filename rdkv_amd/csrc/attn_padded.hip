@@ -176,11 +176,19 @@ __device__ __forceinline__ int k_slot(int width, int p, int j) {
 // of a tile are one contiguous run per width, copied to LDS in aligned 16-byte pieces by loads that go there
 // directly, the next tile's under the current one's arithmetic.  The products run on
 // v_mfma_i32_16x16x64_i8 and are exact: the columns are sixteen tokens, whose bytes are cut from LDS, shifted
-// and masked, nothing more (8-bit codes less 128); the rows are the four base-256 digits of q * scale of four
-// query heads, as integers of 30 bits after a power of two per head that brings its largest just under 2^30.
+// and masked, nothing more (8-bit codes less 128); the rows are the four upper base-256 digits of q * scale of
+// four query heads, as integers of 30 bits after a power of two per head that brings its largest just under
+// 2^30, and a second product's rows are the two digits below those (heads of both groups in one): 46 bits, so a
+// channel keeps all 24 of its fp32 product down to 2^-22 of the head's largest.  (One extreme token widens its
+// channel's scale; all others lie at that channel's zero, and their scores come from channels 2^-10 of it and
+// less.  64 channels of 8 bit, one with a token 512 / 4096 / 30000 times as large and a query 8 times: error of
+// the others' scores 4.3e-8 / 4.7e-8 / 4.9e-8; with 30 bits alone 1.4e-7 / 1.4e-6 / 1.0e-5, with fp16 pairs in
+// fp32 sums 6.9e-8 / 7.0e-8 / 9.3e-8.  The second product is always formed: a test of how many channels need it
+// has heads on its wrong side, 47 of 64 extreme ones for instance.  It costs 1.4 us of a layer's call at 32k, 2.4 at
+// 128k low-bit.)
 // The codes of the narrow widths enter times 2^5 and 2^3, so that every width's q * scale has a like part of
-// those 30 bits (without: 6.8e-8).  The sums start from minus the zero points' part, formed by the same
-// products, so they are sums of the signed values themselves; a lane ends up with the four digits' sums of one
+// those bits.  The sums start from minus the zero points' part, formed by the same
+// products, so they are sums of the signed values themselves; a lane ends up with the six digits' sums of one
 // token and head and joins them in fp32, one rounding and one of the factor 1 / sqrt(128).  Error against 64
 // bits: 4.0e-8 of the scores in the 2-norm (fp16 pairs in fp32 sums: 4.1e-8 .. 5.2e-8).
 // What bounds it: the chain of the set-up (tables and query, digits, first tile) and the padded rows' loads.
@@ -204,6 +212,7 @@ __device__ __forceinline__ int k_slot(int width, int p, int j) {
 template <int NG>
 struct KSetup {
   alignas(16) int8_t digit[kKBlocks][NG][16][64];   // [block][head group][head, digit][code]
+  alignas(16) int8_t low[kKBlocks][4][2 * NG][64];  // [block][head][head group, lower digit][code]
   alignas(16) int8_t zero[kKBlocks][2][64];         // zero points: low and high digit of base 128
   float q[4 * NG][kD];
   float big[4][4 * NG], rest[4][4 * NG];            // by wavefront: largest |q * scale| of a head, its bias
@@ -225,6 +234,7 @@ constexpr int kKNewKeys = 64;      // appended keys of a pass of a workgroup: tw
 constexpr int kKNewGroups = 128;   // workgroups of a KV head that take appended keys, at most
 constexpr int kKMaxPairs = 1024 + kKNewGroups;
 
+constexpr int kKMaxLds = 160 * 1024;   // LDS of a compute unit, and of a workgroup at most
 constexpr int kKResident = 4;      // workgroups per compute unit (wavefronts per SIMD) the kernel is compiled for
 
 // 16-byte pieces of a tile of 256 rows of `sub` bytes that may start and end anywhere in a piece.
@@ -424,7 +434,7 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     m_run[hg] = -INFINITY;
     l_run[hg] = 0.0f;
   }
-  for (int i = tl; i < (int)(sizeof(su.digit) + sizeof(su.zero)) / 16; i += 256)
+  for (int i = tl; i < (int)(sizeof(su.digit) + sizeof(su.low) + sizeof(su.zero)) / 16; i += 256)
     reinterpret_cast<u32x4 *>(smem)[i] = u32x4{0, 0, 0, 0};
 #pragma unroll
   for (int u = 0; u < 2 * NG; ++u) (&su.q[0][0])[tl + 256 * u] = qrow[u];
@@ -498,9 +508,14 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
       su.zero[blk][1][at] = (int8_t)((z - zlo) >> 7);
 #pragma unroll
       for (int g = 0; g < NHD; ++g) {
-        const int x = ((int)rintf(ldexpf(qv[u][g], ex[g] - log)) + 0x00808080) ^ 0x00808080;
+        // the nearest integer and sixteen bits of what it leaves (exact), within what two digits reach
+        const float v = ldexpf(qv[u][g], ex[g] - log), whole = rintf(v);
+        const int rest16 = (int)rintf((v - whole) * 65536.0f), carry = rest16 > 0x7f7f ? 1 : 0;
+        const int x = ((int)whole + carry + 0x00808080) ^ 0x00808080, y = (rest16 - (carry << 16) + 0x80) ^ 0x80;
 #pragma unroll
         for (int l = 0; l < 4; ++l) su.digit[blk][g >> 2][4 * (g & 3) + l][at] = (int8_t)(x >> (8 * l));
+#pragma unroll
+        for (int l = 0; l < 2; ++l) su.low[blk][g & 3][2 * (g >> 2) + l][at] = (int8_t)(y >> (8 * l));
       }
     }
   }
@@ -512,7 +527,14 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
             e8 = __builtin_amdgcn_readfirstlane((int)ext[2]);
   const int blocks[3] = {(min(e2, sub2) + 15) >> 4, (min(e4, sub4) + 31) >> 5, (e8 + 63) >> 6};
   lds_barrier();
-  intx4 dig[kKBlocks][NG], start[NG];
+  constexpr bool kHeld = NG == 1;      // (eight heads: the digits stay in LDS, as the lower ones do)
+  intx4 dig[kHeld ? kKBlocks : 1][NG], start[NG], start_low{0, 0, 0, 0};
+  auto digits = [&](int b, int hg) __attribute__((always_inline)) {
+    return kHeld ? dig[kHeld ? b : 0][hg] : *reinterpret_cast<const intx4 *>(&su.digit[b][hg][r][16 * grp]);
+  };
+  auto low_digits = [&](int b) __attribute__((always_inline)) {
+    return *reinterpret_cast<const intx4 *>(&su.low[b][r >> 2][r & (2 * NG - 1)][16 * grp]);
+  };
 #pragma unroll
   for (int hg = 0; hg < NG; ++hg) start[hg] = intx4{0, 0, 0, 0};
 #pragma unroll
@@ -520,21 +542,28 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     if ((b & 1) < blocks[b >> 1]) {
       intx4 z = *reinterpret_cast<const intx4 *>(&su.zero[b][r & 1][16 * grp]);
       if (r > 1) z = intx4{0, 0, 0, 0};
+      start_low = __builtin_amdgcn_mfma_i32_16x16x64_i8(low_digits(b), z, start_low, 0, 0, 0);
 #pragma unroll
       for (int hg = 0; hg < NG; ++hg) {
-        dig[b][hg] = *reinterpret_cast<const intx4 *>(&su.digit[b][hg][r][16 * grp]);
-        start[hg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(dig[b][hg], z, start[hg], 0, 0, 0);
+        if (kHeld) dig[kHeld ? b : 0][hg] = *reinterpret_cast<const intx4 *>(&su.digit[b][hg][r][16 * grp]);
+        start[hg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(digits(b, hg), z, start[hg], 0, 0, 0);
       }
     }
   }
+  // minus the zero points' part, from its two digits' columns
+  auto minus_zero = [&](intx4 v) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = -(__shfl(v[i], 16 * grp, 64) + 128 * __shfl(v[i], 16 * grp + 1, 64));
+    return v;
+  };
+  start_low = minus_zero(start_low);
   float half_up[NG], factor[NG], offset[NG];    // of this lane's head, lane / 16 of the group: 2^-e in two parts
   constexpr bool kParked = STATS && NG > 1;     // (eight heads and their softmax: no registers for these)
   floatx4 *parked = reinterpret_cast<floatx4 *>(su.q);   // (the query is done with) by head: the sums' start, then these
+  if (kParked && wave == 0 && r == 0) reinterpret_cast<intx4 *>(parked)[8 * NG + grp] = start_low;
 #pragma unroll
   for (int hg = 0; hg < NG; ++hg) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      start[hg][i] = -(__shfl(start[hg][i], 16 * grp, 64) + 128 * __shfl(start[hg][i], 16 * grp + 1, 64));
+    start[hg] = minus_zero(start[hg]);
     const int g = 4 * hg + grp;
     const float big = fmaxf(fmaxf(su.big[0][g], su.big[1][g]), fmaxf(su.big[2][g], su.big[3][g]));
     const int e = 30 - ((int)(__float_as_uint(big) >> 23) - 126);
@@ -564,11 +593,13 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     const int64_t t0 = (int64_t)tile * 256;
     const int ntok = T - t0 < 256 ? (int)(T - t0) : 256;
     const int tok = wave * 64 + 4 * r;
-    intx4 acc[4][NG];
+    intx4 acc[4][NG], acc_low[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      acc_low[j] = kParked ? reinterpret_cast<const intx4 *>(parked)[8 * NG + grp] : start_low;
 #pragma unroll
       for (int hg = 0; hg < NG; ++hg) acc[j][hg] = kParked ? reinterpret_cast<const intx4 *>(parked)[8 * hg + grp] : start[hg];
+    }
     {
       const Run r0 = run_of(tile, 0), r1 = run_of(tile, 1), r2 = run_of(tile, 2);
       const int begin = rows_off + buffer * tile_lds;
@@ -578,6 +609,10 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
       for (int b = 0; b < kKBlocks; ++b) {
         if ((b & 1) < blocks[b >> 1]) {
           const int w = b >> 1, nd = 1 << w;       // dwords a lane takes of a row
+          const intx4 low = low_digits(b);
+          intx4 high[NG];
+#pragma unroll
+          for (int hg = 0; hg < NG; ++hg) high[hg] = digits(b, hg);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const int off = base[w] + j * rowb[w] + (b & 1) * 16 * nd;
@@ -600,7 +635,8 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
                             (int)(d[3] ^ 0x80808080u)};
 #pragma unroll
             for (int hg = 0; hg < NG; ++hg)
-              acc[j][hg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(dig[b][hg], codes, acc[j][hg], 0, 0, 0);
+              acc[j][hg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(high[hg], codes, acc[j][hg], 0, 0, 0);
+            acc_low[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(low, codes, acc_low[j], 0, 0, 0);
           }
         }
       }
@@ -614,10 +650,10 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const intx4 x = acc[j][hg];
-          // (the upper two digits' sum, below 2^31, as an fp32 number and what it leaves: one rounding that counts)
-          const int top = x[3] * 256 + x[2];
-          const float head = (float)top, left = (float)(top - (int)head);
-          const float sum = fmaf(head, 65536.0f, fmaf(left, 65536.0f, fmaf((float)x[1], 256.0f, (float)x[0])));
+          // (the upper two digits' sum as an fp32 number and what it leaves: one rounding that counts)
+          const float x3 = (float)x[3], x2 = (float)x[2], head = fmaf(x3, 256.0f, x2), left = fmaf(x3, 256.0f, -head) + x2;
+          const float low = fmaf((float)acc_low[j][2 * hg + 1], 256.0f, (float)acc_low[j][2 * hg]);
+          const float sum = fmaf(head, 65536.0f, fmaf(left, 65536.0f, fmaf((float)x[1], 256.0f, fmaf(low, 0x1p-16f, (float)x[0]))));
           v[j] = fmaf(sum * join[0], join[1], join[2]);
           if (STATS) v[j] += mask[hg][j];
         }
@@ -1571,7 +1607,7 @@ static int k_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int
   const int ng = G > 4 ? 2 : 1;
   const size_t setup = ng == 2 ? sizeof(KSetup<2>) : sizeof(KSetup<1>);
   const int tile_lds = 16 * (k_tile_pieces(sub2) + k_tile_pieces(sub4) + k_tile_pieces(n8)) + 128;
-  if (dense && sub2 <= 32 && sub4 <= 64 && n8 <= 128 && setup + tile_lds <= 64 * 1024) {
+  if (dense && sub2 <= 32 && sub4 <= 64 && n8 <= 128 && setup + tile_lds <= kKMaxLds) {
     // Workgroups per KV head: a tile each where all are resident at once (or LDS has no room for two tiles), else
     // an even share of the tiles, the next one's rows loaded under the current one.
     const int64_t cus = compute_units();
@@ -1583,12 +1619,12 @@ static int k_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int
     // (the workgroups of the appended keys come first; what walks the tiles fills the rest of the device)
     const int64_t beside = stats ? stats->new_groups : 0;
     auto resident = [&](size_t lds) {
-      const int64_t all = std::max<int64_t>(1, std::min<int64_t>(kKResident, (160 * 1024) / (int64_t)(lds + 512)) * cus / H_kv);
+      const int64_t all = std::max<int64_t>(1, std::min<int64_t>(kKResident, kKMaxLds / (int64_t)(lds + 512)) * cus / H_kv);
       return std::max(all - beside, (all + 1) / 2);
     };
     size_t staged = setup + tile_lds;
     int64_t wph = tblocks;
-    if (tblocks > resident(staged) && staged + tile_lds <= 64 * 1024) {
+    if (tblocks > resident(staged) && staged + tile_lds <= kKMaxLds) {
       staged += tile_lds;
       wph = rdkv_cdiv(tblocks, rdkv_cdiv(tblocks, resident(staged)));
     }
@@ -1598,11 +1634,17 @@ static int k_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int
       wph += beside;
     }
 #define RDKV_LAUNCH_K_MFMA(NG_, CPT_, STATS_)                                                                      \
-  for (int g0 = 0; g0 < G; g0 += 4 * NG_)                                                                          \
-  hipLaunchKernelGGL((k_qk_dot_mfma_kernel<NG_, CPT_, STATS_>), dim3((unsigned)wph, H_kv), dim3(256), staged, s,   \
+  do {                                                                                                             \
+    if (staged > 64 * 1024)                                                                                        \
+      RDKV_REQUIRE(hipFuncSetAttribute(reinterpret_cast<const void *>(k_qk_dot_mfma_kernel<NG_, CPT_, STATS_>),    \
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, kKMaxLds) == hipSuccess,        \
+                   "rdkv_k_qk_dot: the device refuses %d bytes of LDS per workgroup", (int)staged);                \
+    for (int g0 = 0; g0 < G; g0 += 4 * NG_)                                                                          \
+      hipLaunchKernelGGL((k_qk_dot_mfma_kernel<NG_, CPT_, STATS_>), dim3((unsigned)wph, H_kv), dim3(256), staged, s,   \
                      q, q_dtype, q_stride_h, G, g0, K2, k2_stride_h, K4, k4_stride_h, K8, k8_stride_h,             \
                      (const __half *)scale_f16, (const __half *)zp_f16, ks_stride_h, perm, perm_stride_h, n2p,     \
-                     n4p, n8, T_eff, out, out_stride_h, tile_lds, stats ? *stats : KStats{})
+                     n4p, n8, T_eff, out, out_stride_h, tile_lds, stats ? *stats : KStats{});                      \
+  } while (0)
 #define RDKV_LAUNCH_K_MFMA_S(NG_, CPT_)                                                                            \
   do {                                                                                                             \
     if (stats) RDKV_LAUNCH_K_MFMA(NG_, CPT_, true);                                                                \

@@ -89,6 +89,47 @@ def test_queries_of_any_size(q_scale):
     _check(t2n(kk.k_mixed_qk_dot(torch.from_numpy(q).to(DEV), layer, 500)), terms, centred, (20, 22, 9))
 
 
+@pytest.mark.parametrize("G", [4, 9])
+@pytest.mark.parametrize("width", [2, 4, 8])
+@pytest.mark.parametrize("extreme,n_ext,q_up", [(64, 1, 1), (512, 1, 8), (4096, 1, 8), (4096, 47, 1), (30000, 20, 8)])
+def test_channels_far_below_the_largest(extreme, n_ext, q_up, width, G):
+    """One token is extreme in some channels, which widens their scales; every other token lies at their zero
+    points and its score is the small channels' alone.  Per token: the fp32 products q * scale (2^-24 of each), the
+    join of the digits (2^-24 of the part below the upper two) and two roundings of the score; 2^-47 of the
+    head's largest (times its width's power of two) for what lies below the last digit, per channel and code."""
+    require_gpu()
+    H, T, n = 2, 520, 64
+    rng = np.random.default_rng(extreme + n_ext + width)
+    k = rng.standard_normal((H, T, n))
+    k[:, 0, :n_ext] *= extreme
+    top = (1 << width) - 1
+    lo, hi = k.min(axis=1, keepdims=True), k.max(axis=1, keepdims=True)
+    scale = ((hi - lo) / top).astype(np.float16).astype(float)
+    zp = np.clip(np.rint(-lo / scale), 0, top)
+    codes = np.clip(np.rint(k / scale) + zp, 0, top).astype(np.uint8)
+    counts = [0, 0, 0]
+    counts[(2, 4, 8).index(width)] = n
+    layer, q, _, _ = _layer(*counts, H, T, G, seed=3)
+    perm = t2n(layer.K_ch_perm_padded_idx_for_Q)
+    perm[:] = rng.permutation(128)[:n]
+    q[:, perm[0, :n_ext]] *= q_up
+    per, sub = 8 // width, n * width // 8
+    rows = sum(codes[..., i * sub:(i + 1) * sub].astype(np.uint8) << (width * i) for i in range(per)).astype(np.uint8)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)   # noqa: E731
+    setattr(layer, f"K_{width}bit", dev(rows))
+    layer.K_ch_scale, layer.K_ch_zp = dev(scale.astype(np.float16)), dev(zp.astype(np.float16))
+    layer.K_ch_perm_padded_idx_for_Q = dev(perm)
+    got = t2n(kk.k_mixed_qk_dot(dev(q), layer, T)).astype(float).reshape(H, G, T)
+    terms = np.take_along_axis(q.astype(float), perm, axis=1).reshape(H, G, n) * scale
+    centred = codes.astype(float) - zp
+    parts = np.einsum("hgc,htc->hgt", np.abs(terms), np.abs(centred)) / np.sqrt(128.0)
+    exp = np.einsum("hgc,htc->hgt", terms, centred) / np.sqrt(128.0)
+    below = np.abs(terms).max(axis=2) * n * 2.0 ** -47 * 255
+    tol = 3 * 2.0 ** -24 * np.abs(exp) + 2 * 2.0 ** -24 * parts + below[..., None]
+    err = np.abs(got - exp)
+    assert (err <= tol).all(), float((err / tol).max())
+
+
 def test_zero_points_outside_the_codes_and_unused_channels():
     require_gpu()
     for kw in ({"odd_zero_points": True}, {"unused": 7}, {"unused": 300}):
