@@ -413,19 +413,15 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
   const int r = lane & 15, grp = lane >> 4;
   // the mask values of a lane's four tokens and NG heads
   auto load_mask = [&](int tile) __attribute__((always_inline)) {
-    const int64_t t = (int64_t)tile * 256 + wave * 64 + 4 * r;
+    const int64_t t = (int64_t)tile * 256 + wave * 64 + r;
 #pragma unroll
     for (int hg = 0; hg < NG; ++hg) mask_next[hg] = floatx4{0.f, 0.f, 0.f, 0.f};
     if (!st.mask) return;
 #pragma unroll
     for (int hg = 0; hg < NG; ++hg) {
       const float *row = st.mask + (int64_t)(hkv * G + min(g0 + 4 * hg + grp, G - 1)) * st.mask_sh;
-      if ((int64_t)tile * 256 + 256 <= T) {
-        mask_next[hg] = *reinterpret_cast<const floatx4_a4 *>(row + t);
-      } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) mask_next[hg][i] = row[min(t + i, T - 1)];
-      }
+      for (int i = 0; i < 4; ++i) mask_next[hg][i] = row[min(t + 16 * i, T - 1)];
     }
   };
   float m_run[NG], l_run[NG];
@@ -576,7 +572,10 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     }
   }
 
-  // ---- tiles: a wavefront's 64 tokens are four products of sixteen, lane r of product j token 4 r + j ------
+  // ---- tiles: a wavefront's 64 tokens are four products of sixteen, lane r of product j token r + 16 j ------
+  // (Sixteen lanes then read rows that lie one row apart.  Four apart, with one 16-byte store a lane for its four
+  // tokens, rows of whole 32 or 64 bytes put them on two or four LDS banks: the scores of 8 KV heads x 128k, 96
+  // 8-bit channels, 48.6 us, now 26.3; 64 of 8 and 64 of 4 bit 40.4 / 28.0; 128 of 4 bit 36.8 / 26.1.)
   for (int buffer = 0;; buffer ^= 1) {
     __builtin_amdgcn_s_waitcnt(0x0f70);      // vmcnt(0): this wavefront's pieces are in LDS
     __syncthreads();                         // all are; and every wavefront has done with the other buffer
@@ -592,7 +591,7 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     if (more) issue_rows(next, buffer ^ 1);
     const int64_t t0 = (int64_t)tile * 256;
     const int ntok = T - t0 < 256 ? (int)(T - t0) : 256;
-    const int tok = wave * 64 + 4 * r;
+    const int tok = wave * 64 + r;
     intx4 acc[4][NG], acc_low[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -615,7 +614,7 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
           for (int hg = 0; hg < NG; ++hg) high[hg] = digits(b, hg);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
-            const int off = base[w] + j * rowb[w] + (b & 1) * 16 * nd;
+            const int off = base[w] + 16 * j * rowb[w] + (b & 1) * 16 * nd;
             const uint32_t *W = lds32 + (off >> 2);
             const uint32_t sh = (uint32_t)off & 3u;
             uint32_t raw[5], d[4];
@@ -660,20 +659,16 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
         if (STATS) {
           float to = m_run[hg];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) to = tok + j < ntok ? fmaxf(to, v[j]) : to;
+          for (int j = 0; j < 4; ++j) to = tok + 16 * j < ntok ? fmaxf(to, v[j]) : to;
           softmax_rebase(m_run[hg], l_run[hg], to);
           m_run[hg] = to;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) l_run[hg] += tok + j < ntok ? __expf(v[j] - softmax_at(to)) : 0.0f;
+          for (int j = 0; j < 4; ++j) l_run[hg] += tok + 16 * j < ntok ? __expf(v[j] - softmax_at(to)) : 0.0f;
         }
         float *dst = out + (int64_t)(hkv * G + g) * out_sh + t0 + tok;
-        if (tok + 3 < ntok) {
-          *reinterpret_cast<floatx4_a4 *>(dst) = v;
-        } else {
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (tok + i < ntok) dst[i] = v[i];
-        }
+        for (int i = 0; i < 4; ++i)
+          if (tok + 16 * i < ntok) dst[16 * i] = v[i];
       }
     }
     if (!more) break;
@@ -1608,8 +1603,10 @@ static int k_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int
   const size_t setup = ng == 2 ? sizeof(KSetup<2>) : sizeof(KSetup<1>);
   const int tile_lds = 16 * (k_tile_pieces(sub2) + k_tile_pieces(sub4) + k_tile_pieces(n8)) + 128;
   if (dense && sub2 <= 32 && sub4 <= 64 && n8 <= 128 && setup + tile_lds <= kKMaxLds) {
-    // Workgroups per KV head: a tile each where all are resident at once (or LDS has no room for two tiles), else
-    // an even share of the tiles, the next one's rows loaded under the current one.
+    // Workgroups per KV head: a tile each where all are resident at once, else an even share of the tiles, the next
+    // one's rows loaded under the current one.  (Also where two tiles leave room for two workgroups a compute unit
+    // only: 8 KV heads x 128k, 128 channels of 8 bit 48.9 us, with a tile and its set-up a workgroup, three
+    // resident, 62.7; 64 of each width 31.6 and 62.4; 64 + 80 + 120 58.3 and 72.9.)
     const int64_t cus = compute_units();
     if (stats && stats->n_new > 0) {
       const int64_t passes = rdkv_cdiv(stats->n_new, kKNewKeys), per = rdkv_cdiv(passes, kKNewGroups);

@@ -82,6 +82,20 @@ def test_more_tiles_than_are_resident(H, T, dtype, G):
     _check(t2n(kk.k_mixed_qk_dot(qd.to(DEV), layer, T)), terms, centred, (8, 6, 3))
 
 
+@pytest.mark.parametrize("counts", [(0, 0, 96), (0, 0, 128), (64, 64, 64), (128, 128, 128)])
+@pytest.mark.parametrize("H,T,G", [(8, 33001, 8), (1, 270000, 4)])
+def test_wide_rows_over_more_tiles_than_are_resident(counts, H, T, G):
+    """Two tiles of up to 57 KB a workgroup; the last of them of 233 and 176 tokens."""
+    require_gpu()
+    layer, q, terms, centred = _layer(*counts, 1, T, G, seed=sum(counts))
+    many = SimpleNamespace(**{k: v.expand(H, *v.shape[1:]).contiguous() if torch.is_tensor(v) and k != "K_ch_perm_padded_idx_for_Q"
+                              else v for k, v in vars(layer).items()})
+    many.K_ch_perm_padded_idx_for_Q = layer.K_ch_perm_padded_idx_for_Q.repeat(H, 1)
+    got = t2n(kk.k_mixed_qk_dot(torch.from_numpy(q).repeat(H, 1).to(DEV), many, T)).reshape(H, G, T)
+    _check(got[:1], terms, centred, counts)
+    assert (got == got[:1]).all()
+
+
 @pytest.mark.parametrize("q_scale", [1e-30, 1e-6, 1e6, 1e30])
 def test_queries_of_any_size(q_scale):
     require_gpu()
