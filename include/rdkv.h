@@ -226,8 +226,9 @@ int rdkv_softmax_rows_new_keys(const float *scores_old, int64_t so_stride_h, con
 /* The scores of rows [packed | appended keys] in one call, T_old > 0: scores[hq, t] = rdkv_k_qk_dot + mask for
  * t < T_old, then the appended keys' as rdkv_softmax_rows_new_keys forms them.  *n_pairs > 0: the rows hold
  * scores, and `workspace` (rdkv_attn_scores_workspace_bytes(H_q) bytes) their softmax as that many partial
- * {maximum, sum of exp} pairs a row, for rdkv_v_weighted_sum_scores.  *n_pairs == 0 (K rows not stored back to
- * back, no kept channels): the rows hold the weights. */
+ * {maximum, sum of exp} pairs a row, for rdkv_v_weighted_sum_scores.  *n_pairs == 0: the rows hold the weights.
+ * That is so where the K rows are not stored back to back, are longer than 32, 64 or 128 bytes in their 2-, 4- or
+ * 8-bit part, or have no kept channels; a caller looks at *n_pairs after every call. */
 int64_t rdkv_attn_scores_workspace_bytes(int H_q);
 int rdkv_attn_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int H_kv,
                      const uint8_t *K2, int64_t k2_stride_h, int64_t k2_stride_t,

@@ -232,13 +232,18 @@ struct KStats {
 
 constexpr int kKNewKeys = 64;      // appended keys of a pass of a workgroup: two for each eight lanes
 constexpr int kKNewGroups = 128;   // workgroups of a KV head that take appended keys, at most
-constexpr int kKMaxPairs = 1024 + kKNewGroups;
+constexpr int kKMaxPairs = 1024 + kKNewGroups;   // what a row's softmax comes in, at most
+constexpr int kKMaxSub2 = 32, kKMaxSub4 = 64, kKMaxSub8 = 128;   // bytes of a row by width: two blocks each
 
 constexpr int kKMaxLds = 160 * 1024;   // LDS of a compute unit, and of a workgroup at most
 constexpr int kKResident = 4;      // workgroups per compute unit (wavefronts per SIMD) the kernel is compiled for
 
 // 16-byte pieces of a tile of 256 rows of `sub` bytes that may start and end anywhere in a piece.
 constexpr int k_tile_pieces(int sub) { return sub ? (256 * sub + 30) / 16 : 0; }
+constexpr int k_tile_lds(int sub2, int sub4, int sub8) {
+  return 16 * (k_tile_pieces(sub2) + k_tile_pieces(sub4) + k_tile_pieces(sub8)) + 128;
+}
+static_assert(sizeof(KSetup<2>) + 2 * k_tile_lds(kKMaxSub2, kKMaxSub4, kKMaxSub8) <= kKMaxLds, "two tiles of any row fit");
 
 // One pair per query head of a workgroup from its wavefronts' (su.big: maxima, su.rest: sums).
 template <int NG>
@@ -1566,7 +1571,7 @@ v_reduce_kernel(const float *__restrict__ partial, int H_q, float *__restrict__ 
 }  // namespace
 
 // stats (or null): mask and appended keys of a launch that leaves the rows' softmax in pairs; *n_pairs of them a
-// row, 0 where the scores of the packed keys are all that was formed.
+// row, 0 where the rows are not for the int8 products and the scores of the packed keys are all that was formed.
 static int k_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int H_kv, const uint8_t *K2,
                     int64_t k2_stride_h, int64_t k2_stride_t, const uint8_t *K4, int64_t k4_stride_h, int64_t k4_stride_t,
                     const uint8_t *K8, int64_t k8_stride_h, int64_t k8_stride_t, const void *scale_f16, const void *zp_f16,
@@ -1601,8 +1606,8 @@ static int k_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int
   const int G = H_q / H_kv;
   const int ng = G > 4 ? 2 : 1;
   const size_t setup = ng == 2 ? sizeof(KSetup<2>) : sizeof(KSetup<1>);
-  const int tile_lds = 16 * (k_tile_pieces(sub2) + k_tile_pieces(sub4) + k_tile_pieces(n8)) + 128;
-  if (dense && sub2 <= 32 && sub4 <= 64 && n8 <= 128 && setup + tile_lds <= kKMaxLds) {
+  const int tile_lds = k_tile_lds(sub2, sub4, n8);
+  if (dense && sub2 <= kKMaxSub2 && sub4 <= kKMaxSub4 && n8 <= kKMaxSub8) {
     // Workgroups per KV head: a tile each where all are resident at once, else an even share of the tiles, the next
     // one's rows loaded under the current one.  (Also where two tiles leave room for two workgroups a compute unit
     // only: 8 KV heads x 128k, 128 channels of 8 bit 48.9 us, with a tile and its set-up a workgroup, three
@@ -1613,23 +1618,22 @@ static int k_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int
       stats->per_group = (int)std::min<int64_t>(per * kKNewKeys, 0x7fffffc0);
       stats->new_groups = (int)rdkv_cdiv(passes, per);
     }
-    // (the workgroups of the appended keys come first; what walks the tiles fills the rest of the device)
+    // (the workgroups of the appended keys come first; what walks the tiles fills the rest of the device, as far as
+    // there are pairs for it: all of it up to 256 compute units)
     const int64_t beside = stats ? stats->new_groups : 0;
     auto resident = [&](size_t lds) {
       const int64_t all = std::max<int64_t>(1, std::min<int64_t>(kKResident, kKMaxLds / (int64_t)(lds + 512)) * cus / H_kv);
-      return std::max(all - beside, (all + 1) / 2);
+      const int64_t walkers = std::max(all - beside, (all + 1) / 2);
+      return stats ? std::min<int64_t>(walkers, kKMaxPairs - beside) : walkers;
     };
     size_t staged = setup + tile_lds;
     int64_t wph = tblocks;
-    if (tblocks > resident(staged) && staged + tile_lds <= kKMaxLds) {
+    if (tblocks > resident(staged)) {
       staged += tile_lds;
       wph = rdkv_cdiv(tblocks, rdkv_cdiv(tblocks, resident(staged)));
     }
-    if (wph + beside > kKMaxPairs) stats = nullptr;    // (single tiles of very wide rows: the softmax is a launch of its own)
-    if (stats) {
-      *n_pairs = (int)(wph + beside);
-      wph += beside;
-    }
+    wph += beside;
+    if (stats) *n_pairs = (int)wph;
 #define RDKV_LAUNCH_K_MFMA(NG_, CPT_, STATS_)                                                                      \
   do {                                                                                                             \
     if (staged > 64 * 1024)                                                                                        \

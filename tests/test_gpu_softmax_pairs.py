@@ -91,6 +91,27 @@ def test_rows_in_pairs(monkeypatch, H, T, G, n_new, kept, dtype, mask):
     assert torch.equal(out, again)
 
 
+def test_wide_keys_come_in_pairs_at_any_length(monkeypatch):
+    """One KV head whose tiles are resident at once only in part, every channel 8 bits wide."""
+    require_gpu()
+    g = torch.Generator().manual_seed(8)
+    T, n_new = 300_001, 900
+    K, V = (torch.randn(1, 1, T, 128, generator=g).half().to(DEV) for _ in range(2))
+    layer, v16 = packing.pack_layer_per_head(K, V, torch.tensor([2, 4, 8, 16])[torch.randint(0, 4, (1, T), generator=g)],
+                                             torch.full((1, 128), 8), 4)
+    layer, v16 = fast_decode._pre_squeeze_packed((layer,))[0], v16[0].contiguous()
+    q = torch.randn(4, 128, generator=g).to(DEV)
+    kn, vn = (torch.randn(1, n_new, 128, generator=g).to(DEV) for _ in range(2))
+    w, exp = _separately(q, layer, v16, kn, vn, 4)
+    seen = _pairs(monkeypatch)
+    buf = torch.empty(4, T + n_new, device=DEV)
+    out = fast_decode.trizone_attention(q, layer, v16, layer.n_v16_per_head, kn, vn, 4, scores_buf=buf)
+    assert len(seen) == 1 and seen[0] > 0
+    np.testing.assert_allclose(t2n(buf), t2n(w), rtol=1e-5, atol=1e-12)
+    err = (out.double() - exp.double()).norm() / exp.double().norm()      # (sums of the same fp32 terms in another order)
+    assert float(err) < 2e-6, float(err)
+
+
 @pytest.mark.parametrize("G", [4, 6])
 @pytest.mark.parametrize("what", ["row -inf", "all -inf", "new inf", "nan", "inf", "lowest", "tile -inf", "tile nan"])
 def test_masked_and_infinite_rows(what, G):
