@@ -104,17 +104,9 @@ k_qk_dot_strided_kernel(const void *__restrict__ q, int q_dtype, int64_t q_strid
   }
 }
 
-typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef floatx4 __attribute__((aligned(4))) floatx4_a4;   // a 16-byte load from any float
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ half4_t mk_op(uint32_t a, uint32_t b) {
-  union { uint32_t u[2]; half4_t h; } x;
-  x.u[0] = a;
-  x.u[1] = b;
-  return x.h;
-}
 
 typedef int intx4 __attribute__((ext_vector_type(4)));
 
@@ -1051,30 +1043,30 @@ softmax_rows_split_kernel(const float *__restrict__ so, int64_t so_sh, const flo
 // the wavefronts of a head take its steps in turn, the next step's loads in flight under a step's arithmetic.
 // Eight lanes share four tokens: lane li owns channels 16 li .. + 15 in every class (in a 2- or 4-bit row
 // these are one field of sixteen bytes), 16 bytes of each token per load (fp16: two).
-// The sums run on v_mfma_f32_4x4x4_16b_f16 (16 blocks of 4 heads x 4 tokens x 4 channels):
-// * values: the codes of two tokens, one byte permute and one multiply-add per pair.  An integer below 256
-//   in an fp16 register is that integer times 2^-24; times 2^15 it is a normal number.  (The matrix cores
-//   take subnormals, but drop bits of their products that normal numbers keep: 3e-6 of the result.)  Half of
-//   the largest code is taken off it and off the zero point: smaller sums that cancel;
-// * weights (times the token's scale): an fp16 pair, value and remainder, after a power of two per head
-//   that puts the largest weight so far at 2^11 .. 2^15: 22 bits of a weight and at least 2^-36 of the largest,
-//   which is what fp32 sums keep of it.  A larger weight rescales the sums (a few times per wavefront).
-// Error against 64 bits over random layers of 1.5k .. 128k tokens: 1.1e-7 .. 2.9e-7 of the result in the 2-norm,
-// with fp32 products and sums of uncentred codes 1.4e-7 .. 5.7e-7.
-// What bounds it: set-up and the latency of a few steps per wavefront at 32k, loads at 128k.  On the vector
-// ALU (a conversion and a multiply-add per head and code, 5.5 instructions against 1.5 and half a matrix
-// instruction) the sum of 8 KV heads x 1.5k / 32k / 128k (low-bit) took 10.4 / 19.3 / 36.0 us with its
-// reduction, now 9.5 / 13.6 / 23.0; eight query heads per KV head, 32k: 24.7, now 20.3 (two workgroups of
-// four heads, eight apart in the launch, so that a die's L2 serves the second; one workgroup for all eight
-// had no registers for a step in flight: 24.9).
-// Weights or values that are not finite take the wavefront's sums again in plain fp32 arithmetic
-// (v_plain_class), for the same infinities and NaNs.
+// The sums run on v_mfma_f32_4x4x1_16b_f32 (16 blocks of 4 heads x 1 token x 4 channels), which rounds as a
+// multiply-add does: the weight (times the token's scale) is the fp32 number itself, a value the code less the
+// middle of its width's range (exact; smaller sums that cancel), the zero point's part of it a sum beside; fp16
+// rows as they are.
+// (Weights as an fp16 pair on v_mfma_f32_4x4x4_16b_f16, four tokens an instruction, are 22 or 23 bits and nothing
+// below 2^-36 of the largest: an fp16 row with a weight near 1 and values near 0 - an attention sink - left the others
+// 2.7e-7, here 1.1e-7.  With a third term, 24 bits, the error still grows with the number of tokens: that
+// instruction cuts off, towards minus infinity, whatever lies below 24 bits of its largest product, 5e-7 over 16000
+// 2-bit tokens of like weight, here 1.4e-7.)
+// Error against 64 bits over random layers of 1k .. 128k tokens: a layer's call 2.2e-7 .. 5.9e-7 of the result in the
+// 2-norm, the sum alone 0.9e-7 .. 2.0e-7; with fp16 pairs 2.1e-7 .. 6.1e-7 and 1.0e-7 .. 2.7e-7, on the vector ALU with
+// uncentred codes 2.4e-7 .. 9.5e-7 and 0.9e-7 .. 1.6e-6.
+// What bounds it: set-up and the latency of a few steps per wavefront at 32k, at 128k the vector instructions (half of
+// the cycles) and the products (a fifth), which overlap only between the two wavefronts of a SIMD.  Us with its
+// reduction of 8 KV heads x 1.5k / 32k / 128k (low-bit): on the vector ALU (a conversion and a multiply-add per head and
+// code) 12.9 / 22.5 / 39.7, with fp16 pairs 11.9 / 19.7 / 29.9, now 13.9 / 20.1 / 34.3; eight query heads per KV head, 32k
+// 28.6 / 29.5 / 30.4 (two workgroups of four heads, eight apart in the launch, so that a die's L2 serves the second; one
+// workgroup for all eight had no registers for a step in flight).
+// Weights and values that are not finite stay in their head and channel, as in plain arithmetic.
 // ---------------------------------------------------------------------------
 constexpr int kVChunks = 64;
 constexpr int kVWaves = 4;
 constexpr int kVParts = kVChunks * kVWaves;   // wavefronts that share a head's steps
 constexpr int kVNew = 8;                      // appended tokens a wavefront takes at a time
-constexpr int kVCodeUnit = 9;                 // codes enter as code * 2^-9
 constexpr int v_step_tokens(int cls) { return cls == 3 ? 32 : 64; }   // tokens of a step: 128 bytes of codes a lane
 
 typedef floatx4 __attribute__((aligned(4))) floatx4_w;
@@ -1130,7 +1122,7 @@ __device__ __forceinline__ void v_load(int cls, const VClass c, const uint16_t *
   }
 }
 
-// The last step of a class: what was read early moves to its place, weights past the end become 0.
+// The last step of a class: what was read early moves to its place, weights (fp16 rows: values too) past the end become 0.
 template <bool WIDE>
 __device__ __forceinline__ void v_tail(const VClass c, int t0, int sub, VTile &L) {
 #pragma unroll
@@ -1149,18 +1141,44 @@ __device__ __forceinline__ void v_tail(const VClass c, int t0, int sub, VTile &L
     for (int r = 1; r <= 3; ++r)
       if (d >= r) w = floatx4{w[1], w[2], w[3], w[3]};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) L.w[a][k] = t + k < c.n ? w[k] : 0.0f;
+    for (int k = 0; k < 4; ++k) {
+      L.w[a][k] = t + k < c.n ? w[k] : 0.0f;
+      if (WIDE && t + k >= c.n) L.raw[2 * k] = L.raw[2 * k + 1] = make_uint4(0u, 0u, 0u, 0u);   // (0 times infinity is not 0)
+    }
   }
 }
 
-// Sums of a wavefront: acc[c][i] is channel 16 li + c of head i over the lane's tokens, in units
-// of 2^unit of that head (every lane keeps the state of head lane % 4).
+// Sums of a wavefront: acc[c][i] is channel 16 li + c of head i over the lane's tokens; zacc, of the lane's own head
+// lane % 4, the sum of weight * scale * (zero point - middle code).
 struct VSums {
   floatx4 acc[16];
-  float zacc;      // sum of weight * scale * zero point of the lane's own head
-  float up, lim;   // the power of two on the weights; the largest weight it is good for
-  int unit;
+  float zacc;
 };
+
+// A step's products, token t of `tokens` by `convert(t, weight, values)`: a token's values are formed under the products
+// of the token before, eight vector instructions to four products (a value that a product waits for costs it two idle
+// cycles and more, at two wavefronts per SIMD; 2, 4, 16 and 30 instructions at a time, or left to the compiler, the sum
+// of 8 KV heads x 128k low-bit takes 0.6 .. 3.8 us more).
+template <int TOKENS, class Convert>
+__device__ __forceinline__ void v_products(VSums &S, Convert convert) {
+  float ws[2], v[2][16];
+  convert(0, ws[0], v[0]);
+#pragma unroll
+  for (int t = 0; t < TOKENS; ++t) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 16; ++c) S.acc[c] = __builtin_amdgcn_mfma_f32_4x4x1f32(ws[t & 1], v[t & 1][c], S.acc[c], 0, 0, 0);
+    if (t + 1 < TOKENS) {
+      convert(t + 1, ws[(t + 1) & 1], v[(t + 1) & 1]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x2, 8, 0);      // vector instructions
+        __builtin_amdgcn_sched_group_barrier(0x8, 4, 0);      // matrix instructions
+      }
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
 
 template <int I>
 __device__ __forceinline__ float v_quad_lane(float v) { return rdkv_dpp_mov<0x55 * I>(v); }
@@ -1168,87 +1186,42 @@ __device__ __forceinline__ float v_quad_value(float v, int i) {   // (i is a con
   return i == 0 ? v_quad_lane<0>(v) : i == 1 ? v_quad_lane<1>(v) : i == 2 ? v_quad_lane<2>(v) : v_quad_lane<3>(v);
 }
 
-// New scaling for the heads whose weights have outgrown theirs; base: the unit of the values (a power of
-// two).  Never so fine that a sum in hand would leave its range (40 bits below its unit is nothing to it); at
-// 2^126 an fp16 remainder still reaches below the smallest fp32 number.
-__device__ __forceinline__ void v_rescale(VSums &S, float mx, int base) {
-  mx = fmaxf(mx, rdkv_dpp_mov<0x124>(mx));
-  mx = fmaxf(mx, rdkv_dpp_mov<0x128>(mx));
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));          // the head's largest
-  float f = 1.0f;
-  if (mx > S.lim) {
-    const int x = (int)(__float_as_uint(mx) >> 23) - 126;            // mx = m * 2^x, 0.5 <= m < 1
-    const int e = min(min(max(12 - x, -100), 126), base - S.unit + 40);
-    f = ldexpf(1.0f, S.unit - (base - e));
-    S.unit = base - e;
-    S.up = __uint_as_float((uint32_t)(127 + e) << 23);
-    S.lim = ldexpf(1.0f, 15 - e);
-  }
-  float fi[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) fi[i] = v_quad_value(f, i);
-#pragma unroll
-  for (int c = 0; c < 16; ++c)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) S.acc[c][i] *= fi[i];
-}
-
 // The widths share one body (shift and mask at run time): a body each made a small call wait for their
 // instructions (1.5k tokens: 11.9 us of V, not 9.5).
-template <bool WIDE>
 __device__ __forceinline__ void v_step(const VTile &L, int cls, int li, VSums &S) {
-  constexpr int kDwords = WIDE ? 8 : 4, kValues = 16 / kDwords;
-  const float mid = cls == 0 ? 1.5f : cls == 1 ? 7.5f : 127.5f;       // half of the largest code
-  const _Float16 mid16 = (_Float16)(mid * (1.0f / 512.0f));
-  const int shift = cls == 0 ? 2 * (li >> 1) : cls == 1 ? 4 * (li >> 2) : 0;    // field inside each byte
-  const uint32_t mask = cls == 0 ? 0x03030303u : cls == 1 ? 0x0F0F0F0Fu : 0xFFFFFFFFu;
-  float mx = 0.0f;
+  // a code's field goes to the top of its byte, top bit flipped, and half of the field's unit under it: as a signed
+  // byte the code less the middle of its range, times 2^6, 2^4 or 1, which the weights carry the other way
+  const int shift = cls == 0 ? 6 - 2 * (li >> 1) : cls == 1 ? 4 - 4 * (li >> 2) : 0;
+  const uint32_t mask = cls == 0 ? 0xC0C0C0C0u : cls == 1 ? 0xF0F0F0F0u : 0xFFFFFFFFu;
+  const uint32_t flip = cls == 0 ? 0xA0A0A0A0u : cls == 1 ? 0x88888888u : 0x80808080u;
+  const float mid = cls == 0 ? 1.5f : cls == 1 ? 7.5f : 128.0f, down = cls == 0 ? 0x1p-6f : cls == 1 ? 0x1p-4f : 1.0f;
+  v_products<8>(S, [&](int t, float &ws, float (&v)[16]) __attribute__((always_inline)) {
+    const uint4 r = L.raw[t];
+    const int a = t >> 2, k = t & 3;
+    ws = L.w[a][k] * rdkv_h2f((uint16_t)(L.s[a] >> (16 * k)));
+    S.zacc = fmaf(ws, rdkv_h2f((uint16_t)(L.z[a] >> (16 * k))) - mid, S.zacc);
+    ws *= down;
 #pragma unroll
-  for (int a = 0; a < (WIDE ? 1 : 2); ++a)
+    for (int q = 0; q < 4; ++q) {
+      const uint32_t f = (((q == 0 ? r.x : q == 1 ? r.y : q == 2 ? r.z : r.w) << shift) & mask) ^ flip;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      mx = fmaxf(mx, fabsf(L.w[a][k] * (WIDE ? 1.0f : rdkv_h2f((uint16_t)(L.s[a] >> (16 * k))))));
-  if (__builtin_amdgcn_ballot_w64(mx > S.lim) != 0) v_rescale(S, mx, WIDE ? 0 : kVCodeUnit);
-#pragma unroll
-  for (int a = 0; a < (WIDE ? 1 : 2); ++a) {
-    half4_t hi, lo;
-    floatx4 ws = L.w[a];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      if (!WIDE) {
-        ws[k] *= rdkv_h2f((uint16_t)(L.s[a] >> (16 * k)));
-        S.zacc += ws[k] * (rdkv_h2f((uint16_t)(L.z[a] >> (16 * k))) - mid);
-      }
-      const float x = ws[k] * S.up;
-      hi[k] = (_Float16)x;
-      lo[k] = (_Float16)(x - (float)hi[k]);
+      for (int j = 0; j < 4; ++j) v[4 * q + j] = (float)(int8_t)(f >> (8 * j));
     }
+  });
+}
+
+// A step of fp16 rows.
+__device__ __forceinline__ void v_step_wide(const VTile &L, VSums &S) {
+  v_products<4>(S, [&](int t, float &ws, float (&v)[16]) __attribute__((always_inline)) {
+    ws = L.w[0][t];
 #pragma unroll
-    for (int q = 0; q < kDwords; ++q) {
-      uint32_t f[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint4 r = WIDE ? L.raw[2 * k + (q >> 2)] : L.raw[4 * a + k];
-        const uint32_t d = (q & 3) == 0 ? r.x : (q & 3) == 1 ? r.y : (q & 3) == 2 ? r.z : r.w;
-        f[k] = WIDE ? d : (d >> shift) & mask;
-      }
-      half4_t b[kValues];
-#pragma unroll
-      for (int j = 0; j < kValues; ++j) {
-        // value j of tokens 0 | 1 and of tokens 2 | 3
-        const uint32_t sel = WIDE ? (j ? 0x07060302u : 0x05040100u) : 0x0c040c00u + 0x00010001u * (uint32_t)j;
-        b[j] = mk_op(__builtin_amdgcn_perm(f[1], f[0], sel), __builtin_amdgcn_perm(f[3], f[2], sel));
-        if (!WIDE) b[j] = b[j] * (_Float16)32768.0f - mid16;
-      }
-#pragma unroll
-      for (int j = 0; j < kValues; ++j)
-        S.acc[kValues * q + j] = __builtin_amdgcn_mfma_f32_4x4x4f16(hi, b[j], S.acc[kValues * q + j], 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < kValues; ++j)
-        S.acc[kValues * q + j] = __builtin_amdgcn_mfma_f32_4x4x4f16(lo, b[j], S.acc[kValues * q + j], 0, 0, 0);
+    for (int q = 0; q < 8; ++q) {
+      const uint4 r = L.raw[2 * t + (q >> 2)];
+      const uint32_t d = (q & 3) == 0 ? r.x : (q & 3) == 1 ? r.y : (q & 3) == 2 ? r.z : r.w;
+      v[2 * q] = rdkv_h2f((uint16_t)d);
+      v[2 * q + 1] = rdkv_h2f((uint16_t)(d >> 16));
     }
-  }
+  });
 }
 
 // The weight of a score; weights that are given are {0, 1, false}.
@@ -1384,9 +1357,7 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
   const float *w0 = w + (int64_t)(hkv * G + g0) * w_sh, *wrow = w0 + (live ? lane & 3 : 0) * w_sh;
   __shared__ float s_acc[kVWaves][4][kD];
   VSums S;
-  S.zacc = S.lim = 0.0f;
-  S.up = 1.0f;
-  S.unit = -1000;      // (nothing summed: any unit will do)
+  S.zacc = 0.0f;
 #pragma unroll
   for (int c = 0; c < 16; ++c) S.acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
   // (weight or scale rows of fewer than four columns: the plain sums below)
@@ -1431,27 +1402,21 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
           for (int k = 0; k < 4; ++k) cur.w[a][k] = weight(cur.w[a][k]);
       }
       if (t0 + v_step_tokens(cls) > c.n) v_tail<WIDE>(c, t0, sub, cur);
-      if (!live) cur.w[0] = cur.w[1] = floatx4{0.f, 0.f, 0.f, 0.f};
-      v_step<WIDE>(cur, cls, li, S);
+      if (WIDE) v_step_wide(cur, S);
+      else v_step(cur, cls, li, S);
       cur = nxt;
       s += kVParts;
     }
   };
   run(std::false_type{}, e2);
-  S.lim = 0.0f;      // (other values, other unit: the sums are rescaled when the first weights come in)
-  run(std::true_type{}, e3);
-  float odd = narrow ? __builtin_nanf("") : 0.0f;
-#pragma unroll
-  for (int c = 0; c < 16; ++c)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) odd = fmaf(S.acc[c][i], 0.0f, odd);
-  const bool plain = __builtin_amdgcn_ballot_w64(!(odd == 0.0f)) != 0;
+  // (an infinite weight makes NaN of the codes' and the zero points' part together, whatever the middle code is)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const float zi = v_quad_value(S.zacc, i), unit = v_quad_value(ldexpf(1.0f, S.unit), i);      // (2^-1000: 0 of 0)
+    const float zi = v_quad_value(fmaf(S.zacc, 0.0f, S.zacc), i);
 #pragma unroll
-    for (int c = 0; c < 16; ++c) S.acc[c][i] = plain ? 0.0f : fmaf(S.acc[c][i], unit, -zi);
+    for (int c = 0; c < 16; ++c) S.acc[c][i] -= zi;
   }
+  run(std::true_type{}, e3);
   // the new zone, fp32: eight tokens at a time, the last wavefronts first (they have the fewest steps)
   if (nv.v) {
     const float *vh = nv.v + hkv * nv.v_sh + 16 * li, *wh = nv.w + (int64_t)(hkv * G + g0 + (live ? lane & 3 : 0)) * nv.w_sh;
@@ -1487,7 +1452,7 @@ v_weighted_sum_kernel(const float *__restrict__ w, int64_t w_sh, int G,
     for (int c = 0; c < 2; ++c) r[c] = (b3 ? b[c + 2] : b[c]) + rdkv_dpp_mov<0x128>(b3 ? b[c] : b[c + 2]);
     *reinterpret_cast<float2 *>(&s_acc[wave][i][ch]) = make_float2(r[0], r[1]);
   }
-  if (plain) {
+  if (narrow) {
 #pragma unroll 1
     for (int g = 0; g < ng; ++g) {
       float acc[16], zacc = 0.0f;

@@ -86,6 +86,74 @@ def test_weights_of_any_size(lo, hi):
     _close(_run(torch.from_numpy(w).to(DEV), case), w, case[4], 4)
 
 
+@pytest.mark.parametrize("width", [2, 4, 8, 16])
+def test_a_weight_is_used_with_all_its_bits(width):
+    """One token counts, of value 1 as code and zero point on the two sides of the middle: its weight is the result."""
+    require_gpu()
+    G, n = 4, 40
+    counts = {2: (n, 0, 0), 4: (0, n, 0), 8: (0, 0, n), 16: (0, 0, 0)}[width]
+    args, seg, counts, kw, dense, _ = _case(counts, n if width == 16 else 0, G, seed=1)
+    seg[1] = seg[0]
+    kw["n_v16_per_head"] = torch.tensor([n if width == 16 else 0] * 2, dtype=torch.int32, device=DEV)
+    if width == 16:
+        kw["V16"][:] = 1.0
+    else:
+        codes = {2: 0xAA, 4: 0x88, 8: 0x81}[width]           # code 2, 8, 129 in every field
+        args[(2, 4, 8).index(width)].fill_(codes)
+        args[3].fill_(1.0)
+        args[4].fill_({2: 1.0, 4: 7.0, 8: 128.0}[width])
+    w = np.zeros((2 * G, n), dtype=np.float32)
+    rng = np.random.default_rng(width)
+    for trial in range(20):
+        w[:] = 0
+        at = rng.integers(0, n, 2 * G)
+        value = (rng.random(2 * G) * 2.0 ** rng.uniform(-60, 20, 2 * G)).astype(np.float32)
+        w[np.arange(2 * G), at] = value
+        got = _run(torch.from_numpy(w).to(DEV), (args, seg, counts, kw, dense, None))
+        assert np.array_equal(got, np.repeat(value[:, None].astype(float), 128, axis=1))
+
+
+def test_small_weights_beside_one_of_no_value():
+    """A sink: the weight of one fp16 row is 2^24 .. 2^40 times the others', its values are zero.  fp32 products and sums
+    of the others: 2^-20 of the products' magnitudes."""
+    require_gpu()
+    case = _case((0, 0, 0), 3000, 4, seed=2)
+    dense, v16 = case[4], case[5]
+    v16[:, 700] = 0
+    dense[:, 700] = 0
+    case[3]["V16"] = torch.from_numpy(v16).to(DEV)
+    rng = np.random.default_rng(3)
+    for e in (24, 32, 40):
+        w = (rng.random((8, 3000)) * 2.0 ** -e).astype(np.float32)
+        w[:, 700] = 1.0
+        got = _run(torch.from_numpy(w).to(DEV), case).reshape(2, 4, 128)
+        w8 = w.astype(float).reshape(2, 4, -1)
+        exp, size = w8 @ dense, w8 @ np.abs(dense)
+        assert (np.abs(got - exp) <= 2.0 ** -20 * size).all(), float((np.abs(got - exp) / size).max())
+
+
+@pytest.mark.parametrize("width", [2, 4, 8, 16])
+def test_many_tokens_of_like_weight(width):
+    """The error grows as roundings do, without a bias: about 64 additions on a result's way, each off by 2^-25 of a
+    partial sum no larger than the results' own size, make sqrt(64) * 2^-25 in the 2-norm; twice that is allowed."""
+    require_gpu()
+    n = 16000
+    counts = {2: (n, 0, 0), 4: (0, n, 0), 8: (0, 0, n), 16: (0, 0, 0)}[width]
+    args, seg, counts, kw, dense, v16 = _case(counts, n if width == 16 else 0, 4, seed=9)
+    if width < 16:         # values around zero, as the quantizer leaves them
+        zp = torch.randint(0, 2, args[4].shape, generator=torch.Generator().manual_seed(4)).half().to(DEV) + (1 << (width - 1)) - 1
+        scale = t2n(args[3]).astype(float)
+        dense = dense + (t2n(args[4]).astype(float) - t2n(zp).astype(float)) * scale
+        dense[1, n // 2:] = 0
+        args = (*args[:4], zp)
+    w = np.random.default_rng(5).uniform(0.5, 1.5, (8, n)).astype(np.float32)
+    got = _run(torch.from_numpy(w).to(DEV), (args, seg, counts, kw, dense, v16)).reshape(2, 4, 128)
+    w8 = w.astype(float).reshape(2, 4, -1)
+    exp = w8 @ dense
+    err = np.linalg.norm(got - exp) / np.linalg.norm(exp)
+    assert err < 2 * 8 * 2.0 ** -25, err
+
+
 def test_infinities_and_nan_stay_where_they_are():
     require_gpu()
     case = _case((100, 100, 100), 200, 4, seed=8)
@@ -99,6 +167,10 @@ def test_infinities_and_nan_stay_where_they_are():
     keep = np.ones((2, 128), dtype=bool)
     keep[0, 5] = keep[0, 6] = keep[1, 100] = False
     assert np.isfinite(got[np.broadcast_to(keep[:, None], got.shape)]).all()
+    for bad in (np.inf, -np.inf):               # (infinity times a code less infinity times a zero point)
+        w[2, 50] = bad
+        got = _run(torch.from_numpy(w).to(DEV), case).reshape(2, 4, 128)
+        assert np.isnan(got[0, 2]).all() and np.isfinite(got[0, [0, 1, 3]][:, 10:]).all()
     w[2, 50], w[5, 320] = np.nan, np.inf        # head 0: a quantized token; head 1: an fp16 one
     got = _run(torch.from_numpy(w).to(DEV), case).reshape(2, 4, 128)
     assert np.isnan(got[0, 2]).all() and np.isfinite(got[0, [0, 1, 3]][:, 10:]).all()
