@@ -176,29 +176,26 @@ __device__ __forceinline__ int k_slot(int width, int p, int j) {
 // less.  64 channels of 8 bit, one with a token 512 / 4096 / 30000 times as large and a query 8 times: error of
 // the others' scores 4.3e-8 / 4.7e-8 / 4.9e-8; with 30 bits alone 1.4e-7 / 1.4e-6 / 1.0e-5, with fp16 pairs in
 // fp32 sums 6.9e-8 / 7.0e-8 / 9.3e-8.  The second product is always formed: a test of how many channels need it
-// has heads on its wrong side, 47 of 64 extreme ones for instance.  It costs 1.4 us of a layer's call at 32k, 2.4 at
-// 128k low-bit.)
+// has heads on its wrong side, 47 of 64 extreme ones for instance.)
 // The codes of the narrow widths enter times 2^5 and 2^3, so that every width's q * scale has a like part of
 // those bits.  The sums start from minus the zero points' part, formed by the same
 // products, so they are sums of the signed values themselves; a lane ends up with the six digits' sums of one
 // token and head and joins them in fp32, one rounding and one of the factor 1 / sqrt(128).  Error against 64
 // bits: 4.0e-8 of the scores in the 2-norm (fp16 pairs in fp32 sums: 4.1e-8 .. 5.2e-8).
-// What bounds it: the chain of the set-up (tables and query, digits, first tile) and the padded rows' loads.
-// With v_mfma_f32_4x4x4_16b_f16 over code - zp as fp16 (7 vector instructions and three table reads from LDS
-// per four codes, here 2 and none, and rows through registers, with 40 scalar instructions and 5 branches a
-// piece) the scores of 8 KV heads x 1.5k / 32k / 128k (low-bit) took 8.1 / 17.7 / 32.6 us, now 6.1 / 11.9 /
-// 16.6; eight query heads per KV head, 32k: 20.9, now 15.3.
+// What bounds it: the chain of the set-up (tables and query, digits, first tile) and the padded rows' loads; at 128k
+// the vector instructions (nine tenths of the cycles).  With v_mfma_f32_4x4x4_16b_f16 over code - zp as fp16 (7 vector
+// instructions and three table reads from LDS per four codes, here 2 and none, and rows through registers, with 40
+// scalar instructions and 5 branches a piece) the scores alone of 8 KV heads x 1.5k / 32k / 128k (low-bit) took 8.8 /
+// 18.6 / 32.5 us, now 7.3 / 13.4 / 17.9 (with 30 bits 6.9 / 12.5 / 16.7); eight query heads per KV head, 32k 21.9, now
+// 17.3 (15.8), 100k 44.5, now 30.7 (28.9).
 // The reference layout pads every head's segments to the widest head's: channels whose stored scale is zero
 // contribute exactly nothing, blocks past a head's last such channel are skipped.
 // CPT = channels per thread (Dp <= 256 CPT).
 // STATS: the launch also forms the scores of the appended keys (its first st.new_groups workgroups of a KV head),
 // adds the mask, and every workgroup leaves its part of a row's softmax, maximum and sum, as a pair, so no
-// launch reads the rows again for them (13.3 us at 32k, 13.4 + 10.1 in two launches at 128k).  With it this
-// launch takes 13.8 us where the scores alone take 13.4, 19.1 for 18.2 at 128k, with eight query heads per KV
-// head 19.8 for 16.9 at 32k and 39 for 30 at 100k; the sum takes 1.2 .. 4 us more.  Error of the weights against 64
-// bits 5.1e-8 .. 6.4e-8 in the 2-norm (a launch of their own: 6.4e-8 .. 1.2e-7).  A layer's call, us: 8 KV heads x
-// 32k 40.0 -> 35.9 (issued one by one; the launches 44 -> 34), 128k low-bit 61.2 -> 47.3, eight heads 32k
-// 50.7 -> 47.2, 100k 96 -> 86.
+// launch reads the rows again for them (13.1 us at 32k, two launches of 11.7 at 128k).  With it this launch takes 8.1
+// us at 1.5k, 15.5 at 32k, 20.6 at 128k, with eight query heads per KV head 20.9 at 32k and 41.8 at 100k (same run as
+// above).  Error of the weights against 64 bits 5.1e-8 .. 6.4e-8 in the 2-norm (a launch of their own: 6.4e-8 .. 1.2e-7).
 // Dynamic LDS: KSetup, then one or two tiles of 16-byte pieces, each with 128 bytes that reads past the
 // last row may touch.
 template <int NG>
@@ -228,7 +225,10 @@ constexpr int kKMaxPairs = 1024 + kKNewGroups;   // what a row's softmax comes i
 constexpr int kKMaxSub2 = 32, kKMaxSub4 = 64, kKMaxSub8 = 128;   // bytes of a row by width: two blocks each
 
 constexpr int kKMaxLds = 160 * 1024;   // LDS of a compute unit, and of a workgroup at most
-constexpr int kKResident = 4;      // workgroups per compute unit (wavefronts per SIMD) the kernel is compiled for
+// Workgroups per compute unit (wavefronts per SIMD) the kernel is compiled for.  Eight heads' digits take 72
+// registers; with four wavefronts they are read from LDS for every tile: 8 KV heads x 100k 42.3 us, now 31.6 (with the
+// softmax 50.3 / 42.4), 128k of 128 4-bit channels 40.2 / 30.2.
+constexpr int k_resident(int ng) { return ng == 1 ? 4 : 3; }
 
 // 16-byte pieces of a tile of 256 rows of `sub` bytes that may start and end anywhere in a piece.
 constexpr int k_tile_pieces(int sub) { return sub ? (256 * sub + 30) / 16 : 0; }
@@ -323,7 +323,7 @@ __device__ __forceinline__ void k_new_keys(KSetup<NG> &su, const float (&qrow)[2
 }
 
 template <int NG, int CPT, bool STATS>
-__global__ void __launch_bounds__(256, kKResident)
+__global__ void __launch_bounds__(256, k_resident(NG))
 k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h, int G, int g0,
                      const uint8_t *__restrict__ K2, int64_t k2_sh, const uint8_t *__restrict__ K4,
                      int64_t k4_sh, const uint8_t *__restrict__ K8, int64_t k8_sh,
@@ -520,12 +520,9 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
             e8 = __builtin_amdgcn_readfirstlane((int)ext[2]);
   const int blocks[3] = {(min(e2, sub2) + 15) >> 4, (min(e4, sub4) + 31) >> 5, (e8 + 63) >> 6};
   lds_barrier();
-  constexpr bool kHeld = NG == 1;      // (eight heads: the digits stay in LDS, as the lower ones do)
-  intx4 dig[kHeld ? kKBlocks : 1][NG], start[NG], start_low{0, 0, 0, 0};
-  auto digits = [&](int b, int hg) __attribute__((always_inline)) {
-    return kHeld ? dig[kHeld ? b : 0][hg] : *reinterpret_cast<const intx4 *>(&su.digit[b][hg][r][16 * grp]);
-  };
-  auto low_digits = [&](int b) __attribute__((always_inline)) {
+  constexpr bool kLowHeld = !STATS;      // (no registers for them beside the softmax: from LDS for every tile)
+  intx4 dig[kKBlocks][NG], low[kLowHeld ? kKBlocks : 1], start[NG], start_low{0, 0, 0, 0};
+  auto low_from_lds = [&](int b) __attribute__((always_inline)) {
     return *reinterpret_cast<const intx4 *>(&su.low[b][r >> 2][r & (2 * NG - 1)][16 * grp]);
   };
 #pragma unroll
@@ -535,11 +532,13 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
     if ((b & 1) < blocks[b >> 1]) {
       intx4 z = *reinterpret_cast<const intx4 *>(&su.zero[b][r & 1][16 * grp]);
       if (r > 1) z = intx4{0, 0, 0, 0};
-      start_low = __builtin_amdgcn_mfma_i32_16x16x64_i8(low_digits(b), z, start_low, 0, 0, 0);
+      const intx4 lower = low_from_lds(b);
+      if (kLowHeld) low[kLowHeld ? b : 0] = lower;
+      start_low = __builtin_amdgcn_mfma_i32_16x16x64_i8(lower, z, start_low, 0, 0, 0);
 #pragma unroll
       for (int hg = 0; hg < NG; ++hg) {
-        if (kHeld) dig[kHeld ? b : 0][hg] = *reinterpret_cast<const intx4 *>(&su.digit[b][hg][r][16 * grp]);
-        start[hg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(digits(b, hg), z, start[hg], 0, 0, 0);
+        dig[b][hg] = *reinterpret_cast<const intx4 *>(&su.digit[b][hg][r][16 * grp]);
+        start[hg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(dig[b][hg], z, start[hg], 0, 0, 0);
       }
     }
   }
@@ -605,10 +604,7 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
       for (int b = 0; b < kKBlocks; ++b) {
         if ((b & 1) < blocks[b >> 1]) {
           const int w = b >> 1, nd = 1 << w;       // dwords a lane takes of a row
-          const intx4 low = low_digits(b);
-          intx4 high[NG];
-#pragma unroll
-          for (int hg = 0; hg < NG; ++hg) high[hg] = digits(b, hg);
+          const intx4 lower = kLowHeld ? low[kLowHeld ? b : 0] : low_from_lds(b);
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             const int off = base[w] + 16 * j * rowb[w] + (b & 1) * 16 * nd;
@@ -631,8 +627,8 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
                             (int)(d[3] ^ 0x80808080u)};
 #pragma unroll
             for (int hg = 0; hg < NG; ++hg)
-              acc[j][hg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(high[hg], codes, acc[j][hg], 0, 0, 0);
-            acc_low[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(low, codes, acc_low[j], 0, 0, 0);
+              acc[j][hg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(dig[b][hg], codes, acc[j][hg], 0, 0, 0);
+            acc_low[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(lower, codes, acc_low[j], 0, 0, 0);
           }
         }
       }
@@ -648,8 +644,8 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
           const intx4 x = acc[j][hg];
           // (the upper two digits' sum as an fp32 number and what it leaves: one rounding that counts)
           const float x3 = (float)x[3], x2 = (float)x[2], head = fmaf(x3, 256.0f, x2), left = fmaf(x3, 256.0f, -head) + x2;
-          const float low = fmaf((float)acc_low[j][2 * hg + 1], 256.0f, (float)acc_low[j][2 * hg]);
-          const float sum = fmaf(head, 65536.0f, fmaf(left, 65536.0f, fmaf((float)x[1], 256.0f, fmaf(low, 0x1p-16f, (float)x[0]))));
+          const float tail = fmaf((float)acc_low[j][2 * hg + 1], 256.0f, (float)acc_low[j][2 * hg]);
+          const float sum = fmaf(head, 65536.0f, fmaf(left, 65536.0f, fmaf((float)x[1], 256.0f, fmaf(tail, 0x1p-16f, (float)x[0]))));
           v[j] = fmaf(sum * join[0], join[1], join[2]);
           if (STATS) v[j] += mask[hg][j];
         }
@@ -1587,7 +1583,7 @@ static int k_scores(const void *q, int q_dtype, int64_t q_stride_h, int H_q, int
     // there are pairs for it: all of it up to 256 compute units)
     const int64_t beside = stats ? stats->new_groups : 0;
     auto resident = [&](size_t lds) {
-      const int64_t all = std::max<int64_t>(1, std::min<int64_t>(kKResident, kKMaxLds / (int64_t)(lds + 512)) * cus / H_kv);
+      const int64_t all = std::max<int64_t>(1, std::min<int64_t>(k_resident(ng), kKMaxLds / (int64_t)(lds + 512)) * cus / H_kv);
       const int64_t walkers = std::max(all - beside, (all + 1) / 2);
       return stats ? std::min<int64_t>(walkers, kKMaxPairs - beside) : walkers;
     };
