@@ -763,7 +763,8 @@ int rdkv_knapsack_batched_value(const float *scores, int64_t stride_b, int B, in
 /* obkv_fast.py:1033-1035: the per-head K budget k_budget_bits / (head_dim * max(kept_h, 1)) as
  * the reference's fp32 tensor expression evaluates it (product, reciprocal, product), from the
  * per-option token counts of rdkv_knapsack_batched: kept_h = T - counts[h][zero_option]
- * (zero_option < 0: every token is kept).  out: fp32 [rows] on the device. */
+ * (zero_option < 0: every token is kept).  out: fp32 [rows] on the device.  For callers that look at the
+ * budgets themselves: rdkv_knapsack_batched_value forms the same ones where it uses them. */
 int rdkv_k_budget_per_head(const int32_t *counts, int n_options, int zero_option, int rows, int64_t T,
                            int head_dim, float k_budget_bits, float *out, void *stream);
 

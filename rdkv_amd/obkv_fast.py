@@ -18,7 +18,7 @@ from torch import Tensor
 from . import _lib
 from .knapsack_solver import (DEFAULT_EPSILON_K, DEFAULT_EPSILON_V, KeptBudget, knapsack_allocate,   # noqa: F401 (re-exported
                               knapsack_bit_allocation_batched, load_epsilon_kv_from_calibration)  # as obkv_fast.py:38-46 does)
-from .packing import _pack_layer_per_head, pack_layer_per_head, pack_layers_per_head  # noqa: F401
+from .packing import _pack_layer_per_head, pack_layer_per_head, pack_layers_per_head  # noqa: F401 (its public name stays here)
 
 
 def apply_score_pooling(scores: Tensor, pool_type: str, kernel_size: int, padding_mode: str = "zero") -> Tensor:
@@ -82,20 +82,20 @@ def _score_one_layer(aw: Tensor, q: Tensor, o, v: Tensor, head_dim: int, v_score
     return token, channel
 
 
-def _allocate_k_bits_per_head(channel_scores: Tensor, k_avg: Union[float, Tensor], *, epsilon,
-                              bit_options) -> Tensor:
-    """obkv_fast.py:579-618: ``[H_kv, D]`` channel scores, a shared float budget or one per head;
-    one batched solve.  Returns ``[H_kv, D]`` long."""
+def _allocate_k_bits_per_head(channel_scores: Tensor, k_avg: Union[float, Tensor, KeptBudget], *, epsilon,
+                              bit_options, out_dtype=torch.int64) -> Tensor:
+    """obkv_fast.py:579-618: ``[H_kv, D]`` channel scores, a shared float budget or one per head (or the counts it
+    comes from, ``_k_budget_per_head``); one batched solve.  Returns ``[H_kv, D]`` long (uint8 on request)."""
     assert channel_scores.dim() == 2, (
         f"_allocate_k_bits_per_head expects [H_kv, D]; got {tuple(channel_scores.shape)}")
     H_kv = int(channel_scores.shape[0])
     if torch.is_tensor(k_avg):
         assert k_avg.dim() == 1 and int(k_avg.shape[0]) == H_kv, (
             f"k_avg tensor must be [H_kv={H_kv}]; got {tuple(k_avg.shape)}")
-        k_avg_arg: Union[float, Tensor] = k_avg.detach().float()
+        k_avg_arg: Union[float, Tensor, KeptBudget] = k_avg.detach().float()
     else:
-        k_avg_arg = float(k_avg)
-    return knapsack_bit_allocation_batched(channel_scores, k_avg_arg, epsilon=epsilon, bit_options=bit_options)
+        k_avg_arg = k_avg if isinstance(k_avg, KeptBudget) else float(k_avg)
+    return knapsack_allocate(channel_scores, k_avg_arg, epsilon, bit_options=bit_options, out_dtype=out_dtype)
 
 
 def _k_budget_per_head(v_counts: Tensor, v_bit_options: Optional[Tensor], T: int, head_dim: int,
@@ -155,8 +155,8 @@ def _perhead_select_and_pack_joint(
     t_v = stamp()
 
     k_avg_per_head = _k_budget_per_head(v_counts, v_bit_options, T, head_dim, k_budget_bits)
-    k_bits_perhead = knapsack_allocate(channel_scores.float().to(dev), k_avg_per_head, epsilon=eps_K,
-                                       bit_options=k_bit_options)
+    k_bits_perhead = _allocate_k_bits_per_head(channel_scores.float().to(dev), k_avg_per_head, epsilon=eps_K,
+                                               bit_options=k_bit_options, out_dtype=torch.uint8)
     t_k = stamp()
 
     retained: list = []

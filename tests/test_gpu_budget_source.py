@@ -3,7 +3,7 @@ against the same budgets as a tensor: every form of the solver, heads that keep 
 import pytest
 import torch
 
-from rdkv_amd import _lib, knapsack_solver as ks
+from rdkv_amd import _lib, knapsack_solver as ks, obkv_fast
 from tests.gpu_util import DEV, require_gpu
 
 pytestmark = pytest.mark.gpu
@@ -44,6 +44,23 @@ def test_budget_from_counts(B, T, zero_col):
     exp = ks.knapsack_allocate(s, tensor, ks.DEFAULT_EPSILON_K, group_rows=B)
     got = ks.knapsack_allocate(s, ks.KeptBudget(counts, zero_col, tokens, D, bits), ks.DEFAULT_EPSILON_K, group_rows=B)
     assert torch.equal(got, exp)
+
+
+def test_a_heads_allocation_takes_every_kind_of_budget():
+    """One value, a tensor, or what ``_k_budget_per_head`` makes of a V allocation's counts."""
+    require_gpu()
+    s = _scores(8, 128)
+    counts = torch.tensor([[h * 100, 0, 0, 0, 900 - h * 100] for h in range(8)], dtype=torch.int32, device=DEV)
+    budget = obkv_fast._k_budget_per_head(counts, None, 900, 128, 900 * 128 * 1.5)
+    tensor = 900 * 128 * 1.5 / (128 * (900 - counts[:, 0]).float())
+    kw = dict(epsilon=ks.DEFAULT_EPSILON_K, bit_options=torch.tensor([0.0, 2.0, 4.0, 8.0]))
+    exp = obkv_fast._allocate_k_bits_per_head(s, tensor, **kw)
+    got = obkv_fast._allocate_k_bits_per_head(s, budget, **kw)
+    assert got.dtype == exp.dtype == torch.int64 and torch.equal(got, exp)
+    narrow = obkv_fast._allocate_k_bits_per_head(s, budget, out_dtype=torch.uint8, **kw)
+    assert narrow.dtype == torch.uint8 and torch.equal(narrow.long(), exp)
+    assert torch.equal(obkv_fast._allocate_k_bits_per_head(s, 1.5, **kw),
+                       obkv_fast._allocate_k_bits_per_head(s, torch.full((8,), 1.5, device=DEV), **kw))
 
 
 def test_counts_that_do_not_fit_are_refused():
