@@ -705,7 +705,9 @@ static void finish_work(RdkvUnit *units, int U, int multi_source, RdkvWork *work
 // other, 4 us more than one of the same number of tiles, and every workgroup waits for the slowest: 8 units of
 // 4k / 16k / 32k tokens, a decode step 19.4 / 19.5 / 22.5 us with a boundary inside some workgroups, 15.1 / 16.6 /
 // 19.4 without; 256 units of 2k tokens 37.1 / 26.8.
-constexpr int kMaxRuns = 96;      // (the merge takes up to 128 partials of a row in one pass)
+// (The merge takes up to 128 partials of a row in one pass: a row of several sources may have more, each of its units
+// up to kMaxRuns; work_count of its first unit says how many, for the caller to decide.)
+constexpr int kMaxRuns = 96;
 RDKV_API int rdkv_stream_partition_units(RdkvUnit *units, int n_units, int n_items, const double *cost_tile,
                                          double cost_k_dword, int multi_source, RdkvWork *work, int work_capacity,
                                          int *n_work, double *costs) {

@@ -623,6 +623,27 @@ def _partition_whole_units(units_np: np.ndarray, n_items: int, cost: dict, multi
     return (units_np, work_np[:n], np.arange(n + 1, dtype=np.int32)), float(costs[0]), float(costs[1])
 
 
+MERGE_PASS = 128             # partials of an output row that a merge takes in one pass
+
+
+def _whole_units(units_np: np.ndarray, total_tiles: int, n_groups: int, cus: int, model: dict, multi_source: bool):
+    """The partition of a cache of no more units than compute units into runs that keep to one unit; None where they
+    come out more uneven than the second item of a workgroup costs in ``n_groups`` runs across units, or where the
+    sources of an output row make more partials together than its merge takes in one pass (a unit alone has at most 96).
+
+    A step costs a * tiles / runs + b * runs / rows (the partials a row's merge reads), least at runs ~
+    sqrt(tiles * rows); measured with 32 / 64 / 96 / 128 / 192 / 256 runs: 8 units of 4k tokens 17.4 / 15.9 / 15.1 /
+    15.1 / 15.5 / 15.9 us, of 16k 27.4 / 21.0 / 18.4 / 17.5 / 16.8 / 16.9; 2 of 4k 14.9 / 15.6 / 16.1 / 16.8, 4 of 32k 26.7 /
+    21.3 / 19.0 / 18.4 / 18.2 / 18.6 (in runs across units 19.4, 19.5, 19.1, 19.8).  More than one per compute unit: 23.7
+    against 14.9.  64 units of 32k tokens, four runs each, are uneven: 58.2 us against 56.6."""
+    n_rows = len(np.unique(units_np["q_row"])) if multi_source else len(units_np)
+    whole, longest, total = _partition_whole_units(
+        units_np, min(cus, int(round((5.3 * total_tiles * n_rows) ** 0.5))), model, multi_source)
+    if longest > 0.97 * (total + model["item"] * len(units_np)) / n_groups or int(whole[0]["work_count"].max()) > MERGE_PASS:
+        return None
+    return whole
+
+
 def _finish_cache(units_np: np.ndarray, blobs, G: int, H_q: int, stream_bytes: int, kv_algo_bytes: int,
                   scale_max: np.ndarray, *, multi_source: bool, work_bytes, n_groups, groups_per_cu: int,
                   cost) -> StreamCache:
@@ -664,19 +685,8 @@ def _finish_caches(specs) -> List[StreamCache]:
             # caches get one group per compute unit, tiny ones at least 4 tiles per group.
             total_tiles = int(tiles_np.sum())
             n_groups = max(1, min(opt["groups_per_cu"] * cus, int(round((6.0 * total_tiles) ** 0.5)), total_tiles // 4))
-            # No more units than compute units: runs that keep to one unit, unless they come out more uneven
-            # than the second item of a workgroup costs.  A step costs a * tiles / runs + b * runs / rows (the
-            # partials a row's merge reads), least at runs ~ sqrt(tiles * rows); measured with 32 / 64 / 96 / 128 /
-            # 192 / 256 runs: 8 units of 4k tokens 17.4 / 15.9 / 15.1 / 15.1 / 15.5 / 15.9 us, of 16k 27.4 / 21.0 / 18.4 /
-            # 17.5 / 16.8 / 16.9; 2 of 4k 14.9 / 15.6 / 16.1 / 16.8, 4 of 32k 26.7 / 21.3 / 19.0 / 18.4 / 18.2 / 18.6 (in
-            # runs across units 19.4, 19.5, 19.1, 19.8).  More than one per compute unit: 23.7 against 14.9.
-            # 64 units of 32k tokens, four runs each, are uneven: 58.2 us against 56.6.
-            n_rows = len(np.unique(units_np["q_row"])) if multi_source else len(units_np)
             if 0 < len(units_np) <= cus and opt["groups_per_cu"] == 1:
-                whole, longest, total = _partition_whole_units(
-                    units_np, min(cus, int(round((5.3 * total_tiles * n_rows) ** 0.5))), model, multi_source)
-                if longest > 0.97 * (total + model["item"] * len(units_np)) / n_groups:
-                    whole = None
+                whole = _whole_units(units_np, total_tiles, n_groups, cus, model, multi_source)
         if whole is not None:
             units_np, work_np, groups_np = whole
         elif work_bytes is None:

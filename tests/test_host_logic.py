@@ -309,6 +309,35 @@ def test_partition_by_whole_units(multi):
         assert work["u"].tobytes() == got[work["unit"]].tobytes()
 
 
+def test_whole_units_keep_a_rows_partials_to_one_pass_of_its_merge(monkeypatch):
+    """Rows of several sources: a partition is taken only if none has more partials than a merge takes in one
+    pass, whatever their units have each."""
+    from rdkv_amd import stream_cache as sc
+    rng = np.random.default_rng(17)
+
+    def units_of(tokens, rows):
+        u = np.zeros(len(tokens), dtype=sc.UNIT_DTYPE)
+        u["n_tok"][:, 2], u["d8"], u["q_row"] = tokens, 16, np.asarray(rows) * 8
+        return u
+
+    def cut(u, cus=256):
+        tiles = int((-(-u["n_tok"].astype(np.int64) // 64)).sum())
+        n_groups = max(1, min(cus, int(round((6.0 * tiles) ** 0.5)), tiles // 4))
+        return sc._whole_units(u, tiles, n_groups, cus, sc.DEFAULT_COST, True)
+    taken = refused = 0
+    for case in range(400):
+        n = int(rng.integers(1, 30))
+        u = units_of(rng.choice([64, 300, 5000, 30000, 120000], n), np.sort(rng.integers(0, 4, n)))
+        whole = cut(u)
+        with monkeypatch.context() as m:
+            m.setattr(sc, "MERGE_PASS", 1 << 30)       # by the evenness of its runs alone
+            even = cut(u)
+        assert (whole is None) == (even is None or even[0]["work_count"].max() > 128)
+        taken += whole is not None
+        refused += even is not None and whole is None
+    assert taken > 20 and refused > 5
+
+
 def test_library_partition_matches_partition_work():
     """The library's host-side work partition against ``partition_work`` and the merge bookkeeping
     restated here, on random unit tables: empty units (leading, trailing, in runs), single-tile
