@@ -508,6 +508,16 @@ class _DecodeStep:
         self.rope = (cos.view(D)[:D // 2], sin.view(D)[:D // 2])
 
 
+def _rope_ahead_end(model, rotary_emb) -> float:
+    """The position from which on the rotary embedding is asked for a decoded token only, not ahead of it (the token may
+    turn out to be an EOS, and its position never be decoded): the length the model is configured for, beyond which
+    a module may have no entry; 0 for the kinds whose frequencies follow the longest position they have seen."""
+    if getattr(rotary_emb, "rope_type", "default") in ("dynamic", "longrope"):
+        return 0
+    limit = getattr(getattr(model, "config", None), "max_position_embeddings", None)
+    return math.inf if limit is None else limit
+
+
 def _layer_stream_caches(dual_cache, num_kv_groups: int) -> List[StreamCache]:
     """One streaming cache per layer (a sequential model attends layer by layer), built once per
     packed cache and kept on it like the reference keeps its pre-squeezed views."""
@@ -563,6 +573,7 @@ def greedy_decode_fast(model, dual_cache, next_token_logits, max_new_tokens, eos
     generated: List[int] = []
     collected = [] if return_logits else None
     step_state = _DecodeStep(W, caches, new_kv_buf, model_dtype)
+    ahead = _rope_ahead_end(model, W.rotary_emb)
     graph = None
     with torch.inference_mode():
         position = int(decode_position_start)
@@ -589,7 +600,7 @@ def greedy_decode_fast(model, dual_cache, next_token_logits, max_new_tokens, eos
                 graph.replay()
             else:
                 step_state.run()
-                if not use_cuda_graph and step + 1 < max_new_tokens:
+                if not use_cuda_graph and step + 1 < max_new_tokens and position + step + 1 < ahead:
                     step_state.rope_ahead()
             if collected is not None:
                 collected.append(step_state.logits[:, -1, :].detach().float().clone().cpu())

@@ -137,6 +137,31 @@ def test_decode_loop_matches_restated_model_over_oracle_attention(setup, fp32_mo
             assert ids[step + 1] == int(got.argmax())
 
 
+@pytest.mark.parametrize("kind", ["table", "dynamic"])
+def test_rotary_embedding_is_asked_for_decoded_positions_only(setup, monkeypatch, kind):
+    """A module whose table ends with the model's length, and one that adapts to the longest position it has seen:
+    tokens up to an EOS at the last position, and no position beyond the decoded ones."""
+    model, prompt, pre, kv = setup
+    cache, first = _pack(kv, *_mixed_bits(11)), pre.logits[0, -1]
+    ids = fast_decode.greedy_decode_fast(model, cache, first, 8, [], torch.device(DEV), T_PROMPT)
+    stop = next(i for i in range(4, 8) if ids[i] not in ids[:i])
+    rotary, asked = model.model.rotary_emb, []
+    forward = rotary.forward
+
+    def bounded(x, position_ids):
+        asked.append(int(position_ids))
+        if asked[-1] >= T_PROMPT + stop:
+            raise IndexError("no such position")
+        return forward(x, position_ids)
+    monkeypatch.setattr(rotary, "forward", bounded)
+    if kind == "table":
+        monkeypatch.setattr(model.config, "max_position_embeddings", T_PROMPT + stop)
+    else:
+        monkeypatch.setattr(rotary, "rope_type", "dynamic")
+    got = fast_decode.greedy_decode_fast(model, cache, first, 100, [ids[stop]], torch.device(DEV), T_PROMPT)
+    assert got == ids[:stop] and asked == list(range(T_PROMPT, T_PROMPT + stop))
+
+
 def test_decode_loop_tracks_model_forward(setup):
     """All V kept as fp16, all K channels at 8 bits: the packed cache is the dense one up to the
     K quantization, so the loop must follow ``model.forward`` over the dense cache closely."""
