@@ -39,6 +39,26 @@ def _separately(q, layer, v16, kn, vn, G):
     return w, out
 
 
+def _sum64(w, layer, v16, vn):
+    """The weighted sum in 64 bits, over the packed values and the appended ones."""
+    H, n = vn.shape[:2]
+    T_v, G = int(layer.T_eff), w.shape[0] // H
+    out = torch.empty(w.shape[0], 128, dtype=torch.float64, device=DEV)
+    for h in range(H):
+        V = torch.zeros(w.shape[1], 128, dtype=torch.float64, device=DEV)
+        at = 0
+        for t, bits, m in zip((layer.V_2bit, layer.V_4bit, layer.V_8bit), (2, 4, 8), layer.seg_bounds_per_head[h].tolist()):
+            if m:
+                codes = torch.cat([(t[h, :m].long() >> i) & ((1 << bits) - 1) for i in range(0, 8, bits)], dim=1)
+                V[at:at + m] = (codes.double() - layer.V_zp[h, at:at + m].double()) * layer.V_scale[h, at:at + m].double()
+            at += m
+        n16 = int(layer.n_v16_per_head[h])
+        V[T_v:T_v + n16] = v16[h, :n16].double()
+        V[w.shape[1] - n:] = vn[h].double()
+        out[h * G:(h + 1) * G] = w[h * G:(h + 1) * G].double() @ V
+    return out
+
+
 def _pairs(monkeypatch):
     """The number of pairs of every call."""
     seen, load = [], _lib.load()
@@ -89,6 +109,11 @@ def test_rows_in_pairs(monkeypatch, H, T, G, n_new, kept, dtype, mask):
     assert float((buf[:, t_old + n_new:] - 7.0).abs().max()) == 0
     np.testing.assert_allclose(t2n(out), t2n(exp), rtol=0, atol=1e-5)
     assert torch.equal(out, again)
+    # The weights that the sum forms itself: an exponential's last bits (1.2e-7 of the weights in the 2-norm) and some
+    # sixty roundings of the sum (sqrt(64) * 2^-25 = 2.4e-7), twice, and rows whose terms cancel to half.
+    exact = _sum64(w, layer, v16, vn)
+    err = (out.double() - exact).norm(dim=1) / exact.norm(dim=1)
+    assert float(err.max()) < 1.5e-6, float(err.max())
 
 
 def test_wide_keys_come_in_pairs_at_any_length(monkeypatch):
