@@ -1,9 +1,12 @@
 // Decode attention over the reference's padded ("shared-max stripe") tensor layout:
 // K scores, masked softmax and the V weighted sum as three separate entry points with
-// the call shape of obkv_accel/triton_k_kernel.py:1211 and triton_v_kernel.py:1729.
-// These keep the reference's semantics for callers that overwrite packed tensors in
-// place or pass strided score buffers; the streaming fused kernel is the fast path.
-// fp32 math throughout, fixed summation order (deterministic).
+// the call shape of obkv_accel/triton_k_kernel.py:1211 and triton_v_kernel.py:1729, and a
+// layer's call in which the softmax is part of the other two (rdkv_attn_scores,
+// rdkv_v_weighted_sum_scores).  These keep the reference's semantics for callers that overwrite
+// packed tensors in place or pass strided score buffers; the streaming fused kernel is the fast path.
+// Arithmetic: K scores of rows stored back to back are exact integer products of the codes with
+// q * scale in 46 bits, joined in fp32 at the end; everything else - scores of other rows, softmax,
+// V sum - is fp32 operands, products and sums.  Fixed summation order (deterministic).
 #include "rdkv_common.h"
 
 #include <algorithm>
@@ -1051,8 +1054,8 @@ softmax_rows_split_kernel(const float *__restrict__ so, int64_t so_sh, const flo
 // Error against 64 bits over random layers of 1k .. 128k tokens: a layer's call 2.2e-7 .. 5.9e-7 of the result in the
 // 2-norm, the sum alone 0.9e-7 .. 2.0e-7; with fp16 pairs 2.1e-7 .. 6.1e-7 and 1.0e-7 .. 2.7e-7, on the vector ALU with
 // uncentred codes 2.4e-7 .. 9.5e-7 and 0.9e-7 .. 1.6e-6.
-// What bounds it: set-up and the latency of a few steps per wavefront at 32k, at 128k the vector instructions (half of
-// the cycles) and the products (a fifth), which overlap only between the two wavefronts of a SIMD.  Us with its
+// What bounds it: set-up and the latency of a few steps per wavefront at 32k, at 128k the vector instructions (63 % of
+// the cycles) and the products (24 %), which overlap only between the two wavefronts of a SIMD.  Us with its
 // reduction of 8 KV heads x 1.5k / 32k / 128k (low-bit): on the vector ALU (a conversion and a multiply-add per head and
 // code) 12.9 / 22.5 / 39.7, with fp16 pairs 11.9 / 19.7 / 29.9, now 13.9 / 20.1 / 34.3; eight query heads per KV head, 32k
 // 28.6 / 29.5 / 30.4 (two workgroups of four heads, eight apart in the launch, so that a die's L2 serves the second; one
@@ -1092,8 +1095,7 @@ __device__ __forceinline__ int v_lane_offset(int cls, int li) { return cls == 3 
 __device__ __forceinline__ void v_load(int cls, const VClass c, const uint16_t *sc, const uint16_t *zz, int t0,
                                        const float *wrow, int sub, int li, VTile &L) {
   // Bases are the wavefront's, offsets from them 32 bits a lane: 64-bit addresses by lane were 31 of the step's 480
-  // vector instructions.  (The sum at 128k low-bit issues vector instructions 85 % of its time: 25.9 -> 25.0 us, a layer's
-  // call 47.0 -> 46.2.)
+  // vector instructions.  (The sum at 128k low-bit, with 85 % of its cycles in vector instructions: 25.9 -> 25.0 us.)
   const int row_log = 5 + cls, last = c.n - 1 - t0;
   const bool wide = cls == 3;
   const uint8_t *base = c.codes + ((int64_t)t0 << row_log);
