@@ -46,8 +46,9 @@ def _layer(n2, n4, n8, H, T, G, seed, q_scale=1.0, odd_zero_points=False, unused
 
 
 def _check(got, terms, centred, counts):
-    """Roundings of the sum and of the factor 1 / sqrt(128) (itself rounded), and 30 bits of every term against
-    the head's largest (each times its width's power of two) with codes below 2^7.  Zero points outside a
+    """Roundings of the sum and of the factor 1 / sqrt(128) (itself rounded), and of every term 30 bits against
+    the head's largest (each times its width's power of two; the operands hold 46, of which the scales here, like each
+    other, need no more: ``test_channels_far_below_the_largest``) with codes below 2^7.  Zero points outside a
     width's codes enter as an fp32 sum: 2^-20 of its magnitude."""
     exp = np.einsum("hgc,htc->hgt", terms, centred) / np.sqrt(128.0)
     sizes = np.abs(terms) * np.repeat([1 / 32, 1 / 8, 1.0], counts)

@@ -137,6 +137,35 @@ def test_wide_keys_come_in_pairs_at_any_length(monkeypatch):
     assert float(err) < 2e-6, float(err)
 
 
+@pytest.mark.parametrize("G", [4, 8])
+def test_wide_rows_under_capture(G):
+    """Rows whose two tiles take more than 64 KB of LDS, recorded and replayed with other queries in between."""
+    require_gpu()
+    g = torch.Generator().manual_seed(9)
+    H, T, n_new = 2, 140_000, 30
+    K, V = (torch.randn(1, H, T, 128, generator=g).half().to(DEV) for _ in range(2))
+    layer, v16 = packing.pack_layer_per_head(K, V, torch.tensor([2, 4, 8, 16])[torch.randint(0, 4, (H, T), generator=g)],
+                                             torch.full((H, 128), 8), G)
+    layer, v16 = fast_decode._pre_squeeze_packed((layer,))[0], v16[0].contiguous()
+    q = torch.randn(H * G, 128, generator=g).to(DEV)
+    kn, vn = (torch.randn(H, n_new, 128, generator=g).to(DEV) for _ in range(2))
+    buf, out = torch.empty(H * G, int(layer.T_eff_k) + n_new, device=DEV), torch.empty(H * G, 128, device=DEV)
+    call = lambda: fast_decode.trizone_attention(q, layer, v16, layer.n_v16_per_head, kn, vn, G, scores_buf=buf, out=out)   # noqa: E731
+    call()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for seed in range(3):
+        q.copy_(torch.randn(H * G, 128, generator=g))
+        call()
+        torch.cuda.synchronize()
+        exp, w = out.clone(), buf.clone()
+        out.zero_(), buf.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, exp) and torch.equal(buf, w)
+
+
 @pytest.mark.parametrize("G", [4, 6])
 @pytest.mark.parametrize("what", ["row -inf", "all -inf", "new inf", "nan", "inf", "lowest", "tile -inf", "tile nan"])
 def test_masked_and_infinite_rows(what, G):
