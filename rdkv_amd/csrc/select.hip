@@ -48,12 +48,13 @@ struct MaxI { __device__ int operator()(int a, int b) const { return a > b ? a :
 struct MaxF { __device__ float operator()(float a, float b) const { return a > b ? a : b; } };
 
 // Index of the cheapest option for one score; `width` receives its bit width.
-__device__ __forceinline__ int choose(float s, const Options& o, const float* lb, int& width) {
+template <int N = kMaxOptions>
+__device__ __forceinline__ int choose(float s, const Options& o, const float (&lb)[N], int& width) {
   float best = __fadd_rn(__fmul_rn(s, o.eps[0]), lb[0]);
   int idx = 0;
   width = o.ibits[0];
 #pragma unroll
-  for (int n = 1; n < kMaxOptions; ++n) {
+  for (int n = 1; n < N; ++n) {
     if (n < o.n) {
       const float c = __fadd_rn(__fmul_rn(s, o.eps[n]), lb[n]);
       if (c < best) { best = c; idx = n; width = o.ibits[n]; }      // strict: the first minimum wins
@@ -228,7 +229,11 @@ knapsack_bisect_kernel(const float* __restrict__ scores, int64_t stride_b, int g
 // resident together; a wait that does not end within a bound makes the workgroup give up and write
 // the invalid width 255 instead of hanging.
 // ---------------------------------------------------------------------------------------------
-constexpr int kCoopThreads = 256;
+// A workgroup is one, two or four sets of kCoopLanes threads (SETS).  Every set holds the whole chunk and takes its
+// share of a pass's candidates: a pass is bound by its chain of vector instructions (3.5 ns each where they depend), and
+// one set leaves a SIMD a wavefront or less.  With the midpoints and the way down their tree taken by lanes instead of
+// one thread in turn, a call of 8 rows of 4k / 31k scores 34.6 / 43.0 -> 24.2 / 29.5 us (four / two sets).
+constexpr int kCoopLanes = 256;
 constexpr int kCoopMaxSplit = 64;          // workgroups per row at most
 constexpr int kCoopWords = 32;             // words a workgroup can publish per pass (17 are used at most)
 constexpr int kCoopMaxIters = 64;          // passes stay below the 255 the tag byte can tell apart
@@ -265,7 +270,7 @@ __device__ __forceinline__ uint32_t coop_poll(const uint32_t* p, uint32_t tag, i
 // Publishes this workgroup's n values (mine[i] in LDS, each below 2^24) and leaves in c.tot[i] their
 // sum over the row's workgroups (MAX: the maximum of the 32-bit numbers mine[0] << 16 | mine[1]
 // in c.tot[0]).
-template <bool MAX>
+template <bool MAX, int SETS>
 __device__ void coop_exchange(CoopCtx& c, int n, const int* mine) {
   const uint32_t tag = (uint32_t)(c.pass + 1);
   uint32_t* buf = c.words + (c.pass & 1) * (kCoopMaxSplit * kCoopWords);
@@ -281,23 +286,23 @@ __device__ void coop_exchange(CoopCtx& c, int n, const int* mine) {
       atomicMax(reinterpret_cast<unsigned int*>(&c.tot[0]), (hi << 16) | lo);
     }
   } else {
-    // a thread's words (word i of every kCoopThreads / kCoopWords-th workgroup) are requested together and
+    // a thread's words (word i of every kThreads / kCoopWords-th workgroup) are requested together and
     // asked for again until all carry the tag
-    constexpr int kPer = kCoopMaxSplit * kCoopWords / kCoopThreads;
-    static_assert(kCoopWords == 32 && kCoopThreads % kCoopWords == 0, "the lane pairing below assumes 32 words");
+    constexpr int kThreads = SETS * kCoopLanes, kPer = kCoopMaxSplit * kCoopWords / kThreads;
+    static_assert(kCoopWords == 32 && kThreads % kCoopWords == 0, "the lane pairing below assumes 32 words");
     const int i = threadIdx.x & (kCoopWords - 1);
     uint32_t w[kPer];
     bool want[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      want[k] = i < n && (int)threadIdx.x + k * kCoopThreads < c.S * kCoopWords;
+      want[k] = i < n && (int)threadIdx.x + k * kThreads < c.S * kCoopWords;
       w[k] = tag << 24;
     }
     int spins = 0;
     for (;;) {
 #pragma unroll
       for (int k = 0; k < kPer; ++k)
-        if (want[k]) w[k] = __hip_atomic_load(&buf[threadIdx.x + k * kCoopThreads], __ATOMIC_RELAXED, RDKV_COOP_SCOPE);
+        if (want[k]) w[k] = __hip_atomic_load(&buf[threadIdx.x + k * kThreads], __ATOMIC_RELAXED, RDKV_COOP_SCOPE);
       bool ok = true;
 #pragma unroll
       for (int k = 0; k < kPer; ++k) ok = ok && (w[k] >> 24) == tag;
@@ -325,32 +330,39 @@ __device__ void coop_exchange(CoopCtx& c, int n, const int* mine) {
 // workgroup into red[0 .. n) (LDS, zero on entry).  se[j][k] = held score j times eps[k], +inf for
 // the options past the last (their cost is never the smallest, so all eight are walked without a
 // branch); valid[j]: the thread has a j-th score.
-template <int HELD, int NOPT>
+template <int HELD, int NOPT, int SETS>
 __device__ void coop_chunk_sums_n(const float* __restrict__ row, const CoopCtx& c, const float (&se)[HELD][kMaxOptions],
                                   const bool (&valid)[HELD], const float* lam, int n, const Options& o, int* red) {
-#pragma unroll 2
-  for (int i = 0; i < n; ++i) {
-    float lb[kMaxOptions];
+  // Two candidates a step (one with more than five options, whose products take too many registers): their sums go
+  // through the rows of sixteen lanes as the halves of one integer (16 lanes of up to eight widths of at most 255).
+  constexpr int kEach = NOPT <= 5 ? 2 : 1;
+  const int set = __builtin_amdgcn_readfirstlane(threadIdx.x / kCoopLanes), lane = threadIdx.x % kCoopLanes;
+  for (int i = kEach * set; i < n; i += kEach * SETS) {
+    float lb[kEach][NOPT];
 #pragma unroll
-    for (int k = 0; k < kMaxOptions; ++k) lb[k] = __fmul_rn(lam[i], o.bits[k]);
+    for (int e = 0; e < kEach; ++e) {
+      const float at = lam[i + e < n ? i + e : i];
+#pragma unroll
+      for (int k = 0; k < NOPT; ++k) lb[e][k] = __fmul_rn(at, o.bits[k]);
+    }
     int acc = 0;
 #pragma unroll
-    for (int j = 0; j < HELD; ++j) {
-      float best = __fadd_rn(se[j][0], lb[0]);
-      int width = o.ibits[0];
+    for (int e = 0; e < kEach; ++e) {
+      int sum = 0;
 #pragma unroll
-      for (int k = 1; k < NOPT; ++k) {
-        const float cst = __fadd_rn(se[j][k], lb[k]);
-        const bool lt = cst < best;                                  // strict: the first minimum wins
-        best = lt ? cst : best;
-        width = lt ? o.ibits[k] : width;
+      for (int j = 0; j < HELD; ++j) {
+        float best = __fadd_rn(se[j][0], lb[e][0]);
+        int width = o.ibits[0];
+#pragma unroll
+        for (int k = 1; k < NOPT; ++k) {
+          const float cst = __fadd_rn(se[j][k], lb[e][k]);
+          const bool lt = cst < best;                                  // strict: the first minimum wins
+          best = lt ? cst : best;
+          width = lt ? o.ibits[k] : width;
+        }
+        sum += valid[j] ? width : 0;
       }
-      acc += valid[j] ? width : 0;
-    }
-    for (int t = c.t0 + (int)threadIdx.x + HELD * (int)blockDim.x; t < c.t1; t += blockDim.x) {
-      int width;
-      choose(row[t], o, lb, width);
-      acc += width;
+      acc |= sum << (16 * e);
     }
     // the wavefront's sum without a trip through LDS per step: within rows of sixteen lanes by
     // lane permutations, then the four row totals
@@ -358,20 +370,60 @@ __device__ void coop_chunk_sums_n(const float* __restrict__ row, const CoopCtx& 
     acc += __builtin_amdgcn_update_dpp(0, acc, 0x4E, 0xF, 0xF, false);     // lane ^ 2
     acc += __builtin_amdgcn_update_dpp(0, acc, 0x141, 0xF, 0xF, false);    // mirror within eight
     acc += __builtin_amdgcn_update_dpp(0, acc, 0x140, 0xF, 0xF, false);    // mirror within sixteen
-    const int total = __builtin_amdgcn_readlane(acc, 0) + __builtin_amdgcn_readlane(acc, 16) +
-                      __builtin_amdgcn_readlane(acc, 32) + __builtin_amdgcn_readlane(acc, 48);
-    if ((threadIdx.x & 63) == 0) atomicAdd(&red[i], total);
+    int total[kEach];
+#pragma unroll
+    for (int e = 0; e < kEach; ++e) total[e] = 0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t v = (uint32_t)__builtin_amdgcn_readlane(acc, 16 * r);
+      total[0] += (int)(v & 0xffffu);
+      if (kEach == 2) total[kEach - 1] += (int)(v >> 16);
+    }
+    if (HELD == 8 && c.t1 - c.t0 > HELD * kCoopLanes) {      // (uniform) a chunk beyond what is held
+#pragma unroll
+      for (int e = 0; e < kEach; ++e) {
+        int rest = 0;
+        for (int t = c.t0 + lane + HELD * kCoopLanes; t < c.t1; t += kCoopLanes) {
+          int width;
+          choose(row[t], o, lb[e], width);
+          rest += width;
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) rest += __shfl_xor(rest, off, 64);
+        total[e] += rest;
+      }
+    }
+    if ((threadIdx.x & 63) == 0) {
+      atomicAdd(&red[i], total[0]);
+      if (kEach == 2 && i + 1 < n) atomicAdd(&red[i + 1], total[kEach - 1]);
+    }
   }
   __syncthreads();
 }
 
+// The midpoints that four bisection levels over (lo, hi) can reach: node 1 is that of the interval itself, node 2n
+// that of the lower half of node n's, node 2n + 1 that of the upper half.  Thread n goes its own way down to node n (one
+// thread writing all fifteen in turn, with divisions: 0.7 us of a pass).  (Halving by a product is the same
+// correctly rounded number as the reference's division by two.)
+__device__ __forceinline__ void coop_midpoints(float lo, float hi, float* cand) {
+  const int n = threadIdx.x;
+  if (n >= 1 && n < 16) {
+    float mid = __fmul_rn(__fadd_rn(lo, hi), 0.5f);
+    for (int bit = 30 - __clz(n); bit >= 0; --bit) {
+      if ((n >> bit) & 1) lo = mid; else hi = mid;
+      mid = __fmul_rn(__fadd_rn(lo, hi), 0.5f);
+    }
+    cand[n] = mid;
+  }
+}
+
 // (the options are walked to a compile-time count: the usual four or five, or all eight)
-template <int HELD>
+template <int HELD, int SETS>
 __device__ void coop_chunk_sums(const float* __restrict__ row, const CoopCtx& c, const float (&se)[HELD][kMaxOptions],
                                 const bool (&valid)[HELD], const float* lam, int n, const Options& o, int* red) {
-  if (o.n <= 4) coop_chunk_sums_n<HELD, 4>(row, c, se, valid, lam, n, o, red);
-  else if (o.n == 5) coop_chunk_sums_n<HELD, 5>(row, c, se, valid, lam, n, o, red);
-  else coop_chunk_sums_n<HELD, kMaxOptions>(row, c, se, valid, lam, n, o, red);
+  if (o.n <= 4) coop_chunk_sums_n<HELD, 4, SETS>(row, c, se, valid, lam, n, o, red);
+  else if (o.n == 5) coop_chunk_sums_n<HELD, 5, SETS>(row, c, se, valid, lam, n, o, red);
+  else coop_chunk_sums_n<HELD, kMaxOptions, SETS>(row, c, se, valid, lam, n, o, red);
 }
 
 __global__ void coop_init_kernel(uint32_t* state, int64_t n_words) {
@@ -379,8 +431,8 @@ __global__ void coop_init_kernel(uint32_t* state, int64_t n_words) {
   if (i < n_words) state[i] = 0u;
 }
 
-template <int HELD>
-__global__ void __launch_bounds__(kCoopThreads) __attribute__((amdgpu_waves_per_eu(4)))
+template <int HELD, int SETS>
+__global__ void __launch_bounds__(SETS * kCoopLanes) __attribute__((amdgpu_waves_per_eu(4)))
 knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int group_rows, int T, int S,
                      Budget budget, Options o, int max_iters, float tol,
                      uint32_t* __restrict__ state, void* __restrict__ out, int out_elem_size,
@@ -409,14 +461,14 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
   float m = -__builtin_inff();
 #pragma unroll
   for (int j = 0; j < HELD; ++j) {
-    const int t = c.t0 + (int)threadIdx.x + j * kCoopThreads;
+    const int t = c.t0 + (int)(threadIdx.x % kCoopLanes) + j * kCoopLanes;
     valid[j] = t < c.t1;
     const float v = valid[j] ? row[t] : 0.f;
     if (valid[j]) m = fmaxf(m, v);
 #pragma unroll
     for (int k = 0; k < kMaxOptions; ++k) se[j][k] = k < o.n ? __fmul_rn(v, o.eps[k]) : __builtin_inff();
   }
-  for (int t = c.t0 + (int)threadIdx.x + HELD * kCoopThreads; t < c.t1; t += kCoopThreads) m = fmaxf(m, row[t]);
+  for (int t = c.t0 + (int)threadIdx.x + HELD * kCoopLanes; t < c.t1; t += SETS * kCoopLanes) m = fmaxf(m, row[t]);
   __syncthreads();
 
   // ---- the row maximum
@@ -427,7 +479,7 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
     red[1] = (int)(bits & 0xffffu);
   }
   __syncthreads();
-  coop_exchange<true>(c, 2, red);
+  coop_exchange<true, SETS>(c, 2, red);
   const float lam0 = fmaxf(__fmul_rn(rdkv_ordered_to_float((uint32_t)tot[0]), 0.375f), 1e-8f);
   __syncthreads();
   if (threadIdx.x < 2) red[threadIdx.x] = 0;
@@ -440,23 +492,13 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
   int d = -1;
   {
     if (threadIdx.x == 0) {
-      float lo[16], hi[16];
-      lo[1] = 0.f; hi[1] = lam0;
       cand[0] = lam0;
       cand[1] = 0.f;
-#pragma unroll
-      for (int n = 1; n < 16; ++n) {
-        const float mid = __fdiv_rn(__fadd_rn(lo[n], hi[n]), 2.0f);
-        cand[1 + n] = mid;
-        if (2 * n < 16) {
-          lo[2 * n] = lo[n]; hi[2 * n] = mid;
-          lo[2 * n + 1] = mid; hi[2 * n + 1] = hi[n];
-        }
-      }
     }
+    coop_midpoints(0.f, lam0, cand + 1);
     __syncthreads();
-    coop_chunk_sums<HELD>(row, c, se, valid, cand, 17, o, red);
-    coop_exchange<false>(c, 17, red);
+    coop_chunk_sums<HELD, SETS>(row, c, se, valid, cand, 17, o, red);
+    coop_exchange<false, SETS>(c, 17, red);
     if ((int)threadIdx.x < 17) red[threadIdx.x] = 0;
     if (!(__fdiv_rn((float)tot[0], (float)T) > bud)) d = 0;
     __syncthreads();
@@ -472,8 +514,8 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
       }
       __syncthreads();
       lam = cand[kCoopWords];
-      coop_chunk_sums<HELD>(row, c, se, valid, cand, n, o, red);
-      coop_exchange<false>(c, n, red);
+      coop_chunk_sums<HELD, SETS>(row, c, se, valid, cand, n, o, red);
+      coop_exchange<false, SETS>(c, n, red);
       if ((int)threadIdx.x < n) red[threadIdx.x] = 0;
       for (int i = 0; i < n; ++i) {
         const float avg = __fdiv_rn((float)tot[i], (float)T);
@@ -502,7 +544,7 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
     // end no earlier than this row's own lambda reaches 1e12 (g_own, below): while g_own + 1 >= d
     // the minimum leaves d as it is whatever the other rows say, and nothing is waited for.
     int g_own = kMaxDoublings + 1;
-    {
+    if (d > 0) {
       float lam = lam0;
       for (int it = 0; it < kMaxDoublings; ++it) {
         if (it < d) lam = __fmul_rn(lam, 2.0f);
@@ -558,23 +600,11 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
     while (!done) {
       const int at = have_first ? 1 : 0;   // where lambda = 0 sits in cand / tot; the nodes follow it
       if (!have_first) {
-        if (threadIdx.x == 0) {
-          float lo[16], hi[16];
-          lo[1] = lam_lo; hi[1] = lam_hi;
-          cand[0] = 0.f;   // lambda = 0 decides whether to bisect at all (first pass; unused afterwards)
-#pragma unroll
-          for (int n = 1; n < 16; ++n) {
-            const float mid = __fdiv_rn(__fadd_rn(lo[n], hi[n]), 2.0f);
-            cand[n] = mid;
-            if (2 * n < 16) {
-              lo[2 * n] = lo[n]; hi[2 * n] = mid;
-              lo[2 * n + 1] = mid; hi[2 * n + 1] = hi[n];
-            }
-          }
-        }
+        if (threadIdx.x == 0) cand[0] = 0.f;   // lambda = 0 decides whether to bisect at all (first pass; unused afterwards)
+        coop_midpoints(lam_lo, lam_hi, cand);
         __syncthreads();
-        coop_chunk_sums<HELD>(row, c, se, valid, cand, 16, o, red);
-        coop_exchange<false>(c, 16, red);
+        coop_chunk_sums<HELD, SETS>(row, c, se, valid, cand, 16, o, red);
+        coop_exchange<false, SETS>(c, 16, red);
         if (threadIdx.x < kCoopWords) red[threadIdx.x] = 0;
       }
       have_first = false;
@@ -582,24 +612,28 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
         first = false;
         if (__fdiv_rn((float)tot[at], (float)T) <= bud) done = true;
       }
-      int node = 1;
+      // every node's comparisons at once, one in each of sixteen lanes, then the way down over their bits
+      const float avg = __fdiv_rn((float)tot[at + (threadIdx.x & 15)], (float)T);
+      const uint32_t hit = (uint32_t)__ballot(__fdiv_rn(fabsf(__fsub_rn(avg, bud)), denom) < tol);
+      const uint32_t over = (uint32_t)__ballot(avg > bud);
+      int node = 1, last = 0, lo_node = 0, hi_node = 0;
       for (int lvl = 0; lvl < 4 && !done; ++lvl) {
-        const float mid = cand[at + node];
-        const float avg = __fdiv_rn((float)tot[at + node], (float)T);
-        lam_final = mid;
+        last = node;
         ++it;
-        const float rel = __fdiv_rn(fabsf(__fsub_rn(avg, bud)), denom);
-        if (rel < tol) {
+        if ((hit >> node) & 1) {
           done = true;
-        } else if (avg > bud) {
-          lam_lo = mid;
+        } else if ((over >> node) & 1) {
+          lo_node = node;
           node = 2 * node + 1;
         } else {
-          lam_hi = mid;
+          hi_node = node;
           node = 2 * node;
         }
         if (it >= max_iters) done = true;
       }
+      if (last) lam_final = cand[at + last];
+      if (lo_node) lam_lo = cand[at + lo_node];
+      if (hi_node) lam_hi = cand[at + hi_node];
       __syncthreads();                                // everyone has read the totals before the next pass rewrites them
     }
   }
@@ -638,7 +672,7 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
         }
       }
       __syncthreads();
-      coop_exchange<false>(c, o.n, red);
+      coop_exchange<false, SETS>(c, o.n, red);
       if (c.sub == 0 && (int)threadIdx.x < o.n) counts[(int64_t)b * o.n + threadIdx.x] = tot[threadIdx.x];
     }
   }
@@ -895,33 +929,46 @@ int check_common(const void* scores, int B, int64_t T, const void* budget, const
 }  // namespace
 
 // 0 / 1 / 2: the kernel that holds 2 / 4 / 8 scores of a chunk per thread in registers
-static int coop_held_index(int64_t chunk) { return chunk <= 2 * kCoopThreads ? 0 : (chunk <= 4 * kCoopThreads ? 1 : 2); }
+static int coop_held_index(int64_t chunk) { return chunk <= 2 * kCoopLanes ? 0 : (chunk <= 4 * kCoopLanes ? 1 : 2); }
+
+typedef void (*CoopKernel)(const float*, int64_t, int, int, int, Budget, Options, int, float, uint32_t*, void*, int, int64_t, int*);
+// [sets 1 / 2 / 4][scores held]
+static const CoopKernel kCoopKernels[3][3] = {
+    {knapsack_coop_kernel<2, 1>, knapsack_coop_kernel<4, 1>, knapsack_coop_kernel<8, 1>},
+    {knapsack_coop_kernel<2, 2>, knapsack_coop_kernel<4, 2>, knapsack_coop_kernel<8, 2>},
+    {knapsack_coop_kernel<2, 4>, knapsack_coop_kernel<4, 4>, knapsack_coop_kernel<8, 4>}};
 
 // Workgroups a row is shared by in the cooperative form (0: one workgroup per row, the two-launch
 // form): a power of two, chunks of at least 512 scores, at most 64 per row, the whole launch on at
 // most half of the workgroup slots the device has for the kernel variant the chunk length selects,
 // and only when that gives a row at least sixteen (with fewer, one workgroup per row was as fast or
-// faster on 64 rows of 32k scores) - or its full eight for a row of 4096 .. 8191 in a launch of at most
-// kCoopShortGrid workgroups: 8 rows of 4096 / 6000 scores 41.1 / 54.0 -> 33.5 / 40.8 us a call, 64 rows
-// 46.8 / 56.6 -> 36.4 / 44.6, 256 rows (four or fewer each) 47.3 against 60.2.
+// faster on 64 rows of 32k scores) - or all that its length allows for a row of 1024 .. 8191 in a launch of at
+// most kCoopShortGrid workgroups.  A call of 8 rows in two launches / shared: 1024 scores 34.6 / 22.8 us, 2048
+// 39.3 / 23.6, 3000 46.8 / 26.6, 4096 41.1 / 24.3; 64 rows of 1024 / 2048 34.6 / 23.1 and 40.9 / 24.0; 256 rows of 4096,
+// which would get two each, 52.4 / 58.0; 8 of 512, one each, 27.
+// kernel: the workgroups' sets (log2).  As many as leave the launch on half of the slots of their kernel, one set /
+// the rule's: 8 rows of 4096 / 16k / 31k scores 34.6 / 24.3, 36.3 / 25.7, 43.0 / 29.4, 2 of 128k 55.3 / 38.2; and a row is
+// shared by half as many where that makes room for a second set and a thread still holds its scores (8 rows of
+// 64k 44.2 -> 38.4, 16 of 32k 46.4 -> 40.3 with it).
 constexpr int64_t kCoopShortGrid = 512;
-static int coop_split(int B, int64_t T, int max_iters) {
-  if (B <= 0 || T < 4096 || max_iters > kCoopMaxIters) return 0;
-  // workgroup slots of the device for the kernel that holds 2 / 4 / 8 scores per thread
-  static int slots_of_device[64][3];       // (0 = not asked yet; a race between first callers writes the same value)
+static int coop_split(int B, int64_t T, int max_iters, int* kernel) {
+  if (B <= 0 || T < 1024 || max_iters > kCoopMaxIters) return 0;
+  // workgroup slots of the device for every kernel
+  static int slots_of_device[64][3][3];       // (0 = not asked yet; a race between first callers writes the same value)
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (slots_of_device[dev][2] == 0) {
-    int cus = 0, per_cu[3] = {0, 0, 0};
-    const bool ok =
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0 &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu[0], knapsack_coop_kernel<2>, kCoopThreads, 0) == hipSuccess &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu[1], knapsack_coop_kernel<4>, kCoopThreads, 0) == hipSuccess &&
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu[2], knapsack_coop_kernel<8>, kCoopThreads, 0) == hipSuccess &&
-        per_cu[0] > 0 && per_cu[1] > 0 && per_cu[2] > 0;
+  if (slots_of_device[dev][2][2] == 0) {
+    int cus = 0, per_cu[3][3];
+    bool ok = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0;
+    for (int e = 0; e < 3; ++e)
+      for (int k = 0; k < 3; ++k)
+        ok = ok && hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu[e][k], kCoopKernels[e][k], kCoopLanes << e, 0) == hipSuccess &&
+             per_cu[e][k] > 0;
     if (!ok) return 0;                     // (asked again next time: the query can fail while a stream is being captured)
-    for (int k = 0; k < 3; ++k) slots_of_device[dev][k] = cus * per_cu[k];
+    for (int e = 0; e < 3; ++e)
+      for (int k = 0; k < 3; ++k) slots_of_device[dev][e][k] = cus * per_cu[e][k];
   }
+  const int(&slots)[3][3] = slots_of_device[dev];
   int64_t S = T / 512;
   if (S > kCoopMaxSplit) S = kCoopMaxSplit;
   // the launch may take half the slots of the kernel its chunk length selects (a shorter split means
@@ -930,16 +977,29 @@ static int coop_split(int B, int64_t T, int max_iters) {
   // split in between - 16 rows of 32k: 68 us with 32 workgroups per row, 74 us with 40)
   auto pow2_floor = [](int64_t v) { int64_t p = 1; while (2 * p <= v) p *= 2; return v >= 1 ? p : 0; };
   S = pow2_floor(S);
+  const int64_t allowed = S;
   for (int step = 0; step < 3 && S >= 1; ++step) {
     const int64_t chunk = (T + S - 1) / S;
     const int k = coop_held_index(chunk);
-    const int64_t cap = slots_of_device[dev][k] / 2 / B;
+    const int64_t cap = slots[0][k] / 2 / B;
     if (S <= cap) break;
     S = pow2_floor(cap);
   }
-  if (S < 16 && !(T < 8192 && S == 8 && (int64_t)B * S <= kCoopShortGrid)) return 0;
-  const int64_t chunk = (T + S - 1) / S;
-  if ((int64_t)B * S > slots_of_device[dev][coop_held_index(chunk)] / 2) return 0;
+  if (S < 16 && !(T < 8192 && S == allowed && (int64_t)B * S <= kCoopShortGrid)) return 0;
+  int64_t chunk = (T + S - 1) / S;
+  if ((int64_t)B * S > slots[0][coop_held_index(chunk)] / 2) return 0;
+  auto sets_for = [&](int64_t split) {
+    const int held = coop_held_index((T + split - 1) / split);
+    for (int e = 2; e > 0; --e)
+      if ((int64_t)B * split <= slots[e][held] / 2) return e;
+    return 0;
+  };
+  *kernel = sets_for(S);
+  if (*kernel == 0 && S >= 32 && (T + S / 2 - 1) / (S / 2) <= 8 * kCoopLanes && sets_for(S / 2) > 0) {
+    S /= 2;
+    chunk = (T + S - 1) / S;
+    *kernel = sets_for(S);
+  }
   // (a chunk's width sum must fit the 24 value bits of an exchange word)
   return chunk <= 32768 ? (int)S : 0;
 }
@@ -968,16 +1028,16 @@ static int knapsack_batched(const float* scores, int64_t stride_b, int B, int64_
   float* lam0 = reinterpret_cast<float*>(workspace);
   int* doublings = reinterpret_cast<int*>(lam0 + B);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (const int S = coop_split(B, T, max_iters)) {
+  int sets = 0;      // (log2)
+  if (const int S = coop_split(B, T, max_iters, &sets)) {
     // few long rows: every row shared by S workgroups, one launch after clearing its state
     uint8_t* base = reinterpret_cast<uint8_t*>(workspace) + (((int64_t)B * 8 + 255) / 256) * 256;
     uint32_t* state = reinterpret_cast<uint32_t*>(base);
     const int64_t n_words = (int64_t)B * kCoopRowWords;
     hipLaunchKernelGGL(coop_init_kernel, dim3((unsigned)rdkv_cdiv(n_words, 256)), dim3(256), 0, s, state, n_words);
     const int64_t chunk = (T + S - 1) / S;
-    const int held = coop_held_index(chunk);
-    auto kernel = held == 0 ? knapsack_coop_kernel<2> : (held == 1 ? knapsack_coop_kernel<4> : knapsack_coop_kernel<8>);
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(B * S)), dim3(kCoopThreads), 0, s, scores, stride_b, group_rows, (int)T, S,
+    hipLaunchKernelGGL(kCoopKernels[sets][coop_held_index(chunk)], dim3((unsigned)(B * S)), dim3(kCoopLanes << sets), 0, s,
+                       scores, stride_b, group_rows, (int)T, S,
                        budget, o, max_iters, tol, state, out, out_elem_size, out_stride_b, counts);
     RDKV_CHECK_LAUNCH("rdkv_knapsack_batched");
     return RDKV_OK;
