@@ -512,7 +512,7 @@ decode_fused_kernel(const uint8_t *__restrict__ blob,
       st_q[b][e] = rdkv_load_dword_of(q, q_dtype, at);
       st_qo[b][e] = st_cs[b][e] = st_sn[b][e] = 0;
       if (rope_cos) {   // rotary embedding on the fly: the partner channel, the angle's cosine and sine
-        st_qo[b][e] = rdkv_load_dword_of(q, q_dtype, at ^ 64);
+        st_qo[b][e] = rdkv_load_dword_of(q, q_dtype, at + ((ic & 64) ? -64 : 64));
         st_cs[b][e] = rdkv_load_dword_of(rope_cos, rope_dtype, ic & 63);
         st_sn[b][e] = rdkv_load_dword_of(rope_sin, rope_dtype, ic & 63);
       }
@@ -538,7 +538,7 @@ decode_fused_kernel(const uint8_t *__restrict__ blob,
         if (rope_cos) {
           // what the reference writes back to q in its storage type before the K kernel reads
           // it (triton_rope.py:36-77)
-          const float other = rdkv_decode_dword(st_qo[b][e], q, q_dtype, at ^ 64);
+          const float other = rdkv_decode_dword(st_qo[b][e], q, q_dtype, at + ((c & 64) ? -64 : 64));
           const float cs = rdkv_decode_dword(st_cs[b][e], rope_cos, rope_dtype, c & 63);
           const float sn = rdkv_decode_dword(st_sn[b][e], rope_sin, rope_dtype, c & 63);
           float out_lo, out_hi;
