@@ -23,6 +23,7 @@ class RdkvTailScores(ctypes.Structure):
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG, "librdkv_hip.so")
+NATIVE_PATH = os.path.join(_PKG, "_native.so")
 
 RDKV_OK = 0
 RDKV_EINVAL = -1
@@ -130,7 +131,7 @@ SIGNATURES = {
 }
 
 _lib: Optional[ctypes.CDLL] = None
-
+native = None          # csrc/native.cpp as a module, bound to the library with it
 
 _seen_library: Optional[str] = None
 
@@ -141,7 +142,7 @@ def available() -> bool:
     global _seen_library
     if _seen_library == LIB_PATH:
         return True
-    if os.path.exists(LIB_PATH):
+    if os.path.exists(LIB_PATH) and os.path.exists(NATIVE_PATH):
         _seen_library = LIB_PATH
         return True
     return False
@@ -161,8 +162,21 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    _bind_native(lib)
     _lib = lib
     return lib
+
+
+def _bind_native(lib: ctypes.CDLL) -> None:
+    """Load the extension module (built with the library) and give it the library's functions."""
+    global native
+    try:
+        from . import _native
+    except ImportError as e:
+        raise RuntimeError(f"rdkv HIP backend is not available: its extension module has not been built ({e}); "
+                           "run `python -m rdkv_amd.build_ext`") from None
+    _native.bind({name: ctypes.cast(getattr(lib, name), c_void_p).value for name in _native.names().split()}, check)
+    native = _native
 
 
 def check(rc: int) -> None:

@@ -12,6 +12,7 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
 CSRC = os.path.join(PKG, "csrc")
 LIB = os.path.join(PKG, "librdkv_hip.so")
+NATIVE = os.path.join(PKG, "_native.so")
 
 COMMON = [
     "-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-fvisibility=hidden",
@@ -38,6 +39,25 @@ def sources():
     return sorted(f for f in os.listdir(CSRC) if f.endswith(".hip"))
 
 
+def build_native() -> None:
+    """The host-side extension module (csrc/native.cpp): the Python and torch C++ interfaces, no HIP."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    cxx = os.environ.get("CXX") or shutil.which("g++") or "c++"
+    tmp = NATIVE + ".tmp"
+    cmd = [cxx, "-O2", "-fPIC", "-shared", "-std=c++17", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I" + os.path.join(ROOT, "include"),
+           "-I" + sysconfig.get_paths()["include"], *(f"-isystem{p}" for p in cpp_extension.include_paths()),
+           os.path.join(CSRC, "native.cpp"), "-o", tmp, *(f"-L{p}" for p in cpp_extension.library_paths()),
+           "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("the extension module failed to build:\n" + r.stderr)
+    os.replace(tmp, NATIVE)
+
+
 def build(verbose: bool = True) -> str:
     hipcc = _hipcc()
     objdir = os.path.join(PKG, "build")
@@ -55,7 +75,9 @@ def build(verbose: bool = True) -> str:
         return obj
 
     with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as ex:
+        native = ex.submit(build_native)
         objs = list(ex.map(compile_one, sources()))
+        native.result()
     tmp = LIB + ".tmp"
     cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -63,7 +85,7 @@ def build(verbose: bool = True) -> str:
         raise RuntimeError("link failed:\n" + r.stderr)
     os.replace(tmp, LIB)
     if verbose:
-        print(f"built {LIB} from {len(objs)} sources")
+        print(f"built {LIB} from {len(objs)} sources, {NATIVE}")
     return LIB
 
 

@@ -24,10 +24,15 @@ DEFAULT_EPSILON_V: Dict[int, float] = {0: 1.0, 2: 0.312, 4: 0.0138, 8: 0.000048,
 BITS = torch.tensor([0, 2, 4, 8, 16], dtype=torch.float32)
 
 
-def _option_arrays(epsilon: Dict[int, float], bit_options: Optional[Tensor]):
+def option_lists(epsilon: Dict[int, float], bit_options: Optional[Tensor]):
+    """The widths an allocation chooses from and their errors, as two lists of floats."""
     bits = [float(b) for b in (BITS if bit_options is None else bit_options).tolist()]
     assert 1 <= len(bits) <= 8, f"between 1 and 8 bit options are supported, got {len(bits)}"
-    eps = [float(epsilon[int(b)]) for b in bits]           # KeyError for an unknown width, as in the reference
+    return bits, [float(epsilon[int(b)]) for b in bits]    # KeyError for an unknown width, as in the reference
+
+
+def _option_arrays(epsilon: Dict[int, float], bit_options: Optional[Tensor]):
+    bits, eps = option_lists(epsilon, bit_options)
     n = len(bits)
     return (ctypes.c_float * n)(*bits), (ctypes.c_float * n)(*eps), n
 

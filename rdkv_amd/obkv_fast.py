@@ -15,9 +15,9 @@ from typing import Dict, List, Optional, Sequence, Union
 import torch
 from torch import Tensor
 
-from . import _lib
+from . import _lib, packing
 from .knapsack_solver import (DEFAULT_EPSILON_K, DEFAULT_EPSILON_V, KeptBudget, knapsack_allocate,   # noqa: F401 (re-exported
-                              knapsack_bit_allocation_batched, load_epsilon_kv_from_calibration)  # as obkv_fast.py:38-46 does)
+                              knapsack_bit_allocation_batched, load_epsilon_kv_from_calibration, option_lists)  # as obkv_fast.py:38-46 does)
 from .packing import _pack_layer_per_head, pack_layer_per_head, pack_layers_per_head  # noqa: F401 (its public name stays here)
 
 
@@ -105,6 +105,42 @@ def _k_budget_per_head(v_counts: Tensor, v_bit_options: Optional[Tensor], T: int
     return KeptBudget(v_counts, opts.index(0.0) if 0.0 in opts else -1, T, head_dim, float(k_budget_bits))
 
 
+def _select_and_pack_native(K, V, layer_scores, channel_scores, gqa_factor, token_budget, k_budget_ratio, pool_kernel_size,
+                            pool_padding, pool_type, v_bit_options, k_bit_options, eps_V, eps_K, retain):
+    """The launches of a layer's selection in one call and of its packing in another (csrc/native.cpp), for dense fp16
+    K / V and fp32 scores on one device; None for anything else."""
+    _lib.load()
+    if not (K.is_cuda and layer_scores.is_cuda and V.dtype == torch.float16):
+        return None
+    dev, H_kv, T, head_dim = K.device, int(layer_scores.shape[0]), int(layer_scores.shape[1]), int(K.shape[3])
+    if T == 0 or H_kv == 0 or int(K.shape[1]) != H_kv or int(K.shape[2]) != T:
+        return None
+    total_budget_bits = 2 * token_budget * head_dim * 16
+    v_avg = (1.0 - k_budget_ratio) * total_budget_bits / (T * head_dim)
+    v_widths, v_errors = option_lists(eps_V, v_bit_options)
+    k_widths, k_errors = option_lists(eps_K, k_bit_options)
+    ws = _lib.workspace(dev, _lib.load().rdkv_knapsack_workspace_bytes(H_kv))
+    words = _lib.host_words(dev, 12 * H_kv)
+    stream = _lib.stream_of(dev)
+    chosen = _lib.native.select_layer(
+        K, V, layer_scores, channel_scores, (int(pool_kernel_size), int(pool_type == "avg"), int(pool_padding == "reflect")),
+        v_widths, v_errors, v_avg, k_widths, k_errors, float(k_budget_ratio * total_budget_bits),
+        v_widths.index(0.0) if 0.0 in v_widths else -1, packing._EARLY_MINMAX_TOKENS, retain, words.take(12 * H_kv), words.tag,
+        ws.data_ptr(), ws.numel(), stream)
+    if chosen is None:
+        words.pending = False           # nothing was launched
+        return None
+    v_bits, k_bits, order, rank3, plan, minmax, v_kept, k_kept = chosen
+    planned = order, rank3, plan, *packing._plan_rows(words.read(dev)), k_bits, minmax
+    done = packing._pack_planned_layer(K, V, gqa_factor, planned, 0, H_kv)
+    if done is None:
+        done = packing._pack_layer_per_head_composed(K, V, v_bits, k_bits, gqa_factor)
+    layer, new_v_only = done
+    if retain:
+        layer.allocation_v_bits, layer.allocation_k_bits = v_kept, k_kept
+    return layer, new_v_only, layer.T_eff
+
+
 def _perhead_select_and_pack_joint(
     K: Tensor, V: Tensor, layer_scores: Tensor, channel_scores: Tensor, *,
     gqa_factor: int, token_budget: int, k_budget_ratio: float, obs_window: int,
@@ -130,6 +166,13 @@ def _perhead_select_and_pack_joint(
     dev = _lib.require_device(K, V)
     H_kv, T = int(layer_scores.shape[0]), int(layer_scores.shape[1])
     head_dim = int(K.shape[3])
+
+    if timing is None and eps_V is not None and eps_K is not None and not torch.cuda.is_current_stream_capturing():
+        done = _select_and_pack_native(K, V, layer_scores, channel_scores, gqa_factor, token_budget, k_budget_ratio,
+                                       pool_kernel_size, pool_padding, pool_type, v_bit_options, k_bit_options, eps_V, eps_K,
+                                       retain_allocation_metadata)
+        if done is not None:
+            return done
 
     def stamp() -> float:
         if timing is None:

@@ -92,6 +92,10 @@ class TriZoneCache:
 
 DualZoneCache = TriZoneCache
 
+# what a layer that the packer makes leaves unset
+_NO_LAYER_FIELDS = dict.fromkeys(("n_fp16_per_head", "fp16_gap_mask", "allocation_v_bits", "allocation_k_bits",
+                                  "deferred_k_for_stack"))
+
 
 def _seg_padded_len(n: int, align: int) -> int:
     return 0 if n == 0 else -(-n // align) * align
@@ -774,12 +778,16 @@ def _plan_layers(v_bits: Tensor, k_bits: Tensor, dev, Ks: Sequence[Tensor] = (),
                                                  plan.data_ptr(), mm.data_ptr(), H * minmax_per_head, _lib.stream_of(dev)))
     if meanwhile is not None:
         meanwhile()
-    numbers = words.read(plan.device)                           # the one synchronization
-    counts_h = [numbers[12 * h:12 * h + 4] for h in range(N)]
-    info_h = [numbers[12 * h + 4:12 * h + 12] for h in range(N)]
-    assert all(row[1] == 0 for row in info_h), "v_bits must be in {0,2,4,8,16}"
-    assert all(row[5] == 0 for row in info_h), "k_bits must be in {0,2,4,8,16}"
-    return order, rank3, plan, counts_h, info_h, kb, mm
+    return order, rank3, plan, *_plan_rows(words.read(plan.device)), kb, mm          # (the one synchronization)
+
+
+def _plan_rows(numbers: list):
+    """The twelve numbers of every head of a plan as rows: class counts [4], then the channels' info [8]."""
+    counts_h = [numbers[at:at + 4] for at in range(0, len(numbers), 12)]
+    info_h = [numbers[at + 4:at + 12] for at in range(0, len(numbers), 12)]
+    assert not any(numbers[5::12]), "v_bits must be in {0,2,4,8,16}"
+    assert not any(numbers[9::12]), "k_bits must be in {0,2,4,8,16}"
+    return counts_h, info_h
 
 
 def _pack_planned_layer(K: Tensor, V: Tensor, gqa_factor: int, planned, first: int, n_total: int,
@@ -792,6 +800,14 @@ def _pack_planned_layer(K: Tensor, V: Tensor, gqa_factor: int, planned, first: i
     dev = K.device
     lib = _lib.load()
     stream = _lib.stream_of(dev)
+    if not one_call and _lib.native is not None:
+        done = _lib.native.pack_layer(K, V, kb_all, order, rank3, plan, mm_all, counts_all, info_all, first, n_total,
+                                      gqa_factor, stream)
+        if done is not None:
+            packed = PackedKVLayer.__new__(PackedKVLayer)
+            packed.__dict__.update(_NO_LAYER_FIELDS)
+            packed.__dict__.update(done[0])
+            return packed, done[1]
     H_kv, T, D = int(K.shape[1]), int(K.shape[2]), int(K.shape[3])
     counts_h, info_h = counts_all[first:first + H_kv], info_all[first:first + H_kv]
     seg = [tuple(row[:3]) for row in counts_h]

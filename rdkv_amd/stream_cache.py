@@ -401,6 +401,38 @@ def _pack_scratch(dev, stream: int, H_kv: int) -> torch.Tensor:
     return t
 
 
+def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, stream: int):
+    """``_pack_entries_direct`` for entries of one shape that the direct kernel takes and that all keep something, with its
+    loops over entries in csrc/native.cpp: (units, blobs, sizes per entry, largest scales [n, 2, H] on the device); None
+    for any others."""
+    from . import packing
+    if _POISON_BLOBS or not entries[0][0].is_cuda or torch.cuda.is_current_stream_capturing():
+        return None
+    Ks, Vs, vbs, kbs = (list(c) for c in zip(*entries))
+    n, H_kv = len(entries), int(Ks[0].shape[1])
+    if len(Ks[0].shape) != 4 or any(len(t.shape) != 2 for t in vbs + kbs):
+        return None
+    words = _lib.host_words(dev, 12 * n * H_kv)
+    planned = _lib.native.stream_order(Ks, Vs, vbs, kbs, packing._EARLY_MINMAX_TOKENS, words.take(12 * n * H_kv), words.tag, stream)
+    if planned is None:
+        words.pending = False           # nothing was launched
+        return None
+    order, plan, kb, mm = planned
+    units = np.zeros(n * H_kv, dtype=UNIT_DTYPE)
+    slots = np.empty((n * H_kv, 4 * MAX_STEPS), dtype=np.int16)
+    sizes, dims = np.zeros((n, 4), dtype=np.int64), np.empty((n, 5), dtype=np.int32)
+    scales = torch.empty(n, 2, H_kv, dtype=torch.float32, device=dev)
+    counts, info = packing._plan_rows(words.read(dev))
+    if _lib.native.stream_tables(counts, info, [int(r) * H_kv * G for r in rows_of_entries], H_kv, G, units, slots, sizes,
+                                 dims) is None:
+        return None
+    units_dev, slots_dev = _lib.upload(dev, units, slots)
+    blobs = _lib.native.stream_pack(Ks, Vs, order, plan, kb, mm if mm is not None else _pack_scratch(dev, stream, H_kv),
+                                    _SCRATCH_PREPARED if mm is None else 2, units, units_dev, slots_dev, sizes, dims, scales, stream)
+    assert blobs is not None
+    return units, blobs, sizes.tolist(), scales
+
+
 def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_bytes: Optional[list] = None):
     """What ``_relayout_entries`` returns, from fp16 K / V and bit allocations instead of packed
     layers: every entry (K, V [1, H_kv, T, 128] fp16, v_bits [H_kv, T], k_bits [H_kv, 128]) is
@@ -418,6 +450,17 @@ def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_
     H_q = None
     # entries by shape: one plan per group
     groups: dict = {}
+    whole = _pack_entries_native(entries, G, rows_of_entries, dev, stream) if _lib.native is not None else None
+    if whole is not None:
+        units_all, blobs, sizes, sm_all = whole
+        if entry_bytes is not None:
+            entry_bytes.extend((int(sb), int(ab)) for _, _, sb, ab in sizes)
+        heads = int(sm_all.shape[2])
+
+        def largest():
+            return _lib.download(sm_all).transpose(0, 2, 1).reshape(n * heads, 2).astype(np.float32)    # (synchronizes)
+
+        return units_all, blobs, sum(int(s[2]) for s in sizes), sum(int(s[3]) for s in sizes), heads * G, largest
     for i, (K, V, vb, kb) in enumerate(entries):
         H_q = int(K.shape[1]) * G
         if _direct_packable(K, V):
@@ -866,6 +909,17 @@ def decode_attn_fused(cache: StreamCache, q: torch.Tensor, out: Optional[torch.T
     workgroup to deliver a partial of an output row combines that row; same bits); default: for
     caches of at most ONE_LAUNCH_MAX_WORK work items (none, as shipped)."""
     lib = _lib.load()
+    if zone_c_weights is None and q_rotated_out is None and tail_scores is None and not one_launch and q.is_cuda \
+            and (zone_c is not None or one_launch is not None or cache.n_work > ONE_LAUNCH_MAX_WORK) and _lib.native is not None:
+        # (a layer of a decode loop comes through here once a step)
+        stream, ws = _lib.stream_workspace(q.device)
+        kn, vn, counts = (None, None, None) if zone_c is None else (zone_c[0], zone_c[1], zone_c[2] if len(zone_c) > 2 else None)
+        cos, sin = (None, None) if rope is None else rope
+        k_step, v_step, row = (None, None, None) if append is None or zone_c is None else append
+        done = _lib.native.decode_attn(cache.__dict__, cache.units_host, q, out, lse, cos, sin, kn, vn, counts, k_step, v_step,
+                                       row, ws.data_ptr(), ws.numel(), stream)
+        if done is not None:
+            return done
     dev = _lib.require_device(q)
     q_dt = _lib.DTYPE_CODE.get(q.dtype)
     if q_dt is None:

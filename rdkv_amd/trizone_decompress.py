@@ -158,13 +158,26 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
     heads = sum(int(t.shape[1]) for pl in dual_cache.packed for t in (pl.K_ch_scale, pl.V_scale) if t is not None)
     for i, pl in enumerate(dual_cache.packed):
         to = _words_of(pl.K_ch_scale.device, words, heads) if pl.K_ch_scale is not None else None
-        K_full, k_check = _unpack_k_enqueue(pl, head_dim, to)
-        if isinstance(k_check, int):
-            words[pl.K_ch_scale.device][1].append((_check_k_counts, pl, k_check))
-        elif k_check is not None:
-            unchecked.append((_check_k_counts, pl, (k_check,)))
         zone_b = dual_cache.new_v_only[i] if i < len(dual_cache.new_v_only) else None
-        if _is_perhead_layout(pl):
+        pair = None
+        if to is not None and _lib.native is not None and _is_perhead_layout(pl):
+            used, n = to.used, int(pl.K_ch_scale.shape[1])
+            pair = _lib.native.dense_layer(pl.__dict__, zone_b, head_dim, to.take(4 * n), to.take(4 * n), to.tag,
+                                           _lib.stream_of(pl.K_ch_scale.device))
+            if pair is None:
+                to.used = used
+            else:
+                K_full, V_full = pair
+                words[pl.K_ch_scale.device][1].extend(((_check_k_counts, pl, n), (_check_v_counts, pl, n)))
+        if pair is None:
+            K_full, k_check = _unpack_k_enqueue(pl, head_dim, to)
+            if isinstance(k_check, int):
+                words[pl.K_ch_scale.device][1].append((_check_k_counts, pl, k_check))
+            elif k_check is not None:
+                unchecked.append((_check_k_counts, pl, (k_check,)))
+        if pair is not None:
+            pass
+        elif _is_perhead_layout(pl):
             rows_b = None
             if int(pl.n_v16) > 0:
                 assert zone_b is not None, f"layer {i}: max_n_v16={pl.n_v16} > 0 but new_v_only is None"
