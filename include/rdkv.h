@@ -760,6 +760,23 @@ int rdkv_knapsack_batched_value(const float *scores, int64_t stride_b, int B, in
                                 int64_t out_stride_b, int32_t *counts, void *workspace, int64_t workspace_bytes,
                                 void *stream);
 
+/* A layer's selection up to the token order of its packer (obkv_fast.py:899-1040), in three launches: rdkv_pool_scores
+ * (kernel_size > 1; pooled [H, T]; its length must stay T), rdkv_knapsack_batched_value over the H rows of tokens as one
+ * group at v_budget (v_bits: bytes, rows of v_stride, a multiple of 16, the base 16-byte aligned; v_counts
+ * [H, n_v_options]), the K allocation over channels [H, D] at the budgets that v_counts leave (k_bits [H, D] bytes), and
+ * what rdkv_pack_layer_plan_start leaves for those widths: order and rank3 [H, T], plan
+ * (rdkv_pack_layer_plan_ints(H, T) ints, of which the histogram stays unwritten), minmax_ws, host_words.
+ * v_bits16 / k_bits16: the widths as int16 [H, T] / [H, D] too, or null.  workspace: rdkv_knapsack_workspace_bytes(H).
+ * RDKV_EUNSUPPORTED beyond 16 heads, 65536 tokens or 256 channels: the calls one by one. */
+int rdkv_select_layer_start(const float *scores, int64_t stride_b, int H, int64_t T, int kernel_size, int is_avg,
+                            int reflect, float *pooled, float v_budget, const float *v_bits_host,
+                            const float *v_eps_host, int n_v_options, int zero_option, uint8_t *v_bits,
+                            int64_t v_stride, int32_t *v_counts, const float *channels, int64_t channel_stride, int D,
+                            float k_kept_bits, const float *k_bits_host, const float *k_eps_host, int n_k_options,
+                            uint8_t *k_bits, int max_iters, float tol, int32_t *order, int32_t *rank3, int32_t *plan,
+                            float *minmax_ws, int minmax_floats_per_head, int16_t *v_bits16, int16_t *k_bits16,
+                            uint64_t *host_words, uint32_t tag, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* obkv_fast.py:1033-1035: the per-head K budget k_budget_bits / (head_dim * max(kept_h, 1)) as
  * the reference's fp32 tensor expression evaluates it (product, reciprocal, product), from the
  * per-option token counts of rdkv_knapsack_batched: kept_h = T - counts[h][zero_option]

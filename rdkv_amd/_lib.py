@@ -117,6 +117,8 @@ SIGNATURES = {
     "rdkv_knapsack_workspace_bytes": (L, [I]),
     "rdkv_knapsack_batched": (I, [P, L, I, L, P, P, P, I, I, F, I, P, I, L, P, P, L, P]),
     "rdkv_knapsack_batched_value": (I, [P, L, I, L, F, P, I, I, L, I, P, P, I, I, F, I, P, I, L, P, P, L, P]),
+    "rdkv_select_layer_start": (I, [P, L, I, L, I, I, I, P, F, P, P, I, I, P, L, P, P, L, I, F, P, P, I, P, I, F, P, P, P, P, I,
+                                    P, P, P, ctypes.c_uint32, P, L, P]),
     "rdkv_k_budget_per_head": (I, [P, I, I, I, L, I, F, P, P]),
     "rdkv_knapsack_rows": (I, [P, L, I, L, P, P, P, I, I, Dbl, P, I, L, P, P]),
     "rdkv_block_score_workspace_bytes": (L, [I, I, L, I]),

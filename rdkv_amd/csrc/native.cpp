@@ -29,7 +29,8 @@ namespace {
   X(rdkv_pool_scores) X(rdkv_knapsack_batched_value) X(rdkv_pack_layer_plan_ints) X(rdkv_pack_layer_plan_start)  \
   X(rdkv_pack_layers_k_minmax) X(rdkv_pack_layer_v_rows) X(rdkv_pack_layer_tables) X(rdkv_pack_layer_k_rows)     \
   X(rdkv_decode_fused) X(rdkv_decode_fused_zone_c) X(rdkv_decode_fused_workspace_bytes)                           \
-  X(rdkv_unpack_layer_k_words) X(rdkv_unpack_layer_v_words) X(rdkv_stream_plan_layer) X(rdkv_pack_layer_stream)
+  X(rdkv_unpack_layer_k_words) X(rdkv_unpack_layer_v_words) X(rdkv_stream_plan_layer) X(rdkv_pack_layer_stream)   \
+  X(rdkv_select_layer_start)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
   RDKV_NATIVE_FUNCTIONS(X)
@@ -286,25 +287,41 @@ PyObject *select_layer(PyObject *const *a, Py_ssize_t) {
     Unlocked u;
     const float *rows = data<float>(scores);
     int64_t row_stride = scores.stride(0);
-    if (kernel > 1) {
+    const bool together = H <= 16 && T <= 65536 && D <= 256 && channels.stride(0) >= D;      // (rdkv_select_layer_start)
+    if (together) {
+      const int64_t T16 = (T + 15) / 16 * 16;
+      if (kernel > 1) pooled = make({H, T}, at::kFloat);
+      vb = make({H, T16}, at::kByte), counts = make({H, (int64_t)v_bits.size()}, at::kInt), kb = make({H, D}, at::kByte);
+      order = make({H, T}, at::kInt), rank3 = make({H, T}, at::kInt);
+      plan = make({lib.rdkv_pack_layer_plan_ints(H, T)}, at::kInt);
+      if (early) mm = make({H * 2 * D}, at::kFloat);
+      if (keep) v16 = make({H, T}, at::kShort), k16 = make({H, D}, at::kShort);
+      rc = lib.rdkv_select_layer_start(rows, row_stride, H, T, kernel, average, reflect, data<float>(pooled), (float)v_avg,
+                                       v_bits.data(), v_eps.data(), v_bits.size(), zero_col, data<uint8_t>(vb), T16,
+                                       data<int32_t>(counts), data<float>(channels), channels.stride(0), D, (float)k_kept,
+                                       k_bits.data(), k_eps.data(), k_bits.size(), data<uint8_t>(kb), 64, 0.01f, data<int32_t>(order),
+                                       data<int32_t>(rank3), data<int32_t>(plan), data<float>(mm), early ? 2 * D : 0,
+                                       data<int16_t>(v16), data<int16_t>(k16), words, tag, ws, ws_bytes, stream);
+      vb = vb.narrow(1, 0, T);
+    } else if (kernel > 1) {
       pooled = make({H, T}, at::kFloat);
       rc = lib.rdkv_pool_scores(rows, row_stride, H, T, kernel, average, reflect, data<float>(pooled), T, stream);
       rows = data<float>(pooled);
       row_stride = T;
     }
-    if (rc == RDKV_OK) {
+    if (rc == RDKV_OK && !together) {
       vb = make({H, T}, at::kByte), counts = make({H, (int64_t)v_bits.size()}, at::kInt);
       rc = lib.rdkv_knapsack_batched_value(rows, row_stride, H, T, (float)v_avg, nullptr, 0, 0, 0, 0, v_bits.data(), v_eps.data(),
                                            v_bits.size(), 64, 0.01f, 0, data(vb), 1, T, data<int32_t>(counts), ws, ws_bytes,
                                            stream);
     }
-    if (rc == RDKV_OK) {
+    if (rc == RDKV_OK && !together) {
       kb = make({H, D}, at::kByte);
       rc = lib.rdkv_knapsack_batched_value(data<float>(channels), channels.stride(0), H, D, (float)k_kept, data<int32_t>(counts),
                                            v_bits.size(), zero_col, T, D, k_bits.data(), k_eps.data(), k_bits.size(), 64, 0.01f,
                                            0, data(kb), 1, D, nullptr, ws, ws_bytes, stream);
     }
-    if (rc == RDKV_OK) {
+    if (rc == RDKV_OK && !together) {
       order = make({H, T}, at::kInt), rank3 = make({H, T}, at::kInt);
       plan = make({lib.rdkv_pack_layer_plan_ints(H, T)}, at::kInt);
       if (early) mm = make({H * 2 * D}, at::kFloat);
@@ -317,7 +334,7 @@ PyObject *select_layer(PyObject *const *a, Py_ssize_t) {
       rc = lib.rdkv_pack_layers_k_minmax(&K_at, strides, 1, H, T, D, data<int32_t>(order), T, data<int32_t>(plan),
                                          data<float>(mm), 2 * H * D, stream);
     }
-    if (rc == RDKV_OK && keep) v16 = at::_to_copy(vb, at::kShort), k16 = at::_to_copy(kb, at::kShort);
+    if (rc == RDKV_OK && keep && !together) v16 = at::_to_copy(vb, at::kShort), k16 = at::_to_copy(kb, at::kShort);
   }
   status(rc);
   Ref r(PyTuple_New(8));

@@ -698,15 +698,20 @@ __device__ __forceinline__ int wave_sum_uniform(int v) {
          __builtin_amdgcn_readlane(v, 48);
 }
 
-template <int HELD, int NOPT>
-__global__ void __launch_bounds__(kMaxThreads)
-knapsack_group_kernel(const float* __restrict__ scores, int64_t stride_b, int group_rows, int T,
-                      Budget budget, Options o, int max_iters, float tol, void* __restrict__ out,
-                      int out_elem_size, int64_t out_stride_b, int* __restrict__ counts) {
+// The rows first .. first + group_rows, by the first group_rows wavefronts of the workgroup (the others meet its one
+// barrier).  taken(row, score, width): called by the lane of every score.  Returns the counts of the wavefront's row.
+template <int NOPT>
+struct GroupCounts {
+  int n[NOPT];
+};
+template <int HELD, int NOPT, typename Taken>
+__device__ __forceinline__ GroupCounts<NOPT> knapsack_group_rows(const float* __restrict__ scores, int64_t stride_b, int first,
+                                                                 int group_rows, int T, const Budget& budget, const Options& o,
+                                                                 int max_iters, float tol, Taken taken) {
   __shared__ float s_lam0[kGroupMaxRows];
   __shared__ int s_d[kGroupMaxRows];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int b = blockIdx.x * group_rows + wave;
+  const int b = first + (wave < group_rows ? wave : 0);
   const float* row = scores + (int64_t)b * stride_b;
   const float bud = budget(b);
   float se[HELD][NOPT];       // score times eps (+inf for the options past the last: never the smallest)
@@ -760,7 +765,7 @@ knapsack_group_kernel(const float* __restrict__ scores, int64_t stride_b, int gr
       lam = __fmul_rn(lam, 2.0f);
     }
   }
-  if (lane == 0) {
+  if (lane == 0 && wave < group_rows) {
     s_lam0[wave] = lam0;
     s_d[wave] = d;
   }
@@ -800,10 +805,9 @@ knapsack_group_kernel(const float* __restrict__ scores, int64_t stride_b, int gr
   float lb[NOPT];
 #pragma unroll
   for (int k = 0; k < NOPT; ++k) lb[k] = __fmul_rn(lam_final, o.bits[k]);
-  uint8_t* out_row = reinterpret_cast<uint8_t*>(out) + (int64_t)b * out_stride_b * out_elem_size;
-  int cnt[NOPT];
+  GroupCounts<NOPT> cnt;
 #pragma unroll
-  for (int k = 0; k < NOPT; ++k) cnt[k] = 0;
+  for (int k = 0; k < NOPT; ++k) cnt.n[k] = 0;
 #pragma unroll
   for (int j = 0; j < HELD; ++j) {
     const int t = lane + 64 * j;
@@ -811,19 +815,199 @@ knapsack_group_kernel(const float* __restrict__ scores, int64_t stride_b, int gr
     const int idx = pick(j, lb, w);
     if (t < T) {
 #pragma unroll
-      for (int k = 0; k < NOPT; ++k) cnt[k] += k == idx ? 1 : 0;
-      if (out_elem_size == 1) out_row[t] = (uint8_t)w;
-      else reinterpret_cast<int64_t*>(out_row)[t] = (int64_t)w;
+      for (int k = 0; k < NOPT; ++k) cnt.n[k] += k == idx ? 1 : 0;
+      if (wave < group_rows) taken(b, t, w);
     }
   }
+  return cnt;
+}
+
+template <int HELD, int NOPT>
+__global__ void __launch_bounds__(kMaxThreads)
+knapsack_group_kernel(const float* __restrict__ scores, int64_t stride_b, int group_rows, int T,
+                      Budget budget, Options o, int max_iters, float tol, void* __restrict__ out,
+                      int out_elem_size, int64_t out_stride_b, int* __restrict__ counts) {
+  const auto cnt = knapsack_group_rows<HELD, NOPT>(
+      scores, stride_b, blockIdx.x * group_rows, group_rows, T, budget, o, max_iters, tol, [&](int b, int t, int w) {
+        if (out_elem_size == 1) reinterpret_cast<uint8_t*>(out)[(int64_t)b * out_stride_b + t] = (uint8_t)w;
+        else reinterpret_cast<int64_t*>(out)[(int64_t)b * out_stride_b + t] = (int64_t)w;
+      });
   if (counts != nullptr) {
+    const int b = blockIdx.x * group_rows + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
     for (int k = 0; k < NOPT; ++k) {
       if (k < o.n) {
-        const int total = wave_sum_uniform(cnt[k]);
-        if (lane == 0) counts[(int64_t)b * o.n + k] = total;
+        const int total = wave_sum_uniform(cnt.n[k]);
+        if ((threadIdx.x & 63) == 0) counts[(int64_t)b * o.n + k] = total;
       }
     }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// The K allocation of a layer and the token order of its V allocation in one launch: neither needs the other, and both
+// stand between the V allocation and the host, which sizes the packed tensors by what they find.  As launches of
+// their own (the K rows 7 us on one compute unit, a histogram of the widths, the order) they followed each other.
+//  * Workgroup (0, 0): the K rows, a wavefront each; their class counts.
+//  * Workgroups (chunk, 1 + head): 1024 tokens of a head each.  What lies ahead of its tokens a workgroup counts itself,
+//    from all of the row's bytes (16 a load; a dword's four widths by one count of set bits per class), instead of reading
+//    a histogram that another launch has written; beyond 64k tokens that would be more than the histogram's launch.
+// With the exchange words cleared by the pooling launch, three launches instead of nine (two of them conversions of the
+// widths to int16) up to the host's read: a selected layer of 8 heads, 4k / 31k tokens 108.0 / 109.8 -> 97.1 / 97.3 us.
+// Results and words as plan_hist_kernel and plan_scatter_kernel leave them (pack_plan.hip).
+// ---------------------------------------------------------------------------------------------
+constexpr int kOrderThreads = 1024;
+constexpr int64_t kOrderMaxTokens = 65536;
+struct OrderArgs {
+  const uint8_t* v_bits;          // rows of v_stride bytes, a multiple of 16
+  int64_t v_stride;
+  int T, H;
+  int32_t *order, *rank3;         // [H, T]
+  int32_t *counts4, *info;
+  uint32_t* minmax;
+  int minmax_per_head, D;
+  int16_t *v16, *k16;             // the widths as [H, T] and [H, D], or null
+  uint64_t* words;
+  uint32_t tag;
+};
+struct KRows {
+  const float* scores;
+  int64_t stride_b;
+  Options o;
+  uint8_t* out;                   // [H, D]
+};
+
+__device__ __forceinline__ int width_class(uint32_t w) {
+  return w == 2 ? 0 : w == 4 ? 1 : w == 8 ? 2 : w == 16 ? 3 : w == 0 ? 4 : 5;
+}
+
+template <int HELD, int NOPT>
+__global__ void __launch_bounds__(kOrderThreads)
+select_order_kernel(OrderArgs a, KRows k, Budget budget, int max_iters, float tol) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (blockIdx.y == 0) {
+    if (blockIdx.x > 0) return;
+    int own[4] = {0, 0, 0, 0};    // this lane's channels of 2, 4, 8 or 16 bit, and of another width
+    knapsack_group_rows<HELD, NOPT>(k.scores, k.stride_b, 0, a.H, a.D, budget, k.o, max_iters, tol, [&](int b, int t, int w) {
+      k.out[(int64_t)b * a.D + t] = (uint8_t)w;
+      if (a.k16) a.k16[(int64_t)b * a.D + t] = (int16_t)w;
+      own[0] += w == 2 ? 1 : 0;
+      own[1] += w == 4 ? 1 : 0;
+      own[2] += w == 8 || w == 16 ? 1 : 0;
+      own[3] += w != 0 && w != 2 && w != 4 && w != 8 && w != 16 ? 1 : 0;
+    });
+    if (wave < a.H) {
+      const int n2 = wave_sum_uniform(own[0]), n4 = wave_sum_uniform(own[1]), n8 = wave_sum_uniform(own[2]);
+      const int bad = wave_sum_uniform(own[3]);
+      if (lane < 6) {
+        const int v = lane == 0 ? n2 : lane == 1 ? n4 : lane == 2 ? n8 : lane == 3 ? bad : 0;
+        a.info[8 * wave + 2 + lane] = v;
+        rdkv_host_word(a.words, 12 * (int64_t)wave + 6 + lane, a.tag, v);
+      }
+    }
+    return;
+  }
+  constexpr int kWaves = kOrderThreads / 64;
+  __shared__ int wsum[kWaves][10];             // all of the row's tokens by class 2, 4, 8, 16 bit, other; those ahead
+  __shared__ int wcnt[kWaves][6], wpre[kWaves][6], red[12];
+  const int h = blockIdx.y - 1, chunk = blockIdx.x, T = a.T;
+  const uint8_t* row = a.v_bits + (int64_t)h * a.v_stride;
+  const int t = chunk * kOrderThreads + tid;
+  const uint32_t width = t < T ? row[t] : 0u;
+  int all[5] = {0, 0, 0, 0, 0}, ahead[5] = {0, 0, 0, 0, 0};
+  const int vectors = (T + 15) / 16, before = chunk * (kOrderThreads / 16);
+  for (int v = tid; v < vectors; v += kOrderThreads) {
+    const uint4 q = reinterpret_cast<const uint4*>(row)[v];
+    uint32_t w[4] = {q.x, q.y, q.z, q.w};
+    int n[5] = {0, 0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int left = T - (16 * v + 4 * e);         // bytes past the row's end hold anything
+      if (left < 4) w[e] = left <= 0 ? 0u : w[e] & ((1u << (8 * left)) - 1u);
+      const uint32_t one = w[e] & 0x1e1e1e1eu;
+      // (more bits in a byte than the widths have, or more than one of them: byte by byte)
+      const uint32_t two = one & ((one | 0x80808080u) - 0x01010101u) & 0x1e1e1e1eu;
+      if (one != w[e] || two != 0) {
+        for (int i = 0; i < 4; ++i) {
+          const int c = width_class((w[e] >> (8 * i)) & 255u);
+#pragma unroll
+          for (int m = 0; m < 4; ++m) n[m] += c == m ? 1 : 0;
+          n[4] += c == 5 ? 1 : 0;
+        }
+      } else {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) n[m] += __popc(one & (0x02020202u << m));
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < 5; ++m) {
+      all[m] += n[m];
+      ahead[m] += v < before ? n[m] : 0;
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < 5; ++m) {
+    const int s_all = wave_sum_uniform(all[m]), s_ahead = wave_sum_uniform(ahead[m]);
+    if (lane == 0) {
+      wsum[wave][m] = s_all;
+      wsum[wave][5 + m] = s_ahead;
+    }
+  }
+  const int cls = t < T ? width_class(width) : -1;
+  int my_rank = 0;
+  uint64_t qmask = 0;
+  auto lanes_below = [](uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+  };
+#pragma unroll
+  for (int m = 0; m < 6; ++m) {
+    const uint64_t in = __ballot(cls == m);
+    if (m < 3) qmask |= in;
+    if (cls == m) my_rank = lanes_below(in);
+    if (lane == 0) wcnt[wave][m] = __popcll(in);
+  }
+  const int my_q = lanes_below(qmask);
+  __syncthreads();
+  if (tid < 10) {
+    int s = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) s += wsum[w][tid];
+    red[tid < 4 ? tid : tid == 4 ? 5 : tid < 9 ? 1 + tid : 11] = s;      // [0 .. 5] all, [6 .. 11] ahead, by class
+  } else if (tid >= 64 && tid < 70) {
+    const int m = tid - 64;
+    int s = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      wpre[w][m] = s;
+      s += wcnt[w][m];
+    }
+  }
+  __syncthreads();
+  // (class 4, evicted, is what the others leave)
+  const int evicted = T - (red[0] + red[1] + red[2] + red[3] + red[5]);
+  const int evicted_ahead = chunk * kOrderThreads - (red[6] + red[7] + red[8] + red[9] + red[11]);
+  int pos = 0, before_q = 0, base = 0;
+#pragma unroll
+  for (int m = 0; m < 6; ++m) {
+    const int before_me = (m == 4 ? evicted_ahead : red[6 + m]) + wpre[wave][m];
+    if (cls == m) pos = base + before_me + my_rank;
+    if (m < 3) before_q += before_me;
+    base += m == 4 ? evicted : red[m];
+  }
+  if (t < T) {
+    a.order[(int64_t)h * T + pos] = t;
+    a.rank3[(int64_t)h * T + t] = before_q + my_q;
+    if (a.v16) a.v16[(int64_t)h * T + t] = (int16_t)width;
+  }
+  if (chunk == 0) {
+    if (tid < 6) {
+      const int v = tid == 4 ? evicted : red[tid];
+      if (tid < 4) a.counts4[4 * h + tid] = v;
+      else a.info[8 * h + tid - 4] = v;
+      rdkv_host_word(a.words, 12 * (int64_t)h + tid, a.tag, v);
+    }
+    for (int i = tid; a.minmax && i < a.minmax_per_head; i += kOrderThreads)
+      a.minmax[(int64_t)h * a.minmax_per_head + i] = rdkv_float_to_ordered(((i / a.D) & 1) ? -__builtin_inff() : __builtin_inff());
   }
 }
 
@@ -862,8 +1046,10 @@ knapsack_rows_kernel(const float* __restrict__ scores, int64_t stride_b, int T,
 // out[b, l] over the window l-pad .. l-pad+k-1 of row b; left-to-right fp32 sum from 0, one division.
 template <bool AVG, bool REFLECT>
 __global__ void pool_kernel(const float* __restrict__ in, int64_t in_stride_b, int T, int k, int pad,
-                            float* __restrict__ out, int64_t out_stride_b, int L) {
+                            float* __restrict__ out, int64_t out_stride_b, int L, uint32_t* clear, int clear_words) {
   const int l = blockIdx.x * blockDim.x + threadIdx.x;
+  // (the row's exchange words of the allocation that follows, for which they would be a launch ahead of it)
+  for (int i = l; i < clear_words; i += gridDim.x * blockDim.x) clear[(int64_t)blockIdx.y * clear_words + i] = 0u;
   if (l >= L) return;
   const float* row = in + (int64_t)blockIdx.y * in_stride_b;
   float acc = AVG ? 0.f : -__builtin_inff();
@@ -1009,10 +1195,14 @@ RDKV_API int64_t rdkv_knapsack_workspace_bytes(int B) {
   return b * 8 + 256 + b * (int64_t)kCoopRowWords * 4;
 }
 
+static uint32_t* coop_state(void* workspace, int B) {
+  return reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(workspace) + (((int64_t)B * 8 + 255) / 256) * 256);
+}
+
 static int knapsack_batched(const float* scores, int64_t stride_b, int B, int64_t T, const Budget& budget,
                             const void* given, const float* bits_host, const float* eps_host, int n_options, int max_iters, float tol,
                             int group_rows, void* out, int out_elem_size, int64_t out_stride_b, int32_t* counts,
-                            void* workspace, int64_t workspace_bytes, void* stream) {
+                            void* workspace, int64_t workspace_bytes, void* stream, bool cleared = false) {
   Options o;
   if (int rc = make_options(bits_host, eps_host, n_options, &o)) return rc;
   if (int rc = check_common(scores, B, T, given, out, out_elem_size)) return rc;
@@ -1031,10 +1221,10 @@ static int knapsack_batched(const float* scores, int64_t stride_b, int B, int64_
   int sets = 0;      // (log2)
   if (const int S = coop_split(B, T, max_iters, &sets)) {
     // few long rows: every row shared by S workgroups, one launch after clearing its state
-    uint8_t* base = reinterpret_cast<uint8_t*>(workspace) + (((int64_t)B * 8 + 255) / 256) * 256;
-    uint32_t* state = reinterpret_cast<uint32_t*>(base);
+    uint32_t* state = coop_state(workspace, B);
     const int64_t n_words = (int64_t)B * kCoopRowWords;
-    hipLaunchKernelGGL(coop_init_kernel, dim3((unsigned)rdkv_cdiv(n_words, 256)), dim3(256), 0, s, state, n_words);
+    if (!cleared)
+      hipLaunchKernelGGL(coop_init_kernel, dim3((unsigned)rdkv_cdiv(n_words, 256)), dim3(256), 0, s, state, n_words);
     const int64_t chunk = (T + S - 1) / S;
     hipLaunchKernelGGL(kCoopKernels[sets][coop_held_index(chunk)], dim3((unsigned)(B * S)), dim3(kCoopLanes << sets), 0, s,
                        scores, stride_b, group_rows, (int)T, S,
@@ -1104,8 +1294,8 @@ RDKV_API int rdkv_knapsack_rows(const float* scores, int64_t stride_b, int B, in
   return RDKV_OK;
 }
 
-RDKV_API int rdkv_pool_scores(const float* scores, int64_t stride_b, int B, int64_t T, int kernel_size,
-                              int is_avg, int reflect, float* out, int64_t out_stride_b, void* stream) {
+static int pool_scores(const float* scores, int64_t stride_b, int B, int64_t T, int kernel_size, int is_avg, int reflect,
+                       float* out, int64_t out_stride_b, uint32_t* clear, void* stream) {
   if (B < 0 || T < 0 || kernel_size < 1) return fail("pool_scores: bad size");
   if (T > (1 << 30)) return fail("pool_scores: row too long");
   int k = kernel_size;
@@ -1122,11 +1312,74 @@ RDKV_API int rdkv_pool_scores(const float* scores, int64_t stride_b, int B, int6
   const dim3 grid((unsigned)((L + 255) / 256), (unsigned)B), block(256);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
 #define RDKV_POOL(A, R) \
-  hipLaunchKernelGGL((pool_kernel<A, R>), grid, block, 0, s, scores, stride_b, (int)T, k, pad, out, out_stride_b, (int)L)
+  hipLaunchKernelGGL((pool_kernel<A, R>), grid, block, 0, s, scores, stride_b, (int)T, k, pad, out, out_stride_b, (int)L, \
+                     clear, clear ? kCoopRowWords : 0)
   if (is_avg) { if (reflect) RDKV_POOL(true, true); else RDKV_POOL(true, false); }
   else        { if (reflect) RDKV_POOL(false, true); else RDKV_POOL(false, false); }
 #undef RDKV_POOL
   RDKV_CHECK_LAUNCH("rdkv_pool_scores");
+  return RDKV_OK;
+}
+
+RDKV_API int rdkv_pool_scores(const float* scores, int64_t stride_b, int B, int64_t T, int kernel_size,
+                              int is_avg, int reflect, float* out, int64_t out_stride_b, void* stream) {
+  return pool_scores(scores, stride_b, B, T, kernel_size, is_avg, reflect, out, out_stride_b, nullptr, stream);
+}
+
+// What rdkv_pool_scores, the V and the K allocation and rdkv_pack_layer_plan_start do for a layer, in three launches.
+RDKV_API int rdkv_select_layer_start(const float* scores, int64_t stride_b, int H, int64_t T, int kernel_size, int is_avg,
+                                     int reflect, float* pooled, float v_budget, const float* v_bits_host,
+                                     const float* v_eps_host, int n_v_options, int zero_option, uint8_t* v_bits,
+                                     int64_t v_stride, int32_t* v_counts, const float* channels, int64_t channel_stride, int D,
+                                     float k_kept_bits, const float* k_bits_host, const float* k_eps_host, int n_k_options,
+                                     uint8_t* k_bits, int max_iters, float tol, int32_t* order, int32_t* rank3, int32_t* plan,
+                                     float* minmax_ws, int minmax_floats_per_head, int16_t* v_bits16, int16_t* k_bits16,
+                                     uint64_t* host_words, uint32_t tag, void* workspace, int64_t workspace_bytes, void* stream) {
+  if (H < 1 || H > kGroupMaxRows || T < 1 || T > kOrderMaxTokens || D < 1 || D > 64 * kGroupMaxHeld) {
+    rdkv_set_error("rdkv_select_layer_start: %d heads of %lld tokens and %d channels", H, (long long)T, D);
+    return RDKV_EUNSUPPORTED;
+  }
+  if (!v_counts || !channels || !k_bits || !order || !rank3 || !plan || !host_words || v_stride < T || v_stride % 16 != 0 ||
+      reinterpret_cast<uintptr_t>(v_bits) % 16 != 0 || zero_option >= n_v_options || channel_stride < D)
+    return fail("rdkv_select_layer_start: bad arguments");
+  if (workspace == nullptr || workspace_bytes < rdkv_knapsack_workspace_bytes(H)) {
+    rdkv_set_error("rdkv_select_layer_start: workspace too small");
+    return RDKV_EWORKSPACE;
+  }
+  if (max_iters < 0) return fail("knapsack: negative max_iters");
+  Options ko;
+  if (int rc = make_options(k_bits_host, k_eps_host, n_k_options, &ko)) return rc;
+  bool cleared = false;
+  const float* rows = scores;
+  int64_t row_stride = stride_b;
+  if (kernel_size > 1) {
+    int sets = 0;
+    cleared = coop_split(H, T, max_iters, &sets) > 0;
+    if (int rc = pool_scores(scores, stride_b, H, T, kernel_size, is_avg, reflect, pooled, T, cleared ? coop_state(workspace, H) : nullptr,
+                             stream))
+      return rc;
+    rows = pooled;
+    row_stride = T;
+  }
+  if (int rc = knapsack_batched(rows, row_stride, H, T, Budget{nullptr, nullptr, 0, 0, 0, 0.f, v_budget}, rows, v_bits_host, v_eps_host,
+                                n_v_options, max_iters, tol, H, v_bits, 1, v_stride, v_counts, workspace, workspace_bytes, stream,
+                                cleared))
+    return rc;
+  OrderArgs a;
+  a.v_bits = v_bits; a.v_stride = v_stride; a.T = (int)T; a.H = H; a.order = order; a.rank3 = rank3;
+  a.counts4 = plan; a.info = plan + 4 * H; a.minmax = reinterpret_cast<uint32_t*>(minmax_ws);
+  a.minmax_per_head = minmax_floats_per_head; a.D = D; a.v16 = v_bits16; a.k16 = k_bits16; a.words = host_words; a.tag = tag;
+  const KRows k = {channels, channel_stride, ko, k_bits};
+  const Budget kept = {nullptr, v_counts, n_v_options, zero_option, (int)T, (float)D, k_kept_bits};
+  const dim3 grid((unsigned)rdkv_cdiv(T, kOrderThreads), (unsigned)(H + 1));
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+#define RDKV_LAUNCH_ORDER(HELD, NOPT) \
+  hipLaunchKernelGGL((select_order_kernel<HELD, NOPT>), grid, dim3(kOrderThreads), 0, s, a, k, kept, max_iters, tol)
+  if (D <= 128 && ko.n <= 5) RDKV_LAUNCH_ORDER(2, 5);
+  else if (ko.n <= 5) RDKV_LAUNCH_ORDER(4, 5);
+  else RDKV_LAUNCH_ORDER(4, kMaxOptions);
+#undef RDKV_LAUNCH_ORDER
+  RDKV_CHECK_LAUNCH("rdkv_select_layer_start");
   return RDKV_OK;
 }
 
