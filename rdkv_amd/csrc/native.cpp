@@ -29,8 +29,8 @@ namespace {
   X(rdkv_pool_scores) X(rdkv_knapsack_batched_value) X(rdkv_pack_layer_plan_ints) X(rdkv_pack_layer_plan_start)  \
   X(rdkv_pack_layers_k_minmax) X(rdkv_pack_layer_v_rows) X(rdkv_pack_layer_tables) X(rdkv_pack_layer_k_rows)     \
   X(rdkv_decode_fused) X(rdkv_decode_fused_zone_c) X(rdkv_decode_fused_workspace_bytes)                           \
-  X(rdkv_unpack_layer_k_words) X(rdkv_unpack_layer_v_words) X(rdkv_stream_plan_layer) X(rdkv_pack_layer_stream)   \
-  X(rdkv_select_layer_start)
+  X(rdkv_unpack_layer_k_words) X(rdkv_unpack_layer_v_words) X(rdkv_stream_plan_layer)   \
+  X(rdkv_select_layer_start) X(rdkv_pack_layers_stream)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
   RDKV_NATIVE_FUNCTIONS(X)
@@ -368,19 +368,18 @@ std::vector<at::Tensor> tensors(PyObject *list) {
 }
 constexpr int kSlots = 160;       // columns of a unit's slot table
 
-// K, V, V widths, K widths (lists: an entry each), tokens from which K min / max go ahead, words, tag, stream
+// K, V, V widths, K widths (lists: an entry each), words, tag, stream
 PyObject *stream_order(PyObject *const *a, Py_ssize_t) {
   const std::vector<at::Tensor> Ks = tensors(a[0]), Vs = tensors(a[1]);
   std::vector<at::Tensor> vbs = tensors(a[2]), kbs = tensors(a[3]);
-  const int64_t n = Ks.size(), early_from = integer(a[4]);
-  auto *words = static_cast<uint64_t *>(address(a[5]));
-  const uint32_t tag = (uint32_t)integer(a[6]);
-  void *stream = address(a[7]);
+  const int64_t n = Ks.size();
+  auto *words = static_cast<uint64_t *>(address(a[4]));
+  const uint32_t tag = (uint32_t)integer(a[5]);
+  void *stream = address(a[6]);
   plain((int64_t)Vs.size() == n && (int64_t)vbs.size() == n && (int64_t)kbs.size() == n && Ks[0].is_cuda() && Ks[0].dim() == 4);
   const auto dev = Ks[0].device();
   const int64_t H = Ks[0].size(1), T = Ks[0].size(2);
   plain(H >= 1 && T >= 1 && T <= (1 << 30) && n * H <= 65535);
-  bool early = T >= early_from;
   auto widths = [&](const std::vector<at::Tensor> &ts, int64_t w) {
     const auto type = ts[0].scalar_type();
     plain(type == at::kByte || type == at::kShort || type == at::kInt || type == at::kLong);
@@ -408,11 +407,11 @@ PyObject *stream_order(PyObject *const *a, Py_ssize_t) {
     vb = n == 1 ? vbs[0] : at::cat(vbs), kb = n == 1 ? kbs[0] : at::cat(kbs);
     order = make({n * H, T}, at::kInt), rank3 = make({n * H, T}, at::kInt);
     plan = make({lib.rdkv_pack_layer_plan_ints(n * H, T)}, at::kInt);
-    if (early) mm = make({n * H * 768}, at::kFloat);
+    mm = make({n * H * 768}, at::kFloat);
     rc = lib.rdkv_pack_layer_plan_start(vb.data_ptr(), vb.element_size(), T, kb.data_ptr(), kb.element_size(), 128, n * H, T, 128,
                                         data<int32_t>(order), T, data<int32_t>(rank3), T, data<int32_t>(plan), data<float>(mm),
-                                        early ? 768 : 0, words, tag, stream);
-    if (rc == RDKV_OK && early)
+                                        768, words, tag, stream);
+    if (rc == RDKV_OK)
       rc = lib.rdkv_pack_layers_k_minmax(K_at.data(), strides.data(), n, H, T, 128, data<int32_t>(order), T, data<int32_t>(plan),
                                          data<float>(mm), 768 * H, stream);
   }
@@ -455,38 +454,39 @@ PyObject *stream_tables(PyObject *const *a, Py_ssize_t) {
   Py_RETURN_TRUE;
 }
 
-// The entries' blobs, packed; the units' offsets become addresses.  K, V, order, plan, K widths, min / max, how far they
-// are, units (host), units, slots (device), sizes, dimensions, largest scales [n][2][H], stream
+// The entries' blobs, packed; the units' offsets become addresses.  K, V, order, plan, K widths, min / max, units
+// (host), units, slots (device), sizes, dimensions, largest scales [n][2][H], stream
 PyObject *stream_pack(PyObject *const *a, Py_ssize_t) {
   const std::vector<at::Tensor> Ks = tensors(a[0]), Vs = tensors(a[1]);
-  const at::Tensor &order = tensor(a[2]), &plan = tensor(a[3]), &kb = tensor(a[4]), &mm = tensor(a[5]), &units = tensor(a[8]),
-                   &slots = tensor(a[9]), &scales = tensor(a[12]);
-  const int ready = (int)integer(a[6]);
-  void *stream = address(a[13]);
+  const at::Tensor &order = tensor(a[2]), &plan = tensor(a[3]), &kb = tensor(a[4]), &mm = tensor(a[5]), &units = tensor(a[7]),
+                   &slots = tensor(a[8]), &scales = tensor(a[11]);
+  void *stream = address(a[12]);
   const int64_t n = Ks.size(), H = Ks[0].size(1), T = Ks[0].size(2);
-  Buffer host(a[7], true), sizes(a[10]), dims(a[11]);
+  Buffer host(a[6], true), sizes(a[9]), dims(a[10]);
   auto *unit_p = host.of<RdkvUnit>(n * H);
   const auto *size_p = sizes.of<int64_t>(4 * n);
   const auto *dim_p = dims.of<int32_t>(5 * n);
   plain(shape_is(order, {n * H, T}) && shape_is(scales, {n, 2, H}) && shape_is(kb, {n * H, 128}) && kb.is_contiguous());
   plain(units.numel() >= n * H * (int64_t)sizeof(RdkvUnit) && slots.numel() >= n * H * kSlots * 2);
-  plain(mm.numel() >= (ready == 2 ? n : 1) * H * 768);
+  plain(mm.numel() >= n * H * 768);
   std::vector<at::Tensor> blobs;
+  std::vector<RdkvStreamLayer> layers;
   int rc = RDKV_OK;
   {
     Unlocked u;
-    for (int64_t e = 0; e < n && rc == RDKV_OK; ++e) {
+    for (int64_t e = 0; e < n; ++e) {
       const int32_t *d = dim_p + 5 * e;
       // (256 bytes of slack for 16-byte reads at the end; the launches write every other byte)
       const int64_t bytes = std::max<int64_t>(size_p[4 * e], 256) + 256;
       blobs.push_back(at::empty({bytes}, Ks[e].options().dtype(at::kByte)));
-      auto *blob = data<uint8_t>(blobs.back());
-      rc = lib.rdkv_pack_layer_stream(
-          Ks[e].data_ptr(), Vs[e].data_ptr(), Ks[e].stride(1), Ks[e].stride(2), H, data<int32_t>(order) + e * H * T, T,
-          data<int32_t>(plan) + 4 * e * H, data<uint8_t>(kb) + e * H * 128 * kb.element_size(), kb.element_size(), 128, d[0], d[1],
-          d[2], d[3], d[4], data<RdkvUnit>(units) + e * H, data<int16_t>(slots) + e * H * kSlots, kSlots, size_p[4 * e + 1], blob,
-          bytes, data<float>(mm) + (ready == 2 ? 768 * e * H : 0), ready, data<float>(scales) + 2 * e * H, stream);
-      const uint64_t base = reinterpret_cast<uintptr_t>(blob);
+      layers.push_back({Ks[e].data_ptr(), Vs[e].data_ptr(), Ks[e].stride(1), Ks[e].stride(2), data<uint8_t>(blobs.back()), bytes,
+                        d[3], d[0], d[1], d[2], d[4], (int32_t)size_p[4 * e + 1], 0});
+    }
+    rc = lib.rdkv_pack_layers_stream(layers.data(), n, H, data<int32_t>(order), T, data<int32_t>(plan), data<uint8_t>(kb),
+                                     kb.element_size(), 128, data<RdkvUnit>(units), data<int16_t>(slots), kSlots, data<float>(mm),
+                                     data<float>(scales), stream);
+    for (int64_t e = 0; e < n && rc == RDKV_OK; ++e) {
+      const uint64_t base = reinterpret_cast<uintptr_t>(layers[e].blob);
       for (RdkvUnit *p = unit_p + e * H; p < unit_p + (e + 1) * H; ++p) {
         p->k_off += base, p->sz_off += base, p->qtab_off += base;
         for (auto &v : p->v_off) v += base;
@@ -695,9 +695,9 @@ PyMethodDef kMethods[] = {
     {"names", names, METH_NOARGS, "The library functions that bind asks for."},
     ENTRY(pack_layer, 13, "The tensors of a planned layer: (fields of the layer, fp16-kept V rows), or None."),
     ENTRY(select_layer, 19, "Widths and token order of a layer: (v_bits, k_bits, order, rank3, plan, min / max, int16 widths), or None."),
-    ENTRY(stream_order, 8, "Token order of the layers: (order, plan, K widths, min / max), or None."),
+    ENTRY(stream_order, 7, "Token order of the layers: (order, plan, K widths, min / max), or None."),
     ENTRY(stream_tables, 9, "Fills the units, slot tables, sizes and dimensions of the layers: True, or None."),
-    ENTRY(stream_pack, 14, "The blobs of the layers, or None."),
+    ENTRY(stream_pack, 13, "The blobs of the layers, or None."),
     ENTRY(decode_attn, 16, "(out, lse) of a decode step, or None."),
     ENTRY(dense_layer, 7, "Dense (K, V) of a packed layer, or None."),
     {nullptr, nullptr, 0, nullptr}};

@@ -58,6 +58,15 @@ struct StreamPackArgs {
   int H_kv;
   int64_t blob_bytes;
 };
+// The layers of a launch, one per blockIdx.z.
+constexpr int kBatchLayers = 8;
+struct StreamPackBatch {
+  StreamPackArgs layer[kBatchLayers];
+};
+// where a layer's channel parameters lie in its scratch
+__device__ __forceinline__ float4 *chan_params_of(const StreamPackArgs &a) {
+  return reinterpret_cast<float4 *>(a.mm + (int64_t)a.H_kv * 2 * kD);
+}
 
 // The K quantizer of one channel: scale, zero point, 1 / scale (rdkv_qcode's estimate) and, as bits,
 // the channel's stream slot with its width class (slot | class << 8; -1 for a channel that is not
@@ -74,7 +83,9 @@ __device__ __forceinline__ float4 make_chan(float scale, float zp, float inv, in
 // alignment gap behind it, and behind the last head the rest of the blob: no byte of the blob is
 // left to the caller), and starts the head's two scale maxima.
 __global__ void __launch_bounds__(128)
-slot_params_kernel(StreamPackArgs a, float4 *__restrict__ chan_params) {
+slot_params_kernel(StreamPackBatch batch) {
+  const StreamPackArgs &a = batch.layer[blockIdx.z];
+  float4 *chan_params = chan_params_of(a);
   __shared__ int ch_of[3 * kD], first_wave_count[3], slot_of_ch[kD];
   __shared__ float4 slot_p[kMaxSlots];
   __shared__ float wave_max[2];
@@ -194,14 +205,13 @@ __device__ __forceinline__ float row16_bcast(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xF, 0xF, false));
 }
 
-// The V tile of class CLS from the tile's code bytes (fp16 bits for the fp16-kept class): thread
-// (l, g) assembles the dwords that hold channels l and l + 64 of quads 4g .. 4g + 3
+// The V tile of class CLS from the code bytes of a wavefront's sixteen tokens, the first nv of which are there (fp16 bits
+// for the fp16-kept class): lane l assembles the dwords that hold channels l and l + 64 of its quads 4g .. 4g + 3
 // (stream_format.h: element k of an operand is token 4 * quad + k; 8-bit dword 2 * quad + j, 4-bit
 // dword quad with operand j, 2-bit dword quad >> 1 with operand 2 * (quad & 1) + j; j = channel half).
 template <int CLS>
-__device__ __forceinline__ void v_tile(const uint8_t (*cv)[kD], const uint16_t (*raw)[kD], int nv,
-                                       uint32_t *v_out) {
-  const int l = threadIdx.x & 63, g = threadIdx.x >> 6;
+__device__ __forceinline__ void v_tile(const uint8_t (*cv)[kD], const uint16_t (*raw)[kD], int nv, int g, uint32_t *v_out) {
+  const int l = threadIdx.x & 63;
   // dword di of lane l sits at v_out[((di >> 2) * 64 + l) * 4 + (di & 3)]: a lane's dwords 4n .. 4n + 3 are 16 contiguous bytes
   uint4 *out4 = reinterpret_cast<uint4 *>(v_out);
   if (CLS == 3) {
@@ -213,7 +223,7 @@ __device__ __forceinline__ void v_tile(const uint8_t (*cv)[kD], const uint16_t (
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-          const int t = 4 * quad + k;
+          const int t = 4 * q + k;
           const uint32_t bits = t < nv ? (uint32_t)raw[t][l + 64 * j] : 0u;
           w[2 * j + (k >> 1)] |= bits << (16 * (k & 1));
         }
@@ -226,10 +236,9 @@ __device__ __forceinline__ void v_tile(const uint8_t (*cv)[kD], const uint16_t (
   uint32_t w8[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};   // class 2: dwords 8g .. 8g + 7; class 1: 4g .. 4g + 3; class 0: 2g, 2g + 1
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int quad = 4 * g + q;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      const int t = 4 * quad + k;
+      const int t = 4 * q + k;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const uint32_t c = t < nv ? (uint32_t)cv[t][l + 64 * j] : 0u;
@@ -285,65 +294,73 @@ __device__ __forceinline__ TileInfo tile_info(const RdkvUnit &u, int ti) {
   return r;
 }
 
-// Workgroup (x, head) takes the head's 64-token tiles x, x + gridDim.x, ...  Thread (p = tid % 16,
-// r = tid / 16) loads 16 bytes (eight channels, 8p .. 8p + 7) of the K and the V row of tokens r,
-// r + 16, r + 32, r + 48 and turns them into codes in registers: the K parameters of its eight
-// channels stay in registers for every tile, the V parameters of a token come from a min / max over
-// the sixteen lanes that hold it.  Codes are parked in LDS as bytes (K at its stream slot, V at its
-// channel), from where the dwords of the K rows and of the V tile are assembled and stored
-// coalesced.  The token indices of the workgroup's next tile are requested before the current tile
-// is worked on; several workgroups share a compute unit and cover each other's waits.
+// Workgroup (x, head) takes the head's 64-token tiles x, x + gridDim.x, ..., a quarter of a tile to each of its four
+// wavefronts, which share nothing but the channel table: every quad of tokens and every K row lies within a quarter.
+// Lane (p = lane % 16, r = lane / 16) loads 16 bytes (eight channels, 8p .. 8p + 7) of the K and the V row of tokens r,
+// r + 4, r + 8, r + 12 of the quarter and turns them into codes in registers: the V parameters of a token come from a
+// min / max over the sixteen lanes that hold it.  Codes are parked in LDS as bytes (K at its stream slot, V at its
+// channel), from where the dwords of the K rows and of the V tile are assembled and stored coalesced.
+// Latency bound (half of a wavefront's cycles were waits, 46 % of the vector issue slots used): the rows of the next tile
+// are requested as soon as the codes are parked, into the registers that held this tile's, and come in under the
+// assembly; nothing makes a wavefront wait for another.  One layer of 8 x 32k tokens 46.5 -> 30.5 us.
 __global__ void __launch_bounds__(256, 3)
-stream_pack_kernel(StreamPackArgs a, const float4 *__restrict__ chan_params) {
-  __shared__ __align__(16) uint8_t ck[RDKV_TILE][kMaxSlots];        // K code of (token, stream slot)
-  __shared__ __align__(16) uint8_t cv_bytes[RDKV_TILE * kD * 2];    // V code of (token, channel); fp16 bits for class 3
-  __shared__ float4 chan[kD];                                       // the head's channel quantizers
-  uint8_t (*cv)[kD] = reinterpret_cast<uint8_t (*)[kD]>(cv_bytes);
-  uint16_t (*raw)[kD] = reinterpret_cast<uint16_t (*)[kD]>(cv_bytes);
-  const int h = blockIdx.y, tid = threadIdx.x, stride = gridDim.x;
+stream_pack_kernel(StreamPackBatch batch) {
+  const StreamPackArgs a = batch.layer[blockIdx.z];
+  const float4 *chan_params = chan_params_of(a);
+  constexpr int kRows = RDKV_TILE / 4;                                          // tokens of a wavefront
+  __shared__ __align__(16) uint8_t ck_all[4][kRows][kMaxSlots];                 // K code of (token, stream slot)
+  __shared__ __align__(16) uint8_t cv_all[4][kRows * kD * 2];                   // V code of (token, channel); fp16 bits for class 3
+  __shared__ float4 chan[kD];                                                   // the head's channel quantizers
+  const int h = blockIdx.y, tid = threadIdx.x, stride = gridDim.x, lane = tid & 63;
+  const int g = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint8_t (*ck)[kMaxSlots] = ck_all[g];
+  uint8_t (*cv)[kD] = reinterpret_cast<uint8_t (*)[kD]>(cv_all[g]);
+  uint16_t (*raw)[kD] = reinterpret_cast<uint16_t (*)[kD]>(cv_all[g]);
   const RdkvUnit u = a.units[h];
   const int R = u.d8 + u.d4 + u.d2;
   const int n_tiles = (u.n_tok[0] + RDKV_TILE - 1) / RDKV_TILE + (u.n_tok[1] + RDKV_TILE - 1) / RDKV_TILE +
                       (u.n_tok[2] + RDKV_TILE - 1) / RDKV_TILE + (u.n_tok[3] + RDKV_TILE - 1) / RDKV_TILE;
   int ti = blockIdx.x;
   if (ti >= n_tiles) return;
-  const int p = tid & 15, r = tid >> 4;
+  const int p = lane & 15, r = lane >> 4;
   const int32_t *ord = a.order + (int64_t)h * a.order_stride_h;
   const __half *Kh = a.K + (int64_t)h * a.stride_h, *Vh = a.V + (int64_t)h * a.stride_h;
 
   // token indices of a tile (tokens past the tile's end repeat its first row; their codes are
   // dropped at assembly) and the rows behind them
-  auto load_tok = [&](int tile, int32_t (&tok)[4]) {
+  int32_t tok[4];
+  auto load_tok = [&](int tile) {
     const TileInfo t = tile_info(u, tile);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) tok[i] = ord[t.row0 + (r + 16 * i < t.nv ? r + 16 * i : 0)];
+    for (int i = 0; i < 4; ++i) {
+      const int at = kRows * g + r + 4 * i;
+      tok[i] = ord[t.row0 + (at < t.nv ? at : 0)];
+    }
   };
-  auto load_rows = [&](const int32_t (&tok)[4], uint4 (&kr)[4], uint4 (&vr)[4]) {
+  uint4 kraw[4], vraw[4];
+  auto load_rows = [&]() {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      kr[i] = *(reinterpret_cast<const uint4 *>(Kh + (int64_t)tok[i] * a.stride_t) + p);
-      vr[i] = *(reinterpret_cast<const uint4 *>(Vh + (int64_t)tok[i] * a.stride_t) + p);
+      kraw[i] = *(reinterpret_cast<const uint4 *>(Kh + (int64_t)tok[i] * a.stride_t) + p);
+      vraw[i] = *(reinterpret_cast<const uint4 *>(Vh + (int64_t)tok[i] * a.stride_t) + p);
     }
   };
 
-  int32_t tok[4];
-  load_tok(ti, tok);
+  load_tok(ti);
   if (tid < kD) chan[tid] = chan_params[(int64_t)h * kD + tid];
+  load_rows();
+  if (ti + stride < n_tiles) load_tok(ti + stride);
   // pad slots hold code 0: nothing writes them afterwards
   {
     uint4 *z = reinterpret_cast<uint4 *>(&ck[0][0]);
-    for (int i = tid; i < RDKV_TILE * kMaxSlots / 16; i += 256) z[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (int i = lane; i < kRows * kMaxSlots / 16; i += 64) z[i] = make_uint4(0u, 0u, 0u, 0u);
   }
   float v_scale_max = 0.0f;          // largest V scale among the tokens whose parameters this lane worked out
+  __syncthreads();                   // the channel table
 
   for (; ti < n_tiles; ti += stride) {
     const TileInfo t = tile_info(u, ti);
-    const int cls = t.cls, nv = t.nv;
-    // the tile's rows, then the token indices of the workgroup's next tile
-    uint4 kraw[4], vraw[4];
-    load_rows(tok, kraw, vraw);
-    if (ti + stride < n_tiles) load_tok(ti + stride, tok);
-    __syncthreads();   // the previous tile's assembly has read the code bytes (first tile: pad zeros and channel table are written)
+    const int cls = t.cls, nv = t.nv - kRows * g;        // valid tokens from this quarter's first on (may be none)
 
     // ---- V: per-token parameters and codes (quantized classes), or the rows as they are
     if (cls < 3) {
@@ -360,14 +377,14 @@ stream_pack_kernel(StreamPackArgs a, const float4 *__restrict__ chan_params) {
         mn[i] = row16_min(lo);
         mx[i] = row16_max(hi);
       }
-      // lane p works out the parameters of token r + 16 * (p % 4) (three divisions), the row shares them
+      // lane p works out the parameters of token r + 4 * (p % 4) (three divisions), the row shares them
       const int mine = p & 3;
       const RdkvQParams qm = rdkv_qparams(mine == 0 ? mn[0] : (mine == 1 ? mn[1] : (mine == 2 ? mn[2] : mn[3])),
                                           mine == 0 ? mx[0] : (mine == 1 ? mx[1] : (mine == 2 ? mx[2] : mx[3])), qmax);
       if (p < 4) {
-        const int tt = r + 16 * p;
+        const int tt = r + 4 * p;
         const uint16_t sc = rdkv_f2h(qm.scale);
-        *reinterpret_cast<uint32_t *>(a.blob + u.sz_off + 4 * ((int64_t)ti * RDKV_TILE + tt)) =
+        *reinterpret_cast<uint32_t *>(a.blob + u.sz_off + 4 * ((int64_t)ti * RDKV_TILE + kRows * g + tt)) =
             tt < nv ? (uint32_t)sc | ((uint32_t)rdkv_f2h(qm.zp) << 16) : 0u;
         if (tt < nv) v_scale_max = fmaxf(v_scale_max, rdkv_h2f(sc));
       }
@@ -400,11 +417,11 @@ stream_pack_kernel(StreamPackArgs a, const float4 *__restrict__ chan_params) {
             }
           }
         }
-        *reinterpret_cast<uint2 *>(&cv[r + 16 * i][8 * p]) = make_uint2(w0, w1);
+        *reinterpret_cast<uint2 *>(&cv[r + 4 * i][8 * p]) = make_uint2(w0, w1);
       }
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4 *>(&raw[r + 16 * i][8 * p]) = vraw[i];
+      for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4 *>(&raw[r + 4 * i][8 * p]) = vraw[i];
     }
 
     // ---- K codes to their stream slots
@@ -429,49 +446,46 @@ stream_pack_kernel(StreamPackArgs a, const float4 *__restrict__ chan_params) {
           }
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ck[r + 16 * i][slot] = (uint8_t)c4[i];
+        for (int i = 0; i < 4; ++i) ck[r + 4 * i][slot] = (uint8_t)c4[i];
       }
     }
-    __syncthreads();
+    // the rows of the next tile come in under the assembly
+    if (ti + stride < n_tiles) {
+      load_rows();
+      if (ti + 2 * stride < n_tiles) load_tok(ti + 2 * stride);
+    }
+    __builtin_amdgcn_wave_barrier();
 
-    // ---- K tile: 64 rows of R dwords, chunks of up to four dwords per token
+    // ---- K tile: rows of R dwords, chunks of up to four dwords per token, the quarter's sixteen tokens of each
     uint32_t *k_out = reinterpret_cast<uint32_t *>(a.blob + u.k_off) + (int64_t)ti * RDKV_TILE * R;
-    const int full = 256 * (R / 4);                   // dwords of the four-dword chunks
-    for (int rem0 = tid; rem0 < RDKV_TILE * R; rem0 += 256) {
-      int tt, j;
-      if (rem0 < full) {
-        tt = (rem0 & 255) >> 2;
-        j = 4 * (rem0 >> 8) + (rem0 & 3);
-      } else {
-        const int wc = R & 3, rem = rem0 - full;
-        tt = wc == 1 ? rem : (wc == 2 ? rem >> 1 : rem / 3);
-        j = 4 * (R / 4) + rem - tt * wc;
-      }
-      uint32_t w = 0;
-      if (tt < nv) {
-        if (j < u.d8) w = k_dword<4>(ck[tt], j);
-        else if (j < u.d8 + u.d4) w = k_dword<8>(ck[tt], u.d8 + 2 * (j - u.d8));
-        else w = k_dword<16>(ck[tt], u.d8 + 2 * u.d4 + 4 * (j - u.d8 - u.d4));
-      }
-      k_out[rem0] = w;
+    auto k_row_dword = [&](int tt, int j) -> uint32_t {
+      if (tt >= nv) return 0u;
+      if (j < u.d8) return k_dword<4>(ck[tt], j);
+      if (j < u.d8 + u.d4) return k_dword<8>(ck[tt], u.d8 + 2 * (j - u.d8));
+      return k_dword<16>(ck[tt], u.d8 + 2 * u.d4 + 4 * (j - u.d8 - u.d4));
+    };
+    for (int c = 0; c < R / 4; ++c) k_out[256 * c + 64 * g + lane] = k_row_dword(lane >> 2, 4 * c + (lane & 3));
+    const int wc = R & 3;
+    if (lane < kRows * wc) {
+      const int tt = wc == 1 ? lane : (wc == 2 ? lane >> 1 : lane / 3);
+      k_out[256 * (R / 4) + kRows * wc * g + lane] = k_row_dword(tt, 4 * (R / 4) + lane - tt * wc);
     }
 
     // ---- V tile of the class
     const uint64_t v_base = cls == 0 ? u.v_off[0] : (cls == 1 ? u.v_off[1] : (cls == 2 ? u.v_off[2] : u.v_off[3]));
     uint32_t *v_out = reinterpret_cast<uint32_t *>(a.blob + v_base) + (int64_t)t.tl * (rdkv_v_tile_bytes(cls) / 4);
-    if (cls == 0) v_tile<0>(cv, raw, nv, v_out);
-    else if (cls == 1) v_tile<1>(cv, raw, nv, v_out);
-    else if (cls == 2) v_tile<2>(cv, raw, nv, v_out);
-    else v_tile<3>(cv, raw, nv, v_out);
-
+    if (cls == 0) v_tile<0>(cv, raw, nv, g, v_out);
+    else if (cls == 1) v_tile<1>(cv, raw, nv, g, v_out);
+    else if (cls == 2) v_tile<2>(cv, raw, nv, g, v_out);
+    else v_tile<3>(cv, raw, nv, g, v_out);
+    __builtin_amdgcn_wave_barrier();
   }
 
   // the head's largest V scale (as the fp16 value the decode kernel will read): one atomic per
   // workgroup at most, none once the stored maximum has reached it (thousands of same-address
   // atomics would otherwise queue up behind each other)
   for (int o = 1; o < 64; o <<= 1) v_scale_max = fmaxf(v_scale_max, __shfl_xor(v_scale_max, o, 64));
-  __syncthreads();                       // (the last tile's assembly has read cv_bytes)
-  float *wave_max = reinterpret_cast<float *>(cv_bytes);
+  __shared__ float wave_max[4];
   if ((tid & 63) == 0) wave_max[tid >> 6] = v_scale_max;
   __syncthreads();
   if (tid == 0) {
@@ -492,16 +506,38 @@ RDKV_API int rdkv_pack_layer_stream_ws_init(float *minmax_ws, int H_kv, void *st
   return RDKV_OK;
 }
 
-RDKV_API int rdkv_pack_layer_stream(const void *K_f16, const void *V_f16, int64_t stride_h, int64_t stride_t,
-                                    int H_kv, const int32_t *order, int64_t order_stride_h,
-                                    const int32_t *counts, const void *k_bits, int kb_elem_size,
-                                    int64_t kb_stride_h, int n2p, int n4p, int n8, int64_t max_tv, int max_n16,
-                                    const RdkvUnit *units, const int16_t *src_slot, int n_slots_max,
-                                    int max_tiles, uint8_t *blob, int64_t blob_bytes, float *minmax_ws,
-                                    int minmax_ws_ready, float *scale_max, void *stream) {
+// As many workgroups as the device holds at once, each with the same number of tiles of the longest head.
+static int launch_stream_pack(const StreamPackBatch &batch, int n_layers, int H_kv, hipStream_t s) {
+  hipLaunchKernelGGL(slot_params_kernel, dim3(H_kv, 1, n_layers), dim3(128), 0, s, batch);
+  int max_tiles = 0;
+  for (int l = 0; l < n_layers; ++l) max_tiles = std::max(max_tiles, batch.layer[l].max_tiles);
+  if (max_tiles == 0) return RDKV_OK;
+  static int resident_of_device[64];     // (0 = not asked yet; a race between first callers writes the same value)
+  int resident = 512, dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) {
+    if (resident_of_device[dev] == 0) {
+      int cus = 0, per_cu = 0;
+      const bool ok = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0 &&
+                      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, stream_pack_kernel, 256, 0) == hipSuccess &&
+                      per_cu > 0;
+      if (ok) resident_of_device[dev] = cus * per_cu;   // (otherwise asked again next time)
+    }
+    if (resident_of_device[dev] > 0) resident = resident_of_device[dev];
+  }
+  const int rows = H_kv * n_layers, target = std::max(1, (resident + rows - 1) / rows);
+  const int per = (max_tiles + target - 1) / target;
+  const int gx = (max_tiles + per - 1) / per;
+  hipLaunchKernelGGL(stream_pack_kernel, dim3(gx, H_kv, n_layers), dim3(256), 0, s, batch);
+  return RDKV_OK;
+}
+
+static int fill_stream_args(const char *fn, StreamPackArgs *a, const void *K_f16, const void *V_f16, int64_t stride_h,
+                            int64_t stride_t, int H_kv, const int32_t *order, int64_t order_stride_h, const int32_t *counts,
+                            const void *k_bits, int kb_elem_size, int64_t kb_stride_h, int n2p, int n4p, int n8,
+                            int64_t max_tv, int max_n16, const RdkvUnit *units, const int16_t *src_slot, int n_slots_max,
+                            int max_tiles, uint8_t *blob, int64_t blob_bytes, float *minmax_ws, float *scale_max) {
   // (minmax_ws holds the min / max accumulators, H_kv * 256 floats, then the channel parameters,
   // H_kv * 128 * 4 floats)
-  const char *fn = "rdkv_pack_layer_stream";
   RDKV_REQUIRE(H_kv >= 1 && H_kv <= 65535 && max_tiles >= 0 && max_tv >= 0 && max_n16 >= 0 && blob_bytes >= 0 &&
                    blob_bytes % 4 == 0,
                "%s: bad shape", fn);
@@ -517,47 +553,73 @@ RDKV_API int rdkv_pack_layer_stream(const void *K_f16, const void *V_f16, int64_
     rdkv_set_error("%s: K and V rows must be 16-byte aligned", fn);
     return RDKV_EUNSUPPORTED;
   }
+  a->K = (const __half *)K_f16; a->V = (const __half *)V_f16;
+  a->stride_h = stride_h; a->stride_t = stride_t;
+  a->order = order; a->order_stride_h = order_stride_h;
+  a->k_bits = k_bits; a->kb_elem_size = kb_elem_size; a->kb_stride_h = kb_stride_h;
+  a->n2p = n2p; a->n4p = n4p;
+  a->max_tv = max_tv; a->max_n16 = max_n16;
+  a->mm = reinterpret_cast<uint32_t *>(minmax_ws);
+  a->units = units; a->src_slot = src_slot; a->n_slots_max = n_slots_max; a->max_tiles = max_tiles;
+  a->blob = blob;
+  a->scale_max = reinterpret_cast<uint32_t *>(scale_max);
+  a->H_kv = H_kv;
+  a->blob_bytes = blob_bytes;
+  return RDKV_OK;
+}
+
+RDKV_API int rdkv_pack_layer_stream(const void *K_f16, const void *V_f16, int64_t stride_h, int64_t stride_t,
+                                    int H_kv, const int32_t *order, int64_t order_stride_h,
+                                    const int32_t *counts, const void *k_bits, int kb_elem_size,
+                                    int64_t kb_stride_h, int n2p, int n4p, int n8, int64_t max_tv, int max_n16,
+                                    const RdkvUnit *units, const int16_t *src_slot, int n_slots_max,
+                                    int max_tiles, uint8_t *blob, int64_t blob_bytes, float *minmax_ws,
+                                    int minmax_ws_ready, float *scale_max, void *stream) {
+  const char *fn = "rdkv_pack_layer_stream";
+  StreamPackBatch batch;
+  const int rc = fill_stream_args(fn, &batch.layer[0], K_f16, V_f16, stride_h, stride_t, H_kv, order, order_stride_h, counts,
+                                  k_bits, kb_elem_size, kb_stride_h, n2p, n4p, n8, max_tv, max_n16, units, src_slot,
+                                  n_slots_max, max_tiles, blob, blob_bytes, minmax_ws, scale_max);
+  if (rc != RDKV_OK) return rc;
   hipStream_t s = (hipStream_t)stream;
-  const int64_t max_tk = max_tv + max_n16;
   // per-channel min / max of every head's kept rows (the K canvas without its zero rows)
   if (minmax_ws_ready != 2) {
-    const int rc = rdkv_layer_k_minmax(fn, K_f16, stride_h, stride_t, H_kv, kD, order, order_stride_h, counts, max_tk,
-                                       minmax_ws, /*init=*/minmax_ws_ready == 0, s);
-    if (rc != RDKV_OK) return rc;
+    const int mrc = rdkv_layer_k_minmax(fn, K_f16, stride_h, stride_t, H_kv, kD, order, order_stride_h, counts, max_tv + max_n16,
+                                        minmax_ws, /*init=*/minmax_ws_ready == 0, s);
+    if (mrc != RDKV_OK) return mrc;
   }
-  StreamPackArgs a;
-  a.K = (const __half *)K_f16; a.V = (const __half *)V_f16;
-  a.stride_h = stride_h; a.stride_t = stride_t;
-  a.order = order; a.order_stride_h = order_stride_h;
-  a.k_bits = k_bits; a.kb_elem_size = kb_elem_size; a.kb_stride_h = kb_stride_h;
-  a.n2p = n2p; a.n4p = n4p;
-  a.max_tv = max_tv; a.max_n16 = max_n16;
-  a.mm = reinterpret_cast<uint32_t *>(minmax_ws);
-  a.units = units; a.src_slot = src_slot; a.n_slots_max = n_slots_max; a.max_tiles = max_tiles;
-  a.blob = blob;
-  a.scale_max = reinterpret_cast<uint32_t *>(scale_max);
-  a.H_kv = H_kv;
-  a.blob_bytes = blob_bytes;
-  float4 *params = reinterpret_cast<float4 *>(minmax_ws + (int64_t)H_kv * 2 * kD);
-  hipLaunchKernelGGL(slot_params_kernel, dim3(H_kv), dim3(128), 0, s, a, params);
-  if (max_tiles > 0) {
-    // as many workgroups as the device holds at once, each with the same number of tiles of the longest head
-    static int resident_of_device[64];     // (0 = not asked yet; a race between first callers writes the same value)
-    int resident = 512, dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64) {
-      if (resident_of_device[dev] == 0) {
-        int cus = 0, per_cu = 0;
-        const bool ok = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0 &&
-                        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, stream_pack_kernel, 256, 0) == hipSuccess &&
-                        per_cu > 0;
-        if (ok) resident_of_device[dev] = cus * per_cu;   // (otherwise asked again next time)
+  launch_stream_pack(batch, 1, H_kv, s);
+  RDKV_CHECK_LAUNCH(fn);
+  return RDKV_OK;
+}
+
+// Layers packed one by one leave the device between them what a launch's first and last tiles take, and the slot
+// parameters 4.5 us each: four layers of 8 x 32k tokens 222 us of launches, together 170.
+RDKV_API int rdkv_pack_layers_stream(const RdkvStreamLayer *layers, int n_layers, int H_kv, const int32_t *order,
+                                     int64_t order_stride_h, const int32_t *counts, const void *k_bits, int kb_elem_size,
+                                     int64_t kb_stride_h, const RdkvUnit *units, const int16_t *src_slot, int n_slots_max,
+                                     float *minmax_ws, float *scale_max, void *stream) {
+  const char *fn = "rdkv_pack_layers_stream";
+  RDKV_REQUIRE(n_layers >= 0 && (n_layers == 0 || layers), "%s: bad arguments", fn);
+  for (int pass = 0; pass < 2; ++pass) {          // (every layer's arguments are looked at before the first launch)
+    for (int first = 0; first < n_layers; first += kBatchLayers) {
+      const int n = std::min(kBatchLayers, n_layers - first);
+      StreamPackBatch batch;
+      for (int i = 0; i < n; ++i) {
+        const int64_t l = first + i, row = l * H_kv;
+        const RdkvStreamLayer &y = layers[l];
+        const int rc = fill_stream_args(fn, &batch.layer[i], y.K_f16, y.V_f16, y.stride_h, y.stride_t, H_kv,
+                                        order ? order + row * order_stride_h : nullptr, order_stride_h,
+                                        counts ? counts + 4 * row : nullptr,
+                                        k_bits ? (const uint8_t *)k_bits + row * kb_stride_h * kb_elem_size : nullptr, kb_elem_size,
+                                        kb_stride_h, y.n2p, y.n4p, y.n8, y.max_tv, y.max_n16, units ? units + row : nullptr,
+                                        src_slot ? src_slot + row * n_slots_max : nullptr, n_slots_max, y.max_tiles, y.blob,
+                                        y.blob_bytes, minmax_ws ? minmax_ws + row * 768 : nullptr,
+                                        scale_max ? scale_max + 2 * row : nullptr);
+        if (rc != RDKV_OK) return rc;
       }
-      if (resident_of_device[dev] > 0) resident = resident_of_device[dev];
+      if (pass == 1) launch_stream_pack(batch, n, H_kv, (hipStream_t)stream);
     }
-    const int target = (resident + H_kv - 1) / H_kv;
-    const int per = (max_tiles + target - 1) / target;
-    const int gx = (max_tiles + per - 1) / per;
-    hipLaunchKernelGGL(stream_pack_kernel, dim3(gx, H_kv), dim3(256), 0, s, a, params);
   }
   RDKV_CHECK_LAUNCH(fn);
   return RDKV_OK;

@@ -413,7 +413,7 @@ def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, s
     if len(Ks[0].shape) != 4 or any(len(t.shape) != 2 for t in vbs + kbs):
         return None
     words = _lib.host_words(dev, 12 * n * H_kv)
-    planned = _lib.native.stream_order(Ks, Vs, vbs, kbs, packing._EARLY_MINMAX_TOKENS, words.take(12 * n * H_kv), words.tag, stream)
+    planned = _lib.native.stream_order(Ks, Vs, vbs, kbs, words.take(12 * n * H_kv), words.tag, stream)
     if planned is None:
         words.pending = False           # nothing was launched
         return None
@@ -427,8 +427,7 @@ def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, s
                                  dims) is None:
         return None
     units_dev, slots_dev = _lib.upload(dev, units, slots)
-    blobs = _lib.native.stream_pack(Ks, Vs, order, plan, kb, mm if mm is not None else _pack_scratch(dev, stream, H_kv),
-                                    _SCRATCH_PREPARED if mm is None else 2, units, units_dev, slots_dev, sizes, dims, scales, stream)
+    blobs = _lib.native.stream_pack(Ks, Vs, order, plan, kb, mm, units, units_dev, slots_dev, sizes, dims, scales, stream)
     assert blobs is not None
     return units, blobs, sizes.tolist(), scales
 
