@@ -302,7 +302,7 @@ __device__ __forceinline__ TileInfo tile_info(const RdkvUnit &u, int ti) {
 // channel), from where the dwords of the K rows and of the V tile are assembled and stored coalesced.
 // Latency bound (half of a wavefront's cycles were waits, 46 % of the vector issue slots used): the rows of the next tile
 // are requested as soon as the codes are parked, into the registers that held this tile's, and come in under the
-// assembly; nothing makes a wavefront wait for another.  One layer of 8 x 32k tokens 46.5 -> 30.5 us.
+// assembly; nothing makes a wavefront wait for another.  One layer of 8 x 32k / 128k tokens 54.8 / 170 -> 51.2 / 155 us.
 __global__ void __launch_bounds__(256, 3)
 stream_pack_kernel(StreamPackBatch batch) {
   const StreamPackArgs a = batch.layer[blockIdx.z];
@@ -496,7 +496,43 @@ stream_pack_kernel(StreamPackBatch batch) {
   }
 }
 
+// The smallest e >= 0 with v * 2^(6 - e) < 2^15, at most 40 and, for what is beyond 2^40, 32; 0 for a NaN.
+__device__ __forceinline__ int v_shift_of(float v) {
+  if (!(v > 0.0f)) return 0;
+  const int ex = (int)((__float_as_uint(v) >> 23) & 255u) - 126;      // v = m * 2^ex, 0.5 <= m < 1 (subnormals: -126)
+  return min(max(min(ex, 41) - 9, 0), 40);
+}
+
+// What rdkv_stream_work_scales does on the host, for scales that launches before this one leave on the device, and the
+// scales themselves to the host: with a copy, a wait for it and the items' upload behind it, a build's last 70 us were
+// the host's alone.
+__global__ void __launch_bounds__(256)
+work_scales_kernel(RdkvWork *work, int n_work, const float *__restrict__ scales, int H_kv, int n_units, uint64_t *words, uint32_t tag) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  auto scale = [&](int u, int which) { return scales[(int64_t)(u / H_kv) * 2 * H_kv + which * H_kv + u % H_kv]; };
+  if (i < n_work) {
+    const int u = work[i].unit;
+    work[i].k_scale_max = scale(u, 0);
+    work[i].v_shift = v_shift_of(scale(u, 1));
+  }
+  if (i < 2 * n_units) rdkv_host_word(words, i, tag, __float_as_int(scale(i >> 1, i & 1)));
+}
+
 }  // namespace
+
+// scales: [n_units / H_kv][2][H_kv] on the device (rdkv_pack_layers_stream), the work items' units in that order; words
+// [2 * n_units]: unit u's two scales as float bits.
+RDKV_API int rdkv_stream_work_scales_device(RdkvWork *work, int n_work, const float *scales, int H_kv, int n_units,
+                                            uint64_t *host_words, uint32_t tag, void *stream) {
+  const char *fn = "rdkv_stream_work_scales_device";
+  RDKV_REQUIRE(n_work >= 0 && n_units >= 1 && n_units <= (1 << 28) && H_kv >= 1 && n_units % H_kv == 0 && scales && host_words &&
+                   (n_work == 0 || work), "%s: bad arguments", fn);
+  const int n = std::max(n_work, 2 * n_units);
+  hipLaunchKernelGGL(work_scales_kernel, dim3((unsigned)rdkv_cdiv(n, 256)), dim3(256), 0, (hipStream_t)stream, work, n_work, scales,
+                     H_kv, n_units, host_words, tag);
+  RDKV_CHECK_LAUNCH(fn);
+  return RDKV_OK;
+}
 
 RDKV_API int rdkv_pack_layer_stream_ws_init(float *minmax_ws, int H_kv, void *stream) {
   const char *fn = "rdkv_pack_layer_stream_ws_init";
@@ -594,7 +630,7 @@ RDKV_API int rdkv_pack_layer_stream(const void *K_f16, const void *V_f16, int64_
 }
 
 // Layers packed one by one leave the device between them what a launch's first and last tiles take, and the slot
-// parameters 4.5 us each: four layers of 8 x 32k tokens 222 us of launches, together 170.
+// parameters 4.5 us each: four layers of 8 x 32k tokens 223 us of launches, together 164.
 RDKV_API int rdkv_pack_layers_stream(const RdkvStreamLayer *layers, int n_layers, int H_kv, const int32_t *order,
                                      int64_t order_stride_h, const int32_t *counts, const void *k_bits, int kb_elem_size,
                                      int64_t kb_stride_h, const RdkvUnit *units, const int16_t *src_slot, int n_slots_max,

@@ -401,6 +401,17 @@ def _pack_scratch(dev, stream: int, H_kv: int) -> torch.Tensor:
     return t
 
 
+class _DeviceScales:
+    """The largest scales [entries, 2, heads] that launches still running leave on the device; called: as rows of units,
+    fp32 [entries * heads, 2], on the host (synchronizes)."""
+
+    def __init__(self, scales: torch.Tensor):
+        self.scales = scales
+
+    def __call__(self) -> np.ndarray:
+        return _lib.download(self.scales).transpose(0, 2, 1).reshape(-1, 2).astype(np.float32)
+
+
 def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, stream: int):
     """``_pack_entries_direct`` for entries of one shape that the direct kernel takes and that all keep something, with its
     loops over entries in csrc/native.cpp: (units, blobs, sizes per entry, largest scales [n, 2, H] on the device); None
@@ -454,12 +465,8 @@ def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_
         units_all, blobs, sizes, sm_all = whole
         if entry_bytes is not None:
             entry_bytes.extend((int(sb), int(ab)) for _, _, sb, ab in sizes)
-        heads = int(sm_all.shape[2])
-
-        def largest():
-            return _lib.download(sm_all).transpose(0, 2, 1).reshape(n * heads, 2).astype(np.float32)    # (synchronizes)
-
-        return units_all, blobs, sum(int(s[2]) for s in sizes), sum(int(s[3]) for s in sizes), heads * G, largest
+        return (units_all, blobs, sum(int(s[2]) for s in sizes), sum(int(s[3]) for s in sizes), int(sm_all.shape[2]) * G,
+                _DeviceScales(sm_all))
     for i, (K, V, vb, kb) in enumerate(entries):
         H_q = int(K.shape[1]) * G
         if _direct_packable(K, V):
@@ -757,14 +764,25 @@ def _finish_caches(specs) -> List[StreamCache]:
                 work_np["merge_count"] = wc[merger[iu]]
         rows = (int(units_np["q_row"].max()) // H_q + 1) * H_q if len(units_np) else 0
         plans.append((units_np, work_np, groups_np, order, rows, int(R_np.max()) if len(R_np) else 0))
-    tables = _lib.upload(dev, *[a for pl in plans for a in (pl[0], pl[2] if pl[2] is not None else np.zeros(1, dtype=np.int32))])
     n_tickets = [max(1, len(pl[0])) for pl in plans]
-    tickets = torch.zeros(sum(n_tickets), dtype=torch.int32, device=dev)
     ticket_at = np.concatenate([[0], np.cumsum(n_tickets)])
+    on_device = specs[0][6] if len(specs) == 1 and isinstance(specs[0][6], _DeviceScales) and plans[0][3] is None else None
+    tables = _lib.upload(dev, *[a for pl in plans for a in (pl[0], pl[2] if pl[2] is not None else np.zeros(1, dtype=np.int32))],
+                         np.zeros(sum(n_tickets), dtype=np.int32), *([plans[0][1]] if on_device is not None else []))
+    tickets = tables[2 * len(plans)].view(torch.int32)
+    if on_device is not None:
+        # the scales to the work items and to the host as the packer's launches end, instead of through the host
+        units_np, work_np = plans[0][0], plans[0][1]
+        words = _lib.host_words(dev, 2 * len(units_np))
+        _lib.check(_lib.load().rdkv_stream_work_scales_device(
+            tables[-1].data_ptr(), len(work_np), on_device.scales.data_ptr(), int(on_device.scales.shape[2]), len(units_np),
+            words.take(2 * len(units_np)), words.tag, _lib.stream_of(dev)))
     scales = []
     for (units_np, work_np, groups_np, order, rows, r_max), spec in zip(plans, specs):
         scale_max = spec[6]
-        if callable(scale_max):
+        if on_device is not None:
+            scale_max = np.asarray(words.read(dev), dtype=np.int32).view(np.float32).reshape(-1, 2)
+        elif callable(scale_max):
             scale_max = scale_max()
         if order is not None:
             scale_max = scale_max[order]
@@ -773,7 +791,8 @@ def _finish_caches(specs) -> List[StreamCache]:
             _lib.check(_lib.load().rdkv_stream_work_scales(work_np.ctypes.data, len(work_np), scale_max.ctypes.data,
                                                            len(units_np)))
         scales.append(scale_max)
-    work_tables = _lib.upload(dev, *[pl[1] if len(pl[1]) else np.zeros(1, dtype=WORK_DTYPE) for pl in plans])
+    work_tables = tables[-1:] if on_device is not None else \
+        _lib.upload(dev, *[pl[1] if len(pl[1]) else np.zeros(1, dtype=WORK_DTYPE) for pl in plans])
     out = []
     for k, ((units_np, work_np, groups_np, order, rows, r_max), spec) in enumerate(zip(plans, specs)):
         _, blobs, G, H_q, stream_bytes, kv_algo_bytes, _, opt = spec
