@@ -178,6 +178,25 @@ int rdkv_unpack_layer_v_words(const uint8_t *V2, int64_t v2_stride_h, const uint
                         const void *V16_f16, int64_t v16_stride_h, int n16, int H_kv, int D,
                         void *out_f16, const int32_t *totals, uint64_t *words, uint32_t tag, void *stream);
 
+/* A whole layer in one launch: rdkv_unpack_layer_k_words and rdkv_unpack_layer_v_words with the arguments of
+ * the same names (arrays: by class), and, where mask is not NULL, mask [mask_rows][mask_width] fp32 as fp16 rows of
+ * mask_width + mask_extra elements, zeros behind the mask's. */
+typedef struct RdkvDenseLayer {
+  const uint8_t *K[3], *V[3];
+  int64_t k_stride_h[3], k_stride_t[3], v_stride_h[3];
+  const void *k_scale_f16, *k_zp_f16, *v_scale_f16, *v_zp_f16, *V16_f16;
+  int64_t ks_stride_h, vs_stride_h, v16_stride_h, sort_stride_h, T, max_tv;
+  const int64_t *sort_idx;
+  const int32_t *k_counts, *v_counts, *totals;
+  void *K_out_f16, *V_out_f16, *mask_out_f16;
+  const float *mask;
+  int64_t mask_rows, mask_width, mask_extra;
+  uint64_t *k_words, *v_words;
+  int32_t n[3], np[3], m[3], sort_n, n16, H_kv, D;
+  uint32_t tag;
+} RdkvDenseLayer;
+int rdkv_unpack_layer(const RdkvDenseLayer *layer, void *stream);
+
 /* ---- triton_k_kernel.py : k_mixed_qk_dot_into (:1211-1411) ---------------- */
 /* out[hq, t] = (sum_c code[hkv,t,c] * q[hq, perm[c]] * s[hkv,c] - sum_c z*q*s) / sqrt(128),
  * t < T_eff, reading the reference's padded layout.  q: [H_q,128] of q_dtype.

@@ -60,6 +60,7 @@ SIGNATURES = {
     "rdkv_unpack_layer_k_checked": (I, [P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, P, I, I, I, I, I, I, I, L, I, P, P, P]),
     "rdkv_unpack_layer_k_words": (I, [P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, P, I, I, I, I, I, I, I, L, I, P, P,
                                       ctypes.c_uint32, P]),
+    "rdkv_unpack_layer": (I, [P, P]),
     "rdkv_unpack_layer_v": (I, [P, L, P, L, P, L, P, P, L, P, I, I, I, L, P, L, I, I, I, P, P]),
     "rdkv_unpack_layer_v_words": (I, [P, L, P, L, P, L, P, P, L, P, I, I, I, L, P, L, I, I, I, P, P, P, ctypes.c_uint32, P]),
     "rdkv_k_qk_dot": (I, [P, I, L, I, I, P, L, L, P, L, L, P, L, L, P, P, L, P, L, I, I, I, L, P, L, P]),

@@ -29,7 +29,7 @@ namespace {
   X(rdkv_pool_scores) X(rdkv_knapsack_batched_value) X(rdkv_pack_layer_plan_ints) X(rdkv_pack_layer_plan_start)  \
   X(rdkv_pack_layers_k_minmax) X(rdkv_pack_layer_v_rows) X(rdkv_pack_layer_tables) X(rdkv_pack_layer_k_rows)     \
   X(rdkv_decode_fused) X(rdkv_decode_fused_zone_c) X(rdkv_decode_fused_workspace_bytes)                           \
-  X(rdkv_unpack_layer_k_words) X(rdkv_unpack_layer_v_words) X(rdkv_stream_plan_layer)   \
+  X(rdkv_unpack_layer) X(rdkv_stream_plan_layer)                                                                 \
   X(rdkv_select_layer_start) X(rdkv_pack_layers_stream)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -600,6 +600,14 @@ PyObject *dense_layer(PyObject *const *a, Py_ssize_t) {
   auto *k_words = static_cast<uint64_t *>(address(a[3])), *v_words = static_cast<uint64_t *>(address(a[4]));
   const uint32_t tag = (uint32_t)integer(a[5]);
   void *stream = address(a[6]);
+  // the fp16 rows, or (the fp16 rows, the mask, zeros behind its rows)
+  PyObject *rows_b = a[1], *mask_o = Py_None;
+  int64_t extra = 0;
+  if (PyTuple_Check(rows_b)) {
+    plain(PyTuple_GET_SIZE(a[1]) == 3);
+    rows_b = PyTuple_GET_ITEM(a[1], 0), mask_o = PyTuple_GET_ITEM(a[1], 1);
+    extra = std::max<int64_t>(integer(PyTuple_GET_ITEM(a[1], 2)), 0);
+  }
   auto maybe = [&](const char *name) {
     PyObject *o = field(f, name);
     return o == Py_None ? at::Tensor() : tensor(o);
@@ -645,29 +653,47 @@ PyObject *dense_layer(PyObject *const *a, Py_ssize_t) {
   dense(totals, at::kInt, {H});
   at::Tensor zone_b;
   if (n16 > 0) {
-    zone_b = tensor(a[1]);
+    zone_b = tensor(rows_b);
     dense(zone_b, at::kHalf, {1, H, n16, D});
   }
-  at::Tensor Kd, Vd;
+  at::Tensor mask;
+  if (mask_o != Py_None) {
+    mask = tensor(mask_o);
+    plain(mask.device() == dev && mask.scalar_type() == at::kFloat && mask.dim() == 2 && mask.is_contiguous() && mask.numel() > 0 &&
+          !mask.requires_grad() && extra < (1 << 30) && mask.size(0) * (mask.size(1) + extra) < (int64_t(1) << 31));
+  }
+  at::Tensor Kd, Vd, Md;
   int rc;
   {
     Unlocked u;
     Kd = at::empty({1, H, T_k, D}, ks.options()), Vd = at::empty({1, H, T_k, D}, ks.options());
-    auto head = [&](const at::Tensor &t) { return t.defined() ? t.stride(1) : 0; };
-    auto token = [&](const at::Tensor &t) { return t.defined() ? t.stride(2) : 0; };
-    rc = lib.rdkv_unpack_layer_k_words(data<uint8_t>(K[0]), head(K[0]), token(K[0]), data<uint8_t>(K[1]), head(K[1]), token(K[1]),
-                                       data<uint8_t>(K[2]), head(K[2]), token(K[2]), data(ks), data(kz), ks.stride(1),
-                                       data<int64_t>(sort), sort.stride(0), sort.size(1), data<int32_t>(k_counts), m[0], m[1], m[2],
-                                       w[0], w[1], w[2], H, T_k, D, data(Kd), k_words, tag, stream);
-    if (rc == RDKV_OK)
-      rc = lib.rdkv_unpack_layer_v_words(data<uint8_t>(V[0]), head(V[0]), data<uint8_t>(V[1]), head(V[1]), data<uint8_t>(V[2]),
-                                         head(V[2]), data(vs), data(vz), vs.stride(1), data<int32_t>(v_counts), mv[0], mv[1], mv[2],
-                                         T_v, data(zone_b), n16 ? zone_b.stride(1) : 0, n16, H, D, data(Vd), data<int32_t>(totals),
-                                         v_words, tag, stream);
+    RdkvDenseLayer y{};
+    for (int i = 0; i < 3; ++i) {
+      y.K[i] = data<uint8_t>(K[i]), y.V[i] = data<uint8_t>(V[i]);
+      if (K[i].defined()) y.k_stride_h[i] = K[i].stride(1), y.k_stride_t[i] = K[i].stride(2);
+      if (V[i].defined()) y.v_stride_h[i] = V[i].stride(1);
+      y.n[i] = m[i], y.np[i] = w[i], y.m[i] = mv[i];
+    }
+    y.k_scale_f16 = data(ks), y.k_zp_f16 = data(kz), y.ks_stride_h = ks.stride(1);
+    y.sort_idx = data<int64_t>(sort), y.sort_stride_h = sort.stride(0), y.sort_n = sort.size(1), y.k_counts = data<int32_t>(k_counts);
+    y.v_scale_f16 = data(vs), y.v_zp_f16 = data(vz), y.vs_stride_h = vs.stride(1);
+    y.v_counts = data<int32_t>(v_counts), y.totals = data<int32_t>(totals);
+    y.V16_f16 = data(zone_b), y.v16_stride_h = n16 ? zone_b.stride(1) : 0, y.n16 = n16;
+    y.H_kv = H, y.D = D, y.T = T_k, y.max_tv = T_v;
+    y.K_out_f16 = data(Kd), y.V_out_f16 = data(Vd);
+    y.k_words = k_words, y.v_words = v_words, y.tag = tag;
+    if (mask.defined()) {
+      Md = at::empty({1, mask.size(0), 1, mask.size(1) + extra}, ks.options());
+      y.mask = data<float>(mask), y.mask_out_f16 = data(Md);
+      y.mask_rows = mask.size(0), y.mask_width = mask.size(1), y.mask_extra = extra;
+    }
+    rc = lib.rdkv_unpack_layer(&y, stream);
   }
   status(rc);
   Ref k(wrap(Kd)), v(wrap(Vd));
-  return Ref(PyTuple_Pack(2, k.o, v.o)).release();
+  if (!mask.defined()) return Ref(PyTuple_Pack(2, k.o, v.o)).release();
+  Ref additive(wrap(Md));
+  return Ref(PyTuple_Pack(3, k.o, v.o, additive.o)).release();
 }
 
 // {name: address of the function}, check
@@ -699,7 +725,7 @@ PyMethodDef kMethods[] = {
     ENTRY(stream_tables, 9, "Fills the units, slot tables, sizes and dimensions of the layers: True, or None."),
     ENTRY(stream_pack, 13, "The blobs of the layers, or None."),
     ENTRY(decode_attn, 16, "(out, lse) of a decode step, or None."),
-    ENTRY(dense_layer, 7, "Dense (K, V) of a packed layer, or None."),
+    ENTRY(dense_layer, 7, "Dense (K, V) of a packed layer, with its additive mask where one is given; or None."),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_native", "Host side of the per-layer entry points.", -1, kMethods,
                        nullptr, nullptr, nullptr, nullptr};

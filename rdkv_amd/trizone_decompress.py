@@ -159,15 +159,17 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
     for i, pl in enumerate(dual_cache.packed):
         to = _words_of(pl.K_ch_scale.device, words, heads) if pl.K_ch_scale is not None else None
         zone_b = dual_cache.new_v_only[i] if i < len(dual_cache.new_v_only) else None
-        pair = None
+        pair = mask = None
         if to is not None and _lib.native is not None and _is_perhead_layout(pl):
             used, n = to.used, int(pl.K_ch_scale.shape[1])
-            pair = _lib.native.dense_layer(pl.__dict__, zone_b, head_dim, to.take(4 * n), to.take(4 * n), to.tag,
+            if return_masks and mask_dtype == torch.float16 and device is None:
+                mask = pl.softmax_mask
+            pair = _lib.native.dense_layer(pl.__dict__, zone_b if mask is None else (zone_b, mask, max_new_tokens), head_dim, to.take(4 * n), to.take(4 * n), to.tag,
                                            _lib.stream_of(pl.K_ch_scale.device))
             if pair is None:
                 to.used = used
             else:
-                K_full, V_full = pair
+                K_full, V_full = pair[:2]
                 words[pl.K_ch_scale.device][1].extend(((_check_k_counts, pl, n), (_check_v_counts, pl, n)))
         if pair is None:
             K_full, k_check = _unpack_k_enqueue(pl, head_dim, to)
@@ -214,6 +216,9 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
                 m = pl.softmax_mask
                 if H_q is not None:
                     assert H_q == int(m.shape[0]), f"layer {i}: caller H_q={H_q} != softmax_mask H_q={m.shape[0]}"
+                if mask is not None and pair is not None:      # (left the layer's launch)
+                    masks.append(pair[2])
+                    continue
                 tgt = device if device is not None else m.device
                 m4 = m.to(device=tgt, dtype=mask_dtype).view(1, m.shape[0], 1, m.shape[1])
                 if max_new_tokens > 0:
