@@ -754,6 +754,22 @@ int rdkv_pack_layer_tables(const void *k_bits, int kb_elem_size, int64_t kb_stri
                            int32_t *seg_ch, int32_t *seg_tok, int32_t *t_eff, int32_t *t_eff_k,
                            int32_t *n_v16, int64_t *sort_idx, float *softmax_mask, void *stream);
 
+/* A whole layer (D = 128, rows 16-byte aligned) whose K min / max are in minmax (rdkv_pack_layers_k_minmax) in one
+ * launch: what rdkv_pack_layer_v_rows, rdkv_pack_layer_tables (without slot_channel) and rdkv_pack_layer_k_rows write from
+ * the arguments of the same names (mN: mN2, mN4, mN8). */
+typedef struct RdkvPackLayer {
+  const void *K_f16, *V_f16, *k_bits;
+  const int32_t *order, *rank3, *counts, *info;
+  const float *minmax;
+  int64_t stride_h, stride_t, order_stride_h, rank3_stride_h, kb_stride_h, max_tv, tv_ref;
+  uint8_t *V2, *V4, *V8, *K2, *K4, *K8;
+  void *V_scale_f16, *V_zp_f16, *V16_f16, *K_scale_f16, *K_zp_f16;
+  int64_t *perm, *perm_for_q, *sort_ch, *sort_idx;
+  int32_t *seg_ch, *seg_tok, *t_eff, *t_eff_k, *n_v16;
+  float *softmax_mask;
+  int32_t H_kv, G, kb_elem_size, mN[3], max_n16, n2p, n4p, n8, kept_max, ref_head;
+} RdkvPackLayer;
+int rdkv_pack_layer(const RdkvPackLayer *layer, void *stream);
 /* ---- prefill-time selection feeding the packer ---------------------------------------------
  * obkv_fast.py:208-249  apply_score_pooling, as used on the per-head token scores at
  * obkv_fast.py:961-967.  Stride-1 pooling of B rows of T fp32 scores (row stride in elements).

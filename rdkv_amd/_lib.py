@@ -114,6 +114,7 @@ SIGNATURES = {
     "rdkv_pack_layer_plan_start": (I, [P, I, L, P, I, L, I, L, I, P, L, P, L, P, P, I, P, ctypes.c_uint32, P]),
     "rdkv_host_words_wait": (I, [P, L, ctypes.c_uint32, P, L]),
     "rdkv_pack_layers_k_minmax": (I, [P, P, I, I, L, I, P, L, P, P, L, P]),
+    "rdkv_pack_layer": (I, [P, P]),
     "rdkv_pack_layer_tables": (I, [P, I, L, I, I, I, P, P, I, I, I, I, L, I, P, L, P, L, I, L,
                                    P, P, P, P, P, P, P, P, P, P, P, P]),
     "rdkv_pool_scores": (I, [P, L, I, L, I, I, I, P, L, P]),

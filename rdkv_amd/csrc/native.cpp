@@ -29,7 +29,7 @@ namespace {
   X(rdkv_pool_scores) X(rdkv_knapsack_batched_value) X(rdkv_pack_layer_plan_ints) X(rdkv_pack_layer_plan_start)  \
   X(rdkv_pack_layers_k_minmax) X(rdkv_pack_layer_v_rows) X(rdkv_pack_layer_tables) X(rdkv_pack_layer_k_rows)     \
   X(rdkv_decode_fused) X(rdkv_decode_fused_zone_c) X(rdkv_decode_fused_workspace_bytes)                           \
-  X(rdkv_unpack_layer) X(rdkv_stream_plan_layer)                                                                 \
+  X(rdkv_unpack_layer) X(rdkv_stream_plan_layer) X(rdkv_pack_layer)                                                           \
   X(rdkv_select_layer_start) X(rdkv_pack_layers_stream)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -201,34 +201,66 @@ PyObject *pack_layer(PyObject *const *a, Py_ssize_t) {
   int rc;
   {
     Unlocked u;
-    // V rows first: they need neither the channel tables nor the K outputs
     V2 = bytes(mN[0], D / 4), V4 = bytes(mN[1], D / 2), V8 = bytes(mN[2], D);
     vs = make({1, H, max_tv, 1}, at::kHalf), vz = make({1, H, max_tv, 1}, at::kHalf);
     if (max_n16 > 0) v16 = make({1, H, max_n16, D}, at::kHalf);
-    if (!early) mm = make({H * 2 * D}, at::kFloat);
-    float *mm_at = early ? data<float>(mm_all) + first * 2 * D : data<float>(mm);
-    rc = lib.rdkv_pack_layer_v_rows(V.data_ptr(), K.stride(1), K.stride(2), H, D, order_l, order.stride(0), counts4, mN[0],
-                                    mN[1], mN[2], max_tv, max_n16, data<uint8_t>(V2), data<uint8_t>(V4), data<uint8_t>(V8),
-                                    data(vs), data(vz), data(v16), early ? nullptr : mm_at, stream);
-    if (rc == RDKV_OK) {
-      slot_ch = make({H, Dp}, at::kInt), perm = make({H, Dp}, at::kLong), perm_q = make({H * G, Dp}, at::kLong);
+    auto tables = [&] {
+      perm = make({H, Dp}, at::kLong), perm_q = make({H * G, Dp}, at::kLong);
       sort_ph = make({H, kept_max}, at::kLong), seg_ph = make({H, 3}, at::kInt), seg_tok = make({H, 3}, at::kInt);
       t_eff = make({H}, at::kInt), t_eff_k = make({H}, at::kInt), n_v16 = make({H}, at::kInt);
       sort_idx = make({tv_ref}, at::kLong), mask = make({H * G, max_tk}, at::kFloat);
-      rc = lib.rdkv_pack_layer_tables(kb_l, kb.element_size(), kb.stride(0), H, D, G, counts4, info, 4 * sub2, 2 * sub4, m[2],
-                                      kept_max, max_tv, max_n16, order_l, order.stride(0), rank3_l, rank3.stride(0), ref,
-                                      tv_ref, data<int32_t>(slot_ch), data<int64_t>(perm), data<int64_t>(perm_q),
-                                      data<int64_t>(sort_ph), data<int32_t>(seg_ph), data<int32_t>(seg_tok),
-                                      data<int32_t>(t_eff), data<int32_t>(t_eff_k), data<int32_t>(n_v16),
-                                      data<int64_t>(sort_idx), data<float>(mask), stream);
-    }
-    if (rc == RDKV_OK) {
+    };
+    auto k_outputs = [&] {
       K2 = bytes(max_tk, sub2), K4 = bytes(max_tk, sub4), K8 = bytes(max_tk, m[2]);
       ks = make({1, H, 1, Dp}, at::kHalf), kz = make({1, H, 1, Dp}, at::kHalf);
-      rc = lib.rdkv_pack_layer_k_rows(K.data_ptr(), K.stride(1), K.stride(2), H, D, order_l, order.stride(0), counts4, max_tv,
-                                      max_n16, data<int32_t>(slot_ch), 4 * sub2, 2 * sub4, m[2], data<uint8_t>(K2),
-                                      data<uint8_t>(K4), data<uint8_t>(K8), data(ks), data(kz), mm_at,
-                                      early ? 2 : mN[0] + mN[1] + mN[2] + max_n16 > 0 ? 1 : 0, stream);
+    };
+    const float *mm_at = early ? data<float>(mm_all) + first * 2 * D : nullptr;
+    const uintptr_t at16 = reinterpret_cast<uintptr_t>(K.data_ptr()) | reinterpret_cast<uintptr_t>(V.data_ptr());
+    if (early && D == 128 && Dp <= 512 && at16 % 16 == 0 && K.stride(1) % 8 == 0 && K.stride(2) % 8 == 0 &&
+        max_tk < 0x7fff0000 && mN[0] + mN[1] + mN[2] + max_n16 < 0x7fff0000) {
+      // one launch (the lines that rdkv_pack_layer requires)
+      tables();
+      k_outputs();
+      RdkvPackLayer y{};
+      y.K_f16 = K.data_ptr(), y.V_f16 = V.data_ptr(), y.stride_h = K.stride(1), y.stride_t = K.stride(2);
+      y.k_bits = kb_l, y.kb_elem_size = kb.element_size(), y.kb_stride_h = kb.stride(0);
+      y.order = order_l, y.order_stride_h = order.stride(0), y.rank3 = rank3_l, y.rank3_stride_h = rank3.stride(0);
+      y.counts = counts4, y.info = info, y.minmax = mm_at, y.max_tv = max_tv, y.tv_ref = tv_ref;
+      y.V2 = data<uint8_t>(V2), y.V4 = data<uint8_t>(V4), y.V8 = data<uint8_t>(V8);
+      y.K2 = data<uint8_t>(K2), y.K4 = data<uint8_t>(K4), y.K8 = data<uint8_t>(K8);
+      y.V_scale_f16 = data(vs), y.V_zp_f16 = data(vz), y.V16_f16 = data(v16), y.K_scale_f16 = data(ks), y.K_zp_f16 = data(kz);
+      y.perm = data<int64_t>(perm), y.perm_for_q = data<int64_t>(perm_q), y.sort_ch = data<int64_t>(sort_ph);
+      y.sort_idx = data<int64_t>(sort_idx), y.softmax_mask = data<float>(mask);
+      y.seg_ch = data<int32_t>(seg_ph), y.seg_tok = data<int32_t>(seg_tok), y.t_eff = data<int32_t>(t_eff);
+      y.t_eff_k = data<int32_t>(t_eff_k), y.n_v16 = data<int32_t>(n_v16);
+      y.H_kv = H, y.G = G, y.max_n16 = max_n16, y.n2p = 4 * sub2, y.n4p = 2 * sub4, y.n8 = m[2];
+      for (int i = 0; i < 3; ++i) y.mN[i] = mN[i];
+      y.kept_max = kept_max, y.ref_head = ref;
+      rc = lib.rdkv_pack_layer(&y, stream);
+    } else {
+      // V rows first: they need neither the channel tables nor the K outputs
+      if (!early) mm = make({H * 2 * D}, at::kFloat);
+      float *mm_ws = early ? const_cast<float *>(mm_at) : data<float>(mm);
+      rc = lib.rdkv_pack_layer_v_rows(V.data_ptr(), K.stride(1), K.stride(2), H, D, order_l, order.stride(0), counts4, mN[0],
+                                      mN[1], mN[2], max_tv, max_n16, data<uint8_t>(V2), data<uint8_t>(V4), data<uint8_t>(V8),
+                                      data(vs), data(vz), data(v16), early ? nullptr : mm_ws, stream);
+      if (rc == RDKV_OK) {
+        tables();
+        slot_ch = make({H, Dp}, at::kInt);
+        rc = lib.rdkv_pack_layer_tables(kb_l, kb.element_size(), kb.stride(0), H, D, G, counts4, info, 4 * sub2, 2 * sub4,
+                                        m[2], kept_max, max_tv, max_n16, order_l, order.stride(0), rank3_l, rank3.stride(0),
+                                        ref, tv_ref, data<int32_t>(slot_ch), data<int64_t>(perm), data<int64_t>(perm_q),
+                                        data<int64_t>(sort_ph), data<int32_t>(seg_ph), data<int32_t>(seg_tok),
+                                        data<int32_t>(t_eff), data<int32_t>(t_eff_k), data<int32_t>(n_v16),
+                                        data<int64_t>(sort_idx), data<float>(mask), stream);
+      }
+      if (rc == RDKV_OK) {
+        k_outputs();
+        rc = lib.rdkv_pack_layer_k_rows(K.data_ptr(), K.stride(1), K.stride(2), H, D, order_l, order.stride(0), counts4,
+                                        max_tv, max_n16, data<int32_t>(slot_ch), 4 * sub2, 2 * sub4, m[2], data<uint8_t>(K2),
+                                        data<uint8_t>(K4), data<uint8_t>(K8), data(ks), data(kz), mm_ws,
+                                        early ? 2 : mN[0] + mN[1] + mN[2] + max_n16 > 0 ? 1 : 0, stream);
+      }
     }
     if (rc == RDKV_OK) sort0 = sort_ph.select(0, 0), perm0 = perm.select(0, 0);
   }

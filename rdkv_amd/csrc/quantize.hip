@@ -2,7 +2,9 @@
 // 296-351, 751-773, 1427-1444).  All arithmetic is IEEE fp32 in the reference's operation
 // order (correctly rounded division, no FMA contraction, round-half-even) so codes,
 // scales and zero-points are bit-identical to the reference's CPU results.
-#include "rdkv_common.h"
+#include <algorithm>
+
+#include "pack_tables.h"
 
 // No fused multiply-adds in this file, whatever the command line says: the reference rounds every
 // product and every sum on its own, and HIP's __fmul_rn / __fadd_rn do not stop the compiler from
@@ -395,8 +397,7 @@ pack_v_rows_d128(const __half *__restrict__ Vh, int64_t stride_t, const int32_t 
   }
 }
 
-__global__ void __launch_bounds__(256)
-pack_v_layer_d128_kernel(const __half *__restrict__ V, int64_t stride_h, int64_t stride_t,
+__device__ __forceinline__ void pack_v_layer_d128(int bx, int nbx, const __half *__restrict__ V, int64_t stride_h, int64_t stride_t,
                          const int32_t *__restrict__ order, int64_t order_stride_h,
                          const int32_t *__restrict__ counts, int mN2, int mN4, int mN8, int max_n16,
                          int64_t max_tv, uint8_t *__restrict__ V2, uint8_t *__restrict__ V4,
@@ -410,17 +411,17 @@ pack_v_layer_d128_kernel(const __half *__restrict__ V, int64_t stride_h, int64_t
   const __half *Vh = V + (int64_t)h * stride_h;
   __half *vsh = vs + (int64_t)h * max_tv, *vzh = vz + (int64_t)h * max_tv;
   // Two small jobs ride along instead of being launches of their own (see pack_v_layer_kernel).
-  for (int64_t i = (int64_t)n2 + n4 + n8 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < max_tv;
-       i += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t i = (int64_t)n2 + n4 + n8 + (int64_t)bx * blockDim.x + threadIdx.x; i < max_tv;
+       i += (int64_t)nbx * blockDim.x) {
     vsh[i] = __float2half_rn(0.0f);
     vzh[i] = __float2half_rn(0.0f);
   }
-  if (mm_init && blockIdx.x == 0)
+  if (mm_init && bx == 0)
     for (int i = threadIdx.x; i < 2 * D; i += blockDim.x)
       mm_init[(int64_t)h * 2 * D + i] = rdkv_float_to_ordered(i >= D ? -INFINITY : INFINITY);
   // block -> (class, first row): the classes' blocks follow each other
   const int b2 = (mN2 + kRows - 1) / kRows, b4 = (mN4 + kRows - 1) / kRows, b8 = (mN8 + kRows - 1) / kRows;
-  int b = blockIdx.x;
+  int b = bx;
   if (b < b2) {
     pack_v_rows_d128<0>(Vh, stride_t, ord, b * kRows, n2, mN2, 0, V2 + (int64_t)h * mN2 * 32, vsh, vzh);
   } else if ((b -= b2) < b4) {
@@ -432,6 +433,16 @@ pack_v_layer_d128_kernel(const __half *__restrict__ V, int64_t stride_h, int64_t
     pack_v_rows_d128<3>(Vh, stride_t, ord, b * kRows, n16, max_n16, n2 + n4 + n8,
                         reinterpret_cast<uint8_t *>(V16 + (int64_t)h * max_n16 * D), vsh, vzh);
   }
+}
+
+__global__ void __launch_bounds__(256)
+pack_v_layer_d128_kernel(const __half *__restrict__ V, int64_t stride_h, int64_t stride_t,
+                         const int32_t *__restrict__ order, int64_t order_stride_h,
+                         const int32_t *__restrict__ counts, int mN2, int mN4, int mN8, int max_n16,
+                         int64_t max_tv, uint8_t *__restrict__ V2, uint8_t *__restrict__ V4,
+                         uint8_t *__restrict__ V8, __half *__restrict__ vs, __half *__restrict__ vz,
+                         __half *__restrict__ V16, uint32_t *__restrict__ mm_init) {
+  pack_v_layer_d128(blockIdx.x, gridDim.x, V, stride_h, stride_t, order, order_stride_h, counts, mN2, mN4, mN8, max_n16, max_tv, V2, V4, V8, vs, vz, V16, mm_init);
 }
 
 // ---------------------------------------------------------------------------
@@ -850,9 +861,16 @@ k_emit_layer_kernel(const __half *__restrict__ K, int64_t stride_h, int64_t stri
 #define RDKV_EMIT_ROWS_D128 (8 * RDKV_EMIT_STEP_ROWS_D128)
 // ANY_ROW: some row of the workgroup exists (otherwise all are zero rows and nothing is loaded;
 // the two cases are separate instantiations so that the waits of one do not constrain the other).
-template <bool ANY_ROW>
+// WIDTHS: the channels' slots from the head's bit widths (kb) instead of a table that an earlier launch wrote: a
+// wavefront ranks all 128 channels by ballots, and the extremes are a channel's own, requested in the first round trip.
+struct KWidths {
+  const void *p;
+  int es;
+  int64_t stride_h;
+};
+template <bool ANY_ROW, bool WIDTHS>
 __device__ __forceinline__ void
-k_emit_layer_d128_body(float *smem, const __half *__restrict__ K, int64_t stride_h, int64_t stride_t,
+k_emit_layer_d128_body(int bx, KWidths kb, float *smem, const __half *__restrict__ K, int64_t stride_h, int64_t stride_t,
                        const int32_t *__restrict__ order, int64_t order_stride_h,
                        const int32_t *__restrict__ counts, int64_t max_tv, int max_n16,
                        const uint32_t *__restrict__ mm, const int32_t *__restrict__ slot_channel,
@@ -871,7 +889,7 @@ k_emit_layer_d128_body(float *smem, const __half *__restrict__ K, int64_t stride
   const int64_t max_tk = max_tv + max_n16;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int sub = lane >> 4, l = lane & 15;
-  const int t0 = blockIdx.x * RDKV_EMIT_ROWS_D128;
+  const int t0 = bx * RDKV_EMIT_ROWS_D128;
   const int t1 = (int)((int64_t)t0 + RDKV_EMIT_ROWS_D128 < max_tk ? (int64_t)t0 + RDKV_EMIT_ROWS_D128 : max_tk);
   const int mtv = (int)max_tv;
   const int rl = wave * 4 + sub;               // this lane's row of step 0, within the workgroup
@@ -881,11 +899,20 @@ k_emit_layer_d128_body(float *smem, const __half *__restrict__ K, int64_t stride
   const int32_t *ord = order + (int64_t)h * order_stride_h;
   const __half *Kh = K + (int64_t)h * stride_h;
   // this thread's slot(s) of the channel plan
-  int ch[kSlotPasses];
+  const uint32_t *mmh = mm + (int64_t)h * 2 * D;
+  int ch[kSlotPasses], width[2];
+  uint32_t mn_bits[kSlotPasses], mx_bits[kSlotPasses];
+  if (WIDTHS) {
 #pragma unroll
-  for (int k = 0; k < kSlotPasses; ++k) {
-    const int slot = (int)threadIdx.x + kThreads * k;
-    ch[k] = slot_channel[(int64_t)h * Dp + (slot < Dp ? slot : 0)];
+    for (int k = 0; k < 2; ++k) width[k] = load_int(kb.p, kb.es, (int64_t)h * kb.stride_h + lane + 64 * k);
+    mn_bits[0] = mmh[threadIdx.x & (D - 1)];
+    mx_bits[0] = mmh[D + (threadIdx.x & (D - 1))];
+  } else {
+#pragma unroll
+    for (int k = 0; k < kSlotPasses; ++k) {
+      const int slot = (int)threadIdx.x + kThreads * k;
+      ch[k] = slot_channel[(int64_t)h * Dp + (slot < Dp ? slot : 0)];
+    }
   }
   // (zero rows are masked with AND, not selected: a select invites the compiler to branch around
   // the load, which puts a full wait between that load and its neighbours)
@@ -907,10 +934,8 @@ k_emit_layer_d128_body(float *smem, const __half *__restrict__ K, int64_t stride
   }
   __builtin_amdgcn_sched_barrier(0);
   // ---- second round trip: the channel's extremes, then the rows ---------------------------------
-  const uint32_t *mmh = mm + (int64_t)h * 2 * D;
-  uint32_t mn_bits[kSlotPasses], mx_bits[kSlotPasses];
 #pragma unroll
-  for (int k = 0; k < kSlotPasses; ++k) {
+  for (int k = 0; k < (WIDTHS ? 0 : kSlotPasses); ++k) {
     const bool has_ch = (int)threadIdx.x + kThreads * k < Dp && ch[k] >= 0;
     mn_bits[k] = mmh[has_ch ? ch[k] : 0];
     mx_bits[k] = mmh[D + (has_ch ? ch[k] : 0)];
@@ -934,12 +959,62 @@ k_emit_layer_d128_body(float *smem, const __half *__restrict__ K, int64_t stride
   float *c_scale = smem, *c_zp = smem + D, *c_qmax = smem + 2 * D;
   int *c_slot = reinterpret_cast<int *>(smem + 3 * D);
   uint8_t *rowbufs = reinterpret_cast<uint8_t *>(smem + 4 * D);
-  for (int c = threadIdx.x; c < D; c += blockDim.x) c_slot[c] = -1;
+  if (!WIDTHS)
+    for (int c = threadIdx.x; c < D; c += blockDim.x) c_slot[c] = -1;
   for (int i = threadIdx.x; i < kStepRows * Dp4 / 4; i += blockDim.x)
     reinterpret_cast<uint32_t *>(rowbufs)[i] = 0u;               // slots without a channel stay 0
-  __syncthreads();
+  if (WIDTHS) {
+    int cls[2], in[3];                     // of this lane's two channels; the head's channels of each class
+    uint64_t lo[3], hi[3];
 #pragma unroll
-  for (int k = 0; k < kSlotPasses; ++k) {
+    for (int k = 0; k < 2; ++k) cls[k] = channel_class(width[k]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      lo[k] = __ballot(cls[0] == k);
+      hi[k] = __ballot(cls[1] == k);
+      in[k] = __popcll(lo[k]) + __popcll(hi[k]);
+    }
+    auto store_params = [&](int s, const RdkvQParams &p) {
+      scale_out[(int64_t)h * Dp + s] = __float2half_rn(p.scale);
+      zp_out[(int64_t)h * Dp + s] = __float2half_rn(p.zp);
+    };
+    if (threadIdx.x < D) {
+      const int c = threadIdx.x, k = wave == 0 ? cls[0] : cls[1];
+      int rank = 0;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) rank = k == i ? (wave == 0 ? lanes_below(lo[i]) : __popcll(lo[i]) + lanes_below(hi[i])) : rank;
+      int at = -1;
+      // (a width that was overwritten since the class sizes were counted must not lead outside the slots)
+      if (k >= 0 && rank < (k == 0 ? n2p : k == 1 ? n4p : n8)) {
+        float mn = rdkv_ordered_to_float(mn_bits[0]), mx = rdkv_ordered_to_float(mx_bits[0]);
+        if (has_pad) {
+          mn = fminf(mn, 0.0f);
+          mx = fmaxf(mx, 0.0f);
+        }
+        const float qmax = k == 0 ? 3.0f : k == 1 ? 15.0f : 255.0f;
+        const RdkvQParams p = rdkv_qparams(mn, mx, qmax);
+        c_scale[c] = p.scale;
+        c_zp[c] = p.zp;
+        c_qmax[c] = qmax;
+        // (the 2-bit slots are four runs of sub2, the 4-bit ones two of sub4)
+        const int part = k == 0 ? (rank >= sub2) + (rank >= 2 * sub2) + (rank >= 3 * sub2) : k == 1 ? rank >= sub4 : 0;
+        at = k == 0 ? part * sub2p + rank - part * sub2 : k == 1 ? o4 + part * sub4p + rank - part * sub4 : o8 + rank;
+        if (bx == 0) store_params((k == 0 ? 0 : k == 1 ? n2p : n2p + n4p) + rank, p);
+      }
+      c_slot[c] = at;
+    } else if (bx == 0) {
+      // slots without a channel: the zero column of the padded layout
+      for (int s = (int)threadIdx.x - D; s < Dp; s += kThreads - D) {
+        const int k = s < n2p ? 0 : s < n2p + n4p ? 1 : 2;
+        if (s - (k == 0 ? 0 : k == 1 ? n2p : n2p + n4p) >= (k == 0 ? in[0] : k == 1 ? in[1] : in[2]))
+          store_params(s, rdkv_qparams(0.0f, 0.0f, k == 0 ? 3.0f : k == 1 ? 15.0f : 255.0f));
+      }
+    }
+  } else {
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < (WIDTHS ? 0 : kSlotPasses); ++k) {
     const int s = (int)threadIdx.x + kThreads * k;
     if (s >= Dp) continue;
     const float qmax = s < n2p ? 3.0f : (s < n2p + n4p ? 15.0f : 255.0f);
@@ -963,7 +1038,7 @@ k_emit_layer_d128_body(float *smem, const __half *__restrict__ K, int64_t stride
       else at = o8 + (s - n2p - n4p);
       c_slot[ch[k]] = at;
     }
-    if (blockIdx.x == 0) {
+    if (bx == 0) {
       scale_out[(int64_t)h * Dp + s] = __float2half_rn(p.scale);
       zp_out[(int64_t)h * Dp + s] = __float2half_rn(p.zp);
     }
@@ -1043,6 +1118,27 @@ k_emit_layer_d128_body(float *smem, const __half *__restrict__ K, int64_t stride
   }
 }
 
+template <bool WIDTHS>
+__device__ __forceinline__ void k_emit_layer_d128(int bx, KWidths kb, float *smem, const __half *__restrict__ K, int64_t stride_h,
+                                                  int64_t stride_t, const int32_t *__restrict__ order,
+                                                  int64_t order_stride_h, const int32_t *__restrict__ counts,
+                                                  int64_t max_tv, int max_n16, const uint32_t *__restrict__ mm,
+                                                  const int32_t *__restrict__ slot_channel, int n2p, int n4p, int n8,
+                                                  uint8_t *__restrict__ K2, uint8_t *__restrict__ K4,
+                                                  uint8_t *__restrict__ K8, __half *__restrict__ scale_out,
+                                                  __half *__restrict__ zp_out) {
+  const int h = blockIdx.y;
+  const int tv = counts[4 * h] + counts[4 * h + 1] + counts[4 * h + 2], n16 = counts[4 * h + 3];
+  const int64_t t0 = (int64_t)bx * RDKV_EMIT_ROWS_D128;
+  const int64_t t1 = t0 + RDKV_EMIT_ROWS_D128 < max_tv + max_n16 ? t0 + RDKV_EMIT_ROWS_D128 : max_tv + max_n16;
+  if (t0 < tv || (t1 > max_tv && t0 < max_tv + n16))               // uniform over the workgroup
+    k_emit_layer_d128_body<true, WIDTHS>(bx, kb, smem, K, stride_h, stride_t, order, order_stride_h, counts, max_tv, max_n16,
+                                         mm, slot_channel, n2p, n4p, n8, K2, K4, K8, scale_out, zp_out);
+  else
+    k_emit_layer_d128_body<false, WIDTHS>(bx, kb, smem, K, stride_h, stride_t, order, order_stride_h, counts, max_tv, max_n16,
+                                          mm, slot_channel, n2p, n4p, n8, K2, K4, K8, scale_out, zp_out);
+}
+
 __global__ void __launch_bounds__(64 * RDKV_EMIT_WAVES_D128)
 k_emit_layer_d128_kernel(const __half *__restrict__ K, int64_t stride_h, int64_t stride_t,
                          const int32_t *__restrict__ order, int64_t order_stride_h,
@@ -1052,16 +1148,45 @@ k_emit_layer_d128_kernel(const __half *__restrict__ K, int64_t stride_h, int64_t
                          uint8_t *__restrict__ K8, __half *__restrict__ scale_out,
                          __half *__restrict__ zp_out) {
   extern __shared__ float smem[];
+  k_emit_layer_d128<false>(blockIdx.x, KWidths{}, smem, K, stride_h, stride_t, order, order_stride_h, counts, max_tv, max_n16,
+                           mm, slot_channel, n2p, n4p, n8, K2, K4, K8, scale_out, zp_out);
+}
+
+// A whole layer whose K min / max are known: K rows, V rows, the channel tables and the mask side by side.  x of the
+// grid: K's workgroups of a head (the longest), then V's, then the tables', then the mask's.
+// Bound: 8 heads of 13 700 kept rows of 31k (28 MB gathered and 8 written a side) take 23.2 us, 3.1 TB/s; V rows (13.0
+// us), tables and mask (4.6) and K rows (16.0) as launches of their own 33.6.  K's workgroups hold 100 registers, so
+// four wavefronts a SIMD are resident, V's among them; five or six spill.  K no longer waits for the tables: 128
+// channels are ranked by the ballots of a wavefront.
+struct PackLayer {
+  const __half *K, *V;
+  int64_t stride_h, stride_t;
+  const int32_t *order;
+  int64_t order_stride_h;
+  const uint32_t *mm;
+  int mN2, mN4, mN8, max_n16;
+  uint8_t *V2, *V4, *V8, *K2, *K4, *K8;
+  __half *vs, *vz, *V16, *ks, *kz;
+  int k_blocks, v_blocks, mask_blocks;         // of a head; of a query head
+};
+__global__ void __launch_bounds__(256) pack_layer_d128_kernel(PackLayer a, LayerTables t, LayerMask m) {
+  extern __shared__ float smem[];
+  int x = blockIdx.x;
   const int h = blockIdx.y;
-  const int tv = counts[4 * h] + counts[4 * h + 1] + counts[4 * h + 2], n16 = counts[4 * h + 3];
-  const int64_t t0 = (int64_t)blockIdx.x * RDKV_EMIT_ROWS_D128;
-  const int64_t t1 = t0 + RDKV_EMIT_ROWS_D128 < max_tv + max_n16 ? t0 + RDKV_EMIT_ROWS_D128 : max_tv + max_n16;
-  if (t0 < tv || (t1 > max_tv && t0 < max_tv + n16))               // uniform over the workgroup
-    k_emit_layer_d128_body<true>(smem, K, stride_h, stride_t, order, order_stride_h, counts, max_tv, max_n16, mm,
-                                 slot_channel, n2p, n4p, n8, K2, K4, K8, scale_out, zp_out);
-  else
-    k_emit_layer_d128_body<false>(smem, K, stride_h, stride_t, order, order_stride_h, counts, max_tv, max_n16, mm,
-                                  slot_channel, n2p, n4p, n8, K2, K4, K8, scale_out, zp_out);
+  if (x < a.k_blocks) {
+    k_emit_layer_d128<true>(x, KWidths{t.k_bits, t.kb_es, t.kb_stride_h}, smem, a.K, a.stride_h, a.stride_t, a.order,
+                            a.order_stride_h, t.counts4, t.max_tv, a.max_n16, a.mm, nullptr, t.n2p, t.n4p, t.n8o, a.K2, a.K4,
+                            a.K8, a.ks, a.kz);
+  } else if ((x -= a.k_blocks) < a.v_blocks) {
+    pack_v_layer_d128(x, a.v_blocks, a.V, a.stride_h, a.stride_t, a.order, a.order_stride_h, t.counts4, a.mN2, a.mN4, a.mN8,
+                      a.max_n16, t.max_tv, a.V2, a.V4, a.V8, a.vs, a.vz, a.V16, nullptr);
+  } else if (x == a.v_blocks) {
+    layer_tables_block(t, h);
+  } else {
+    x -= a.v_blocks + 1;
+    const int g = x / a.mask_blocks;
+    softmax_mask_block(m, x - g * a.mask_blocks, a.mask_blocks, h * t.G + g);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1395,6 +1520,53 @@ RDKV_API int rdkv_pack_layer_k_rows(const void *K_f16, int64_t stride_h, int64_t
   return pack_layer_k_rows("rdkv_pack_layer_k_rows", K_f16, stride_h, stride_t, H_kv, D, order, order_stride_h,
                            counts, max_tv, max_n16, slot_channel, n2p, n4p, n8, K2, K4, K8, K_scale_f16, K_zp_f16,
                            minmax_ws, minmax_started, (hipStream_t)stream);
+}
+
+RDKV_API int rdkv_pack_layer(const RdkvPackLayer *y, void *stream) {
+  const char *fn = "rdkv_pack_layer";
+  RDKV_REQUIRE(y && y->H_kv >= 1 && y->H_kv <= 65535 && y->G >= 1, "%s: bad shape", fn);
+  const int64_t max_tk = y->max_tv + y->max_n16, v_rows = (int64_t)y->mN[0] + y->mN[1] + y->mN[2] + y->max_n16;
+  const int Dp = y->n2p + y->n4p + y->n8;
+  RDKV_REQUIRE(y->mN[0] >= 0 && y->mN[1] >= 0 && y->mN[2] >= 0 && y->max_n16 >= 0 && y->max_tv >= 0 && max_tk > 0 &&
+                   max_tk < 0x7fff0000LL && v_rows < 0x7fff0000LL && y->max_tv <= v_rows - y->max_n16,
+               "%s: bad token counts", fn);
+  RDKV_REQUIRE(y->n2p >= 0 && y->n4p >= 0 && y->n8 >= 0 && y->n2p % 4 == 0 && y->n4p % 2 == 0 && Dp >= 1 && Dp <= 512 &&
+                   y->kept_max >= 0 && y->kept_max <= Dp,
+               "%s: bad segment sizes (%d,%d,%d)", fn, y->n2p, y->n4p, y->n8);
+  RDKV_REQUIRE(y->ref_head >= 0 && y->ref_head < y->H_kv && y->tv_ref >= 0 && y->tv_ref <= y->max_tv, "%s: bad head", fn);
+  RDKV_REQUIRE(y->kb_elem_size == 1 || y->kb_elem_size == 2 || y->kb_elem_size == 4 || y->kb_elem_size == 8,
+               "%s: element size must be 1, 2, 4 or 8", fn);
+  RDKV_REQUIRE(y->K_f16 && y->V_f16 && y->order && y->k_bits && y->counts && y->info && y->minmax, "%s: null input", fn);
+  RDKV_REQUIRE((y->mN[0] == 0 || y->V2) && (y->mN[1] == 0 || y->V4) && (y->mN[2] == 0 || y->V8) &&
+                   (y->max_n16 == 0 || y->V16_f16) && (y->max_tv == 0 || (y->V_scale_f16 && y->V_zp_f16)) &&
+                   (y->n2p == 0 || y->K2) && (y->n4p == 0 || y->K4) && (y->n8 == 0 || y->K8) && y->K_scale_f16 &&
+                   y->K_zp_f16 && y->perm && y->perm_for_q && (y->kept_max == 0 || y->sort_ch) && y->seg_ch && y->seg_tok &&
+                   y->t_eff && y->t_eff_k && y->n_v16 && (y->tv_ref == 0 || (y->sort_idx && y->rank3)) && y->softmax_mask,
+               "%s: null output", fn);
+  RDKV_REQUIRE(y->stride_t % 8 == 0 && y->stride_h % 8 == 0 &&
+                   (((uintptr_t)y->K_f16 | (uintptr_t)y->V_f16 | (uintptr_t)y->V16_f16) % 16) == 0 &&
+                   (((uintptr_t)y->V2 | (uintptr_t)y->V4 | (uintptr_t)y->V8) % 8) == 0,
+               "%s: rows must be 16-byte aligned", fn);
+  const int rows_wg = 4 * RDKV_PACK_V_ROWS_PER_WAVE;
+  PackLayer a{(const __half *)y->K_f16, (const __half *)y->V_f16, y->stride_h, y->stride_t, y->order, y->order_stride_h,
+              reinterpret_cast<const uint32_t *>(y->minmax), y->mN[0], y->mN[1], y->mN[2], y->max_n16, y->V2, y->V4, y->V8,
+              y->K2, y->K4, y->K8, (__half *)y->V_scale_f16, (__half *)y->V_zp_f16, (__half *)y->V16_f16,
+              (__half *)y->K_scale_f16, (__half *)y->K_zp_f16, (int)rdkv_cdiv(max_tk, RDKV_EMIT_ROWS_D128),
+              (int)(rdkv_cdiv(y->mN[0], rows_wg) + rdkv_cdiv(y->mN[1], rows_wg) + rdkv_cdiv(y->mN[2], rows_wg) +
+                    rdkv_cdiv(y->max_n16, rows_wg)),
+              (int)std::min<int64_t>(rdkv_cdiv(max_tk, 256 * 4), 1024)};
+  const LayerTables t{y->k_bits, y->kb_elem_size, y->kb_stride_h, 128, y->G, y->counts, y->info, y->n2p, y->n4p, y->n8,
+                      y->kept_max, y->max_tv, nullptr, y->perm, y->perm_for_q, y->sort_ch, y->seg_ch, y->seg_tok, y->t_eff,
+                      y->t_eff_k, y->n_v16};
+  const LayerMask m{y->counts, y->G, y->max_tv, max_tk, y->softmax_mask, y->order + (int64_t)y->ref_head * y->order_stride_h,
+                    y->rank3 + (int64_t)y->ref_head * y->rank3_stride_h, y->tv_ref, y->sort_idx};
+  const int64_t blocks = (int64_t)a.k_blocks + a.v_blocks + 1 + (int64_t)a.mask_blocks * y->G;
+  RDKV_REQUIRE(blocks <= 0x7fffffffLL, "%s: too many rows", fn);
+  const size_t lds = (size_t)128 * 16 + RDKV_EMIT_STEP_ROWS_D128 * (size_t)(4 * ((y->n2p / 4 + 3) & ~3) +
+                                                                            2 * ((y->n4p / 2 + 3) & ~3) + ((y->n8 + 3) & ~3) + 4);
+  hipLaunchKernelGGL(pack_layer_d128_kernel, dim3((unsigned)blocks, y->H_kv), dim3(256), lds, (hipStream_t)stream, a, t, m);
+  RDKV_CHECK_LAUNCH(fn);
+  return RDKV_OK;
 }
 
 RDKV_API int rdkv_pack_layers_k_minmax(const void *const *K_f16, const int64_t *strides, int n_layers, int H_kv, int64_t T, int D,

@@ -726,11 +726,11 @@ def _pad_and_stack_per_head_layers(
 
 _PLAN_INT_DTYPES = (torch.uint8, torch.int16, torch.int32, torch.int64)
 
-# Tokens from which a layer's K min / max are launched ahead of the host's read of the plan.  Below, the host is
-# the longer side and their own call costs 3 .. 7 us of it.  Us a call ahead / behind, 8 KV heads: selection and packing
-# of 16k tokens 177 / 176, 31k 178 / 178, 64k 200 / 222, 100k 272 / 304; four layers to the streaming format 4k
-# 507 / 501, 16k 524 / 520, 24k 547 / 543, 32k 543 / 583.
-_EARLY_MINMAX_TOKENS = 28672
+# Tokens from which a layer's K min / max are launched ahead of the host's read of the plan: always, for they run
+# while the numbers travel and the layer's rows, tables and mask are then one launch.  Us a call ahead / behind, 8 KV
+# heads: packing of 1k tokens 62 / 72, 4k 62 / 72, 16k 62 / 72, 31k 72 / 80, 100k 168 / 176; selection and packing of
+# 4k 87 / 100, 16k 88 / 99, 31k 89 / 101, 100k 150 / 162.
+_EARLY_MINMAX_TOKENS = 1
 
 
 def _early_minmax(Ks: Sequence[Tensor], dev) -> bool:
