@@ -727,6 +727,13 @@ int rdkv_pack_layer_plan_start(const void *v_bits, int vb_elem_size, int64_t vb_
                                int32_t *plan, float *minmax_ws, int minmax_floats_per_head, uint64_t *host_words,
                                uint32_t tag, void *stream);
 
+/* A plan of n_layers layers of one shape from the layers' own widths (v_bits[l] [H_kv, T], k_bits[l] [H_kv, D], rows
+ * back to back; the arrays in host memory): order [n_layers * H_kv, T] and plan as above for n_layers * H_kv heads,
+ * layer by layer, without rank3; k_bits_u8 [n_layers * H_kv, D] (NULL: not): the channel widths as bytes. */
+int rdkv_plan_layers(const void *const *v_bits, int vb_elem_size, const void *const *k_bits, int kb_elem_size,
+                     int n_layers, int H_kv, int64_t T, int D, int32_t *order, int32_t *plan, float *minmax_ws,
+                     int minmax_floats_per_head, uint8_t *k_bits_u8, uint64_t *host_words, uint32_t tag, void *stream);
+
 /* K min / max of the kept rows of n_layers layers of one shape, from what the planning launches left on the
  * device (order, counts: rows of layer l from l * H_kv on), before the host has read the class sizes: K_f16[l]
  * with strides[2 l], strides[2 l + 1] (head, token), rows 4-byte aligned; layer l's accumulators, started, at

@@ -113,6 +113,7 @@ SIGNATURES = {
     "rdkv_pack_layer_plan": (I, [P, I, L, P, I, L, I, L, I, P, L, P, L, P, P]),
     "rdkv_pack_layer_plan_start": (I, [P, I, L, P, I, L, I, L, I, P, L, P, L, P, P, I, P, ctypes.c_uint32, P]),
     "rdkv_host_words_wait": (I, [P, L, ctypes.c_uint32, P, L]),
+    "rdkv_plan_layers": (I, [P, I, P, I, I, I, L, I, P, P, P, I, P, P, ctypes.c_uint32, P]),
     "rdkv_pack_layers_k_minmax": (I, [P, P, I, I, L, I, P, L, P, P, L, P]),
     "rdkv_pack_layer": (I, [P, P]),
     "rdkv_pack_layer_tables": (I, [P, I, L, I, I, I, P, P, I, I, I, I, L, I, P, L, P, L, I, L,

@@ -29,7 +29,7 @@ namespace {
   X(rdkv_pool_scores) X(rdkv_knapsack_batched_value) X(rdkv_pack_layer_plan_ints) X(rdkv_pack_layer_plan_start)  \
   X(rdkv_pack_layers_k_minmax) X(rdkv_pack_layer_v_rows) X(rdkv_pack_layer_tables) X(rdkv_pack_layer_k_rows)     \
   X(rdkv_decode_fused) X(rdkv_decode_fused_zone_c) X(rdkv_decode_fused_workspace_bytes)                           \
-  X(rdkv_unpack_layer) X(rdkv_stream_plan_layer) X(rdkv_pack_layer)                                                           \
+  X(rdkv_unpack_layer) X(rdkv_stream_plan_layer) X(rdkv_pack_layer) X(rdkv_plan_layers)                                                           \
   X(rdkv_select_layer_start) X(rdkv_pack_layers_stream)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
@@ -411,7 +411,7 @@ PyObject *stream_order(PyObject *const *a, Py_ssize_t) {
   plain((int64_t)Vs.size() == n && (int64_t)vbs.size() == n && (int64_t)kbs.size() == n && Ks[0].is_cuda() && Ks[0].dim() == 4);
   const auto dev = Ks[0].device();
   const int64_t H = Ks[0].size(1), T = Ks[0].size(2);
-  plain(H >= 1 && T >= 1 && T <= (1 << 30) && n * H <= 65535);
+  plain(H >= 1 && T >= 1 && T <= (1 << 30) && n * H <= 65535 && H <= 8191);
   auto widths = [&](const std::vector<at::Tensor> &ts, int64_t w) {
     const auto type = ts[0].scalar_type();
     plain(type == at::kByte || type == at::kShort || type == at::kInt || type == at::kLong);
@@ -431,18 +431,19 @@ PyObject *stream_order(PyObject *const *a, Py_ssize_t) {
     K_at.push_back(K.data_ptr());
     strides.insert(strides.end(), {K.stride(1), K.stride(2)});
   }
-  at::Tensor vb, kb, order, rank3, plan, mm;
+  std::vector<const void *> vb_at, kb_at;
+  for (int64_t i = 0; i < n; ++i) vb_at.push_back(vbs[i].data_ptr()), kb_at.push_back(kbs[i].data_ptr());
+  at::Tensor kb, order, plan, mm;
   int rc;
   {
     Unlocked u;
     auto make = [&](at::IntArrayRef s, at::ScalarType t) { return at::empty(s, Ks[0].options().dtype(t)); };
-    vb = n == 1 ? vbs[0] : at::cat(vbs), kb = n == 1 ? kbs[0] : at::cat(kbs);
-    order = make({n * H, T}, at::kInt), rank3 = make({n * H, T}, at::kInt);
+    kb = make({n * H, 128}, at::kByte), order = make({n * H, T}, at::kInt);
     plan = make({lib.rdkv_pack_layer_plan_ints(n * H, T)}, at::kInt);
     mm = make({n * H * 768}, at::kFloat);
-    rc = lib.rdkv_pack_layer_plan_start(vb.data_ptr(), vb.element_size(), T, kb.data_ptr(), kb.element_size(), 128, n * H, T, 128,
-                                        data<int32_t>(order), T, data<int32_t>(rank3), T, data<int32_t>(plan), data<float>(mm),
-                                        768, words, tag, stream);
+    rc = lib.rdkv_plan_layers(vb_at.data(), vbs[0].element_size(), kb_at.data(), kbs[0].element_size(), n, H, T, 128,
+                              data<int32_t>(order), data<int32_t>(plan), data<float>(mm), 768, data<uint8_t>(kb), words, tag,
+                              stream);
     if (rc == RDKV_OK)
       rc = lib.rdkv_pack_layers_k_minmax(K_at.data(), strides.data(), n, H, T, 128, data<int32_t>(order), T, data<int32_t>(plan),
                                          data<float>(mm), 768 * H, stream);

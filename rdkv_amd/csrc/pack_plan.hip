@@ -13,128 +13,167 @@ __device__ __forceinline__ int token_class(int bits) {
   return bits == 2 ? 0 : bits == 4 ? 1 : bits == 8 ? 2 : bits == 16 ? 3 : bits == 0 ? 4 : 5;
 }
 
-// Token planning in two launches over a (chunk, head) grid, kPlanThreads tokens per chunk.
+// Widths of up to eight layers of one shape, H heads each.
+constexpr int kPlanLayers = 8;
+struct PlanWidths {
+  const void *v[kPlanLayers], *k[kPlanLayers];
+  int64_t v_stride_h, k_stride_h;
+  int v_es, k_es, H, T, D;
+};
+
+// Token planning in two launches over a (chunk, head) grid.  A thread takes four tokens of a chunk, 64 apart, a
+// wavefront 256 neighbours: 32 heads of 32k tokens are one workgroup a compute unit (with one token a thread two rounds
+// of four times the workgroups: 7 + 14 us for the pair, now 7.5 + 8.7).  Bound: the chain of a workgroup - widths, the
+// counts of its wavefronts, the head's counts by chunk, the order's stores.
+constexpr int kPlanTokens = 4;      // per thread
+constexpr int kPlanChunk = kPlanThreads * kPlanTokens, kPlanWaves = kPlanThreads / 64;
+
 // First launch: per-chunk class histogram hist[h][chunk][6]; the chunk-0 block of each head also
-// counts the head's channel classes and writes the start values of its share of the K min / max scratch.
+// counts the head's channel classes, writes the start values of its share of the K min / max scratch and, where asked
+// for, the head's widths as bytes (invalid ones as 255).
 __global__ void __launch_bounds__(kPlanThreads)
-plan_hist_kernel(const void *__restrict__ v_bits, int vb_es, int64_t vb_stride_h, int T,
-                 const void *__restrict__ k_bits, int kb_es, int64_t kb_stride_h, int D,
-                 int32_t *__restrict__ hist, int32_t *__restrict__ info, uint32_t *__restrict__ minmax,
-                 int minmax_per_head) {
-  __shared__ int cnt[kTokClasses];
+plan_hist_kernel(PlanWidths w, int32_t *__restrict__ hist, int32_t *__restrict__ info, uint32_t *__restrict__ minmax,
+                 int minmax_per_head, uint8_t *__restrict__ k8) {
+  __shared__ int wcnt[kPlanWaves][kTokClasses];
   __shared__ int kcnt[4];
-  const int h = blockIdx.y, chunk = blockIdx.x, nchunks = gridDim.x, tid = threadIdx.x, lane = tid & 63;
-  if (tid < kTokClasses) cnt[tid] = 0;
+  const int h = blockIdx.y, layer = h / w.H, hl = h - layer * w.H, chunk = blockIdx.x, nchunks = gridDim.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   if (tid < 4) kcnt[tid] = 0;
-  __syncthreads();
-  const int t = chunk * kPlanThreads + tid;
-  const int cls = t < T ? token_class(load_int(v_bits, vb_es, (int64_t)h * vb_stride_h + t)) : -1;
+  const int t0 = chunk * kPlanChunk + wave * 64 * kPlanTokens + lane;
+  int cls[kPlanTokens];
+#pragma unroll
+  for (int i = 0; i < kPlanTokens; ++i) {
+    const int t = t0 + 64 * i;
+    cls[i] = t < w.T ? token_class(load_int(w.v[layer], w.v_es, hl * w.v_stride_h + t)) : -1;
+  }
 #pragma unroll
   for (int k = 0; k < kTokClasses; ++k) {
-    const uint64_t m = __ballot(cls == k);
-    if (lane == 0 && m) atomicAdd(&cnt[k], __popcll(m));
-  }
-  if (chunk == 0 && minmax) {
-    for (int i = tid; i < minmax_per_head; i += blockDim.x)
-      minmax[(int64_t)h * minmax_per_head + i] = rdkv_float_to_ordered(((i / D) & 1) ? -INFINITY : INFINITY);
-  }
-  if (chunk == 0) {
-    int bad = 0;
-    for (int ch = tid; ch < D; ch += blockDim.x) {
-      const int kc = channel_class(load_int(k_bits, kb_es, (int64_t)h * kb_stride_h + ch));
-      if (kc >= 0) atomicAdd(&kcnt[kc], 1);
-      if (kc == -2) bad = 1;
-    }
-    if (bad) atomicAdd(&kcnt[3], 1);
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < kPlanTokens; ++i) n += __popcll(__ballot(cls[i] == k));
+    if (lane == 0) wcnt[wave][k] = n;
   }
   __syncthreads();
-  if (tid < kTokClasses) hist[((int64_t)h * nchunks + chunk) * kTokClasses + tid] = cnt[tid];
   if (chunk == 0) {
+    if (minmax)
+      for (int i = tid; i < minmax_per_head; i += kPlanThreads)
+        minmax[(int64_t)h * minmax_per_head + i] = rdkv_float_to_ordered(((i / w.D) & 1) ? -INFINITY : INFINITY);
+    int bad = 0;
+    for (int ch = tid; ch < w.D; ch += kPlanThreads) {
+      const int bits = load_int(w.k[layer], w.k_es, hl * w.k_stride_h + ch), kc = channel_class(bits);
+      if (kc >= 0) atomicAdd(&kcnt[kc], 1);
+      if (kc == -2) bad = 1;
+      if (k8) k8[(int64_t)h * w.D + ch] = kc == -2 ? 255 : bits;
+    }
+    if (bad) atomicAdd(&kcnt[3], 1);
+    __syncthreads();
     if (tid < 4) info[8 * h + 2 + tid] = kcnt[tid];
     if (tid >= 4 && tid < 6) info[8 * h + 2 + tid] = 0;
   }
+  if (tid < kTokClasses) {
+    int n = 0;
+#pragma unroll
+    for (int i = 0; i < kPlanWaves; ++i) n += wcnt[i][tid];
+    hist[((int64_t)h * nchunks + chunk) * kTokClasses + tid] = n;
+  }
+}
+
+// The sum over the 64 lanes, in every lane.
+__device__ __forceinline__ int wave_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);       // quad_perm [1,0,3,2]
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, true);       // quad_perm [2,3,0,1]
+  v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);      // row_half_mirror
+  v += __builtin_amdgcn_update_dpp(0, v, 0x140, 0xf, 0xf, true);      // row_mirror
+  const auto r = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+  v = (int)(r[0] + r[1]);
+  const auto t = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+  return (int)(t[0] + t[1]);
 }
 
 // Second launch: every block sums the histograms of its head (class totals and what lies before
 // its chunk) and scatters its tokens.  order[h, :] = token indices sorted by class, stable (the
-// classes in the order 2, 4, 8, 16 bit, evicted, invalid); rank3[h, t] = number of tokens before
+// classes in the order 2, 4, 8, 16 bit, evicted, invalid); rank3[h, t] (or null) = number of tokens before
 // t that are quantized (2/4/8 bit); counts4[h] = (n2, n4, n8, n16); info[h][0..1] = (evicted,
 // invalid widths).
 __global__ void __launch_bounds__(kPlanThreads)
-plan_scatter_kernel(const void *__restrict__ v_bits, int vb_es, int64_t vb_stride_h, int T,
-                    const int32_t *__restrict__ hist, int32_t *__restrict__ order, int64_t order_stride_h,
+plan_scatter_kernel(PlanWidths w, const int32_t *__restrict__ hist, int32_t *__restrict__ order, int64_t order_stride_h,
                     int32_t *__restrict__ rank3, int64_t rank3_stride_h, int32_t *__restrict__ counts4,
                     int32_t *__restrict__ info, uint64_t *__restrict__ host_words, uint32_t tag) {
-  __shared__ int wsum[kPlanThreads / 64][2 * kTokClasses];
-  __shared__ int red[2 * kTokClasses];
-  __shared__ int wcnt[kPlanThreads / 64][kTokClasses];
-  __shared__ int wpre[kPlanThreads / 64][kTokClasses];
-  const int h = blockIdx.y, chunk = blockIdx.x, nchunks = gridDim.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nwaves = blockDim.x >> 6;
-  // totals over all chunks and over the chunks before this one
-  int acc[2 * kTokClasses];
+  __shared__ int total[kTokClasses], before[kTokClasses];       // of the head, of its chunks before this one
+  __shared__ int wcnt[kPlanWaves][kTokClasses];
+  const int h = blockIdx.y, layer = h / w.H, hl = h - layer * w.H, chunk = blockIdx.x, nchunks = gridDim.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int t0 = chunk * kPlanChunk + wave * 64 * kPlanTokens + lane;
+  int cls[kPlanTokens];
 #pragma unroll
-  for (int k = 0; k < 2 * kTokClasses; ++k) acc[k] = 0;
-  for (int c = tid; c < nchunks; c += blockDim.x) {
+  for (int i = 0; i < kPlanTokens; ++i) {
+    const int t = t0 + 64 * i;
+    cls[i] = t < w.T ? token_class(load_int(w.v[layer], w.v_es, hl * w.v_stride_h + t)) : -1;
+  }
+  if (wave < kTokClasses) {            // a class a wavefront
+    int all = 0, ahead = 0;
+    for (int c = lane; c < nchunks; c += 64) {
+      const int v = hist[((int64_t)h * nchunks + c) * kTokClasses + wave];
+      all += v;
+      ahead += c < chunk ? v : 0;
+    }
+    all = wave_sum(all);
+    ahead = wave_sum(ahead);
+    if (lane == 0) {
+      total[wave] = all;
+      before[wave] = ahead;
+    }
+  }
+  // of the wavefront's 256 tokens: those of a token's class before it, the quantized ones before it
+  int rank[kPlanTokens], q_rank[kPlanTokens], run[kTokClasses], q_run = 0;
+#pragma unroll
+  for (int k = 0; k < kTokClasses; ++k) run[k] = 0;
+#pragma unroll
+  for (int i = 0; i < kPlanTokens; ++i) {
+    uint64_t q = 0;
+    rank[i] = 0;
 #pragma unroll
     for (int k = 0; k < kTokClasses; ++k) {
-      const int v = hist[((int64_t)h * nchunks + c) * kTokClasses + k];
-      acc[k] += v;
-      acc[kTokClasses + k] += c < chunk ? v : 0;
+      const uint64_t m = __ballot(cls[i] == k);
+      if (k < 3) q |= m;
+      if (cls[i] == k) rank[i] = run[k] + lanes_below(m);
+      run[k] += __popcll(m);
     }
+    q_rank[i] = q_run + lanes_below(q);
+    q_run += __popcll(q);
   }
-  // (a wavefront none of whose threads had a chunk has nothing to add up)
-  const bool wave_has_chunks = wave * 64 < nchunks;
 #pragma unroll
-  for (int k = 0; k < 2 * kTokClasses; ++k) {
-    if (wave_has_chunks) {
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) acc[k] += __shfl_xor(acc[k], off, 64);
-    }
-    if (lane == 0) wsum[wave][k] = acc[k];
-  }
-  const int t = chunk * kPlanThreads + tid;
-  const int cls = t < T ? token_class(load_int(v_bits, vb_es, (int64_t)h * vb_stride_h + t)) : -1;
-  int my_rank = 0;
-  uint64_t qmask = 0;
+  for (int k = 0; k < kTokClasses; ++k)
+    if (lane == 0) wcnt[wave][k] = run[k];
+  __syncthreads();
+  int base[kTokClasses], before_q = 0, seg_base = 0;     // where the wavefront's tokens of a class begin
 #pragma unroll
   for (int k = 0; k < kTokClasses; ++k) {
-    const uint64_t m = __ballot(cls == k);
-    if (k < 3) qmask |= m;
-    if (cls == k) my_rank = lanes_below(m);
-    if (lane == 0) wcnt[wave][k] = __popcll(m);
-  }
-  const int my_q = lanes_below(qmask);
-  __syncthreads();
-  if (tid < 2 * kTokClasses) {
-    int s = 0;
-    for (int w = 0; w < nwaves; ++w) s += wsum[w][tid];
-    red[tid] = s;
-  } else if (tid >= 64 && tid < 64 + kTokClasses) {
-    const int k = tid - 64;
-    int s = 0;
-    for (int w = 0; w < nwaves; ++w) { wpre[w][k] = s; s += wcnt[w][k]; }
-  }
-  __syncthreads();
-  int pos = 0, before_q = 0, seg_base = 0;
-#pragma unroll
-  for (int k = 0; k < kTokClasses; ++k) {
-    const int ahead = red[kTokClasses + k] + wpre[wave][k];
-    if (cls == k) pos = seg_base + ahead + my_rank;
+    int ahead = before[k];
+    // (lane i holds what wavefront i counted)
+    ahead += wave_sum(lane < wave ? wcnt[lane & (kPlanWaves - 1)][k] : 0);
+    base[k] = seg_base + ahead;
     if (k < 3) before_q += ahead;
-    seg_base += red[k];
+    seg_base += total[k];
   }
-  if (t < T) {
-    order[(int64_t)h * order_stride_h + pos] = t;
-    rank3[(int64_t)h * rank3_stride_h + t] = before_q + my_q;
+#pragma unroll
+  for (int i = 0; i < kPlanTokens; ++i) {
+    const int t = t0 + 64 * i;
+    int pos = rank[i];
+#pragma unroll
+    for (int k = 0; k < kTokClasses; ++k) pos += cls[i] == k ? base[k] : 0;
+    if (t < w.T) {
+      order[(int64_t)h * order_stride_h + pos] = t;
+      if (rank3) rank3[(int64_t)h * rank3_stride_h + t] = before_q + q_rank[i];
+    }
   }
   if (chunk == 0) {
-    if (tid < 4) counts4[4 * h + tid] = red[tid];
-    if (tid == 4) info[8 * h + 0] = red[4];
-    if (tid == 5) info[8 * h + 1] = red[5];
+    if (tid < 4) counts4[4 * h + tid] = total[tid];
+    if (tid == 4) info[8 * h + 0] = total[4];
+    if (tid == 5) info[8 * h + 1] = total[5];
     // the head's twelve numbers to the host, each word with the call's tag: whole whenever its tag is there
     if (host_words && tid < 12) {
-      const int v = tid < 6 ? red[tid] : info[8 * h + tid - 4];
+      const int v = tid < 6 ? total[tid] : info[8 * h + tid - 4];
       rdkv_host_word(host_words, 12 * (int64_t)h + tid, tag, v);
     }
   }
@@ -165,7 +204,22 @@ bool elem_size_ok(int es) { return es == 1 || es == 2 || es == 4 || es == 8; }
 
 RDKV_API int64_t rdkv_pack_layer_plan_ints(int H_kv, int64_t T) {
   if (H_kv < 0 || T < 0) return 0;
-  return (int64_t)H_kv * (12 + kTokClasses * rdkv_cdiv(T, kPlanThreads));
+  return (int64_t)H_kv * (12 + kTokClasses * rdkv_cdiv(T, kPlanChunk));
+}
+
+// n_layers of a plan from layer `first` on: their rows of order, rank3, counts and info, their part of the histograms
+static void launch_plan(const PlanWidths &w, int n_heads, int64_t first_head, int64_t all_heads, int32_t *order,
+                        int64_t order_stride_h, int32_t *rank3, int64_t rank3_stride_h, int32_t *plan, float *minmax_ws,
+                        int minmax_floats_per_head, uint8_t *k8, uint64_t *host_words, uint32_t tag, hipStream_t s) {
+  const int64_t nchunks = rdkv_cdiv(w.T, kPlanChunk), f = first_head;
+  int32_t *counts4 = plan + 4 * f, *info = plan + 4 * all_heads + 8 * f, *hist = plan + 12 * all_heads + kTokClasses * nchunks * f;
+  const dim3 grid((unsigned)nchunks, n_heads);
+  hipLaunchKernelGGL(plan_hist_kernel, grid, dim3(kPlanThreads), 0, s, w, hist, info,
+                     minmax_ws ? (uint32_t *)minmax_ws + f * minmax_floats_per_head : nullptr, minmax_floats_per_head,
+                     k8 ? k8 + f * w.D : nullptr);
+  hipLaunchKernelGGL(plan_scatter_kernel, grid, dim3(kPlanThreads), 0, s, w, hist, order + f * order_stride_h, order_stride_h,
+                     rank3 ? rank3 + f * rank3_stride_h : nullptr, rank3_stride_h, counts4, info,
+                     host_words ? host_words + 12 * f : nullptr, tag);
 }
 
 RDKV_API int rdkv_pack_layer_plan_start(const void *v_bits, int vb_elem_size, int64_t vb_stride_h, const void *k_bits,
@@ -177,15 +231,30 @@ RDKV_API int rdkv_pack_layer_plan_start(const void *v_bits, int vb_elem_size, in
   RDKV_REQUIRE(H_kv >= 1 && H_kv <= 65535 && D >= 1 && T >= 1 && T <= (1LL << 30), "%s: bad shape", fn);
   RDKV_REQUIRE(elem_size_ok(vb_elem_size) && elem_size_ok(kb_elem_size), "%s: element sizes must be 1, 2, 4 or 8", fn);
   RDKV_REQUIRE(k_bits && plan && v_bits && order && rank3, "%s: null pointer", fn);
-  const int64_t nchunks = rdkv_cdiv(T, kPlanThreads);
-  int32_t *counts4 = plan, *info = plan + 4 * (int64_t)H_kv, *hist = plan + 12 * (int64_t)H_kv;
-  hipStream_t s = (hipStream_t)stream;
-  hipLaunchKernelGGL(plan_hist_kernel, dim3((unsigned)nchunks, H_kv), dim3(kPlanThreads), 0, s, v_bits, vb_elem_size,
-                     vb_stride_h, (int)T, k_bits, kb_elem_size, kb_stride_h, D, hist, info, (uint32_t *)minmax_ws,
-                     minmax_floats_per_head);
-  hipLaunchKernelGGL(plan_scatter_kernel, dim3((unsigned)nchunks, H_kv), dim3(kPlanThreads), 0, s, v_bits,
-                     vb_elem_size, vb_stride_h, (int)T, hist, order, order_stride_h, rank3, rank3_stride_h, counts4,
-                     info, host_words, tag);
+  const PlanWidths w{{v_bits}, {k_bits}, vb_stride_h, kb_stride_h, vb_elem_size, kb_elem_size, H_kv, (int)T, D};
+  launch_plan(w, H_kv, 0, H_kv, order, order_stride_h, rank3, rank3_stride_h, plan, minmax_ws, minmax_floats_per_head, nullptr,
+              host_words, tag, (hipStream_t)stream);
+  RDKV_CHECK_LAUNCH(fn);
+  return RDKV_OK;
+}
+
+RDKV_API int rdkv_plan_layers(const void *const *v_bits, int vb_elem_size, const void *const *k_bits, int kb_elem_size,
+                              int n_layers, int H_kv, int64_t T, int D, int32_t *order, int32_t *plan, float *minmax_ws,
+                              int minmax_floats_per_head, uint8_t *k_bits_u8, uint64_t *host_words, uint32_t tag,
+                              void *stream) {
+  const char *fn = "rdkv_plan_layers";
+  RDKV_REQUIRE(n_layers >= 0 && H_kv >= 1 && H_kv <= 65535 / kPlanLayers && D >= 1 && T >= 1 && T <= (1LL << 30), "%s: bad shape",
+               fn);
+  RDKV_REQUIRE(elem_size_ok(vb_elem_size) && elem_size_ok(kb_elem_size), "%s: element sizes must be 1, 2, 4 or 8", fn);
+  RDKV_REQUIRE(n_layers == 0 || (v_bits && k_bits && plan && order), "%s: null pointer", fn);
+  for (int l = 0; l < n_layers; ++l) RDKV_REQUIRE(v_bits[l] && k_bits[l], "%s: null pointer", fn);
+  for (int first = 0; first < n_layers; first += kPlanLayers) {
+    const int n = n_layers - first < kPlanLayers ? n_layers - first : kPlanLayers;
+    PlanWidths w{{}, {}, T, D, vb_elem_size, kb_elem_size, H_kv, (int)T, D};
+    for (int l = 0; l < n; ++l) w.v[l] = v_bits[first + l], w.k[l] = k_bits[first + l];
+    launch_plan(w, n * H_kv, (int64_t)first * H_kv, (int64_t)n_layers * H_kv, order, T, nullptr, 0, plan, minmax_ws,
+                minmax_floats_per_head, k_bits_u8, host_words, tag, (hipStream_t)stream);
+  }
   RDKV_CHECK_LAUNCH(fn);
   return RDKV_OK;
 }

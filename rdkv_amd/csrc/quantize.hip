@@ -684,11 +684,21 @@ k_minmax_layer_kernel(const __half *__restrict__ K, int64_t stride_h, int64_t st
 // packed fp16 (exact) until the end.
 #define RDKV_LAYER_MINMAX_WAVES_D128 8
 #define RDKV_LAYER_MINMAX_ROWS_D128 (64 * RDKV_LAYER_MINMAX_WAVES_D128)
+// Up to eight layers of one shape side by side (four of 32k: 38.8 us, one after the other 48).
+constexpr int kMinmaxLayers = 8;
+struct MinmaxLayers {
+  const __half *K[kMinmaxLayers];
+  int64_t stride_h[kMinmaxLayers], stride_t[kMinmaxLayers];
+};
 __global__ void __launch_bounds__(64 * RDKV_LAYER_MINMAX_WAVES_D128)
-k_minmax_layer_d128_kernel(const __half *__restrict__ K, int64_t stride_h, int64_t stride_t,
-                           const int32_t *__restrict__ order, int64_t order_stride_h,
-                           const int32_t *__restrict__ counts, uint32_t *__restrict__ mm) {
-  const int h = blockIdx.y;
+k_minmax_layer_d128_kernel(MinmaxLayers layers, const int32_t *__restrict__ order, int64_t order_stride_h,
+                           const int32_t *__restrict__ counts, uint32_t *__restrict__ mm, int64_t mm_stride) {
+  const int h = blockIdx.y, layer = blockIdx.z;
+  const __half *K = layers.K[layer];
+  const int64_t stride_h = layers.stride_h[layer], stride_t = layers.stride_t[layer];
+  order += (int64_t)layer * gridDim.y * order_stride_h;
+  counts += 4 * (int64_t)layer * gridDim.y;
+  mm += layer * mm_stride;
   const int tk = counts[4 * h] + counts[4 * h + 1] + counts[4 * h + 2] + counts[4 * h + 3];
   const int t0 = blockIdx.x * RDKV_LAYER_MINMAX_ROWS_D128;
   if (t0 >= tk) return;
@@ -1404,7 +1414,7 @@ static int layer_k_minmax(const char *fn, const void *K_f16, int64_t stride_h, i
     hipLaunchKernelGGL(k_minmax_layer_d128_kernel,
                        dim3((unsigned)rdkv_cdiv(max_tk, RDKV_LAYER_MINMAX_ROWS_D128), H_kv),
                        dim3(64 * RDKV_LAYER_MINMAX_WAVES_D128), 0, s,
-                       (const __half *)K_f16, stride_h, stride_t, order, order_stride_h, counts, mm);
+                       MinmaxLayers{{(const __half *)K_f16}, {stride_h}, {stride_t}}, order, order_stride_h, counts, mm, 0);
   } else {
     hipLaunchKernelGGL(k_minmax_layer_kernel, dim3((unsigned)mblocks, H_kv), dim3(64, 4), 0, s,
                        (const __half *)K_f16, stride_h, stride_t, D, order, order_stride_h, counts, mm);
@@ -1577,14 +1587,31 @@ RDKV_API int rdkv_pack_layers_k_minmax(const void *const *K_f16, const int64_t *
                "%s: bad shape", fn);
   RDKV_REQUIRE(n_layers == 0 || (K_f16 && strides && order && counts && minmax_ws && ws_stride >= (int64_t)H_kv * 2 * D),
                "%s: bad arguments", fn);
-  for (int l = 0; l < n_layers; ++l) {
-    const int64_t sh = strides[2 * l], st = strides[2 * l + 1];
-    RDKV_REQUIRE(K_f16[l] && st % 2 == 0 && sh % 2 == 0 && ((uintptr_t)K_f16[l] % 4) == 0, "%s: rows must be 4-byte aligned",
-                 fn);
-    const int rc = layer_k_minmax(fn, K_f16[l], sh, st, H_kv, D, order + (int64_t)l * H_kv * order_stride_h, order_stride_h,
-                                  counts + 4 * (int64_t)l * H_kv, T, reinterpret_cast<uint32_t *>(minmax_ws + l * ws_stride),
-                                  false, (hipStream_t)stream);
-    if (rc != RDKV_OK) return rc;
+  for (int l = 0; l < n_layers; ++l)
+    RDKV_REQUIRE(K_f16[l] && strides[2 * l] % 2 == 0 && strides[2 * l + 1] % 2 == 0 && ((uintptr_t)K_f16[l] % 4) == 0,
+                 "%s: rows must be 4-byte aligned", fn);
+  for (int l = 0, n; l < n_layers; l += n) {
+    auto rows16 = [&](int i) {
+      return D == 128 && strides[2 * i] % 8 == 0 && strides[2 * i + 1] % 8 == 0 && ((uintptr_t)K_f16[i] % 16) == 0;
+    };
+    const int32_t *order_l = order + (int64_t)l * H_kv * order_stride_h, *counts_l = counts + 4 * (int64_t)l * H_kv;
+    uint32_t *mm = reinterpret_cast<uint32_t *>(minmax_ws + l * ws_stride);
+    n = 1;
+    if (!rows16(l)) {
+      const int rc = layer_k_minmax(fn, K_f16[l], strides[2 * l], strides[2 * l + 1], H_kv, D, order_l, order_stride_h, counts_l,
+                                    T, mm, false, (hipStream_t)stream);
+      if (rc != RDKV_OK) return rc;
+      continue;
+    }
+    while (n < kMinmaxLayers && l + n < n_layers && rows16(l + n)) ++n;
+    MinmaxLayers y{};
+    for (int i = 0; i < n; ++i) {
+      y.K[i] = (const __half *)K_f16[l + i];
+      y.stride_h[i] = strides[2 * (l + i)], y.stride_t[i] = strides[2 * (l + i) + 1];
+    }
+    hipLaunchKernelGGL(k_minmax_layer_d128_kernel, dim3((unsigned)rdkv_cdiv(T, RDKV_LAYER_MINMAX_ROWS_D128), H_kv, n),
+                       dim3(64 * RDKV_LAYER_MINMAX_WAVES_D128), 0, (hipStream_t)stream, y, order_l, order_stride_h, counts_l, mm,
+                       ws_stride);
   }
   RDKV_CHECK_LAUNCH(fn);
   return RDKV_OK;

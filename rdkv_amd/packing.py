@@ -728,7 +728,7 @@ _PLAN_INT_DTYPES = (torch.uint8, torch.int16, torch.int32, torch.int64)
 
 # Tokens from which a layer's K min / max are launched ahead of the host's read of the plan: always, for they run
 # while the numbers travel and the layer's rows, tables and mask are then one launch.  Us a call ahead / behind, 8 KV
-# heads: packing of 1k tokens 62 / 72, 4k 62 / 72, 16k 62 / 72, 31k 72 / 80, 100k 168 / 176; selection and packing of
+# heads: packing of 1k tokens 57 / 65, 4k 59 / 67, 16k 60 / 67, 31k 70 / 79, 100k 163 / 169; selection and packing of
 # 4k 87 / 100, 16k 88 / 99, 31k 89 / 101, 100k 150 / 162.
 _EARLY_MINMAX_TOKENS = 1
 
