@@ -204,7 +204,7 @@ bool elem_size_ok(int es) { return es == 1 || es == 2 || es == 4 || es == 8; }
 
 RDKV_API int64_t rdkv_pack_layer_plan_ints(int H_kv, int64_t T) {
   if (H_kv < 0 || T < 0) return 0;
-  return (int64_t)H_kv * (12 + kTokClasses * rdkv_cdiv(T, kPlanChunk));
+  return (int64_t)H_kv * (12 + kTokClasses * rdkv_cdiv(T, kPlanThreads));      // (the histograms take a quarter of theirs)
 }
 
 // n_layers of a plan from layer `first` on: their rows of order, rank3, counts and info, their part of the histograms
