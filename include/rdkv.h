@@ -528,8 +528,10 @@ int rdkv_stream_relayout_layer(const uint8_t *K2, int64_t k2_stride_h, int64_t k
 int rdkv_pack_layer_stream_ws_init(float *minmax_ws, int H_kv, void *stream);
 
 /* Several layers of one plan (and one head count) in two launches: layer l's heads are rows l * H_kv .. of order,
- * counts, k_bits, units, src_slot; its accumulators, complete (rdkv_pack_layers_k_minmax), lie at minmax_ws + l * H_kv *
- * 768, its largest scales at scale_max + 2 * l * H_kv.  layers[l] (host memory): what differs. */
+ * counts, info, k_bits, units; its accumulators, complete (rdkv_pack_layers_k_minmax), lie at minmax_ws + l * H_kv *
+ * 768, its largest scales at scale_max + 2 * l * H_kv.  layers[l] (host memory): what differs.  units (device, written)
+ * and the slots are planned by the first launch from counts and info, the two parts of the layers' plan, as
+ * rdkv_stream_plan_layer plans them (q_row 0). */
 typedef struct RdkvStreamLayer {
   const void *K_f16, *V_f16;
   int64_t stride_h, stride_t;
@@ -538,9 +540,9 @@ typedef struct RdkvStreamLayer {
   int32_t n2p, n4p, n8, max_n16, max_tiles, reserved;
 } RdkvStreamLayer;
 int rdkv_pack_layers_stream(const RdkvStreamLayer *layers, int n_layers, int H_kv, const int32_t *order,
-                            int64_t order_stride_h, const int32_t *counts, const void *k_bits, int kb_elem_size,
-                            int64_t kb_stride_h, const RdkvUnit *units, const int16_t *src_slot, int n_slots_max,
-                            float *minmax_ws, float *scale_max, void *stream);
+                            int64_t order_stride_h, const int32_t *counts, const int32_t *info, const void *k_bits,
+                            int kb_elem_size, int64_t kb_stride_h, RdkvUnit *units, float *minmax_ws, float *scale_max,
+                            void *stream);
 int rdkv_pack_layer_stream(const void *K_f16, const void *V_f16, int64_t stride_h, int64_t stride_t,
                            int H_kv, const int32_t *order, int64_t order_stride_h, const int32_t *counts,
                            const void *k_bits, int kb_elem_size, int64_t kb_stride_h, int n2p, int n4p, int n8,

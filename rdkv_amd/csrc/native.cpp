@@ -398,7 +398,6 @@ std::vector<at::Tensor> tensors(PyObject *list) {
   for (Py_ssize_t i = 0; i < PyList_GET_SIZE(list); ++i) v.push_back(tensor(PyList_GET_ITEM(list, i)));
   return v;
 }
-constexpr int kSlots = 160;       // columns of a unit's slot table
 
 // K, V, V widths, K widths (lists: an entry each), words, tag, stream
 PyObject *stream_order(PyObject *const *a, Py_ssize_t) {
@@ -453,15 +452,14 @@ PyObject *stream_order(PyObject *const *a, Py_ssize_t) {
   return Ref(PyTuple_Pack(4, o.o, p.o, k.o, w.o)).release();
 }
 
-// Unit descriptors, slot tables, sizes [n][4] and dimensions [n][5] of the entries, into the arrays given; None if an
-// entry keeps nothing.  Counts rows, info rows, first query rows, heads, G, units, slots, sizes, dimensions
+// Unit descriptors, sizes [n][4] and dimensions [n][5] of the entries, into the arrays given; None if an
+// entry keeps nothing.  Counts rows, info rows, first query rows, heads, G, units, sizes, dimensions
 PyObject *stream_tables(PyObject *const *a, Py_ssize_t) {
   plain(PyList_Check(a[0]) && PyList_Check(a[1]) && PyList_Check(a[2]));
   const int64_t n = PyList_GET_SIZE(a[2]), H = integer(a[3]), G = integer(a[4]);
   plain(n >= 1 && H >= 1 && PyList_GET_SIZE(a[0]) == n * H && PyList_GET_SIZE(a[1]) == n * H);
-  Buffer units(a[5], true), slots(a[6], true), sizes(a[7], true), dims(a[8], true);
+  Buffer units(a[5], true), sizes(a[6], true), dims(a[7], true);
   auto *unit_p = units.of<RdkvUnit>(n * H);
-  auto *slot_p = slots.of<int16_t>(n * H * kSlots);
   auto *size_p = sizes.of<int64_t>(4 * n);
   auto *dim_p = dims.of<int32_t>(5 * n);
   std::vector<int32_t> tok(4 * H), ch(3 * H);
@@ -482,26 +480,24 @@ PyObject *stream_tables(PyObject *const *a, Py_ssize_t) {
     int32_t *d = dim_p + 5 * e;
     d[0] = (m[0] + 3) / 4 * 4, d[1] = (m[1] + 1) / 2 * 2, d[2] = m[2], d[3] = max_tv, d[4] = max_n16;
     status(lib.rdkv_stream_plan_layer(tok.data(), 4, ch.data(), 3, H, d[0], d[1], (int)integer(PyList_GET_ITEM(a[2], e)), G,
-                                      unit_p + e * H, slot_p + e * H * kSlots, kSlots, size_p + 4 * e));
+                                      unit_p + e * H, nullptr, 0, size_p + 4 * e));
   }
   Py_RETURN_TRUE;
 }
 
 // The entries' blobs, packed; the units' offsets become addresses.  K, V, order, plan, K widths, min / max, units
-// (host), units, slots (device), sizes, dimensions, largest scales [n][2][H], stream
+// (host), sizes, dimensions, largest scales [n][2][H], stream
 PyObject *stream_pack(PyObject *const *a, Py_ssize_t) {
   const std::vector<at::Tensor> Ks = tensors(a[0]), Vs = tensors(a[1]);
-  const at::Tensor &order = tensor(a[2]), &plan = tensor(a[3]), &kb = tensor(a[4]), &mm = tensor(a[5]), &units = tensor(a[7]),
-                   &slots = tensor(a[8]), &scales = tensor(a[11]);
-  void *stream = address(a[12]);
+  const at::Tensor &order = tensor(a[2]), &plan = tensor(a[3]), &kb = tensor(a[4]), &mm = tensor(a[5]), &scales = tensor(a[9]);
+  void *stream = address(a[10]);
   const int64_t n = Ks.size(), H = Ks[0].size(1), T = Ks[0].size(2);
-  Buffer host(a[6], true), sizes(a[9]), dims(a[10]);
+  Buffer host(a[6], true), sizes(a[7]), dims(a[8]);
   auto *unit_p = host.of<RdkvUnit>(n * H);
   const auto *size_p = sizes.of<int64_t>(4 * n);
   const auto *dim_p = dims.of<int32_t>(5 * n);
   plain(shape_is(order, {n * H, T}) && shape_is(scales, {n, 2, H}) && shape_is(kb, {n * H, 128}) && kb.is_contiguous());
-  plain(units.numel() >= n * H * (int64_t)sizeof(RdkvUnit) && slots.numel() >= n * H * kSlots * 2);
-  plain(mm.numel() >= n * H * 768);
+  plain(mm.numel() >= n * H * 768 && plan.numel() >= 12 * n * H);
   std::vector<at::Tensor> blobs;
   std::vector<RdkvStreamLayer> layers;
   int rc = RDKV_OK;
@@ -515,9 +511,10 @@ PyObject *stream_pack(PyObject *const *a, Py_ssize_t) {
       layers.push_back({Ks[e].data_ptr(), Vs[e].data_ptr(), Ks[e].stride(1), Ks[e].stride(2), data<uint8_t>(blobs.back()), bytes,
                         d[3], d[0], d[1], d[2], d[4], (int32_t)size_p[4 * e + 1], 0});
     }
-    rc = lib.rdkv_pack_layers_stream(layers.data(), n, H, data<int32_t>(order), T, data<int32_t>(plan), data<uint8_t>(kb),
-                                     kb.element_size(), 128, data<RdkvUnit>(units), data<int16_t>(slots), kSlots, data<float>(mm),
-                                     data<float>(scales), stream);
+    const at::Tensor units = at::empty({n * H * (int64_t)sizeof(RdkvUnit)}, kb.options().dtype(at::kByte));
+    rc = lib.rdkv_pack_layers_stream(layers.data(), n, H, data<int32_t>(order), T, data<int32_t>(plan),
+                                     data<int32_t>(plan) + 4 * n * H, data<uint8_t>(kb), kb.element_size(), 128,
+                                     data<RdkvUnit>(units), data<float>(mm), data<float>(scales), stream);
     for (int64_t e = 0; e < n && rc == RDKV_OK; ++e) {
       const uint64_t base = reinterpret_cast<uintptr_t>(layers[e].blob);
       for (RdkvUnit *p = unit_p + e * H; p < unit_p + (e + 1) * H; ++p) {
@@ -755,8 +752,8 @@ PyMethodDef kMethods[] = {
     ENTRY(pack_layer, 13, "The tensors of a planned layer: (fields of the layer, fp16-kept V rows), or None."),
     ENTRY(select_layer, 19, "Widths and token order of a layer: (v_bits, k_bits, order, rank3, plan, min / max, int16 widths), or None."),
     ENTRY(stream_order, 7, "Token order of the layers: (order, plan, K widths, min / max), or None."),
-    ENTRY(stream_tables, 9, "Fills the units, slot tables, sizes and dimensions of the layers: True, or None."),
-    ENTRY(stream_pack, 13, "The blobs of the layers, or None."),
+    ENTRY(stream_tables, 8, "Fills the units, sizes and dimensions of the layers: True, or None."),
+    ENTRY(stream_pack, 11, "The blobs of the layers, or None."),
     ENTRY(decode_attn, 16, "(out, lse) of a decode step, or None."),
     ENTRY(dense_layer, 7, "Dense (K, V) of a packed layer, with its additive mask where one is given; or None."),
     {nullptr, nullptr, 0, nullptr}};

@@ -38,6 +38,71 @@ __device__ __forceinline__ int load_bits(const void *p, int elem_size, int64_t i
   }
 }
 
+// The K row of a head with c2 / c4 / c8 channels at 2 / 4 / 8 bit.  Slot order: 8-bit channels, 4-bit, 2-bit, each
+// padded to whole dwords (4 / 8 / 16 channels).  A narrow code is the same number in a wider field, so the stragglers
+// of a narrow class move into the pad slots of the wider ones when that saves a whole dword of the row; a row still
+// longer than 32 dwords is stored entirely as 8 bit.
+struct RowPlan {
+  int c4, c8;
+  int m4, t8, t4;         // stragglers: 4-bit channels among the 8-bit slots, 2-bit ones among the 8- and 4-bit slots
+  int n8, n4, n2;         // channels in the slots of a class
+  int all8;               // 4- and 2-bit slots' channels follow the 8-bit ones
+  int d8, d4, d2;
+  __host__ __device__ static int pad_to(int n, int a) { return (a - n % a) % a; }
+  __host__ __device__ RowPlan(int c2, int c4_, int c8_) : c4(c4_), c8(c8_), m4(0), t8(0), t4(0), all8(0) {
+    const int r4 = c4 % 8;
+    if (r4 > 0 && r4 <= pad_to(c8, 4)) m4 = r4;
+    n8 = c8 + m4;
+    n4 = c4 - m4;
+    const int r2 = c2 % 16, p8 = pad_to(n8, 4), p4 = pad_to(n4, 8);
+    if (r2 > 0 && r2 <= p8 + p4) {
+      t8 = r2 < p8 ? r2 : p8;
+      t4 = r2 - t8;
+    }
+    n8 += t8;
+    n4 += t4;
+    n2 = c2 - t8 - t4;
+    all8 = (n8 + 3) / 4 + (n4 + 7) / 8 + (n2 + 15) / 16 > 32;
+    d8 = ((all8 ? n8 + n4 + n2 : n8) + 3) / 4;
+    d4 = all8 ? 0 : (n4 + 7) / 8;
+    d2 = all8 ? 0 : (n2 + 15) / 16;
+  }
+  __host__ __device__ int slots() const { return 4 * (d8 + 2 * d4 + 4 * d2); }
+  // what slot i holds: the position in the layer's padded sorted channel order, or -1
+  __host__ __device__ int source(int i, int n2p, int n4p) const {
+    int in8 = i, in4 = i - 4 * d8, in2 = in4 - 8 * d4;
+    if (all8) in4 = i - n8, in2 = in4 - n4;
+    if (in8 < (all8 ? n8 : 4 * d8))
+      return in8 < c8 ? n2p + n4p + in8 : in8 < c8 + m4 ? n2p + c4 - m4 + in8 - c8 : in8 < n8 ? n2 + in8 - c8 - m4 : -1;
+    if (in4 < (all8 ? n4 : 8 * d4)) return in4 < c4 - m4 ? n2p + in4 : in4 < n4 ? n2 + t8 + in4 - (c4 - m4) : -1;
+    return in2 < n2 ? in2 : -1;
+  }
+};
+__host__ __device__ inline int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
+// A unit's sections from `off` on (a multiple of 256); returns where they end.
+__host__ __device__ inline int64_t lay_out_unit(const RowPlan &r, const int32_t *n_tok, int64_t off, RdkvUnit &u) {
+  int64_t tiles[4], n_q_tiles = 0, n_tiles = 0;
+  for (int c = 0; c < 4; ++c) {
+    tiles[c] = ((int64_t)n_tok[c] + RDKV_TILE - 1) / RDKV_TILE;
+    n_tiles += tiles[c];
+    if (c < 3) n_q_tiles += tiles[c];
+    u.n_tok[c] = n_tok[c];
+  }
+  u.d8 = r.d8;
+  u.d4 = r.d4;
+  u.d2 = r.d2;
+  u.k_off = (uint64_t)off;
+  off = align256(off + n_tiles * RDKV_TILE * 4 * (r.d8 + r.d4 + r.d2));
+  for (int c = 0; c < 4; ++c) {
+    u.v_off[c] = (uint64_t)off;
+    off = align256(off + tiles[c] * rdkv_v_tile_bytes(c));
+  }
+  u.sz_off = (uint64_t)off;
+  off = align256(off + n_q_tiles * RDKV_TILE * 4);
+  u.qtab_off = (uint64_t)off;
+  return align256(off + (int64_t)r.slots() * (int64_t)sizeof(RdkvSlot));
+}
+
 struct StreamPackArgs {
   const __half *K, *V;
   int64_t stride_h, stride_t;
@@ -50,7 +115,8 @@ struct StreamPackArgs {
   int64_t max_tv;
   int max_n16;
   uint32_t *mm;                   // per head: 128 minima, 128 maxima (order-preserving integers)
-  const RdkvUnit *units;          // offsets relative to `blob`
+  RdkvUnit *units;                // offsets relative to `blob`; written by the first launch where src_slot is null,
+  const int32_t *counts, *info;   // ... from the plan's numbers
   const int16_t *src_slot;
   int n_slots_max, max_tiles;
   uint8_t *blob;
@@ -77,7 +143,7 @@ __device__ __forceinline__ float4 make_chan(float scale, float zp, float inv, in
 }
 
 // One workgroup per head: stream slot -> position in the reference's padded sorted channel order
-// (src_slot) -> width class and rank in the class -> the rank-th channel of that width in ascending
+// (src_slot, or RowPlan where the unit is planned here) -> width class and rank in the class -> the rank-th channel of that width in ascending
 // channel order (the stable sort of packing.py:241-294) -> the channel's parameters from its
 // min / max.  Writes the per-channel parameters, the unit's slot table in the blob (with the
 // alignment gap behind it, and behind the last head the rest of the blob: no byte of the blob is
@@ -90,7 +156,26 @@ slot_params_kernel(StreamPackBatch batch) {
   __shared__ float4 slot_p[kMaxSlots];
   __shared__ float wave_max[2];
   const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
-  const RdkvUnit u = a.units[h];
+  // the head's unit: given, or planned here as the host plans it (the heads ahead of it only for where it begins)
+  const bool planned = a.src_slot == nullptr;
+  const RowPlan row(planned ? a.info[8 * h + 2] : 0, planned ? a.info[8 * h + 3] : 0, planned ? a.info[8 * h + 4] : 0);
+  RdkvUnit u;
+  if (planned) {
+    __shared__ int64_t ahead[2];
+    int64_t off = 0;
+    for (int i = tid; i < h; i += 128) {
+      RdkvUnit other;
+      off += lay_out_unit(RowPlan(a.info[8 * i + 2], a.info[8 * i + 3], a.info[8 * i + 4]), a.counts + 4 * i, 0, other);
+    }
+    for (int o = 1; o < 64; o <<= 1) off += __shfl_xor((long long)off, o, 64);
+    if (lane == 0) ahead[tid >> 6] = off;
+    __syncthreads();
+    lay_out_unit(row, a.counts + 4 * h, ahead[0] + ahead[1], u);
+    u.q_row = u.work_begin = u.work_count = 0;      // (the packer's launches do not look at them)
+    if (tid == 0) a.units[h] = u;
+  } else {
+    u = a.units[h];
+  }
   const int n_slots = 4 * (u.d8 + 2 * u.d4 + 4 * u.d2);
   // rank of channel c inside its width class = channels below it of the same class: a ballot per
   // class in each of the two wavefronts that hold the 128 channels, plus the first wavefront's count
@@ -113,7 +198,7 @@ slot_params_kernel(StreamPackBatch batch) {
   const int16_t *slots = a.src_slot + (int64_t)h * a.n_slots_max;
   float smax = 0.0f;
   for (int i = tid; i < n_slots; i += 128) {
-    const int r = slots[i];
+    const int r = planned ? row.source(i, a.n2p, a.n4p) : slots[i];
     uint32_t w0 = 0, w1 = 0;
     if (r >= 0) {
       int c, rk;
@@ -570,14 +655,15 @@ static int launch_stream_pack(const StreamPackBatch &batch, int n_layers, int H_
 static int fill_stream_args(const char *fn, StreamPackArgs *a, const void *K_f16, const void *V_f16, int64_t stride_h,
                             int64_t stride_t, int H_kv, const int32_t *order, int64_t order_stride_h, const int32_t *counts,
                             const void *k_bits, int kb_elem_size, int64_t kb_stride_h, int n2p, int n4p, int n8,
-                            int64_t max_tv, int max_n16, const RdkvUnit *units, const int16_t *src_slot, int n_slots_max,
-                            int max_tiles, uint8_t *blob, int64_t blob_bytes, float *minmax_ws, float *scale_max) {
+                            int64_t max_tv, int max_n16, RdkvUnit *units, const int32_t *info, const int16_t *src_slot,
+                            int n_slots_max, int max_tiles, uint8_t *blob, int64_t blob_bytes, float *minmax_ws,
+                            float *scale_max) {
   // (minmax_ws holds the min / max accumulators, H_kv * 256 floats, then the channel parameters,
   // H_kv * 128 * 4 floats)
   RDKV_REQUIRE(H_kv >= 1 && H_kv <= 65535 && max_tiles >= 0 && max_tv >= 0 && max_n16 >= 0 && blob_bytes >= 0 &&
                    blob_bytes % 4 == 0,
                "%s: bad shape", fn);
-  RDKV_REQUIRE(K_f16 && V_f16 && order && counts && k_bits && units && src_slot && blob && minmax_ws && scale_max,
+  RDKV_REQUIRE(K_f16 && V_f16 && order && counts && k_bits && units && (src_slot || info) && blob && minmax_ws && scale_max,
                "%s: null pointer", fn);
   RDKV_REQUIRE(kb_elem_size == 1 || kb_elem_size == 2 || kb_elem_size == 4 || kb_elem_size == 8,
                "%s: element size of k_bits must be 1, 2, 4 or 8", fn);
@@ -596,7 +682,7 @@ static int fill_stream_args(const char *fn, StreamPackArgs *a, const void *K_f16
   a->n2p = n2p; a->n4p = n4p;
   a->max_tv = max_tv; a->max_n16 = max_n16;
   a->mm = reinterpret_cast<uint32_t *>(minmax_ws);
-  a->units = units; a->src_slot = src_slot; a->n_slots_max = n_slots_max; a->max_tiles = max_tiles;
+  a->units = units; a->counts = counts; a->info = info; a->src_slot = src_slot; a->n_slots_max = n_slots_max; a->max_tiles = max_tiles;
   a->blob = blob;
   a->scale_max = reinterpret_cast<uint32_t *>(scale_max);
   a->H_kv = H_kv;
@@ -614,8 +700,8 @@ RDKV_API int rdkv_pack_layer_stream(const void *K_f16, const void *V_f16, int64_
   const char *fn = "rdkv_pack_layer_stream";
   StreamPackBatch batch;
   const int rc = fill_stream_args(fn, &batch.layer[0], K_f16, V_f16, stride_h, stride_t, H_kv, order, order_stride_h, counts,
-                                  k_bits, kb_elem_size, kb_stride_h, n2p, n4p, n8, max_tv, max_n16, units, src_slot,
-                                  n_slots_max, max_tiles, blob, blob_bytes, minmax_ws, scale_max);
+                                  k_bits, kb_elem_size, kb_stride_h, n2p, n4p, n8, max_tv, max_n16,
+                                  const_cast<RdkvUnit *>(units), nullptr, src_slot, n_slots_max, max_tiles, blob, blob_bytes, minmax_ws, scale_max);
   if (rc != RDKV_OK) return rc;
   hipStream_t s = (hipStream_t)stream;
   // per-channel min / max of every head's kept rows (the K canvas without its zero rows)
@@ -632,9 +718,8 @@ RDKV_API int rdkv_pack_layer_stream(const void *K_f16, const void *V_f16, int64_
 // Layers packed one by one leave the device between them what a launch's first and last tiles take, and the slot
 // parameters 4.5 us each: four layers of 8 x 32k tokens 223 us of launches, together 164.
 RDKV_API int rdkv_pack_layers_stream(const RdkvStreamLayer *layers, int n_layers, int H_kv, const int32_t *order,
-                                     int64_t order_stride_h, const int32_t *counts, const void *k_bits, int kb_elem_size,
-                                     int64_t kb_stride_h, const RdkvUnit *units, const int16_t *src_slot, int n_slots_max,
-                                     float *minmax_ws, float *scale_max, void *stream) {
+                                     int64_t order_stride_h, const int32_t *counts, const int32_t *info, const void *k_bits,
+                                     int kb_elem_size, int64_t kb_stride_h, RdkvUnit *units, float *minmax_ws, float *scale_max, void *stream) {
   const char *fn = "rdkv_pack_layers_stream";
   RDKV_REQUIRE(n_layers >= 0 && (n_layers == 0 || layers), "%s: bad arguments", fn);
   for (int pass = 0; pass < 2; ++pass) {          // (every layer's arguments are looked at before the first launch)
@@ -649,7 +734,7 @@ RDKV_API int rdkv_pack_layers_stream(const RdkvStreamLayer *layers, int n_layers
                                         counts ? counts + 4 * row : nullptr,
                                         k_bits ? (const uint8_t *)k_bits + row * kb_stride_h * kb_elem_size : nullptr, kb_elem_size,
                                         kb_stride_h, y.n2p, y.n4p, y.n8, y.max_tv, y.max_n16, units ? units + row : nullptr,
-                                        src_slot ? src_slot + row * n_slots_max : nullptr, n_slots_max, y.max_tiles, y.blob,
+                                        info ? info + 8 * row : nullptr, nullptr, kMaxSlots, y.max_tiles, y.blob,
                                         y.blob_bytes, minmax_ws ? minmax_ws + row * 768 : nullptr,
                                         scale_max ? scale_max + 2 * row : nullptr);
         if (rc != RDKV_OK) return rc;
@@ -662,23 +747,13 @@ RDKV_API int rdkv_pack_layers_stream(const RdkvStreamLayer *layers, int n_layers
 }
 
 // Host side of the streaming format (no GPU work): the unit descriptors of one layer's heads.
-namespace {
-struct SlotList {
-  int16_t v[kMaxSlots + 3 * kD];
-  int n = 0;
-  void push(int x) { v[n++] = (int16_t)x; }
-};
-inline int pad_to(int n, int a) { return (a - n % a) % a; }
-inline int64_t align256(int64_t x) { return (x + 255) / 256 * 256; }
-}  // namespace
-
 RDKV_API int rdkv_stream_plan_layer(const int32_t *tok_counts, int64_t tok_stride, const int32_t *ch_counts,
                                     int64_t ch_stride, int H_kv, int n2p, int n4p, int first_q_row, int G,
                                     RdkvUnit *units, int16_t *src_slot, int n_slots_max, int64_t *sizes) {
   const char *fn = "rdkv_stream_plan_layer";
-  RDKV_REQUIRE(tok_counts && ch_counts && units && src_slot && sizes, "%s: null pointer", fn);
+  RDKV_REQUIRE(tok_counts && ch_counts && units && sizes, "%s: null pointer", fn);
   RDKV_REQUIRE(H_kv >= 1 && G >= 1 && n2p >= 0 && n4p >= 0 && n2p % 4 == 0 && n4p % 2 == 0, "%s: bad shape", fn);
-  RDKV_REQUIRE(n_slots_max == kMaxSlots, "%s: n_slots_max must be %d", fn, kMaxSlots);
+  RDKV_REQUIRE(!src_slot || n_slots_max == kMaxSlots, "%s: n_slots_max must be %d", fn, kMaxSlots);
   int64_t off = 0, stream_bytes = 0, algo_bytes = 0;
   int max_tiles = 0;
   for (int h = 0; h < H_kv; ++h) {
@@ -687,72 +762,27 @@ RDKV_API int rdkv_stream_plan_layer(const int32_t *tok_counts, int64_t tok_strid
     RDKV_REQUIRE(c2 >= 0 && c4 >= 0 && c8 >= 0 && c2 <= n2p && c4 <= n4p && c2 + c4 + c8 <= kD &&
                      nt[0] >= 0 && nt[1] >= 0 && nt[2] >= 0 && nt[3] >= 0,
                  "%s: bad counts of head %d", fn, h);
-    // Slot order: 8-bit channels, 4-bit, 2-bit, each padded to whole dwords (4 / 8 / 16 channels).
-    // A narrow code is the same number in a wider field, so the stragglers of a narrow class move
-    // into the pad slots of the wider ones when that saves a whole dword of the K row; a row still
-    // longer than RDKV_MAX_ROW_DWORDS is stored entirely as 8 bit.
-    SlotList l8, l4, l2;
-    for (int i = 0; i < c8; ++i) l8.push(n2p + n4p + i);
-    for (int i = 0; i < c4; ++i) l4.push(n2p + i);
-    for (int i = 0; i < c2; ++i) l2.push(i);
-    const int r4 = l4.n % 8;
-    if (r4 > 0 && r4 <= pad_to(l8.n, 4)) {
-      for (int i = l4.n - r4; i < l4.n; ++i) l8.push(l4.v[i]);
-      l4.n -= r4;
-    }
-    const int r2 = l2.n % 16, p8 = pad_to(l8.n, 4), p4 = pad_to(l4.n, 8);
-    if (r2 > 0 && r2 <= p8 + p4) {
-      const int first = l2.n - r2, to8 = r2 < p8 ? r2 : p8;
-      for (int i = 0; i < to8; ++i) l8.push(l2.v[first + i]);
-      for (int i = to8; i < r2; ++i) l4.push(l2.v[first + i]);
-      l2.n = first;
-    }
-    if ((l8.n + 3) / 4 + (l4.n + 7) / 8 + (l2.n + 15) / 16 > 32) {
-      for (int i = 0; i < l4.n; ++i) l8.push(l4.v[i]);
-      for (int i = 0; i < l2.n; ++i) l8.push(l2.v[i]);
-      l4.n = l2.n = 0;
-    }
-    const int d8 = (l8.n + 3) / 4, d4 = (l4.n + 7) / 8, d2 = (l2.n + 15) / 16;
-    const int steps = d8 + 2 * d4 + 4 * d2;
-    RDKV_REQUIRE(steps <= RDKV_MAX_STEPS, "%s: %d channel steps exceed %d", fn, steps, RDKV_MAX_STEPS);
-    int16_t *src = src_slot + (int64_t)h * n_slots_max;
-    int n = 0;
-    for (int i = 0; i < l8.n; ++i) src[n++] = l8.v[i];
-    while (n < 4 * d8) src[n++] = -1;
-    for (int i = 0; i < l4.n; ++i) src[n++] = l4.v[i];
-    while (n < 4 * d8 + 8 * d4) src[n++] = -1;
-    for (int i = 0; i < l2.n; ++i) src[n++] = l2.v[i];
-    while (n < n_slots_max) src[n++] = -1;
-    const int n_slots = 4 * steps;
-    const int64_t qt_bytes = (int64_t)n_slots * (int64_t)sizeof(RdkvSlot);
-    int64_t tiles[4], n_tiles = 0, n_q_tiles = 0;
+    const RowPlan row_plan(c2, c4, c8);
+    const int n_slots = row_plan.slots(), R = row_plan.d8 + row_plan.d4 + row_plan.d2;
+    RDKV_REQUIRE(n_slots <= kMaxSlots, "%s: %d channel steps exceed %d", fn, n_slots / 4, RDKV_MAX_STEPS);
+    if (src_slot)
+      for (int i = 0; i < n_slots_max; ++i)
+        src_slot[(int64_t)h * n_slots_max + i] = i < n_slots ? (int16_t)row_plan.source(i, n2p, n4p) : (int16_t)-1;
+    int64_t n_tiles = 0, n_q_tiles = 0, v_bytes = 0;
     for (int c = 0; c < 4; ++c) {
-      tiles[c] = ((int64_t)nt[c] + RDKV_TILE - 1) / RDKV_TILE;
-      n_tiles += tiles[c];
-      if (c < 3) n_q_tiles += tiles[c];
+      const int64_t tiles = ((int64_t)nt[c] + RDKV_TILE - 1) / RDKV_TILE;
+      n_tiles += tiles;
+      if (c < 3) n_q_tiles += tiles;
+      v_bytes += tiles * rdkv_v_tile_bytes(c);
     }
     RDKV_REQUIRE(n_tiles <= 0x7fffffff, "%s: too many tiles", fn);
     if (n_tiles > max_tiles) max_tiles = (int)n_tiles;
-    const int R = d8 + d4 + d2;
     RdkvUnit u;
     memset(&u, 0, sizeof(u));
-    u.k_off = (uint64_t)off;
-    off = align256(off + n_tiles * RDKV_TILE * 4 * R);
-    int64_t v_bytes = 0;
-    for (int c = 0; c < 4; ++c) {
-      u.v_off[c] = (uint64_t)off;
-      off = align256(off + tiles[c] * rdkv_v_tile_bytes(c));
-      v_bytes += tiles[c] * rdkv_v_tile_bytes(c);
-    }
-    u.sz_off = (uint64_t)off;
-    off = align256(off + n_q_tiles * RDKV_TILE * 4);
-    u.qtab_off = (uint64_t)off;
-    off = align256(off + qt_bytes);
-    for (int c = 0; c < 4; ++c) u.n_tok[c] = nt[c];
-    u.d8 = d8; u.d4 = d4; u.d2 = d2;
+    off = lay_out_unit(row_plan, nt, off, u);
     u.q_row = first_q_row + h * G;
     units[h] = u;
-    stream_bytes += n_tiles * RDKV_TILE * 4 * R + v_bytes + n_q_tiles * RDKV_TILE * 4 + qt_bytes;
+    stream_bytes += n_tiles * RDKV_TILE * 4 * R + v_bytes + n_q_tiles * RDKV_TILE * 4 + (int64_t)n_slots * (int64_t)sizeof(RdkvSlot);
     // the reference's own bytes for the same content: packed K rows and channel parameters, packed
     // V rows, per-token parameters, fp16-kept rows
     const int64_t row = (c2 + 3) / 4 + (c4 + 1) / 2 + c8;

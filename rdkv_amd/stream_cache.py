@@ -430,15 +430,13 @@ def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, s
         return None
     order, plan, kb, mm = planned
     units = np.zeros(n * H_kv, dtype=UNIT_DTYPE)
-    slots = np.empty((n * H_kv, 4 * MAX_STEPS), dtype=np.int16)
     sizes, dims = np.zeros((n, 4), dtype=np.int64), np.empty((n, 5), dtype=np.int32)
     scales = torch.empty(n, 2, H_kv, dtype=torch.float32, device=dev)
     counts, info = packing._plan_rows(words.read(dev))
-    if _lib.native.stream_tables(counts, info, [int(r) * H_kv * G for r in rows_of_entries], H_kv, G, units, slots, sizes,
+    if _lib.native.stream_tables(counts, info, [int(r) * H_kv * G for r in rows_of_entries], H_kv, G, units, sizes,
                                  dims) is None:
         return None
-    units_dev, slots_dev = _lib.upload(dev, units, slots)
-    blobs = _lib.native.stream_pack(Ks, Vs, order, plan, kb, mm, units, units_dev, slots_dev, sizes, dims, scales, stream)
+    blobs = _lib.native.stream_pack(Ks, Vs, order, plan, kb, mm, units, sizes, dims, scales, stream)
     assert blobs is not None
     return units, blobs, sizes.tolist(), scales
 
