@@ -473,11 +473,12 @@ int rdkv_stream_partition_units(RdkvUnit *units, int n_units, int n_items, const
  * at most 40. */
 int rdkv_stream_work_scales(RdkvWork *work, int n_work, const float *scale_max, int n_units);
 
-/* The same for work items on the device, from scales that earlier launches of the stream leave there as
- * rdkv_pack_layers_stream does ([n_units / H_kv][2][H_kv], units in that order; every item's unit in 0 .. n_units);
- * host_words [2 * n_units] receive them as float bits, unit by unit (rdkv_host_words_wait). */
-int rdkv_stream_work_scales_device(RdkvWork *work, int n_work, const float *scales, int H_kv, int n_units,
-                                   uint64_t *host_words, uint32_t tag, void *stream);
+/* A cache's tables (bytes, a multiple of 16) from host memory that the device can read to dst on the device, with the
+ * scale fields of the n_work items (RdkvWork, from byte work_at on, a multiple of 128) filled as
+ * rdkv_stream_work_scales fills them, from scales on the device: [n_units / H_kv][2][H_kv] (rdkv_pack_layers_stream), the
+ * items' units in that order.  host_words [2 * n_units]: unit u's two scales as float bits (rdkv_host_words_wait). */
+int rdkv_stream_tables_device(const void *src, void *dst, int64_t bytes, int64_t work_at, int n_work, const float *scales,
+                              int H_kv, int n_units, uint64_t *host_words, uint32_t tag, void *stream);
 
 /* Re-lay one layer (H_kv units) from the reference's padded tensors into the blob.
  * src_slot: int16 [H_kv][n_slots_max] = for each stream slot the index of the source channel

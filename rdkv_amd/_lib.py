@@ -81,7 +81,7 @@ SIGNATURES = {
     "rdkv_stream_partition": (I, [P, I, I, P, ctypes.c_double, ctypes.c_double, P, I, I, P, I, P, P]),
     "rdkv_stream_partition_units": (I, [P, I, I, P, ctypes.c_double, I, P, I, P, P]),
     "rdkv_stream_work_scales": (I, [P, I, P, I]),
-    "rdkv_stream_work_scales_device": (I, [P, I, P, I, I, P, ctypes.c_uint32, P]),
+    "rdkv_stream_tables_device": (I, [P, P, L, L, I, P, I, I, P, ctypes.c_uint32, P]),
     "rdkv_pack_layers_stream": (I, [P, I, I, P, L, P, P, P, I, L, P, P, P, P]),
     "rdkv_pack_layer_stream_ws_init": (I, [P, I, P]),
     "rdkv_pack_layer_stream": (I, [P, P, L, L, I, P, L, P, P, I, L, I, I, I, L, I, P, P, I, I, P, L, P, I, P, P]),
@@ -271,9 +271,10 @@ def stream_workspace(dev: torch.device):
 _stagers: dict = {}
 
 
-def upload(dev: torch.device, *arrays) -> list:
+def upload(dev: torch.device, *arrays, copy=None) -> list:
     """The NumPy arrays as byte tensors on ``dev`` (views of one device buffer, each 256-byte
-    aligned), sent as one queued copy on the current stream."""
+    aligned), sent as one queued copy on the current stream, or by the launch that ``copy(to, from, bytes, where each
+    array begins)`` makes there."""
     import threading
 
     import numpy as np
@@ -297,7 +298,10 @@ def upload(dev: torch.device, *arrays) -> list:
         if a.nbytes:
             host[o:o + a.nbytes] = np.ascontiguousarray(a).reshape(-1).view(np.uint8)
     d = torch.empty(total, dtype=torch.uint8, device=dev)
-    d.copy_(slot[0][:total], non_blocking=True)
+    if copy is None:
+        d.copy_(slot[0][:total], non_blocking=True)
+    else:
+        copy(d.data_ptr(), slot[0].data_ptr(), total, offs)
     ev = torch.cuda.Event()
     ev.record(torch.cuda.current_stream(dev))
     slot[1] = ev

@@ -18,6 +18,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cstddef>
 #include <vector>
 
 #include "stream_format.h"
@@ -588,33 +589,45 @@ __device__ __forceinline__ int v_shift_of(float v) {
   return min(max(min(ex, 41) - 9, 0), 40);
 }
 
-// What rdkv_stream_work_scales does on the host, for scales that launches before this one leave on the device, and the
-// scales themselves to the host: with a copy, a wait for it and the items' upload behind it, a build's last 70 us were
-// the host's alone.
+// A cache's tables from the host memory they were written to (`src`, which the device reads itself) to where they stay,
+// the work items among them (from byte `work_at` on) with the scales that launches before this one have left on the
+// device, as rdkv_stream_work_scales fills them, and the scales to the host.  A copy queued behind the packer began
+// 15 us after its end and this launch behind the copy; with a copy back, a wait for it and the upload behind it, a
+// build's last 70 us were the host's alone.
 __global__ void __launch_bounds__(256)
-work_scales_kernel(RdkvWork *work, int n_work, const float *__restrict__ scales, int H_kv, int n_units, uint64_t *words, uint32_t tag) {
+stream_tables_kernel(const uint4 *src, uint4 *dst, int pieces, int work_at, int n_work, const float *__restrict__ scales, int H_kv,
+                     int n_units, uint64_t *words, uint32_t tag) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   auto scale = [&](int u, int which) { return scales[(int64_t)(u / H_kv) * 2 * H_kv + which * H_kv + u % H_kv]; };
-  if (i < n_work) {
-    const int u = work[i].unit;
-    work[i].k_scale_max = scale(u, 0);
-    work[i].v_shift = v_shift_of(scale(u, 1));
+  uint4 v = i < pieces ? src[i] : make_uint4(0u, 0u, 0u, 0u);
+  // (an item is eight pieces, its unit the first word of the first, the scale fields the last words of the last)
+  static_assert(sizeof(RdkvWork) == 128 && offsetof(RdkvWork, unit) == 0 && offsetof(RdkvWork, k_scale_max) == 120 &&
+                    offsetof(RdkvWork, v_shift) == 124, "an item's layout");
+  const int unit = __shfl((int)v.x, (threadIdx.x & 63) & ~7);
+  const int at = i - work_at;
+  if (at >= 0 && at < 8 * n_work && (at & 7) == 7) {
+    v.z = __float_as_uint(scale(unit, 0));
+    v.w = (uint32_t)v_shift_of(scale(unit, 1));
   }
+  if (i < pieces) dst[i] = v;
   if (i < 2 * n_units) rdkv_host_word(words, i, tag, __float_as_int(scale(i >> 1, i & 1)));
 }
 
 }  // namespace
 
-// scales: [n_units / H_kv][2][H_kv] on the device (rdkv_pack_layers_stream), the work items' units in that order; words
-// [2 * n_units]: unit u's two scales as float bits.
-RDKV_API int rdkv_stream_work_scales_device(RdkvWork *work, int n_work, const float *scales, int H_kv, int n_units,
-                                            uint64_t *host_words, uint32_t tag, void *stream) {
-  const char *fn = "rdkv_stream_work_scales_device";
-  RDKV_REQUIRE(n_work >= 0 && n_units >= 1 && n_units <= (1 << 28) && H_kv >= 1 && n_units % H_kv == 0 && scales && host_words &&
-                   (n_work == 0 || work), "%s: bad arguments", fn);
-  const int n = std::max(n_work, 2 * n_units);
-  hipLaunchKernelGGL(work_scales_kernel, dim3((unsigned)rdkv_cdiv(n, 256)), dim3(256), 0, (hipStream_t)stream, work, n_work, scales,
-                     H_kv, n_units, host_words, tag);
+RDKV_API int rdkv_stream_tables_device(const void *src, void *dst, int64_t bytes, int64_t work_at, int n_work, const float *scales,
+                                       int H_kv, int n_units, uint64_t *host_words, uint32_t tag, void *stream) {
+  const char *fn = "rdkv_stream_tables_device";
+  RDKV_REQUIRE(bytes >= 0 && bytes % 16 == 0 && bytes < (1LL << 34) && (bytes == 0 || (src && dst)) &&
+                   (((uintptr_t)src | (uintptr_t)dst) % 16) == 0, "%s: bad tables", fn);
+  // (whole items in whole groups of eight lanes)
+  RDKV_REQUIRE(n_work >= 0 && work_at >= 0 && work_at % 128 == 0 && work_at + n_work * (int64_t)sizeof(RdkvWork) <= bytes,
+               "%s: work items outside the tables", fn);
+  RDKV_REQUIRE(n_units >= 1 && n_units <= (1 << 28) && H_kv >= 1 && n_units % H_kv == 0 && scales && host_words,
+               "%s: bad arguments", fn);
+  const int64_t n = std::max<int64_t>(bytes / 16, 2 * (int64_t)n_units);
+  hipLaunchKernelGGL(stream_tables_kernel, dim3((unsigned)rdkv_cdiv(n, 256)), dim3(256), 0, (hipStream_t)stream, (const uint4 *)src,
+                     (uint4 *)dst, (int)(bytes / 16), (int)(work_at / 16), n_work, scales, H_kv, n_units, host_words, tag);
   RDKV_CHECK_LAUNCH(fn);
   return RDKV_OK;
 }

@@ -765,16 +765,19 @@ def _finish_caches(specs) -> List[StreamCache]:
     n_tickets = [max(1, len(pl[0])) for pl in plans]
     ticket_at = np.concatenate([[0], np.cumsum(n_tickets)])
     on_device = specs[0][6] if len(specs) == 1 and isinstance(specs[0][6], _DeviceScales) and plans[0][3] is None else None
-    tables = _lib.upload(dev, *[a for pl in plans for a in (pl[0], pl[2] if pl[2] is not None else np.zeros(1, dtype=np.int32))],
-                         np.zeros(sum(n_tickets), dtype=np.int32), *([plans[0][1]] if on_device is not None else []))
-    tickets = tables[2 * len(plans)].view(torch.int32)
+    copy = None
     if on_device is not None:
-        # the scales to the work items and to the host as the packer's launches end, instead of through the host
+        # the launch that fills the scales into the work items, as the packer's launches end, also fetches the tables
         units_np, work_np = plans[0][0], plans[0][1]
         words = _lib.host_words(dev, 2 * len(units_np))
-        _lib.check(_lib.load().rdkv_stream_work_scales_device(
-            tables[-1].data_ptr(), len(work_np), on_device.scales.data_ptr(), int(on_device.scales.shape[2]), len(units_np),
-            words.take(2 * len(units_np)), words.tag, _lib.stream_of(dev)))
+
+        def copy(to, at, n, begins):
+            _lib.check(_lib.load().rdkv_stream_tables_device(
+                at, to, n, begins[-1], len(work_np), on_device.scales.data_ptr(), int(on_device.scales.shape[2]), len(units_np),
+                words.take(2 * len(units_np)), words.tag, _lib.stream_of(dev)))
+    tables = _lib.upload(dev, *[a for pl in plans for a in (pl[0], pl[2] if pl[2] is not None else np.zeros(1, dtype=np.int32))],
+                         np.zeros(sum(n_tickets), dtype=np.int32), *([plans[0][1]] if on_device is not None else []), copy=copy)
+    tickets = tables[2 * len(plans)].view(torch.int32)
     scales = []
     for (units_np, work_np, groups_np, order, rows, r_max), spec in zip(plans, specs):
         scale_max = spec[6]

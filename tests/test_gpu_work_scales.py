@@ -23,15 +23,21 @@ def test_scale_fields(heads, n_work):
     work = np.zeros(n_work, dtype=stream_cache.WORK_DTYPE)
     work["unit"] = np.arange(n_work) * 5 % units
     work["tile_begin"] = np.arange(n_work)
-    on_dev = torch.from_numpy(work.view(np.uint8).reshape(-1).copy() if n_work else np.zeros(1, np.uint8)).to(DEV)
+    head = np.arange(256, dtype=np.uint8)                # another table ahead of the items
+    host = torch.zeros(256 + 128 * n_work, dtype=torch.uint8, pin_memory=True)
+    host.numpy()[:256] = head
+    host.numpy()[256:] = work.view(np.uint8).reshape(-1)
+    on_dev = torch.full((256 + 128 * n_work + 16,), 7, dtype=torch.uint8, device=DEV)
     words = _lib.host_words(dev, 2 * units)
-    _lib.check(lib.rdkv_stream_work_scales_device(on_dev.data_ptr(), n_work, scales.data_ptr(), heads, units, words.take(2 * units), words.tag,
-                                                  _lib.stream_of(dev)))
+    call = lambda n, h, u: lib.rdkv_stream_tables_device(host.data_ptr(), on_dev.data_ptr(), 256 + 128 * n_work, 256, n,
+                                                         scales.data_ptr(), h, u, words.ptr, words.tag, _lib.stream_of(dev))
+    words.take(2 * units)
+    _lib.check(call(n_work, heads, units))
     got = np.asarray(words.read(dev), dtype=np.int32)
     both = np.stack([k, v], axis=1)
     assert (got == both.reshape(-1).view(np.int32)).all()
     if n_work:
         _lib.check(lib.rdkv_stream_work_scales(work.ctypes.data, n_work, both.ctypes.data, units))
-        assert on_dev.cpu().numpy().tobytes() == work.tobytes()
-    assert lib.rdkv_stream_work_scales_device(None, 1, scales.data_ptr(), heads, units, words.ptr, 1, None) == _lib.RDKV_EINVAL
-    assert lib.rdkv_stream_work_scales_device(None, 0, scales.data_ptr(), heads, units + (1 if heads > 1 else -units), words.ptr, 1, None) == _lib.RDKV_EINVAL
+    assert on_dev.cpu().numpy().tobytes() == head.tobytes() + work.tobytes() + bytes([7] * 16)
+    assert call(n_work + 1, heads, units) == _lib.RDKV_EINVAL
+    assert call(n_work, heads, units + (1 if heads > 1 else -units)) == _lib.RDKV_EINVAL
