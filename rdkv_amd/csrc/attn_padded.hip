@@ -153,6 +153,13 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
+// Sixteen bytes of LDS as words.  (Read as a vector, which may be anything, the compiler waits for every load into LDS
+// that is in flight, which the next tile's rows are: a call of 8 KV heads x 128k, low-bit 53.8 us, now 53.1.)
+__device__ __forceinline__ intx4 lds_row(const int8_t *p) {
+  const uint32_t *w = reinterpret_cast<const uint32_t *>(p);
+  return intx4{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+}
+
 // Blocks of the int8 products: 64 channels each, at most two per width (2 | 4 | 8 bit: blocks 0, 1 | 2, 3 | 4, 5).
 constexpr int kKBlocks = 6;
 
@@ -526,21 +533,21 @@ k_qk_dot_mfma_kernel(const void *__restrict__ q, int q_dtype, int64_t q_stride_h
   constexpr bool kLowHeld = !STATS;      // (no registers for them beside the softmax: from LDS for every tile)
   intx4 dig[kKBlocks][NG], low[kLowHeld ? kKBlocks : 1], start[NG], start_low{0, 0, 0, 0};
   auto low_from_lds = [&](int b) __attribute__((always_inline)) {
-    return *reinterpret_cast<const intx4 *>(&su.low[b][r >> 2][r & (2 * NG - 1)][16 * grp]);
+    return lds_row(&su.low[b][r >> 2][r & (2 * NG - 1)][16 * grp]);
   };
 #pragma unroll
   for (int hg = 0; hg < NG; ++hg) start[hg] = intx4{0, 0, 0, 0};
 #pragma unroll
   for (int b = 0; b < kKBlocks; ++b) {
     if ((b & 1) < blocks[b >> 1]) {
-      intx4 z = *reinterpret_cast<const intx4 *>(&su.zero[b][r & 1][16 * grp]);
+      intx4 z = lds_row(&su.zero[b][r & 1][16 * grp]);
       if (r > 1) z = intx4{0, 0, 0, 0};
       const intx4 lower = low_from_lds(b);
       if (kLowHeld) low[kLowHeld ? b : 0] = lower;
       start_low = __builtin_amdgcn_mfma_i32_16x16x64_i8(lower, z, start_low, 0, 0, 0);
 #pragma unroll
       for (int hg = 0; hg < NG; ++hg) {
-        dig[b][hg] = *reinterpret_cast<const intx4 *>(&su.digit[b][hg][r][16 * grp]);
+        dig[b][hg] = lds_row(&su.digit[b][hg][r][16 * grp]);
         start[hg] = __builtin_amdgcn_mfma_i32_16x16x64_i8(dig[b][hg], z, start[hg], 0, 0, 0);
       }
     }
