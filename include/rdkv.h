@@ -539,6 +539,7 @@ typedef struct RdkvStreamLayer {
   uint8_t *blob;
   int64_t blob_bytes, max_tv;
   int32_t n2p, n4p, n8, max_n16, max_tiles, reserved;
+  const int32_t *head_tiles;     /* [H_kv] or NULL: the 64-token tiles of every head, from which the launch is divided */
 } RdkvStreamLayer;
 int rdkv_pack_layers_stream(const RdkvStreamLayer *layers, int n_layers, int H_kv, const int32_t *order,
                             int64_t order_stride_h, const int32_t *counts, const int32_t *info, const void *k_bits,

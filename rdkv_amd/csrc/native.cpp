@@ -500,6 +500,9 @@ PyObject *stream_pack(PyObject *const *a, Py_ssize_t) {
   plain(mm.numel() >= n * H * 768 && plan.numel() >= 12 * n * H);
   std::vector<at::Tensor> blobs;
   std::vector<RdkvStreamLayer> layers;
+  std::vector<int32_t> tiles(n * H, 0);
+  for (int64_t i = 0; i < n * H; ++i)
+    for (const int32_t tokens : unit_p[i].n_tok) tiles[i] += (tokens + 63) / 64;      // (a tile: 64 tokens)
   int rc = RDKV_OK;
   {
     Unlocked u;
@@ -509,7 +512,7 @@ PyObject *stream_pack(PyObject *const *a, Py_ssize_t) {
       const int64_t bytes = std::max<int64_t>(size_p[4 * e], 256) + 256;
       blobs.push_back(at::empty({bytes}, Ks[e].options().dtype(at::kByte)));
       layers.push_back({Ks[e].data_ptr(), Vs[e].data_ptr(), Ks[e].stride(1), Ks[e].stride(2), data<uint8_t>(blobs.back()), bytes,
-                        d[3], d[0], d[1], d[2], d[4], (int32_t)size_p[4 * e + 1], 0});
+                        d[3], d[0], d[1], d[2], d[4], (int32_t)size_p[4 * e + 1], 0, tiles.data() + e * H});
     }
     const at::Tensor units = at::empty({n * H * (int64_t)sizeof(RdkvUnit)}, kb.options().dtype(at::kByte));
     rc = lib.rdkv_pack_layers_stream(layers.data(), n, H, data<int32_t>(order), T, data<int32_t>(plan),

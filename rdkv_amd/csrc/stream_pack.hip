@@ -125,10 +125,14 @@ struct StreamPackArgs {
   int H_kv;
   int64_t blob_bytes;
 };
-// The layers of a launch, one per blockIdx.z.
-constexpr int kBatchLayers = 8;
+// The layers of a launch.  Where the host knows the tiles of every head, and the heads are few enough for a lane each,
+// the packing workgroups of head r (over all layers) are begin[r] .. begin[r + 1] of a flat grid; otherwise every head
+// has as many, and blockIdx is (workgroup, head, layer).
+constexpr int kBatchLayers = 8, kTableHeads = 64;
 struct StreamPackBatch {
   StreamPackArgs layer[kBatchLayers];
+  int32_t begin[kTableHeads + 1];
+  int32_t by_table;
 };
 // where a layer's channel parameters lie in its scratch
 __device__ __forceinline__ float4 *chan_params_of(const StreamPackArgs &a) {
@@ -391,13 +395,21 @@ __device__ __forceinline__ TileInfo tile_info(const RdkvUnit &u, int ti) {
 // assembly; nothing makes a wavefront wait for another.  One layer of 8 x 32k / 128k tokens 54.8 / 170 -> 51.2 / 155 us.
 __global__ void __launch_bounds__(256, 3)
 stream_pack_kernel(StreamPackBatch batch) {
-  const StreamPackArgs a = batch.layer[blockIdx.z];
+  int layer = blockIdx.z, h = blockIdx.y, ti = blockIdx.x, stride = gridDim.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  if (batch.by_table) {
+    const int row = __popcll(__ballot(batch.begin[lane] <= ti)) - 1;      // (a head without tiles begins where the next does)
+    stride = batch.begin[row + 1] - batch.begin[row];
+    ti -= batch.begin[row];
+    layer = row / batch.layer[0].H_kv;
+    h = row - layer * batch.layer[0].H_kv;
+  }
+  const StreamPackArgs a = batch.layer[layer];
   const float4 *chan_params = chan_params_of(a);
   constexpr int kRows = RDKV_TILE / 4;                                          // tokens of a wavefront
   __shared__ __align__(16) uint8_t ck_all[4][kRows][kMaxSlots];                 // K code of (token, stream slot)
   __shared__ __align__(16) uint8_t cv_all[4][kRows * kD * 2];                   // V code of (token, channel); fp16 bits for class 3
   __shared__ float4 chan[kD];                                                   // the head's channel quantizers
-  const int h = blockIdx.y, tid = threadIdx.x, stride = gridDim.x, lane = tid & 63;
   const int g = __builtin_amdgcn_readfirstlane(tid >> 6);
   uint8_t (*ck)[kMaxSlots] = ck_all[g];
   uint8_t (*cv)[kD] = reinterpret_cast<uint8_t (*)[kD]>(cv_all[g]);
@@ -406,7 +418,6 @@ stream_pack_kernel(StreamPackBatch batch) {
   const int R = u.d8 + u.d4 + u.d2;
   const int n_tiles = (u.n_tok[0] + RDKV_TILE - 1) / RDKV_TILE + (u.n_tok[1] + RDKV_TILE - 1) / RDKV_TILE +
                       (u.n_tok[2] + RDKV_TILE - 1) / RDKV_TILE + (u.n_tok[3] + RDKV_TILE - 1) / RDKV_TILE;
-  int ti = blockIdx.x;
   if (ti >= n_tiles) return;
   const int p = lane & 15, r = lane >> 4;
   const int32_t *ord = a.order + (int64_t)h * a.order_stride_h;
@@ -640,8 +651,11 @@ RDKV_API int rdkv_pack_layer_stream_ws_init(float *minmax_ws, int H_kv, void *st
   return RDKV_OK;
 }
 
-// As many workgroups as the device holds at once, each with the same number of tiles of the longest head.
-static int launch_stream_pack(const StreamPackBatch &batch, int n_layers, int H_kv, hipStream_t s) {
+// As many workgroups as the device holds at once.  With the tiles of every head, the most that any workgroup has is as
+// small as that number allows: the heads of a layer keep between half and all of their tokens, and with the longest head's
+// share given to every head the launch ran its last quarter on a part of its wavefronts (four layers of 8 x 32k, Dirichlet
+// shares, 153 -> 132 us; equal heads the same).  One and a third times as many workgroups 160, twice 139, four times 138.
+static int launch_stream_pack(StreamPackBatch &batch, const int32_t *const *head_tiles, int n_layers, int H_kv, hipStream_t s) {
   hipLaunchKernelGGL(slot_params_kernel, dim3(H_kv, 1, n_layers), dim3(128), 0, s, batch);
   int max_tiles = 0;
   for (int l = 0; l < n_layers; ++l) max_tiles = std::max(max_tiles, batch.layer[l].max_tiles);
@@ -657,6 +671,26 @@ static int launch_stream_pack(const StreamPackBatch &batch, int n_layers, int H_
       if (ok) resident_of_device[dev] = cus * per_cu;   // (otherwise asked again next time)
     }
     if (resident_of_device[dev] > 0) resident = resident_of_device[dev];
+  }
+  batch.by_table = head_tiles != nullptr && (int64_t)H_kv * n_layers <= std::min(kTableHeads, resident);
+  for (int l = 0; l < n_layers && batch.by_table; ++l) batch.by_table = head_tiles[l] != nullptr;
+  if (batch.by_table) {
+    const int heads = H_kv * n_layers;
+    auto tiles = [&](int r) { return (int64_t)head_tiles[r / H_kv][r % H_kv]; };
+    int64_t all = 0, n = 0;
+    for (int r = 0; r < heads; ++r) all += tiles(r);
+    if (all == 0) return RDKV_OK;
+    for (int64_t per = (all + resident - 1) / resident;; ++per) {
+      n = 0;
+      for (int r = 0; r < heads; ++r) {
+        batch.begin[r] = (int32_t)n;
+        n += (tiles(r) + per - 1) / per;
+      }
+      if (n <= resident) break;        // (at the latest with a workgroup a head)
+    }
+    for (int r = heads; r <= kTableHeads; ++r) batch.begin[r] = (int32_t)n;
+    hipLaunchKernelGGL(stream_pack_kernel, dim3((unsigned)n), dim3(256), 0, s, batch);
+    return RDKV_OK;
   }
   const int rows = H_kv * n_layers, target = std::max(1, (resident + rows - 1) / rows);
   const int per = (max_tiles + target - 1) / target;
@@ -723,7 +757,7 @@ RDKV_API int rdkv_pack_layer_stream(const void *K_f16, const void *V_f16, int64_
                                         minmax_ws, /*init=*/minmax_ws_ready == 0, s);
     if (mrc != RDKV_OK) return mrc;
   }
-  launch_stream_pack(batch, 1, H_kv, s);
+  launch_stream_pack(batch, nullptr, 1, H_kv, s);
   RDKV_CHECK_LAUNCH(fn);
   return RDKV_OK;
 }
@@ -739,9 +773,13 @@ RDKV_API int rdkv_pack_layers_stream(const RdkvStreamLayer *layers, int n_layers
     for (int first = 0; first < n_layers; first += kBatchLayers) {
       const int n = std::min(kBatchLayers, n_layers - first);
       StreamPackBatch batch;
+      const int32_t *head_tiles[kBatchLayers];
       for (int i = 0; i < n; ++i) {
         const int64_t l = first + i, row = l * H_kv;
         const RdkvStreamLayer &y = layers[l];
+        head_tiles[i] = y.head_tiles;
+        for (int h = 0; y.head_tiles && h < H_kv; ++h)
+          RDKV_REQUIRE(y.head_tiles[h] >= 0 && y.head_tiles[h] <= y.max_tiles, "%s: head_tiles outside 0..max_tiles", fn);
         const int rc = fill_stream_args(fn, &batch.layer[i], y.K_f16, y.V_f16, y.stride_h, y.stride_t, H_kv,
                                         order ? order + row * order_stride_h : nullptr, order_stride_h,
                                         counts ? counts + 4 * row : nullptr,
@@ -752,7 +790,7 @@ RDKV_API int rdkv_pack_layers_stream(const RdkvStreamLayer *layers, int n_layers
                                         scale_max ? scale_max + 2 * row : nullptr);
         if (rc != RDKV_OK) return rc;
       }
-      if (pass == 1) launch_stream_pack(batch, n, H_kv, (hipStream_t)stream);
+      if (pass == 1) launch_stream_pack(batch, head_tiles, n, H_kv, (hipStream_t)stream);
     }
   }
   RDKV_CHECK_LAUNCH(fn);

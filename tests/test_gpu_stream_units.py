@@ -9,7 +9,7 @@ from tests.gpu_util import DEV, require_gpu
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("H,T,layers", [(1, 65, 1), (300, 70, 1), (24, 200, 9)])
+@pytest.mark.parametrize("H,T,layers", [(1, 65, 1), (300, 70, 1), (24, 200, 9), (8, 5000, 8), (64, 700, 1), (65, 700, 1)])
 def test_blobs_equal_the_general_path(H, T, layers, monkeypatch):
     require_gpu()
     g = torch.Generator(device=DEV).manual_seed(H)
