@@ -7,6 +7,7 @@
 // the Python code it was called from then takes them, with its own conversions and its own errors.  Nothing is kept
 // from one call for the next but the addresses of the library's functions.
 #include <Python.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/_to_copy.h>
@@ -14,7 +15,6 @@
 #include <ATen/ops/empty.h>
 
 #include <algorithm>
-#include <exception>
 #include <initializer_list>
 #include <string>
 #include <utility>
@@ -125,20 +125,20 @@ PyObject *ints(std::initializer_list<int64_t> v) {
   return t.release();
 }
 
-// The entry points: a function of (args, count) that returns a new reference.
+// The entry points: a function of (args, count) that returns a new reference.  Errors of torch's own come out as torch's
+// bindings raise them (an allocation that fails: torch.OutOfMemoryError, which callers catch to free memory).
 template <PyObject *(*F)(PyObject *const *, Py_ssize_t), int N>
 PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (n != N) return PyErr_Format(PyExc_TypeError, "%d arguments expected, got %zd", N, n);
+  HANDLE_TH_ERRORS
   try {
     return F(args, n);
   } catch (const NotPlain &) {
     Py_RETURN_NONE;
   } catch (const PythonError &) {
     return nullptr;
-  } catch (const std::exception &e) {
-    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
   }
+  END_HANDLE_TH_ERRORS
 }
 
 // ---- packing of a planned layer (packing._pack_planned_layer) -----------------------------------------------------

@@ -1,0 +1,79 @@
+"""Errors out of csrc/native.cpp: an allocation that fails is torch's own OutOfMemoryError, which programs catch to free
+memory and try again, from every entry point that allocates, and the call after it gives what it gave before."""
+import contextlib
+
+import pytest
+import torch
+
+from rdkv_amd import _lib, knapsack_solver as ks, obkv_fast, packing, stream_cache, trizone_decompress as tz
+from tests.gpu_util import DEV, require_gpu
+
+pytestmark = pytest.mark.gpu
+H, T, G = 2, 300, 4
+
+
+@contextlib.contextmanager
+def _no_memory_left():
+    """The process may take no more of the device than it has, and the allocator's free pieces are taken."""
+    taken = []
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.set_per_process_memory_fraction(0.0)
+    try:
+        for n in (1 << 20, 1 << 16, 512):
+            with contextlib.suppress(torch.OutOfMemoryError):
+                while True:
+                    taken.append(torch.empty(n, dtype=torch.uint8, device=DEV))
+        yield
+    finally:
+        del taken
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+@pytest.fixture(scope="module")
+def calls():
+    """By entry point: (the function of the module that it has to reach, the call)."""
+    require_gpu()
+    g = torch.Generator(device=DEV).manual_seed(5)
+    K, V = (torch.randn(1, H, T, 128, device=DEV, dtype=torch.float16, generator=g) for _ in range(2))
+    v_bits = torch.tensor([0, 2, 4, 8, 16], device=DEV)[torch.randint(0, 5, (H, T), device=DEV, generator=g)]
+    k_bits = torch.full((H, 128), 4, device=DEV)
+    scores, channels = torch.rand(H, T, device=DEV, generator=g), torch.rand(H, 128, device=DEV, generator=g)
+    options = dict(gqa_factor=G, token_budget=100, k_budget_ratio=0.5, obs_window=32, pool_kernel_size=7, pool_padding="reflect",
+                   v_bit_options=None, k_bit_options=None, eps_V=ks.DEFAULT_EPSILON_V, eps_K=ks.DEFAULT_EPSILON_K)
+    planned = packing._plan_layers(v_bits, k_bits, K.device, (K,), 256)
+    layer, v16 = packing.pack_layer_per_head(K, V, v_bits, k_bits, G)
+    cache = stream_cache.build_stream_cache_from_kv([(K, V, v_bits, k_bits)], G)
+    q = torch.randn(cache.rows, 128, device=DEV, dtype=torch.float16, generator=g)
+    dense = packing.TriZoneCache((layer,), [v16], [None], [None], T)
+    return {
+        "select_layer": lambda: obkv_fast._perhead_select_and_pack(K, V, scores, channels, **options)[0].V_scale,
+        "pack_layer": lambda: packing._pack_planned_layer(K, V, G, planned, 0, H)[0].K_4bit,
+        "stream_order": lambda: stream_cache.build_stream_cache_from_kv([(K, V, v_bits, k_bits)], G).blobs[0],
+        "dense_layer": lambda: tz.unpack_trizone_to_past_kv(dense, head_dim=128)[0][0],
+        "decode_attn": lambda: stream_cache.decode_attn_fused(cache, q)[0],
+    }
+
+
+class _Reached:
+    """The module, with the names of the functions that were called."""
+
+    def __init__(self, native):
+        self.native, self.names = native, []
+
+    def __getattr__(self, name):
+        self.names.append(name)
+        return getattr(self.native, name)
+
+
+@pytest.mark.parametrize("name", ["select_layer", "pack_layer", "stream_order", "dense_layer", "decode_attn"])
+def test_out_of_memory(calls, name, monkeypatch):
+    reached = _Reached(_lib.native)
+    monkeypatch.setattr(_lib, "native", reached)
+    want = calls[name]().clone()
+    reached.names.clear()
+    with _no_memory_left():
+        with pytest.raises(torch.OutOfMemoryError):
+            calls[name]()
+        assert reached.names == [name]
+    assert torch.equal(calls[name](), want)
