@@ -544,12 +544,13 @@ PyObject *field(PyObject *dict, const char *name) {
 PyObject *decode_attn(PyObject *const *a, Py_ssize_t) {
   PyObject *c = a[0];
   plain(PyDict_Check(c));
-  const at::Tensor &q = tensor(a[2]), &units = tensor(field(c, "units")), &work = tensor(field(c, "work"));
+  // (what is reached through a dictionary is held: another thread may replace it while the lock is released)
+  const at::Tensor &q = tensor(a[2]), units = tensor(field(c, "units")), work = tensor(field(c, "work"));
   const int64_t n_units = integer(field(c, "n_units")), n_work = integer(field(c, "n_work")), G = integer(field(c, "G")),
                 rows = integer(field(c, "rows")), n_groups = integer(field(c, "n_groups"));
   const int row_dwords = (int)(integer(field(c, "max_row_dwords")) | integer(field(c, "row_shape")) << 8);
-  const int32_t *groups = nullptr;
-  if (n_groups != n_work) groups = data<int32_t>(tensor(field(c, "groups")));
+  const at::Tensor group_table = n_groups != n_work ? tensor(field(c, "groups")) : at::Tensor();
+  const int32_t *groups = data<int32_t>(group_table);
   const auto dev = q.device();
   const int q_dt = dtype_code(q);
   plain(q.is_cuda() && q_dt >= 0 && shape_is(q, {rows, 128}) && q.stride(1) == 1 && units.device() == dev && work.device() == dev);
@@ -645,10 +646,11 @@ PyObject *dense_layer(PyObject *const *a, Py_ssize_t) {
     PyObject *o = field(f, name);
     return o == Py_None ? at::Tensor() : tensor(o);
   };
-  const at::Tensor &ks = tensor(field(f, "K_ch_scale")), &kz = tensor(field(f, "K_ch_zp")),
-                   &sort = tensor(field(f, "K_ch_sort_idx_per_head")), &k_counts = tensor(field(f, "K_ch_seg_bounds_per_head")),
-                   &vs = tensor(field(f, "V_scale")), &vz = tensor(field(f, "V_zp")),
-                   &v_counts = tensor(field(f, "seg_bounds_per_head")), &totals = tensor(field(f, "T_eff_per_head"));
+  // (held, not referred to: another thread may replace a field while the lock is released)
+  const at::Tensor ks = tensor(field(f, "K_ch_scale")), kz = tensor(field(f, "K_ch_zp")),
+                   sort = tensor(field(f, "K_ch_sort_idx_per_head")), k_counts = tensor(field(f, "K_ch_seg_bounds_per_head")),
+                   vs = tensor(field(f, "V_scale")), vz = tensor(field(f, "V_zp")),
+                   v_counts = tensor(field(f, "seg_bounds_per_head")), totals = tensor(field(f, "T_eff_per_head"));
   const auto dev = ks.device();
   const int64_t T_v = integer(field(f, "T_eff")), T_k = integer(field(f, "T_eff_k")), n16 = integer(field(f, "n_v16"));
   plain(ks.is_cuda() && ks.dim() == 4 && T_v > 0 && T_k == T_v + n16 && n16 >= 0);

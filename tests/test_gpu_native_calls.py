@@ -1,9 +1,12 @@
-"""Errors out of csrc/native.cpp: an allocation that fails is torch's own OutOfMemoryError, which programs catch to free
-memory and try again, from every entry point that allocates, and the call after it gives what it gave before."""
+"""Errors and lifetimes in csrc/native.cpp: an allocation that fails is torch's own OutOfMemoryError, which programs catch
+to free memory and try again, from every entry point that allocates, and the call after it gives what it gave before;
+fields that another thread replaces while a call runs without the interpreter's lock stay whole for that call."""
 import contextlib
+import gc
 
 import pytest
 import torch
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from rdkv_amd import _lib, knapsack_solver as ks, obkv_fast, packing, stream_cache, trizone_decompress as tz
 from tests.gpu_util import DEV, require_gpu
@@ -77,3 +80,60 @@ def test_out_of_memory(calls, name, monkeypatch):
             calls[name]()
         assert reached.names == [name]
     assert torch.equal(calls[name](), want)
+
+
+class _Replacing(TorchDispatchMode):
+    """Runs ``change`` under the first allocation, which a native call makes without the lock, as another thread might."""
+
+    def __init__(self, change):
+        super().__init__()
+        self.change = change
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        if self.change is not None:
+            change, self.change = self.change, None
+            change()
+            gc.collect()
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("fields", [("K_ch_scale", "K_ch_zp", "K_ch_sort_idx_per_head", "K_ch_seg_bounds_per_head"),
+                                    ("V_scale", "V_zp", "seg_bounds_per_head", "T_eff_per_head", "K_4bit", "V_2bit", "softmax_mask")])
+def test_layer_fields_replaced_under_a_call(fields):
+    require_gpu()
+    g = torch.Generator(device=DEV).manual_seed(5)
+    K, V = (torch.randn(1, H, T, 128, device=DEV, dtype=torch.float16, generator=g) for _ in range(2))
+    v_bits = torch.tensor([0, 2, 4, 8, 16], device=DEV)[torch.randint(0, 5, (H, T), device=DEV, generator=g)]
+    layer, v16 = packing.pack_layer_per_head(K, V, v_bits, torch.full((H, 128), 4, device=DEV), G)
+    dense = packing.TriZoneCache((layer,), [v16], [None], [None], T)
+    (want,), (mask,) = tz.unpack_trizone_to_past_kv(dense, head_dim=128, return_masks=True)
+    spare = {f: torch.full_like(getattr(layer, f), 1) for f in fields}
+    with _Replacing(lambda: layer.__dict__.update(spare)) as mode:
+        native = _lib.native.dense_layer(layer.__dict__, (v16, layer.softmax_mask, 0), 128, *_words(layer), _lib.stream_of(K.device))
+    assert mode.change is None and all(getattr(layer, f) is spare[f] for f in fields)
+    torch.cuda.synchronize()
+    for a, b in zip(native, (*want, mask)):
+        assert torch.equal(a, b)
+
+
+def _words(layer):
+    n = int(layer.K_ch_scale.shape[1])
+    words = _lib.host_words(layer.K_ch_scale.device, 8 * n)
+    return words.take(4 * n), words.take(4 * n), words.tag
+
+
+def test_cache_tables_replaced_under_a_call():
+    require_gpu()
+    g = torch.Generator(device=DEV).manual_seed(6)
+    K, V = (torch.randn(1, H, 3000, 128, device=DEV, dtype=torch.float16, generator=g) for _ in range(2))
+    bits = torch.full((H, 3000), 4, device=DEV)
+    cache = stream_cache.build_stream_cache_from_kv([(K, V, bits, torch.full((H, 128), 4, device=DEV))], G, n_groups=3)
+    assert cache.n_groups != cache.n_work
+    q = torch.randn(cache.rows, 128, device=DEV, dtype=torch.float16, generator=g)
+    want = stream_cache.decode_attn_fused(cache, q)
+    tables = {f: getattr(cache, f).clone() for f in ("units", "work", "groups")}
+    with _Replacing(lambda: cache.__dict__.update(tables)) as mode:
+        got = stream_cache.decode_attn_fused(cache, q)
+    assert mode.change is None and cache.units is tables["units"]
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
