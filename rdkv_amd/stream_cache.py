@@ -935,10 +935,12 @@ def decode_attn_fused(cache: StreamCache, q: torch.Tensor, out: Optional[torch.T
         kn, vn, counts = (None, None, None) if zone_c is None else (zone_c[0], zone_c[1], zone_c[2] if len(zone_c) > 2 else None)
         cos, sin = (None, None) if rope is None else rope
         k_step, v_step, row = (None, None, None) if append is None or zone_c is None else append
-        done = _lib.native.decode_attn(cache.__dict__, cache.units_host, q, out, lse, cos, sin, kn, vn, counts, k_step, v_step,
-                                       row, ws.data_ptr(), ws.numel(), stream)
-        if done is not None:
-            return done
+        # (a part that is given as None is not a part that is not given: the checks below refuse it)
+        if (rope is None or cos is not None) and (zone_c is None or (kn is not None and (append is None or k_step is not None))):
+            done = _lib.native.decode_attn(cache.__dict__, cache.units_host, q, out, lse, cos, sin, kn, vn, counts, k_step, v_step,
+                                           row, ws.data_ptr(), ws.numel(), stream)
+            if done is not None:
+                return done
     dev = _lib.require_device(q)
     q_dt = _lib.DTYPE_CODE.get(q.dtype)
     if q_dt is None:

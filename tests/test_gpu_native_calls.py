@@ -137,3 +137,21 @@ def test_cache_tables_replaced_under_a_call():
     assert mode.change is None and cache.units is tables["units"]
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+def test_parts_of_a_step_that_are_none_are_refused():
+    """Given, but empty, is not the same as not given: no step without the rotation or the appended row that was asked for."""
+    require_gpu()
+    g = torch.Generator(device=DEV).manual_seed(7)
+    K, V = (torch.randn(1, H, T, 128, device=DEV, dtype=torch.float16, generator=g) for _ in range(2))
+    cache = stream_cache.build_stream_cache_from_kv([(K, V, torch.full((H, T), 4, device=DEV), torch.full((H, 128), 4, device=DEV))], G)
+    q = torch.randn(cache.rows, 128, device=DEV, dtype=torch.float16, generator=g)
+    new = torch.zeros(H, 4, 128, device=DEV)
+    zone_c = (new, new.clone(), torch.ones(H, dtype=torch.int32, device=DEV))
+    row, x = torch.zeros(1, dtype=torch.int64, device=DEV), torch.zeros(H, 128, device=DEV, dtype=torch.float16)
+    for bad in (dict(rope=(None, None)), dict(zone_c=(None, None)), dict(zone_c=(None, None, zone_c[2])), dict(zone_c=zone_c, append=(None, None, None)),
+                dict(zone_c=zone_c, append=(None, x, row)), dict(zone_c=zone_c, append=(x, None, row)), dict(zone_c=zone_c, append=(x, x, None)),
+                dict(rope=(torch.zeros(64, device=DEV), None)), dict(zone_c=(new, None))):
+        with pytest.raises((AttributeError, AssertionError)):
+            stream_cache.decode_attn_fused(cache, q, **bad)
+    assert not new.any()
