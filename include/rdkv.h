@@ -828,7 +828,7 @@ int rdkv_knapsack_batched_value(const float *scores, int64_t stride_b, int B, in
                                 void *stream);
 
 /* A layer's selection up to the token order of its packer (obkv_fast.py:899-1040), in three launches: rdkv_pool_scores
- * (kernel_size > 1; pooled [H, T]; its length must stay T), rdkv_knapsack_batched_value over the H rows of tokens as one
+ * (kernel_size > 1; pooled [H, T]; RDKV_EINVAL for an even kernel, whose rows would be longer), rdkv_knapsack_batched_value over the H rows of tokens as one
  * group at v_budget (v_bits: bytes, rows of v_stride, a multiple of 16, the base 16-byte aligned; v_counts
  * [H, n_v_options]), the K allocation over channels [H, D] at the budgets that v_counts leave (k_bits [H, D] bytes), and
  * what rdkv_pack_layer_plan_start leaves for those widths: order and rank3 [H, T], plan

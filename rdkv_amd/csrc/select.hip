@@ -9,6 +9,8 @@
 // several workgroups each, and short rows as a wavefront each with the row in registers.
 // All lambda arithmetic is single IEEE operations in the order the reference's tensor
 // expressions imply; this file is compiled without floating-point contraction.
+#include <algorithm>
+
 #include "rdkv_common.h"
 
 // No fused multiply-adds in this file, whatever the command line says: the reference rounds every
@@ -1342,6 +1344,8 @@ RDKV_API int rdkv_select_layer_start(const float* scores, int64_t stride_b, int 
   if (!v_counts || !channels || !k_bits || !order || !rank3 || !plan || !host_words || v_stride < T || v_stride % 16 != 0 ||
       reinterpret_cast<uintptr_t>(v_bits) % 16 != 0 || zero_option >= n_v_options || channel_stride < D)
     return fail("rdkv_select_layer_start: bad arguments");
+  if (kernel_size > 1 && (reflect ? std::min<int64_t>(kernel_size, 2 * T - 1) : kernel_size) % 2 == 0)
+    return fail("rdkv_select_layer_start: an even kernel changes the rows' length");
   if (workspace == nullptr || workspace_bytes < rdkv_knapsack_workspace_bytes(H)) {
     rdkv_set_error("rdkv_select_layer_start: workspace too small");
     return RDKV_EWORKSPACE;

@@ -496,3 +496,20 @@ def test_pre_extract_weights_on_a_cpu_model():
     with pytest.raises((RuntimeError, AssertionError)):
         fast_decode.greedy_decode_fast(llama, packing.TriZoneCache((), [], [], [], 0), torch.zeros(64), 1, [],
                                        torch.device("cpu"), 0)
+
+
+def test_selection_call_refuses_kernels_that_change_the_length():
+    """Pooling with an even kernel gives one value more than a row has: refused before anything is launched (here, where
+    nothing can be)."""
+    import ctypes
+    lib = _lib.load()
+    room = np.zeros(4096, dtype=np.float32)
+    p = (room.ctypes.data + 15) // 16 * 16
+    one = (ctypes.c_float * 1)(0.0)
+
+    def call(kernel, reflect, T):
+        return lib.rdkv_select_layer_start(p, T, 1, T, kernel, 1, reflect, p, 1.0, one, one, 1, 0, p, 16 * T, p, p, 4, 4, 1.0, one, one, 1, p, 64,
+                                           0.01, p, p, p, None, 0, None, None, p, 1, p, 1 << 24, None)
+
+    for kernel, reflect, T in ((2, 0, 8), (4, 1, 8), (14, 1, 8), (100, 0, 3)):
+        assert call(kernel, reflect, T) == _lib.RDKV_EINVAL and b"even kernel" in lib.rdkv_last_error()
