@@ -160,12 +160,14 @@ def unpack_trizone_to_past_kv(dual_cache: TriZoneCache, *, head_dim: int,
         to = _words_of(pl.K_ch_scale.device, words, heads) if pl.K_ch_scale is not None else None
         zone_b = dual_cache.new_v_only[i] if i < len(dual_cache.new_v_only) else None
         pair = mask = None
-        if to is not None and _lib.native is not None and _is_perhead_layout(pl):
-            used, n = to.used, int(pl.K_ch_scale.shape[1])
+        n = 0 if to is None else int(pl.K_ch_scale.shape[1])
+        # (words were counted by the scales there are: a layer without V scales has none for V)
+        if to is not None and _lib.native is not None and _is_perhead_layout(pl) and to.used + 8 * n <= to.size:
+            used = to.used
             if return_masks and mask_dtype == torch.float16 and device is None:
                 mask = pl.softmax_mask
-            pair = _lib.native.dense_layer(pl.__dict__, zone_b if mask is None else (zone_b, mask, max_new_tokens), head_dim, to.take(4 * n), to.take(4 * n), to.tag,
-                                           _lib.stream_of(pl.K_ch_scale.device))
+            pair = _lib.native.dense_layer(pl.__dict__, zone_b if mask is None else (zone_b, mask, max_new_tokens), head_dim,
+                                           to.take(4 * n), to.take(4 * n), to.tag, _lib.stream_of(pl.K_ch_scale.device))
             if pair is None:
                 to.used = used
             else:

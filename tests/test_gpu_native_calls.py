@@ -2,6 +2,7 @@
 to free memory and try again, from every entry point that allocates, and the call after it gives what it gave before;
 fields that another thread replaces while a call runs without the interpreter's lock stay whole for that call."""
 import contextlib
+import dataclasses
 import gc
 
 import pytest
@@ -155,3 +156,20 @@ def test_parts_of_a_step_that_are_none_are_refused():
         with pytest.raises((AttributeError, AssertionError)):
             stream_cache.decode_attn_fused(cache, q, **bad)
     assert not new.any()
+
+
+def test_layers_without_v_scales_take_no_words_for_them(monkeypatch):
+    """As many layers that keep only fp16 tokens, and have no tensor of V scales, as fill the words of one call."""
+    require_gpu()
+    g = torch.Generator(device=DEV).manual_seed(8)
+    heads, layers = 8, 128
+    K, V = (torch.randn(1, heads, 5, 128, device=DEV, dtype=torch.float16, generator=g) for _ in range(2))
+    layer, v16 = packing.pack_layer_per_head(K, V, torch.full((heads, 5), 16, device=DEV), torch.full((heads, 128), 4, device=DEV), G)
+    assert layer.T_eff == 0
+    bare = dataclasses.replace(layer, V_scale=None, V_zp=None)
+    monkeypatch.setattr(_lib, "_host_words", {})
+    assert _lib.host_words(K.device, 4 * heads * layers).size == 4 * heads * layers
+    _lib.host_words(K.device, 1).pending = False
+    got = tz.unpack_trizone_to_past_kv(packing.TriZoneCache((bare,) * layers, [v16] * layers, [None] * layers, [None] * layers, 5), head_dim=128)
+    want, = tz.unpack_trizone_to_past_kv(packing.TriZoneCache((layer,), [v16], [None], [None], 5), head_dim=128)
+    assert len(got) == layers and all(torch.equal(k, want[0]) and torch.equal(v, want[1]) for k, v in got)
