@@ -68,7 +68,17 @@ int64_t integer(PyObject *o) {
   if (v == -1 && PyErr_Occurred()) throw PythonError{};
   return v;
 }
+int64_t whole(PyObject *o) {      // a field or an option: other numbers are another form
+  plain(PyIndex_Check(o));
+  const long long v = PyLong_AsLongLong(o);
+  if (v == -1 && PyErr_Occurred()) {
+    PyErr_Clear();
+    throw NotPlain{};
+  }
+  return v;
+}
 double real(PyObject *o) {
+  plain(PyFloat_Check(o) || PyLong_Check(o));
   const double v = PyFloat_AsDouble(o);
   if (v == -1.0 && PyErr_Occurred()) throw PythonError{};
   return v;
@@ -546,9 +556,9 @@ PyObject *decode_attn(PyObject *const *a, Py_ssize_t) {
   plain(PyDict_Check(c));
   // (what is reached through a dictionary is held: another thread may replace it while the lock is released)
   const at::Tensor &q = tensor(a[2]), units = tensor(field(c, "units")), work = tensor(field(c, "work"));
-  const int64_t n_units = integer(field(c, "n_units")), n_work = integer(field(c, "n_work")), G = integer(field(c, "G")),
-                rows = integer(field(c, "rows")), n_groups = integer(field(c, "n_groups"));
-  const int row_dwords = (int)(integer(field(c, "max_row_dwords")) | integer(field(c, "row_shape")) << 8);
+  const int64_t n_units = whole(field(c, "n_units")), n_work = whole(field(c, "n_work")), G = whole(field(c, "G")),
+                rows = whole(field(c, "rows")), n_groups = whole(field(c, "n_groups"));
+  const int row_dwords = (int)(whole(field(c, "max_row_dwords")) | whole(field(c, "row_shape")) << 8);
   const at::Tensor group_table = n_groups != n_work ? tensor(field(c, "groups")) : at::Tensor();
   const int32_t *groups = data<int32_t>(group_table);
   const auto dev = q.device();
@@ -640,7 +650,7 @@ PyObject *dense_layer(PyObject *const *a, Py_ssize_t) {
   if (PyTuple_Check(rows_b)) {
     plain(PyTuple_GET_SIZE(a[1]) == 3);
     rows_b = PyTuple_GET_ITEM(a[1], 0), mask_o = PyTuple_GET_ITEM(a[1], 1);
-    extra = std::max<int64_t>(integer(PyTuple_GET_ITEM(a[1], 2)), 0);
+    extra = std::max<int64_t>(whole(PyTuple_GET_ITEM(a[1], 2)), 0);
   }
   auto maybe = [&](const char *name) {
     PyObject *o = field(f, name);
@@ -652,13 +662,13 @@ PyObject *dense_layer(PyObject *const *a, Py_ssize_t) {
                    vs = tensor(field(f, "V_scale")), vz = tensor(field(f, "V_zp")),
                    v_counts = tensor(field(f, "seg_bounds_per_head")), totals = tensor(field(f, "T_eff_per_head"));
   const auto dev = ks.device();
-  const int64_t T_v = integer(field(f, "T_eff")), T_k = integer(field(f, "T_eff_k")), n16 = integer(field(f, "n_v16"));
+  const int64_t T_v = whole(field(f, "T_eff")), T_k = whole(field(f, "T_eff_k")), n16 = whole(field(f, "n_v16"));
   plain(ks.is_cuda() && ks.dim() == 4 && T_v > 0 && T_k == T_v + n16 && n16 >= 0);
   const int64_t H = ks.size(1);
   auto three = [&](const char *name, int64_t *out) {
     PyObject *t = field(f, name);
     plain(PyTuple_Check(t) && PyTuple_GET_SIZE(t) == 3);
-    for (int i = 0; i < 3; ++i) out[i] = integer(PyTuple_GET_ITEM(t, i));
+    for (int i = 0; i < 3; ++i) out[i] = whole(PyTuple_GET_ITEM(t, i));
   };
   auto dense = [&](const at::Tensor &t, at::ScalarType type, std::initializer_list<int64_t> s) {
     plain(t.device() == dev && t.scalar_type() == type && shape_is(t, s) && t.is_contiguous());

@@ -173,3 +173,16 @@ def test_layers_without_v_scales_take_no_words_for_them(monkeypatch):
     got = tz.unpack_trizone_to_past_kv(packing.TriZoneCache((bare,) * layers, [v16] * layers, [None] * layers, [None] * layers, 5), head_dim=128)
     want, = tz.unpack_trizone_to_past_kv(packing.TriZoneCache((layer,), [v16], [None], [None], 5), head_dim=128)
     assert len(got) == layers and all(torch.equal(k, want[0]) and torch.equal(v, want[1]) for k, v in got)
+
+
+@pytest.mark.parametrize("extra", [0.0, -1.0, -3, True, 2])
+def test_numbers_of_new_tokens(extra):
+    """Zero and less, as any number, add nothing to the masks; a layer's sizes may be any numbers too."""
+    require_gpu()
+    g = torch.Generator(device=DEV).manual_seed(9)
+    K, V = (torch.randn(1, H, T, 128, device=DEV, dtype=torch.float16, generator=g) for _ in range(2))
+    layer, v16 = packing.pack_layer_per_head(K, V, torch.full((H, T), 4, device=DEV), torch.full((H, 128), 4, device=DEV), G)
+    dense = packing.TriZoneCache((layer,), [v16], [None], [None], T)
+    layer.T_eff, layer.n_v16 = float(layer.T_eff), torch.tensor(float(layer.n_v16))            # (sizes of a layer made by hand)
+    _, (mask,) = tz.unpack_trizone_to_past_kv(dense, head_dim=128, return_masks=True, max_new_tokens=extra)
+    assert torch.equal(mask, torch.zeros(1, H * G, 1, T + max(int(extra), 0), dtype=torch.float16, device=DEV))
