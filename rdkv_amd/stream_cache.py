@@ -403,13 +403,15 @@ def _pack_scratch(dev, stream: int, H_kv: int) -> torch.Tensor:
 
 class _DeviceScales:
     """The largest scales [entries, 2, heads] that launches still running leave on the device; called: as rows of units,
-    fp32 [entries * heads, 2], on the host (synchronizes)."""
+    fp32 [entries * heads, 2], on the host (the first call synchronizes, the caches of several entries ask one by one)."""
 
     def __init__(self, scales: torch.Tensor):
-        self.scales = scales
+        self.scales, self.on_host = scales, None
 
     def __call__(self) -> np.ndarray:
-        return _lib.download(self.scales).transpose(0, 2, 1).reshape(-1, 2).astype(np.float32)
+        if self.on_host is None:
+            self.on_host = _lib.download(self.scales).transpose(0, 2, 1).reshape(-1, 2).astype(np.float32)
+        return self.on_host
 
 
 def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, stream: int):

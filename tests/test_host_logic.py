@@ -513,3 +513,14 @@ def test_selection_call_refuses_kernels_that_change_the_length():
 
     for kernel, reflect, T in ((2, 0, 8), (4, 1, 8), (14, 1, 8), (100, 0, 3)):
         assert call(kernel, reflect, T) == _lib.RDKV_EINVAL and b"even kernel" in lib.rdkv_last_error()
+
+
+def test_scales_of_several_caches_are_read_once(monkeypatch):
+    """Caches extended together ask for the same launches' scales one by one: one copy and one wait, not one a cache."""
+    from rdkv_amd import stream_cache
+    reads = []
+    monkeypatch.setattr(_lib, "download", lambda t: (reads.append(1), t.numpy().copy())[1])
+    scales = stream_cache._DeviceScales(torch.arange(12.0).reshape(2, 2, 3))
+    first = scales()
+    assert np.array_equal(first, [[0, 3], [1, 4], [2, 5], [6, 9], [7, 10], [8, 11]]) and first.dtype == np.float32
+    assert np.array_equal(scales(), first) and reads == [1]
