@@ -415,21 +415,21 @@ class _DeviceScales:
 
 
 def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, stream: int):
-    """``_pack_entries_direct`` for entries of one shape that the direct kernel takes and that all keep something, with its
-    loops over entries in csrc/native.cpp: (units, blobs, sizes per entry, largest scales [n, 2, H] on the device); None
-    for any others."""
+    """``_pack_entries_direct`` for entries of one shape that the direct kernel takes, with its loops over entries in
+    csrc/native.cpp: ((units, blobs, sizes per entry, largest scales [n, 2, H] on the device), None) where all keep
+    something, (None, their plan as ``packing._plan_layers`` returns it) where one does not, (None, None) for any others."""
     from . import packing
     if _POISON_BLOBS or not entries[0][0].is_cuda or torch.cuda.is_current_stream_capturing():
-        return None
+        return None, None
     Ks, Vs, vbs, kbs = (list(c) for c in zip(*entries))
     n, H_kv = len(entries), int(Ks[0].shape[1])
     if len(Ks[0].shape) != 4 or any(len(t.shape) != 2 for t in vbs + kbs):
-        return None
+        return None, None
     words = _lib.host_words(dev, 12 * n * H_kv)
     planned = _lib.native.stream_order(Ks, Vs, vbs, kbs, words.take(12 * n * H_kv), words.tag, stream)
     if planned is None:
         words.pending = False           # nothing was launched
-        return None
+        return None, None
     order, plan, kb, mm = planned
     units = np.zeros(n * H_kv, dtype=UNIT_DTYPE)
     sizes, dims = np.zeros((n, 4), dtype=np.int64), np.empty((n, 5), dtype=np.int32)
@@ -437,10 +437,10 @@ def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, s
     counts, info = packing._plan_rows(words.read(dev))
     if _lib.native.stream_tables(counts, info, [int(r) * H_kv * G for r in rows_of_entries], H_kv, G, units, sizes,
                                  dims) is None:
-        return None
+        return None, (order, None, plan, counts, info, kb, mm)
     blobs = _lib.native.stream_pack(Ks, Vs, order, plan, kb, mm, units, sizes, dims, scales, stream)
     assert blobs is not None
-    return units, blobs, sizes.tolist(), scales
+    return (units, blobs, sizes.tolist(), scales), None
 
 
 def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_bytes: Optional[list] = None):
@@ -460,7 +460,7 @@ def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_
     H_q = None
     # entries by shape: one plan per group
     groups: dict = {}
-    whole = _pack_entries_native(entries, G, rows_of_entries, dev, stream) if _lib.native is not None else None
+    whole, planned = _pack_entries_native(entries, G, rows_of_entries, dev, stream) if _lib.native is not None else (None, None)
     if whole is not None:
         units_all, blobs, sizes, sm_all = whole
         if entry_bytes is not None:
@@ -494,10 +494,13 @@ def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_
                 ts = [t.to(torch.int16) for t in ts]
             return torch.cat(ts)
 
-        vb_all, kb_all = joined(2, T), joined(3, 128)
-        Ks = [entries[i][0] for i in idx]
-        order, _, plan, counts_h, info_h, kb_dev, mm_all = packing._plan_layers(
-            vb_all.reshape(-1, T), kb_all.reshape(-1, 128), dev, Ks if packing._early_minmax(Ks, dev) else (), 768)
+        if planned is None:
+            vb_all, kb_all = joined(2, T), joined(3, 128)
+            Ks = [entries[i][0] for i in idx]
+            planned = packing._plan_layers(vb_all.reshape(-1, T), kb_all.reshape(-1, 128), dev,
+                                           Ks if packing._early_minmax(Ks, dev) else (), 768)
+        order, _, plan, counts_h, info_h, kb_dev, mm_all = planned
+        planned = None                           # (made ahead, it is of entries that are one group)
         plans = []
         counts_a = np.asarray(counts_h, dtype=np.int32).reshape(-1, 4)
         chan_a = np.ascontiguousarray(np.asarray(info_h, dtype=np.int32).reshape(-1, 8)[:, 2:5])

@@ -186,3 +186,31 @@ def test_numbers_of_new_tokens(extra):
     layer.T_eff, layer.n_v16 = float(layer.T_eff), torch.tensor(float(layer.n_v16))            # (sizes of a layer made by hand)
     _, (mask,) = tz.unpack_trizone_to_past_kv(dense, head_dim=128, return_masks=True, max_new_tokens=extra)
     assert torch.equal(mask, torch.zeros(1, H * G, 1, T + max(int(extra), 0), dtype=torch.float16, device=DEV))
+
+
+def test_an_entry_that_keeps_no_channel_leaves_the_plan_to_the_others(monkeypatch):
+    """The general path takes the entries with the plan that the native call has made: none is planned again but the one
+    that is packed on its own."""
+    require_gpu()
+    g = torch.Generator(device=DEV).manual_seed(10)
+    entries = []
+    for i in range(3):
+        K, V = (torch.randn(1, H, T, 128, device=DEV, dtype=torch.float16, generator=g) for _ in range(2))
+        v_bits = torch.tensor([0, 2, 4, 8, 16], device=DEV)[torch.randint(0, 5, (H, T), device=DEV, generator=g)]
+        k_bits = torch.tensor([0, 2, 4, 8], device=DEV)[torch.randint(0, 4, (H, 128), device=DEV, generator=g)]
+        if i == 1:
+            k_bits.zero_()
+        entries.append((K, V, v_bits, k_bits))
+    plans, plan_layers = [], packing._plan_layers
+    monkeypatch.setattr(packing, "_plan_layers", lambda v, *a, **k: (plans.append(len(v)), plan_layers(v, *a, **k))[1])
+    got = stream_cache.build_stream_cache_from_kv(entries, G)
+    assert plans and set(plans) == {H}
+    monkeypatch.setattr(_lib, "native", None)
+    exp = stream_cache.build_stream_cache_from_kv(entries, G)
+    assert 3 * H in plans
+    for a, b in zip(got.blobs, exp.blobs):
+        assert torch.equal(a[:-256], b[:-256])
+    assert (got.unit_scale_max == exp.unit_scale_max).all()
+    q = torch.randn(got.rows, 128, device=DEV, dtype=torch.float16, generator=g)
+    for a, b in zip(stream_cache.decode_attn_fused(got, q), stream_cache.decode_attn_fused(exp, q)):
+        assert torch.equal(a, b)
