@@ -30,6 +30,15 @@ void rdkv_set_error(const char *fmt, ...) __attribute__((format(printf, 1, 2)));
     }                                                                               \
   } while (0)
 
+// Between lanes of one wavefront that hand values to each other through LDS.  LDS serves a wavefront in order; the fences
+// (no instructions) tell the compiler, to which a wave barrier alone touches no memory: only that it could not prove the
+// addresses apart kept one lane's reads behind another's writes.
+__device__ __forceinline__ void rdkv_wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 static inline int64_t rdkv_cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Library-internal (quantize.hip): per-channel min / max of every head's kept K rows, gathered

@@ -551,7 +551,7 @@ stream_pack_kernel(StreamPackBatch batch) {
       load_rows();
       if (ti + 2 * stride < n_tiles) load_tok(ti + 2 * stride);
     }
-    __builtin_amdgcn_wave_barrier();
+    rdkv_wave_order();
 
     // ---- K tile: rows of R dwords, chunks of up to four dwords per token, the quarter's sixteen tokens of each
     uint32_t *k_out = reinterpret_cast<uint32_t *>(a.blob + u.k_off) + (int64_t)ti * RDKV_TILE * R;
@@ -575,7 +575,7 @@ stream_pack_kernel(StreamPackBatch batch) {
     else if (cls == 1) v_tile<1>(cv, raw, nv, g, v_out);
     else if (cls == 2) v_tile<2>(cv, raw, nv, g, v_out);
     else v_tile<3>(cv, raw, nv, g, v_out);
-    __builtin_amdgcn_wave_barrier();
+    rdkv_wave_order();
   }
 
   // the head's largest V scale (as the fp16 value the decode kernel will read): one atomic per
