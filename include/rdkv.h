@@ -805,13 +805,18 @@ int rdkv_pool_scores(const float *scores, int64_t stride_b, int B, int64_t T, in
  * workspace: rdkv_knapsack_workspace_bytes(B) bytes.  Two launches (one for rows of at most
  * 256 scores in groups of at most 16), no host synchronization.
  * Batches of few long rows (max_iters <= 64; T >= 8192 and so few rows that each can have 16 or
- * more resident workgroups, or 4096 <= T < 8192 and at most 64 rows) run with every row shared by
- * 8, 16, 32 or 64 workgroups that exchange
+ * more resident workgroups, or fewer rows of 1024 <= T < 8192) run with every row shared by up to 64
+ * workgroups (rdkv_knapsack_split) that exchange
  * integer width sums once per pass of 15 doublings or four bisection levels (the first pass takes
  * the starting multiplier and the first four levels together); the same bits.  The
  * workgroups wait for each other with a bound: should a wait not end (it cannot while the launch
  * is resident as sized), the row's output is the invalid width 255 instead of a hang. */
 int64_t rdkv_knapsack_workspace_bytes(int B);
+/* How such a call is shared on a device of that many compute units: the workgroups of a row (0: rows are not
+ * shared) and the sets of 256 threads in each.  Four such launches on streams of their own, what the default hardware
+ * queues of a process run side by side, find room together; larger ones, of more than about one workgroup per compute unit
+ * and over rows of 4096 scores or more, two or three. */
+int rdkv_knapsack_split(int compute_units, int B, int64_t T, int max_iters, int n_options, int *sets);
 int rdkv_knapsack_batched(const float *scores, int64_t stride_b, int B, int64_t T,
                           const float *budget, const float *bits_host, const float *eps_host,
                           int n_options, int max_iters, float tol, int group_rows, void *out,

@@ -120,6 +120,7 @@ SIGNATURES = {
                                    P, P, P, P, P, P, P, P, P, P, P, P]),
     "rdkv_pool_scores": (I, [P, L, I, L, I, I, I, P, L, P]),
     "rdkv_knapsack_workspace_bytes": (L, [I]),
+    "rdkv_knapsack_split": (I, [I, I, L, I, I, P]),
     "rdkv_knapsack_batched": (I, [P, L, I, L, P, P, P, I, I, F, I, P, I, L, P, P, L, P]),
     "rdkv_knapsack_batched_value": (I, [P, L, I, L, F, P, I, I, L, I, P, P, I, I, F, I, P, I, L, P, P, L, P]),
     "rdkv_select_layer_start": (I, [P, L, I, L, I, I, I, P, F, P, P, I, I, P, L, P, P, L, I, F, P, P, I, P, I, F, P, P, P, P, I,

@@ -332,9 +332,9 @@ __device__ void coop_exchange(CoopCtx& c, int n, const int* mine) {
 // workgroup into red[0 .. n) (LDS, zero on entry).  se[j][k] = held score j times eps[k], +inf for
 // the options past the last (their cost is never the smallest, so all eight are walked without a
 // branch); valid[j]: the thread has a j-th score.
-template <int HELD, int NOPT, int SETS>
-__device__ void coop_chunk_sums_n(const float* __restrict__ row, const CoopCtx& c, const float (&se)[HELD][kMaxOptions],
-                                  const bool (&valid)[HELD], const float* lam, int n, const Options& o, int* red) {
+template <int HELD, int SETS, int NOPT>
+__device__ void coop_chunk_sums(const float* __restrict__ row, const CoopCtx& c, const float (&se)[HELD][NOPT],
+                                const bool (&valid)[HELD], const float* lam, int n, const Options& o, int* red) {
   // Two candidates a step (one with more than five options, whose products take too many registers): their sums go
   // through the rows of sixteen lanes as the halves of one integer (16 lanes of up to eight widths of at most 255).
   constexpr int kEach = NOPT <= 5 ? 2 : 1;
@@ -419,22 +419,17 @@ __device__ __forceinline__ void coop_midpoints(float lo, float hi, float* cand) 
   }
 }
 
-// (the options are walked to a compile-time count: the usual four or five, or all eight)
-template <int HELD, int SETS>
-__device__ void coop_chunk_sums(const float* __restrict__ row, const CoopCtx& c, const float (&se)[HELD][kMaxOptions],
-                                const bool (&valid)[HELD], const float* lam, int n, const Options& o, int* red) {
-  if (o.n <= 4) coop_chunk_sums_n<HELD, 4, SETS>(row, c, se, valid, lam, n, o, red);
-  else if (o.n == 5) coop_chunk_sums_n<HELD, 5, SETS>(row, c, se, valid, lam, n, o, red);
-  else coop_chunk_sums_n<HELD, kMaxOptions, SETS>(row, c, se, valid, lam, n, o, red);
-}
-
 __global__ void coop_init_kernel(uint32_t* state, int64_t n_words) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n_words) state[i] = 0u;
 }
 
-template <int HELD, int SETS>
-__global__ void __launch_bounds__(SETS * kCoopLanes) __attribute__((amdgpu_waves_per_eu(4)))
+// Wavefronts that a SIMD has room for: with the products of five options at most and up to four scores a thread the
+// kernel fits 64 registers without scratch (62 .. 83 with eight products always held), beyond that 128.
+constexpr int coop_waves(int held, int options) { return held <= 4 && options <= 5 ? 8 : 4; }
+// (NOPT: the options are walked to a compile-time count, the usual four or five, or all eight)
+template <int HELD, int SETS, int NOPT>
+__global__ void __launch_bounds__(SETS * kCoopLanes) __attribute__((amdgpu_waves_per_eu(coop_waves(HELD, NOPT))))
 knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int group_rows, int T, int S,
                      Budget budget, Options o, int max_iters, float tol,
                      uint32_t* __restrict__ state, void* __restrict__ out, int out_elem_size,
@@ -458,7 +453,7 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
   if (threadIdx.x == 0) failed = 0;
   const float* row = scores + (int64_t)b * stride_b;
   const float bud = budget(b);
-  float se[HELD][kMaxOptions];
+  float se[HELD][NOPT];
   bool valid[HELD];
   float m = -__builtin_inff();
 #pragma unroll
@@ -468,7 +463,7 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
     const float v = valid[j] ? row[t] : 0.f;
     if (valid[j]) m = fmaxf(m, v);
 #pragma unroll
-    for (int k = 0; k < kMaxOptions; ++k) se[j][k] = k < o.n ? __fmul_rn(v, o.eps[k]) : __builtin_inff();
+    for (int k = 0; k < NOPT; ++k) se[j][k] = k < o.n ? __fmul_rn(v, o.eps[k]) : __builtin_inff();
   }
   for (int t = c.t0 + (int)threadIdx.x + HELD * kCoopLanes; t < c.t1; t += SETS * kCoopLanes) m = fmaxf(m, row[t]);
   __syncthreads();
@@ -499,7 +494,7 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
     }
     coop_midpoints(0.f, lam0, cand + 1);
     __syncthreads();
-    coop_chunk_sums<HELD, SETS>(row, c, se, valid, cand, 17, o, red);
+    coop_chunk_sums<HELD, SETS, NOPT>(row, c, se, valid, cand, 17, o, red);
     coop_exchange<false, SETS>(c, 17, red);
     if ((int)threadIdx.x < 17) red[threadIdx.x] = 0;
     if (!(__fdiv_rn((float)tot[0], (float)T) > bud)) d = 0;
@@ -516,7 +511,7 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
       }
       __syncthreads();
       lam = cand[kCoopWords];
-      coop_chunk_sums<HELD, SETS>(row, c, se, valid, cand, n, o, red);
+      coop_chunk_sums<HELD, SETS, NOPT>(row, c, se, valid, cand, n, o, red);
       coop_exchange<false, SETS>(c, n, red);
       if ((int)threadIdx.x < n) red[threadIdx.x] = 0;
       for (int i = 0; i < n; ++i) {
@@ -605,7 +600,7 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
         if (threadIdx.x == 0) cand[0] = 0.f;   // lambda = 0 decides whether to bisect at all (first pass; unused afterwards)
         coop_midpoints(lam_lo, lam_hi, cand);
         __syncthreads();
-        coop_chunk_sums<HELD, SETS>(row, c, se, valid, cand, 16, o, red);
+        coop_chunk_sums<HELD, SETS, NOPT>(row, c, se, valid, cand, 16, o, red);
         coop_exchange<false, SETS>(c, 16, red);
         if (threadIdx.x < kCoopWords) red[threadIdx.x] = 0;
       }
@@ -642,12 +637,12 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
 
   // ---- the allocation of this workgroup's chunk and the per-option counts of the row
   {
-    float lb[kMaxOptions];
+    float lb[NOPT];
 #pragma unroll
-    for (int n = 0; n < kMaxOptions; ++n) lb[n] = n < o.n ? __fmul_rn(lam_final, o.bits[n]) : 0.f;
-    int cnt[kMaxOptions];
+    for (int n = 0; n < NOPT; ++n) lb[n] = n < o.n ? __fmul_rn(lam_final, o.bits[n]) : 0.f;
+    int cnt[NOPT];
 #pragma unroll
-    for (int n = 0; n < kMaxOptions; ++n) cnt[n] = 0;
+    for (int n = 0; n < NOPT; ++n) cnt[n] = 0;
     uint8_t* out_row = reinterpret_cast<uint8_t*>(out) + (int64_t)b * out_stride_b * out_elem_size;
     const bool bad = failed != 0;
     for (int t = c.t0 + threadIdx.x; t < c.t1; t += blockDim.x) {
@@ -655,13 +650,13 @@ knapsack_coop_kernel(const float* __restrict__ scores, int64_t stride_b, int gro
       const int idx = choose(row[t], o, lb, w);
       if (bad) w = 255;
 #pragma unroll
-      for (int n = 0; n < kMaxOptions; ++n) cnt[n] += (n == idx) ? 1 : 0;
+      for (int n = 0; n < NOPT; ++n) cnt[n] += (n == idx) ? 1 : 0;
       if (out_elem_size == 1) out_row[t] = (uint8_t)w;
       else reinterpret_cast<int64_t*>(out_row)[t] = (int64_t)w;
     }
     if (counts != nullptr) {
 #pragma unroll
-      for (int n = 0; n < kMaxOptions; ++n) {
+      for (int n = 0; n < NOPT; ++n) {
         if (n < o.n) {
           int v = cnt[n];
           v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);
@@ -1120,76 +1115,81 @@ int check_common(const void* scores, int B, int64_t T, const void* budget, const
 static int coop_held_index(int64_t chunk) { return chunk <= 2 * kCoopLanes ? 0 : (chunk <= 4 * kCoopLanes ? 1 : 2); }
 
 typedef void (*CoopKernel)(const float*, int64_t, int, int, int, Budget, Options, int, float, uint32_t*, void*, int, int64_t, int*);
-// [sets 1 / 2 / 4][scores held]
-static const CoopKernel kCoopKernels[3][3] = {
-    {knapsack_coop_kernel<2, 1>, knapsack_coop_kernel<4, 1>, knapsack_coop_kernel<8, 1>},
-    {knapsack_coop_kernel<2, 2>, knapsack_coop_kernel<4, 2>, knapsack_coop_kernel<8, 2>},
-    {knapsack_coop_kernel<2, 4>, knapsack_coop_kernel<4, 4>, knapsack_coop_kernel<8, 4>}};
+// [up to four / five / eight options][sets 1 / 2 / 4][scores held]
+#define RDKV_COOP_SETS(SETS, NOPT) {knapsack_coop_kernel<2, SETS, NOPT>, knapsack_coop_kernel<4, SETS, NOPT>, knapsack_coop_kernel<8, SETS, NOPT>}
+#define RDKV_COOP(NOPT) {RDKV_COOP_SETS(1, NOPT), RDKV_COOP_SETS(2, NOPT), RDKV_COOP_SETS(4, NOPT)}
+static const CoopKernel kCoopKernels[3][3][3] = {RDKV_COOP(4), RDKV_COOP(5), RDKV_COOP(kMaxOptions)};
 
 // Workgroups a row is shared by in the cooperative form (0: one workgroup per row, the two-launch
-// form): a power of two, chunks of at least 512 scores, at most 64 per row, the whole launch on at
-// most half of the workgroup slots the device has for the kernel variant the chunk length selects,
-// and only when that gives a row at least sixteen (with fewer, one workgroup per row was as fast or
+// form): a power of two, chunks of at least 512 scores, at most 64 per row, at most 3.5 / 2.5 / 2 workgroups per compute
+// unit by the scores held, and only when that gives a row at least sixteen (with fewer, one workgroup per row was as fast or
 // faster on 64 rows of 32k scores) - or all that its length allows for a row of 1024 .. 8191 in a launch of at
-// most kCoopShortGrid workgroups.  A call of 8 rows in two launches / shared: 1024 scores 34.6 / 22.8 us, 2048
-// 39.3 / 23.6, 3000 46.8 / 26.6, 4096 41.1 / 24.3; 64 rows of 1024 / 2048 34.6 / 23.1 and 40.9 / 24.0; 256 rows of 4096,
+// most kCoopShortGrid workgroups.  A call of 8 rows in two launches / shared: 1024 scores 34.6 / 21.7 us, 2048
+// 39.3 / 22.4, 3000 46.8 / 26.6, 4096 41.1 / 23.6; 64 rows of 1024 / 2048 34.6 / 24.7 and 40.9 / 23.5; 256 rows of 4096,
 // which would get two each, 52.4 / 58.0; 8 of 512, one each, 27.
-// kernel: the workgroups' sets (log2).  As many as leave the launch on half of the slots of their kernel, one set /
-// the rule's: 8 rows of 4096 / 16k / 31k scores 34.6 / 24.3, 36.3 / 25.7, 43.0 / 29.4, 2 of 128k 55.3 / 38.2; and a row is
-// shared by half as many where that makes room for a second set and a thread still holds its scores (8 rows of
-// 64k 44.2 -> 38.4, 16 of 32k 46.4 -> 40.3 with it).
+// kernel: the workgroups' sets (log2).  One set / the rule's: 8 rows of 4096 / 16k / 31k scores 34.6 / 23.6, 36.3 / 28.8,
+// 43.0 / 33.5, 64 rows of 2048 29.0 / 23.5; and a row is shared by half as many where that makes room for a second set and
+// a thread still holds its scores (16 rows of 16k 36.0 -> 31.9).
+// The workgroups of a launch wait for each other, so launches on streams of their own must find room together, or each
+// holds what the others wait for until the bound ends all of them.  Four run side by side on the hardware queues that a
+// process has by default.  So a launch takes sets only while it leaves room for three more like it, or, from 4096 scores
+// on, for as many as its one-set form did (two or three, for more than about one workgroup per compute unit).  Room is
+// counted in eighths of a SIMD's registers, whatever the kernel: one, two or four workgroups' wavefronts of 64 or 128
+// registers are powers of two of them, and what is short of room is never kept out by smaller pieces for good.  (Sets taken up
+// to half of a kernel's slots: three selections of 8 x 31k side by side had no room, and 2 rows of 128k took four sets,
+// 43.2 us against 44.6 now.)
 constexpr int64_t kCoopShortGrid = 512;
-static int coop_split(int B, int64_t T, int max_iters, int* kernel) {
+static int coop_split_rule(int cus, int B, int64_t T, int max_iters, int n_options, int* kernel) {
   if (B <= 0 || T < 1024 || max_iters > kCoopMaxIters) return 0;
-  // workgroup slots of the device for every kernel
-  static int slots_of_device[64][3][3];       // (0 = not asked yet; a race between first callers writes the same value)
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (slots_of_device[dev][2][2] == 0) {
-    int cus = 0, per_cu[3][3];
-    bool ok = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0;
-    for (int e = 0; e < 3; ++e)
-      for (int k = 0; k < 3; ++k)
-        ok = ok && hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu[e][k], kCoopKernels[e][k], kCoopLanes << e, 0) == hipSuccess &&
-             per_cu[e][k] > 0;
-    if (!ok) return 0;                     // (asked again next time: the query can fail while a stream is being captured)
-    for (int e = 0; e < 3; ++e)
-      for (int k = 0; k < 3; ++k) slots_of_device[dev][e][k] = cus * per_cu[e][k];
-  }
-  const int(&slots)[3][3] = slots_of_device[dev];
+  auto held_of = [T](int64_t split) { return coop_held_index((T + split - 1) / split); };
+  constexpr int kMost[3] = {7, 5, 4};            // halves of a workgroup per compute unit, by scores held
   int64_t S = T / 512;
   if (S > kCoopMaxSplit) S = kCoopMaxSplit;
-  // the launch may take half the slots of the kernel its chunk length selects (a shorter split means
-  // longer chunks, which can select the next kernel: settle in at most three steps)
+  // (a shorter split means longer chunks, which can select the next kernel: settle in at most three steps)
   // (a power of two: chunks of a whole number of scores per thread measured faster than the larger
   // split in between - 16 rows of 32k: 68 us with 32 workgroups per row, 74 us with 40)
   auto pow2_floor = [](int64_t v) { int64_t p = 1; while (2 * p <= v) p *= 2; return v >= 1 ? p : 0; };
   S = pow2_floor(S);
   const int64_t allowed = S;
   for (int step = 0; step < 3 && S >= 1; ++step) {
-    const int64_t chunk = (T + S - 1) / S;
-    const int k = coop_held_index(chunk);
-    const int64_t cap = slots[0][k] / 2 / B;
+    const int64_t cap = (int64_t)cus * kMost[held_of(S)] / 2 / B;
     if (S <= cap) break;
     S = pow2_floor(cap);
   }
+  if (S < 1 || (int64_t)B * S > (int64_t)cus * kMost[held_of(S)] / 2) return 0;
   if (S < 16 && !(T < 8192 && S == allowed && (int64_t)B * S <= kCoopShortGrid)) return 0;
-  int64_t chunk = (T + S - 1) / S;
-  if ((int64_t)B * S > slots[0][coop_held_index(chunk)] / 2) return 0;
-  auto sets_for = [&](int64_t split) {
-    const int held = coop_held_index((T + split - 1) / split);
-    for (int e = 2; e > 0; --e)
-      if ((int64_t)B * split <= slots[e][held] / 2) return e;
-    return 0;
+  const int64_t beside = T < 4096 ? 4 : std::min<int64_t>(4, (int64_t)cus * kMost[held_of(S)] / (B * S));
+  auto fits = [&](int64_t split, int e) {
+    return ((int64_t)B * split << e) * beside <= (int64_t)cus * coop_waves(2 << held_of(split), n_options);
   };
+  auto sets_for = [&](int64_t split) { return fits(split, 2) ? 2 : fits(split, 1) ? 1 : 0; };
+  if (T < 4096 && !fits(S, 0)) return 0;
   *kernel = sets_for(S);
   if (*kernel == 0 && S >= 32 && (T + S / 2 - 1) / (S / 2) <= 8 * kCoopLanes && sets_for(S / 2) > 0) {
     S /= 2;
-    chunk = (T + S - 1) / S;
     *kernel = sets_for(S);
   }
   // (a chunk's width sum must fit the 24 value bits of an exchange word)
-  return chunk <= 32768 ? (int)S : 0;
+  return (T + S - 1) / S <= 32768 ? (int)S : 0;
+}
+static int coop_split(int B, int64_t T, int max_iters, int n_options, int* kernel) {
+  if (B <= 0 || T < 1024 || max_iters > kCoopMaxIters) return 0;
+  static int cus_of_device[64];            // (0 = not asked yet; a race between first callers writes the same value)
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if (cus_of_device[dev] == 0) {
+    int cus = 0;                           // (asked again next time where it fails)
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 0;
+    cus_of_device[dev] = cus;
+  }
+  return coop_split_rule(cus_of_device[dev], B, T, max_iters, n_options, kernel);
+}
+
+RDKV_API int rdkv_knapsack_split(int compute_units, int B, int64_t T, int max_iters, int n_options, int* sets) {
+  int kernel = 0;
+  const int S = coop_split_rule(compute_units, B, T, max_iters, n_options, &kernel);
+  *sets = S ? 1 << kernel : 0;
+  return S;
 }
 
 RDKV_API int64_t rdkv_knapsack_workspace_bytes(int B) {
@@ -1221,14 +1221,14 @@ static int knapsack_batched(const float* scores, int64_t stride_b, int B, int64_
   int* doublings = reinterpret_cast<int*>(lam0 + B);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   int sets = 0;      // (log2)
-  if (const int S = coop_split(B, T, max_iters, &sets)) {
+  if (const int S = coop_split(B, T, max_iters, o.n, &sets)) {
     // few long rows: every row shared by S workgroups, one launch after clearing its state
     uint32_t* state = coop_state(workspace, B);
     const int64_t n_words = (int64_t)B * kCoopRowWords;
     if (!cleared)
       hipLaunchKernelGGL(coop_init_kernel, dim3((unsigned)rdkv_cdiv(n_words, 256)), dim3(256), 0, s, state, n_words);
     const int64_t chunk = (T + S - 1) / S;
-    hipLaunchKernelGGL(kCoopKernels[sets][coop_held_index(chunk)], dim3((unsigned)(B * S)), dim3(kCoopLanes << sets), 0, s,
+    hipLaunchKernelGGL(kCoopKernels[o.n <= 4 ? 0 : o.n == 5 ? 1 : 2][sets][coop_held_index(chunk)], dim3((unsigned)(B * S)), dim3(kCoopLanes << sets), 0, s,
                        scores, stride_b, group_rows, (int)T, S,
                        budget, o, max_iters, tol, state, out, out_elem_size, out_stride_b, counts);
     RDKV_CHECK_LAUNCH("rdkv_knapsack_batched");
@@ -1358,7 +1358,7 @@ RDKV_API int rdkv_select_layer_start(const float* scores, int64_t stride_b, int 
   int64_t row_stride = stride_b;
   if (kernel_size > 1) {
     int sets = 0;
-    cleared = coop_split(H, T, max_iters, &sets) > 0;
+    cleared = coop_split(H, T, max_iters, n_v_options, &sets) > 0;
     if (int rc = pool_scores(scores, stride_b, H, T, kernel_size, is_avg, reflect, pooled, T, cleared ? coop_state(workspace, H) : nullptr,
                              stream))
       return rc;

@@ -46,3 +46,26 @@ def test_options_and_budgets(T):
     _check(s, budget, (0, 2, 4, 8), 4, max_iters=5)
     _check(s, np.array([1.0, 6.0, 1.0, 3.0], np.float32), (2, 4, 8), 2)      # (none below 2: every doubling)
     _check(np.full((2, T), 3.0, np.float32), np.array([4.0, 300.0], np.float32), (0, 4, 255), 2)
+
+
+@pytest.mark.parametrize("B,T", [(8, 31744), (8, 16384), (2, 131072), (64, 2048), (8, 4096)])
+def test_four_launches_side_by_side(B, T):
+    """Calls on streams of their own, whose workgroups wait for each other, find room together: the results of the calls
+    alone, none with the width of a wait that was given up."""
+    require_gpu()
+    g = torch.Generator(device="cuda:0").manual_seed(T)
+    scores = [(torch.randn(B, T, generator=g, device="cuda:0") * 1.5 + 2).exp() for _ in range(4)]
+    want = [ks.knapsack_allocate(s, 2.0, ks.DEFAULT_EPSILON_V, with_counts=True) for s in scores]
+    streams = [torch.cuda.Stream() for _ in scores]
+    for stream, s in zip(streams, scores):
+        with torch.cuda.stream(stream):
+            ks.knapsack_allocate(s, 2.0, ks.DEFAULT_EPSILON_V)            # (the stream's scratch)
+    torch.cuda.synchronize()
+    got = []
+    for _ in range(20):
+        for stream, s in zip(streams, scores):
+            with torch.cuda.stream(stream):
+                got.append(ks.knapsack_allocate(s, 2.0, ks.DEFAULT_EPSILON_V, with_counts=True))
+    torch.cuda.synchronize()
+    for i, (widths, counts) in enumerate(got):
+        assert torch.equal(widths, want[i % 4][0]) and torch.equal(counts, want[i % 4][1])

@@ -524,3 +524,32 @@ def test_scales_of_several_caches_are_read_once(monkeypatch):
     first = scales()
     assert np.array_equal(first, [[0, 3], [1, 4], [2, 5], [6, 9], [7, 10], [8, 11]]) and first.dtype == np.float32
     assert np.array_equal(scales(), first) and reads == [1]
+
+
+def test_shared_rows_leave_room_for_launches_beside_theirs():
+    """The workgroups of a launch wait for each other, so launches on several streams have to find room together: as many
+    as a process has hardware queues (four), or two where the rows alone are more than a workgroup per compute unit.  Room
+    by the kernels' registers: eight wavefronts a SIMD with up to four scores a thread and five options, else four."""
+    import ctypes
+    lib, sets, found = _lib.load(), ctypes.c_int32(), set()
+    for cus in (256, 304, 64):
+        for B in (1, 2, 3, 4, 5, 8, 9, 12, 16, 24, 31, 32, 40, 64, 65, 96, 128, 200, 256, 300, 512, 1024):
+            for T in (1, 1023, 1024, 1025, 2047, 2048, 3000, 4095, 4096, 5000, 8191, 8192, 12000, 16384, 16385, 31337, 31744, 32768,
+                      40000, 65536, 65537, 100000, 131072, 131073, 400000, 1 << 20):
+                for options in (2, 4, 5, 6, 8):
+                    S = lib.rdkv_knapsack_split(cus, B, T, 64, options, ctypes.byref(sets))
+                    found.add((S, sets.value))
+                    if S == 0:
+                        assert sets.value == 0
+                        continue
+                    chunk = -(-T // S)
+                    assert T >= 1024 and S <= 64 and S & (S - 1) == 0 and sets.value in (1, 2, 4) and chunk <= 32768
+                    if sets.value == 1 and T >= 4096:                               # (a workgroup's wavefronts are one a SIMD)
+                        assert 2 * B * S <= cus * (7 if chunk <= 512 else 5 if chunk <= 1024 else 4)
+                        continue
+                    waves = 8 if chunk <= 1024 and options <= 5 else 4
+                    unshared = min(64, 1 << (T // 512).bit_length() - 1) * B        # workgroups where the device sets no limit
+                    beside = 4 if T < 4096 or unshared <= cus else 2
+                    assert beside * B * S * sets.value <= cus * waves, (cus, B, T, options, S, sets.value)
+            assert lib.rdkv_knapsack_split(cus, B, 20000, 65, 5, ctypes.byref(sets)) == 0
+    assert {1, 2, 4} <= {n for _, n in found} and {0, 2, 4, 8, 16, 32, 64} <= {S for S, _ in found}
