@@ -13,6 +13,7 @@
 #include <ATen/ops/_to_copy.h>
 #include <ATen/ops/cat.h>
 #include <ATen/ops/empty.h>
+#include <ATen/ops/full.h>
 
 #include <algorithm>
 #include <initializer_list>
@@ -496,11 +497,12 @@ PyObject *stream_tables(PyObject *const *a, Py_ssize_t) {
 }
 
 // The entries' blobs, packed; the units' offsets become addresses.  K, V, order, plan, K widths, min / max, units
-// (host), sizes, dimensions, largest scales [n][2][H], stream
+// (host), sizes, dimensions, largest scales [n][2][H], whether every byte of the blobs is set beforehand, stream
 PyObject *stream_pack(PyObject *const *a, Py_ssize_t) {
   const std::vector<at::Tensor> Ks = tensors(a[0]), Vs = tensors(a[1]);
   const at::Tensor &order = tensor(a[2]), &plan = tensor(a[3]), &kb = tensor(a[4]), &mm = tensor(a[5]), &scales = tensor(a[9]);
-  void *stream = address(a[10]);
+  const bool poison = PyObject_IsTrue(a[10]) == 1;      // (tests: a byte that the launches leave out cannot pass for a right one)
+  void *stream = address(a[11]);
   const int64_t n = Ks.size(), H = Ks[0].size(1), T = Ks[0].size(2);
   Buffer host(a[6], true), sizes(a[7]), dims(a[8]);
   auto *unit_p = host.of<RdkvUnit>(n * H);
@@ -520,7 +522,8 @@ PyObject *stream_pack(PyObject *const *a, Py_ssize_t) {
       const int32_t *d = dim_p + 5 * e;
       // (256 bytes of slack for 16-byte reads at the end; the launches write every other byte)
       const int64_t bytes = std::max<int64_t>(size_p[4 * e], 256) + 256;
-      blobs.push_back(at::empty({bytes}, Ks[e].options().dtype(at::kByte)));
+      const auto options = Ks[e].options().dtype(at::kByte);
+      blobs.push_back(poison ? at::full({bytes}, 0xAB, options) : at::empty({bytes}, options));
       layers.push_back({Ks[e].data_ptr(), Vs[e].data_ptr(), Ks[e].stride(1), Ks[e].stride(2), data<uint8_t>(blobs.back()), bytes,
                         d[3], d[0], d[1], d[2], d[4], (int32_t)size_p[4 * e + 1], 0, tiles.data() + e * H});
     }
@@ -768,7 +771,7 @@ PyMethodDef kMethods[] = {
     ENTRY(select_layer, 19, "Widths and token order of a layer: (v_bits, k_bits, order, rank3, plan, min / max, int16 widths), or None."),
     ENTRY(stream_order, 7, "Token order of the layers: (order, plan, K widths, min / max), or None."),
     ENTRY(stream_tables, 8, "Fills the units, sizes and dimensions of the layers: True, or None."),
-    ENTRY(stream_pack, 11, "The blobs of the layers, or None."),
+    ENTRY(stream_pack, 12, "The blobs of the layers, or None."),
     ENTRY(decode_attn, 16, "(out, lse) of a decode step, or None."),
     ENTRY(dense_layer, 7, "Dense (K, V) of a packed layer, with its additive mask where one is given; or None."),
     {nullptr, nullptr, 0, nullptr}};

@@ -419,7 +419,7 @@ def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, s
     csrc/native.cpp: ((units, blobs, sizes per entry, largest scales [n, 2, H] on the device), None) where all keep
     something, (None, their plan as ``packing._plan_layers`` returns it) where one does not, (None, None) for any others."""
     from . import packing
-    if _POISON_BLOBS or not entries[0][0].is_cuda or torch.cuda.is_current_stream_capturing():
+    if not entries[0][0].is_cuda or torch.cuda.is_current_stream_capturing():
         return None, None
     Ks, Vs, vbs, kbs = (list(c) for c in zip(*entries))
     n, H_kv = len(entries), int(Ks[0].shape[1])
@@ -438,7 +438,7 @@ def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, s
     if _lib.native.stream_tables(counts, info, [int(r) * H_kv * G for r in rows_of_entries], H_kv, G, units, sizes,
                                  dims) is None:
         return None, (order, None, plan, counts, info, kb, mm)
-    blobs = _lib.native.stream_pack(Ks, Vs, order, plan, kb, mm, units, sizes, dims, scales, stream)
+    blobs = _lib.native.stream_pack(Ks, Vs, order, plan, kb, mm, units, sizes, dims, scales, _POISON_BLOBS, stream)
     assert blobs is not None
     return (units, blobs, sizes.tolist(), scales), None
 

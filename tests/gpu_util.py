@@ -13,6 +13,33 @@ def require_gpu():
     _lib.load()
 
 
+class NativeCalls:
+    """Stands in for ``_lib.native`` (csrc/native.cpp): the names of the entry points that were asked, and of those that
+    took their call instead of leaving it to the general path."""
+
+    def __init__(self, native):
+        self.native, self.asked, self.taken = native, [], []
+
+    def __getattr__(self, name):
+        fn = getattr(self.native, name)
+
+        def call(*args):
+            self.asked.append(name)
+            result = fn(*args)
+            if result is not None:
+                self.taken.append(name)
+            return result
+        return call
+
+
+def record_native(monkeypatch):
+    """Records the native calls from here on."""
+    from rdkv_amd import _lib
+    calls = NativeCalls(_lib.native)
+    monkeypatch.setattr(_lib, "native", calls)
+    return calls
+
+
 def t2n(t):
     return None if t is None else t.detach().cpu().numpy()
 

@@ -22,7 +22,7 @@ from rdkv_amd import blockwise_decode as bw
 from rdkv_amd import trizone_decompress as tz
 from rdkv_amd import triton_k_kernel as kk
 from rdkv_amd import triton_v_kernel as vk
-from tests.gpu_util import (DEV, assert_bits_equal, assert_layers_equal, fused_both, lse_merge, require_gpu, t2n,
+from tests.gpu_util import (DEV, assert_bits_equal, assert_layers_equal, fused_both, lse_merge, record_native, require_gpu, t2n,
                             to_dev, with_allocation)
 
 pytestmark = pytest.mark.gpu
@@ -588,12 +588,13 @@ def test_stream_caches_random_sources_partitions_files(block, tmp_path):
 def test_direct_stream_packer_random_layers(block, monkeypatch):
     """40 calls per block of the packer that writes the streaming format directly, each over 1-4
     random layers (lengths may differ inside a call; allocations on the device or on
-    the host, in several integer types; classes missing, heads that keep nothing, constant rows,
+    the host, in several integer types, and as the native calls take them; classes missing, heads that keep nothing, constant rows,
     offsets, three magnitudes): the same unit descriptors, largest scales and blob bytes as packing
     every layer and re-laying it, on blobs that start as 0xAB bytes; every fourth call also extends
     per-layer caches by the layers as further sources, both ways."""
     monkeypatch.setattr(stream_cache, "_POISON_BLOBS", True)
     from tests.test_gpu_stream import _assert_same_cache
+    calls, packed_natively = record_native(monkeypatch), 0
     widths = np.array([0, 2, 4, 8, 16])
     for case in range(40):
         rng = np.random.default_rng(9100 + 100 * block + case)
@@ -628,9 +629,13 @@ def test_direct_stream_packer_random_layers(block, monkeypatch):
             with pytest.raises((AssertionError, ValueError, IndexError)):
                 stream_cache.build_stream_cache_from_kv(entries, G)
             continue
+        native = [(K, V, vb.to(DEV, torch.int16), kb.to(DEV, torch.int16)) for K, V, vb, kb in entries]
         try:
-            _assert_same_cache(stream_cache.build_stream_cache_from_kv(entries, G),
-                               stream_cache.build_stream_cache(packed, G))
+            want = stream_cache.build_stream_cache(packed, G)
+            _assert_same_cache(stream_cache.build_stream_cache_from_kv(entries, G), want)
+            calls.asked.clear()
+            _assert_same_cache(stream_cache.build_stream_cache_from_kv(native, G), want)
+            packed_natively += "stream_pack" in calls.asked
         except AssertionError as e:
             raise AssertionError(f"{what}: {e}") from e
         if case % 4 == 0 and same_shape:
@@ -646,6 +651,7 @@ def test_direct_stream_packer_random_layers(block, monkeypatch):
                 for f in ("unit", "tile_begin", "tile_end", "merge_unit", "merge_begin", "merge_count", "k_scale_max",
                           "v_shift"):
                     assert np.array_equal(x.work_host[f], y.work_host[f]), f
+    assert packed_natively >= 15, packed_natively          # (entries of one shape, as every second call's are, or one entry)
 
 
 def test_reference_layout_entry_points_shared_layout_and_views():

@@ -8,8 +8,8 @@ import torch
 
 from oracle import rdkv_oracle as O
 from rdkv_amd import _lib, packing, stream_cache, synth
-from tests.gpu_util import (DEV, attn_close, fused_both, layer_to_device, layer_to_oracle, lse_merge, require_gpu, t2n,
-                            to_dev)
+from tests.gpu_util import (DEV, attn_close, fused_both, layer_to_device, layer_to_oracle, lse_merge, record_native,
+                            require_gpu, t2n, to_dev)
 from tests.helpers import golden_to_oracle_layer, load_golden
 from tests.stream_decode import decode_unit
 
@@ -115,32 +115,45 @@ def _assert_same_cache(a, b):
         assert x.numel() == y.numel() and torch.equal(x, y), f"blob {i} differs"
 
 
-@pytest.fixture
-def poisoned_blobs(monkeypatch):
-    """The direct packer's blobs start as 0xAB bytes: a byte its launches leave out cannot pass for a zero."""
+@pytest.fixture(params=["native", "general"])
+def direct_packer(request, monkeypatch):
+    """The direct packer by its native calls and by the general path, whose blobs start as 0xAB bytes: a byte that the
+    launches leave out cannot pass for a zero.  Returns the device of the allocations (the native calls take them from
+    the packer's own, the general path from anywhere) and a check of which path took what was built since the last one."""
     monkeypatch.setattr(stream_cache, "_POISON_BLOBS", True)
+    calls = record_native(monkeypatch)
+    if request.param == "general":
+        monkeypatch.setattr(_lib, "native", None)
+
+    def check(packed=True):
+        assert ("stream_pack" in calls.taken) == (packed and request.param == "native")
+        calls.taken.clear()
+    return (DEV if request.param == "native" else "cpu"), check
 
 
 @pytest.mark.parametrize("name", ["perhead_d128_a", "perhead_d128_b"])
-def test_direct_stream_packer_golden(name, poisoned_blobs):
+def test_direct_stream_packer_golden(name, direct_packer):
     """fp16 K / V + allocations straight into the streaming format: every bit the reference wrote
     for the layer (its own packed tensors, stored as golden data) is found in the blob."""
     g = load_golden(name)
     G = int(g["groups"])
     ora = golden_to_oracle_layer(g, "pl")
+    where, check = direct_packer
     cache = stream_cache.build_stream_cache_from_kv(
-        [(to_dev(g["keys"]), to_dev(g["values"]), torch.from_numpy(g["v_bits"]), torch.from_numpy(g["k_bits"]))], G)
+        [(to_dev(g["keys"]), to_dev(g["values"]), *(torch.from_numpy(g[k]).to(where) for k in ("v_bits", "k_bits")))], G)
+    check()
     _assert_cache_holds_layer(cache, ora, g.get("new_v_only"))
     out, lse = stream_cache.decode_attn_fused(cache, to_dev(g["q"]))
     attn_close(t2n(out), g["out"], "out")
 
 
 @pytest.mark.parametrize("cfg_idx,ctx,layers", [(0, 700, 1), (1, 2300, 2), (2, 1500, 1), (3, 900, 2), (1, 64, 1), (0, 130, 1), (1, 32768, 1), (2, 131072, 1)])
-def test_direct_stream_packer_matches_pack_then_relayout(cfg_idx, ctx, layers, poisoned_blobs):
+def test_direct_stream_packer_matches_pack_then_relayout(cfg_idx, ctx, layers, direct_packer):
     """The direct packer's cache against packing + re-layout of the same layers: the same unit
     descriptors, largest scales and blob bytes; and the layer the oracle packs from the same CPU
     data is found in the blob."""
     cfg = synth.scaled(synth.CONFIGS[cfg_idx], context=ctx, layers=layers)
+    where, check = direct_packer
     entries, packed, oracle_layers = [], [], []
     for layer in range(layers):
         vb, kb, oc = synth.layer_allocation(cfg, layer)
@@ -148,9 +161,10 @@ def test_direct_stream_packer_matches_pack_then_relayout(cfg_idx, ctx, layers, p
         if ctx <= 700 and layer == 0:
             oracle_layers.append(O.pack_layer_per_head(K.numpy(), V.numpy(), vb.numpy(), kb.numpy(), cfg.G))
         K, V = K.to(DEV), V.to(DEV)
-        entries.append((K, V, vb, kb))
+        entries.append((K, V, vb.to(where), kb.to(where)))
         packed.append(packing.pack_layer_per_head(K, V, vb, kb, cfg.G))
     direct = stream_cache.build_stream_cache_from_kv(entries, cfg.G)
+    check()
     two_step = stream_cache.build_stream_cache(packed, cfg.G)
     _assert_same_cache(direct, two_step)
     if ctx <= 700:      # (the NumPy decoder walks the blob field by field)
@@ -158,7 +172,7 @@ def test_direct_stream_packer_matches_pack_then_relayout(cfg_idx, ctx, layers, p
         _assert_cache_holds_layer(one, *oracle_layers[0])
 
 
-def test_direct_stream_packer_ragged_and_degenerate_entries(poisoned_blobs):
+def test_direct_stream_packer_ragged_and_degenerate_entries(direct_packer):
     """Heads that keep nothing, a head that keeps only fp16 tokens, a layer where every head keeps
     the same counts (no zero rows in the K canvas: 0 must not join a min / max), inputs the direct
     kernel does not take (a strided view, fp32 values): always the bytes of packing + re-layout."""
@@ -166,8 +180,11 @@ def test_direct_stream_packer_ragged_and_degenerate_entries(poisoned_blobs):
     H, T, G = 3, 300, 2
     choices = np.array([0, 2, 4, 8, 16])
 
-    def run(K, V, vb, kb):
-        direct = stream_cache.build_stream_cache_from_kv([(K, V, vb, kb)], G)
+    where, check = direct_packer
+
+    def run(K, V, vb, kb, packed=True):
+        direct = stream_cache.build_stream_cache_from_kv([(K, V, vb.to(where), kb.to(where))], G)
+        check(packed)
         two_step = stream_cache.build_stream_cache([packing.pack_layer_per_head(K, V, vb, kb, G)], G)
         _assert_same_cache(direct, two_step)
 
@@ -186,16 +203,17 @@ def test_direct_stream_packer_ragged_and_degenerate_entries(poisoned_blobs):
     vb = torch.full((H, T), 4)                                         # one class only
     run(K, V, vb, kb)
     big = torch.randn(1, H, T, 256 + 4, device=DEV).half()             # rows 8-byte aligned only
-    run(big[..., 2:130], big[..., 130:258], torch.from_numpy(rng.choice(choices, size=(H, T))), kb)
+    run(big[..., 2:130], big[..., 130:258], torch.from_numpy(rng.choice(choices, size=(H, T))), kb, packed=False)
     kb0 = kb.clone()
     kb0[2] = 0                                                         # a head without kept channels
     run(K, V, torch.from_numpy(rng.choice(choices, size=(H, T))), kb0)
 
 
-def test_direct_stream_packer_prepares_an_unprepared_scratch(monkeypatch, poisoned_blobs):
+def test_direct_stream_packer_prepares_an_unprepared_scratch(monkeypatch):
     """Told that its scratch is not prepared, the packer starts the min / max accumulators itself:
     the same cache from a scratch full of ones as from the kept, prepared one - and the call leaves
     the scratch prepared (a second call that is told so gives the same bytes again)."""
+    monkeypatch.setattr(stream_cache, "_POISON_BLOBS", True)
     cfg = synth.scaled(synth.CONFIGS[1], context=900, layers=2)
     entries = []
     for layer in range(2):

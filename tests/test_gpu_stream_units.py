@@ -3,8 +3,8 @@ launch has threads, channel splits whose stragglers move into wider slots, rows 
 import pytest
 import torch
 
-from rdkv_amd import stream_cache
-from tests.gpu_util import DEV, require_gpu
+from rdkv_amd import _lib, stream_cache
+from tests.gpu_util import DEV, record_native, require_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -25,10 +25,13 @@ def test_blobs_equal_the_general_path(H, T, layers, monkeypatch):
             kb[h, torch.randperm(128)[:sum(splits[(h + l) % 8])]] = torch.tensor([2, 4, 8]).repeat_interleave(
                 torch.tensor(splits[(h + l) % 8]))
         entries.append((K, V, vb, kb.to(DEV)))
+    monkeypatch.setattr(stream_cache, "_POISON_BLOBS", True)
+    calls = record_native(monkeypatch)
     got = stream_cache.build_stream_cache_from_kv(entries, 2)
-    monkeypatch.setattr(stream_cache, "_POISON_BLOBS", True)             # (the general path)
+    assert "stream_pack" in calls.taken
+    monkeypatch.setattr(_lib, "native", None)                            # (the general path)
     exp = stream_cache.build_stream_cache_from_kv(entries, 2)
-    assert all(torch.equal(a[:-256], b[:-256]) for a, b in zip(got.blobs, exp.blobs))
+    assert all(torch.equal(a, b) for a, b in zip(got.blobs, exp.blobs))
     assert (got.unit_scale_max == exp.unit_scale_max).all()
     q = torch.randn(got.rows, 128, device=DEV, dtype=torch.float16, generator=g)
     for a, b in zip(stream_cache.decode_attn_fused(got, q), stream_cache.decode_attn_fused(exp, q)):
