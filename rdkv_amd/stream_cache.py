@@ -386,21 +386,6 @@ def _direct_packable(K: torch.Tensor, V: torch.Tensor) -> bool:
             and K.data_ptr() % 16 == 0 and V.data_ptr() % 16 == 0)
 
 
-_pack_scratch_of: dict = {}
-_SCRATCH_PREPARED = 1        # what the packer is told about its scratch (tests hand it an unprepared one)
-
-
-def _pack_scratch(dev, stream: int, H_kv: int) -> torch.Tensor:
-    """The direct packer's scratch (min / max accumulators and channel quantizers of one layer's
-    heads), one per device, stream and head count: prepared when made, left ready by every call."""
-    key = (dev.index, stream, H_kv)
-    t = _pack_scratch_of.get(key)
-    if t is None:
-        t = _pack_scratch_of[key] = torch.empty(H_kv * 768, dtype=torch.float32, device=dev)
-        _lib.check(_lib.load().rdkv_pack_layer_stream_ws_init(t.data_ptr(), H_kv, stream))
-    return t
-
-
 class _DeviceScales:
     """The largest scales [entries, 2, heads] that launches still running leave on the device; called: as rows of units,
     fp32 [entries * heads, 2], on the host (the first call synchronizes, the caches of several entries ask one by one)."""
@@ -497,8 +482,7 @@ def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_
         if planned is None:
             vb_all, kb_all = joined(2, T), joined(3, 128)
             Ks = [entries[i][0] for i in idx]
-            planned = packing._plan_layers(vb_all.reshape(-1, T), kb_all.reshape(-1, 128), dev,
-                                           Ks if packing._early_minmax(Ks, dev) else (), 768)
+            planned = packing._plan_layers(vb_all.reshape(-1, T), kb_all.reshape(-1, 128), dev, Ks, 768)
         order, _, plan, counts_h, info_h, kb_dev, mm_all = planned
         planned = None                           # (made ahead, it is of entries that are one group)
         plans = []
@@ -530,7 +514,6 @@ def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_
         live = [p for p in plans if p is not None]
         if live:
             units_dev, src_dev = _lib.upload(dev, units_grp[:n_live * H_kv], src_grp[:n_live * H_kv])
-            mm = _pack_scratch(dev, stream, H_kv) if mm_all is None else None
             sm_all = torch.empty(len(live), 2, H_kv, dtype=torch.float32, device=dev)
         row = 0
         for j, (i, p) in enumerate(zip(idx, plans)):
@@ -556,8 +539,7 @@ def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_
                 kb_dev.element_size(), kb_dev.stride(0),
                 n2p, n4p, m8, max_tv, max_n16, units_dev.data_ptr() + row * UNIT_DTYPE.itemsize,
                 src_dev.data_ptr() + row * src_tab.shape[1] * 2, src_tab.shape[1], max_tiles, base, blob_bytes,
-                mm.data_ptr() if mm is not None else mm_all.data_ptr() + 4 * 768 * j * H_kv,
-                _SCRATCH_PREPARED if mm is not None else 2, sm_all.data_ptr() + 4 * k * sm_all.stride(0), stream))
+                mm_all.data_ptr() + 4 * 768 * j * H_kv, 2, sm_all.data_ptr() + 4 * k * sm_all.stride(0), stream))
             row += H_kv
             _add_base(units, base)
             pending.append((i, units, blob, sm_all[k], sb, ab, None))

@@ -209,24 +209,38 @@ def test_direct_stream_packer_ragged_and_degenerate_entries(direct_packer):
     run(K, V, torch.from_numpy(rng.choice(choices, size=(H, T))), kb0)
 
 
-def test_direct_stream_packer_prepares_an_unprepared_scratch(monkeypatch):
-    """Told that its scratch is not prepared, the packer starts the min / max accumulators itself:
-    the same cache from a scratch full of ones as from the kept, prepared one - and the call leaves
-    the scratch prepared (a second call that is told so gives the same bytes again)."""
-    monkeypatch.setattr(stream_cache, "_POISON_BLOBS", True)
-    cfg = synth.scaled(synth.CONFIGS[1], context=900, layers=2)
-    entries = []
-    for layer in range(2):
-        vb, kb, oc = synth.layer_allocation(cfg, layer)
-        K, V, _ = synth.layer_data(cfg, layer, DEV, outliers=oc)
-        entries.append((K, V, vb.to(DEV), kb.to(DEV)))
-    want = stream_cache.build_stream_cache_from_kv(entries, cfg.G)
-    dirty = torch.ones(cfg.H_kv * 768, dtype=torch.float32, device=DEV)
-    monkeypatch.setattr(stream_cache, "_pack_scratch", lambda dev, stream, H_kv: dirty)
-    monkeypatch.setattr(stream_cache, "_SCRATCH_PREPARED", 0)
-    _assert_same_cache(stream_cache.build_stream_cache_from_kv(entries, cfg.G), want)
-    monkeypatch.setattr(stream_cache, "_SCRATCH_PREPARED", 1)
-    _assert_same_cache(stream_cache.build_stream_cache_from_kv(entries, cfg.G), want)
+def test_direct_stream_packer_prepares_an_unprepared_scratch():
+    """``rdkv_pack_layer_stream`` and its scratch: told that it is not prepared, the call starts the min / max accumulators
+    itself (in a scratch full of ones) and leaves them ready for the next, which may be told so; prepared by
+    ``rdkv_pack_layer_stream_ws_init``; and with the accumulators complete, as ``rdkv_pack_layers_k_minmax`` leaves them.
+    The same blob and scales each time, those of the whole cache."""
+    cfg = synth.scaled(synth.CONFIGS[1], context=900, layers=1)
+    H, lib, stream = cfg.H_kv, _lib.load(), _lib.stream_of(torch.device(DEV))
+    vb, kb, oc = synth.layer_allocation(cfg, 0)
+    K, V, _ = synth.layer_data(cfg, 0, DEV, outliers=oc)
+    vb, kb = vb.to(DEV), kb.to(DEV)
+    cache = stream_cache.build_stream_cache_from_kv([(K, V, vb, kb)], cfg.G)
+    order, _, plan, counts, info, kb_dev, complete = packing._plan_layers(vb, kb, K.device, (K,), 768)
+    counts, chans = np.asarray(counts, dtype=np.int32), np.ascontiguousarray(np.asarray(info, dtype=np.int32)[:, 2:5])
+    n2p, n4p, n8 = -(-chans[:, 0].max() // 4) * 4, -(-chans[:, 1].max() // 2) * 2, chans[:, 2].max()
+    units, src = np.zeros(H, dtype=stream_cache.UNIT_DTYPE), np.empty((H, 4 * stream_cache.MAX_STEPS), dtype=np.int16)
+    sizes = np.zeros(4, dtype=np.int64)
+    _lib.check(lib.rdkv_stream_plan_layer(counts.ctypes.data, 4, chans.ctypes.data, 3, H, n2p, n4p, 0, cfg.G, units.ctypes.data,
+                                          src.ctypes.data, src.shape[1], sizes.ctypes.data))
+    units_dev, src_dev = _lib.upload(K.device, units, src)
+    blob_bytes = max(int(sizes[0]), 256) + 256
+    ones, prepared = (torch.ones(H * 768, dtype=torch.float32, device=DEV) for _ in range(2))
+    _lib.check(lib.rdkv_pack_layer_stream_ws_init(prepared.data_ptr(), H, stream))
+    for ready, scratch in ((0, ones), (1, ones), (0, ones), (1, prepared), (1, prepared), (2, complete)):
+        blob = torch.full((blob_bytes,), 0xAB, dtype=torch.uint8, device=DEV)
+        scales = torch.full((2, H), -1.0, device=DEV)
+        _lib.check(lib.rdkv_pack_layer_stream(
+            K.data_ptr(), V.data_ptr(), K.stride(1), K.stride(2), H, order.data_ptr(), order.stride(0), plan.data_ptr(),
+            kb_dev.data_ptr(), kb_dev.element_size(), kb_dev.stride(0), n2p, n4p, n8, int(counts[:, :3].sum(axis=1).max()),
+            int(counts[:, 3].max()), units_dev.data_ptr(), src_dev.data_ptr(), src.shape[1], int(sizes[1]), blob.data_ptr(),
+            blob_bytes, scratch.data_ptr(), ready, scales.data_ptr(), stream))
+        assert torch.equal(blob, cache.blobs[0]), ready
+        assert np.array_equal(t2n(scales).T, cache.unit_scale_max), ready
 
 
 @pytest.mark.parametrize("name", ["perhead_d128_a", "perhead_d128_b", "shared_layout"])

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from rdkv_amd import _lib, fast_decode, packing, stream_cache, trizone_decompress as tz
-from tests.gpu_util import DEV, require_gpu
+from tests.gpu_util import DEV, record_native, require_gpu
 
 gpu = pytest.mark.gpu
 
@@ -205,9 +205,15 @@ def test_minmax_ahead_of_the_read(monkeypatch, T, D, form):
         layers = packing.pack_layers_per_head(Ks, Vs, vb, kb, 2)
         layers += [packing.pack_layer_per_head(Ks[1], Vs[1], vb[1], kb[1], 2)]
         cache = None
-        if D == 128:
-            cache = stream_cache.build_stream_cache_from_kv(
-                [(K, V, vb[l], kb[l]) for l, (K, V) in enumerate(zip(Ks, Vs))], 2)
+        if D == 128:            # (the streaming packer takes them ahead always: by its native calls, by the general path)
+            with monkeypatch.context() as m:
+                if tokens == 1:
+                    calls = record_native(m)
+                else:
+                    m.setattr(_lib, "native", None)
+                cache = stream_cache.build_stream_cache_from_kv(
+                    [(K, V, vb[l], kb[l]) for l, (K, V) in enumerate(zip(Ks, Vs))], 2)
+            assert ("stream_pack" in calls.taken) == (form != "odd")
         got.append((layers, cache))
     for (a, va), (b, vb_) in zip(got[0][0], got[1][0]):
         _same(a, b)
