@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from rdkv_amd import _lib, packing, trizone_decompress as tz
-from tests.gpu_util import DEV, require_gpu
+from tests.gpu_util import DEV, NativeCalls, require_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -31,12 +31,13 @@ def test_one_launch_equals_the_general_path(T, H, D, extra, whole, monkeypatch):
     assert pl.softmax_mask is not None and pl.softmax_mask.dtype == torch.float32
     pl.softmax_mask[0, 0] = -1e30
     cache = packing.TriZoneCache((pl,), [v16], [None], [None], T)
-    results = []
-    for native in (_lib.native, None):
+    results, calls = [], NativeCalls(_lib.native)
+    for native in (calls, None):
         with monkeypatch.context() as m:
             m.setattr(_lib, "native", native)
             ((k, v),), (mask,) = tz.unpack_trizone_to_past_kv(cache, head_dim=D, return_masks=True, H_q=4 * H, max_new_tokens=extra)
             results.append((k, v, mask))
+    assert calls.taken == ["dense_layer"]
     for a, b in zip(*results):
         assert a.shape == b.shape and a.dtype == b.dtype == torch.float16
         assert torch.equal(a.view(torch.int16), b.view(torch.int16))

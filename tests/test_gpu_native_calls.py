@@ -10,7 +10,7 @@ import torch
 from torch.utils._python_dispatch import TorchDispatchMode
 
 from rdkv_amd import _lib, knapsack_solver as ks, obkv_fast, packing, stream_cache, trizone_decompress as tz
-from tests.gpu_util import DEV, require_gpu
+from tests.gpu_util import DEV, record_native, require_gpu
 
 pytestmark = pytest.mark.gpu
 H, T, G = 2, 300, 4
@@ -36,7 +36,7 @@ def _no_memory_left():
 
 @pytest.fixture(scope="module")
 def calls():
-    """By entry point: (the function of the module that it has to reach, the call)."""
+    """By the entry point that it has to reach: the call."""
     require_gpu()
     g = torch.Generator(device=DEV).manual_seed(5)
     K, V = (torch.randn(1, H, T, 128, device=DEV, dtype=torch.float16, generator=g) for _ in range(2))
@@ -59,27 +59,16 @@ def calls():
     }
 
 
-class _Reached:
-    """The module, with the names of the functions that were called."""
-
-    def __init__(self, native):
-        self.native, self.names = native, []
-
-    def __getattr__(self, name):
-        self.names.append(name)
-        return getattr(self.native, name)
-
-
 @pytest.mark.parametrize("name", ["select_layer", "pack_layer", "stream_order", "dense_layer", "decode_attn"])
 def test_out_of_memory(calls, name, monkeypatch):
-    reached = _Reached(_lib.native)
-    monkeypatch.setattr(_lib, "native", reached)
+    reached = record_native(monkeypatch)
     want = calls[name]().clone()
-    reached.names.clear()
+    assert name in reached.taken
+    reached.asked.clear()
     with _no_memory_left():
         with pytest.raises(torch.OutOfMemoryError):
             calls[name]()
-        assert reached.names == [name]
+        assert reached.asked == [name]
     assert torch.equal(calls[name](), want)
 
 

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from rdkv_amd import _lib, packing
-from tests.gpu_util import DEV, require_gpu
+from tests.gpu_util import DEV, NativeCalls, require_gpu
 
 pytestmark = pytest.mark.gpu
 
@@ -27,12 +27,13 @@ def test_one_launch_equals_the_general_path(T, H, G, widths, dtype, monkeypatch)
     if H > 2:
         vb[-1], kb[-2] = 0, 0                # a head without tokens, one without channels
     kb = torch.cat([kb, kb], dim=1).to(dtype)[:, :128]
-    results = []
-    for native, early in ((_lib.native, 1), (None, 1 << 30)):
+    results, calls = [], NativeCalls(_lib.native)
+    for native, early in ((calls, 1), (None, 1 << 30)):
         with monkeypatch.context() as m:
             m.setattr(_lib, "native", native)
             m.setattr(packing, "_EARLY_MINMAX_TOKENS", early)
             results.append(packing.pack_layer_per_head(K, V, vb, kb, G))
+    assert calls.taken == ["pack_layer"]
     (a, a16), (b, b16) = results
     assert (a16 is None) == (b16 is None) and (a16 is None or torch.equal(a16, b16))
     for name in a.__dataclass_fields__:

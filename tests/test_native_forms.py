@@ -1,13 +1,13 @@
 """The host side in C++ (csrc/native.cpp) against the Python it stands in for, which takes every form that it leaves: the
 same tensors, bit for bit, over the layouts, types and options that it takes, and the general path's own results and
-errors over those that it does not."""
+errors over those that it does not.  Which of the two took a call is asserted."""
 import dataclasses
 
 import pytest
 import torch
 
 from rdkv_amd import _lib, knapsack_solver as ks, obkv_fast, packing, stream_cache, trizone_decompress as tz
-from tests.gpu_util import DEV, require_gpu
+from tests.gpu_util import DEV, record_native, require_gpu
 
 gpu = pytest.mark.gpu
 
@@ -62,17 +62,26 @@ def test_selection(monkeypatch, layout, H, G, T, pool):
         args = dict(gqa_factor=G, token_budget=max(T // 3, 1), k_budget_ratio=0.5, obs_window=32, pool_kernel_size=pool[1],
                     pool_padding=pool[2], pool_type=pool[0], v_bit_options=torch.tensor([0.0, 2.0, 4.0, 8.0]) if layout == "f32 V" else None,
                     k_bit_options=k_options, eps_V=ks.DEFAULT_EPSILON_V, eps_K=ks.DEFAULT_EPSILON_K, retain_allocation_metadata=H != 3)
-        got = obkv_fast._perhead_select_and_pack(K, V, tokens, channels, **args)
+        with monkeypatch.context() as m:
+            calls = record_native(m)
+            got = obkv_fast._perhead_select_and_pack(K, V, tokens, channels, **args)
+            plain = [] if layout == "f32 V" else ["select_layer", "pack_layer"] if K.stride() == V.stride() else ["select_layer"]
+            assert calls.taken == plain
         with monkeypatch.context() as m:
             m.setattr(obkv_fast, "_select_and_pack_native", lambda *a: None)
             m.setattr(_lib, "native", None)
             exp = obkv_fast._perhead_select_and_pack(K, V, tokens, channels, **args)
         for f in dataclasses.fields(packing.PackedKVLayer):
             assert _same(getattr(got[0], f.name), getattr(exp[0], f.name)), f.name
-        assert _same(got[1], exp[1]) and got[2] == exp[2] and got[0]._host_counts == exp[0]._host_counts if layout != "f32 V" else True
+        assert _same(got[1], exp[1]) and got[2] == exp[2]
+        if "pack_layer" in plain:
+            assert got[0]._host_counts == exp[0]._host_counts
         # the dense tensors of that layer
         cache = packing.TriZoneCache((got[0],), [got[1]], [None], [None], T)
-        a = tz.unpack_trizone_to_past_kv(cache, head_dim=128)
+        with monkeypatch.context() as m:
+            calls = record_native(m)
+            a = tz.unpack_trizone_to_past_kv(cache, head_dim=128)
+            assert calls.taken == ["dense_layer"]
         with monkeypatch.context() as m:
             m.setattr(_lib, "native", None)
             b = tz.unpack_trizone_to_past_kv(cache, head_dim=128)
@@ -140,7 +149,10 @@ def test_decode_step(monkeypatch, G, q_dtype):
         return out, lse, buf
 
     for form in forms:
-        got = run(form)
+        with monkeypatch.context() as m:
+            calls = record_native(m)
+            got = run(form)
+            assert calls.taken == ([] if q_dtype is torch.float64 else ["decode_attn"])
         with monkeypatch.context() as m:
             m.setattr(_lib, "native", None)
             exp = run(form)
@@ -172,13 +184,19 @@ def test_layers_to_the_streaming_format(monkeypatch, widths, T, layers, layout):
     for empty_layer in (False, True) if T == 65 else (False,):
         if empty_layer:
             entries[-1] = (*entries[-1][:3], torch.zeros_like(entries[-1][3]))
-        monkeypatch.setattr(stream_cache, "_POISON_BLOBS", False)
-        got = stream_cache.build_stream_cache_from_kv(entries, G)
-        monkeypatch.setattr(stream_cache, "_POISON_BLOBS", True)             # (the general path)
-        exp = stream_cache.build_stream_cache_from_kv(entries, G)
+        monkeypatch.setattr(stream_cache, "_POISON_BLOBS", True)
+        with monkeypatch.context() as m:
+            calls = record_native(m)
+            got = stream_cache.build_stream_cache_from_kv(entries, G)
+            plain = layout != "apart" and widths is not torch.float32
+            assert calls.taken == ([] if not plain else ["stream_order"] if empty_layer else ["stream_order", "stream_tables", "stream_pack"])
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "native", None)                                  # (the general path)
+            exp = stream_cache.build_stream_cache_from_kv(entries, G)
         assert len(got.blobs) == len(exp.blobs) == layers
-        for a, b in zip(got.blobs, exp.blobs):
-            assert torch.equal(a[:-256], b[:-256]) and a.shape == b.shape
+        for i, (a, b) in enumerate(zip(got.blobs, exp.blobs)):
+            end = -256 if empty_layer and i == layers - 1 or not plain else None      # (the re-layout leaves its slack)
+            assert torch.equal(a[:end], b[:end]) and a.shape == b.shape
         for name in ("n_units", "n_work", "rows", "stream_bytes", "algorithmic_bytes", "max_row_dwords", "row_shape", "n_groups",
                      "kv_algorithmic_bytes", "h_q"):
             assert getattr(got, name) == getattr(exp, name), name
