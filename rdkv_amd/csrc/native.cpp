@@ -295,7 +295,7 @@ PyObject *pack_layer(PyObject *const *a, Py_ssize_t) {
 }
 
 // ---- a layer's selection up to its token order (obkv_fast._perhead_select_and_pack_joint) --------------------------
-// K, V, token scores, channel scores, (kernel, average, reflect), V widths, V errors, V budget, K widths, K errors, K bits
+// K, V, token scores, channel scores, (kernel, average, reflect, iterations, tolerance), V widths, V errors, V budget, K widths, K errors, K bits
 // of a head, the column of the V width 0, tokens from which K min / max go ahead, keep the widths, host words, tag,
 // workspace, its bytes, stream
 PyObject *select_layer(PyObject *const *a, Py_ssize_t) {
@@ -306,9 +306,10 @@ PyObject *select_layer(PyObject *const *a, Py_ssize_t) {
   plain(H >= 1 && H <= 65535 && T >= 1 && T <= (1 << 20) && D >= 1);
   plain(scores.scalar_type() == at::kFloat && shape_is(scores, {H, T}) && scores.stride(1) == 1);
   plain(channels.scalar_type() == at::kFloat && shape_is(channels, {H, D}) && channels.stride(1) == 1);
-  plain(PyTuple_Check(a[4]) && PyTuple_GET_SIZE(a[4]) == 3);
+  plain(PyTuple_Check(a[4]) && PyTuple_GET_SIZE(a[4]) == 5);
   const int64_t kernel = integer(PyTuple_GET_ITEM(a[4], 0)), average = integer(PyTuple_GET_ITEM(a[4], 1)),
-                reflect = integer(PyTuple_GET_ITEM(a[4], 2));
+                reflect = integer(PyTuple_GET_ITEM(a[4], 2)), iters = integer(PyTuple_GET_ITEM(a[4], 3));
+  const float tol = (float)real(PyTuple_GET_ITEM(a[4], 4));
   const std::vector<float> v_bits = reals(a[5]), v_eps = reals(a[6]), k_bits = reals(a[8]), k_eps = reals(a[9]);
   plain(v_bits.size() >= 1 && v_bits.size() <= 8 && k_bits.size() >= 1 && k_bits.size() <= 8);
   const double v_avg = real(a[7]), k_kept = real(a[10]);
@@ -342,7 +343,7 @@ PyObject *select_layer(PyObject *const *a, Py_ssize_t) {
       rc = lib.rdkv_select_layer_start(rows, row_stride, H, T, kernel, average, reflect, data<float>(pooled), (float)v_avg,
                                        v_bits.data(), v_eps.data(), v_bits.size(), zero_col, data<uint8_t>(vb), T16,
                                        data<int32_t>(counts), data<float>(channels), channels.stride(0), D, (float)k_kept,
-                                       k_bits.data(), k_eps.data(), k_bits.size(), data<uint8_t>(kb), 64, 0.01f, data<int32_t>(order),
+                                       k_bits.data(), k_eps.data(), k_bits.size(), data<uint8_t>(kb), iters, tol, data<int32_t>(order),
                                        data<int32_t>(rank3), data<int32_t>(plan), data<float>(mm), early ? 2 * D : 0,
                                        data<int16_t>(v16), data<int16_t>(k16), words, tag, ws, ws_bytes, stream);
       vb = vb.narrow(1, 0, T);
@@ -355,13 +356,13 @@ PyObject *select_layer(PyObject *const *a, Py_ssize_t) {
     if (rc == RDKV_OK && !together) {
       vb = make({H, T}, at::kByte), counts = make({H, (int64_t)v_bits.size()}, at::kInt);
       rc = lib.rdkv_knapsack_batched_value(rows, row_stride, H, T, (float)v_avg, nullptr, 0, 0, 0, 0, v_bits.data(), v_eps.data(),
-                                           v_bits.size(), 64, 0.01f, 0, data(vb), 1, T, data<int32_t>(counts), ws, ws_bytes,
+                                           v_bits.size(), iters, tol, 0, data(vb), 1, T, data<int32_t>(counts), ws, ws_bytes,
                                            stream);
     }
     if (rc == RDKV_OK && !together) {
       kb = make({H, D}, at::kByte);
       rc = lib.rdkv_knapsack_batched_value(data<float>(channels), channels.stride(0), H, D, (float)k_kept, data<int32_t>(counts),
-                                           v_bits.size(), zero_col, T, D, k_bits.data(), k_eps.data(), k_bits.size(), 64, 0.01f,
+                                           v_bits.size(), zero_col, T, D, k_bits.data(), k_eps.data(), k_bits.size(), iters, tol,
                                            0, data(kb), 1, D, nullptr, ws, ws_bytes, stream);
     }
     if (rc == RDKV_OK && !together) {

@@ -22,6 +22,7 @@ DEFAULT_EPSILON: Dict[int, float] = {0: 1.0, 2: 0.25, 4: 0.011, 8: 0.000057, 16:
 DEFAULT_EPSILON_K: Dict[int, float] = {0: 1.0, 2: 0.277, 4: 0.011, 8: 0.000061, 16: 0.0}
 DEFAULT_EPSILON_V: Dict[int, float] = {0: 1.0, 2: 0.312, 4: 0.0138, 8: 0.000048, 16: 0.0}
 BITS = torch.tensor([0, 2, 4, 8, 16], dtype=torch.float32)
+MAX_ITERS, TOLERANCE = 64, 0.01        # of an allocation that names no others
 
 
 def option_lists(epsilon: Dict[int, float], bit_options: Optional[Tensor]):
@@ -53,8 +54,8 @@ class KeptBudget(NamedTuple):
     bits: float
 
 
-def knapsack_allocate(scores: Tensor, budget_per_token: Union[float, Tensor, KeptBudget], epsilon=None, max_iters: int = 64,
-                      tol: float = 0.01, bit_options: Optional[Tensor] = None, *, out_dtype=torch.uint8,
+def knapsack_allocate(scores: Tensor, budget_per_token: Union[float, Tensor, KeptBudget], epsilon=None,
+                      max_iters: int = MAX_ITERS, tol: float = TOLERANCE, bit_options: Optional[Tensor] = None, *, out_dtype=torch.uint8,
                       with_counts: bool = False, group_rows: int = 0):
     """``knapsack_bit_allocation_batched`` with the output type of the caller's choice (uint8 for
     the packer, int64 for the reference's return type) and, on request, the per-row number of
@@ -96,15 +97,15 @@ def knapsack_allocate(scores: Tensor, budget_per_token: Union[float, Tensor, Kep
 
 
 def knapsack_bit_allocation_batched(scores: Tensor, budget_per_token: Union[float, Tensor],
-                                    epsilon: Optional[Dict[int, float]] = None, max_iters: int = 64,
-                                    tol: float = 0.01, bit_options: Optional[Tensor] = None) -> Tensor:
+                                    epsilon: Optional[Dict[int, float]] = None, max_iters: int = MAX_ITERS,
+                                    tol: float = TOLERANCE, bit_options: Optional[Tensor] = None) -> Tensor:
     """knapsack_solver.py:121-248.  ``scores [B, T]``, budget a float or ``[B]`` tensor; returns a
     ``[B, T]`` LongTensor with values from ``bit_options`` (default {0,2,4,8,16})."""
     return knapsack_allocate(scores, budget_per_token, epsilon, max_iters, tol, bit_options, out_dtype=torch.int64)
 
 
 def knapsack_bit_allocation(scores: Tensor, budget_per_token: float, epsilon: Optional[Dict[int, float]] = None,
-                            max_iters: int = 64, tol: float = 0.01,
+                            max_iters: int = MAX_ITERS, tol: float = TOLERANCE,
                             bit_options: Optional[Tensor] = None) -> Tensor:
     """knapsack_solver.py:39-118: one row ``[num_tokens]``, lambda bisected in double."""
     if epsilon is None:
@@ -123,8 +124,8 @@ def knapsack_bit_allocation(scores: Tensor, budget_per_token: float, epsilon: Op
 
 
 def allocate_v_bits_with_fp16_topk(scores: Tensor, budget_per_token: float, fp16_topk: int = 0,
-                                   epsilon: Optional[Dict[int, float]] = None, max_iters: int = 64,
-                                   tol: float = 0.01,
+                                   epsilon: Optional[Dict[int, float]] = None, max_iters: int = MAX_ITERS,
+                                   tol: float = TOLERANCE,
                                    bit_options: Optional[Tensor] = None) -> Tuple[Tensor, Dict[str, Any]]:
     """knapsack_solver.py:251-367: reserve the ``fp16_topk`` highest scores for 16 bits, solve the
     rest with the remaining budget; same fallbacks, warnings and diagnostics."""

@@ -16,7 +16,7 @@ import torch
 from torch import Tensor
 
 from . import _lib, packing
-from .knapsack_solver import (DEFAULT_EPSILON_K, DEFAULT_EPSILON_V, KeptBudget, knapsack_allocate,   # noqa: F401 (re-exported
+from .knapsack_solver import (DEFAULT_EPSILON_K, DEFAULT_EPSILON_V, MAX_ITERS, TOLERANCE, KeptBudget, knapsack_allocate,   # noqa: F401 (re-exported
                               knapsack_bit_allocation_batched, load_epsilon_kv_from_calibration, option_lists)  # as obkv_fast.py:38-46 does)
 from .packing import _pack_layer_per_head, pack_layer_per_head, pack_layers_per_head  # noqa: F401 (its public name stays here)
 
@@ -123,7 +123,8 @@ def _select_and_pack_native(K, V, layer_scores, channel_scores, gqa_factor, toke
     words = _lib.host_words(dev, 12 * H_kv)
     stream = _lib.stream_of(dev)
     chosen = _lib.native.select_layer(
-        K, V, layer_scores, channel_scores, (int(pool_kernel_size), int(pool_type == "avg"), int(pool_padding == "reflect")),
+        K, V, layer_scores, channel_scores,
+        (int(pool_kernel_size), int(pool_type == "avg"), int(pool_padding == "reflect"), MAX_ITERS, TOLERANCE),
         v_widths, v_errors, v_avg, k_widths, k_errors, float(k_budget_ratio * total_budget_bits),
         v_widths.index(0.0) if 0.0 in v_widths else -1, packing._EARLY_MINMAX_TOKENS, retain, words.take(12 * H_kv), words.tag,
         ws.data_ptr(), ws.numel(), stream)
