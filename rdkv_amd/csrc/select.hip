@@ -234,7 +234,7 @@ knapsack_bisect_kernel(const float* __restrict__ scores, int64_t stride_b, int g
 // A workgroup is one, two or four sets of kCoopLanes threads (SETS).  Every set holds the whole chunk and takes its
 // share of a pass's candidates: a pass is bound by its chain of vector instructions (3.5 ns each where they depend), and
 // one set leaves a SIMD a wavefront or less.  With the midpoints and the way down their tree taken by lanes instead of
-// one thread in turn, a call of 8 rows of 4k / 31k scores 34.6 / 43.0 -> 24.2 / 29.5 us (four / two sets).
+// one thread in turn, a call of 8 rows of 4k / 31k scores 34.6 / 43.0 -> 23.6 / 33.4 us (four / two sets).
 constexpr int kCoopLanes = 256;
 constexpr int kCoopMaxSplit = 64;          // workgroups per row at most
 constexpr int kCoopWords = 32;             // words a workgroup can publish per pass (17 are used at most)
@@ -425,7 +425,8 @@ __global__ void coop_init_kernel(uint32_t* state, int64_t n_words) {
 }
 
 // Wavefronts that a SIMD has room for: with the products of five options at most and up to four scores a thread the
-// kernel fits 64 registers without scratch (62 .. 83 with eight products always held), beyond that 128.
+// kernel fits 64 registers (two of one set's, five options, go to scratch; 62 .. 83 with eight products always held), beyond
+// that 128.
 constexpr int coop_waves(int held, int options) { return held <= 4 && options <= 5 ? 8 : 4; }
 // (NOPT: the options are walked to a compile-time count, the usual four or five, or all eight)
 template <int HELD, int SETS, int NOPT>

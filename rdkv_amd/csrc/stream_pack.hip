@@ -7,12 +7,12 @@
 // re-quantizes K from (packing.py:1186-1215: a head with fewer rows than the layer's maxima has
 // zero rows there, so 0 joins its per-channel min / max).
 //
-// Three launches: the per-channel K min / max of every head (quantize.hip), one small workgroup per
-// head that turns them into the quantizer of every channel and writes the unit's slot table, and one
-// workgroup per (64-token tile, KV head) that reads the tile's K and V rows (gathered through the
-// head's class-sorted token order) with 16-byte loads, every request out before the first is used,
-// quantizes them in registers, parks the codes in LDS as bytes and assembles the tile's dwords from
-// there.  Between them the launches write every byte of the blob.
+// Three launches for up to eight layers: the per-channel K min / max of every head (quantize.hip), one small
+// workgroup per head that turns them into the quantizer of every channel and writes the unit's slot table, and
+// resident workgroups that walk the heads' 64-token tiles, a quarter of a tile to each wavefront: it reads its tokens'
+// K and V rows (gathered through the head's class-sorted token order) with 16-byte loads, quantizes them in
+// registers, parks the codes in LDS as bytes, requests the next tile's rows and assembles this one's dwords from LDS
+// meanwhile.  Between them the launches write every byte of the blob.
 #include "rdkv_common.h"
 #include <math.h>
 #include <string.h>
@@ -141,15 +141,15 @@ __device__ __forceinline__ float4 *chan_params_of(const StreamPackArgs &a) {
 
 // The K quantizer of one channel: scale, zero point, 1 / scale (rdkv_qcode's estimate) and, as bits,
 // the channel's stream slot with its width class (slot | class << 8; -1 for a channel that is not
-// kept).  One launch per layer makes them for every head (slot_params_kernel), the tile workgroups
+// kept).  slot_params_kernel makes them for every head of a batch's layers, the packing workgroups
 // read them.
 __device__ __forceinline__ float4 make_chan(float scale, float zp, float inv, int slot_cls) {
   return make_float4(scale, zp, inv, __int_as_float(slot_cls));
 }
 
 // One workgroup per head: stream slot -> position in the reference's padded sorted channel order
-// (src_slot, or RowPlan where the unit is planned here) -> width class and rank in the class -> the rank-th channel of that width in ascending
-// channel order (the stable sort of packing.py:241-294) -> the channel's parameters from its
+// (src_slot, or RowPlan where the unit is planned here) -> width class and rank in the class -> the rank-th
+// channel of that width in ascending channel order (the stable sort of packing.py:241-294) -> the channel's parameters from its
 // min / max.  Writes the per-channel parameters, the unit's slot table in the blob (with the
 // alignment gap behind it, and behind the last head the rest of the blob: no byte of the blob is
 // left to the caller), and starts the head's two scale maxima.

@@ -431,9 +431,10 @@ def _pack_entries_native(entries, G: int, rows_of_entries: Sequence[int], dev, s
 def _pack_entries_direct(entries, G: int, rows_of_entries: Sequence[int], entry_bytes: Optional[list] = None):
     """What ``_relayout_entries`` returns, from fp16 K / V and bit allocations instead of packed
     layers: every entry (K, V [1, H_kv, T, 128] fp16, v_bits [H_kv, T], k_bits [H_kv, 128]) is
-    quantized and laid out by ``rdkv_pack_layer_stream`` in two launches, the blob being what the
-    per-layer packer followed by the re-layout writes, bit for bit.  One planning launch pair and one
-    host read serve all entries of one shape.  An entry the direct kernel does not take (other types
+    quantized and laid out directly, the blob being what the
+    per-layer packer followed by the re-layout writes, bit for bit: entries of one shape together
+    (``rdkv_pack_layers_stream``, csrc/native.cpp), others by ``rdkv_pack_layer_stream`` one after the other.  One
+    planning launch pair and one host read serve all entries of one shape.  An entry the direct kernel does not take (other types
     or strides, nothing kept, no K channel kept) goes through ``packing.pack_layer_per_head`` and the
     re-layout instead."""
     from . import packing
@@ -695,7 +696,9 @@ _cus_of_device: dict = {}
 def _finish_caches(specs) -> List[StreamCache]:
     """``_finish_cache`` for several caches on one device at once: the host side of all of them
     first, then their unit and group tables in one queued copy, the largest scales (the one wait, when
-    they come from launches still running), the work tables in a second copy."""
+    they come from launches still running), the work tables in a second copy.  A cache whose scales are still on the
+    device has all its tables fetched by one launch there, which fills the work items' scale fields and sends the
+    scales to the host (``rdkv_stream_tables_device``)."""
     dev = specs[0][1][0].device
     if dev.index not in _cus_of_device:
         _cus_of_device[dev.index] = torch.cuda.get_device_properties(dev).multi_processor_count
