@@ -387,12 +387,14 @@ def pack_layer_sections(cfg, K, V, vb, kb, args, torch, dev):
         obkv_fast._perhead_select_and_pack_joint(K, V, tok_scores, ch_scores, **sel_kw)
         torch.cuda.synchronize()
         sel_ms.append((time.perf_counter() - t0) * 1e3)
-    obkv_fast._perhead_select_and_pack_joint(K, V, tok_scores, ch_scores, timing=stages, **sel_kw)
+    # (the stages are the general path's, which the calls above did not run: once ahead of the one that counts)
+    for times in ({}, stages):
+        obkv_fast._perhead_select_and_pack_joint(K, V, tok_scores, ch_scores, timing=times, **sel_kw)
     select_info = {"select_and_pack_ms_per_layer": float(np.median(sel_ms[1:])),
                    "stages_ms": {k: round(v, 4) for k, v in stages.items()},
                    "rows": H_kv, "tokens_per_row": T_ctx,
                    "note": "wall time of obkv_fast._perhead_select_and_pack_joint on layer 0 (median of "
-                           "5 after 1 warm-up); stages from one extra call that synchronizes after "
+                           "5 after 1 warm-up); stages from a second extra call that synchronizes after "
                            "each stage (quantization_ms = the whole-layer packer)"}
     if not args.no_cpu_baseline:
         from oracle import select_oracle
@@ -679,6 +681,7 @@ def decode_loop_section(cfg, torch, dev, tokens=48):
         res[f"ms_per_token_{name}"] = best
     # the blockwise variant: the generated tokens are re-compressed in blocks of 128 (budget 16)
     import contextlib
+    import gc
     import io
     from rdkv_amd import blockwise_decode as bw, knapsack_solver as ks
     conf = bw.BlockwiseRDKVConfig(
@@ -688,6 +691,7 @@ def decode_loop_section(cfg, torch, dev, tokens=48):
     n_bw = 272
     for name, graph in (("blockwise", False), ("blockwise_graph", True)):
         for _ in range(2):
+            gc.collect()          # a full collection of this process's objects takes 140 ms: not one that is due within a step
             with contextlib.redirect_stdout(io.StringIO()):       # the loop logs one event line per block
                 ids, report = bw.greedy_decode_blockwise(
                     model=model, dual_cache=cache, next_token_logits=first, max_new_tokens=n_bw, eos_token_ids=[],
